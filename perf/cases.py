@@ -9,8 +9,8 @@ brings one token), `seqs` sequences of `lo` to `hi` tokens (prompt lengths, or c
 
 A step is run as the engine runs it: step metadata through set_context, the model's forward, compute_logits; prompts eagerly, a
 decode step as the replay of a captured graph. Weights are seeded random tensors of a trained model's magnitudes: matrices scaled by
-their fan-in, norms around one, and embeddings that lean towards the experts of their token, so that a token's experts are
-chosen by a margin and not by the last bit (as a trained router's are).
+their fan-in, norms around one, and embeddings that say nothing along the routers' rows but which experts are their token's, so that a
+token's experts are chosen by a margin and not by the last bit (as a trained router's are).
 """
 import json
 import math
@@ -182,7 +182,7 @@ class _Weights:
                     steps.append(z)
                     rows[i] = basis[at:at + n]
                     at += n
-                self.leanings = rows, torch.cat(steps, 1) @ basis
+                self.leanings = rows, (torch.cat(steps, 1), basis)
             else:
                 self.leanings = rows, None
         return self.leanings
@@ -199,10 +199,13 @@ class _Weights:
         if fam == "qwen3":
             t = 1.0 + 0.1 * t if len(shape) == 1 else t / shape[-1] ** 0.5 * (shape[-1] ** 0.5 if "embed" in name else 0.5 if "down" in name else 1.0)
         elif name == "embed":
-            lean = self.directions()[1]
-            t = t if lean is None else t + lean
+            if self.directions()[1] is not None:             # nothing but the steps along the routers' rows
+                steps, basis = self.directions()[1]
+                t = t + (steps - t @ basis.T) @ basis
         elif name == "side.embed" or leaf == "sink":
             pass
+        elif "side" in parts and leaf == "norm":
+            t = 0.2 + 0.02 * t
         elif leaf in ("norm", "norm1", "norm2", "norm1b", "norm2b", "out", "D"):
             t = 0.1 * t + (0.0 if offset_norms else 1.0)
             if leaf in ("norm1b", "norm2b"):                 # a branch enters the stream at about half its size
@@ -226,7 +229,7 @@ class _Weights:
         elif leaf == "b" and not (fam == "ligidra" and len(shape) == 2):
             t = (t + (2.0 if name.endswith("f.b") else 0.0)) if fam == "lobidra" else 0.1 * t
         else:
-            t = t / (shape[-1] if shape else 1) ** 0.5 * ((0.25 if fam == "pefazen" else 0.5) if leaf == "down" else 1.0)
+            t = t / (shape[-1] if shape else 1) ** 0.5 * ((0.2 if fam == "pefazen" else 0.4) if leaf == "down" else 1.0)
         return t.to(torch.bfloat16)
 
 
