@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16_t* __rest
 template <bool GLU>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W, int nout,
                                                              int K, const int32_t* __restrict__ tile_expert,
-                                                             const int32_t* __restrict__ row_token, int tiles_m, int tiles_n,
+                                                             const int32_t* __restrict__ row_token, int tiles_m, int tiles_n, int tiles_per,
                                                              bf16_t* __restrict__ out, int64_t ldo, int mode) {
   constexpr int BM = 128, BW = 128, BK = 64, LDK = BK + 8, NG = GLU ? 2 : 1, FB = 4 / NG, BN = BW / NG;   // BN features per tile
   __shared__ __attribute__((aligned(16))) bf16_t Xs[BM][LDK];
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
   const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (logical >= tiles_m * tiles_n) return;
   const int rt = logical % tiles_m, ft = logical / tiles_m;
-  const int e = tile_expert[rt];
+  const int e = tile_expert[rt / tiles_per];
   if (e < 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = (lane >> 4) * 8;
   const int wm = wave & 1, wn = wave >> 1;
@@ -420,6 +420,204 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
       }
     }
   }
+}
+
+// Pipelined matrix-core form (bf16 with K % 64 == 0, 32-bit with K % 32 == 0: rows whose 128-byte pieces are whole). A workgroup of four
+// wavefronts computes BM = 16 RB (4 / WN) rows x BW = 16 WB WN weight rows (GLU: gate and up of the same BW / 2 features) in steps of 128
+// bytes along k; a wavefront owns 16 RB rows x 16 WB weight rows (WN wavefronts side by side along the weight rows).
+//
+// The operands go from memory straight into LDS (16 bytes per lane, no registers) through a ring of ST buffers. A step is two halves of
+// 64 bytes of k: while a half is multiplied the next half's operands are read from LDS; in the middle of a step every wavefront holds the rest
+// of the step's buffer in registers, so behind the one barrier of a step the step ST ahead is requested into it. Requests and reads
+// are issued between groups of MFMAs, where the matrix pipe hides them (one wavefront per SIMD has nobody else to). The barrier waits only
+// for the requests of the next step. A row's piece is 128 bytes of LDS; 16-byte unit c of row r sits at c ^ ((r >> 1) & 7), so
+// the 16 rows an operand read touches lie on 16 different bank quads (the requests fetch the units in that order; the direct path
+// could not write padding). The MFMAs are written out with accumulators in the accumulation registers and operands in the vector registers:
+// left to itself the compiler moves one or the other between the two files in the loop.
+//
+// Workgroups go to the eight XCDs round-robin; each XCD takes units of 8 row tiles x 4 feature tiles, whose operands its L2 then serves 4 and
+// up to 8 times, and neighbouring units go to different XCDs, so the unused row tiles at the end of the plan cost every XCD the same.
+//
+// Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
+// four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
+// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.36 + 1.27 ms = 1154 and 1073 TFLOP/s (the tiled kernel: 4.05 +
+// 2.28 ms; the library's dense product of these sizes: 1.3-1.46 PFLOP/s); what is left is the chip's power limit and half a tile of padding
+// per expert. 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
+// (moe_gemm_mfma_kernel 411 + 217); width 1024, ff 768: 20 + 12 us (58 + 27). 32-bit, 1,044 rows, width 1024: 59 + 32 us (moe_gemm_kernel
+// 1130 + 763), error against 64-bit sums 9e-7 of the result.
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef const __attribute__((address_space(1))) void global_void_t;
+
+__device__ __forceinline__ void dma16(const char* src, char* lds_row) {        // 64 lanes: LDS [lds_row + 16 lane] <- 16 bytes at src
+  __builtin_amdgcn_global_load_lds((global_void_t*)src, (lds_void_t*)lds_row, 16, 0, 0);
+}
+
+// one weight-row block times RB row blocks, 16 bytes of k per lane: 32 (bf16) or 16 (32-bit) of k
+template <typename T, int RB>
+__device__ __forceinline__ void mfma_units(f32x4_t (&acc)[RB], const u32x4_t& w, const u32x4_t (&x)[RB]) {
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[rb]) : "v"(w), "v"(x[rb]));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)                     // (a lane brings the same four entries of k in both operands: any order of k will do)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc[rb]) : "v"(w[i]), "v"(x[rb][i]));
+  }
+}
+
+template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __restrict__ X, int64_t ldx, const T* __restrict__ W, int nout, int K,
+                                                                    const int32_t* __restrict__ tile_expert,
+                                                                    const int32_t* __restrict__ row_token, int tiles_m, int tiles_n,
+                                                                    T* __restrict__ out, int64_t ldo, int mode) {
+  constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, NG = GLU ? 2 : 1, BN = BW / NG, ROW = 128, UNIT = 16 / sizeof(T);
+  constexpr int STAGE = (BM + BW) * ROW, XI = BM >= 32 ? BM / 32 : 1, WI = BW / 32, NR = XI + WI;      // requests of a wavefront per step
+  static_assert(WB % NG == 0 && BW % 32 == 0 && (ST - 2) * NR < 64, "tile");
+  extern __shared__ __attribute__((aligned(128))) char lds[];
+  const int j = blockIdx.x / 8, unit = (j / 32) * 8 + blockIdx.x % 8, units_n = (tiles_n + 3) / 4;
+  const int rt = unit / units_n * 8 + j % 8, ft = unit % units_n * 4 + (j % 32) / 8;
+  if (rt >= tiles_m || ft >= tiles_n) return;
+  const int e = tile_expert[rt];
+  if (e < 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15;
+  const int wn = wave % WN, wm = wave / WN;
+  const int64_t row0 = (int64_t)rt * BM;
+  // requests: one covers 8 rows; lane l brings unit (l & 7) ^ swizzle of row l >> 3. Padding rows and rows beyond the last feature bring
+  // some valid row; what is computed from them is not stored. (Tiles of 16 rows: two wavefronts bring the same rows twice.)
+  const char *xsrc[XI], *wsrc[WI];
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = (wave * XI + i) * 8 % BM + (lane >> 3);
+    const int tok = row_token[row0 + r];
+    const int64_t src = (GLU || mode == 2) ? (tok >= 0 ? tok : 0) : row0 + r;
+    xsrc[i] = (const char*)(X + src * ldx + ((lane & 7) ^ ((r >> 1) & 7)) * UNIT);
+  }
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    const int r = (wave * WI + i) * 8 + (lane >> 3), f = ft * BN + r % BN;
+    wsrc[i] = (const char*)(W + ((int64_t)(e * NG + r / BN) * nout + (f < nout ? f : nout - 1)) * K + ((lane & 7) ^ ((r >> 1) & 7)) * UNIT);
+  }
+  const auto request = [&](int i, int at, int step) {                   // request i of a step into the buffer at byte `at`
+    if (i < XI) dma16(xsrc[i < XI ? i : 0] + (int64_t)step * ROW, lds + at + (wave * XI + i) * 8 % BM * ROW);
+    else dma16(wsrc[i < XI ? 0 : i - XI] + (int64_t)step * ROW, lds + at + (BM + (wave * WI + i - XI) * 8) * ROW);
+  };
+  f32x4_t acc[WB][RB];
+#pragma unroll
+  for (int wb = 0; wb < WB; ++wb)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[wb][rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // operands of a half: weight-row block wb (GLU: the first half gate, the second up of the same features) and row block rb
+  struct Operands {
+    u32x4_t x[RB], w[WB];
+  };
+  constexpr int FB = WB / NG;                                           // feature blocks of a wavefront
+  const int unit0 = ((lane >> 4) ^ ((li >> 1) & 7)) * 16;               // (blocks start at multiples of 16 rows: the swizzle is the lane's)
+  const char* xrow = lds + (wm * 16 * RB + li) * ROW;
+  const char* wrow = lds + (BM + wn * FB * 16 + li) * ROW;
+  const auto load = [&](Operands& o, int g, int at, int half) {         // a WB-th of a half's operands
+    const int place = at + (unit0 ^ (half * 64));                       // unit (4 half + (lane >> 4)) ^ swizzle
+#pragma unroll
+    for (int i = g * RB / WB; i < (g + 1) * RB / WB; ++i) o.x[i] = *(const u32x4_t*)(xrow + place + i * 16 * ROW);
+    o.w[g] = *(const u32x4_t*)(wrow + place + (g / FB * BN + g % FB * 16) * ROW);
+  };
+  const auto half_step = [&](const Operands& now, Operands& next, int next_at, int next_half, bool ask, int ask_at, int ask_step) {
+    constexpr int AG = WB >= 4 ? WB / 2 : WB, PER = (NR + AG - 1) / AG;  // requests go out in the first half of the groups
+#pragma unroll
+    for (int g = 0; g < WB; ++g) {
+      if (ask && g < AG) {
+#pragma unroll
+        for (int i = g * PER; i < (g + 1) * PER; ++i)
+          if (i < NR) request(i, ask_at, ask_step);
+      }
+      load(next, g, next_at, next_half);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma_units<T, RB>(acc[g], now.w[g], now.x);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0): what was read ahead is there (the counter is too short to wait for it behind the next reads)
+  };
+  constexpr int AHEAD = (ST - 2) * NR;       // requests younger than the next step's
+  const auto arrive = [&](bool all) {        // the next step's requests landed (all: every request) and own LDS reads done; then everybody's
+    __builtin_amdgcn_sched_barrier(0);
+    if (all) __builtin_amdgcn_s_waitcnt(0);
+    else __builtin_amdgcn_s_waitcnt((AHEAD & 15) | (AHEAD >> 4) << 14);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int steps = K / (8 * UNIT);
+  Operands a, b;
+#pragma unroll
+  for (int s = 0; s < ST; ++s) {
+    if (s < steps) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) request(i, s * STAGE, s);
+    }
+  }
+  arrive(true);
+#pragma unroll
+  for (int g = 0; g < WB; ++g) load(a, g, 0, 0);
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  int at = 0, s = 0;
+#pragma unroll 1
+  for (; s + ST < steps; ++s) {
+    const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
+    half_step(a, b, at, 1, false, 0, 0);
+    arrive(ST == 2);
+    half_step(b, a, next, 0, true, at, s + ST);
+    at = next;
+  }
+#pragma unroll 1
+  for (; s < steps; ++s) {                   // the last ST steps: nothing left to request (the very last one reads ahead what nobody uses)
+    const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
+    half_step(a, b, at, 1, false, 0, 0);
+    arrive(true);
+    half_step(b, a, next, 0, false, 0, 0);
+    at = next;
+  }
+  asm volatile("s_nop 15\n\ts_nop 15");      // the last products are written before they are read: every read depends on one of
+#pragma unroll                             // these statements, and volatile ones keep their order
+  for (int wb = 0; wb < WB; ++wb)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) asm volatile("" : "+a"(acc[wb][rb]));
+  // lane: row li of row block rb; features 16 fb + 4 (lane >> 4) + 0..3 of its wavefront's
+  const bool quads = ((nout | (int)ldo) & 3) == 0 && ((uintptr_t)out & 15) == 0;
+  typedef __attribute__((ext_vector_type(4))) T t4_t;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int64_t r = row0 + (wm * RB + rb) * 16 + li;
+    if (row_token[r] < 0) continue;
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb) {
+      const int f = ft * BN + (wn * FB + fb) * 16 + (lane >> 4) * 4;
+      t4_t v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = (T)(GLU ? glu_value(acc[fb][rb][i], acc[GLU ? fb + FB : fb][rb][i], 0, 0.f, 0.f) : plain_value(acc[fb][rb][i], mode));
+      if (quads) {
+        if (f < nout) *(t4_t*)(out + r * ldo + f) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (f + i < nout) out[r * ldo + f + i] = v[i];
+      }
+    }
+  }
+}
+
+template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
+int launch_pipe(const void* X, int64_t ldx, const void* W, int nout, int K, const int32_t* tile_expert, const int32_t* row_token, int64_t cap,
+                void* out, int64_t ldo, int mode, hipStream_t st) {
+  constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, BN = GLU ? BW / 2 : BW, LDS = ST * (BM + BW) * 128;
+  const int64_t tiles_m = cap / BM, tiles_n = (nout + BN - 1) / BN;
+  const int64_t units = (tiles_m + 7) / 8 * ((tiles_n + 3) / 4), blocks = (units + 7) / 8 * 256;
+  NVS_REQUIRE(blocks < (1ll << 31), "nvs_moe_gemm: step too large");
+  const auto kernel = moe_gemm_pipe_kernel<T, GLU, WN, WB, RB, ST, PER_CU>;
+  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  NVS_REQUIRE(room == hipSuccess, "nvs_moe_gemm: %d bytes of LDS were refused", LDS);
+  kernel<<<dim3((unsigned)blocks), dim3(256), LDS, st>>>((const T*)X, ldx, (const T*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n,
+                                                         (T*)out, ldo, mode);
+  return nvs_check_launch("nvs_moe_gemm (matrix cores, pipelined)");
 }
 
 // ---- combine: one workgroup per token ------------------------------------------------------------------------------------
@@ -505,7 +703,7 @@ extern "C" int64_t nvs_moe_rows(int64_t pairs, int experts, int tm) { return (pa
 extern "C" int nvs_moe_plan(const int32_t* ids, int64_t n, int top, int experts, int tm, int32_t* tile_expert, int32_t* row_token,
                             int32_t* pair_row, void* stream) {
   NVS_REQUIRE(ids && tile_expert && row_token && pair_row && n >= 0 && top > 0, "nvs_moe_plan: null argument");
-  NVS_REQUIRE(experts > 0 && experts <= MAX_EXPERTS && (tm == 16 || tm == 64 || tm == 128), "nvs_moe_plan: %d experts, tiles of %d rows", experts, tm);
+  NVS_REQUIRE(experts > 0 && experts <= MAX_EXPERTS && (tm == 16 || tm == 64 || tm == 128 || tm == 256), "nvs_moe_plan: %d experts, tiles of %d rows", experts, tm);
   if (n == 0) return NVS_OK;
   const int64_t cap = nvs_moe_rows(n * top, experts, tm);
   NVS_REQUIRE(cap < (1ll << 31), "nvs_moe_plan: step too large");
@@ -517,22 +715,36 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
                             const int32_t* row_token, int64_t cap, int tm, void* out, int64_t ldo, void* stream) {
   NVS_REQUIRE(X && W && tile_expert && row_token && out && mode >= 0 && mode <= 2, "nvs_moe_gemm: bad argument");
   const int glu = mode == 1;
-  NVS_REQUIRE(nout > 0 && K > 0 && ldx >= K && ldo >= nout && (tm == 16 || tm == 64 || tm == 128) && cap >= 0 && cap % tm == 0,
+  NVS_REQUIRE(nout > 0 && K > 0 && ldx >= K && ldo >= nout && (tm == 16 || tm == 64 || tm == 128 || tm == 256) && cap >= 0 && cap % tm == 0,
               "nvs_moe_gemm: %d x %d, %lld rows in tiles of %d", nout, K, (long long)cap, tm);
   if (cap == 0) return NVS_OK;
   hipStream_t st = (hipStream_t)stream;
   const bool matrix_cores = dtype == NVS_BF16 && K % 8 == 0 && ldx % 8 == 0 && !g_moe_plain;
-  if (matrix_cores && tm == 128) {
+  const bool whole = (K % (dtype == NVS_BF16 ? 64 : 32) == 0) && ldx % (dtype == NVS_BF16 ? 8 : 4) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+  if (whole && !g_moe_plain) {
+#define NVS_PIPE(...)                                                                                                       \
+  (dtype == NVS_BF16                                                                                                        \
+       ? (glu ? launch_pipe<bf16_t, true, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st) \
+              : launch_pipe<bf16_t, false, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)) \
+       : (glu ? launch_pipe<float, true, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)  \
+              : launch_pipe<float, false, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)))
+    if (tm == 256) return NVS_PIPE(2, 8, 8, 2, 1);
+    if (tm == 128) return NVS_PIPE(2, 8, 4, 3, 1);
+    if (tm == 64) return NVS_PIPE(4, 4, 4, 2, 2);
+    return NVS_PIPE(4, 2, 1, 4, 2);
+#undef NVS_PIPE
+  }
+  if (matrix_cores && tm >= 128) {
     const int bn = glu ? 64 : 128;                  // features per tile
     const int tiles_m = (int)(cap / 128), tiles_n = (nout + bn - 1) / bn;
     const int64_t blocks = ((int64_t)tiles_m * tiles_n + 7) / 8 * 8;
     NVS_REQUIRE(blocks < (1ll << 31), "nvs_moe_gemm: step too large");
     if (glu)
       moe_gemm_tiled_kernel<true><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const bf16_t*)X, ldx, (const bf16_t*)W, nout, K, tile_expert,
-                                                                                row_token, tiles_m, tiles_n, (bf16_t*)out, ldo, mode);
+                                                                                row_token, tiles_m, tiles_n, tm / 128, (bf16_t*)out, ldo, mode);
     else
       moe_gemm_tiled_kernel<false><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const bf16_t*)X, ldx, (const bf16_t*)W, nout, K, tile_expert,
-                                                                                 row_token, tiles_m, tiles_n, (bf16_t*)out, ldo, mode);
+                                                                                 row_token, tiles_m, tiles_n, tm / 128, (bf16_t*)out, ldo, mode);
     return nvs_check_launch("nvs_moe_gemm (matrix cores, LDS tiles)");
   }
   if (matrix_cores) {

@@ -858,8 +858,7 @@ class RoutedExperts(nn.Module):
         else:
             z = F.linear(wide if wide is not None else xh.float(), self.router, self.router_b)      # 32-bit, [n, total (+ 1: the shared gate)]
             ids, wts = ops_seq.moe_route(z, total, self.correction, self.top, self.count, self.keep, self.scale, self.sigmoid, self.renorm)
-        per_expert = n * self.top // self.E                 # rows an expert gets on average: the tile height follows it
-        plan = ops_seq.moe_plan(ids, self.E, 128 if per_expert >= 256 else (64 if per_expert >= 64 else 16))
+        plan = ops_seq.moe_plan(ids, self.E, ops_seq.moe_tile_rows(n * self.top, self.E, width, self.ff, xh.dtype))
         act = torch.empty(plan.cap, self.ff, dtype=xh.dtype, device=xh.device)
         ops_seq.moe_gemm(xh, self.w_gu, plan, self.gated, act, relu2=not self.gated)
         rows = torch.empty(plan.cap, width, dtype=xh.dtype, device=xh.device)

@@ -604,6 +604,26 @@ class MoePlan:
     __slots__ = ("tile_expert", "row_token", "pair_row", "cap", "tm")
 
 
+def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dtype) -> int:
+    """Rows per tile of a step's plan. It follows the rows an expert gets on average: a tile reads all weights of its features, so few
+    rows want the smallest tile and many the largest. MI355X, gate|up + down of 32 gated experts, us at tiles of 16 / 64 / 128 / 256 rows:
+    width 4096, ff 3072: 8 rows 428 / 436 / 471 / 609; 32: 598 / 455 / 489 / 622; 64: 838 / 580 / 507 / 640; 250: 2256 / 1003 / 879 / 928;
+    1694: 12546 / 4674 / 4103 / 3634. Width 2048: 16 rows 126 / 133 / 149 / 178; 32: 141 / 135 / 155 / 181; 500: 1028 / 456 / 420 / 408.
+    Width 1024, ff 768 (few and short tiles: two small workgroups per compute unit cover each other's start and end better than one large
+    one fills it): 34 rows 40 / 44 / 50 / 66; 68: 52 / 48 / 53 / 70; 533: 287 / 149 / 166 / 179; 1807: 897 / 389 / 422 / 411.
+    32-bit: width 1024, 32 rows 80 / 126 / 228, 500: 830 / 836 / 912; width 2048, 32 rows 312 / 371 / 679, 125: 888 / 839 / 1100.
+    Rows that are no whole 128-byte pieces take the kernels that load their own operands, at the heights measured for those."""
+    per = pairs // experts
+    piece = 64 if dtype == torch.bfloat16 else 32
+    if width % piece or ff % piece:
+        return 128 if per >= 256 else 64 if per >= 64 else 16
+    if dtype != torch.bfloat16:
+        return 64 if per >= (96 if width >= 2048 else 512) else 16
+    if width < 2048:
+        return 64 if per >= 56 else 16
+    return 256 if per >= 448 else 128 if per >= 64 else 64 if per >= 24 else 16
+
+
 def moe_plan(ids: torch.Tensor, experts: int, tm: int) -> MoePlan:
     """Pairs (token, choice) sorted by expert into tiles of tm rows (ids >= experts get no row)."""
     lib = load_library()
