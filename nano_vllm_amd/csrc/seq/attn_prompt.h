@@ -1,0 +1,467 @@
+// Windowed attention over the paged cache, pipelined (bf16, 128-wide heads or latent rows of 256 with values of 192): device code shared by the
+// translation units that instantiate it (attn_prompt.hip: windows, blocks, causal; attn_prompt_pool.hip: the same with pooled blocks, capped
+// scores and row factors). Masks, sink, temperature, norm, rotation and gate mean what they mean in attn_window_core.h, whose kernels take every
+// other size.
+#pragma once
+#include "attn_window_core.h"
+
+int window_attn_prompt(const WindowAttnArgs& a, hipStream_t stream);               // attn_prompt.hip
+int window_attn_prompt_extended(const WindowAttnArgs& a, hipStream_t stream);      // attn_prompt_pool.hip
+
+namespace {
+
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef const __attribute__((address_space(1))) void global_void_t;
+
+__device__ __forceinline__ void dma16(const void* src, char* lds_at) {          // 64 lanes: LDS [lds_at + 16 lane] <- 16 bytes at src
+  __builtin_amdgcn_global_load_lds((global_void_t*)src, (lds_void_t*)lds_at, 16, 0, 0);
+}
+__device__ __forceinline__ float other_half(float v) {                          // the value of lane ^ 32
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
+}
+template <int N>
+struct Int { static constexpr int value = N; };
+template <int BEGIN, int END, typename F>
+__device__ __forceinline__ void static_for(const F& f) {                        // f(Int<BEGIN>) ... f(Int<END - 1>): the index is a constant
+  if constexpr (BEGIN < END) {
+    f(Int<BEGIN>{});
+    static_for<BEGIN + 1, END>(f);
+  }
+}
+
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float HIDDEN = -3e38f;                  // a masked score: its weight is 0 whatever the maximum is
+
+// A wavefront owns 32 consecutive queries of one head and walks over tiles of 64 keys, which all wavefronts of the workgroup share: `hw` heads of one
+// kv head times NW / hw groups of 32 queries. K and V tiles come straight into LDS, double-buffered, a round ahead.
+//
+// Everything is computed transposed, so that a lane owns ONE query (column lane & 31; the two halves of the wavefront hold different keys or value
+// columns of it) and a maximum or sum over keys needs one exchange between the halves:
+//   S^T [32 keys x 32 queries] = K Q^T, O^T [32 columns x 32 queries] += V^T P^T      (v_mfma_f32_32x32x16_bf16)
+// Row r of a block of 32 keys is key 16 (r >> 4) + 8 ((r >> 2) & 1) + 4 ((r >> 3) & 1) + (r & 3): the 16 scores a lane gets are then two runs of 8
+// consecutive keys, which, as bf16 weights, are its operand of the second product as they are.
+//
+// 128-wide heads (PIPE): in one round the matrix cores compute the sums of the round before and the scores of the round after, and between
+// those products stand pieces of this round's maximum and weights, so that a wavefront keeps both units busy; two workgroups of four wavefronts
+// fit a compute unit. Rows of 256: scores, weights, sums one after the other, by two wavefronts per SIMD (a workgroup of eight: 256 registers hold
+// one round's scores only) that fill each other's gaps.
+//
+// What bounds it: per round and wavefront 32 MFMAs (rows of 256: 56) of 32 clocks, as much of the LDS pipe's time for eight wavefronts, and about 900
+// clocks of vector work; the matrix units run at 0.95-1.06 PFLOP/s on one prompt of 16,384 tokens. On shorter ones the time before the first and
+// behind the last round shows: queries, norm and rotation are prepared while the first tile is on its way, cos and sin once per position and
+// workgroup. 64 queries per wavefront (half the LDS reads) need the accumulation registers, and the compiler's moves to and from them cost more.
+// MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 333, blocks of
+// 1024 with rotation 936 -> 261; 16 / 8 heads, causal, rotation, sink 764 -> 196; latent rows, 16 heads, window 1024 1012 -> 261, causal 1014 -> 291.
+template <int D, int DV, int NW, bool EXT>
+__global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_kernel(const WindowAttnArgs A) {
+  constexpr bool PIPE = D == 128;
+  constexpr int KB = 64 * D * 2, VB = DV * 128, TILE = KB + VB, KU = D / 8, KI = KB / 1024 / NW, VI = VB / 1024 / NW, DC = D / 16, DB = DV / 32;
+  extern __shared__ __attribute__((aligned(128))) char lds[];                   // K tile, V tile; K tile, V tile
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ql = lane & 31, hi = lane >> 5;
+  const int H = A.H, G = A.G, hpg = H / G, hw = A.hw, chunks = hpg / hw, window = A.window, chunk = A.chunk, bs = A.block_size;
+  const int g = blockIdx.y / chunks, h = g * hpg + (blockIdx.y % chunks) * hw + wave % hw;
+  const int BQ = (NW / hw) * 32;
+  // the portion of this workgroup's tile: 64 portions at a time, their tile counts summed over the lanes
+  int btile = blockIdx.x, s = 0, len = 0, row0 = 0;
+  for (int base = 0;; base += 64) {
+    const int i = base + lane;
+    const int first = i <= A.nseq ? A.cu_q[i] : 0, n_i = i < A.nseq ? A.cu_q[i + 1] - first : 0, tiles = (n_i + BQ - 1) / BQ;
+    int sum = tiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(sum, d, 64);
+      sum += lane >= d ? up : 0;
+    }
+    const uint64_t in = __ballot(btile < sum);
+    if (in != 0) {
+      const int at = __builtin_ctzll(in);
+      s = base + at;
+      len = __builtin_amdgcn_readlane(n_i, at);
+      row0 = __builtin_amdgcn_readlane(first, at);
+      btile -= __builtin_amdgcn_readlane(sum - tiles, at);
+      break;
+    }
+    btile -= __builtin_amdgcn_readlane(sum, 63);
+    if (base + 64 >= A.nseq) return;                // the whole workgroup leaves
+  }
+  btile = (len + BQ - 1) / BQ - 1 - btile;          // the last query tiles of a portion, which see the most, go first
+  const int c0 = __builtin_amdgcn_readfirstlane(A.ctx0[s]);
+  const int rel0 = btile * BQ + wave / hw * 32, p_first = c0 + rel0, p_hi = p_first + 31;
+  const int b_first = c0 + btile * BQ, b_last = c0 + (btile * BQ + BQ < len ? btile * BQ + BQ : len) - 1;
+  const int32_t* __restrict__ bt = A.block_tables + (int64_t)s * A.bt_stride;
+
+  // ---- rounds: EXT: [0, npr) hold 64 pooled blocks each, the others 64 tokens, the first from a multiple of 64 on
+  const int lo = vis_lo(b_first, window, chunk);
+  const int nb_last = EXT ? seen_blocks(b_last, window, A.pool) : 0, npr = EXT ? (nb_last + 63) >> 6 : 0;
+  const int jt = (lo & ~63) - npr * 64;
+  const int rounds = npr + ((b_last - (lo & ~63)) >> 6) + 1;
+  // the rounds every query of this wavefront sees in whole
+  const int nb_first = EXT ? seen_blocks(p_first, window, A.pool) : 0, lo_hi = vis_lo(p_hi, window, chunk);
+
+  // ---- requests. K tile: row = token, 2 D bytes, 16-byte unit u of token t at u ^ (t & 15). V tile: row = value column, 64 tokens = 128 bytes, unit u of
+  // column c at u ^ ((c >> 1) & 7). Both make the 16-byte operand reads of 16 neighbouring lanes cover all banks once.
+  uint32_t koff[KI], voff[VI];                      // bytes from the tile's first row
+  int kblk[KI], vblk[2];                            // EXT: unit of 8 blocks of a request's rows; of a lane's tokens (even, odd requests)
+#pragma unroll
+  for (int i = 0; i < KI; ++i) {
+    const int r = (wave * KI + i) * (64 / KU) + lane / KU, u = (lane % KU) ^ (r & 15);
+    koff[i] = (uint32_t)(((EXT ? r & 7 : r) * G * D + u * 8) * 2);
+    kblk[i] = r >> 3;
+  }
+#pragma unroll
+  for (int i = 0; i < VI; ++i) {
+    const int c = (wave * VI + i) * 8 + (lane >> 3), u = (lane & 7) ^ ((c >> 1) & 7);
+    voff[i] = (uint32_t)((EXT ? c * 8 : c * bs + u * 8) * 2);
+    if (i < 2) vblk[i] = u;
+  }
+  // Pages (EXT: units of pooled blocks) are looked up a round before the requests that use them: a lookup inside a request would wait for
+  // everything in flight. kpg, vpg: of the next K and V tile to be requested (EXT: of a wavefront's first and last rows, of its even and odd requests).
+  int kpg[2] = {}, vpg[2] = {};
+  const auto unit_of = [&](int it, int u) {         // unit u of pooled round it (one that nobody sees: the round's first)
+    return pool_unit(it * 8 + (it * 64 + u * 8 < nb_last ? u : 0), A.pool, bs, bt);
+  };
+  const auto page_of = [&](int it) { return bt[(jt + it * 64) >> A.bs_shift]; };
+  const auto lookup_k = [&](int it) {
+    if (it >= rounds) return;
+    if (EXT && it < npr) kpg[0] = unit_of(it, kblk[0]), kpg[1] = unit_of(it, kblk[KI - 1]);
+    else kpg[0] = page_of(it);
+  };
+  const auto lookup_v = [&](int it) {
+    if (it >= rounds) return;
+    if (EXT && it < npr) vpg[0] = unit_of(it, vblk[0]), vpg[1] = unit_of(it, vblk[1]);
+    else vpg[0] = page_of(it);
+  };
+  const auto request_k = [&](int it, int buf) {
+    if (it >= rounds) return;
+    char* at = lds + buf * TILE + wave * KI * 1024;
+    if (EXT && it < npr) {
+#pragma unroll
+      for (int i = 0; i < KI; ++i) dma16((const char*)A.pool_k + ((int64_t)kpg[2 * i / KI] * 8 * G + g) * D * 2 + koff[i], at + i * 1024);
+      return;
+    }
+    const int off = (jt + it * 64) & (bs - 1), page = __builtin_amdgcn_readfirstlane(kpg[0]);
+    const char* base = (const char*)A.k_cache + ((((int64_t)page << A.bs_shift) + off) * G + g) * D * 2;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) dma16(base + koff[i] + (EXT ? (uint32_t)kblk[i] * 8 * G * D * 2 : 0u), at + i * 1024);
+  };
+  const auto request_v = [&](int it, int buf) {
+    if (it >= rounds) return;
+    char* at = lds + buf * TILE + KB + wave * VI * 1024;
+    if (EXT && it < npr) {
+#pragma unroll
+      for (int i = 0; i < VI; ++i) dma16((const char*)A.pool_v + ((int64_t)vpg[i & 1] * G + g) * DV * 16 + voff[i], at + i * 1024);
+      return;
+    }
+    const int off = (jt + it * 64) & (bs - 1), page = __builtin_amdgcn_readfirstlane(vpg[0]);
+    const char* base = (const char*)A.v_cache + (((((int64_t)page * G + g) * DV) << A.bs_shift) + off) * 2;
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      const int c = (wave * VI + i) * 8 + (lane >> 3);
+      dma16(base + (EXT ? (uint32_t)((c * bs + vblk[i & 1] * 8) * 2) : voff[i]), at + i * 1024);
+    }
+  };
+  // Tokens behind the step's last one lie in the page but belong to nobody: their weight is 0, and their values are made 0 too, since what a
+  // page held before may be an infinity. (Pooled rounds: blocks nobody sees, likewise; a round behind the last one: all of it.)
+  const auto clear_tail = [&](int it, int buf) {
+    if (it < rounds - 1 && !(EXT && it == npr - 1)) return;
+    const int live = EXT && it < npr ? nb_last - it * 64 : b_last - (jt + it * 64) + 1;
+    if (live >= 64) return;
+    char* at = lds + buf * TILE + KB;
+    for (int i = tid; i < DV * 64; i += 64 * NW) {
+      const int c = i >> 6, t = i & 63;
+      if (t >= live) *(bf16_t*)(at + c * 128 + (((t >> 3) ^ ((c >> 1) & 7)) << 4) + (t & 7) * 2) = (bf16_t)0.f;
+    }
+    __syncthreads();
+  };
+  const auto arrive = [&] {                         // own requests landed and own reads done; then everybody's
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  lookup_k(0);
+  lookup_v(0);
+  request_k(0, 0);
+  request_v(0, 0);
+  lookup_k(1);
+  lookup_v(1);
+
+  // ---- queries, while the first tile is on its way: lane holds entries 16 c + 8 hi .. + 7 of query ql, normed, turned and scaled
+  const int rel = rel0 + ql, pos = c0 + rel;
+  const bool valid = rel < len;
+  const int64_t row = (int64_t)row0 + (valid ? rel : len - 1);
+  bf16x8_t qb[DC];
+  {
+    const bf16_t* qp = (const bf16_t*)A.q + row * A.q_stride + (int64_t)h * D + 8 * hi;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) qb[c] = *(const bf16x8_t*)(qp + 16 * c);
+    const int pairs = A.rot_dims / 2;
+    const bool table = pairs > 0 && BQ * pairs * 8 <= TILE;                     // cos and sin once per position, not once per head
+    float2* turn = (float2*)(lds + TILE);
+    if (table) {
+      for (int i = tid; i < BQ * pairs; i += 64 * NW) {
+        const int p = i / pairs, j = i - p * pairs;
+        float sn, cs;
+        sincosf((float)(b_first + p) * A.rot_freq[j], &sn, &cs);
+        turn[i] = make_float2(cs, sn);
+      }
+      __syncthreads();
+    }
+    float r = A.scale * query_temp(pos, A.qt_coef, A.qt_every);
+    const bf16_t* qw = (const bf16_t*)A.qnorm;
+    if (EXT && A.q_row) {
+      r *= A.q_row[row];
+      qw += (int64_t)h * D;
+    } else if (qw) {
+      float ss = 0.f;
+#pragma unroll
+      for (int c = 0; c < DC; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += (float)qb[c][e] * (float)qb[c][e];
+      ss += other_half(ss);
+      r *= rsqrtf(ss / (float)D + A.eps);
+    }
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      float w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = 1.f;
+      if (qw) ldp<8>(qw + 16 * c + 8 * hi, w);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const int col = 16 * c + 8 * hi + e;
+        float a = (float)qb[c][e] * r * w[e], b = (float)qb[c][e + 1] * r * w[e + 1];
+        if (col < A.rot_dims) {                     // the pair (2i, 2i+1) turns by pos * freq[i]
+          float sn, cs;
+          if (table) {
+            const float2 f = turn[(rel - btile * BQ) * pairs + (col >> 1)];
+            cs = f.x, sn = f.y;
+          } else {
+            sincosf((float)pos * A.rot_freq[col >> 1], &sn, &cs);
+          }
+          const float a2 = a * cs - b * sn;
+          b = b * cs + a * sn;
+          a = a2;
+        }
+        qb[c][e] = (bf16_t)a, qb[c][e + 1] = (bf16_t)b;
+      }
+    }
+  }
+  // a sink is a score in the denominator without a value; the sum starts from it (once per query: in the lower half of the lanes)
+  float m = A.sink ? A.sink[h] : -1e30f, l = A.sink && hi == 0 ? 1.f : 0.f;
+  f32x16_t o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
+
+  // ---- operands
+  const int ktok = 16 * (ql >> 4) + 8 * ((ql >> 2) & 1) + 4 * ((ql >> 3) & 1) + (ql & 3);
+  const char* kread = lds + ktok * D * 2;
+  const int kswz = (hi ^ (ktok & 15)) * 16;          // unit 2 c + hi, swizzled: (2 c) ^ this
+  const char* vread = lds + KB + ql * 128;
+  const int vswz = (hi ^ ((ql >> 1) & 7)) * 16;      // unit 2 a + hi
+  const auto k_operand = [&](int buf, int kb, int c) { return *(const bf16x8_t*)(kread + buf * TILE + kb * 32 * D * 2 + (kswz ^ (c * 32))); };
+  const auto v_operand = [&](int buf, int a, int db) { return *(const bf16x8_t*)(vread + buf * TILE + db * 32 * 128 + (vswz ^ (a * 32))); };
+  const auto s_product = [&](f32x16_t& d, const bf16x8_t& k, int c) {
+    const f32x16_t zero = {};
+    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, qb[c], c == 0 ? zero : d, 0, 0, 0);
+  };
+  const auto o_product = [&](f32x16_t& d, const bf16x8_t& v, const u32x4_t& p) {
+    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, __builtin_bit_cast(bf16x8_t, p), d, 0, 0, 0);
+  };
+
+  // ---- the vector units' part of round `it`, in 13 pieces: caps, masks and maxima of eight scores (0-3), the new maximum (4), four weights (5-12)
+  float mx = HIDDEN, off = 0.f, alpha = 1.f;
+  bool whole = true, moved = false;
+  int rlo = 0;
+  unsigned rlen = 0u;
+  const auto begin = [&](int it) {
+    const bool pooled = EXT && it < npr;
+    const int j0 = pooled ? it * 64 : jt + it * 64;
+    whole = pooled ? j0 + 63 < nb_first : j0 + 63 <= p_first && j0 >= lo_hi;
+    if (!whole) {                                   // visible: tokens rlo .. rlo + rlen of the round, counted from this lane's first
+      const int top = pooled ? seen_blocks(pos, window, A.pool) - 1 : pos, bottom = pooled ? 0 : vis_lo(pos, window, chunk);
+      rlo = top >= bottom ? bottom - j0 - 8 * hi : 0x40000000;
+      rlen = top >= bottom ? (unsigned)(top - bottom) : 0u;
+    }
+  };
+  const auto work = [&](auto unit, f32x16_t (&sc)[2], u32x4_t (&pb)[4]) {
+    constexpr int u = decltype(unit)::value;
+    if constexpr (u < 4) {
+      f32x16_t& v = sc[u >> 1];
+      if constexpr (u == 0) mx = HIDDEN;
+      if (EXT) {
+        if (A.softcap > 0.f) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[(u & 1) * 8 + i] = capped(v[(u & 1) * 8 + i], A.softcap);
+        }
+      }
+      if (!whole) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if ((unsigned)(u * 16 + i - rlo) > rlen) v[(u & 1) * 8 + i] = HIDDEN;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, v[(u & 1) * 8 + i]);
+      asm volatile("" : "+v"(mx));                  // (a piece stays where it stands: the compiler would move all of it to where it is used)
+    } else if constexpr (u == 4) {
+      const float mn = fmaxf(m, fmaxf(mx, other_half(mx)));
+      moved = __ballot(mn != m) != 0ull;
+      alpha = __builtin_amdgcn_exp2f((m - mn) * LOG2E);
+      l *= alpha;
+      m = mn;
+      off = -mn * LOG2E;
+      asm volatile("" : "+v"(alpha), "+v"(off), "+v"(l));
+    } else {
+      typedef __attribute__((ext_vector_type(2))) __bf16 b2_t;
+      constexpr int i0 = (u - 5) * 4;
+      float p[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i0 >> 4][(i0 & 15) + i], LOG2E, off));
+      l += (p[0] + p[1]) + (p[2] + p[3]);
+      unsigned w0 = __builtin_bit_cast(unsigned, b2_t{(bf16_t)p[0], (bf16_t)p[1]}), w1 = __builtin_bit_cast(unsigned, b2_t{(bf16_t)p[2], (bf16_t)p[3]});
+      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(l));
+      pb[i0 >> 3][(i0 & 7) >> 1] = w0;
+      pb[i0 >> 3][((i0 & 7) >> 1) + 1] = w1;
+    }
+  };
+  const auto rescale = [&] {
+    if (moved) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o[db] *= alpha;
+    }
+  };
+  constexpr int UNITS = 13, AHEAD = 3;              // AHEAD: operands read ahead of their products
+
+  if constexpr (PIPE) {
+    f32x16_t sc[2][2];
+    u32x4_t pb[2][4];
+    // Round it: sums of round it - 1 (V tile in buffer nxt), scores of round it + 1 (K tile in buffer nxt); K tile it + 2 and V tile it come into cur.
+    const auto round = [&](auto first, int it, auto which) {
+      constexpr bool WITH_O = decltype(first)::value == 0;
+      constexpr int cur = decltype(which)::value, nxt = cur ^ 1, OS = WITH_O ? 4 * DB : 0, SLOTS = OS + 2 * DC;
+      arrive();
+      if (WITH_O) clear_tail(it - 1, nxt);
+      request_k(it + 2, cur);
+      if (WITH_O) request_v(it, cur);
+      lookup_k(it + 3);
+      if (WITH_O) lookup_v(it + 1);
+      begin(it);
+      bf16x8_t ring[AHEAD + 1];
+      const auto operand = [&](int slot) { return slot < OS ? v_operand(nxt, slot / DB, slot % DB) : k_operand(nxt, (slot - OS) / DC, (slot - OS) % DC); };
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) ring[i] = operand(i);
+      static_for<0, SLOTS>([&](auto index) {
+        constexpr int slot = decltype(index)::value;
+        if constexpr (slot + AHEAD < SLOTS) ring[(slot + AHEAD) % (AHEAD + 1)] = operand(slot + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (slot < OS) o_product(o[slot % DB], ring[slot % (AHEAD + 1)], pb[nxt][slot / DB]);
+        else s_product(sc[nxt][(slot - OS) / DC], ring[slot % (AHEAD + 1)], (slot - OS) % DC);
+        static_for<slot * UNITS / SLOTS, (slot + 1) * UNITS / SLOTS>([&](auto u) { work(u, sc[cur], pb[cur]); });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if (WITH_O) rescale();
+    };
+    arrive();
+    request_k(1, 1);
+    lookup_k(2);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int c = 0; c < DC; ++c) s_product(sc[0][kb], k_operand(0, kb, c), c);
+    round(Int<1>{}, 0, Int<0>{});
+#pragma unroll 1
+    for (int it = 1; it < rounds; it += 2) {        // (in pairs: an odd one at the end is a round that nobody sees)
+      round(Int<0>{}, it, Int<1>{});
+      round(Int<0>{}, it + 1, Int<0>{});
+    }
+    arrive();
+    clear_tail(rounds / 2 * 2, 0);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o_product(o[db], v_operand(0, a, db), pb[0][a]);
+  } else {
+    f32x16_t sc[2];
+    u32x4_t pb[4];
+    const auto round = [&](int it, int cur) {
+      arrive();
+      clear_tail(it, cur);
+      request_k(it + 1, cur ^ 1);
+      request_v(it + 1, cur ^ 1);
+      lookup_k(it + 2);
+      lookup_v(it + 2);
+      begin(it);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int c = 0; c < DC; ++c) s_product(sc[kb], k_operand(cur, kb, c), c);
+      static_for<0, UNITS>([&](auto u) { work(u, sc, pb); });
+      rescale();
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o_product(o[db], v_operand(cur, a, db), pb[a]);
+    };
+#pragma unroll 1
+    for (int it = 0; it < rounds; ++it) round(it, it & 1);
+  }
+
+  // ---- out: lane holds columns 32 db + 8 a + 4 hi .. + 3 of query ql
+  typedef __attribute__((ext_vector_type(4))) __bf16 b4_t;
+  const float inv = 1.f / (l + other_half(l));
+  if (!valid) return;
+  bf16_t* op = (bf16_t*)A.out + (row * H + h) * DV + 4 * hi;
+  const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + row * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
+  const auto gated = [](float x, float gv) { return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-gv * LOG2E)); };
+  const bool wide = gp && A.gate_w != 1;
+  const float ginv = gp && !wide ? gated(inv, (float)gp[0]) : inv;
+  const bool quads = wide && ((A.gate_stride & 3) == 0) && ((uintptr_t)A.gate & 7) == 0;
+#pragma unroll
+  for (int db = 0; db < DB; ++db) {
+    b4_t gv[4];
+    if (quads) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a) gv[a] = *(const b4_t*)(gp + 32 * db + 8 * a + 4 * hi);
+    } else if (wide) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gv[a][i] = gp[32 * db + 8 * a + 4 * hi + i];
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      b4_t v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = o[db][4 * a + i] * ginv;
+        if (wide) x = gated(x, (float)gv[a][i]);
+        v[i] = (bf16_t)x;
+      }
+      *(b4_t*)(op + 32 * db + 8 * a) = v;
+    }
+  }
+}
+
+template <int D, int DV, int NW, bool EXT>
+int launch_prompt(WindowAttnArgs a, hipStream_t stream) {
+  const int hpg = a.H / a.G;
+  a.hw = hpg % NW == 0 ? NW : (hpg % 4 == 0 ? 4 : (hpg % 2 == 0 ? 2 : 1));
+  a.bs_shift = __builtin_ctz(a.block_size);
+  const int bq = (NW / a.hw) * 32;
+  const int64_t btiles = a.n / bq + a.nseq;         // an upper bound: every portion may end with a partial tile
+  constexpr int LDS = 2 * (64 * D * 2 + DV * 128);
+  const auto kernel = window_attn_prompt_kernel<D, DV, NW, EXT>;
+  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  NVS_REQUIRE(room == hipSuccess, "nvs_window_attn: %d bytes of LDS were refused", LDS);
+  kernel<<<dim3((unsigned)btiles, (unsigned)(a.G * (hpg / a.hw))), dim3(64 * NW), LDS, stream>>>(a);
+  return nvs_check_launch("nvs_window_attn (prompts)");
+}
+
+}  // namespace

@@ -1,0 +1,75 @@
+"""The attention kernel for steps of prompts (csrc/seq/attn_prompt.h) against the scalar kernel, which takes every call: portions around its tiles of
+32 queries and 64 keys, behind contexts that end anywhere in a page, all masks, sinks, norms, rotations, gates and pooled blocks, and pages whose
+unused places hold infinities and NaN."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+PAGE = 64
+
+
+def call(scalar, H, G, d, dv, lens, ctx, window=0, chunk=0, rot=0, norm="", sink=False, gate=0, temp=None, pool=0, cap=0.0, seed=0):
+    from nano_vllm_amd import ops_seq
+    g = torch.Generator().manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    n, total = sum(lens), [a + b for a, b in zip(lens, ctx)]
+    need = [-(-t // PAGE) for t in total]
+    ids = torch.randperm(sum(need) + 2, generator=g)[:sum(need)].split(need)
+    table = torch.full((len(lens), max(need) + 1), -1, dtype=torch.int32)
+    pages = sum(need) + 2
+    k, v = rand(pages, PAGE, G, d), rand(pages, G, dv, PAGE)
+    for row, (mine, t) in enumerate(zip(ids, total)):
+        table[row, :len(mine)] = mine.to(torch.int32)
+        if t % PAGE:                                        # what an earlier request left behind the end
+            k[mine[-1], t % PAGE:] = float("nan")
+            v[mine[-1], :, :, t % PAGE:] = float("inf")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    por = ops_seq.Portions(i32([0] + lens).cumsum(0).to(torch.int32), i32(ctx), i32(list(range(len(lens)))),
+                           torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32).cuda(), len(lens), n, max(lens))
+    bf = lambda x: x.to(torch.bfloat16).cuda()
+    q = bf(rand(n, H * d + 8))[:, :H * d]
+    w = bf(1 + 0.1 * rand(H * d if norm == "rows" else d)) if norm else None
+    kw = dict(gate_per_head=gate == 1, sink=rand(H).cuda() if sink else None, q_temp=temp, softcap=cap)
+    if norm == "rows":
+        kw["q_row"] = (0.5 + torch.rand(n, generator=g)).cuda()
+    kc = bf(k).view(pages * PAGE, G, d)
+    vc = bf(v).view(pages * PAGE, G, dv)
+    if pool:
+        rows = ops_seq.pool_rows(PAGE, pool)
+        kw.update(pool=pool, pool_k=bf(rand(pages, rows, G, d)), pool_v=bf(rand(pages, rows // 8, G, dv, 8)))
+    gates = bf(rand(n, H * (1 if gate == 1 else dv))) if gate else None
+    freq = (1000.0 ** (-torch.arange(rot // 2) / max(rot // 2, 1))).float().cuda() if rot else None
+    out = torch.full((n, H * dv), 9.0, dtype=torch.bfloat16, device="cuda")
+    lib = ops_seq.load_library()
+    lib.nvs_window_attn_force_scalar(1 if scalar else 0)
+    try:
+        ops_seq.window_attn(q, w, 1e-6, gates, kc, vc, table.cuda(), PAGE, por, H, G, d, dv, d ** -0.5, window, out, chunk, freq, **kw)
+    finally:
+        lib.nvs_window_attn_force_scalar(0)
+    return out
+
+
+CASES = [
+    dict(H=4, G=2, lens=[1, 31, 32, 33, 63, 64, 65, 129], ctx=[0] * 8),
+    dict(H=8, G=2, lens=[200, 40, 96], ctx=[63, 64, 1], window=33, sink=True),
+    dict(H=3, G=3, lens=[90, 70], ctx=[0, 130], chunk=48, rot=128, norm="head"),
+    dict(H=8, G=1, lens=[300], ctx=[5], window=64, gate=2, temp=(0.3, 16)),
+    dict(H=6, G=2, lens=[65, 64], ctx=[100, 0], rot=40, gate=1, sink=True),
+    dict(H=4, G=2, lens=[400, 66], ctx=[0, 333], window=40, pool=4, cap=5.0, norm="rows", sink=True),
+    dict(H=4, G=4, lens=[150, 64], ctx=[700, 0], window=64, pool=16, cap=30.0, norm="rows", rot=64),
+    dict(H=2, G=1, lens=[130], ctx=[0], cap=4.0),
+    dict(H=1, G=1, lens=[17] * 70, ctx=[i for i in range(70)]),
+]
+
+
+@pytest.mark.parametrize("d,dv,case", [(128, 128, i) for i in range(len(CASES))] +
+                         [(256, 192, i) for i, c in enumerate(CASES) if not (c.get("cap") or c.get("pool"))])      # (those sizes take the kernel without the extensions)
+def test_prompt_kernel_agrees_with_the_scalar_kernel(d, dv, case):
+    kw = dict(CASES[case], d=d, dv=dv, seed=case)
+    got, want = call(False, **kw).double(), call(True, **kw).double()
+    assert torch.isfinite(want).all()
+    # both round the finished query and the result to 8 bits; the matrix cores round the weights too (2^-9 each, averaged over the keys)
+    err = ((got - want).norm() / want.norm()).item()
+    assert err <= 2.0 ** -7, err
+    assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
