@@ -1,6 +1,6 @@
 // The gated delta rule (see nvs_delta_scan in include/nvl_seq.h): a matrix state per head whose write is the ERROR of what the
 // state already answers for the key. Everything from the unit norms on is 32-bit.
-#include "seq_common.h"
+#include "f32_tiles.h"
 
 namespace {
 
@@ -199,18 +199,7 @@ void launch_walk(const DeltaArgs& A, int nseq, hipStream_t stream) {
 // Decay products are multiplied up (no exponential of a difference). Per-channel decays: A and M are products of G k with k / G as
 // long as no channel decays by more than 1e-30 within the chunk; otherwise every pair (j, t) is walked with the product G_t / G_j
 // carried along. A partial chunk is filled with tokens that change nothing (k = q = v = 0, beta = 0, decay 1).
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 constexpr int CHUNK = 16, PREP = 256, MST = 20;      // MST: row stride of the 16 x 16 matrices in LDS (float4-aligned)
-
-__device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-// A barrier for data in LDS only: __syncthreads would also wait for every global load in flight, and the next chunk's loads are
-// meant to stay in flight across the barriers of this one.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // softplus from the hardware exponential and logarithm; the error of the decay's exponent stays at a few 1e-8 (log(1 + e) by its
 // series where e is small)

@@ -1,7 +1,7 @@
 // Stateful sequence kernels: causal convolution, real-gated linear recurrence, state-space-duality recurrence (recurrent
 // form), gated group norm. State lives in 32-bit in per-sequence slots; a portion whose first token is position 0 starts
 // from zeros whatever the slot holds.
-#include "seq_common.h"
+#include "scan_chunk.h"
 #include <stdlib.h>
 
 namespace {
@@ -243,6 +243,7 @@ extern "C" int64_t nvs_rglru_scan_workspace(int channels, int nseq, int64_t max_
 }
 
 // ---- state-space-duality recurrence -------------------------------------------------------------------------------
+// The walk over single tokens, for state sizes and addresses that the chunks of scan_chunk.hip do not take.
 // One workgroup per (portion, head), (P / PP) * NG threads: thread (tid / NG, g = tid % NG) keeps the 16 state entries
 // S[p][16 g .. 16 g + 15] of PP consecutive p in registers (state memory is [heads][P][N], n fastest: a thread's entries are contiguous).
 // Tokens go in rounds of TB: the round's x | B | C | dt | decay are staged in LDS by all threads, then every token costs 16 x (2 FMA + 1 MUL) per thread, LDS
@@ -763,13 +764,19 @@ static void ssd_plan(int heads, int nseq, int64_t max_q, int* seg_len, int* nseg
 extern "C" int64_t nvs_ssd_scan_workspace(int heads, int P, int N, int nseq, int64_t max_q) {
   int seg_len, nseg;
   ssd_plan(heads, nseq, max_q, &seg_len, &nseg);
-  return seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)P * N + 1) : 0;
+  const int64_t walk = seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)P * N + 1) : 0;
+  scan_chunk_plan(heads, P, nseq, max_q, &seg_len, &nseg);
+  const int64_t chunk = seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)P * N + 1) : 0;
+  return walk > chunk ? walk : chunk;               // (which of the two it is also depends on types and addresses)
 }
 
 extern "C" int64_t nvs_gated_memory_scan_workspace(int heads, int dk, int dv, int nseq, int64_t max_q) {
   int seg_len, nseg;
   ssd_plan(heads, nseq, max_q, &seg_len, &nseg, 192);
-  return seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)(dv + 1) * dk + 3) : 0;
+  const int64_t walk = seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)(dv + 1) * dk + 3) : 0;
+  scan_chunk_plan(heads, dv + 1, nseq, max_q, &seg_len, &nseg);
+  const int64_t chunk = seg_len ? (int64_t)nseq * heads * (nseg + 1) * ((int64_t)(dv + 1) * dk + 3) : 0;
+  return walk > chunk ? walk : chunk;
 }
 
 // what only the matrix memory (form 2) passes
@@ -788,6 +795,10 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   NVS_REQUIRE(heads > 0 && G > 0 && heads % G == 0 && P > 0 && P <= 257 && N > 0 && nseq >= 0 && nseq <= 65535,
               "%s: heads %d groups %d head size %d state %d", who, heads, G, P, N);
   if (n == 0 || nseq == 0) return NVS_OK;
+  if (max_q <= 0) max_q = n;
+  NVS_REQUIRE(!ws || ws_floats >= (form == 2 ? nvs_gated_memory_scan_workspace(heads, N, P - 1, nseq, max_q)
+                                             : nvs_ssd_scan_workspace(heads, P, N, nseq, max_q)),
+              "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   int ng = 1;
   while (ng * SSD_R < N) ng <<= 1;                  // a power of two: the threads of one p reduce by lane shuffles
   const int ng0 = ng;
@@ -803,14 +814,20 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
     while (pp > 1 && (P % pp != 0 || (P / pp) * ng0 > (pp == 4 ? 256 : 512))) pp >>= 1;
   }
   NVS_REQUIRE(ng <= 64 && (int64_t)((P + pp - 1) / pp) * ng <= 1024, "%s: state %d x head size %d exceeds one workgroup's registers", who, N, P);
+  ScanArgs ca = {form, xbc, proj, proj_stride, dt_col, x_col, b_col, c_col, ga.i_col, ga.f_col, decay, dt_bias, A_log, D, ga.i_bias, ga.f_bias,
+                 heads, P, N, G, cu_q, ctx0, slot, S, ga.M, y, ga.den, ws, ga.cap, ga.c_scale, 0, 1};
+  // State rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, which win at every length: 100 portions of
+  // 1 / 5 / 8 / 31 tokens, 64 heads of 64 x 128: 118 / 150 / 180 / 471 us here, 112 / 111 / 113 / 170 there. The constant decay
+  // stays here for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is 7.4e-8, not 8.3e-8.
+  if (scan_chunk_fits(ca, dtype) && (form != 1 || max_q >= 16)) {
+    if (ws) scan_chunk_plan(heads, P, nseq, max_q, &ca.seg_len, &ca.nseg);
+    return scan_chunk_launch(ca, dtype, nseq, stream);
+  }
   const int threads = ((P + pp - 1) / pp) * ng, per = (((P + pp - 1) / pp * pp + 3) & ~3) + 2 * ng * SSD_R + 4;
   const int tb = SSD_TB;                            // tokens per LDS round
   const size_t lds = (size_t)tb * per * sizeof(float);
   int seg_len = 0, nseg = 1;
-  if (ws) ssd_plan(heads, nseq, max_q > 0 ? max_q : n, &seg_len, &nseg, form == 2 ? 192 : 512);
-  NVS_REQUIRE(!seg_len || ws_floats >= (form == 2 ? nvs_gated_memory_scan_workspace(heads, N, P - 1, nseq, max_q > 0 ? max_q : n)
-                                                   : nvs_ssd_scan_workspace(heads, P, N, nseq, max_q > 0 ? max_q : n)),
-              "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
+  if (ws) ssd_plan(heads, nseq, max_q, &seg_len, &nseg, form == 2 ? 192 : 512);
   const dim3 grid(heads, (unsigned)nseq, seg_len ? nseg : 1);
 #define NVS_SSD_LAUNCH(PPV, MODE, FORM)                                                                                             \
   NVS_DISPATCH(dtype, ssd_scan_kernel<T, PPV, MODE, FORM><<<grid, dim3(threads), lds, (hipStream_t)stream>>>(                        \

@@ -1,0 +1,98 @@
+"""The matrix-state recurrences in chunks of 16 tokens on 32-bit matrix instructions (state sizes 64 and 128) against a token loop in
+float64: portions at the edges of a chunk and of the four chunks whose weights are computed together, rows that do not fill a
+wavefront or a workgroup, portions cut into segments, states kept from earlier calls, dirty slots."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+def _portions(lens, ctx, slots):
+    from nano_vllm_amd.ops_seq import Portions
+    i = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    p = Portions.__new__(Portions)
+    p.cu_q, p.ctx0, p.slot = i(cu), i(ctx), i(slots)
+    p.tseq = i([s for s, n in enumerate(lens) for _ in range(n)])
+    p.nseq, p.n, p.max_q = len(lens), cu[-1], max(lens)
+    return p
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("lens", [[1, 16, 17, 2], [63, 65, 15], [700, 20, 300]], ids=["short", "group", "segments"])
+@pytest.mark.parametrize("form,heads,P,N,G", [(0, 4, 64, 128, 2), (0, 3, 40, 64, 1), (0, 2, 100, 128, 2), (1, 3, 128, 128, 1), (1, 2, 16, 64, 1),
+                                              (2, 2, 128, 128, 1), (2, 3, 24, 64, 1), (2, 2, 72, 128, 1)])
+def test_chunked_recurrences_against_the_token_loop(form, heads, P, N, G, lens, dtype):
+    from nano_vllm_amd import ops_seq
+    g = torch.Generator(device="cuda").manual_seed(heads * P + N + form)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    n, nseq, F = sum(lens), len(lens), torch.float64
+    rows = P + 1 if form == 2 else P
+    ctx = [7 * (s % 2) for s in range(nseq)]                    # every other portion continues a sequence
+    slots = [nseq - s for s in range(nseq)]                     # slot 0 is nobody's
+    por = _portions(lens, ctx, slots)
+    S, M = rand(nseq + 1, heads, rows, N), rand(nseq + 1, heads).abs()
+    state = torch.stack([S[slots[s]].double() * (ctx[s] > 0) for s in range(nseq)])
+    mx = torch.stack([M[slots[s]].double() * (ctx[s] > 0) for s in range(nseq)])
+    S0, M0 = S[0].clone(), M[0].clone()
+    y, den = torch.empty(n, heads * P, device="cuda"), torch.empty(n, heads, device="cuda")
+    skip = torch.zeros(heads, device="cuda", dtype=dtype)
+    if form == 0:
+        xbc, proj = rand(n, heads * P + 2 * G * N), rand(n, heads + 5).to(dtype)
+        bias, A_log, skip = (rand(heads) - 2).to(dtype), rand(heads).to(dtype), rand(heads).to(dtype)
+        ops_seq.ssd_scan(xbc, proj, 3, bias, A_log, skip, heads, P, N, G, por, S, y)
+        x, B, C = xbc.double().split([heads * P, G * N, G * N], 1)
+        B, C = (t.reshape(n, G, N).repeat_interleave(heads // G, 1) for t in (B, C))
+        step = torch.nn.functional.softplus(proj[:, 3:3 + heads].double() + bias.double())
+        decay = torch.exp(-torch.exp(A_log.double()) * step)
+    else:
+        cols = [heads * P, heads * N, heads * N, 2 * heads]
+        proj = rand(n, (sum(cols) + 7) // 8 * 8).to(dtype)
+        x, B, C, gates = proj.double()[:, :sum(cols)].split(cols, 1)
+        B, C = B.reshape(n, heads, N), C.reshape(n, heads, N)
+    if form == 1:
+        rate = torch.exp(-torch.linspace(0.003, 2.0, heads, device="cuda"))
+        ops_seq.decay_scan(proj, 0, cols[0], cols[0] + cols[1], rate, heads, N, P, por, S, y)
+        x, B, C = (torch.nn.functional.silu(t) for t in (x, B, C))
+        step, decay = torch.ones(n, heads, dtype=F, device="cuda"), rate.double().expand(n, heads)
+    if form == 2:
+        ib, fb, at = rand(heads).to(dtype), (rand(heads) + 2).to(dtype), sum(cols[:3])
+        ops_seq.gated_memory_scan(proj, 0, cols[0], cols[0] + cols[1], at, at + heads, ib, fb, 15.0, N ** -0.5, heads, N, P, por, S, M, y, den)
+        C = C * N ** -0.5
+        ig = 15 * torch.tanh((gates[:, :heads] + ib.double()) / 15)
+        fg = torch.nn.functional.logsigmoid(15 * torch.tanh((gates[:, heads:] + fb.double()) / 15))
+    x = x.reshape(n, heads, P)
+    if form == 2:
+        x = torch.cat([x, torch.ones(n, heads, 1, dtype=F, device="cuda")], 2)
+    size = state.abs()                                          # the same recurrence on absolute values: what an error is measured by
+    at = 0
+    for s, ln in enumerate(lens):
+        for t in range(at, at + ln):
+            if form == 2:
+                m = torch.maximum(fg[t] + mx[s], ig[t])
+                a, w = torch.exp(fg[t] + mx[s] - m), torch.exp(ig[t] - m)
+                mx[s] = m
+            else:
+                a, w = decay[t], step[t]
+            new = (w[:, None] * x[t])[:, :, None] * B[t][:, None]
+            state[s] = a[:, None, None] * state[s] + new
+            size[s] = a[:, None, None] * size[s] + new.abs()
+            out, mag = (state[s] * C[t][:, None]).sum(2), (size[s] * C[t][:, None].abs()).sum(2)
+            # an entry is a sum over N products of state entries, each a sum over the tokens so far; one rounding per step, and a
+            # handful per term for its gate, its decay and the products
+            tol = (t - at + 1 + N + 32) * EPS
+            if form == 2:
+                q, lim = out[:, P], torch.exp(-mx[s])
+                want = torch.maximum(q.abs(), lim) + 1e-6
+                assert ((den[t] - want).abs() <= tol * (mag[:, P] + lim) + 4 * EPS * mx[s].abs() * lim).all(), (s, t - at)
+                out, mag = out[:, :P], mag[:, :P]
+            out, mag = out + skip.double()[:, None] * x[t][:, :P], mag + (skip.double()[:, None] * x[t][:, :P]).abs()
+            assert ((y[t].view(heads, P) - out).abs() <= tol * mag).all(), (s, t - at)
+        assert ((S[slots[s]] - state[s]).abs() <= (ln + 32) * EPS * size[s]).all(), s
+        if form == 2:
+            assert ((M[slots[s]] - mx[s]).abs() <= (ln + 4) * EPS * mx[s].abs().clamp(min=1)).all(), s
+        at += ln
+    assert torch.equal(S[0], S0) and torch.equal(M[0], M0)
