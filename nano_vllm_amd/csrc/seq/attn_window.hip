@@ -53,6 +53,75 @@ __global__ void knorm_kvstore_kernel(const T* __restrict__ k, const T* __restric
   for (int c = lane; c < dv; c += 64) vc[(int64_t)c * block_size] = vp[c];
 }
 
+// The same for long steps and heads of whole 16-byte units: a workgroup takes KV_TILE tokens of one head. What bounds it is the way
+// the values go: a token's dv values lie block_size entries apart in its page, so a wavefront per token writes 2 bytes per
+// memory transaction; through LDS the lanes run along the tile's tokens, neighbours in the page. Keys go a unit per lane, L lanes per token.
+// 13,550 tokens, 8 heads of 128 + 128, bf16: 78 -> 31 us, turned keys 87 -> 38 (111 MB: 23 us at the rate of a copy).
+constexpr int KV_TILE = 64;
+template <typename T>
+__global__ __launch_bounds__(256) void knorm_kvstore_tile_kernel(const T* __restrict__ k, const T* __restrict__ v, int64_t stride,
+                                                                 const T* __restrict__ knorm, float eps, int G, int d, int dv, int block_size,
+                                                                 const int32_t* __restrict__ slots, const int64_t* __restrict__ pos,
+                                                                 const float* __restrict__ rot_freq, int rot_dims, int64_t n, int L,
+                                                                 T* __restrict__ k_cache, T* __restrict__ v_cache) {
+  constexpr int VE = 16 / sizeof(T), LDT = KV_TILE + 4 / (int)sizeof(T);
+  extern __shared__ __attribute__((aligned(16))) char kv_lds[];
+  T* vt = (T*)kv_lds;                               // [dv][LDT]
+  __shared__ int where[KV_TILE];
+  const int64_t t0 = (int64_t)blockIdx.x * KV_TILE;
+  const int g = blockIdx.y, tid = threadIdx.x, nt = (int)(n - t0 < KV_TILE ? n - t0 : KV_TILE);
+  if (tid < nt) where[tid] = slots[t0 + tid];
+  const int units = dv / VE;
+  for (int u = tid; u < nt * units; u += 256) {
+    const int tt = u / units, c = (u - tt * units) * VE;
+    float x[VE];
+    ldp<VE>(v + (t0 + tt) * stride + (int64_t)g * dv + c, x);
+#pragma unroll
+    for (int e = 0; e < VE; ++e) stf(&vt[(c + e) * LDT + tt], x[e]);
+  }
+  const int l = tid & (L - 1), c0 = l * VE;
+  for (int tt = tid / L; tt < nt; tt += 256 / L) {  // (all lanes of a token together)
+    const int64_t t = t0 + tt, slot = slots[t];
+    float x[VE], w[VE], ss = 0.f;
+    if (c0 < d) {
+      ldp<VE>(k + t * stride + (int64_t)g * d + c0, x);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) ss += x[e] * x[e];
+    }
+    if (knorm) {
+      for (int o = L >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float r = rsqrtf(ss / (float)d + eps);
+      if (c0 < d) {
+        ldp<VE>(knorm + c0, w);
+#pragma unroll
+        for (int e = 0; e < VE; ++e) x[e] = x[e] * r * w[e];
+      }
+    }
+    if (slot < 0 || c0 >= d) continue;
+    if (c0 < rot_dims) {
+      const float pf = (float)pos[t];
+#pragma unroll
+      for (int e = 0; e < VE; e += 2) {
+        if (c0 + e >= rot_dims) break;
+        float sn, cs;
+        sincosf(pf * rot_freq[(c0 + e) >> 1], &sn, &cs);
+        const float a = x[e], b = x[e + 1];
+        x[e] = a * cs - b * sn, x[e + 1] = b * cs + a * sn;
+      }
+    }
+    stp<VE>(k_cache + (slot * G + g) * d + c0, x);
+  }
+  __syncthreads();
+  for (int u = tid; u < dv * KV_TILE; u += 256) {
+    const int tt = u % KV_TILE, c = u / KV_TILE;
+    if (tt >= nt) continue;
+    const int slot = where[tt];
+    if (slot < 0) continue;
+    const int page = slot / block_size, off = slot - page * block_size;
+    v_cache[(((int64_t)page * G + g) * dv + c) * block_size + off] = vt[c * LDT + tt];
+  }
+}
+
 // one wavefront per (token, query head). Keys go in rounds of 64 (one per lane): score, running maximum, weights into LDS,
 // then every lane accumulates its value columns over the round's keys. Pooled blocks are keys like any other, in rounds of their own.
 template <typename T, int CH>
@@ -183,6 +252,20 @@ extern "C" int nvs_knorm_kvstore(const void* k, const void* v, int64_t stride, i
   NVS_REQUIRE(G > 0 && G <= 65535 && d > 0 && d <= MAX_HEAD && dv > 0 && dv <= MAX_HEAD && n >= 0 && block_size > 0,
               "nvs_knorm_kvstore: G %d d %d dv %d", G, d, dv);
   if (n == 0) return NVS_OK;
+  // A tile per workgroup where there are workgroups enough: 8 heads of 128 + 128, 512 / 1,024 / 2,048 / 4,096 tokens, 32-bit: 15 / 17 / 24 / 46 us
+  // by wavefronts, 18 / 19 / 21 / 26 by tiles; bf16 15 / 15 / 19 / 30, 14 / 14 / 14 / 17
+  const int ve = dtype == NVS_BF16 ? 8 : 4;
+  const uintptr_t al = (uintptr_t)k | (uintptr_t)v | (uintptr_t)knorm | (uintptr_t)k_cache;
+  if (n >= 2048 && d % ve == 0 && dv % ve == 0 && d <= 256 && dv <= 256 && stride % ve == 0 && al % 16 == 0) {
+    int L = 1;
+    while (L * ve < d) L *= 2;
+    const dim3 grid((unsigned)((n + KV_TILE - 1) / KV_TILE), G);
+    NVS_DISPATCH(dtype, knorm_kvstore_tile_kernel<T><<<grid, dim3(256), (size_t)dv * (KV_TILE + 4 / (int)sizeof(T)) * sizeof(T),
+                                                       (hipStream_t)stream>>>(
+                            (const T*)k, (const T*)v, stride, (const T*)knorm, eps, G, d, dv, block_size, slots, pos, rot_freq, rot_dims, n, L,
+                            (T*)k_cache, (T*)v_cache));
+    return nvs_check_launch("nvs_knorm_kvstore (tiles)");
+  }
   if (d <= 256 && dv <= 256)
     NVS_DISPATCH(dtype, knorm_kvstore_kernel<T, 4><<<dim3((unsigned)n, G), dim3(64), 0, (hipStream_t)stream>>>(
                             (const T*)k, (const T*)v, stride, (const T*)knorm, eps, G, d, dv, block_size, slots, pos, rot_freq, rot_dims,
