@@ -185,9 +185,9 @@ __global__ void add_group_norm_kernel(float* __restrict__ x, const T* __restrict
   }
 }
 
-// The same for ONE group without centering, four columns per access: the row stays in registers between the two passes
-// (PER accesses per thread).
-template <typename T, int PER>
+// The same for ONE group, four columns per access: the row stays in registers between the passes (PER accesses per thread). Centered,
+// 13,550 rows of 1,024 (bf16 input and output): 50 us a column at a time with the row read back, 29 here (4,096: 247, 130).
+template <typename T, int PER, bool CENTER>
 __global__ __launch_bounds__(256) void add_norm_row_kernel(float* __restrict__ x, const T* __restrict__ a, float a_mult, const float* __restrict__ b,
                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, int width, float eps,
                                                            T* __restrict__ out) {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void add_norm_row_kernel(float* __restrict__ x
   const int64_t t = rows ? (int64_t)rows[r] : r;
   float* xr = x + t * width;
   float v[PER][4];
-  float ss = 0.f;
+  float ss = 0.f, sm = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = (i * blockDim.x + threadIdx.x) * 4;
@@ -215,9 +215,18 @@ __global__ __launch_bounds__(256) void add_norm_row_kernel(float* __restrict__ x
     }
     if (a || b) stv<4>(xr + c, v[i]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) ss += v[i][e] * v[i][e];
+    for (int e = 0; e < 4; ++e) CENTER ? sm += v[i][e] : ss += v[i][e] * v[i][e];
   }
   if (!out) return;
+  if (CENTER) {                                     // the mean first, then the squared deviations
+    const float mean = block_sum(sm, red) / (float)width;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if ((i * blockDim.x + threadIdx.x) * 4 >= width) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] -= mean, ss += v[i][e] * v[i][e];
+    }
+  }
   const float k = w ? 1.f / sqrtf(block_sum(ss, red) / (float)width + eps) : 1.f;      // (no weights: the sum itself)
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -633,10 +642,12 @@ extern "C" int nvs_add_group_norm(float* x, const void* a, float a_mult, const f
   if (nrows == 0) return NVS_OK;
   const uintptr_t al = (uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)w | (uintptr_t)out;
   int row_threads = 0;
-  const int per = groups == 1 && !center ? row_plan(width, al, &row_threads) : 0;
+  const int per = groups == 1 ? row_plan(width, al, &row_threads) : 0;
   if (per) {
 #define NVS_ROW(PER)                                                                                                           \
-  NVS_DISPATCH(dtype, add_norm_row_kernel<T, PER><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>(         \
+  NVS_DISPATCH(dtype, if (center) add_norm_row_kernel<T, PER, true><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
+                          x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out);                                     \
+                      else add_norm_row_kernel<T, PER, false><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
                           x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out))
     NVS_ROW_CASES(per, NVS_ROW)
 #undef NVS_ROW
