@@ -253,6 +253,11 @@ int nvs_moe_table_route(const int64_t* tokens, const int32_t* table, int64_t n, 
 int64_t nvs_moe_rows(int64_t pairs, int experts, int tm);
 int nvs_moe_plan(const int32_t* ids, int64_t n, int top, int experts, int tm, int32_t* tile_expert, int32_t* row_token, int32_t* pair_row,
                  void* stream);
+/* The same, by many workgroups where the step is long enough for it to pay: scratch of nvs_moe_plan_scratch(n * top, experts) entries (0: one
+ * workgroup is as fast, scratch may be NULL). Which of an expert's rows a pair gets is not specified. */
+int64_t nvs_moe_plan_scratch(int64_t pairs, int experts);
+int nvs_moe_plan_wide(const int32_t* ids, int64_t n, int top, int experts, int tm, int32_t* tile_expert, int32_t* row_token, int32_t* pair_row,
+                      int32_t* scratch, int64_t scratch_ints, void* stream);
 
 /* Grouped product over the planned rows: out[r, :] = W[expert of r] x(r). mode 1: W [experts, 2 nout, K] (gate rows, then up rows),
  * x(r) = X[row_token[r], :], out = silu(gate) * up; mode 0: W [experts, nout, K], x(r) = X[r, :]; mode 2: W [experts, nout, K],

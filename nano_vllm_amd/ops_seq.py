@@ -58,7 +58,8 @@ SIGNATURES = {
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
     "nvs_moe_route": (c_int, [_P, _L, _P, _L, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P]),
     "nvs_moe_rows": (c_int64, [_L, _I, _I]),
-    "nvs_moe_plan": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P]),
+    "nvs_moe_plan_scratch": (c_int64, [_L, _I]),
+    "nvs_moe_plan_wide": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P, _L, _P]),
     "nvs_moe_gemm": (c_int, [_P, _L, _P, _I, _I, _I, _I, _P, _P, _L, _I, _P, _L, _P]),
     "nvs_moe_force_plain": (None, [_I]),
     "nvs_moe_combine": (c_int, [_P, _L, _P, _P, _I, _P, _L, _P, _P, _L, _I, _L, _I, _P, _P, _P]),
@@ -634,7 +635,10 @@ def moe_plan(ids: torch.Tensor, experts: int, tm: int) -> MoePlan:
     p.tile_expert = torch.empty(p.cap // tm, dtype=torch.int32, device=ids.device)
     p.row_token = torch.empty(p.cap, dtype=torch.int32, device=ids.device)
     p.pair_row = torch.empty(n, top, dtype=torch.int32, device=ids.device)
-    _check(lib.nvs_moe_plan(_ptr(ids), n, top, experts, tm, _ptr(p.tile_expert), _ptr(p.row_token), _ptr(p.pair_row), _stream()))
+    need = lib.nvs_moe_plan_scratch(n * top, experts)
+    scratch = torch.empty(need, dtype=torch.int32, device=ids.device) if need else None
+    _check(lib.nvs_moe_plan_wide(_ptr(ids), n, top, experts, tm, _ptr(p.tile_expert), _ptr(p.row_token), _ptr(p.pair_row), _ptr(scratch),
+                                 need, _stream()))
     return p
 
 
