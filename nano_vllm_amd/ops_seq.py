@@ -8,6 +8,7 @@ stream are float32. The library is built on first use when it is missing (a fres
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 
@@ -100,7 +101,19 @@ def _check(rc: int) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # (the handle alone: building a Stream object around it took 6 of a launch's 25 us on the host)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def _launch(fn):
+    """For functions that only look at their tensors (pointers, shapes, strides), allocate on a named device and launch. With a default
+    device set, torch passes every method and attribute of a tensor through Python first, about 1 us each, 20 to 30 of them per
+    launch: a step of 82 launches in 32-bit took 2.55 ms on the host around 1.4 ms of kernels, 1.45 without that."""
+    @functools.wraps(fn)
+    def run(*args, **kwargs):
+        with torch._C.DisableTorchFunction():
+            return fn(*args, **kwargs)
+    return run
 
 
 def _code(t: torch.Tensor) -> int:
@@ -139,6 +152,7 @@ class Portions:
         assert cu_q.numel() >= nseq + 1 and ctx0.numel() >= nseq and slot.numel() >= nseq and tseq.numel() >= n
 
 
+@_launch
 def embed_sinusoid(table, ids, pos, scale: float, base: float, x: torch.Tensor, xh: torch.Tensor | None):
     lib = load_library()
     n, width = ids.numel(), table.shape[1]
@@ -149,6 +163,7 @@ def embed_sinusoid(table, ids, pos, scale: float, base: float, x: torch.Tensor, 
                                   _ptr(xh), _stream()))
 
 
+@_launch
 def norm_residual(x: torch.Tensor, m: torch.Tensor, g: torch.Tensor, eps: float, xh: torch.Tensor | None,
                   m2: torch.Tensor | None = None, w1: torch.Tensor | None = None, w2: torch.Tensor | None = None):
     """x += g * rms(m), or with a second branch x += g * rms((rms(m) w1 + rms(m2) w2) / 2)."""
@@ -161,6 +176,7 @@ def norm_residual(x: torch.Tensor, m: torch.Tensor, g: torch.Tensor, eps: float,
                                  _ptr(x), _ptr(xh), _stream()))
 
 
+@_launch
 def scalar_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, g: torch.Tensor, eps: float, out: torch.Tensor):
     lib = load_library()
     assert x.dtype == torch.float32 and x.is_contiguous() and out.is_contiguous() and out.shape == (nrows, x.shape[1])
@@ -169,6 +185,7 @@ def scalar_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, g: 
     _check(lib.nvs_scalar_norm_rows(_ptr(x), _ptr(rows), nrows, x.shape[1], _ptr(g), _same(out, g), eps, _ptr(out), _stream()))
 
 
+@_launch
 def xielu(z: torch.Tensor, pq: torch.Tensor, beta: float = 0.5) -> torch.Tensor:
     """In place."""
     lib = load_library()
@@ -177,6 +194,7 @@ def xielu(z: torch.Tensor, pq: torch.Tensor, beta: float = 0.5) -> torch.Tensor:
     return z
 
 
+@_launch
 def causal_conv(inp: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act: int, por: Portions, state: torch.Tensor,
                 out: torch.Tensor):
     """inp: [n, channels] view (unit column stride) of a projection output; state [nslots, taps - 1, channels] fp32; out 32-bit or
@@ -190,6 +208,7 @@ def causal_conv(inp: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
                                _ptr(por.ctx0), _ptr(por.slot), _ptr(por.tseq), por.nseq, por.n, _ptr(state), _ptr(out), _code(out), _stream()))
 
 
+@_launch
 def rglru_scan(gates: torch.Tensor, u: torch.Tensor, ypre: torch.Tensor, lam: torch.Tensor, c: float, blocks: int, por: Portions,
                S: torch.Tensor, out: torch.Tensor):
     lib = load_library()
@@ -206,6 +225,7 @@ def rglru_scan(gates: torch.Tensor, u: torch.Tensor, ypre: torch.Tensor, lam: to
                               _stream()))
 
 
+@_launch
 def ssd_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias, A_log, D, heads: int, P: int, N: int, G: int,
              por: Portions, S: torch.Tensor, y: torch.Tensor):
     lib = load_library()
@@ -223,6 +243,7 @@ def ssd_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias, A_log,
                             por.max_q, _ptr(S), _ptr(y), _ptr(ws), need, _stream()))
 
 
+@_launch
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, w: torch.Tensor, groups: int, eps: float, out: torch.Tensor,
                      norm_first: bool = False, den: torch.Tensor | None = None, silu: bool = False):
     """out = group_rms(y * silu(z)) * w, or with norm_first group_rms(y) * w * sigmoid(z) (silu: * silu(z)); den [n, groups] (32-bit,
@@ -245,6 +266,7 @@ def _rotation(rot_freq: torch.Tensor | None) -> int:
     return 2 * rot_freq.numel()
 
 
+@_launch
 def knorm_kvstore(k: torch.Tensor, v: torch.Tensor, knorm: torch.Tensor | None, eps: float, G: int, d: int, dv: int,
                   block_size: int, slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                   pos: torch.Tensor | None = None, rot_freq: torch.Tensor | None = None):
@@ -263,6 +285,7 @@ def knorm_kvstore(k: torch.Tensor, v: torch.Tensor, knorm: torch.Tensor | None, 
                                  _rotation(rot_freq), n, _ptr(k_cache), _ptr(v_cache), _stream()))
 
 
+@_launch
 def qkv_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, H: int, G: int, d: int, dv: int, block_size: int, slots: torch.Tensor, k_cache,
               v_cache, pos: torch.Tensor | None, rot: "Rotation | None", unit: bool, eps: float, q_scale: float,
               first: torch.Tensor | None = None, mix: torch.Tensor | None = None):
@@ -283,6 +306,7 @@ def qkv_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, H: int, G: int,
                              _ptr(mix) if first is not None else None, block_size, _ptr(slots), n, _ptr(k_cache), _ptr(v_cache), _stream()))
 
 
+@_launch
 def window_attn(q: torch.Tensor, qnorm: torch.Tensor | None, eps: float, gate: torch.Tensor | None, k_cache, v_cache,
                 block_tables: torch.Tensor, block_size: int, por: Portions, H: int, G: int, d: int, dv: int, scale: float,
                 window: int, out: torch.Tensor, chunk: int = 0, rot_freq: torch.Tensor | None = None, gate_per_head: bool = False,
@@ -312,6 +336,7 @@ def window_attn(q: torch.Tensor, qnorm: torch.Tensor | None, eps: float, gate: t
                                _ptr(sink), qt_coef, qt_every, _ptr(out), _stream()))
 
 
+@_launch
 def qk_rows(q: torch.Tensor, k: torch.Tensor | None, v: torch.Tensor | None, knorm: torch.Tensor | None, eps: float, G: int, d: int, dv: int,
             block_size: int, slots: torch.Tensor, k_cache, v_cache, pos: torch.Tensor, rot_freq: torch.Tensor | None, por: Portions,
             block_tables: torch.Tensor, pool: int = 0, pool_k: torch.Tensor | None = None, pool_v: torch.Tensor | None = None) -> torch.Tensor:
@@ -340,6 +365,7 @@ def pool_rows(block_size: int, pool: int) -> int:
     return -(-block_size // (8 * pool)) * 8
 
 
+@_launch
 def pool_blocks(k_cache, v_cache, G: int, d: int, dv: int, block_size: int, pool: int, slots: torch.Tensor, pos: torch.Tensor,
                 block_tables: torch.Tensor, por: Portions, pool_k: torch.Tensor, pool_v: torch.Tensor):
     """Means of the cached keys / values over the blocks of `pool` positions that end in this step."""
@@ -352,6 +378,7 @@ def pool_blocks(k_cache, v_cache, G: int, d: int, dv: int, block_size: int, pool
                                _stream()))
 
 
+@_launch
 def embed_norm(table: torch.Tensor, ids: torch.Tensor, w: torch.Tensor, eps: float, x: torch.Tensor):
     """x (32-bit) = rms(table[ids]) * w."""
     lib = load_library()
@@ -360,6 +387,7 @@ def embed_norm(table: torch.Tensor, ids: torch.Tensor, w: torch.Tensor, eps: flo
     _check(lib.nvs_embed_norm(_ptr(table), _same(table, w), _ptr(ids), n, width, _ptr(w), eps, _ptr(x), _stream()))
 
 
+@_launch
 def shift_norm(x: torch.Tensor, a: torch.Tensor | None, wa: torch.Tensor | None, w: torch.Tensor, mu: torch.Tensor, eps: float, por: Portions,
                state: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """y = x + a (wa None) or x + rms(a) * wa; h = rms(y) * w; out = h + (h of the previous token - h) * mu, with the last h of every
@@ -376,6 +404,7 @@ def shift_norm(x: torch.Tensor, a: torch.Tensor | None, wa: torch.Tensor | None,
     return y
 
 
+@_launch
 def gated_lookup(z: torch.Tensor, table: torch.Tensor, col0: int, ids: torch.Tensor) -> torch.Tensor:
     """gelu_tanh(z) * table[ids, col0 : col0 + dim], z [n, dim]."""
     lib = load_library()
@@ -386,6 +415,7 @@ def gated_lookup(z: torch.Tensor, table: torch.Tensor, col0: int, ids: torch.Ten
     return out
 
 
+@_launch
 def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, b_col: int, a_col: int, decays: torch.Tensor | None, A_log: torch.Tensor,
                dt_bias: torch.Tensor, q_scale: float, heads: int, G: int, dk: int, dv: int, por: Portions, S: torch.Tensor, y: torch.Tensor):
     """The gated delta rule (see include/nvl_seq.h) on qkv [n, 2 G dk + heads dv]; beta from columns b_col of `gates`; one decay per head
@@ -404,6 +434,7 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, b_col: int, a_col: int, d
                               _ptr(S), _ptr(y), _stream()))
 
 
+@_launch
 def add_group_norm(x: torch.Tensor, w: torch.Tensor | None, groups: int, eps: float, out: torch.Tensor | None,
                    a: torch.Tensor | None = None, b: torch.Tensor | None = None, a_mult: float = 1.0, center: bool = False):
     """x += a_mult * a + b (in place; a in the activation type, b 32-bit, both optional), then out = group_rms(x) * w (out None:
@@ -420,6 +451,7 @@ def add_group_norm(x: torch.Tensor, w: torch.Tensor | None, groups: int, eps: fl
                                   width, groups, eps, int(center), _ptr(out), _stream()))
 
 
+@_launch
 def group_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, w: torch.Tensor, groups: int, eps: float, out: torch.Tensor,
                     center: bool = False):
     """out[r] = group_rms(x[rows[r]]) * w (rows None: row r); center: as add_group_norm."""
@@ -431,6 +463,7 @@ def group_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, w: t
                                   _ptr(out), _stream()))
 
 
+@_launch
 def sandwich_norm(x: torch.Tensor, a: torch.Tensor | None, wa: torch.Tensor | None, w: torch.Tensor | None, eps: float,
                   out: torch.Tensor | None, a2: torch.Tensor | None = None, a_mult: float = 1.0, a2_mult: float = 1.0, w_off: float = 1.0):
     """x += rms(a_mult * a + a2_mult * a2) * (w_off + wa) (in place; a None: no add), then out = rms(x) * (w_off + w) (out None: no
@@ -448,6 +481,7 @@ def sandwich_norm(x: torch.Tensor, a: torch.Tensor | None, wa: torch.Tensor | No
                                                                                    w if out is not None else None, out), width, eps, None, _ptr(out), _stream()))
 
 
+@_launch
 def offset_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, w: torch.Tensor, eps: float, out: torch.Tensor, w_off: float = 1.0,
                      a: torch.Tensor | None = None, wa: torch.Tensor | None = None):
     """out[r] = rms(x[rows[r]]) * (w_off + w) (rows None: row r); with a and wa: of x[rows[r]] + rms(a[rows[r]]) * (w_off + wa) (x stays)."""
@@ -461,6 +495,7 @@ def offset_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, w: 
                                  eps, _ptr(sums), _ptr(out), _stream()))
 
 
+@_launch
 def branch_norm(x: torch.Tensor, a: torch.Tensor | None, w: torch.Tensor, ls: torch.Tensor | None, eps: float, out: torch.Tensor | None,
                 chosen: "tuple | None" = None):
     """x += rms(y) * w * ls (in place; ls None: no scale), y = a (may be None) + with chosen = (rows, plan, weights) of a routed layer the
@@ -480,6 +515,7 @@ def branch_norm(x: torch.Tensor, a: torch.Tensor | None, w: torch.Tensor, ls: to
                                _ptr(wts), top, _same(w, a, rows, ls, out), n, _ptr(w), _ptr(ls), width, eps, _ptr(out), _stream()))
 
 
+@_launch
 def gated_memory_scan(proj: torch.Tensor, v_col: int, k_col: int, q_col: int, i_col: int, f_col: int, i_bias: torch.Tensor,
                       f_bias: torch.Tensor, cap: float, q_scale: float, heads: int, dk: int, dv: int, por: Portions, S: torch.Tensor,
                       M: torch.Tensor, y: torch.Tensor, den: torch.Tensor):
@@ -499,6 +535,7 @@ def gated_memory_scan(proj: torch.Tensor, v_col: int, k_col: int, q_col: int, i_
                                      por.max_q, _ptr(S), _ptr(M), _ptr(y), _ptr(den), _ptr(ws), need, _stream()))
 
 
+@_launch
 def scale_softcap(logits: torch.Tensor, scale: float, cap: float) -> torch.Tensor:
     """32-bit cap * tanh(logits * scale / cap) (cap <= 0: logits * scale)."""
     lib = load_library()
@@ -518,6 +555,7 @@ class Rotation:
         self.freq, self.dims, self.halves, self.mag = freq, 2 * freq.numel(), bool(halves), float(mag)
 
 
+@_launch
 def latent_prep(proj: torch.Tensor, q_col: int, q_rank: int, q_norm: torch.Tensor, cq: torch.Tensor, eps: float, kv_col: int = -1,
                 kv_rank: int = 0, rot_dim: int = 0, kv_norm: torch.Tensor | None = None, pos: torch.Tensor | None = None,
                 rot: Rotation | None = None, block_size: int = 0, slots: torch.Tensor | None = None, k_cache: torch.Tensor | None = None,
@@ -540,6 +578,7 @@ def latent_prep(proj: torch.Tensor, q_col: int, q_rank: int, q_norm: torch.Tenso
                                _ptr(k_cache), _ptr(v_cache), n, _stream()))
 
 
+@_launch
 def rotate_heads(inp: torch.Tensor, out: torch.Tensor, pos: torch.Tensor, rot: Rotation | None):
     """inp, out [n, H, width] views (unit stride along the last axis): out = inp with the leading rot.dims entries of every head rotated."""
     lib = load_library()
@@ -551,6 +590,7 @@ def rotate_heads(inp: torch.Tensor, out: torch.Tensor, pos: torch.Tensor, rot: R
                                 rot.mag if rot else 1.0, n, _stream()))
 
 
+@_launch
 def decay_scan(proj: torch.Tensor, v_col: int, k_col: int, q_col: int, decay: torch.Tensor, heads: int, dk: int, dv: int,
                por: Portions, S: torch.Tensor, y: torch.Tensor):
     """Per head S = decay S + k v^T, y = S^T q on SiLU of the named columns of proj; S [nslots, heads, dv, dk], y [n, heads * dv]."""
@@ -566,6 +606,7 @@ def decay_scan(proj: torch.Tensor, v_col: int, k_col: int, q_col: int, decay: to
                               _ptr(por.ctx0), _ptr(por.slot), por.nseq, n, por.max_q, _ptr(S), _ptr(y), _ptr(ws), need, _stream()))
 
 
+@_launch
 def glu_act(gu: torch.Tensor, ff: int, out: torch.Tensor, kind: int = 0, limit: float = 0.0, alpha: float = 1.0):
     """gu [n, 2 ff] = [gate | up] -> out [n, ff]. kind 0: silu(g) u; kind 1: min(g, limit) sigmoid(alpha g) (clamp(u) + 1);
     kind 2: gu [n, ff], no gate: the tanh form of GELU."""
@@ -575,6 +616,7 @@ def glu_act(gu: torch.Tensor, ff: int, out: torch.Tensor, kind: int = 0, limit: 
     _check(lib.nvs_glu_act(_ptr(gu), gu.stride(0), _same(gu, out), ff, kind, limit, alpha, n, _ptr(out), _stream()))
 
 
+@_launch
 def moe_route(z: torch.Tensor, total: int, correction: torch.Tensor | None, top: int, count: int, keep: int, scale: float,
               sigmoid: bool = False, renorm: bool = True):
     """z [n, >= total] 32-bit router logits -> (ids [n, top] int32, weights [n, top] 32-bit). Scores are a softmax over the entries,
@@ -590,6 +632,7 @@ def moe_route(z: torch.Tensor, total: int, correction: torch.Tensor | None, top:
     return ids, wts
 
 
+@_launch
 def moe_table_route(tokens: torch.Tensor, table: torch.Tensor, weight: float):
     """tokens [n] int64, table [vocab, top] int32 -> (ids [n, top] = table[tokens], weights [n, top] = weight)."""
     lib = load_library()
@@ -625,6 +668,7 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     return 256 if per >= 448 else 128 if per >= 64 else 64 if per >= 24 else 16
 
 
+@_launch
 def moe_plan(ids: torch.Tensor, experts: int, tm: int) -> MoePlan:
     """Pairs (token, choice) sorted by expert into tiles of tm rows (ids >= experts get no row)."""
     lib = load_library()
@@ -642,6 +686,7 @@ def moe_plan(ids: torch.Tensor, experts: int, tm: int) -> MoePlan:
     return p
 
 
+@_launch
 def moe_gemm(x: torch.Tensor, w: torch.Tensor, plan: MoePlan, glu: bool, out: torch.Tensor, relu2: bool = False):
     """glu: w [experts, 2 nout, K], rows gathered by token, out = silu(gate) * up; relu2: w [experts, nout, K], rows gathered by
     token, out = max(w x, 0)^2; neither: w [experts, nout, K], x holds the planned rows."""
@@ -654,6 +699,7 @@ def moe_gemm(x: torch.Tensor, w: torch.Tensor, plan: MoePlan, glu: bool, out: to
                             plan.cap, plan.tm, _ptr(out), out.stride(0), _stream()))
 
 
+@_launch
 def moe_combine(rows: torch.Tensor, plan: MoePlan, wts: torch.Tensor, h: torch.Tensor, shared: torch.Tensor | None,
                 shared_gate: torch.Tensor | None, out: torch.Tensor | None, res: torch.Tensor | None = None):
     """out[t] = sum_k wts[t, k] * (row of the pair, or h[t] for a pass-through choice) + sigmoid(shared_gate[t]) * shared[t]. With res
