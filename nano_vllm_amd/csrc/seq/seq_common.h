@@ -109,6 +109,29 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// e^x from the hardware's 2^x of a fraction in [-1/2, 1/2], to a unit in the last place; x is taken as no less than -100 and no more than 88
+__device__ __forceinline__ float exp_hw(float x) {
+  const float c = fminf(fmaxf(x, -100.f), 88.f), hi = c * 1.44269504088896341f, n = rintf(hi);
+  const float lo = fmaf(c, 1.44269504088896341f, -hi) + c * 1.92596299112661747e-8f;
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
+}
+// 1 / (1 + e^-x), the reciprocal with one step of Newton
+__device__ __forceinline__ float sigmoid_hw(float x) {
+  const float d = 1.f + exp_hw(-x), r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
+}
+// (e^x - 1 - x) / x^2 for x in [-1, 0]: the Taylor polynomial
+__device__ __forceinline__ float expm1_tail(float x) {
+  float p = 2.50521083854417188e-8f;                // 1 / 11!, 1 / 10!, ..., 1 / 2!
+  p = fmaf(p, x, 2.75573192239858907e-7f), p = fmaf(p, x, 2.75573192239858907e-6f), p = fmaf(p, x, 2.48015873015873016e-5f);
+  p = fmaf(p, x, 1.98412698412698413e-4f), p = fmaf(p, x, 1.38888888888888889e-3f), p = fmaf(p, x, 8.33333333333333333e-3f);
+  p = fmaf(p, x, 4.16666666666666667e-2f), p = fmaf(p, x, 1.66666666666666667e-1f), p = fmaf(p, x, 0.5f);
+  return p;
+}
+// e^x - 1 - x for x <= 0, and 1 - e^x, both without the cancellation near 0
+__device__ __forceinline__ float expm1_less_x(float x) { return x > -1.f ? expm1_tail(x) * x * x : exp_hw(x) - 1.f - x; }
+__device__ __forceinline__ float one_less_exp(float x) { return x > -1.f ? -fmaf(expm1_tail(x) * x, x, x) : 1.f - exp_hw(x); }
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float siluf_(float x) { return x / (1.f + expf(-x)); }
