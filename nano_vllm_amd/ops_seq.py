@@ -59,6 +59,7 @@ SIGNATURES = {
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
     "nvs_moe_route": (c_int, [_P, _L, _P, _L, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P]),
     "nvs_moe_rows": (c_int64, [_L, _I, _I]),
+    "nvs_moe_plan": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P]),
     "nvs_moe_plan_scratch": (c_int64, [_L, _I]),
     "nvs_moe_plan_wide": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P, _L, _P]),
     "nvs_moe_gemm": (c_int, [_P, _L, _P, _I, _I, _I, _I, _P, _P, _L, _I, _P, _L, _P]),
