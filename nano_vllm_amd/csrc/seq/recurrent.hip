@@ -861,9 +861,8 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
               "%s: heads %d groups %d head size %d state %d", who, heads, G, P, N);
   if (n == 0 || nseq == 0) return NVS_OK;
   if (max_q <= 0) max_q = n;
-  NVS_REQUIRE(!ws || ws_floats >= (form == 2 ? nvs_gated_memory_scan_workspace(heads, N, P - 1, nseq, max_q)
-                                             : nvs_ssd_scan_workspace(heads, P, N, nseq, max_q)),
-              "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
+  // what `n` segments of a plan take (a state and one number per segment and head, form 2 two more)
+  auto need = [&](int segs) { return (int64_t)nseq * heads * (segs + 1) * ((int64_t)P * N + (form == 2 ? 3 : 1)); };
   int ng = 1;
   while (ng * SSD_R < N) ng <<= 1;                  // a power of two: the threads of one p reduce by lane shuffles
   const int ng0 = ng;
@@ -886,6 +885,7 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   // stays here for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is 7.4e-8, not 8.3e-8.
   if (scan_chunk_fits(ca, dtype) && (form != 1 || max_q >= 16)) {
     if (ws) scan_chunk_plan(heads, P, nseq, max_q, &ca.seg_len, &ca.nseg);
+    if (ca.seg_len && ws_floats < need(ca.nseg)) ca.seg_len = 0, ca.nseg = 1;
     return scan_chunk_launch(ca, dtype, nseq, stream);
   }
   const int threads = ((P + pp - 1) / pp) * ng, per = (((P + pp - 1) / pp * pp + 3) & ~3) + 2 * ng * SSD_R + 4;
@@ -893,6 +893,7 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   const size_t lds = (size_t)tb * per * sizeof(float);
   int seg_len = 0, nseg = 1;
   if (ws) ssd_plan(heads, nseq, max_q, &seg_len, &nseg, form == 2 ? 192 : 512);
+  NVS_REQUIRE(!seg_len || ws_floats >= need(nseg), "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   const dim3 grid(heads, (unsigned)nseq, seg_len ? nseg : 1);
 #define NVS_SSD_LAUNCH(PPV, MODE, FORM)                                                                                             \
   NVS_DISPATCH(dtype, ssd_scan_kernel<T, PPV, MODE, FORM><<<grid, dim3(threads), lds, (hipStream_t)stream>>>(                        \

@@ -11,7 +11,8 @@ namespace {
 // products (P x 16 x N). All on v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit ones. The exponents are differences of
 // 64-bit sums, so a pair's weight is as exact as its own exponent however strongly the chunk decays as a whole. Form 2 has
 // exp(F_i - F_j + i_j - m_i) in place of exp(L_i - L_j) w_j and exp(F_i + m_before - m_i) in place of exp(L_i), m the running maximum.
-// A short last chunk is filled with tokens that change nothing (B = C = x = 0, no decay, no step).
+// A short last chunk is filled with tokens that change nothing (B = C = x = 0, no decay, no step). (Tokens of a chunk meet in products
+// whose weight above the diagonal is zero, so an infinity in one reaches the outputs of the up to 15 before it, never another portion's.)
 //
 // A workgroup takes NW * 16 rows p of one (portion, head)'s state, a wavefront 16 of them: its N / 16 accumulator tiles hold
 // S[n = 16 t + 4 (lane / 16) + r][p = lane % 16], which IS the operand layout of C S^T if the four tokens' entries of a product
