@@ -110,11 +110,12 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 }
 
 // e^x from the hardware's 2^x of a fraction in [-1/2, 1/2], to a unit in the last place; x is taken as no less than -100 and no more than 88
-// (by comparisons that a NaN fails: fmaxf would make it -100)
+// (by comparisons that a NaN fails: fmaxf would make it -100). The fraction is taken off in one fused step: x log2 e rounded first, and what
+// rounding took added back, is what the compiler's own fusing of that difference adds twice (27 x 2^-24 at e^28).
 __device__ __forceinline__ float exp_hw(float x) {
-  const float c = x < -100.f ? -100.f : x > 88.f ? 88.f : x, hi = c * 1.44269504088896341f, n = rintf(hi);
-  const float lo = fmaf(c, 1.44269504088896341f, -hi) + c * 1.92596299112661747e-8f;
-  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
+  const float c = x < -100.f ? -100.f : x > 88.f ? 88.f : x, n = rintf(c * 1.44269504088896341f);
+  const float f = fmaf(c, 1.92596299112661747e-8f, fmaf(c, 1.44269504088896341f, -n));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
 }
 // 1 / (1 + e^-x), the reciprocal with one step of Newton
 __device__ __forceinline__ float sigmoid_hw(float x) {
