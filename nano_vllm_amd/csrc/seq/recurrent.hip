@@ -164,13 +164,13 @@ __global__ void conv_state_kernel(const T* __restrict__ in, int64_t in_stride, i
 // ---- real-gated linear recurrence ---------------------------------------------------------------------------------
 // One thread per (portion, channel), sequential over the portion's tokens. What bounds it is the arithmetic
 // of the gates (four exponentials, two reciprocals and a root per token) behind few wavefronts: the library's divisions, roots and expm1 give way
-// to the hardware's with a correction, and eight tokens' operands are in flight. 14,230 tokens of 4,096 channels in nine portions:
-// 618 -> 495 us; states' error against 64 bits 1.5e-7 before and now. Long portions of a step with few (portion, channel) threads are cut
+// to the hardware's with a correction, and eight tokens' operands are in flight. Nine portions of 1,500 tokens, 4,096 channels: 500 ->
+// 385 us; an added term's error against 64 bits is at most 4.1 x 2^-24 of it, before and now. Long portions of a step with few (portion, channel) threads are cut
 // into segments of seg_len tokens (blockIdx.z) and scanned twice, as the SSD scan below does:
 //   mode 1: every segment but a portion's last from zero -> its final value L_k and decay product d_k to `ws`
 //           ([nseq][nseg + 1][2][channels]; entry 0 holds the value the portion starts from);
 //   mode 2: segment k starts from S_k = d_(k-1) S_(k-1) + L_(k-1) and writes the outputs; the last one writes the slot.
-template <typename T, int MODE>
+template <typename T, int MODE, int TT>             // TT tokens' operands asked for together (1: steps of few tokens per portion)
 __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* __restrict__ u, const T* __restrict__ ypre,
                                   int64_t y_stride, const T* __restrict__ lam, float cmul, int channels, int blocks,
                                   const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx0,
@@ -203,39 +203,50 @@ __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* 
   }
   float dsum = 0.f;                                 // sum of log a over the segment
   const float* gp = gates + ((int64_t)blk * n) * (2 * bw) + cc;
-  // Eight tokens' operands are asked for together, the next eight while these are worked on
-  constexpr int TT = 8;
-  float gr[TT], gi[TT], uv[TT], yv[TT];
-  auto load = [&](int64_t t0) {
-#pragma unroll
-    for (int k = 0; k < TT; ++k) {
-      const int64_t t = t0 + k < q1 ? t0 + k : q1 - 1;
-      gr[k] = gp[t * (2 * bw)], gi[k] = gp[t * (2 * bw) + bw], uv[k] = u[t * channels + c];
-      yv[k] = mode != 1 ? ldf(ypre + t * y_stride + c) : 0.f;
-    }
+  struct Gates {
+    float a, add, y, la;
   };
-  load(q0);
-  for (int64_t t0 = q0; t0 < q1; t0 += TT) {
-    float a[TT], b[TT], x[TT], y[TT], la[TT];
+  const auto gates_of = [&](float gr, float gi, float uv, float yv) {
+    Gates v;
+    v.la = -cmul * sigmoid_hw(gr) * sp;
+    v.a = exp_hw(v.la);
+    const float om = fmaxf(one_less_exp(2.f * v.la), 0.f);          // 1 - a^2, without cancellation near a = 1; then its root
+    const float rs = __builtin_amdgcn_rsqf(om), s0 = om * rs;
+    v.add = (om > 1e-30f ? fmaf(fmaf(-s0, s0, om) * 0.5f, rs, s0) : sqrtf(om)) * (sigmoid_hw(gi) * uv);
+    v.y = mode != 1 ? gelu_tanhf_(yv) : 0.f;
+    return v;
+  };
+  const auto advance = [&](const Gates& v, int64_t t) {
+    st = fmaf(v.a, st, v.add);
+    dsum += v.la;
+    if (mode != 1) stf(out + t * channels + c, st * v.y);
+  };
+  // Eight tokens' operands are asked for together, the next eight while these are worked on; what is left over goes a token at a time
+  int64_t t0 = q0;
+  if constexpr (TT > 1) {
+    float gr[TT], gi[TT], uv[TT], yv[TT];
+    const auto load = [&](int64_t first) {
 #pragma unroll
-    for (int k = 0; k < TT; ++k) {
-      la[k] = -cmul * sigmoid_hw(gr[k]) * sp;
-      a[k] = exp_hw(la[k]);
-      const float om = fmaxf(one_less_exp(2.f * la[k]), 0.f);       // 1 - a^2, without cancellation near a = 1; then its root
-      const float rs = __builtin_amdgcn_rsqf(om), s0 = om * rs;
-      b[k] = om > 1e-30f ? fmaf(fmaf(-s0, s0, om) * 0.5f, rs, s0) : sqrtf(om);
-      x[k] = sigmoid_hw(gi[k]) * uv[k];
-      y[k] = mode != 1 ? gelu_tanhf_(yv[k]) : 0.f;
-    }
-    load(t0 + TT);
-    const int cnt = (int)(q1 - t0 < TT ? q1 - t0 : TT);
+      for (int k = 0; k < TT; ++k) {
+        const int64_t t = first + k;
+        gr[k] = gp[t * (2 * bw)], gi[k] = gp[t * (2 * bw) + bw], uv[k] = u[t * channels + c];
+        yv[k] = mode != 1 ? ldf(ypre + t * y_stride + c) : 0.f;
+      }
+    };
+    if (q0 + TT <= q1) load(q0);
+    for (; t0 + TT <= q1; t0 += TT) {
+      Gates v[TT];
 #pragma unroll
-    for (int k = 0; k < TT; ++k) {
-      if (k >= cnt) break;
-      st = fmaf(a[k], st, b[k] * x[k]);
-      dsum += la[k];
-      if (mode != 1) stf(out + (t0 + k) * channels + c, st * y[k]);
+      for (int k = 0; k < TT; ++k) v[k] = gates_of(gr[k], gi[k], uv[k], yv[k]);
+      load(t0 + 2 * TT <= q1 ? t0 + TT : t0);       // (behind the last eight: these again; a branch here costs 20 %)
+#pragma unroll
+      for (int k = 0; k < TT; ++k) advance(v[k], t0 + k);
     }
+  }
+#pragma unroll 4
+  for (; t0 < q1; ++t0) {
+    const float y1 = mode != 1 ? ldf(ypre + t0 * y_stride + c) : 0.f;
+    advance(gates_of(gp[t0 * (2 * bw)], gp[t0 * (2 * bw) + bw], u[t0 * channels + c], y1), t0);
   }
   if (mode == 1) {
     wv[(int64_t)(2 * seg + 2) * channels] = st;
@@ -792,15 +803,19 @@ extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* yp
   NVS_REQUIRE(!seg_len || ws_floats >= nvs_rglru_scan_workspace(channels, nseq, max_q > 0 ? max_q : n),
               "nvs_rglru_scan: workspace of %lld floats is too small", (long long)ws_floats);
   const dim3 block(64);
-#define NVS_RGLRU_LAUNCH(MODE)                                                                                                     \
-  NVS_DISPATCH(dtype, rglru_scan_kernel<T, MODE><<<dim3((channels + 63) / 64, (unsigned)nseq, seg_len ? nseg : 1), block, 0,         \
+  // Portions under eight tokens take the kernel that walks single ones: as part of eight, most of them nobody's, a decode step of 256 sequences of
+  // 4,096 channels took 31 us; by the leftover path of the kernel of eight, whose registers leave fewer wavefronts, 11.9; here 10.9
+#define NVS_RGLRU_LAUNCH(MODE, TT)                                                                                                 \
+  NVS_DISPATCH(dtype, rglru_scan_kernel<T, MODE, TT><<<dim3((channels + 63) / 64, (unsigned)nseq, seg_len ? nseg : 1), block, 0,         \
                                                   (hipStream_t)stream>>>(gates, u, (const T*)ypre, y_stride, (const T*)lam, c, channels, \
                                                                          blocks, cu_q, ctx0, slot, n, S, (T*)out, seg_len, nseg, ws))
   if (seg_len) {
-    NVS_RGLRU_LAUNCH(1);
-    NVS_RGLRU_LAUNCH(2);
+    NVS_RGLRU_LAUNCH(1, 8);
+    NVS_RGLRU_LAUNCH(2, 8);
+  } else if ((max_q > 0 ? max_q : n) < 8) {
+    NVS_RGLRU_LAUNCH(0, 1);
   } else {
-    NVS_RGLRU_LAUNCH(0);
+    NVS_RGLRU_LAUNCH(0, 8);
   }
 #undef NVS_RGLRU_LAUNCH
   return nvs_check_launch("nvs_rglru_scan");

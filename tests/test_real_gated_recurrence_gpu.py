@@ -32,7 +32,7 @@ def _run(x, S, lens, ctx):
 
 
 @pytest.mark.parametrize("spread", [1.0, 30.0])
-@pytest.mark.parametrize("lens", [[1, 7, 8, 9, 17], [700, 3, 64]], ids=["short", "segments"])
+@pytest.mark.parametrize("lens", [[1, 7, 3], [1, 7, 8, 9, 17], [700, 3, 64]], ids=["few", "short", "segments"])
 def test_against_the_token_loop(lens, spread):
     channels, ctx = 64, [5 * (s % 2) for s in range(len(lens))]
     x, S = _inputs(lens, channels, 3, spread)
@@ -58,7 +58,7 @@ def test_against_the_token_loop(lens, spread):
 
 
 @pytest.mark.parametrize("operand", ["recurrence gate", "input gate", "u", "ypre", "lam", "state"])
-@pytest.mark.parametrize("lens,seq,j", [([3, 21, 9], 1, 12), ([900, 5], 0, 333)], ids=["whole", "segments"])
+@pytest.mark.parametrize("lens,seq,j", [([1, 7, 2], 1, 3), ([3, 21, 9], 1, 12), ([900, 5], 0, 333)], ids=["few", "whole", "segments"])
 def test_a_nan_stays_visible(lens, seq, j, operand):
     channels, c, ctx = 32, 13, [2] * len(lens)
     x, S = _inputs(lens, channels, 5)
