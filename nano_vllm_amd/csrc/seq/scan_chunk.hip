@@ -11,8 +11,7 @@ namespace {
 // products (P x 16 x N). All on v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit ones. The exponents are differences of
 // 64-bit sums, so a pair's weight is as exact as its own exponent however strongly the chunk decays as a whole. Form 2 has
 // exp(F_i - F_j + i_j - m_i) in place of exp(L_i - L_j) w_j and exp(F_i + m_before - m_i) in place of exp(L_i), m the running maximum.
-// A short last chunk is filled with tokens that change nothing (B = C = x = 0, no decay, no step). (Tokens of a chunk meet in products
-// whose weight above the diagonal is zero, so an infinity in one reaches the outputs of the up to 15 before it, never another portion's.)
+// A short last chunk is filled with tokens that change nothing (B = C = x = 0, no decay, no step).
 //
 // A workgroup takes NW * 16 rows p of one (portion, head)'s state, a wavefront 16 of them: its N / 16 accumulator tiles hold
 // S[n = 16 t + 4 (lane / 16) + r][p = lane % 16], which IS the operand layout of C S^T if the four tokens' entries of a product
@@ -392,8 +391,26 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
         }
         if (4 * g + r > l16) m[r] = 0.f;
       }
+      // x of every token meets every output of the chunk in this product, above the diagonal with a weight of 0: a value that is not finite
+      // (rare: or a sum of four that overflows) goes to the outputs behind it alone, token by token
+      const bool odd = !((fabsf(xv[0]) + fabsf(xv[1])) + (fabsf(xv[2]) + fabsf(xv[3])) < INFINITY);
+      if (__ballot(odd) == 0ull) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) yo = mfma4(m[r], xv[r], yo);
+        for (int r = 0; r < 4; ++r) yo = mfma4(m[r], xv[r], yo);
+      } else {
+#pragma unroll 1
+        for (int j0 = 0; j0 < CT; j0 += 4) {        // m[i][j] is in lane i + 16 (j / 4), x[j][p] in lane p + 16 (j / 4), entry j % 4
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float xj = __shfl(xv[k], 4 * j0 + l16, 64);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float mij = __shfl(m[k], 4 * j0 + 4 * g + r, 64);
+              if (j0 + k <= 4 * g + r) yo[r] = fmaf(mij, xj, yo[r]);
+            }
+          }
+        }
+      }
       if (FORM == 2 && w == 0) {
         own = (m[0] + m[1]) + (m[2] + m[3]);
         own += __shfl_xor(own, 16, 64);

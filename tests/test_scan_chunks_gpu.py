@@ -96,3 +96,49 @@ def test_chunked_recurrences_against_the_token_loop(form, heads, P, N, G, lens, 
             assert ((M[slots[s]] - mx[s]).abs() <= (ln + 4) * EPS * mx[s].abs().clamp(min=1)).all(), s
         at += ln
     assert torch.equal(S[0], S0) and torch.equal(M[0], M0)
+
+
+def _scan(form, heads, P, N, por, S, M, x, y, den):
+    """One call on prepared operands: x holds xbc / proj and the gates' parameters."""
+    from nano_vllm_amd import ops_seq
+    if form == 0:
+        ops_seq.ssd_scan(x["xbc"], x["proj"], 0, x["bias"], x["A_log"], x["D"], heads, P, N, 1, por, S, y)
+    elif form == 1:
+        ops_seq.decay_scan(x["proj"], 0, heads * P, heads * (P + N), x["rate"], heads, N, P, por, S, y)
+    else:
+        at = heads * (P + 2 * N)
+        ops_seq.gated_memory_scan(x["proj"], 0, heads * P, heads * (P + N), at, at + heads, x["ib"], x["fb"], 15.0, N ** -0.5, heads, N, P, por, S,
+                                  M, y, den)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("form,heads,P,N", [(0, 2, 64, 128), (0, 2, 100, 64), (1, 2, 64, 64), (1, 2, 128, 128), (2, 2, 64, 64), (2, 2, 128, 128)])
+@pytest.mark.parametrize("lens,seq,j", [([40, 70, 20], 1, 27), ([600, 9], 0, 301)], ids=["whole", "segments"])
+def test_a_value_that_is_not_finite_reaches_no_earlier_token(lens, seq, j, form, heads, P, N, value):
+    g = torch.Generator(device="cuda").manual_seed(P + form)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    n, nseq = sum(lens), len(lens)
+    rows = P + (form == 2)
+    x = dict(xbc=rand(n, heads * P + 2 * N), proj=rand(n, heads * (P + 2 * N) + 8), bias=rand(heads) - 2, A_log=rand(heads), D=rand(heads),
+             rate=torch.full((heads,), 0.95, device="cuda"), ib=rand(heads), fb=rand(heads) + 2)
+    S0, M0 = rand(nseq, heads, rows, N), rand(nseq, heads).abs()
+    first = sum(lens[:seq])
+    h, p = 1, P - 3
+
+    def run():
+        S, M, y, den = S0.clone(), M0.clone(), torch.empty(n, heads * P, device="cuda"), torch.ones(n, heads, device="cuda")
+        _scan(form, heads, P, N, _portions(lens, [3] * nseq, list(range(nseq))), S, M, x, y, den)
+        return S, M, y, den
+    clean = run()
+    x["xbc" if form == 0 else "proj"][first + j, h * P + p] = value
+    S, M, y, den = run()
+    col = h * P + p
+    assert not torch.isfinite(y[first + j:first + lens[seq], col]).any()
+    keep = torch.ones_like(y, dtype=torch.bool)
+    keep[first + j:first + lens[seq], col] = False
+    # (within the chunk of the token the products may be summed in another order: 16 of them, of the size of the largest outputs)
+    assert torch.isfinite(y[keep]).all() and ((y - clean[2])[keep].abs() <= 16 * EPS * clean[2].abs().max()).all()
+    hit = torch.zeros_like(S, dtype=torch.bool)
+    hit[seq, h, p] = True
+    assert not torch.isfinite(S[hit]).any() and torch.equal(S[~hit], clean[0][~hit])
+    assert torch.equal(M, clean[1]) and torch.equal(den, clean[3])
