@@ -9,7 +9,7 @@ namespace {
 //   y_i = exp(L_i) S C_i + sum_{j <= i} exp(L_i - L_j) w_j (C_i . B_j) x_j,     S <- exp(L_15) S + sum_j exp(L_15 - L_j) w_j x_j B_j^T,
 // so a chunk is three products: C S^T (16 x N x P), (C B^T, masked and weighted) x (16 x N x 16 and 16 x 16 x P) and the outer
 // products (P x 16 x N). All on v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit ones. The exponents are differences of
-// 64-bit sums, so a pair's weight is as exact as its own exponent however strongly the chunk decays as a whole. Form 2 has
+// 64-bit sums of exponents above -200, so a pair's weight is as exact as its own exponent however strongly the chunk decays as a whole. Form 2 has
 // exp(F_i - F_j + i_j - m_i) in place of exp(L_i - L_j) w_j and exp(F_i + m_before - m_i) in place of exp(L_i), m the running maximum.
 // A short last chunk is filled with tokens that change nothing (B = C = x = 0, no decay, no step).
 //
@@ -235,7 +235,8 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
     float wij[4], wi, em = 0.f;
     if (FORM == 0) {
       const float dt = valid ? softplusf_(ldf(&g0) + dtb) : 0.f;
-      const double L = row_running_sum((double)A * (double)dt), Lj = lane_of(L, 16 * w + l16);
+      // (below -200 a decay is 0 whatever follows; the sums stay small enough to tell the exponents of the tokens behind it apart, and finite)
+      const double l = valid ? (double)A * (double)dt : 0., L = row_running_sum(l < -200. ? -200. : l), Lj = lane_of(L, 16 * w + l16);
       const float dj = __shfl(dt, 16 * w + l16, 64);
 #pragma unroll
       for (int e = 0; e < 4; ++e) wij[e] = exp_(lane_of(L, 16 * w + 4 * g + e) - Lj) * dj;

@@ -142,3 +142,32 @@ def test_a_value_that_is_not_finite_reaches_no_earlier_token(lens, seq, j, form,
     hit[seq, h, p] = True
     assert not torch.isfinite(S[hit]).any() and torch.equal(S[~hit], clean[0][~hit])
     assert torch.equal(M, clean[1]) and torch.equal(den, clean[3])
+
+
+@pytest.mark.parametrize("A_log,gates", [(100.0, (0.0, 0.0)), (80.0, (0.0, -3.0)), (30.0, (0.0, -40.0)), (5.0, (20.0, -8.0))],
+                         ids=["overflows", "huge", "now and then", "large"])
+@pytest.mark.parametrize("lens", [[37], [400]], ids=["whole", "segments"])
+def test_decays_that_forget_everything(lens, A_log, gates):
+    """A token may forget all before it (a decay of 0, or the rate itself overflows) between tokens that hardly forget anything."""
+    heads, P, N, n = 1, 16, 64, sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    proj = torch.full((n, 8), gates[1], device="cuda")
+    proj[::5] = gates[0]
+    x = dict(xbc=rand(n, P + 2 * N), proj=proj, bias=torch.zeros(1, device="cuda"), A_log=torch.full((1,), A_log, device="cuda"), D=rand(1))
+    S, y = rand(1, 1, P, N), torch.empty(n, P, device="cuda")
+    st = S[0, 0].double()
+    _scan(0, heads, P, N, _portions(lens, [1], [0]), S, None, x, y, None)
+    xs, B, C = x["xbc"].double().split([P, N, N], 1)
+    step = torch.nn.functional.softplus(proj[:, 0].double())
+    a = torch.exp(-torch.exp(x["A_log"].double()) * step)
+    # the rate and the step are 32-bit numbers of a few roundings each: a decay is off by that much of its exponent
+    slack = (torch.exp(x["A_log"].double()) * step * a * 16 * EPS).nan_to_num(0.0)
+    size, err = st.abs(), torch.zeros_like(st)
+    for t in range(n):
+        new = step[t] * xs[t][:, None] * B[t]
+        err = a[t] * err + slack[t] * size
+        st, size = a[t] * st + new, a[t] * size + new.abs()
+        want, mag = st @ C[t] + x["D"].double() * xs[t], size @ C[t].abs() + (x["D"].double() * xs[t]).abs()
+        assert ((y[t].double() - want).abs() <= (t + 1 + N + 32) * EPS * mag + err @ C[t].abs()).all(), t
+    assert ((S[0, 0] - st).abs() <= (n + 32) * EPS * size + err).all()
