@@ -58,7 +58,7 @@ __device__ __forceinline__ float silu_(float x) {
   const float e = -c * L2E, lo = fmaf(-c, L2E, -e) - c * L2E_LO;
   const float t = __builtin_amdgcn_exp2f(e), d = fmaf(t, lo * 0.69314718055994531f, t) + 1.f;
   float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  r = x < -87.f ? 0.f : fmaf(fmaf(-d, r, 1.f), r, r);          // (not e^-87: x may be large)
   const float q = x * r;
   return fabsf(q) < 3e38f ? fmaf(fmaf(-d, q, x), r, q) : q;
 }

@@ -171,3 +171,22 @@ def test_decays_that_forget_everything(lens, A_log, gates):
         want, mag = st @ C[t] + x["D"].double() * xs[t], size @ C[t].abs() + (x["D"].double() * xs[t]).abs()
         assert ((y[t].double() - want).abs() <= (t + 1 + N + 32) * EPS * mag + err @ C[t].abs()).all(), t
     assert ((S[0, 0] - st).abs() <= (n + 32) * EPS * size + err).all()
+
+
+@pytest.mark.parametrize("where", ["value", "key", "query"])
+@pytest.mark.parametrize("huge", [-1e32, -3e38])
+def test_silu_of_large_negative_inputs_is_nothing(where, huge):
+    heads, P, N, n = 2, 64, 64, 40
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = dict(proj=rand(n, heads * (P + 2 * N)), rate=torch.full((heads,), 0.9, device="cuda"))
+    S0 = rand(1, heads, P, N)
+    col = {"value": 3, "key": heads * P + 5, "query": heads * (P + N) + 70}[where]
+
+    def run(value):
+        x["proj"][[4, 20, 39], col] = value
+        S, y = S0.clone(), torch.empty(n, heads * P, device="cuda")
+        _scan(1, heads, P, N, _portions([n], [1], [0]), S, None, x, y, None)
+        return S, y
+    for a, b in zip(run(huge), run(-200.0)):                    # (e^-200 is 0 in 32 bits)
+        assert torch.equal(a, b)
