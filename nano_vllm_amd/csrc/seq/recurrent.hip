@@ -893,6 +893,9 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
     while (pp > 1 && (P % pp != 0 || (P / pp) * ng0 > (pp == 4 ? 256 : 512))) pp >>= 1;
   }
   NVS_REQUIRE(ng <= 64 && (int64_t)((P + pp - 1) / pp) * ng <= 1024, "%s: state %d x head size %d exceeds one workgroup's registers", who, N, P);
+  int seg_len = 0, nseg = 1;                        // (checked whichever kernel it is: a call does not come and go with an address)
+  if (ws) ssd_plan(heads, nseq, max_q, &seg_len, &nseg, form == 2 ? 192 : 512);
+  NVS_REQUIRE(!seg_len || ws_floats >= need(nseg), "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   ScanArgs ca = {form, xbc, proj, proj_stride, dt_col, x_col, b_col, c_col, ga.i_col, ga.f_col, decay, dt_bias, A_log, D, ga.i_bias, ga.f_bias,
                  heads, P, N, G, cu_q, ctx0, slot, S, ga.M, y, ga.den, ws, ga.cap, ga.c_scale, 0, 1};
   // State rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, which win at every length: 100 portions of
@@ -906,9 +909,6 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   const int threads = ((P + pp - 1) / pp) * ng, per = (((P + pp - 1) / pp * pp + 3) & ~3) + 2 * ng * SSD_R + 4;
   const int tb = SSD_TB;                            // tokens per LDS round
   const size_t lds = (size_t)tb * per * sizeof(float);
-  int seg_len = 0, nseg = 1;
-  if (ws) ssd_plan(heads, nseq, max_q, &seg_len, &nseg, form == 2 ? 192 : 512);
-  NVS_REQUIRE(!seg_len || ws_floats >= need(nseg), "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   const dim3 grid(heads, (unsigned)nseq, seg_len ? nseg : 1);
 #define NVS_SSD_LAUNCH(PPV, MODE, FORM)                                                                                             \
   NVS_DISPATCH(dtype, ssd_scan_kernel<T, PPV, MODE, FORM><<<grid, dim3(threads), lds, (hipStream_t)stream>>>(                        \

@@ -561,3 +561,20 @@ def test_reselorn_checkpoint_names_loaders_and_layout(tmp_path):
         path = write_synthetic_checkpoint(str(tmp_path / "b"), raw, tensors=bad)
         with pytest.raises(KeyError):
             load_model(ReselornForCausalLM(resolve(path)[1], torch.float32, block_size=16), path)
+
+
+@pytest.mark.parametrize("address", [16, 20])                   # aligned for the chunked kernel, and not
+def test_scans_refuse_a_workspace_too_small_for_their_segments(address):
+    """The host refuses it before anything is launched, whichever kernel the sizes and addresses lead to."""
+    from nano_vllm_amd import ops_seq
+    lib = ops_seq.load_library()
+    heads, P, N, n, p = 8, 64, 128, 4096, address
+    need = lib.nvs_ssd_scan_workspace(heads, P, N, 1, n)
+    assert need > 0
+    rc = lib.nvs_ssd_scan(p, p, heads, 0, 0, p, p, p, heads, P, N, 1, p, p, p, 1, n, n, p, p, p, 100, None)
+    assert rc != 0 and b"workspace of 100 floats is too small" in lib.nvs_last_error()
+    rc = lib.nvs_decay_scan(p, heads * (P + 2 * N), 0, heads * P, heads * (P + N), 0, p, heads, N, P, p, p, p, 1, n, n, p, p, p, 100, None)
+    assert rc != 0 and b"workspace of 100 floats is too small" in lib.nvs_last_error()
+    rc = lib.nvs_gated_memory_scan(p, heads * (P + 2 * N + 2), 0, heads * P, heads * (P + N), heads * (P + 2 * N), heads * (P + 2 * N + 1), 0, p, p, 15.0,
+                                   1.0, heads, N, P, p, p, p, 1, n, n, p, p, p, p, p, 100, None)
+    assert rc != 0 and b"workspace of 100 floats is too small" in lib.nvs_last_error()
