@@ -898,10 +898,22 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   NVS_REQUIRE(!seg_len || ws_floats >= need(nseg), "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   ScanArgs ca = {form, xbc, proj, proj_stride, dt_col, x_col, b_col, c_col, ga.i_col, ga.f_col, decay, dt_bias, A_log, D, ga.i_bias, ga.f_bias,
                  heads, P, N, G, cu_q, ctx0, slot, S, ga.M, y, ga.den, ws, ga.cap, ga.c_scale, 0, 1};
-  // State rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, which win at every length: 100 portions of
-  // 1 / 5 / 8 / 31 tokens, 64 heads of 64 x 128: 118 / 150 / 180 / 471 us here, 112 / 111 / 113 / 170 there. The constant decay
-  // stays here for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is 7.4e-8, not 8.3e-8.
-  if (scan_chunk_fits(ca, dtype) && (form != 1 || max_q >= 16)) {
+  // State rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, except for a few tokens where these lose. us for
+  // portions of 1 / 3 / 6 tokens, walk against chunks:
+  //   small states of many pairs, whose workgroups of at least four wavefronts and their LDS come in turns of 512 where all of the walk's run
+  //   at once: 2,048 pairs of 16 x 64 13 / 16 / 20 against 21, 1,024 of 32 x 128 17 / 20 / 25 against 20, 2,048 of 64 x 64 23 / 26 / 34 against 25; exponential
+  //   gates, 1,024 pairs of 32 x 64, 32-bit, 12 / 14 / 17 against 17. Fewer pairs (512 of 32 x 128 12 against 11) and larger states (512 of 64 x 128 16
+  //   against 13) are the chunks' from the first token on.
+  //   exponential gates with few pairs, where the gates of 64 tokens are computed for one: 8 pairs of 128 x 128 10 / 13 / 17 against 13 (32-bit 14), 128
+  //   pairs 11 / 14 against 13, 256 pairs 16 / 19 against 16 (18), 512 pairs 30 against 25.
+  // The constant decay stays with the walk for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is
+  // 7.4e-8, not 8.3e-8.
+  const int64_t pairs = (int64_t)heads * nseq;
+  bool walk = form == 1 && max_q < 16;
+  if (form != 1 && pairs >= 1024 && P * N < 8192)
+    walk = max_q * (form == 2 ? 256 : 512) <= pairs * (N / 64) && max_q * P <= (form == 2 ? 256 : 160);
+  if (form == 2 && pairs <= 256) walk = max_q <= (pairs <= 128 && P > 65 ? 3 : pairs <= 128 || P > 65);
+  if (scan_chunk_fits(ca, dtype) && !walk) {
     if (ws) scan_chunk_plan(heads, P, nseq, max_q, &ca.seg_len, &ca.nseg);
     if (ca.seg_len && ws_floats < need(ca.nseg)) ca.seg_len = 0, ca.nseg = 1;
     return scan_chunk_launch(ca, dtype, nseq, stream);
