@@ -252,11 +252,15 @@ extern "C" int nvs_knorm_kvstore(const void* k, const void* v, int64_t stride, i
   NVS_REQUIRE(G > 0 && G <= 65535 && d > 0 && d <= MAX_HEAD && dv > 0 && dv <= MAX_HEAD && n >= 0 && block_size > 0,
               "nvs_knorm_kvstore: G %d d %d dv %d", G, d, dv);
   if (n == 0) return NVS_OK;
-  // A tile per workgroup where there are workgroups enough: 8 heads of 128 + 128, 512 / 1,024 / 2,048 / 4,096 tokens, 32-bit: 15 / 17 / 24 / 46 us
-  // by wavefronts, 18 / 19 / 21 / 26 by tiles; bf16 15 / 15 / 19 / 30, 14 / 14 / 14 / 17
+  // A tile per workgroup where there are workgroups enough to fill the chip: the wavefronts' time follows their number, a tile's its d + dv, whose
+  // passes one workgroup does one after the other. us by wavefronts / by tiles: 8 heads of 128 + 128, bf16, 1,024 / 2,048 / 4,096 tokens 15 / 14, 18 / 13,
+  // 29 / 15 (32-bit 17 / 19, 22 / 18, 46 / 21); one such head, 2,048 / 4,096 / 16,000 tokens 5 / 12, 7 / 12, 17 / 13; one of 256 + 256 8 / 22, 12 / 22, 29 / 26; two of
+  // 64 + 64, 2,048 / 4,096 tokens 5 / 7, 7 / 7; 32-bit, four of 128 + 64 turned, 4,096 / 6,200 tokens 14 / 17, 19 / 20.
   const int ve = dtype == NVS_BF16 ? 8 : 4;
   const uintptr_t al = (uintptr_t)k | (uintptr_t)v | (uintptr_t)knorm | (uintptr_t)k_cache;
-  if (n >= 2048 && d % ve == 0 && dv % ve == 0 && d <= 256 && dv <= 256 && stride % ve == 0 && al % 16 == 0) {
+  const int64_t tiles = (n + KV_TILE - 1) / KV_TILE * G;
+  const int fill = dtype == NVS_BF16 ? 192 : 320;
+  if (n >= 2048 && tiles >= (d + dv > fill ? d + dv : fill) && d % ve == 0 && dv % ve == 0 && d <= 256 && dv <= 256 && stride % ve == 0 && al % 16 == 0) {
     int L = 1;
     while (L * ve < d) L *= 2;
     const dim3 grid((unsigned)((n + KV_TILE - 1) / KV_TILE), G);

@@ -1,4 +1,4 @@
-"""Key norm / rotation and the paged store of long steps, 64 tokens of a head per workgroup: whole and ragged last tiles, head sizes that
+"""Key norm / rotation and the paged store of long steps, by wavefronts and, from 192 tiles of 64 tokens of a head on (32-bit: 320), by tiles: whole and ragged last tiles, head sizes that
 fill no power of two of lanes, tokens without a slot, slots in any order, against the definition in float64."""
 import pytest
 import torch
@@ -8,7 +8,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-6), (torch.bfloat16, 2.0 ** -8)], ids=["f32", "bf16"])
 @pytest.mark.parametrize("n,G,d,dv,rot,norm", [(2048, 2, 64, 64, 0, True), (2049, 1, 128, 256, 128, True), (2111, 3, 72, 40, 20, False),
-                                               (4095, 2, 256, 8, 6, True), (2175, 4, 8, 128, 8, False)])
+                                               (4095, 2, 256, 8, 6, True), (2175, 4, 8, 128, 8, False),
+                                               (6145, 2, 64, 64, 0, True), (3073, 8, 128, 256, 128, True), (2111, 6, 72, 40, 20, False),
+                                               (2111, 8, 256, 8, 6, True), (2175, 6, 8, 128, 8, False), (2048, 6, 64, 64, 64, True),
+                                               (6833, 3, 72, 40, 20, False), (2049, 10, 8, 128, 8, True)])
 def test_stored_keys_and_values(n, G, d, dv, rot, norm, dtype, tol):
     from nano_vllm_amd import ops_seq
     g = torch.Generator().manual_seed(n + d)
