@@ -53,7 +53,8 @@ def test_gate_and_wide_groups(group, order):
     assert ((out.double() - want).abs() <= (group.bit_length() + 24) * EPS * want.abs() + 1e-12).all()
 
 
-@pytest.mark.parametrize("shape,dtype", [((3, 5), torch.float32), ((7, 4), torch.float32), ((1, 2056), torch.bfloat16), ((13, 1001), torch.bfloat16)])
+@pytest.mark.parametrize("shape,dtype", [((3, 5), torch.float32), ((7, 4), torch.float32), ((1, 2056), torch.bfloat16), ((13, 1001), torch.bfloat16),
+                                         ((48, 4096), torch.float32), ((96, 2048), torch.bfloat16), ((201, 1000), torch.bfloat16), ((49, 4095), torch.float32)])
 @pytest.mark.parametrize("scale", [0.01, 1.0, 30.0])
 def test_xielu(shape, dtype, scale):
     from nano_vllm_amd import ops_seq
