@@ -165,9 +165,22 @@ __global__ void moe_route_kernel(const float* __restrict__ z, int64_t z_stride, 
 
 // ---- plan: one workgroup sorts the pairs by expert --------------------------------------------------------------------
 // offs[e] = the rows of the experts before e, each expert's filled up to whole tiles (offs[experts]: all rows); 1,024 threads, an
-// expert each (one thread adding 256 experts up took 12 of the plan's 16 us)
+// expert each (one thread adding 256 experts up took 12 of the plan's 16 us; for up to 16 it is the faster way, 2.6 us a plan of 4
+// experts against 3.2)
 __device__ __forceinline__ void expert_offsets(const int* counts, int experts, int tm, int* offs, int* sums) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (experts <= 16) {
+    if (tid == 0) {
+      int o = 0;
+      for (int e = 0; e < experts; ++e) {
+        offs[e] = o;
+        o += (counts[e] + tm - 1) / tm * tm;
+      }
+      offs[experts] = o;
+    }
+    __syncthreads();
+    return;
+  }
   const int own = tid < experts ? (counts[tid] + tm - 1) / tm * tm : 0;
   int v = own;
 #pragma unroll

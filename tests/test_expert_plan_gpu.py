@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("experts,tm", [(1, 16), (30, 256), (64, 64), (65, 128), (1024, 16)])
+@pytest.mark.parametrize("experts,tm", [(1, 16), (4, 64), (16, 16), (17, 128), (30, 256), (64, 64), (65, 128), (1024, 16)])
 @pytest.mark.parametrize("n,top", [(1, 1), (6143, 1), (6144, 1), (2049, 3), (4096, 2), (13550, 4)])
 def test_every_pair_has_a_row_of_its_expert(n, top, experts, tm):
     from nano_vllm_amd import ops_seq
