@@ -419,7 +419,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   if (!valid) return;
   bf16_t* op = (bf16_t*)A.out + (row * H + h) * DV + 4 * hi;
   const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + row * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
-  const auto gated = [](float x, float gv) { return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-gv * LOG2E)); };
+  const auto gated = [](float x, float gv) { return x * sigmoid_hw(gv); };
   const bool wide = gp && A.gate_w != 1;
   const float ginv = gp && !wide ? gated(inv, (float)gp[0]) : inv;
   const bool quads = wide && ((A.gate_stride & 3) == 0) && ((uintptr_t)A.gate & 7) == 0;

@@ -73,3 +73,48 @@ def test_prompt_kernel_agrees_with_the_scalar_kernel(d, dv, case):
     err = ((got - want).norm() / want.norm()).item()
     assert err <= 2.0 ** -7, err
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
+
+
+def step(q, K, V, lens, ctx, H, G, d, dv, scale=1.0, window=0, sink=None, gates=None, per_head=False, page=64):
+    """One call on sequences whose keys K [tokens of all, G, d] and values V [.., G, dv] lie in pages in order."""
+    from nano_vllm_amd import ops_seq
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    need = [-(-(a + b) // page) for a, b in zip(lens, ctx)]
+    kc = torch.zeros(sum(need), page, G, d, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros(sum(need), G, dv, page, dtype=torch.bfloat16, device="cuda")
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    at = first = 0
+    for s, (a, b) in enumerate(zip(lens, ctx)):
+        T = a + b
+        kc[first:first + need[s]].view(-1, G, d)[:T] = K[at:at + T].to(torch.bfloat16)
+        flat = torch.zeros(need[s] * page, G, dv, dtype=torch.bfloat16, device="cuda")
+        flat[:T] = V[at:at + T].to(torch.bfloat16)
+        vc[first:first + need[s]] = flat.view(need[s], page, G, dv).permute(0, 2, 3, 1)
+        table[s, :need[s]] = torch.arange(first, first + need[s])
+        at, first = at + T, first + need[s]
+    n = sum(lens)
+    por = ops_seq.Portions(i32([0] + lens).cumsum(0).to(torch.int32), i32(ctx), i32(list(range(len(lens)))),
+                           torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32).cuda(), len(lens), n, max(lens))
+    out = torch.full((n, H * dv), 9.0, dtype=torch.bfloat16, device="cuda")
+    ops_seq.window_attn(q, None, 1e-6, gates, kc.view(-1, G, d), vc.view(-1, G, dv), table.cuda(), page, por, H, G, d, dv, scale, window, out,
+                        gate_per_head=per_head, sink=sink)
+    return out
+
+
+SIZES = [(128, 128), (256, 192)]
+
+
+@pytest.mark.parametrize("d,dv", SIZES)
+@pytest.mark.parametrize("per_head", [False, True])
+def test_gates_are_exact_to_their_last_bits(d, dv, per_head):
+    """With one visible key the output is its value times the gate, rounded once to bfloat16: it lies between the roundings of the exact
+    product less and plus six roundings of 2^-24 (a sigmoid and a product in 32 bits: its exponential takes two, sum, reciprocal and product one)."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    H, n = 4, 600
+    v = torch.randn(n, 1, dv, generator=g, device="cuda").bfloat16()
+    gates = (torch.rand(n, H * (1 if per_head else dv), generator=g, device="cuda") * 100 - 80).bfloat16()
+    q = torch.randn(n, H * d, generator=g, device="cuda").bfloat16()
+    got = step(q, torch.zeros(n, 1, d, device="cuda"), v, [1] * n, [0] * n, H, 1, d, dv, gates=gates, per_head=per_head).view(n, H, dv)
+    want = v.double() * torch.sigmoid(gates.double().view(n, H, -1))
+    lo, hi = ((want * (1 + f * 6 * 2.0 ** -24)).float().bfloat16() for f in (-1, 1))
+    assert ((got >= torch.minimum(lo, hi)) & (got <= torch.maximum(lo, hi))).all()
