@@ -252,8 +252,11 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
       }
     }
   }
-  // a sink is a score in the denominator without a value; the sum starts from it (once per query: in the lower half of the lanes)
-  float m = A.sink ? A.sink[h] : -1e30f, l = A.sink && hi == 0 ? 1.f : 0.f;
+  // a sink is a score in the denominator without a value; the sum starts from it (once per query: in the lower half of the lanes). One that weighs
+  // nothing beside any score is none: the maximum must lie above that of a round in which the query sees no key
+  const float sink = A.sink ? A.sink[h] : -INFINITY;
+  const bool none = sink < -1e30f;
+  float m = none ? -1e30f : sink, l = none || hi != 0 ? 0.f : 1.f;
   f32x16_t o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)

@@ -118,3 +118,17 @@ def test_gates_are_exact_to_their_last_bits(d, dv, per_head):
     want = v.double() * torch.sigmoid(gates.double().view(n, H, -1))
     lo, hi = ((want * (1 + f * 6 * 2.0 ** -24)).float().bfloat16() for f in (-1, 1))
     assert ((got >= torch.minimum(lo, hi)) & (got <= torch.maximum(lo, hi))).all()
+
+
+@pytest.mark.parametrize("d,dv", SIZES)
+@pytest.mark.parametrize("value", [float("-inf"), torch.finfo(torch.float32).min, -2.5e38, -1e31])
+@pytest.mark.parametrize("window", [0, 33, 64, 100])
+def test_a_sink_without_weight(d, dv, value, window):
+    """A sink that weighs nothing changes nothing, also where a query sees no key of its workgroup's first rounds."""
+    g = torch.Generator(device="cuda").manual_seed(window)
+    H, lens, ctx = 2, [300, 5, 1], [0, 130, 200]
+    n, total = sum(lens), sum(lens) + sum(ctx)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    args = rand(n, H * d).bfloat16(), rand(total, 1, d), rand(total, 1, dv), lens, ctx, H, 1, d, dv, d ** -0.5, window
+    plain, with_sink = step(*args), step(*args, sink=torch.full((H,), value, device="cuda"))
+    assert torch.isfinite(plain).all() and torch.equal(plain, with_sink)
