@@ -132,3 +132,26 @@ def test_a_sink_without_weight(d, dv, value, window):
     args = rand(n, H * d).bfloat16(), rand(total, 1, d), rand(total, 1, dv), lens, ctx, H, 1, d, dv, d ** -0.5, window
     plain, with_sink = step(*args), step(*args, sink=torch.full((H,), value, device="cuda"))
     assert torch.isfinite(plain).all() and torch.equal(plain, with_sink)
+
+
+@pytest.mark.parametrize("d,dv", SIZES)
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("a,b,unit", [(3, 4, 1), (9, 9, 1), (-10, 10, 1), (12, 12, 2), (17, 17, 2048)])
+def test_weights_of_rounds_with_different_maxima(d, dv, a, b, unit, sink):
+    """Scores of 2^(|a| + b) (negative with a) plus small whole numbers, all exact: the largest moves from round to round, and the weights must
+    stay on one scale however far from 0 they all lie. Weights and output are rounded to 8 bits (2^-9 each, and what they add up to)."""
+    g = torch.Generator(device="cuda").manual_seed(b)
+    H, T, n = 2, 500, 40
+    delta = torch.randint(0, 3, (T,), generator=g, device="cuda") + torch.arange(T, device="cuda") // 64 % 5
+    q, K = torch.zeros(n, H, d, device="cuda"), torch.zeros(T, 1, d, device="cuda")
+    q[..., 0], q[..., 1], K[:, 0, 0], K[:, 0, 1] = 2.0 ** abs(a) * (-1 if a < 0 else 1), unit, 2.0 ** b, delta.float()
+    V = torch.randn(T, 1, dv, generator=g, device="cuda").bfloat16()
+    start = 2.0 ** (abs(a) + b) * (-1 if a < 0 else 1)
+    s = torch.full((H,), start + 4 * unit, device="cuda") if sink else None
+    got = step(q.view(n, -1).bfloat16(), K, V, [n], [T - n], H, 1, d, dv, sink=s).view(n, H, dv).double()
+    score = (start + unit * delta.double()).expand(n, T).clone()
+    score[torch.arange(T, device="cuda") > torch.arange(T - n, T, device="cuda")[:, None]] = -torch.inf
+    extra = torch.full((n, 1), start + 4 * unit if sink else -torch.inf, dtype=torch.float64, device="cuda")
+    p = torch.cat([score, extra], 1).softmax(1)[:, :-1]
+    want = (p @ V[:, 0].double())[:, None].expand(n, H, dv)
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
