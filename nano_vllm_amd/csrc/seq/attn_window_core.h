@@ -487,6 +487,20 @@ __global__ __launch_bounds__(256) void window_attn_mfma_lds_kernel(const WindowA
       const int u = tid + i * 256, tok = u / (4 * DK), part = u - tok * (4 * DK);
       *(u32x4_t*)&Ks[tok][part * 8] = kf[i];
     }
+    // Steps of short portions: values behind the last token (pooled rounds: block) anybody sees have a weight of 0, and are made 0 too, since what a page
+    // held before may be an infinity. (A thread's units hold the same eight tokens of different columns.)
+    if constexpr (QT == 1) {
+      const int live = (pooled ? nb_last : b_last + 1) - (j0 + (tid & 7) * 8);
+      if (live > 0 && live < 8) {
+#pragma unroll
+        for (int i = 0; i < VU; ++i) {
+          bf16x8_t v = __builtin_bit_cast(bf16x8_t, vf[i]);
+#pragma unroll
+          for (int e = 1; e < 8; ++e) v[e] = e < live ? v[e] : (bf16_t)0.f;
+          vf[i] = __builtin_bit_cast(u32x4_t, v);
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < VU; ++i) {
       const int u = tid + i * 256, col = u >> 3, grp = u & 7;

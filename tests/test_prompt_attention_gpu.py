@@ -155,3 +155,12 @@ def test_weights_of_rounds_with_different_maxima(d, dv, a, b, unit, sink):
     p = torch.cat([score, extra], 1).softmax(1)[:, :-1]
     want = (p @ V[:, 0].double())[:, None].expand(n, H, dv)
     assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("d,dv,H,G,pool", [(64, 64, 4, 2, 0), (64, 64, 16, 1, 0), (128, 64, 8, 1, 0), (64, 128, 2, 1, 4)])
+def test_single_tokens_of_other_sizes_do_not_see_what_a_page_held_before(d, dv, H, G, pool):
+    kw = dict(H=H, G=G, d=d, dv=dv, lens=[1] * 9, ctx=[0, 6, 7, 8, 62, 63, 64, 70, 199], window=40 if pool else 0, pool=pool, seed=d)
+    got, want = call(False, **kw).double(), call(True, **kw).double()
+    assert torch.isfinite(want).all()
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
+    assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
