@@ -451,18 +451,31 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   }
 }
 
+struct PromptGrid {
+  int hw;                                           // heads of a workgroup
+  int64_t tiles, rows;                              // query tiles, heads / hw
+};
+inline PromptGrid prompt_grid(const WindowAttnArgs& a, int nw) {
+  const int hpg = a.H / a.G;
+  PromptGrid p;
+  p.hw = hpg % nw == 0 ? nw : (hpg % 4 == 0 ? 4 : (hpg % 2 == 0 ? 2 : 1));
+  p.rows = a.H / p.hw;
+  // an upper bound: every portion may end with a partial tile, and every tile holds a token (a workgroup without one takes a live one's place)
+  p.tiles = a.n / ((nw / p.hw) * 32) + a.nseq;
+  if (p.tiles > a.n) p.tiles = a.n;
+  return p;
+}
+
 template <int D, int DV, int NW, bool EXT>
 int launch_prompt(WindowAttnArgs a, hipStream_t stream) {
-  const int hpg = a.H / a.G;
-  a.hw = hpg % NW == 0 ? NW : (hpg % 4 == 0 ? 4 : (hpg % 2 == 0 ? 2 : 1));
+  const PromptGrid p = prompt_grid(a, NW);
+  a.hw = p.hw;
   a.bs_shift = __builtin_ctz(a.block_size);
-  const int bq = (NW / a.hw) * 32;
-  const int64_t btiles = a.n / bq + a.nseq;         // an upper bound: every portion may end with a partial tile
   constexpr int LDS = 2 * (64 * D * 2 + DV * 128);
   const auto kernel = window_attn_prompt_kernel<D, DV, NW, EXT>;
   static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   NVS_REQUIRE(room == hipSuccess, "nvs_window_attn: %d bytes of LDS were refused", LDS);
-  kernel<<<dim3((unsigned)btiles, (unsigned)(a.G * (hpg / a.hw))), dim3(64 * NW), LDS, stream>>>(a);
+  kernel<<<dim3((unsigned)p.tiles, (unsigned)p.rows), dim3(64 * NW), LDS, stream>>>(a);
   return nvs_check_launch("nvs_window_attn (prompts)");
 }
 

@@ -312,10 +312,18 @@ extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnor
     // The pipelined kernel for the sizes it is built for, whenever its tiles lie in one page and its 16-byte pieces are aligned. It is the faster one
     // from a single token (16 query heads on 8 kv heads of 128 behind 900 tokens: 31 us against 50; 64 such sequences 49 against 80; latent
     // rows 68 against 89) to whole prompts (attn_prompt.h); the others take every other size.
+    // Steps of single tokens with eight or more query heads per kv head (`packed`: the other kernel's query tiles hold heads) are its only while its
+    // workgroups run at once, two on a compute unit, one of latent rows or with capped scores, where the vector units have no time left: its queries
+    // are positions, so four (eight) heads each read all keys, and one of a wavefront's 32 queries lives. us by packed heads / here, contexts of
+    // 2,500: 64 heads over one kv head of 128, 24 / 32 / 36 / 48 sequences 110 / 92, 112 / 103, 113 / 132, 114 / 150; 8 heads over each of two, 128 / 144 /
+    // 224 126 / 116, 140 / 151, 161 / 217; latent rows, 16 heads, 96 / 128 / 136 / 192 184 / 134, 190 / 175, 191 / 265, 201 / 290; capped, contexts of
+    // 1,500, 8 heads over each of four, 16 / 32 / 64 91 / 80, 93 / 83, 99 / 126.
     const bool sizes = (d == 128 && dv == 128) || (d == 256 && dv == 192 && !extended);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)qnorm | (uintptr_t)pool_k | (uintptr_t)pool_v) & 15) == 0 &&
                          q_stride % 8 == 0 && ((uintptr_t)out & 7) == 0;
-    if (sizes && aligned && block_size >= 64 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
+    const PromptGrid grid = prompt_grid(a, d == 128 ? 4 : 8);
+    const bool packed = H / G >= 8 && n < 32ll * nseq && 4 * n <= (int64_t)nseq * (H / G) && grid.tiles * grid.rows > (d == 128 && !(softcap > 0.f) ? 512 : 256);
+    if (sizes && aligned && !packed && block_size >= 64 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
       return extended ? window_attn_prompt_extended(a, (hipStream_t)stream) : window_attn_prompt(a, (hipStream_t)stream);
     if (extended) window_attn_extended(a, (hipStream_t)stream);
     else launch_mfma_sizes<false>(a, (hipStream_t)stream);

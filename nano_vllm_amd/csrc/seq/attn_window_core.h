@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void window_attn_mfma_lds_kernel(const WindowA
     }
     // Steps of short portions: values behind the last token (pooled rounds: block) anybody sees have a weight of 0, and are made 0 too, since what a page
     // held before may be an infinity. (A thread's units hold the same eight tokens of different columns.)
-    if constexpr (QT == 1) {
+    if (QT == 1 && (it == rounds - 1 || (EXT && it == npr - 1))) {
       const int live = (pooled ? nb_last : b_last + 1) - (j0 + (tid & 7) * 8);
       if (live > 0 && live < 8) {
 #pragma unroll

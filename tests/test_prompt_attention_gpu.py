@@ -164,3 +164,14 @@ def test_single_tokens_of_other_sizes_do_not_see_what_a_page_held_before(d, dv, 
     assert torch.isfinite(want).all()
     assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
+
+
+@pytest.mark.parametrize("d,dv,H,G,nseq,cap", [(128, 128, 64, 1, 32, 0.0), (128, 128, 64, 1, 33, 0.0), (128, 128, 18, 2, 28, 0.0), (128, 128, 18, 2, 29, 0.0),
+                                               (128, 128, 16, 2, 64, 5.0), (128, 128, 16, 2, 65, 5.0), (256, 192, 72, 1, 28, 0.0), (256, 192, 72, 1, 29, 0.0)])
+def test_single_tokens_with_many_heads_over_a_kv_head(d, dv, H, G, nseq, cap):
+    """On either side of the step where the kernel's workgroups no longer run at once and heads are packed into query tiles instead."""
+    kw = dict(H=H, G=G, d=d, dv=dv, lens=[1] * nseq, ctx=[(37 * i) % 200 for i in range(nseq)], sink=True, cap=cap, seed=nseq)
+    got, want = call(False, **kw).double(), call(True, **kw).double()
+    assert torch.isfinite(want).all()
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
+    assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
