@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvstore_kernel(
     const float* __restrict__ cos_sin, int64_t max_pos, const int32_t* __restrict__ slot_mapping,
     bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_out, void* __restrict__ k_cache,
     void* __restrict__ v_cache, int64_t n_tok, int hq, int hkv, int block_size) {
-  const unsigned htot = hq + 2 * hkv, total = (unsigned)n_tok * htot;       // (below 2^31)
+  const unsigned htot = hq + 2 * hkv, total = (unsigned)n_tok * htot;       // (below 2^31 - 32)
   const unsigned unit0 = blockIdx.x * (16 * UN) + (threadIdx.x >> 4);
   const int sub = threadIdx.x & 15;
   u32x4_t raw[UN];
@@ -185,7 +185,7 @@ extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, 
               "nvl_qknorm_rope_kvstore: pointers must be 16-byte aligned");
   const int64_t total = n_tok * (num_q_heads + 2 * num_kv_heads);
   if (total == 0) return NVL_OK;
-  NVL_REQUIRE((total + 15) / 16 < (1ll << 31), "nvl_qknorm_rope_kvstore: too many rows");
+  NVL_REQUIRE(total + 32 < (1ll << 31), "nvl_qknorm_rope_kvstore: too many rows");       // (the kernel counts heads in 32 bits, up to 31 beyond the last)
   const bool two = total >= 262144;                 // (the kernel's comment has both sides)
 #define NVL_QK(KV8, UN)                                                                                                           \
   hipLaunchKernelGGL((qknorm_rope_kvstore_kernel<KV8, UN>), dim3((unsigned)((total + 16 * UN - 1) / (16 * UN))), dim3(256), 0,     \

@@ -185,3 +185,12 @@ def test_generated_asm_cores_are_fresh():
     env = {k: v for k, v in os.environ.items() if not k.startswith("NVL_PF64_")}
     rc = subprocess.run([sys.executable, os.path.join(ROOT, "tools", "gen_prefill_asm.py"), "--core", "--check"], env=env).returncode
     assert rc == 0, "run `python tools/gen_prefill_asm.py --core` and commit csrc/attn_prefill64_core.inc"
+
+
+def test_qknorm_refuses_more_heads_than_its_kernel_counts():
+    """On the host, before anything is launched: the kernel counts heads in 32 bits, up to 31 beyond the last."""
+    from nano_vllm_amd import ops
+    lib, p = ops.lib(), 16
+    for n in (1 << 26, (1 << 26) - 1, 1 << 27, 1 << 30):         # 32 heads a token: from 2^31 - 32 heads on
+        rc = lib.nvl_qknorm_rope_kvstore(p, 32 * 128, p, p, p, 1e-6, p, 8, p, p, p, p, p, n, 16, 8, 256, 1 << 20, 0, None)
+        assert rc == -1 and b"too many rows" in lib.nvl_last_error(), n

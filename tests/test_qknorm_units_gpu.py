@@ -6,8 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn], ids=["bf16", "fp8"])
 @pytest.mark.parametrize("n,hq,hkv", [(8192, 16, 8), (8193, 16, 8), (15000, 16, 1), (37450, 5, 1), (9001, 28, 2)])
-def test_two_heads_per_row_equal_one(n, hq, hkv):
+def test_two_heads_per_row_equal_one(n, hq, hkv, cache):
     from nano_vllm_amd import ops
     torch.manual_seed(n)
     dev = dict(device="cuda")
@@ -23,11 +24,11 @@ def test_two_heads_per_row_equal_one(n, hq, hkv):
 
     def run(parts):
         q, k = torch.zeros(n, hq, 128, **dev).bfloat16(), torch.zeros(n, hkv, 128, **dev).bfloat16()
-        kc = torch.zeros(blocks, hkv, block, 128, **dev).bfloat16()
+        kc = torch.zeros(blocks, hkv, block, 128, **dev).to(cache)
         vc = torch.zeros_like(kc)
         for lo in range(0, n, parts):
             hi = min(lo + parts, n)
             ops.qknorm_rope_kvstore(qkv[lo:hi], pos[lo:hi], qw, kw, 1e-6, table, slots[lo:hi], q[lo:hi], k[lo:hi], kc, vc, hq, hkv)
-        return q, k, kc, vc
+        return q, k, kc.view(torch.int8), vc.view(torch.int8)
     for name, a, b in zip("q k k_cache v_cache".split(), run(n), run(2048)):
         assert torch.equal(a, b), name
