@@ -24,7 +24,8 @@ def _portions(lens, ctx, slots):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("lens", [[1, 3, 2], [1, 2] * 40, [1, 16, 17, 2], [63, 65, 15], [700, 20, 300]], ids=["few", "crowd", "short", "group", "segments"])
 @pytest.mark.parametrize("form,heads,P,N,G", [(0, 16, 16, 64, 1), (2, 16, 24, 64, 1), (0, 4, 64, 128, 2), (0, 3, 40, 64, 1), (0, 2, 100, 128, 2), (1, 3, 128, 128, 1), (1, 2, 16, 64, 1),
-                                              (2, 2, 128, 128, 1), (2, 3, 24, 64, 1), (2, 2, 72, 128, 1)])
+                                              (2, 2, 128, 128, 1), (2, 3, 24, 64, 1), (2, 2, 72, 128, 1),
+                                              (0, 2, 136, 64, 1), (0, 1, 256, 64, 1), (1, 2, 200, 64, 1)])        # (two workgroups of rows)
 def test_chunked_recurrences_against_the_token_loop(form, heads, P, N, G, lens, dtype):
     from nano_vllm_amd import ops_seq
     g = torch.Generator(device="cuda").manual_seed(heads * P + N + form)
