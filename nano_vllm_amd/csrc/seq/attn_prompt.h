@@ -100,6 +100,11 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   const int rounds = npr + ((b_last - (lo & ~63)) >> 6) + 1;
   // the rounds every query of this wavefront sees in whole
   const int nb_first = EXT ? seen_blocks(p_first, window, A.pool) : 0, lo_hi = vis_lo(p_hi, window, chunk);
+  // Rounds none of them sees are left out: a weight of 0 times a value that is not finite is NaN, in outputs of tokens that do not see it. All
+  // behind `final` are such rounds (-1: a wavefront of nobody's queries) and, without pooled blocks, those that end before `lo_first`. (The branches
+  // cost 0 to 3 % of whole prompts; single tokens with capped scores and one head over each of eight, 64 sequences, 148 -> 109 us.)
+  const int final = rel0 < len ? (c0 + (rel0 + 31 < len ? rel0 + 31 : len - 1) - jt) >> 6 : -1, lo_first = vis_lo(p_first, window, chunk);
+  const auto early = [&](int it) { return !EXT && jt + it * 64 + 63 < lo_first; };
 
   // ---- requests. K tile: row = token, 2 D bytes, 16-byte unit u of token t at u ^ (t & 15). V tile: row = value column, 64 tokens = 128 bytes, unit u of
   // column c at u ^ ((c >> 1) & 7). Both make the 16-byte operand reads of 16 neighbouring lanes cover all banks once.
@@ -294,16 +299,13 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
       rlen = top >= bottom ? (unsigned)(top - bottom) : 0u;
     }
   };
-  // A wavefront of nobody's queries computes along, but for the caps, which would take a live one's time: single tokens, contexts of 1,500, one head over
-  // each of eight, 64 sequences 148 -> 109 us, five over each of four, 16 sequences 118 -> 91
-  const bool live = rel0 < len;
   const auto work = [&](auto unit, f32x16_t (&sc)[2], u32x4_t (&pb)[4]) {
     constexpr int u = decltype(unit)::value;
     if constexpr (u < 4) {
       f32x16_t& v = sc[u >> 1];
       if constexpr (u == 0) mx = HIDDEN;
       if (EXT) {
-        if (A.softcap > 0.f && live) {
+        if (A.softcap > 0.f) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) v[(u & 1) * 8 + i] = capped(v[(u & 1) * 8 + i], A.softcap);
         }
@@ -348,15 +350,18 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
     f32x16_t sc[2][2];
     u32x4_t pb[2][4];
     // Round it: sums of round it - 1 (V tile in buffer nxt), scores of round it + 1 (K tile in buffer nxt); K tile it + 2 and V tile it come into cur.
-    const auto round = [&](auto first, int it, auto which) {
-      constexpr bool WITH_O = decltype(first)::value == 0;
-      constexpr int cur = decltype(which)::value, nxt = cur ^ 1, OS = WITH_O ? 4 * DB : 0, SLOTS = OS + 2 * DC;
+    const auto turn = [&](bool first, int it, int cur) {
       arrive();
-      if (WITH_O) clear_tail(it - 1, nxt);
+      if (!first) clear_tail(it - 1, cur ^ 1);
       request_k(it + 2, cur);
-      if (WITH_O) request_v(it, cur);
+      if (!first) request_v(it, cur);
       lookup_k(it + 3);
-      if (WITH_O) lookup_v(it + 1);
+      if (!first) lookup_v(it + 1);
+    };
+    const auto round = [&](auto first, int it, auto which) {
+      constexpr bool FIRST = decltype(first)::value != 0, WITH_O = !FIRST;
+      constexpr int cur = decltype(which)::value, nxt = cur ^ 1, OS = WITH_O ? 4 * DB : 0, SLOTS = OS + 2 * DC;
+      turn(FIRST, it, cur);
       begin(it);
       bf16x8_t ring[AHEAD + 1];
       const auto operand = [&](int slot) { return slot < OS ? v_operand(nxt, slot / DB, slot % DB) : k_operand(nxt, (slot - OS) / DC, (slot - OS) % DC); };
@@ -371,27 +376,46 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         static_for<slot * UNITS / SLOTS, (slot + 1) * UNITS / SLOTS>([&](auto u) { work(u, sc[cur], pb[cur]); });
         __builtin_amdgcn_sched_barrier(0);
       });
-      if (WITH_O) rescale();
+      if (!FIRST && early(it - 1)) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
+      }
+      if (!FIRST) rescale();
     };
     arrive();
     request_k(1, 1);
     lookup_k(2);
+    if (final >= 0) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int c = 0; c < DC; ++c) s_product(sc[0][kb], k_operand(0, kb, c), c);
-    round(Int<1>{}, 0, Int<0>{});
+        for (int c = 0; c < DC; ++c) s_product(sc[0][kb], k_operand(0, kb, c), c);
+      round(Int<1>{}, 0, Int<0>{});
+    } else {
+      turn(true, 0, 0);
+    }
+    int it = 1;
 #pragma unroll 1
-    for (int it = 1; it < rounds; it += 2) {        // (in pairs: an odd one at the end is a round that nobody sees)
+    for (; it < rounds && it <= final + 1; it += 2) {       // (in pairs: an odd one at the end is a round that nobody sees)
       round(Int<0>{}, it, Int<1>{});
+      if (it > final) {
+        ++it;
+        break;
+      }
       round(Int<0>{}, it + 1, Int<0>{});
     }
+#pragma unroll 1
+    for (; it <= rounds / 2 * 2; ++it) turn(false, it, it & 1);
     arrive();
     clear_tail(rounds / 2 * 2, 0);
+    if (rounds / 2 * 2 <= final) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+      for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o_product(o[db], v_operand(0, a, db), pb[0][a]);
+        for (int db = 0; db < DB; ++db) o_product(o[db], v_operand(0, a, db), pb[0][a]);
+    }
   } else {
     f32x16_t sc[2];
     u32x4_t pb[4];
@@ -402,6 +426,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
       request_v(it + 1, cur ^ 1);
       lookup_k(it + 2);
       lookup_v(it + 2);
+      if (it > final || early(it)) return;
       begin(it);
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)

@@ -175,3 +175,33 @@ def test_single_tokens_with_many_heads_over_a_kv_head(d, dv, H, G, nseq, cap):
     assert torch.isfinite(want).all()
     assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
+
+
+@pytest.mark.parametrize("d,dv", SIZES)
+@pytest.mark.parametrize("H,G", [(3, 3), (2, 1), (4, 1), (8, 1)])
+@pytest.mark.parametrize("window", [0, 40])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_a_value_that_is_not_finite_stays_with_the_tokens_around_it(d, dv, H, G, window, value):
+    """A value of token j lies in a tile of 64 keys, and 32 queries go together: the products of a tile that none of them sees are left out, so
+    what token j brings stays with the queries around it."""
+    g = torch.Generator(device="cuda").manual_seed(H + window)
+    lens, ctx = [500, 130, 31], [0, 70, 300]
+    n, total = sum(lens), sum(lens) + sum(ctx)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q, K, V = rand(n, H * d).bfloat16(), rand(total, G, d), rand(total, G, dv)
+    run = lambda v: step(q, K, v, lens, ctx, H, G, d, dv, d ** -0.5, window).view(n, H, dv)
+    clean = run(V)
+    assert torch.isfinite(clean).all()
+    for s, j in ((0, 0), (0, 70), (0, 130), (0, 319), (0, 499), (1, 5), (1, 110), (1, 199), (2, 20), (2, 330)):
+        at, row = sum(lens[:s]) + sum(ctx[:s]), sum(lens[:s])
+        bad = V.clone()
+        bad[at + j, G - 1, dv // 2] = value
+        got = run(bad)
+        pos = torch.arange(ctx[s], ctx[s] + lens[s], device="cuda")
+        sees = (pos >= j) & (pos - j < window if window else True)
+        first = ctx[s] + torch.arange(lens[s], device="cuda") // 32 * 32
+        touched = (first + 31 >= j // 64 * 64) & (first - window + 1 <= j // 64 * 64 + 63 if window else True)
+        same = torch.ones(n, dtype=torch.bool, device="cuda")
+        same[row:row + lens[s]] = ~touched
+        assert torch.equal(got[same], clean[same]), (s, j)
+        assert not torch.isfinite(got[row:row + lens[s]][sees][:, -1, dv // 2]).any(), (s, j)
