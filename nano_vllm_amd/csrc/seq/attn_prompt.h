@@ -49,12 +49,12 @@ constexpr float HIDDEN = -3e38f;                  // a masked score: its weight 
 // fit a compute unit. Rows of 256: scores, weights, sums one after the other, by two wavefronts per SIMD (a workgroup of eight: 256 registers hold
 // one round's scores only) that fill each other's gaps.
 //
-// What bounds it: per round and wavefront 32 MFMAs (rows of 256: 56) of 32 clocks, as much of the LDS pipe's time for eight wavefronts, and about 900
-// clocks of vector work; the matrix units run at 0.95-1.06 PFLOP/s on one prompt of 16,384 tokens. On shorter ones the time before the first and
+// What bounds it: per round and wavefront 32 MFMAs (rows of 256: 56) of 32 clocks, as much of the LDS pipe's time for eight wavefronts, and about 1,000
+// clocks of vector work; the matrix units run at 0.92-1.03 PFLOP/s on one prompt of 16,384 tokens. On shorter ones the time before the first and
 // behind the last round shows: queries, norm and rotation are prepared while the first tile is on its way, cos and sin once per position and
 // workgroup. 64 queries per wavefront (half the LDS reads) need the accumulation registers, and the compiler's moves to and from them cost more.
-// MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 333, blocks of
-// 1024 with rotation 936 -> 261; 16 / 8 heads, causal, rotation, sink 764 -> 196; latent rows, 16 heads, window 1024 1012 -> 261, causal 1014 -> 291.
+// MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 351, blocks of
+// 1024 with rotation 936 -> 255; 16 / 8 heads, causal, rotation, sink 764 -> 189; latent rows, 16 heads, window 1024 and causal 1013 -> 275.
 template <int D, int DV, int NW, bool EXT>
 __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_kernel(const WindowAttnArgs A) {
   constexpr bool PIPE = D == 128;

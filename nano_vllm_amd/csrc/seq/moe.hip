@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 //
 // Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
 // four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
-// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.36 + 1.27 ms = 1154 and 1073 TFLOP/s (the tiled kernel: 4.05 +
+// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.35 to 2.45 + 1.39 to 1.44 ms = 1110 to 1160 and 950 to 980 TFLOP/s (the tiled kernel: 4.05 +
 // 2.28 ms; the library's dense product of these sizes: 1.3-1.46 PFLOP/s); what is left is the chip's power limit and half a tile of padding
 // per expert. 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
 // (moe_gemm_mfma_kernel 411 + 217); width 1024, ff 768: 20 + 12 us (58 + 27). 32-bit, 1,044 rows, width 1024: 59 + 32 us (moe_gemm_kernel

@@ -43,7 +43,7 @@ __global__ void embed_sinusoid_kernel(const T* __restrict__ table, const int64_t
   }
 }
 
-// the same, four columns per access: two angles, whose sine and cosine come together. 13,550 rows of 4,096, bf16: 125 us, here 65
+// the same, four columns per access: two angles, whose sine and cosine come together. 13,550 rows of 4,096, bf16: 125 us, here 71
 template <typename T>
 __global__ void embed_sinusoid4_kernel(const T* __restrict__ table, const int64_t* __restrict__ ids, const int64_t* __restrict__ pos,
                                        int width, float scale, float log2_base, float* __restrict__ x, T* __restrict__ xh) {
@@ -125,7 +125,7 @@ __global__ void norm_residual_kernel(const T* __restrict__ m, const T* __restric
 }
 
 // The same with four columns per access and the row in registers (PER accesses per thread). Bound by memory: 13,550 rows of 4,096, bf16
-// branches: a column at a time 264 us (two branches) and 186, here 156 and 128 (888 and 777 MB)
+// branches: a column at a time 264 us (two branches) and 186, here 131 and 101 (777 and 666 MB)
 template <typename T, int PER, bool TWO>
 __global__ __launch_bounds__(256) void norm_residual_row_kernel(const T* __restrict__ m, const T* __restrict__ m2, const T* __restrict__ w1,
                                                                 const T* __restrict__ w2, const T* __restrict__ g, int width, float eps,
@@ -204,7 +204,7 @@ __global__ void xielu_kernel(const T* __restrict__ in, const T* __restrict__ pq,
 
 // The same, 16 bytes per access. One element at a time it was bound by the vector units (the library's expm1 alone is some 30
 // instructions); 222 million bf16 elements 310 us,
-// here 222 (888 MB), with the error against 64 bits no larger
+// here 194 (888 MB), with the error against 64 bits no larger
 template <typename T>
 __global__ __launch_bounds__(256) void xielu_units_kernel(const T* __restrict__ in, const T* __restrict__ pq, float beta, int64_t units,
                                                           T* __restrict__ out) {

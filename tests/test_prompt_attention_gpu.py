@@ -205,3 +205,31 @@ def test_a_value_that_is_not_finite_stays_with_the_tokens_around_it(d, dv, H, G,
         same[row:row + lens[s]] = ~touched
         assert torch.equal(got[same], clean[same]), (s, j)
         assert not torch.isfinite(got[row:row + lens[s]][sees][:, -1, dv // 2]).any(), (s, j)
+
+
+@pytest.mark.parametrize("page", [64, 128, 256])
+@pytest.mark.parametrize("d,dv", SIZES)
+@pytest.mark.parametrize("H,G,window,sink,gated", [(4, 2, 0, False, False), (8, 1, 70, True, True), (3, 3, 0, True, False), (12, 2, 40, False, True)])
+def test_prompt_kernel_against_float64(d, dv, H, G, window, sink, gated, page):
+    """Rounded to 8 bits: the scaled query, the weights (2^-9 each, which average out over the keys) and the result."""
+    g = torch.Generator(device="cuda").manual_seed(page + H)
+    lens, ctx = [200, 33, 1, 64], [0, 300, 129, 64]
+    n, total = sum(lens), sum(lens) + sum(ctx)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q, K, V = rand(n, H * d).bfloat16(), rand(total, G, d).bfloat16(), rand(total, G, dv).bfloat16()
+    s0, gates = rand(H) if sink else None, rand(n, H * dv).bfloat16() if gated else None
+    got = step(q, K, V, lens, ctx, H, G, d, dv, d ** -0.5, window, sink=s0, gates=gates, page=page).view(n, H, dv).double()
+    want, row, at = torch.empty_like(got), 0, 0
+    for a, c in zip(lens, ctx):
+        k, v = (t[at:at + a + c].double().repeat_interleave(H // G, 1).transpose(0, 1) for t in (K, V))
+        score = q[row:row + a].double().view(a, H, d).transpose(0, 1) @ k.transpose(1, 2).contiguous() * d ** -0.5
+        i, j = torch.arange(c, c + a, device="cuda")[:, None], torch.arange(a + c, device="cuda")
+        score = score.masked_fill((j > i) | (i - j >= window if window else False), -torch.inf)
+        if sink:
+            score = torch.cat([score, s0.double()[:, None, None].expand(H, a, 1)], 2)
+        want[row:row + a] = (score.softmax(2)[..., :a + c] @ v).transpose(0, 1)
+        row, at = row + a, at + a + c
+    if gated:
+        want *= torch.sigmoid(gates.double()).view(n, H, dv)
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
+    assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
