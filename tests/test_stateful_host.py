@@ -578,3 +578,17 @@ def test_scans_refuse_a_workspace_too_small_for_their_segments(address):
     rc = lib.nvs_gated_memory_scan(p, heads * (P + 2 * N + 2), 0, heads * P, heads * (P + N), heads * (P + 2 * N), heads * (P + 2 * N + 1), 0, p, p, 15.0,
                                    1.0, heads, N, P, p, p, p, 1, n, n, p, p, p, p, p, 100, None)
     assert rc != 0 and b"workspace of 100 floats is too small" in lib.nvs_last_error()
+
+
+def test_expert_tile_heights_follow_the_workgroups_they_leave():
+    """Few workgroups: smaller tiles. (width, ff, experts, rows per expert) -> rows of a tile."""
+    from nano_vllm_amd.ops_seq import moe_tile_rows
+    bf, f32 = torch.bfloat16, torch.float32
+    for width, ff, experts, per, dtype, want in [
+            (4096, 3072, 32, 1694, bf, 256), (4096, 3072, 32, 250, bf, 128), (4096, 3072, 32, 32, bf, 64), (4096, 3072, 32, 8, bf, 16),     # the chip is full
+            (2048, 2048, 1, 8000, bf, 256), (2048, 2048, 1, 4000, bf, 128), (2048, 2048, 1, 700, bf, 64), (2048, 2048, 1, 400, bf, 16),
+            (4096, 3072, 2, 100, bf, 16), (8192, 1024, 4, 350, bf, 64), (2048, 512, 8, 2000, bf, 64), (2048, 128, 4, 500, bf, 16),
+            (1024, 768, 32, 68, bf, 64), (1024, 768, 4, 175, bf, 16), (2048, 1024, 2, 350, f32, 16), (2048, 1024, 2, 1000, f32, 64),
+            (1000, 520, 16, 300, bf, 128), (96, 48, 8, 64, bf, 64)]:                                            # rows that are no whole pieces
+        assert moe_tile_rows(per * experts, experts, width, ff, dtype) == want, (width, ff, experts, per, dtype)
+    assert moe_tile_rows(3, 32, 1024, 768, bf) == 16
