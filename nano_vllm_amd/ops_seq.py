@@ -680,7 +680,7 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
         return 64 if per >= 56 else 16
     if per >= 448 and groups(256) >= (270 if ff >= 1024 else 600):
         return 256
-    return 128 if per >= 64 and groups(128) >= (150 if ff >= 1024 else 600) else 64 if per >= 24 else 16
+    return 128 if per >= 64 and groups(128) >= (150 if ff >= 1024 else 1000) else 64 if per >= 24 else 16
 
 
 @_launch
