@@ -236,6 +236,12 @@ int nvs_pool_blocks(const void* k_cache, const void* v_cache, int dtype, int G, 
  * kind 2: no gate at all, gu [n, ff]: out = 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3))). */
 int nvs_glu_act(const void* gu, int64_t stride, int dtype, int ff, int kind, float limit, float alpha, int64_t n, void* out, void* stream);
 
+/* out [m, n] (row stride ldo) = x [m, k] (row stride ldx) times W^T (+ bias [n], nullable), sums in 32-bit, for few rows m: the products of
+ * decode steps and short prompts. act -1: as it is; 2: the GELU of nvs_glu_act's kind 2; 0 and 1: W [2 n, k] holds n gate rows, then n up
+ * rows, out = its gated activation of that kind (no bias). Rows of x and W are whole pieces of 128 bytes on 16-byte boundaries. */
+int nvs_linear_rows(const void* x, int64_t ldx, const void* w, const void* bias, int dtype, int64_t m, int n, int k, int act, float limit,
+                    float alpha, void* out, int64_t ldo, void* stream);
+
 /* Routing of a mixture of experts, 32-bit. z [n, total] (row stride z_stride): router logits of all `total` entries.
  * s = softmax(z) (score 0) or sigmoid(z) (score 1); choice score c = s + correction (NULL: none). Entries form `count` equal groups of neighbours; a group's score
  * is its largest c, and only entries of the `keep` best groups can be chosen. The `top` entries with the largest c are chosen:

@@ -16,14 +16,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
 
 constexpr int MAX_EXPERTS = 1024;
 
-__device__ __forceinline__ float glu_value(float g, float u, int kind, float limit, float alpha) {
-  if (kind == 0) return g / (1.f + expf(-g)) * u;               // silu(g) * u
-  if (kind == 2) return gelu_tanhf_(g);                         // ungated: the tanh form of GELU (u is not read)
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.f + expf(-alpha * g)) * (u + 1.f);              // clamped: g sigmoid(alpha g) (u + 1)
-}
-
 // ungated products: mode 2 squares the positive part (the input rows are then gathered by token, as for a gated product)
 __device__ __forceinline__ float plain_value(float v, int mode) {
   if (mode != 2) return v;

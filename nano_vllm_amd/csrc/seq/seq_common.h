@@ -141,6 +141,14 @@ __device__ __forceinline__ float gelu_tanhf_(float z) {
   return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
+__device__ __forceinline__ float glu_value(float g, float u, int kind, float limit, float alpha) {
+  if (kind == 0) return g / (1.f + expf(-g)) * u;               // silu(g) * u
+  if (kind == 2) return gelu_tanhf_(g);                         // ungated: the tanh form of GELU (u is not read)
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g / (1.f + expf(-alpha * g)) * (u + 1.f);              // clamped: g sigmoid(alpha g) (u + 1)
+}
+
 #define NVS_DISPATCH(dtype, ...)                       \
   do {                                                 \
     if ((dtype) == NVS_BF16) {                         \

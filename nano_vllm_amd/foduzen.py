@@ -22,7 +22,6 @@ recurrence's decay constant (8) and xIELU's linear coefficient (1/2) are fixed b
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -129,7 +128,7 @@ class FoduzenForCausalLM(nn.Module):
             return torch.empty(0, self.config.vocab_size, dtype=self.dtype, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.scalar_norm_rows(x, rows, nrows, self.final_norm, self.config.eps, normed)
-        return F.linear(normed, self.head)
+        return ops_seq.linear(normed, self.head)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------

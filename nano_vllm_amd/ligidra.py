@@ -30,7 +30,6 @@ shapes; the 1e-6 of the unit vectors and the GELU's constants are fixed by the d
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -193,7 +192,7 @@ class LigidraForCausalLM(nn.Module):
             return torch.empty(0, self.config.vocab_size, dtype=self.dtype, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.offset_norm_rows(x, rows, nrows, self.final_norm, self.config.eps, normed, w_off=0.0, a=branch, wa=wa)
-        return F.linear(normed, self.embed)
+        return ops_seq.linear(normed, self.embed)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------

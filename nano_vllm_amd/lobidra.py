@@ -29,7 +29,6 @@ memory's running maximum starting at 0 and the GELU's constants are fixed by the
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -196,7 +195,7 @@ class LobidraForCausalLM(nn.Module):
             return torch.empty(0, self.config.vocab_size, dtype=self.dtype, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.offset_norm_rows(x, rows, nrows, self.final_norm, self.config.eps, normed)
-        return F.linear(normed, self.head)
+        return ops_seq.linear(normed, self.head)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------

@@ -38,8 +38,8 @@
                       pass-through experts, biased logits, optional shared expert with a sigmoid gate per token; or, instead of a router, a
                       table from token ids to experts with equal weights
 
-Every constant a design may change is a constructor argument. Matrix products are the vendor library's (F.linear /
-baddbmm); everything else is a kernel of libnvl_seq.so (ops_seq). Layers read the step's packed-portion description from
+Every constant a design may change is a constructor argument. Matrix products of many rows are the vendor library's
+(F.linear / baddbmm); those of few rows (ops_seq.linear) and everything else are kernels of libnvl_seq.so (ops_seq). Layers read the step's packed-portion description from
 the attention-metadata context (`portions`, `slot_mapping`, `block_tables`); the runner injects the per-layer cache and
 state tensors named by `kv_shapes()` / `state_shapes()`.
 
@@ -208,13 +208,13 @@ class AttentionMixer(nn.Module):
     def forward(self, xh: torch.Tensor, positions: torch.Tensor, values: list | None = None) -> torch.Tensor:
         """values (with v_mix): a list that lives for one step; the first layer that gets it leaves its own values there (and uses them as
         they are), every later one blends them into its own."""
-        proj = F.linear(xh, self.in_w, self.in_b)
+        proj = ops_seq.linear(xh, self.in_w, self.in_b)
         q, k, _ = self.cols
         kv = (proj[:, q:q + k], proj[:, q + k:]) if k else (None, None)
         first = values[0] if values else None
         if values is not None and not values:
             values.append(kv[1])
-        return F.linear(self.attn(proj[:, :q], *kv, None, positions, first), self.o_w)
+        return ops_seq.linear(self.attn(proj[:, :q], *kv, None, positions, first), self.o_w)
 
 
 def rotary_frequencies(dims: int, base: float, scaling: dict | None = None) -> tuple[list[float], float]:
@@ -288,11 +288,11 @@ class ConvAttentionMixer(nn.Module):
     def forward(self, xh: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         por = get_context().portions
         q, c = self.q_cols, self.channels
-        proj = F.linear(xh, self.in_w)
+        proj = ops_seq.linear(xh, self.in_w)
         qk = torch.empty(xh.shape[0], c, dtype=xh.dtype, device=xh.device)
         ops_seq.causal_conv(proj[:, :c], self.conv_w, None, 0, por, self.conv_state, qk)
         k = qk[:, q:]
-        return F.linear(self.attn(qk[:, :q], k, k, proj[:, c:], positions), self.o_w)
+        return ops_seq.linear(self.attn(qk[:, :q], k, k, proj[:, c:], positions), self.o_w)
 
 
 class GatedMemoryCore(nn.Module):
@@ -363,10 +363,10 @@ class AttentionMemoryMixer(nn.Module):
         return out
 
     def forward(self, xh: torch.Tensor, positions: torch.Tensor | None = None):
-        proj = F.linear(xh, self.in_w)
+        proj = ops_seq.linear(xh, self.in_w)
         q, k, v, g, _ = self.cols
         att = self.attn(proj[:, :q], proj[:, q:q + k], proj[:, q + k:q + k + v], proj[:, q + k + v:q + k + v + g])
-        return F.linear(att, self.left_o), F.linear(self.mem(proj, q + k + v + g), self.right_o)
+        return ops_seq.linear(att, self.left_o), ops_seq.linear(self.mem(proj, q + k + v + g), self.right_o)
 
 
 class LatentAttentionMixer(nn.Module):
@@ -428,11 +428,11 @@ class LatentAttentionMixer(nn.Module):
         n, H, d, dr, dv, r = xh.shape[0], self.H, self.d, self.dr, self.dv, self.r
         owner = self._source[0] if self._source else self
         rot = ops_seq.Rotation(self.rot_freq, self.rot_halves, self.rot_mag) if self.rot_freq is not None else None
-        proj = F.linear(xh, self.in_w)
+        proj = ops_seq.linear(xh, self.in_w)
         cq = torch.empty(n, self.qr, dtype=xh.dtype, device=xh.device)
         ops_seq.latent_prep(proj, 0, self.qr, self.q_norm, cq, self.eps, self.kv_col, r, dr, self.kv_norm, positions, rot,
                             owner.block_size, ctx.slot_mapping, owner.k_cache, owner.v_cache)
-        q = F.linear(cq, self.uq).view(n, H, d + dr)
+        q = ops_seq.linear(cq, self.uq).view(n, H, d + dr)
         qf = torch.empty(n, H, r + dr, dtype=xh.dtype, device=xh.device)
         torch.bmm(q[:, :, :d].transpose(0, 1), self.uk, out=qf[:, :, :r].transpose(0, 1))          # W_uk^T q per head
         ops_seq.rotate_heads(q[:, :, d:], qf[:, :, r:], positions, rot)
@@ -442,7 +442,7 @@ class LatentAttentionMixer(nn.Module):
                             lat, gate_per_head=True)
         out = torch.empty(n, H, dv, dtype=xh.dtype, device=xh.device)
         torch.bmm(lat.view(n, H, r).transpose(0, 1), self.uv.transpose(1, 2), out=out.transpose(0, 1))   # W_uv on the latent output
-        return F.linear(out.view(n, H * dv), self.o_w)
+        return ops_seq.linear(out.view(n, H * dv), self.o_w)
 
 
 class DeltaMixer(nn.Module):
@@ -491,19 +491,19 @@ class DeltaMixer(nn.Module):
     def forward(self, xh: torch.Tensor, positions: torch.Tensor | None = None) -> torch.Tensor:
         por = get_context().portions
         n, c = xh.shape[0], self.channels
-        proj = F.linear(xh, self.in_w)
+        proj = ops_seq.linear(xh, self.in_w)
         g_col, a_col = c, c + self.cols[3]
         b_col = a_col + self.cols[4]
         qkv = torch.empty(n, c, dtype=xh.dtype, device=xh.device)
         ops_seq.causal_conv(proj[:, :c], self.conv_w, None, 1, por, self.conv_state, qkv)
-        decays = F.linear(proj[:, a_col:b_col], self.a2) if self.a_rank else None
-        gate = F.linear(proj[:, g_col:a_col], self.g2) if self.g_rank else proj[:, g_col:a_col]
+        decays = ops_seq.linear(proj[:, a_col:b_col], self.a2) if self.a_rank else None
+        gate = ops_seq.linear(proj[:, g_col:a_col], self.g2) if self.g_rank else proj[:, g_col:a_col]
         y = torch.empty(n, self.H * self.dv, dtype=torch.float32, device=xh.device)
         ops_seq.delta_scan(qkv, proj, b_col, 0 if self.a_rank else a_col, decays, self.A_log, self.dt_bias, self.d ** -0.5, self.H, self.G,
                            self.d, self.dv, por, self.rec_state, y)
         out = torch.empty(n, self.H * self.dv, dtype=xh.dtype, device=xh.device)
         ops_seq.gated_group_norm(y, gate, self.norm, self.H, self.eps, out, norm_first=True, silu=not self.g_rank)
-        return F.linear(out, self.o_w)
+        return ops_seq.linear(out, self.o_w)
 
 
 class TokenShiftNorm(nn.Module):
@@ -538,7 +538,7 @@ class TokenSide(nn.Module):
         return {"gate": _copy_into(self.gate), "proj": _copy_into(self.proj), "norm": _copy_into(self.norm)}
 
     def forward(self, xh: torch.Tensor, table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
-        return F.linear(ops_seq.gated_lookup(F.linear(xh, self.gate), table, self.col0, ids), self.proj)
+        return ops_seq.linear(ops_seq.gated_lookup(ops_seq.linear(xh, self.gate), table, self.col0, ids), self.proj)
 
 
 class LightningMixer(nn.Module):
@@ -569,12 +569,12 @@ class LightningMixer(nn.Module):
         por = get_context().portions
         n = xh.shape[0]
         v, k, q, g = self.cols
-        proj = F.linear(xh, self.in_w)
+        proj = ops_seq.linear(xh, self.in_w)
         y = torch.empty(n, v, dtype=torch.float32, device=xh.device)
         ops_seq.decay_scan(proj, 0, v, v + k, self.decay, self.H, self.d, self.dv, por, self.rec_state, y)
         out = torch.empty(n, v, dtype=xh.dtype, device=xh.device)
         ops_seq.gated_group_norm(y, proj[:, v + k + q:], self.norm, 1, self.eps, out, norm_first=True)
-        return F.linear(out, self.o_w)
+        return ops_seq.linear(out, self.o_w)
 
 
 class SSDMixer(nn.Module):
@@ -649,11 +649,11 @@ class ParallelMixer(nn.Module):
         }
 
     def forward(self, xh: torch.Tensor):
-        proj = F.linear(xh, self.in_w, self.in_b)
+        proj = ops_seq.linear(xh, self.in_w, self.in_b)
         q, k, v, g, _ = self.cols
         att = self.attn(proj[:, :q], proj[:, q:q + k], proj[:, q + k:q + k + v], proj[:, q + k + v:q + k + v + g])
-        left = F.linear(att, self.left_o, self.left_o_b)
-        right = F.linear(self.ssd(proj, q + k + v + g), self.right_o)
+        left = ops_seq.linear(att, self.left_o, self.left_o_b)
+        right = ops_seq.linear(self.ssd(proj, q + k + v + g), self.right_o)
         return left, right
 
 
@@ -700,13 +700,13 @@ class RGLRUMixer(nn.Module):
     def forward(self, xh: torch.Tensor) -> torch.Tensor:
         por = get_context().portions
         n, C, bw = xh.shape[0], self.C, self.C // self.blocks
-        proj = F.linear(xh, self.in_w, self.in_b)
+        proj = ops_seq.linear(xh, self.in_w, self.in_b)
         u = torch.empty(n, C, dtype=torch.float32, device=xh.device)
         ops_seq.causal_conv(proj[:, C:], self.conv_w, self.conv_b, 0, por, self.conv_state, u)
         gates = torch.baddbmm(self.gate_b, u.view(n, self.blocks, bw).transpose(0, 1), self.gate_w)     # [blocks, n, 2 bw] fp32
         s = torch.empty(n, C, dtype=xh.dtype, device=xh.device)
         ops_seq.rglru_scan(gates, u, proj[:, :C], self.lam, self.c, self.blocks, por, self.rec_state, s)
-        return F.linear(s, self.o_w)
+        return ops_seq.linear(s, self.o_w)
 
 
 class XIELUFeedForward(nn.Module):
@@ -719,7 +719,7 @@ class XIELUFeedForward(nn.Module):
         return {"up": _copy_into(self.up), "down": _copy_into(self.down), "act": _copy_into(self.act)}
 
     def forward(self, xh: torch.Tensor) -> torch.Tensor:
-        return F.linear(ops_seq.xielu(F.linear(xh, self.up), self.act, self.beta), self.down)
+        return ops_seq.linear(ops_seq.xielu(ops_seq.linear(xh, self.up), self.act, self.beta), self.down)
 
 
 class GeluFeedForward(nn.Module):
@@ -733,10 +733,7 @@ class GeluFeedForward(nn.Module):
         return {"up": _copy_into(self.up), "down": _copy_into(self.down)}
 
     def forward(self, xh: torch.Tensor) -> torch.Tensor:
-        z = F.linear(xh, self.up)
-        act = torch.empty_like(z)
-        ops_seq.glu_act(z, self.ff, act, kind=2)
-        return F.linear(act, self.down)
+        return ops_seq.linear(ops_seq.linear_act(xh, self.up, self.ff, kind=2), self.down)
 
 
 class SiluGLU(nn.Module):
@@ -750,9 +747,7 @@ class SiluGLU(nn.Module):
         return {"gate": _copy_into(self.gu[:self.ff]), "up": _copy_into(self.gu[self.ff:]), "down": _copy_into(self.down)}
 
     def forward(self, xh: torch.Tensor) -> torch.Tensor:
-        act = torch.empty(xh.shape[0], self.ff, dtype=xh.dtype, device=xh.device)
-        ops_seq.glu_act(F.linear(xh, self.gu), self.ff, act, kind=0)
-        return F.linear(act, self.down)
+        return ops_seq.linear(ops_seq.linear_act(xh, self.gu, self.ff), self.down)
 
 
 class BranchNorm(nn.Module):
@@ -784,10 +779,7 @@ class ClampedGLU(nn.Module):
         return {"gate": _copy_into(self.gu[:self.ff]), "up": _copy_into(self.gu[self.ff:]), "down": _copy_into(self.down)}
 
     def forward(self, xh: torch.Tensor) -> torch.Tensor:
-        gu = F.linear(xh, self.gu)
-        act = torch.empty(xh.shape[0], self.ff, dtype=xh.dtype, device=xh.device)
-        ops_seq.glu_act(gu, self.ff, act, kind=1, limit=self.limit, alpha=self.alpha)
-        return F.linear(act, self.down)
+        return ops_seq.linear(ops_seq.linear_act(xh, self.gu, self.ff, kind=1, limit=self.limit, alpha=self.alpha), self.down)
 
 
 class RoutedExperts(nn.Module):
@@ -865,9 +857,8 @@ class RoutedExperts(nn.Module):
         ops_seq.moe_gemm(act, self.w_down, plan, False, rows)
         shared = gate = None
         if self.shared_ff:
-            sact = torch.empty(n, self.shared_ff, dtype=xh.dtype, device=xh.device)
-            ops_seq.glu_act(F.linear(xh, self.s_gu), self.shared_ff, sact, kind=0)
-            shared, gate = F.linear(sact, self.s_down), (z[:, total:] if self.shared_gate else None)
+            shared = ops_seq.linear(ops_seq.linear_act(xh, self.s_gu, self.shared_ff), self.s_down)
+            gate = z[:, total:] if self.shared_gate else None
         return rows, plan, wts, shared, gate
 
     def forward(self, xh: torch.Tensor, tokens: torch.Tensor | None = None, res: torch.Tensor | None = None) -> torch.Tensor:

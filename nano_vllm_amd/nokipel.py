@@ -27,7 +27,6 @@ All sizes, the layer order and the design's free constants come from config.json
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -179,7 +178,7 @@ class NokipelForCausalLM(nn.Module):
             return torch.empty(0, self.config.vocab_size, dtype=self.dtype, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.group_norm_rows(x, rows, nrows, self.final_norm, self.config.norm_groups, self.config.eps, normed)
-        return F.linear(normed, self.head)
+        return ops_seq.linear(normed, self.head)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------

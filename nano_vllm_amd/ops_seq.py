@@ -57,6 +57,7 @@ SIGNATURES = {
     "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _L, _P]),
     "nvs_rotate_heads": (c_int, [_P, _L, _I, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _L, _P]),
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
+    "nvs_linear_rows": (c_int, [_P, _L, _P, _P, _I, _L, _I, _I, _I, _F, _F, _P, _L, _P]),
     "nvs_moe_route": (c_int, [_P, _L, _P, _L, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P]),
     "nvs_moe_rows": (c_int64, [_L, _I, _I]),
     "nvs_moe_plan": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P]),
@@ -615,6 +616,51 @@ def glu_act(gu: torch.Tensor, ff: int, out: torch.Tensor, kind: int = 0, limit: 
     n = gu.shape[0]
     assert gu.shape[1] == (1 if kind == 2 else 2) * ff and gu.stride(1) == 1 and out.shape == (n, ff) and out.is_contiguous()
     _check(lib.nvs_glu_act(_ptr(gu), gu.stride(0), _same(gu, out), ff, kind, limit, alpha, n, _ptr(out), _stream()))
+
+
+def _few_rows(x: torch.Tensor, w: torch.Tensor, glu: bool) -> bool:
+    """Whether x w^T goes to nvs_linear_rows: whole 128-byte pieces of k, few rows and not too many of w. MI355X, us here / the library's, bf16: 64 rows,
+    1024 x 1024 3.6 / 8.6, 1024 x 3072 4.9 / 10.0, 4096 x 1024 4.5 / 8.6, 4096 x 4096 12.3 / 14.7, 6144 x 1024 5.8 / 8.8, 12288 x 2048 13.8 / 12.9,
+    24576 x 4096 54.8 / 47.9; 256 rows, 1024 x 1024 4.2 / 8.3, 4096 x 4096 19.5 / 22.2, 6144 x 1024 12.8 / 12.3; 128 rows of it 7.5 / 9.5; 16 rows,
+    12288 x 2048 11.7 / 11.6, 32768 x 4096 51.9 / 62.6. The activation on the way saves its launch (4 us and its passes): more is taken. 32-bit: 330 rows,
+    1024 x 1024 10.3 / 11.8, 4096 x 1024 33.6 / 41.3, 3084 x 1024 30.9 / 23.8; 512 rows, 1024 x 2048 21.3 / 21.5, 4096 x 1024 42.9 / 36.2."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        return False
+    m, k = x.shape
+    n = w.shape[0]
+    if w.dtype == torch.bfloat16:
+        if k % 64 or x.stride(0) % 8 or not (m <= 16 or m <= 256 and n <= 4096 or m <= 128 and n <= 6144 or
+                                             glu and (m <= 32 or m * n <= 64 * 12288 or m <= 256 and n <= 8192)):
+            return False
+    elif w.dtype != torch.float32 or k % 32 or x.stride(0) % 4 or not (m <= 16 or m <= 512 and n <= 2048 or m <= 384 and n <= (6144 if glu else 4096)):
+        return False
+    return w.is_cuda and x.dtype == w.dtype and x.stride(1) == 1 and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+def _linear_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act: int, limit: float, alpha: float, out: torch.Tensor) -> torch.Tensor:
+    lib = load_library()
+    m, k = x.shape
+    _check(lib.nvs_linear_rows(_ptr(x), x.stride(0), _ptr(w), _ptr(b), _same(x, w, b, out), m, out.shape[1], k, act, limit, alpha, _ptr(out),
+                               out.stride(0), _stream()))
+    return out
+
+
+@_launch
+def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
+    """x [n, K] times w [N, K]^T (+ b): few rows here, many by the vendor library."""
+    if not _few_rows(x, w, False) or not (b is None or b.dtype == x.dtype and b.is_contiguous() and b.shape == w.shape[:1]):
+        return torch.nn.functional.linear(x, w, b)
+    return _linear_rows(x, w, b, -1, 0.0, 0.0, torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device))
+
+
+@_launch
+def linear_act(x: torch.Tensor, w: torch.Tensor, ff: int, kind: int = 0, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
+    """glu_act of x times w^T, w [2 ff, K] = [gate | up] (kind 2: [ff, K])."""
+    out = torch.empty(x.shape[0], ff, dtype=x.dtype, device=x.device)
+    if _few_rows(x, w, True):
+        return _linear_rows(x, w, None, kind, limit, alpha, out)
+    glu_act(torch.nn.functional.linear(x, w), ff, out, kind, limit, alpha)
+    return out
 
 
 @_launch

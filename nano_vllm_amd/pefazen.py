@@ -33,7 +33,6 @@ rotations is fixed by the design.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -167,7 +166,7 @@ class PefazenForCausalLM(nn.Module):
             return torch.empty(0, cfg.vocab_size, dtype=torch.float32, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.group_norm_rows(x, rows, nrows, self.final_norm, 1, cfg.eps, normed, center=True)
-        return ops_seq.scale_softcap(F.linear(normed, self.head), cfg.logit_scale, cfg.logit_softcap)
+        return ops_seq.scale_softcap(ops_seq.linear(normed, self.head), cfg.logit_scale, cfg.logit_softcap)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------

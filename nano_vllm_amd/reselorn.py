@@ -24,7 +24,6 @@ Sizes, the layer order and free constants come from config.json; the rule of the
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import ops_seq
@@ -157,7 +156,7 @@ class ReselornForCausalLM(nn.Module):
             return torch.empty(0, self.config.vocab_size, dtype=self.dtype, device=x.device)
         normed = torch.empty(nrows, x.shape[1], dtype=self.dtype, device=x.device)
         ops_seq.offset_norm_rows(x, rows, nrows, self.final_norm, self.config.eps, normed, w_off=0.0)
-        return F.linear(normed, self.embed)
+        return ops_seq.linear(normed, self.embed)
 
 
 # ---- synthetic checkpoints (tests, benchmarks, dummy weights) -----------------------------------------------------------
