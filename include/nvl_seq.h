@@ -250,6 +250,15 @@ int nvs_linear_rows(const void* x, int64_t ldx, const void* w, const void* bias,
 int nvs_moe_route(const float* z, int64_t z_stride, const float* correction, int64_t n, int total, int top, int count, int keep, float scale,
                   int score, int renorm, int32_t* ids, float* wts, void* stream);
 
+/* nvs_moe_route on logits of its own: z = x router^T (+ bias) in 32-bit, x [n, k] (`dtype`, row stride ldx), router [entries, k] 32-bit, up to 64
+ * entries. entries == total + 1: the last one is the pre-activation of the shared expert's gate, gate [n]. Rows of x and of the router are whole
+ * 128-byte pieces of x's type (k % 64 == 0 in bf16, k % 32 == 0 in 32-bit) on 16-byte boundaries. ws: nvs_moe_router_workspace floats on a 16-byte boundary, with which several
+ * workgroups share a row's reduction where rows are few (NULL: none do). */
+int64_t nvs_moe_router_workspace(int64_t n, int entries, int k, int dtype);
+int nvs_moe_router(const void* x, int64_t ldx, int dtype, const float* router, const float* bias, int entries, int k, const float* correction, int64_t n,
+                   int total, int top, int count, int keep, float scale, int score, int renorm, int32_t* ids, float* wts, float* gate, float* ws,
+                   int64_t ws_floats, void* stream);
+
 /* Routing without a router: ids[t, k] = table[tokens[t], k] (table [vocab, top], int32; a row's entries differ), wts[t, k] = weight. */
 int nvs_moe_table_route(const int64_t* tokens, const int32_t* table, int64_t n, int top, float weight, int32_t* ids, float* wts, void* stream);
 

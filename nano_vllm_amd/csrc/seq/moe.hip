@@ -1,7 +1,7 @@
 // Gated feed-forward activations and routed mixtures of experts.
 //
-// A routed layer runs as: router logits (a 32-bit library product) -> route kernel (softmax, choice scores, group limit,
-// top-k, weights) -> plan kernel (pairs (token, choice) sorted by expert into row tiles, every expert's rows padded to a whole
+// A routed layer runs as: router (moe_router.hip: 32-bit logits, softmax, choice scores, group limit,
+// top-k, weights; past 64 entries a 32-bit library product and the route kernel here) -> plan kernel (pairs (token, choice) sorted by expert into row tiles, every expert's rows padded to a whole
 // tile) -> grouped product gate|up with the activation in its epilogue -> grouped product down -> combine kernel (weighted sum
 // of a token's choices, pass-through experts, the gated shared expert). Nothing comes back to the host in between, so the
 // sequence can be captured in a hipGraph; the order in which pairs land inside an expert's rows is arbitrary but no sum depends

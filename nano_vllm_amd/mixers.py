@@ -844,21 +844,20 @@ class RoutedExperts(nn.Module):
         gate or None). wide: the layer's input in 32-bit, for the router (default: xh)."""
         n, width = xh.shape
         total = self.E + self.ident
+        gate = None
         if self.table_vocab:
-            z = None
             ids, wts = ops_seq.moe_table_route(tokens, self.table, 1.0 / self.top)
-        else:
-            z = F.linear(wide if wide is not None else xh.float(), self.router, self.router_b)      # 32-bit, [n, total (+ 1: the shared gate)]
-            ids, wts = ops_seq.moe_route(z, total, self.correction, self.top, self.count, self.keep, self.scale, self.sigmoid, self.renorm)
+        else:                                     # 32-bit logits, [n, total (+ 1: the shared gate)]
+            ids, wts, gate = ops_seq.moe_router(wide if wide is not None else xh, self.router, self.router_b, total, self.correction, self.top,
+                                                self.count, self.keep, self.scale, self.sigmoid, self.renorm)
         plan = ops_seq.moe_plan(ids, self.E, ops_seq.moe_tile_rows(n * self.top, self.E, width, self.ff, xh.dtype))
         act = torch.empty(plan.cap, self.ff, dtype=xh.dtype, device=xh.device)
         ops_seq.moe_gemm(xh, self.w_gu, plan, self.gated, act, relu2=not self.gated)
         rows = torch.empty(plan.cap, width, dtype=xh.dtype, device=xh.device)
         ops_seq.moe_gemm(act, self.w_down, plan, False, rows)
-        shared = gate = None
+        shared = None
         if self.shared_ff:
             shared = ops_seq.linear(ops_seq.linear_act(xh, self.s_gu, self.shared_ff), self.s_down)
-            gate = z[:, total:] if self.shared_gate else None
         return rows, plan, wts, shared, gate
 
     def forward(self, xh: torch.Tensor, tokens: torch.Tensor | None = None, res: torch.Tensor | None = None) -> torch.Tensor:

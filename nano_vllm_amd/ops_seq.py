@@ -59,6 +59,8 @@ SIGNATURES = {
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
     "nvs_linear_rows": (c_int, [_P, _L, _P, _P, _I, _L, _I, _I, _I, _F, _F, _P, _L, _P]),
     "nvs_moe_route": (c_int, [_P, _L, _P, _L, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P]),
+    "nvs_moe_router": (c_int, [_P, _L, _I, _P, _P, _I, _I, _P, _L, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P, _L, _P]),
+    "nvs_moe_router_workspace": (c_int64, [_L, _I, _I, _I]),
     "nvs_moe_rows": (c_int64, [_L, _I, _I]),
     "nvs_moe_plan": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P]),
     "nvs_moe_plan_scratch": (c_int64, [_L, _I]),
@@ -677,6 +679,35 @@ def moe_route(z: torch.Tensor, total: int, correction: torch.Tensor | None, top:
     _check(lib.nvs_moe_route(_ptr(z), z.stride(0), _ptr(correction), n, total, top, count, keep, scale, int(sigmoid), int(renorm), _ptr(ids),
                              _ptr(wts), _stream()))
     return ids, wts
+
+
+@_launch
+def moe_router(x: torch.Tensor, router: torch.Tensor, bias: torch.Tensor | None, total: int, correction: torch.Tensor | None, top: int, count: int,
+               keep: int, scale: float, sigmoid: bool = False, renorm: bool = True):
+    """moe_route of the 32-bit logits x router^T (+ bias); a router of total + 1 rows ends with the shared expert's gate. Returns
+    (ids, weights, gate [n, 1] or None). One kernel for up to 64 entries (48 beside 32-bit rows, whose products take five times the matrix pipe's time)
+    and rows of whole 128-byte pieces. MI355X, us, copy + library product + moe_route / here, 33 entries, k 1024 and 4096: bf16, 64 rows 17 / 9 and
+    20 / 13, 2000 rows 23 / 9 and 37 / 17, 13,550 rows 58 / 14 and 138 / 30; 32-bit, 64 rows 12.7 / 10.7 and 16.6 / 15.2, 13,550 rows 43 / 24 and
+    88 / 68 (64 entries 42 / 35 and 87 / 97)."""
+    n, k = x.shape
+    entries = router.shape[0]
+    assert router.dtype == torch.float32 and router.shape[1] == k and total <= entries <= total + 1
+    if entries > (64 if x.dtype == torch.bfloat16 else 48) or k % (64 if x.dtype == torch.bfloat16 else 32) or x.stride(1) != 1 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16 \
+            or not router.is_contiguous() or router.data_ptr() % 16 or not (bias is None or bias.is_contiguous()) or n == 0:
+        z = torch.nn.functional.linear(x.float(), router, bias)
+        ids, wts = moe_route(z, total, correction, top, count, keep, scale, sigmoid, renorm)
+        return ids, wts, z[:, total:] if entries > total else None
+    lib = load_library()
+    assert bias is None or (bias.dtype == torch.float32 and bias.numel() == entries)
+    assert correction is None or (correction.dtype == torch.float32 and correction.numel() == total and correction.is_contiguous())
+    ids = torch.empty(n, top, dtype=torch.int32, device=x.device)
+    wts = torch.empty(n, top, dtype=torch.float32, device=x.device)
+    gate = torch.empty(n, 1, dtype=torch.float32, device=x.device) if entries > total else None
+    need = lib.nvs_moe_router_workspace(n, entries, k, _code(x))
+    ws = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+    _check(lib.nvs_moe_router(_ptr(x), x.stride(0), _code(x), _ptr(router), _ptr(bias), entries, k, _ptr(correction), n, total, top, count, keep, scale,
+                              int(sigmoid), int(renorm), _ptr(ids), _ptr(wts), _ptr(gate), _ptr(ws), need, _stream()))
+    return ids, wts, gate
 
 
 @_launch
