@@ -233,6 +233,7 @@ __global__ void window_attn_kernel(const WindowAttnArgs A) {
 }
 }  // namespace
 
+int window_attn_token(const WindowAttnArgs& a, hipStream_t stream);          // attn_token.hip
 void window_attn_extended(const WindowAttnArgs& a, hipStream_t stream);      // attn_pool.hip
 
 static int g_force_scalar = 0, g_no_lds = 0, g_packed_heads = 1;
@@ -309,20 +310,21 @@ extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnor
   a.q_row = q_row, a.pool_k = pool_k, a.pool_v = pool_v, a.pool = pool, a.softcap = softcap;
   if (dtype == NVS_BF16 && d % 8 == 0 && d <= 256 && dv <= 256 && block_size % 8 == 0 && !g_force_scalar) {
     const bool extended = q_row || pool > 0 || softcap > 0.f;
-    // The pipelined kernel for the sizes it is built for, whenever its tiles lie in one page and its 16-byte pieces are aligned. It is the faster one
-    // from a single token (16 query heads on 8 kv heads of 128 behind 900 tokens: 31 us against 50; 64 such sequences 49 against 80; latent
-    // rows 68 against 89) to whole prompts (attn_prompt.h); the others take every other size.
-    // Steps of single tokens with eight or more query heads per kv head (`packed`: the other kernel's query tiles hold heads) are its only while its
-    // workgroups run at once, two on a compute unit, one of latent rows or with capped scores, where the vector units have no time left: its queries
-    // are positions, so four (eight) heads each read all keys, and one of a wavefront's 32 queries lives. us by packed heads / here, contexts of
-    // 2,500: 64 heads over one kv head of 128, 24 / 32 / 36 / 48 sequences 110 / 92, 112 / 103, 113 / 132, 114 / 150; 8 heads over each of two, 128 / 144 /
-    // 224 126 / 116, 140 / 151, 161 / 217; latent rows, 16 heads, 96 / 128 / 136 / 192 184 / 134, 190 / 175, 191 / 265, 201 / 290; capped, contexts of
-    // 1,500, 8 heads over each of four, 16 / 32 / 64 91 / 80, 93 / 83, 99 / 126.
-    const bool sizes = (d == 128 && dv == 128) || (d == 256 && dv == 192 && !extended);
+    // Steps of single tokens go to the kernel whose wavefronts share a token's keys (attn_token.hip: 1.1 to 5 times as fast for every number of heads,
+    // tokens and sequences measured there), unless there are pooled blocks.
+    // The pipelined kernel for the sizes it is built for, whenever its tiles lie in one page and its 16-byte pieces are aligned: it is the faster one up
+    // to whole prompts (attn_prompt.h); the others take every other size.
+    // Steps of single tokens with pooled blocks, or of few tokens each, with eight or more query heads per kv head (`packed`: the other kernel's query tiles
+    // hold heads) are its only while its workgroups run at once, two on a compute unit, one of latent rows or with capped scores, where the vector units
+    // have no time left: its queries are positions, so four (eight) heads each read all keys, and one of a wavefront's 32 queries lives. us by packed
+    // heads / here, single tokens capped, contexts of 1,500, 8 heads over each of four, 16 / 32 / 64 sequences 91 / 80, 93 / 83, 99 / 126.
+    const bool built = (d == 128 && dv == 128) || (d == 256 && dv == 192), sizes = built && (d == 128 || !extended);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)qnorm | (uintptr_t)pool_k | (uintptr_t)pool_v) & 15) == 0 &&
                          q_stride % 8 == 0 && ((uintptr_t)out & 7) == 0;
     const PromptGrid grid = prompt_grid(a, d == 128 ? 4 : 8);
     const bool packed = H / G >= 8 && n < 32ll * nseq && 4 * n <= (int64_t)nseq * (H / G) && grid.tiles * grid.rows > (d == 128 && !(softcap > 0.f) ? 512 : 256);
+    if (built && aligned && n <= nseq && pool == 0 && block_size >= 32 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
+      return window_attn_token(a, (hipStream_t)stream);
     if (sizes && aligned && !packed && block_size >= 64 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
       return extended ? window_attn_prompt_extended(a, (hipStream_t)stream) : window_attn_prompt(a, (hipStream_t)stream);
     if (extended) window_attn_extended(a, (hipStream_t)stream);
