@@ -122,7 +122,7 @@ struct __attribute__((aligned(16))) PlanEntry { int32_t b, h, t0, nb; };   // fi
 __global__ __launch_bounds__(256) void decode_plan_kernel(const int32_t* __restrict__ ctx, int batch, int hkv, int nwaves,
                                                           PlanHeader* __restrict__ hdr,
                                                           const int32_t* __restrict__ shared_blocks, int tiles_per_block,
-                                                          int px_groups) {
+                                                          int px_groups, int* __restrict__ arrived) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   int* wsum = reinterpret_cast<int*>(smem_raw);
   int* pre = wsum + kWaves;
@@ -130,6 +130,8 @@ __global__ __launch_bounds__(256) void decode_plan_kernel(const int32_t* __restr
   // common. Whatever it says, the tile that takes a member's NEW token stays in that sequence's own share (the stream-K
   // kernel stores the token and starts its softmax there): sh <= min over live members of floor((len - 1) / 32).
   int sh = 0;
+  if (arrived != nullptr)                                 // (decode_few_kernel's counters)
+    for (int i = threadIdx.x; i < batch * hkv; i += 256) arrived[i] = 0;
   const int32_t* member = shared_blocks != nullptr ? shared_blocks + 1 : nullptr;
   if (shared_blocks != nullptr) {
     int* smin = pre + batch + 1;                        // (one more int of the dynamic region: the launcher sizes it)
@@ -1564,6 +1566,314 @@ __global__ __launch_bounds__(128) void decode_stream_combine_kernel(const float*
   if (lse != nullptr && d == 0) lse[row] = cnt > 0 ? 0.6931471805599453f * (M + log2f(den)) : -INFINITY;
 }
 
+// ---------------------------------------------------------------------------------------------------
+// Steps of few sequences (fused form, bf16 cache, group sizes 2 ... 16). The stream-K launch above cuts the step into equal shares
+// whatever its size, so with one sequence of 700 tokens every pair (sequence, kv head) is spread over six wavefronts of different
+// workgroups: split partials through memory, and a merge launch behind (11.5 + 4.3 us). Here a workgroup of eight wavefronts takes a pair, or
+// 1,024 tokens and more of it where the context is longer ("parts"), its wavefronts take every eighth tile of 32 tokens, and the split is merged in LDS: one
+// launch, and nothing but a long context's parts goes through memory. Those are merged by the part that arrives last (a counter in the
+// step's plan, set to 0 by nvl_decode_plan and again by the last one); without a plan by a launch of their own, in the same order and arithmetic.
+//
+// Tiles go memory -> LDS directly, into a place per wavefront that is requested again as soon as its operands are in registers. Same matrix
+// operands as mfma8_body; K slots are swizzled by row & 15, V slots by 2 (row & 7) (the direct path cannot write padding): both kinds of operand reads touch all
+// banks once. What bounds it: one chain of latencies (context length -> rotation and tile -> scores -> merge), and 28 bytes a clock that a compute unit
+// takes in.
+constexpr int kFewWaves = 8, kFewTile = kTile * 512, kFewPart = 32, kFewGroups = 512;       // bytes of a wave's K and V tile; tiles of a part; workgroups of a launch
+
+// Parts of a context of max_context tokens, while the workgroups (most of which leave at once when contexts are shorter) are few; 0: the stream-K kernel
+// takes the step, whose tile loads run ahead and fill the chip at 5.4 to 6.1 TB/s. us, stream-K with its merge / here, 16 heads over 8 kv heads, max_context 4,096: one
+// sequence of 100 tokens 11.5 / 6.2, 700 11.9 / 9.7, 2,000 14.1 / 12.7, 4,096 14.8 / 13.5; 4 and 16 sequences of 100 to 2,047 13.9 / 11.5, 22.6 / 18.1, 16 of 3,000 to
+// 4,096 42.9 / 40.3; max_context 32,768, two of 20,000 to 32,000 58 / 45; 64 sequences, one kv head, 6,000 to 8,000 of 8,192 50 / 42. Beyond 512 workgroups: 24 sequences
+// of 4,096 47.1 / 47.7, 64 of 3,000 to 4,096 153 / 179, 128 of 2,047 103 / 125. More than 16 sequences stay there too, with one kv head 64 of 3,000 to 4,000
+// 31 / 24: a step with a plan for a shared prefix that turns out to have none gives the bits of a step without.
+inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
+  const int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart;
+  return batch <= 16 && batch * hkv * parts <= kFewGroups ? (int)parts : 0;
+}
+
+// parts of a context of `tiles` tiles
+__device__ __forceinline__ int few_split(int tiles, int parts) {
+  const int n = (tiles + kFewPart - 1) / kFewPart;
+  return n < 1 ? 1 : n < parts ? n : parts;
+}
+
+// partials go through to memory and are read from there (another workgroup's L2 may be another one)
+__device__ __forceinline__ void few_put(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float few_get(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// output row (b, head) from its n partials, dim d (and its log-sum-exp); eight partials requested at once
+__device__ __forceinline__ void few_merge(const float* part_o, const float* part_ml, int64_t row, int n, int slots, int d, bf16_t* out, float* lse) {
+  const float* ml = part_ml + row * slots * 2;
+  const float* po = part_o + row * slots * 128 + d;
+  float M = kNegBig, num = 0.f, den = 0.f;
+  for (int k0 = 0; k0 < n; k0 += 8) {
+    float m[8], l[8], o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = k0 + j < n ? k0 + j : n - 1;
+      m[j] = few_get(ml + k * 2), l[j] = few_get(ml + k * 2 + 1), o[j] = few_get(po + (int64_t)k * 128);
+    }
+    float top = M;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
+    const float r = exp2f(M - top);
+    num *= r, den *= r, M = top;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k0 + j < n) {
+        const float f = exp2f(m[j] - M);
+        num += f * o[j];
+        den += f * l[j];
+      }
+  }
+  out[row * 128 + d] = (bf16_t)(num / den);
+  if (lse != nullptr && d == 0) lse[row] = 0.6931471805599453f * (M + log2f(den));
+}
+
+template <bool SLABS>
+__global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
+    const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc, const int32_t* __restrict__ block_tables, int64_t bt_stride,
+    const int32_t* __restrict__ ctx, float* part_o, float* part_ml, bf16_t* __restrict__ out, int batch, int hkv, int block_size, int slots,
+    float scale_log2e, FusedArgs fa, int* arrived, int Gv, int parts, float* __restrict__ lse) {
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  typedef const __attribute__((address_space(1))) void global_void_t;
+  extern __shared__ __attribute__((aligned(128))) unsigned char smem_raw[];           // tiles; q rows [16][256], new k, new v; (m, l) [wave][16]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane & 15, rq = lane >> 4, head = lane & 15, quad = lane >> 4;
+  const int pairs = batch * hkv, part = blockIdx.x / pairs, pair = blockIdx.x % pairs, b = pair / hkv, h = pair % hkv, hq = hkv * Gv;
+  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = few_split(tiles, parts), per = (tiles + n - 1) / n;
+  if (part >= n) return;
+  if (len <= 0) {                                  // graph padding: zero rows
+    for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves) out[((int64_t)b * hq + h * Gv) * 128 + i] = (bf16_t)0.f;
+    if (lse != nullptr && threadIdx.x < Gv) lse[(int64_t)b * hq + h * Gv + threadIdx.x] = -INFINITY;
+    return;
+  }
+  const int t0 = part * per, t1 = min(tiles, t0 + per), len_cached = len - 1;
+  unsigned char* k_lds = smem_raw + wave * kFewTile;
+  unsigned char* v_lds = k_lds + kTile * 256;
+  unsigned char* stage = smem_raw + kFewWaves * kFewTile;
+  float2* ml = reinterpret_cast<float2*>(stage + 18 * 256);
+
+  // ---- what the rows need is requested before the tiles (what has landed is counted in order): wave w < 4 prepares heads 4 w .. 4 w + 3, the last
+  // one the new token's k and v
+  const bool owns_new = t1 == tiles, q_wave = wave * 4 < Gv, kv_wave = owns_new && wave == kFewWaves - 1;
+  const int64_t row_e = (int64_t)b * fa.qkv_tok_stride;
+  u32x4_t raw = {0u, 0u, 0u, 0u}, vnew = {0u, 0u, 0u, 0u}, wraw = {0u, 0u, 0u, 0u};
+  RopeRegs rr = {};
+  if (q_wave || kv_wave) {
+    const int64_t pos = len - 1 >= fa.max_pos ? fa.max_pos - 1 : len - 1;
+    rr = load_rope_regs(fa.cos_sin + pos * 128, sub);
+    if (fa.q_norm_w != nullptr) wraw = *reinterpret_cast<const u32x4_t*>((kv_wave ? fa.k_norm_w : fa.q_norm_w) + sub * 8);
+    if (kv_wave) {
+      raw = load_qkv8<SLABS>(q, row_e + (hq + h) * 128 + sub * 8, fa);
+      vnew = load_qkv8<SLABS>(q, row_e + (hq + hkv + h) * 128 + sub * 8, fa);
+    } else if (rq + 4 * wave < Gv) {
+      raw = load_qkv8<SLABS>(q, row_e + (h * Gv + rq + 4 * wave) * 128 + sub * 8, fa);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // ---- tiles: request i covers 4 token rows; lane l brings 16-byte slot (l & 15) ^ swizzle of row l >> 4
+  uint32_t koff[8], voff[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = i * 4 + rq;
+    koff[i] = (uint32_t)(r * 256 + ((sub ^ (r & 15)) << 4));
+    voff[i] = (uint32_t)(r * 256 + ((sub ^ (2 * (r & 7))) << 4));
+  }
+  const auto block_of = [&](int ti) { return block_tables[(int64_t)b * bt_stride + ti * kTile / block_size]; };
+  const auto request = [&](int ti, int blk) {
+    const int64_t base = (((int64_t)blk * hkv + h) * block_size + ti * kTile % block_size) * 256;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      __builtin_amdgcn_global_load_lds((global_void_t*)((const unsigned char*)kc + base + koff[i]), (lds_void_t*)(k_lds + i * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      __builtin_amdgcn_global_load_lds((global_void_t*)((const unsigned char*)vc + base + voff[i]), (lds_void_t*)(v_lds + i * 1024), 16, 0, 0);
+  };
+  int ti = t0 + wave, blk = ti < t1 ? block_of(ti) : 0;
+  if (ti < t1) request(ti, blk);
+  if (ti + kFewWaves < t1) blk = block_of(ti + kFewWaves);
+
+  if (q_wave || kv_wave) {
+    const u32x4_t row = norm_rope_head_regs(raw, fa.q_norm_w != nullptr, wraw, fa.eps, rr, sub);
+    if (kv_wave) {
+      if (rq == 0) {                               // one 256-byte row each, for later steps and for this one
+        const int blk_new = block_tables[(int64_t)b * bt_stride + (len - 1) / block_size];
+        const int64_t dst = (((int64_t)blk_new * hkv + h) * block_size + (len - 1) % block_size) * 128 + sub * 8;
+        *reinterpret_cast<u32x4_t*>(kc + dst) = row;
+        *reinterpret_cast<u32x4_t*>(vc + dst) = vnew;
+        *reinterpret_cast<u32x4_t*>(stage + 16 * 256 + sub * 16) = row;
+        *reinterpret_cast<u32x4_t*>(stage + 17 * 256 + sub * 16) = vnew;
+      }
+    } else {
+      *reinterpret_cast<u32x4_t*>(stage + (rq + 4 * wave) * 256 + sub * 16) = row;
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): the rows are written (and the tiles keep coming)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8_t qb[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    u32x4_t w = {0u, 0u, 0u, 0u};
+    if (head < Gv) w = *reinterpret_cast<const u32x4_t*>(stage + head * 256 + (4 * c + quad) * 16);
+    qb[c] = __builtin_bit_cast(bf16x8_t, w);
+  }
+  float m_run = kNegBig, l_run = 0.f;
+  f32x4_t oacc[8];
+#pragma unroll
+  for (int db = 0; db < 8; ++db) oacc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (kv_wave) {
+    // the new token is the first key of this wave: m = its score, l = 1 counted once per head, O = v (its cache row is never read inside this launch)
+    f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      u32x4_t w = {0u, 0u, 0u, 0u};
+      if (head == 0) w = *reinterpret_cast<const u32x4_t*>(stage + 16 * 256 + (4 * c + quad) * 16);      // row 0 of the operand; the others are 0
+      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), qb[c], s, 0, 0, 0);
+    }
+    m_run = __shfl(s[0], head, 64) * scale_log2e;
+    l_run = quad == 0 ? 1.f : 0.f;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      const u32x2_t w = *reinterpret_cast<const u32x2_t*>(stage + 17 * 256 + (16 * db + 4 * quad) * 2);
+      oacc[db] = f32x4_t{bf16lo_to_f32(w[0]), bf16hi_to_f32(w[0]), bf16lo_to_f32(w[1]), bf16hi_to_f32(w[1])};
+    }
+  }
+  int kfrag[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) kfrag[c] = head * 256 + (((4 * c + quad) ^ head) << 4);
+  const int vrow = 4 * quad + (head >> 2), vbase = vrow * 256 + (head & 3) * 8;
+  constexpr float kHidden = -3e38f;                // below any running maximum: weighs 0 also where a wave has seen nothing yet
+#pragma unroll 1
+  for (; ti < t1; ti += kFewWaves) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): the tile landed
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8_t kf[2][4];
+    s16x4_t vf[8][2];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) kf[hf][c] = *reinterpret_cast<const bf16x8_t*>(k_lds + hf * 16 * 256 + kfrag[c]);
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      const unsigned char* p0 = v_lds + vbase + ((db ^ (vrow & 7)) << 5);
+      vf[db][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p0));
+      vf[db][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p0 + 16 * 256));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);            // lgkmcnt(0): it is read, its place can be filled again
+    __builtin_amdgcn_sched_barrier(0);
+    if (ti + kFewWaves < t1) {
+      request(ti + kFewWaves, blk);
+      if (ti + 2 * kFewWaves < t1) blk = block_of(ti + 2 * kFewWaves);
+    }
+    f32x4_t sacc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) sacc[hf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[hf][c], qb[c], sacc[hf], 0, 0, 0);
+    const int live = len_cached - ti * kTile;      // token of (hf, r): 16 hf + 4 quad + r
+    float mx = kHidden;
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float sv = 16 * hf + 4 * quad + r < live ? sacc[hf][r] * scale_log2e : kHidden;
+        sacc[hf][r] = sv;
+        mx = fmaxf(mx, sv);
+      }
+    if (live < kTile) {                            // (what the page holds behind the context need not be finite)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * hf + 4 * quad + r >= live) {
+#pragma unroll
+            for (int db = 0; db < 8; ++db) vf[db][hf][r] = 0;
+          }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m_run, mx), alpha = exp2f(m_run - mn);
+    m_run = mn;
+    float psum = 0.f;
+    bf16x8_t pb;
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float pv = exp2f(sacc[hf][r] - mn);
+        psum += pv;
+        pb[hf * 4 + r] = (bf16_t)pv;
+      }
+    l_run = l_run * alpha + psum;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      const s16x8_t a = {vf[db][0][0], vf[db][0][1], vf[db][0][2], vf[db][0][3], vf[db][1][0], vf[db][1][1], vf[db][1][2], vf[db][1][3]};
+      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), pb, oacc[db] * alpha, 0, 0, 0);
+    }
+  }
+
+  // ---- the waves' parts meet in LDS: each leaves its O in its own tile's place
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (quad == 0) ml[wave * 16 + head] = make_float2(m_run, l_run);
+#pragma unroll
+  for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4_t*>(k_lds + (db * 64 + lane) * 16) = oacc[db];
+  __syncthreads();
+  if (head < Gv) {                                 // wave w: dims 16 w + 4 quad .. + 3 of every head
+    float M = kNegBig, den = 0.f, f[kFewWaves];
+#pragma unroll
+    for (int w = 0; w < kFewWaves; ++w) M = fmaxf(M, ml[w * 16 + head].x);
+#pragma unroll
+    for (int w = 0; w < kFewWaves; ++w) {
+      const float2 e = ml[w * 16 + head];
+      f[w] = exp2f(e.x - M);
+      den += f[w] * e.y;
+    }
+    f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kFewWaves; ++w) num += f[w] * *reinterpret_cast<const f32x4_t*>(smem_raw + w * kFewTile + (wave * 64 + lane) * 16);
+    const int64_t row = (int64_t)b * hq + h * Gv + head;
+    const int d = 16 * wave + 4 * quad;
+    if (n == 1) {
+      *reinterpret_cast<u32x2_t*>(out + row * 128 + d) = u32x2_t{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
+      if (lse != nullptr && d == 0) lse[row] = 0.6931471805599453f * (M + log2f(den));
+    } else {
+      // (through to memory: a fence instead, which writes a whole L2 back, took 3 us and, from many workgroups at once, up to 200)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) few_put(part_o + (row * slots + part) * 128 + d + r, num[r]);
+      if (d == 0) {
+        few_put(part_ml + (row * slots + part) * 2, M);
+        few_put(part_ml + (row * slots + part) * 2 + 1, den);
+      }
+    }
+  }
+  if (n == 1 || arrived == nullptr) return;
+  int* last = reinterpret_cast<int*>(stage);
+  __builtin_amdgcn_s_waitcnt(0);                   // the partials are in memory
+  __syncthreads();
+  if (threadIdx.x == 0) *last = __hip_atomic_fetch_add(arrived + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (*last != n - 1) return;
+  for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves)
+    few_merge(part_o, part_ml, (int64_t)b * hq + h * Gv + (i >> 7), n, slots, i & 127, out, lse);
+  if (threadIdx.x == 0) arrived[pair] = 0;
+}
+
+// without a plan: the contexts of several parts
+__global__ __launch_bounds__(128) void decode_few_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                                const int32_t* __restrict__ ctx, bf16_t* __restrict__ out, int hq, int slots, int parts,
+                                                                float* __restrict__ lse) {
+  const int tiles = (ctx[blockIdx.x / hq] + kTile - 1) / kTile, n = few_split(tiles, parts);
+  if (n > 1) few_merge(part_o, part_ml, blockIdx.x, n, slots, threadIdx.x, out, lse);
+}
+
 // (A smaller minimum share per wave for small steps — 2 tiles instead of kMinTilesPerWave = 4, tried in round 4 on the
 // one-kv-head shape of Qwen3-32B per rank at TP = 8 — moves 1.2 us from the main kernel into the split merge, which then
 // has twice the partials: 19.1 + 4.5 -> 18.0 + 5.6 us per launch, nothing on the bench shape.
@@ -1702,6 +2012,36 @@ int launch_decode_mfma8_s(const void* q, void* kc, void* vc, const int32_t* bt, 
   }
   hipLaunchKernelGGL(decode_stream_combine_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml,
                      meta, ctx, (bf16_t*)out, hq, hkv, slots, lse, (const PlanHeader*)plan, prefix ? slots - 1 : -1);
+  return nvl_check_launch("nvl_paged_attn_decode");
+}
+
+// per-wave records of the largest grid the matrix-core kernel launches (2 workgroups per CU) behind the header; behind them the arrival
+// counters of decode_few_kernel
+inline size_t plan_records_bytes() { return sizeof(PlanHeader) + (size_t)nvl_device_cu_count() * 2 * kWaves * sizeof(PlanEntry); }
+
+template <bool SLABS>
+int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, int64_t bt_stride, const int32_t* ctx, void* out, int64_t batch,
+                      int hkv, int G, int block_size, int64_t max_context, float scale, void* workspace, hipStream_t s, const FusedArgs& fa, void* plan,
+                      float* lse, int parts) {
+  constexpr int lds = kFewWaves * (kFewTile + 16 * 8) + 18 * 256;
+  const int hq = hkv * G, slots = stream_slots(max_context);
+  float* part_o = (float*)workspace;
+  float* part_ml = part_o + (size_t)batch * hq * slots * 128;
+  static bool attr_done[NVL_MAX_DEVICES] = {};
+  bool& attr_set = attr_done[nvl_device_slot()];
+  if (!attr_set) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_few_kernel<SLABS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
+      nvl_set_error("nvl_paged_attn_decode: cannot reserve LDS for the kernel of few sequences");
+      return NVL_ELAUNCH;
+    }
+    attr_set = true;
+  }
+  int* arrived = plan != nullptr ? (int*)((unsigned char*)plan + plan_records_bytes()) : nullptr;
+  hipLaunchKernelGGL((decode_few_kernel<SLABS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
+                     (bf16_t*)vc, bt, bt_stride, ctx, part_o, part_ml, (bf16_t*)out, (int)batch, hkv, block_size, slots, scale * 1.4426950408889634f, fa,
+                     arrived, G, parts, lse);
+  if (plan == nullptr && parts > 1)
+    hipLaunchKernelGGL(decode_few_merge_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
   return nvl_check_launch("nvl_paged_attn_decode");
 }
 
@@ -1876,6 +2216,12 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
     NVL_REQUIRE(mfma, "%s: a plan with a shared prefix needs the matrix-core kernel (Hq/Hkv in 2 ... 16; got %d)", who, G);
     NVL_REQUIRE(block_size % 128 == 0, "%s: a shared prefix needs block_size %% 128 == 0 (got %d)", who, block_size);
   }
+  const int few = fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
+  if (few)
+    return fa->qkv_splits > 0 ? launch_decode_few<true>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
+                                                        max_context, softmax_scale, workspace, s, *fa, const_cast<void*>(plan), lse, few)
+                              : launch_decode_few<false>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
+                                                         max_context, softmax_scale, workspace, s, *fa, const_cast<void*>(plan), lse, few);
   if (kv_dtype == NVL_KV_FP8) {
 #define NVL_DECODE8_CASE(GG)                                                                                           \
   case GG:                                                                                                             \
@@ -2021,8 +2367,7 @@ extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stri
 
 // ---- per-step plan ------------------------------------------------------------------------------------------------
 extern "C" size_t nvl_decode_plan_bytes(void) {
-  // header + one record per wave of the largest grid the matrix-core kernel launches (2 workgroups per CU)
-  return sizeof(PlanHeader) + (size_t)nvl_device_cu_count() * 2 * kWaves * sizeof(PlanEntry);
+  return plan_records_bytes() + kFewGroups * sizeof(int);
 }
 
 extern "C" int nvl_decode_plan(const int32_t* context_lens, int64_t batch, int num_q_heads, int num_kv_heads,
@@ -2063,7 +2408,8 @@ extern "C" int nvl_decode_plan(const int32_t* context_lens, int64_t batch, int n
   }
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(256), lds, (hipStream_t)stream, context_lens, (int)batch,
                      num_kv_heads, nwaves, (PlanHeader*)plan, shared_prefix_blocks,
-                     shared_prefix_blocks ? block_size / kTile : 0, shared_prefix_blocks ? shared_prefix_groups : 0);
+                     shared_prefix_blocks ? block_size / kTile : 0, shared_prefix_blocks ? shared_prefix_groups : 0,
+                     few_parts(batch, num_kv_heads, max_context) > 1 ? (int*)((unsigned char*)plan + plan_records_bytes()) : nullptr);
   const int rc = nvl_check_launch(who);
   if (rc == NVL_OK) plan_shadow_put(plan, batch, num_kv_heads, max_context, shared_prefix_blocks != nullptr ? shared_prefix_groups : 0);   // (a failed launch leaves no record)
   return rc;
