@@ -134,6 +134,14 @@ int nvl_linear_wide(const void* x, const void* weight, void* out, int64_t m, int
                     int weight_layout, void* workspace, size_t workspace_bytes, void* stream);
 int nvl_pack_weight_tiles(const void* weight, void* packed, int64_t n, int64_t k, void* stream);
 
+/* The residual add and norm in front of a linear layer, and the layer, in one launch (m <= 16 rows, k <= 2048 and a multiple of 64, n a multiple of 4;
+ * silu: W [2n, k] = gate | up rows, out = silu(gate) * up as in mode 1 above):
+ *   s = float(x) + float(residual) (residual NULL: s = x); residual_out <- bf16(s); out = layer(bf16(s * rsqrt(mean(s^2) + eps) * float(norm_weight))),
+ * i.e. RMSNorm.add_rms_forward (layers/layernorm.py:28-40) and the merged projection behind it.  residual_out is another buffer than residual.
+ * slabs 1, 2 or 4: x is that many fp32 slabs of nvl_linear_decode mode 2, summed and rounded to bf16 first (0: x is bf16). */
+int nvl_norm_linear(const void* x, int slabs, const void* residual, const void* norm_weight, float eps, const void* weight, void* out, void* residual_out,
+                    int64_t m, int n, int k, int silu, void* stream);
+
 /* Fused split-K reduction + residual add + RMSNorm: replaces
  * RMSNorm.add_rms_forward (layers/layernorm.py:28-40) when its input is the
  * fp32 partials of nvl_linear_decode mode 2:

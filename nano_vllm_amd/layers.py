@@ -62,6 +62,23 @@ class RMSNorm(nn.Module):
         return y, residual
 
 
+    def into_linear(self, x, residual: torch.Tensor | None, linear: "LinearBase", silu: bool = False):
+        """(linear(self(x, residual)), the new residual) in one launch where the step is small enough (one launch fewer per norm: a step of one
+        sequence is a chain of launches of 4 us), or None. silu: `linear` is a gate|up pair and its activation comes along."""
+        w = linear.weight
+        if (not isinstance(x, torch.Tensor) or not _NORM_INTO_LINEAR or linear.bias is not None or w.dtype != torch.bfloat16
+                or w.shape[1] > ops.NORM_LINEAR_MAX_K or w.shape[1] % 64 or w.shape[0] % 8 or not x.is_cuda or not x.is_contiguous()
+                or x.dim() not in (2, 3) or x.shape[-2] > ops.NORM_LINEAR_MAX_ROWS):
+            return None
+        if x.dim() == 2 and x.dtype != torch.bfloat16 or x.dim() == 3 and (x.dtype != torch.float32 or x.shape[0] not in (1, 2, 4)):
+            return None
+        return ops.norm_linear(x, residual, self.weight, self.eps, w, silu)
+
+
+# NVL_NORM_LINEAR=0 keeps the norm of small decode steps a launch of its own (A/B measurements)
+_NORM_INTO_LINEAR = os.environ.get("NVL_NORM_LINEAR", "1") != "0"
+
+
 class SiluAndMul(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

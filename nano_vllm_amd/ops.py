@@ -32,6 +32,7 @@ SIGNATURES = {
     "nvl_linear_wide": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p, c_size_t,
                                 c_void_p]),
     "nvl_pack_weight_tiles": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
+    "nvl_norm_linear": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "nvl_add_rmsnorm_splitk": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_float, c_void_p]),
     "nvl_silu_mul": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p]),
     "nvl_rope_neox": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p]),
@@ -267,6 +268,27 @@ def linear_wide(x: torch.Tensor, weight: torch.Tensor, mode: int = LINEAR_BF16, 
     _check(lib().nvl_linear_wide(x.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, mode, 1 if packed else 0,
                                  workspace.data_ptr() if ws_bytes else None, ws_bytes, _stream()))
     return out
+
+
+NORM_LINEAR_MAX_ROWS, NORM_LINEAR_MAX_K = 16, 2048
+
+
+def norm_linear(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                silu: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
+    """(the linear layer of the RMS norm of x + residual, the new residual, a tensor of its own); silu: of [gate | up] halves, [M, N / 2]. x: bf16 [M, K], or the fp32 slabs [S, M, K] of a linear_decode
+    (S 1, 2 or 4). Up to 16 rows, K up to 2048."""
+    _dev(x, "x")
+    slabs = x.shape[0] if x.dim() == 3 else 0
+    assert x.is_contiguous() and weight.is_contiguous() and x.dtype == (torch.float32 if slabs else torch.bfloat16) and weight.dtype == torch.bfloat16
+    m, k = x.shape[-2:]
+    n = weight.shape[0] // (2 if silu else 1)
+    assert weight.shape[1] == k and weight.shape[0] == n * (2 if silu else 1) and norm_weight.numel() == k and norm_weight.dtype == torch.bfloat16
+    assert residual is None or (residual.shape == (m, k) and residual.is_contiguous() and residual.dtype == torch.bfloat16)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    new = torch.empty((m, k), dtype=torch.bfloat16, device=x.device)
+    _check(lib().nvl_norm_linear(x.data_ptr(), slabs, residual.data_ptr() if residual is not None else None, norm_weight.data_ptr(), eps,
+                                 weight.data_ptr(), out.data_ptr(), new.data_ptr(), m, n, k, 1 if silu else 0, _stream()))
+    return out, new
 
 
 def add_rmsnorm_splitk(partials: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,

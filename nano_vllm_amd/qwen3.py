@@ -16,7 +16,10 @@ shapes) the chain is 8 launches:
    -> split merge -> o GEMM (fp32 split-K slabs) -> add+RMSNorm(slabs) -> gate_up GEMM + SiLU*mul epilogue
    -> down GEMM (slabs)
 
-with the GEMMs on the hand-written skinny kernel (nvl_linear_decode).
+with the GEMMs on the hand-written skinny kernel (nvl_linear_decode). Up to 16 rows (TP=1, width <= 2048) it is 5:
+
+   [add+RMSNorm + qkv GEMM] -> [norm + RoPE + KV store + attention, split merged in LDS] -> o GEMM
+   -> [add+RMSNorm + gate_up GEMM + SiLU*mul] -> down GEMM
 """
 from __future__ import annotations
 
@@ -47,12 +50,15 @@ class Qwen3Attention(nn.Module):
             self.q_norm = RMSNorm(self.head_dim, eps=self.eps)
             self.k_norm = RMSNorm(self.head_dim, eps=self.eps)
 
-    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
+    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, qkv: torch.Tensor | None = None) -> torch.Tensor:
+        """qkv: the projection of hidden_states, where the norm in front of it has made it already."""
         ctx = get_context()
         # (a step whose plan carries a shared prefix takes bf16 qkv: the attention kernel that also serves the shared-prefix packs
         #  in the SAME launch has no scalar registers left for the slab-sum prologue — attn_decode.hip — and with slabs the pass
         #  would be a launch of its own on a divided grid)
-        if self.attn.fuses_decode_step(ctx) and not ctx.shared_prefix:
+        if qkv is not None:
+            pass
+        elif self.attn.fuses_decode_step(ctx) and not ctx.shared_prefix:
             qkv = self.qkv_proj.forward_for_fused_decode(hidden_states)      # bf16 [N, out], or fp32 split-K slabs
         else:
             qkv = self.qkv_proj(hidden_states)
@@ -74,6 +80,14 @@ class Qwen3MLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.down_proj.forward_decode(self.gate_up_proj.forward_silu(x))
 
+    def forward_normed(self, norm: RMSNorm, x, residual):
+        """(self(norm(x, residual)), the new residual) of a decode step; up to 16 rows take norm, gate|up and activation in one launch."""
+        both = norm.into_linear(x, residual, self.gate_up_proj, silu=True)
+        if both is not None:
+            return self.down_proj.forward_decode(both[0]), both[1]
+        hidden_states, residual = norm(x, residual)
+        return self(hidden_states), residual
+
 
 class Qwen3DecoderLayer(nn.Module):
 
@@ -86,12 +100,21 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions, hidden_states, residual):
-        if residual is None:                                 # first layer: residual = embeddings
-            residual = hidden_states
-            hidden_states = self.input_layernorm(hidden_states)
-        else:
-            hidden_states, residual = self.input_layernorm(hidden_states, residual)
-        hidden_states = self.self_attn(positions, hidden_states)
+        attn, qkv = self.self_attn, None
+        decode = attn.qkv_proj.tp_size == 1 and not get_context().is_prefill
+        if decode:
+            both = self.input_layernorm.into_linear(hidden_states, residual, attn.qkv_proj)
+            if both is not None:
+                qkv, residual = both
+        if qkv is None:
+            if residual is None:                             # first layer: residual = embeddings
+                residual = hidden_states
+                hidden_states = self.input_layernorm(hidden_states)
+            else:
+                hidden_states, residual = self.input_layernorm(hidden_states, residual)
+        hidden_states = attn(positions, hidden_states, qkv)
+        if decode:
+            return self.mlp.forward_normed(self.post_attention_layernorm, hidden_states, residual)
         hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
         return self.mlp(hidden_states), residual
 
