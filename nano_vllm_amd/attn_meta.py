@@ -12,6 +12,10 @@ tokens earlier steps already processed and its state slot).
 """
 from __future__ import annotations
 
+import functools
+
+import torch
+
 _FIELDS = ("is_prefill", "cu_seqlens_q", "cu_seqlens_k", "max_seqlen_q", "max_seqlen_k", "slot_mapping",
            "context_lens", "block_tables", "decode_workspace", "max_context", "decode_plan", "shared_prefix", "portions")
 _DEFAULTS = (False, None, None, 0, 0, None, None, None, None, 0, None, False, None)
@@ -48,3 +52,14 @@ def set_context(*args, **kwargs) -> None:
 
 def reset_context() -> None:
     _Holder.current = Context()
+
+
+def plain_calls(fn):
+    """For code that looks at tensors (pointers, shapes, strides), allocates on a named device and launches, as the models' forward passes do. With a
+    default device set (the runner's set_default_device leaves one), torch passes every function, method and attribute of a tensor through Python
+    first, about 1 us each, 20 to 30 of them per launch: 250 launches of a short prompt step took 6.1 ms on the host, 2.2 without that."""
+    @functools.wraps(fn)
+    def run(*args, **kwargs):
+        with torch._C.DisableTorchFunction():
+            return fn(*args, **kwargs)
+    return run

@@ -25,7 +25,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import ParallelMixer, RGLRUMixer, XIELUFeedForward, _copy_into, _param
 
 
@@ -105,6 +105,7 @@ class FoduzenForCausalLM(nn.Module):
             out.update({f"l{i}.{k}": v for k, v in layer.named_loaders().items()})
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """Returns the 32-bit residual stream after the last layer, [n, width]."""
         n, cfg = input_ids.numel(), self.config
@@ -118,6 +119,7 @@ class FoduzenForCausalLM(nn.Module):
                 trace.append(x.clone())
         return x
 
+    @plain_calls
     def compute_logits(self, x: torch.Tensor, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """Logits of the residual rows `rows` (int32 device indices; default: each portion's last token)."""
         if rows is None:

@@ -33,7 +33,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import (AttentionMixer, DeltaMixer, RoutedExperts, TokenShiftNorm, TokenSide, _copy_into, _param,
                      banded_rotary_frequencies)
 
@@ -140,6 +140,7 @@ class LigidraForCausalLM(nn.Module):
             out.update({f"l{i}.{k}": v for k, v in layer.named_loaders().items()})
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> tuple:
         """Returns what compute_logits takes: the 32-bit residual stream [n, width] before the last layer's last branch, that branch, and
         the weight of the norm on it (None: it is added as it is). A layer's last branch is always added by the kernel that norms the
@@ -181,6 +182,7 @@ class LigidraForCausalLM(nn.Module):
             x, pending = add(x, *pending), (None, None)
         return x, *pending
 
+    @plain_calls
     def compute_logits(self, hidden: tuple, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """Logits of the rows `rows` (int32 device indices; default: each portion's last token) of what forward() returned."""
         x, branch, wa = hidden

@@ -32,7 +32,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import (AttentionMemoryMixer, ConvAttentionMixer, GeluFeedForward, RoutedExperts, _copy_into, _param,
                      banded_rotary_frequencies, tie_parameters)
 
@@ -147,6 +147,7 @@ class LobidraForCausalLM(nn.Module):
                 out.update({f"l{i}.{k}": v for k, v in layer.named_loaders().items()})
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """Returns the 32-bit residual stream after the last layer, [n, width]. A sublayer's output is normed and added to the
         stream by the kernel that norms the stream for the NEXT sublayer (`pending` below: output(s), scales, the norm's weight)."""
@@ -185,6 +186,7 @@ class LobidraForCausalLM(nn.Module):
             sandwich(None)
         return x
 
+    @plain_calls
     def compute_logits(self, x: torch.Tensor, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """Logits of the residual rows `rows` (int32 device indices; default: each portion's last token)."""
         if rows is None:

@@ -30,7 +30,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import AttentionMixer, ClampedGLU, LightningMixer, RoutedExperts, _copy_into, _param, tie_parameters
 
 
@@ -139,6 +139,7 @@ class NokipelForCausalLM(nn.Module):
             out.update({f"l{i}.{k}": v for k, v in layer.named_loaders().items()})
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """Returns the 32-bit residual stream after the last layer, [n, width]. Every sublayer's output is added to the
         stream by the kernel that norms the stream for the NEXT sublayer (`pending` below)."""
@@ -168,6 +169,7 @@ class NokipelForCausalLM(nn.Module):
             ops_seq.add_group_norm(x, None, cfg.norm_groups, cfg.eps, None, a=pending)
         return x
 
+    @plain_calls
     def compute_logits(self, x: torch.Tensor, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """Logits of the residual rows `rows` (int32 device indices; default: each portion's last token)."""
         if rows is None:

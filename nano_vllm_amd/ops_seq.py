@@ -8,13 +8,13 @@ stream are float32. The library is built on first use when it is missing (a fres
 from __future__ import annotations
 
 import ctypes
-import functools
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 
 import torch
 
 from . import build as _build
+from .attn_meta import plain_calls as _launch
 
 ABI_VERSION = 7
 _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
@@ -107,17 +107,6 @@ def _check(rc: int) -> None:
 def _stream() -> int:
     # (the handle alone: building a Stream object around it took 6 of a launch's 25 us on the host)
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
-
-
-def _launch(fn):
-    """For functions that only look at their tensors (pointers, shapes, strides), allocate on a named device and launch. With a default
-    device set, torch passes every method and attribute of a tensor through Python first, about 1 us each, 20 to 30 of them per
-    launch: a step of 82 launches in 32-bit took 2.55 ms on the host around 1.4 ms of kernels, 1.45 without that."""
-    @functools.wraps(fn)
-    def run(*args, **kwargs):
-        with torch._C.DisableTorchFunction():
-            return fn(*args, **kwargs)
-    return run
 
 
 def _code(t: torch.Tensor) -> int:

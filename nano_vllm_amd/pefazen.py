@@ -36,7 +36,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import LatentAttentionMixer, RoutedExperts, _copy_into, _param
 
 MIXERS = ("latent_attention", "latent_attention_2")
@@ -130,6 +130,7 @@ class PefazenForCausalLM(nn.Module):
             out.update({f"l{i}.{k}": v for k, v in layer.named_loaders().items()})
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """Returns the 32-bit residual stream after the last layer, [n, width]. Every sublayer's output is added to the
         stream, times m, by the kernel that norms the stream for the NEXT sublayer (`pending` below)."""
@@ -155,6 +156,7 @@ class PefazenForCausalLM(nn.Module):
             ops_seq.add_group_norm(x, None, 1, cfg.eps, None, a=pending, a_mult=m)
         return x
 
+    @plain_calls
     def compute_logits(self, x: torch.Tensor, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """32-bit logits of the residual rows `rows` (int32 device indices; default: each portion's last token)."""
         cfg = self.config

@@ -27,7 +27,7 @@ import torch
 from torch import nn
 
 from .api import model_geometry
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .layers import (Attention, MergedColumnParallelLinear, ParallelLMHead, QKVParallelLinear, RMSNorm,
                      RowParallelLinear, SiluAndMul, VocabParallelEmbedding, get_rope)
 from . import tp
@@ -155,9 +155,11 @@ class Qwen3ForCausalLM(nn.Module):
         if self.geo["tie"]:
             self.lm_head.weight.data = self.model.embed_tokens.weight.data
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         return self.model(input_ids, positions)
 
+    @plain_calls
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         return self.lm_head(hidden_states)
 

@@ -27,7 +27,7 @@ import torch
 from torch import nn
 
 from . import ops_seq
-from .attn_meta import get_context
+from .attn_meta import get_context, plain_calls
 from .mixers import AttentionMixer, BranchNorm, RoutedExperts, SiluGLU, _copy_into, _param, rotary_frequencies
 
 
@@ -127,6 +127,7 @@ class ReselornForCausalLM(nn.Module):
                     out[name] = lambda t: None
         return out
 
+    @plain_calls
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """Returns the 32-bit residual stream after the last layer, [n, width]."""
         n, width = input_ids.numel(), self.config.hidden_size
@@ -146,6 +147,7 @@ class ReselornForCausalLM(nn.Module):
                 trace.append(x.clone())
         return x
 
+    @plain_calls
     def compute_logits(self, x: torch.Tensor, rows: torch.Tensor | None = None, nrows: int | None = None) -> torch.Tensor:
         """Logits of the residual rows `rows` (int32 device indices; default: each portion's last token)."""
         if rows is None:
