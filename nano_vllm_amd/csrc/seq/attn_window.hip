@@ -234,6 +234,7 @@ __global__ void window_attn_kernel(const WindowAttnArgs A) {
 }  // namespace
 
 int window_attn_token(const WindowAttnArgs& a, hipStream_t stream);          // attn_token.hip
+int window_attn_f32(const WindowAttnArgs& a, hipStream_t stream);            // attn_f32.hip
 void window_attn_extended(const WindowAttnArgs& a, hipStream_t stream);      // attn_pool.hip
 
 static int g_force_scalar = 0, g_no_lds = 0, g_packed_heads = 1;
@@ -331,6 +332,11 @@ extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnor
     else launch_mfma_sizes<false>(a, (hipStream_t)stream);
     return nvs_check_launch("nvs_window_attn (matrix cores)");
   }
+  // in 32-bit, the matrix cores for the sizes they are built for (attn_f32.hip), whenever a tile of 16 keys lies in one page and rows are aligned
+  if (dtype == NVS_F32 && ((d == 128 && dv == 128) || (d == 256 && dv == 192)) && block_size >= 16 && (block_size & (block_size - 1)) == 0 &&
+      (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)qnorm | (uintptr_t)pool_k | (uintptr_t)pool_v | (uintptr_t)out) & 15) == 0 &&
+      q_stride % 4 == 0 && n < (1ll << 31) && !g_force_scalar)
+    return window_attn_f32(a, (hipStream_t)stream);
   if (d <= 256 && dv <= 256)
     NVS_DISPATCH(dtype, window_attn_kernel<T, 4><<<dim3((unsigned)n, H), dim3(64), 0, (hipStream_t)stream>>>(a));
   else                                               // heads of up to 1024 entries: the same kernel with 16 entries per lane
