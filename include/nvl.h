@@ -327,6 +327,14 @@ int nvl_attn_prefill_varlen(const void* q, const void* k, const void* v,
                             int num_q_heads, int num_kv_heads,
                             int block_size, int64_t num_blocks,
                             float softmax_scale, int kv_dtype, float* lse, void* stream);
+/* The same on queries as the qkv projection leaves them: q rows q_tok_stride elements apart, head h at h * 128, normed with q_norm_w (NULL: not) and turned
+ * by cos_sin[positions[t]] as nvl_qknorm_rope_kvstore would (same roundings), bf16 keys and values. For steps whose longest prompt is short (the kernels of
+ * longer query tiles take finished queries only); nvl_qknorm_rope_kvstore with q_out NULL leaves the query heads out. */
+int nvl_attn_prefill_varlen_raw(const void* q, int64_t q_tok_stride, const int64_t* positions, const void* q_norm_w, float eps, const float* cos_sin,
+                                int64_t max_pos, const void* k, const void* v, int64_t k_tok_stride, int64_t v_tok_stride, const int32_t* cu_seqlens_q,
+                                const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride, void* out, int64_t total_q, int num_seqs,
+                                int max_seqlen_q, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, float softmax_scale, float* lse,
+                                void* stream);
 
 /* ---- Token sampler ---------------------------------------------------------
  * Replaces Sampler.forward (layers/sampler.py:7-12):

@@ -61,12 +61,23 @@ constexpr int kTileBytes = kKBlk * (kKRowB + kVRowB);   // one K + V tile pair i
 // tile requested during the last tile of the current one — was built and measured in round 4: +13 % on equal-length
 // batches, -8 ... -12 % on the bench's ragged ones, a dynamic per-XCD ticket queue slower than both. Retired:
 // tools/probes/rejected/attn_prefill_persistent_walk.hip.txt, profiles/r04_prefill_persist_ab.json.)
-template <bool PAGED, bool KV8, int NW>
+// RAWQ: q is the qkv projection's output as it is; a lane norms and turns its query's row when it loads it. As a pass of its own that read and wrote every q
+// row once more: 26 prompts of 100 to 1,024 tokens (14,600 tokens, 16 heads over 8), q/k norm + rotation + store and this kernel together 150 us a layer, now 136.
+struct RawQ {
+  int64_t tok_stride;                                    // elements between tokens of q
+  const int64_t* positions;
+  const bf16_t* norm_w;                                  // nullptr: no norm
+  const float* cos_sin;
+  int64_t max_pos;
+  float eps;
+};
+
+template <bool PAGED, bool KV8, int NW, bool RAWQ = false>
 __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int64_t k_tok_stride,
     int64_t v_tok_stride, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k,
     const int32_t* __restrict__ block_tables, int64_t bt_stride, bf16_t* __restrict__ out, int num_seqs, int hq,
-    int hkv, int block_size, float scale_log2e, int xcd_map, float* __restrict__ lse, float rescale_thr) {
+    int hkv, int block_size, float scale_log2e, int xcd_map, float* __restrict__ lse, float rescale_thr, RawQ raw) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // two {K: 64 x 256 B, V: 64 x 320 B} tile buffers, then the tile-lookup scratch
   constexpr int NT = NW * 64;                            // threads per workgroup
@@ -204,13 +215,21 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   item_geometry();
 
   // ---- Q fragments: B operand of S^T = K.Q^T : lane (query, hi) holds d = ds*16 + 8*hi .. +8
-  bf16x8_t qf[8];
+  bf16x8_t qf[8], qw[RAWQ ? 8 : 1];
+  int64_t qpos = 0;
   auto load_q = [&](int q0_, int lq_, int qblk_, int head_) {
     int row = qblk_ * kQBlk + wave * 32 + qcol;
     row = row < lq_ ? row : lq_ - 1;
-    const bf16_t* qp = q + ((int64_t)(q0_ + row) * hq + head_) * 128 + hi * 8;
+    const bf16_t* qp = RAWQ ? q + (int64_t)(q0_ + row) * raw.tok_stride + head_ * 128 + hi * 8 : q + ((int64_t)(q0_ + row) * hq + head_) * 128 + hi * 8;
+    if constexpr (RAWQ) qpos = raw.positions[q0_ + row];
 #pragma unroll
     for (int ds = 0; ds < 8; ++ds) qf[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(qp + ds * 16));
+    if constexpr (RAWQ) {
+      if (raw.norm_w != nullptr) {
+#pragma unroll
+        for (int ds = 0; ds < 8; ++ds) qw[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(raw.norm_w + ds * 16 + hi * 8));
+      }
+    }
   };
   load_q(q0, lq, qblk, head);
   // Keep the Q loads ahead of the first tile's staging loads: the prologue's wait for that tile then also
@@ -334,6 +353,46 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   // the Q fragment loads have landed before the loop (with a conditional prologue it assumes they may be pending at the
   // loop head and puts vmcnt waits on their first uses inside QK^T, which drain whatever tile loads are in flight).
   stage_load(0);
+  if constexpr (RAWQ) {
+    // norm and rotation as rope_common.h has them (roundings included): the lane holds entries ds * 16 + 8 hi .. + 7 and their partners 64 further on; the
+    // two halves of a row meet once
+#pragma clang fp contract(off)
+    const int64_t p = qpos < 0 ? 0 : (qpos >= raw.max_pos ? raw.max_pos - 1 : qpos);
+    const float* cs = raw.cos_sin + p * 128 + hi * 8;
+    f32x4_t c[4][2], sn[4][2];
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        c[ds][j] = *reinterpret_cast<const f32x4_t*>(cs + ds * 16 + j * 4);
+        sn[ds][j] = *reinterpret_cast<const f32x4_t*>(cs + 64 + ds * 16 + j * 4);
+      }
+    float rstd = 1.f;
+    if (raw.norm_w != nullptr) {
+      float ss = 0.f;
+#pragma unroll
+      for (int ds = 0; ds < 8; ++ds)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += (float)qf[ds][i] * (float)qf[ds][i];
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+      rstd = rsqrtf(ss * (1.f / 128.f) + raw.eps);
+    }
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float x1 = (float)qf[ds][i], x2 = (float)qf[ds + 4][i];
+        if (raw.norm_w != nullptr) {
+          x1 = round_bf16(x1 * rstd * (float)qw[ds][i]);
+          x2 = round_bf16(x2 * rstd * (float)qw[RAWQ ? ds + 4 : 0][i]);
+        }
+        const float co = c[ds][i >> 2][i & 3], si = sn[ds][i >> 2][i & 3];
+        const float a = x1 * co, b = x2 * si, a2 = x2 * co, b2 = x1 * si;
+        qf[ds][i] = (bf16_t)(a - b);
+        qf[ds + 4][i] = (bf16_t)(a2 + b2);
+      }
+  }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), expcnt / lgkmcnt untouched
   // a (no-op) use of the Q fragments HERE: without it LLVM sinks their loads into the loop preheader, behind this wait
 #pragma unroll
@@ -514,12 +573,12 @@ int nvl_prefill_w64_launch(const void* q, const void* k, const void* v, int64_t 
                            int block_size, void* out, int64_t total_q, int num_seqs, int num_q_heads, int num_kv_heads,
                            float scale_log2e, float* lse, float rescale_thr, hipStream_t s);
 
-extern "C" int nvl_attn_prefill_varlen(const void* q, const void* k, const void* v, int64_t k_tok_stride,
+static int prefill_common(const void* q, const void* k, const void* v, int64_t k_tok_stride,
                                        int64_t v_tok_stride, const int32_t* cu_seqlens_q,
                                        const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride,
                                        void* out, int64_t total_q, int num_seqs, int max_seqlen_q, int num_q_heads,
                                        int num_kv_heads, int block_size, int64_t num_blocks, float softmax_scale,
-                                       int kv_dtype, float* lse, void* stream) {
+                                       int kv_dtype, float* lse, const RawQ* raw, void* stream) {
   NVL_REQUIRE(q && k && v && cu_seqlens_q && cu_seqlens_k && out, "nvl_attn_prefill_varlen: null pointer");
   NVL_REQUIRE(kv_dtype == NVL_KV_BF16 || (kv_dtype == NVL_KV_FP8 && block_tables != nullptr),
               "nvl_attn_prefill_varlen: kv_dtype=%d (0 bf16; 1 fp8 e4m3 only with a paged cache)", kv_dtype);
@@ -573,13 +632,13 @@ extern "C" int nvl_attn_prefill_varlen(const void* q, const void* k, const void*
   // (1 x 16,384) over the 8-wave loop, profiles/r06_prefill_w64_asm_*.txt
   // (packed: its tile offsets are 32-bit buffer offsets — the K / V of the launch must span < 2 GiB; paged: 64-bit)
   const bool w64_fits = paged || total_q * (k_tok_stride > v_tok_stride ? k_tok_stride : v_tok_stride) * 2 < (1ll << 31);
-  if (w64 && ((max_seqlen_q >= 2048 && total_q >= (int64_t)num_seqs * 1024) || w64 == 2) && num_seqs <= 64 &&
+  if (w64 && !raw && ((max_seqlen_q >= 2048 && total_q >= (int64_t)num_seqs * 1024) || w64 == 2) && num_seqs <= 64 &&
       kv_dtype == NVL_KV_BF16 && !waves && w64_fits) {
     const int rc = nvl_prefill_w64_launch(q, k, v, k_tok_stride, v_tok_stride, cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride,
                                           block_size, out, total_q, num_seqs, num_q_heads, num_kv_heads, sl2, lse, thr, s);
     if (rc != 1) return rc;
   }
-  const int want = waves ? waves : (max_seqlen_q >= 2048 ? 8 : 4);
+  const int want = raw ? 4 : waves ? waves : (max_seqlen_q >= 2048 ? 8 : 4);
   const bool eight_ok = (num_q_heads / num_kv_heads) % 2 == 0;
   const int xcd_map = xcd_env >= 0 ? xcd_env : ((want == 4 || !eight_ok) && num_seqs <= 64 ? 1 : 0);
   const bool eight = want == 8 && !xcd_map && eight_ok;
@@ -602,18 +661,24 @@ extern "C" int nvl_attn_prefill_varlen(const void* q, const void* k, const void*
     (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<P, K8, NWV>),                  \
                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)cap) != hipSuccess)
     if (NVL_PF_ATTR(true, false, 4) || NVL_PF_ATTR(true, true, 4) || NVL_PF_ATTR(false, false, 4) ||
-        NVL_PF_ATTR(true, false, 8) || NVL_PF_ATTR(true, true, 8) || NVL_PF_ATTR(false, false, 8)) {
+        NVL_PF_ATTR(true, false, 8) || NVL_PF_ATTR(true, true, 8) || NVL_PF_ATTR(false, false, 8) ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<false, false, 4, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)cap) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<true, false, 4, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)cap) != hipSuccess) {
       nvl_set_error("nvl_attn_prefill_varlen: cannot reserve %zu B of LDS", cap);
       return NVL_ELAUNCH;
     }
 #undef NVL_PF_ATTR
     lds_cap = cap;
   }
-#define NVL_PF_LAUNCH(P, K8, NWV)                                                                                      \
-  hipLaunchKernelGGL((prefill_attn_kernel<P, K8, NWV>), grid, dim3(NWV * 64), lds, s, (const bf16_t*)q,                 \
+#define NVL_PF_LAUNCH(...)                                                                                             \
+  hipLaunchKernelGGL((prefill_attn_kernel<__VA_ARGS__>), grid, dim3(eight ? 512 : 256), lds, s, (const bf16_t*)q,       \
                      (const bf16_t*)k, (const bf16_t*)v, k_tok_stride, v_tok_stride, cu_seqlens_q, cu_seqlens_k,        \
-                     block_tables, bt_stride, (bf16_t*)out, num_seqs, num_q_heads, num_kv_heads, block_size, sl2, xcd_map, lse, thr)
-  if (paged && kv_dtype == NVL_KV_FP8) {
+                     block_tables, bt_stride, (bf16_t*)out, num_seqs, num_q_heads, num_kv_heads, block_size, sl2, xcd_map, lse, thr, raw ? *raw : RawQ{})
+  if (raw) {
+    if (paged) NVL_PF_LAUNCH(true, false, 4, true); else NVL_PF_LAUNCH(false, false, 4, true);
+  } else if (paged && kv_dtype == NVL_KV_FP8) {
     if (eight) NVL_PF_LAUNCH(true, true, 8); else NVL_PF_LAUNCH(true, true, 4);
   } else if (paged) {
     if (eight) NVL_PF_LAUNCH(true, false, 8); else NVL_PF_LAUNCH(true, false, 4);
@@ -622,4 +687,25 @@ extern "C" int nvl_attn_prefill_varlen(const void* q, const void* k, const void*
   }
 #undef NVL_PF_LAUNCH
   return nvl_check_launch("nvl_attn_prefill_varlen");
+}
+
+extern "C" int nvl_attn_prefill_varlen(const void* q, const void* k, const void* v, int64_t k_tok_stride, int64_t v_tok_stride,
+                                       const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride, void* out,
+                                       int64_t total_q, int num_seqs, int max_seqlen_q, int num_q_heads, int num_kv_heads, int block_size,
+                                       int64_t num_blocks, float softmax_scale, int kv_dtype, float* lse, void* stream) {
+  return prefill_common(q, k, v, k_tok_stride, v_tok_stride, cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, out, total_q, num_seqs, max_seqlen_q,
+                        num_q_heads, num_kv_heads, block_size, num_blocks, softmax_scale, kv_dtype, lse, nullptr, stream);
+}
+
+extern "C" int nvl_attn_prefill_varlen_raw(const void* q, int64_t q_tok_stride, const int64_t* positions, const void* q_norm_w, float eps,
+                                           const float* cos_sin, int64_t max_pos, const void* k, const void* v, int64_t k_tok_stride, int64_t v_tok_stride,
+                                           const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride,
+                                           void* out, int64_t total_q, int num_seqs, int max_seqlen_q, int num_q_heads, int num_kv_heads, int block_size,
+                                           int64_t num_blocks, float softmax_scale, float* lse, void* stream) {
+  NVL_REQUIRE(positions && cos_sin && max_pos > 0 && q_tok_stride % 8 == 0 && q_tok_stride >= (int64_t)num_q_heads * 128,
+              "nvl_attn_prefill_varlen_raw: positions, a rotation table and token rows of %d heads (stride %lld)", num_q_heads, (long long)q_tok_stride);
+  NVL_REQUIRE(((uintptr_t)q_norm_w | (uintptr_t)cos_sin) % 16 == 0, "nvl_attn_prefill_varlen_raw: pointers must be 16-byte aligned");
+  const RawQ raw{q_tok_stride, positions, (const bf16_t*)q_norm_w, cos_sin, max_pos, eps};
+  return prefill_common(q, k, v, k_tok_stride, v_tok_stride, cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, out, total_q, num_seqs, max_seqlen_q,
+                        num_q_heads, num_kv_heads, block_size, num_blocks, softmax_scale, NVL_KV_BF16, lse, &raw, stream);
 }

@@ -81,7 +81,8 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvstore_kernel(
     const float* __restrict__ cos_sin, int64_t max_pos, const int32_t* __restrict__ slot_mapping,
     bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_out, void* __restrict__ k_cache,
     void* __restrict__ v_cache, int64_t n_tok, int hq, int hkv, int block_size) {
-  const unsigned htot = hq + 2 * hkv, total = (unsigned)n_tok * htot;       // (below 2^31 - 32)
+  // (q_out nullptr: the attention kernel norms and turns the query heads itself, units are the others)
+  const unsigned skip = q_out == nullptr ? hq : 0, htot = hq - skip + 2 * hkv, total = (unsigned)n_tok * htot;       // (below 2^31 - 32)
   const unsigned unit0 = blockIdx.x * (16 * UN) + (threadIdx.x >> 4);
   const int sub = threadIdx.x & 15;
   u32x4_t raw[UN];
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvstore_kernel(
 #pragma unroll
   for (int i = 0; i < UN; ++i) {
     const unsigned unit = unit0 + 16 * i < total ? unit0 + 16 * i : 0;
-    tok[i] = unit / htot, head[i] = unit - tok[i] * htot;
+    tok[i] = unit / htot, head[i] = unit - tok[i] * htot + skip;
     raw[i] = *reinterpret_cast<const u32x4_t*>(qkv + tok[i] * qkv_tok_stride + head[i] * 128 + sub * 8);
     slot[i] = k_cache != nullptr ? slot_mapping[tok[i]] : -1;
     pos[i] = positions[tok[i]];
@@ -171,7 +172,7 @@ extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, 
                                        void* k_cache, void* v_cache, int64_t n_tok, int num_q_heads,
                                        int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype,
                                        void* stream) {
-  NVL_REQUIRE(qkv && positions && cos_sin && q_out, "nvl_qknorm_rope_kvstore: null pointer");
+  NVL_REQUIRE(qkv && positions && cos_sin && (q_out || k_out || k_cache), "nvl_qknorm_rope_kvstore: null pointer");
   NVL_REQUIRE(kv_dtype == NVL_KV_BF16 || kv_dtype == NVL_KV_FP8, "nvl_qknorm_rope_kvstore: kv_dtype=%d (0 bf16, 1 fp8 e4m3)", kv_dtype);
   NVL_REQUIRE((q_norm_w == nullptr) == (k_norm_w == nullptr), "nvl_qknorm_rope_kvstore: q/k norm weights must both be set or both NULL");
   NVL_REQUIRE((k_cache == nullptr) == (v_cache == nullptr), "nvl_qknorm_rope_kvstore: k_cache/v_cache must both be set or both NULL");
@@ -183,7 +184,7 @@ extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, 
   NVL_REQUIRE(((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_out | (uintptr_t)k_cache | (uintptr_t)v_cache |
                (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_sin) % 16 == 0,
               "nvl_qknorm_rope_kvstore: pointers must be 16-byte aligned");
-  const int64_t total = n_tok * (num_q_heads + 2 * num_kv_heads);
+  const int64_t total = n_tok * ((q_out ? num_q_heads : 0) + 2 * num_kv_heads);
   if (total == 0) return NVL_OK;
   NVL_REQUIRE(total + 32 < (1ll << 31), "nvl_qknorm_rope_kvstore: too many rows");       // (the kernel counts heads in 32 bits, up to 31 beyond the last)
   const bool two = total >= 262144;                 // (the kernel's comment has both sides)

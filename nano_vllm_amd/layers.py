@@ -120,6 +120,10 @@ def get_rope(head_size: int, rotary_dim: int, max_position: int, base: float, de
 # NVL_FUSED_DECODE=0 keeps the separate q/k-norm+RoPE+KV-store launch on decode steps (A/B measurements)
 _FUSED_DECODE = os.environ.get("NVL_FUSED_DECODE", "1") != "0"
 
+# NVL_RAW_Q=0 keeps the query heads of prompt steps in the q/k-norm launch (A/B measurements)
+_RAW_Q = os.environ.get("NVL_RAW_Q", "1") != "0" and os.environ.get("NVL_PREFILL_W64") is None and os.environ.get("NVL_PREFILL_WAVES") is None
+
+
 class Attention(nn.Module):
     """Paged attention. `k_cache` / `v_cache` are injected by the runner; layout
     [num_blocks, num_kv_heads, block_size, 128] (head-major — see include/nvl.h)."""
@@ -162,8 +166,16 @@ class Attention(nn.Module):
             return ops.paged_attn_decode_fused(qkv, q_norm_w, k_norm_w, eps, rope_table, self.k_cache, self.v_cache,
                                                ctx.block_tables, ctx.context_lens, hq, self.scale, max_context, ws,
                                                plan=ctx.decode_plan)
-        q = torch.empty((n, hq, 128), dtype=qkv.dtype, device=qkv.device)
         need_k = ctx.is_prefill and ctx.block_tables is None      # non-paged prefill reads packed K
+        if (_RAW_Q and ctx.is_prefill and 0 < ctx.max_seqlen_q <= ops.RAW_Q_MAX_SEQLEN
+                and (need_k or self.k_cache.dtype == torch.bfloat16)):        # the attention kernel norms and turns the queries
+            k = torch.empty((n, hkv, 128), dtype=qkv.dtype, device=qkv.device) if need_k else self.k_cache
+            ops.qknorm_rope_kvstore(qkv, positions, q_norm_w, k_norm_w, eps, rope_table, ctx.slot_mapping if has_cache else None, None,
+                                    k if need_k else None, self.k_cache if has_cache else None, self.v_cache if has_cache else None, hq, hkv)
+            v = qkv[:, (hq + hkv) * 128:].view(n, hkv, 128) if need_k else self.v_cache
+            return ops.attn_prefill_raw(qkv, hq, positions, q_norm_w, eps, rope_table, k, v, ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.max_seqlen_q,
+                                        self.scale, block_tables=ctx.block_tables)
+        q = torch.empty((n, hq, 128), dtype=qkv.dtype, device=qkv.device)
         k = torch.empty((n, hkv, 128), dtype=qkv.dtype, device=qkv.device) if need_k else None
         ops.qknorm_rope_kvstore(qkv, positions, q_norm_w, k_norm_w, eps, rope_table,
                                 ctx.slot_mapping if has_cache else None, q, k,

@@ -54,6 +54,9 @@ SIGNATURES = {
     "nvl_attn_prefill_varlen": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                         c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64, c_float,
                                         c_int, c_void_p, c_void_p]),
+    "nvl_attn_prefill_varlen_raw": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64,
+                                            c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64,
+                                            c_float, c_void_p, c_void_p]),
     "nvl_sample_workspace_bytes": (c_size_t, [c_int64]),
     "nvl_sample": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_uint64, c_uint64, c_void_p,
                            c_void_p, c_void_p, c_size_t, c_void_p]),
@@ -334,8 +337,9 @@ def store_kvcache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cac
 
 
 def qknorm_rope_kvstore(qkv: torch.Tensor, positions: torch.Tensor, q_norm_w, k_norm_w, eps: float,
-                        cos_sin: torch.Tensor, slot_mapping, q_out: torch.Tensor, k_out, k_cache, v_cache,
+                        cos_sin: torch.Tensor, slot_mapping, q_out: torch.Tensor | None, k_out, k_cache, v_cache,
                         num_q_heads: int, num_kv_heads: int) -> None:
+    """(q_out None: the query heads are left to attn_prefill_raw.)"""
     _dev(qkv, "qkv")
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.dtype == torch.bfloat16
     has_cache = k_cache is not None and k_cache.numel() > 0
@@ -345,7 +349,7 @@ def qknorm_rope_kvstore(qkv: torch.Tensor, positions: torch.Tensor, q_norm_w, k_
         k_norm_w.data_ptr() if k_norm_w is not None else None, eps,
         cos_sin.data_ptr(), cos_sin.shape[0],
         slot_mapping.data_ptr() if (has_cache and slot_mapping is not None) else None,
-        q_out.data_ptr(), k_out.data_ptr() if k_out is not None else None,
+        q_out.data_ptr() if q_out is not None else None, k_out.data_ptr() if k_out is not None else None,
         k_cache.data_ptr() if has_cache else None, v_cache.data_ptr() if has_cache else None,
         qkv.shape[0], num_q_heads, num_kv_heads,
         k_cache.shape[2] if has_cache else 0, k_cache.shape[0] if has_cache else 0,
@@ -487,6 +491,32 @@ def attn_prefill_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_se
                                              block_tables.data_ptr(), block_tables.stride(0), out.data_ptr(), nq,
                                              num_seqs, max_seqlen_q, hq, k.shape[1], k.shape[2], k.shape[0], scale,
                                              kv_dtype_of(k), _lse_ptr(lse, (nq, hq)), _stream()))
+    return out
+
+
+RAW_Q_MAX_SEQLEN = 2047       # longer prompts take the kernels of longer query tiles, whose queries are finished
+
+
+def attn_prefill_raw(qkv: torch.Tensor, num_q_heads: int, positions: torch.Tensor, q_norm_w, eps: float, cos_sin: torch.Tensor, k: torch.Tensor,
+                     v: torch.Tensor, cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_q: int, scale: float,
+                     block_tables: torch.Tensor | None = None) -> torch.Tensor:
+    """attn_prefill_varlen whose queries are the first num_q_heads heads of the qkv projection [Nq, >= Hq * 128] as they are: normed (q_norm_w or None) and
+    turned inside. bf16 keys and values."""
+    _dev(qkv, "qkv")
+    n, hq = qkv.shape[0], num_q_heads
+    assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and qkv.shape[1] >= hq * 128
+    assert cu_seqlens_q.dtype == torch.int32 and cu_seqlens_k.dtype == torch.int32 and positions.dtype == torch.int64 and positions.numel() >= n
+    out = torch.empty((n, hq, 128), dtype=torch.bfloat16, device=qkv.device)
+    paged = block_tables is not None
+    if paged:
+        assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
+    else:
+        assert k.stride(1) == 128 and v.stride(1) == 128 and k.stride(2) == 1 and v.stride(2) == 1
+    _check(lib().nvl_attn_prefill_varlen_raw(
+        qkv.data_ptr(), qkv.stride(0), positions.data_ptr(), q_norm_w.data_ptr() if q_norm_w is not None else None, eps, cos_sin.data_ptr(),
+        cos_sin.shape[0], k.data_ptr(), v.data_ptr(), 0 if paged else k.stride(0), 0 if paged else v.stride(0), cu_seqlens_q.data_ptr(),
+        cu_seqlens_k.data_ptr(), block_tables.data_ptr() if paged else None, block_tables.stride(0) if paged else 0, out.data_ptr(), n,
+        cu_seqlens_q.numel() - 1, max_seqlen_q, hq, k.shape[1], k.shape[2] if paged else 0, k.shape[0] if paged else 0, scale, None, _stream()))
     return out
 
 
