@@ -518,12 +518,20 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 // could not write padding). The MFMAs are written out with accumulators in the accumulation registers and operands in the vector registers:
 // left to itself the compiler moves one or the other between the two files in the loop.
 //
+// As many workgroups as fit on the chip at once, and each goes on from tile to tile: the last ST steps of a tile ask for the first ones of the next, whose
+// rows were looked up a whole tile earlier, so no tile but the first waits for its plan, its addresses and its operands, and the stores drain behind the next
+// tile's first steps. Full tiles of 256 rows x 256 weight rows, us per tile at k = 256 / 1024 / 4096, before and after (the products alone take 5.9 / 23.6 /
+// 94): gated 22.4 / 42.2 / 111.8 -> 13.1 / 32.0 / 106.9, plain 20.7 / 41.0 / 111.0 -> 14.7 / 36.8 / 109.0; tiles of 128 rows, gated 12.5 / 22.3 / 62.5 -> 7.3 / 17.4 / 58.3; of
+// 64 rows, two at a time 9.7 / 20.5 / 68.0 -> 7.5 / 18.6 / 64.8. Of that the tiles' overlap gives 2 to 3 us; the SiLU of 128 values per lane on the hardware's exponential
+// and reciprocal 3 to 5 (it took 30 instructions a value, and no product runs beside it); and the results' way through LDS, so that a store writes whole
+// rows of 128 or 256 bytes instead of 32 bytes in each of 16 rows, 2 to 5.
+//
 // Workgroups go to the eight XCDs round-robin; each XCD takes units of 8 row tiles x 4 feature tiles, whose operands its L2 then serves 4 and
 // up to 8 times, and neighbouring units go to different XCDs, so the unused row tiles at the end of the plan cost every XCD the same.
 //
 // Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
 // four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
-// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.35 to 2.45 + 1.39 to 1.44 ms = 1110 to 1160 and 950 to 980 TFLOP/s (the tiled kernel: 4.05 +
+// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.27 to 2.31 + 1.32 to 1.34 ms = 1180 to 1200 and 1020 to 1030 TFLOP/s (the tiled kernel: 4.05 +
 // 2.28 ms; the library's dense product of these sizes: 1.3-1.46 PFLOP/s); what is left is the chip's power limit and half a tile of padding
 // per expert. 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
 // (moe_gemm_mfma_kernel 411 + 217); width 1024, ff 768: 20 + 12 us (58 + 27). 32-bit, 1,044 rows, width 1024: 59 + 32 us (moe_gemm_kernel
@@ -549,6 +557,18 @@ __device__ __forceinline__ void mfma_units(f32x4_t (&acc)[RB], const u32x4_t& w,
   }
 }
 
+// bytes of LDS per wavefront beside the ring: one row block of its results (two workgroups per compute unit leave none)
+template <typename T, int PER_CU>
+constexpr int pipe_turn = sizeof(T) == 2 && PER_CU == 1 ? 4096 : 0;
+
+// silu(g) u. 16-bit results: 1 / (1 + 2^(-g log2 e)) with the hardware's exponential and reciprocal, a few units of the last 32-bit place each. Results in bfloat16
+// against 64-bit sums, gates of 0.3 to 20 and 512 products each: root mean square 1.655e-3 to 1.662e-3 and every maximum the same as with expf and a division.
+template <typename T>
+__device__ __forceinline__ float silu_times(float g, float u) {
+  if constexpr (sizeof(T) == 4) return glu_value(g, u, 0, 0.f, 0.f);
+  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
+}
+
 template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
 __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __restrict__ X, int64_t ldx, const T* __restrict__ W, int nout, int K,
                                                                     const int32_t* __restrict__ tile_expert,
@@ -556,53 +576,74 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
                                                                     T* __restrict__ out, int64_t ldo, int mode) {
   constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, NG = GLU ? 2 : 1, BN = BW / NG, ROW = 128, UNIT = 16 / sizeof(T);
   constexpr int STAGE = (BM + BW) * ROW, XI = BM >= 32 ? BM / 32 : 1, WI = BW / 32, NR = XI + WI;      // requests of a wavefront per step
+  constexpr int FB = WB / NG;                 // feature blocks of a wavefront
+  // 16-bit tiles with room beside the ring: two feature blocks lie side by side, so a lane's results are 8 features in a row, and a row
+  // block goes through LDS for stores of whole rows (pipe_turn bytes per wavefront)
+  constexpr bool PAIR = pipe_turn<T, PER_CU> > 0;
   static_assert(WB % NG == 0 && BW % 32 == 0 && (ST - 2) * NR < 64, "tile");
   extern __shared__ __attribute__((aligned(128))) char lds[];
-  const int j = blockIdx.x / 8, unit = (j / 32) * 8 + blockIdx.x % 8, units_n = (tiles_n + 3) / 4;
-  const int rt = unit / units_n * 8 + j % 8, ft = unit % units_n * 4 + (j % 32) / 8;
-  if (rt >= tiles_m || ft >= tiles_n) return;
-  const int e = tile_expert[rt];
+  const int units_n = (tiles_n + 3) / 4;
+  // this workgroup's tiles are blocks blockIdx.x, blockIdx.x + gridDim.x, ... (the same XCD's: the grid is a multiple of 8); row tiles only grow on the way,
+  // so the first one that holds no rows is the end
+  int block = blockIdx.x, rt = 0, ft = 0;
+  const auto find = [&] {
+    for (;; block += gridDim.x) {
+      const int j = block / 8, unit = (j / 32) * 8 + block % 8;
+      rt = unit / units_n * 8 + j % 8, ft = unit % units_n * 4 + (j % 32) / 8;
+      if (unit / units_n * 8 >= tiles_m) return false;
+      if (rt < tiles_m && ft < tiles_n) return true;
+    }
+  };
+  if (!find()) return;
+  int e = tile_expert[rt];
   if (e < 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15;
   const int wn = wave % WN, wm = wave / WN;
-  const int64_t row0 = (int64_t)rt * BM;
   // requests: one covers 8 rows; lane l brings unit (l & 7) ^ swizzle of row l >> 3. Padding rows and rows beyond the last feature bring
   // some valid row; what is computed from them is not stored. (Tiles of 16 rows: two wavefronts bring the same rows twice.)
-  const char *xsrc[XI], *wsrc[WI];
+  uint32_t xoff[XI], woff[WI];               // in units of 16 bytes: half the registers of addresses
+  static_assert(XI <= RB, "tile");
+  int tok[RB];                               // tokens of the rows a lane asks for, near a tile's end of the rows it stores
+  const auto look = [&] {
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int r = (wave * XI + i) * 8 % BM + (lane >> 3);
-    const int tok = row_token[row0 + r];
-    const int64_t src = (GLU || mode == 2) ? (tok >= 0 ? tok : 0) : row0 + r;
-    xsrc[i] = (const char*)(X + src * ldx + ((lane & 7) ^ ((r >> 1) & 7)) * UNIT);
-  }
+    for (int i = 0; i < XI; ++i) tok[i] = row_token[(int64_t)rt * BM + (wave * XI + i) * 8 % BM + (lane >> 3)];
+  };
+  const char* wbase;
+  const auto point = [&] {
+    int l = lane;
+    asm volatile("" : "+v"(l));              // (what follows from the lane alone is worked out here, not kept over the loop)
+    wbase = (const char*)(W + (int64_t)e * NG * nout * K);
 #pragma unroll
-  for (int i = 0; i < WI; ++i) {
-    const int r = (wave * WI + i) * 8 + (lane >> 3), f = ft * BN + r % BN;
-    wsrc[i] = (const char*)(W + ((int64_t)(e * NG + r / BN) * nout + (f < nout ? f : nout - 1)) * K + ((lane & 7) ^ ((r >> 1) & 7)) * UNIT);
-  }
+    for (int i = 0; i < XI; ++i) {
+      const int r = (wave * XI + i) * 8 % BM + (l >> 3);
+      const uint32_t src = (GLU || mode == 2) ? (tok[i] >= 0 ? tok[i] : 0) : rt * BM + r;
+      xoff[i] = src * (uint32_t)(ldx / UNIT) + ((l & 7) ^ ((r >> 1) & 7));
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      const int r = (wave * WI + i) * 8 + (l >> 3), f = ft * BN + r % BN;
+      woff[i] = (uint32_t)(r / BN * nout + (f < nout ? f : nout - 1)) * (uint32_t)(K / UNIT) + ((l & 7) ^ (PAIR ? ((r >> 1) & 1) | ((r >> 2) & 6) : (r >> 1) & 7));
+    }
+  };
+  look();
+  point();
   const auto request = [&](int i, int at, int step) {                   // request i of a step into the buffer at byte `at`
-    if (i < XI) dma16(xsrc[i < XI ? i : 0] + (int64_t)step * ROW, lds + at + (wave * XI + i) * 8 % BM * ROW);
-    else dma16(wsrc[i < XI ? 0 : i - XI] + (int64_t)step * ROW, lds + at + (BM + (wave * WI + i - XI) * 8) * ROW);
+    if (i < XI) dma16((const char*)X + step * ROW + (uint64_t)xoff[i < XI ? i : 0] * 16, lds + at + (wave * XI + i) * 8 % BM * ROW);
+    else dma16(wbase + step * ROW + (uint64_t)woff[i < XI ? 0 : i - XI] * 16, lds + at + (BM + (wave * WI + i - XI) * 8) * ROW);
   };
   f32x4_t acc[WB][RB];
-#pragma unroll
-  for (int wb = 0; wb < WB; ++wb)
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[wb][rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // operands of a half: weight-row block wb (GLU: the first half gate, the second up of the same features) and row block rb
   struct Operands {
     u32x4_t x[RB], w[WB];
   };
-  constexpr int FB = WB / NG;                                           // feature blocks of a wavefront
   const int unit0 = ((lane >> 4) ^ ((li >> 1) & 7)) * 16;               // (blocks start at multiples of 16 rows: the swizzle is the lane's)
   const char* xrow = lds + (wm * 16 * RB + li) * ROW;
-  const char* wrow = lds + (BM + wn * FB * 16 + li) * ROW;
+  const char* wrow = lds + (BM + wn * FB * 16 + (PAIR ? (li >> 2) * 8 + (li & 3) : li)) * ROW;
   const auto load = [&](Operands& o, int g, int at, int half) {         // a WB-th of a half's operands
     const int place = at + (unit0 ^ (half * 64));                       // unit (4 half + (lane >> 4)) ^ swizzle
 #pragma unroll
     for (int i = g * RB / WB; i < (g + 1) * RB / WB; ++i) o.x[i] = *(const u32x4_t*)(xrow + place + i * 16 * ROW);
-    o.w[g] = *(const u32x4_t*)(wrow + place + (g / FB * BN + g % FB * 16) * ROW);
+    o.w[g] = *(const u32x4_t*)(wrow + place + (g / FB * BN + (PAIR ? g % FB / 2 * 32 + g % 2 * 4 : g % FB * 16)) * ROW);
   };
   const auto half_step = [&](const Operands& now, Operands& next, int next_at, int next_half, bool ask, int ask_at, int ask_step) {
     constexpr int AG = WB >= 4 ? WB / 2 : WB, PER = (NR + AG - 1) / AG;  // requests go out in the first half of the groups
@@ -621,9 +662,10 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
     __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0): what was read ahead is there (the counter is too short to wait for it behind the next reads)
   };
   constexpr int AHEAD = (ST - 2) * NR;       // requests younger than the next step's
-  const auto arrive = [&](bool all) {        // the next step's requests landed (all: every request) and own LDS reads done; then everybody's
+  const auto arrive = [&](bool all, bool none) {        // the next step's requests landed (all: every request) and own LDS reads done; then everybody's
     __builtin_amdgcn_sched_barrier(0);
-    if (all) __builtin_amdgcn_s_waitcnt(0);
+    if (none) __builtin_amdgcn_s_waitcnt(0xC07F);
+    else if (all) __builtin_amdgcn_s_waitcnt(0);
     else __builtin_amdgcn_s_waitcnt((AHEAD & 15) | (AHEAD >> 4) << 14);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -637,67 +679,119 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
       for (int i = 0; i < NR; ++i) request(i, s * STAGE, s);
     }
   }
-  arrive(true);
+  arrive(true, false);
 #pragma unroll
   for (int g = 0; g < WB; ++g) load(a, g, 0, 0);
   __builtin_amdgcn_s_waitcnt(0xC07F);
-  int at = 0, s = 0;
+  int at = 0;
+  const bool whole = ((nout | (int)ldo) & (PAIR ? 7 : 3)) == 0 && ((uintptr_t)out & 15) == 0;
 #pragma unroll 1
-  for (; s + ST < steps; ++s) {
-    const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
-    half_step(a, b, at, 1, false, 0, 0);
-    arrive(ST == 2);
-    half_step(b, a, next, 0, true, at, s + ST);
-    at = next;
-  }
+  for (;;) {
+    // what the tile after this one needs is looked up now and used behind the loop
+    const int64_t row0 = (int64_t)rt * BM;
+    const int f0 = ft * BN;
+    block += gridDim.x;
+    bool more = find();
+    const int e_next = more ? tile_expert[rt] : -1;
+    if (more) look();
+#pragma unroll
+    for (int wb = 0; wb < WB; ++wb)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[wb][rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    int s = 0;
 #pragma unroll 1
-  for (; s < steps; ++s) {                   // the last ST steps: nothing left to request (the very last one reads ahead what nobody uses)
-    const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
-    half_step(a, b, at, 1, false, 0, 0);
-    arrive(true);
-    half_step(b, a, next, 0, false, 0, 0);
-    at = next;
-  }
-  asm volatile("s_nop 15\n\ts_nop 15");      // the last products are written before they are read: every read depends on one of
+    do {
+      if (s == (steps > ST ? steps - ST : 0)) {
+        more = more && e_next >= 0;
+        if (more) {
+          e = e_next;
+          point();
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) tok[rb] = row_token[row0 + (wm * RB + rb) * 16 + li];
+      }
+      const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
+      half_step(a, b, at, 1, false, 0, 0);
+      arrive(ST == 2 || (!more && s + ST > steps), s < ST - 1);
+      const bool same = s + ST < steps;        // the last ST steps ask for the first ones of the tile that follows
+      half_step(b, a, next, 0, same || more, at, same ? s + ST : s + ST - steps);
+      at = next;
+    } while (++s < steps);
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    const int wi = l & 15;
+    asm volatile("s_nop 15\n\ts_nop 15");      // the last products are written before they are read: every read depends on one of
 #pragma unroll                             // these statements, and volatile ones keep their order
-  for (int wb = 0; wb < WB; ++wb)
+    for (int wb = 0; wb < WB; ++wb)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) asm volatile("" : "+a"(acc[wb][rb]));
-  // lane: row li of row block rb; features 16 fb + 4 (lane >> 4) + 0..3 of its wavefront's
-  const bool quads = ((nout | (int)ldo) & 3) == 0 && ((uintptr_t)out & 15) == 0;
-  typedef __attribute__((ext_vector_type(4))) T t4_t;
+      for (int rb = 0; rb < RB; ++rb) asm volatile("" : "+a"(acc[wb][rb]));
+    __builtin_amdgcn_s_waitcnt(0x0F70);        // the requests for the next tile are there: its first ST - 1 steps need not wait behind the stores
+    // lane: row li of row block rb; features 16 fb + 4 (lane >> 4) + 0..3 of its wavefront's, or 32 fb + 8 (lane >> 4) + 0..7 of a pair's
+    constexpr int RUN = PAIR ? 8 : 4, RUNS = FB * 4 / RUN;
+    const auto value = [&](int rb, int i) {    // number i of a lane's results of a row block
+      const float y = acc[i / 4][rb][i % 4];
+      if constexpr (GLU) return (T)silu_times<T>(y, acc[i / 4 + FB][rb][i % 4]);
+      else return (T)plain_value(y, mode);
+    };
+    const int first = f0 + wn * FB * 16;       // the wavefront's features
+    if (PAIR && whole) {
+      constexpr int UNITS = PAIR ? RUNS * 4 : 4, PER = 64 / UNITS;       // 16-byte units of a row, rows of a store
+      u32x4_t* turn = (u32x4_t*)(lds + ST * STAGE + wave * pipe_turn<T, PER_CU>);
+      const auto place = [&](int r, int u) { return r * UNITS + (u ^ ((UNITS == 16 ? r : r >> 1) & (UNITS - 1))); };
+      const int f = first + l % UNITS * 8, sub = l / UNITS;
+      T* to = out + (row0 + wm * RB * 16 + sub) * ldo + f;
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int64_t r = row0 + (wm * RB + rb) * 16 + li;
-    if (row_token[r] < 0) continue;
+      for (int rb = 0; rb < RB; ++rb) {
+        const uint32_t live = (uint32_t)__ballot(tok[rb] >= 0);
 #pragma unroll
-    for (int fb = 0; fb < FB; ++fb) {
-      const int f = ft * BN + (wn * FB + fb) * 16 + (lane >> 4) * 4;
-      t4_t v;
+        for (int u = 0; u < RUNS; ++u) {
+          union { T v[RUN]; u32x4_t q; } o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = (T)(GLU ? glu_value(acc[fb][rb][i], acc[GLU ? fb + FB : fb][rb][i], 0, 0.f, 0.f) : plain_value(acc[fb][rb][i], mode));
-      if (quads) {
-        if (f < nout) *(t4_t*)(out + r * ldo + f) = v;
-      } else {
+          for (int i = 0; i < RUN; ++i) o.v[i] = value(rb, u * RUN + i);
+          turn[place(wi, u * 4 + (l >> 4))] = o.q;
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (f + i < nout) out[r * ldo + f + i] = v[i];
+        for (int p = 0; p < 16 / PER; ++p) {
+          const u32x4_t q = turn[place(p * PER + sub, l % UNITS)];
+          if ((live >> (p * PER + sub) & 1) && f < nout) *(u32x4_t*)(to + (int64_t)(rb * 16 + p * PER) * ldo) = q;
+        }
+      }
+    } else {
+      const int mine = first + (l >> 4) * RUN;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        T* to = out + (row0 + (wm * RB + rb) * 16 + wi) * ldo + mine;
+        if (tok[rb] < 0) continue;
+#pragma unroll
+        for (int u = 0; u < RUNS; ++u) {
+          typedef __attribute__((ext_vector_type(4))) T t4_t;
+          if (!PAIR && whole) {
+            if (mine + u * RUN * 4 < nout) *(t4_t*)(to + u * RUN * 4) = t4_t{value(rb, u * RUN), value(rb, u * RUN + 1), value(rb, u * RUN + 2), value(rb, u * RUN + 3)};
+          } else {
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+              if (mine + u * RUN * 4 + i < nout) to[u * RUN * 4 + i] = value(rb, u * RUN + i);
+          }
+        }
       }
     }
+    if (!more) break;
   }
 }
 
 template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
 int launch_pipe(const void* X, int64_t ldx, const void* W, int nout, int K, const int32_t* tile_expert, const int32_t* row_token, int64_t cap,
                 void* out, int64_t ldo, int mode, hipStream_t st) {
-  constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, BN = GLU ? BW / 2 : BW, LDS = ST * (BM + BW) * 128;
+  constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, BN = GLU ? BW / 2 : BW, LDS = ST * (BM + BW) * 128 + 4 * pipe_turn<T, PER_CU>;
   const int64_t tiles_m = cap / BM, tiles_n = (nout + BN - 1) / BN;
-  const int64_t units = (tiles_m + 7) / 8 * ((tiles_n + 3) / 4), blocks = (units + 7) / 8 * 256;
+  const int64_t units = (tiles_m + 7) / 8 * ((tiles_n + 3) / 4);
+  int64_t blocks = (units + 7) / 8 * 256;
   NVS_REQUIRE(blocks < (1ll << 31), "nvs_moe_gemm: step too large");
   const auto kernel = moe_gemm_pipe_kernel<T, GLU, WN, WB, RB, ST, PER_CU>;
   static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   NVS_REQUIRE(room == hipSuccess, "nvs_moe_gemm: %d bytes of LDS were refused", LDS);
+  // the ring goes on over the tiles of a workgroup if every stage holds a step of every tile
+  if (K / (128 / (int)sizeof(T)) >= ST && blocks > 256 * PER_CU) blocks = 256 * PER_CU;
   kernel<<<dim3((unsigned)blocks), dim3(256), LDS, st>>>((const T*)X, ldx, (const T*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n,
                                                          (T*)out, ldo, mode);
   return nvs_check_launch("nvs_moe_gemm (matrix cores, pipelined)");
@@ -824,7 +918,8 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
   if (cap == 0) return NVS_OK;
   hipStream_t st = (hipStream_t)stream;
   const bool matrix_cores = dtype == NVS_BF16 && K % 8 == 0 && ldx % 8 == 0 && !g_moe_plain;
-  const bool whole = (K % (dtype == NVS_BF16 ? 64 : 32) == 0) && ldx % (dtype == NVS_BF16 ? 8 : 4) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+  const int64_t size = dtype == NVS_BF16 ? 2 : 4, reach = 16ll << 32;      // (its offsets are 32 bits of 16-byte units: rows and an expert's weights up to 64 GiB)
+  const bool whole = cap * ldx * size < reach && 2ll * nout * K * size < reach && (K % (dtype == NVS_BF16 ? 64 : 32) == 0) && ldx % (dtype == NVS_BF16 ? 8 : 4) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
   if (whole && !g_moe_plain) {
 #define NVS_PIPE(...)                                                                                                       \
   (dtype == NVS_BF16                                                                                                        \

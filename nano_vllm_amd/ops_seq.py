@@ -721,13 +721,14 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     width 4096, ff 3072: 8 rows 428 / 436 / 471 / 609; 32: 598 / 455 / 489 / 622; 64: 838 / 580 / 507 / 640; 250: 2256 / 1003 / 879 / 928;
     1694: 12546 / 4674 / 4103 / 3634. Width 2048: 16 rows 126 / 133 / 149 / 178; 32: 141 / 135 / 155 / 181; 500: 1028 / 456 / 420 / 408.
     Width 1024, ff 768 (few and short tiles: two small workgroups per compute unit cover each other's start and end better than one large
-    one fills it): 34 rows 40 / 44 / 50 / 66; 68: 52 / 48 / 53 / 70; 533: 287 / 149 / 166 / 179; 1807: 897 / 389 / 422 / 411.
+    one fills it): 34 rows 40 / 44 / 50 / 66; 68: 52 / 48 / 53 / 70; 500: - / 131 / 140 / 144; 700: - / 162 / 155 / 144; 1400: - / 285 / 280 / 244; 1750: - / 344 / 348 / 305; 32 of
+    ff 512: 700 - / 96 / 89 / 100, 1400 - / 181 / 175 / 145; eight of ff 1024: 1000 - / 82 / 86 / 89, 2000 - / 115 / 115 / 97.
     32-bit: width 1024, 32 rows 80 / 126 / 228, 500: 830 / 836 / 912; width 2048, 32 rows 312 / 371 / 679, 125: 888 / 839 / 1100.
     Few workgroups leave most of the chip idle, and then the smaller tile is the faster one: 64-row workgroups on half of the compute units or fewer
     lose to 16 rows, 128-row ones to 64 below about 150, 256-row ones to 128 until the chip is full. Gated, 16 / 64 / 128 / 256 rows: one expert of 2048 x 2048, 64 rows 23 / 58 / 66 / 99,
     400: 48 / 59 / 68 / 112, 700: - / 61 / 74 / 113, 4000: - / 127 / 121 / 137, 8000: - / 243 / 221 / 200; two of 4096 x 3072, 100 rows each 70 / 92 / 100 / 162, 1000: - / 188 /
     178 / 197; four of 8192 x 1024, 2000 rows each - / 502 / 422 / 379. A down product of a short reduction prefers 64 rows until there are many: eight of 2048 x 512, 2000 rows
-    each - / 150 / 173 / 179; 16 of 2048 x 768, 1000 rows each - / 236 / 259 / 260, 64 of them, 750 rows each - / 742 / - / 669. 32-bit, two of 2048 x 1024, 100 rows each 46 / 197 / 370.
+    each - / 150 / 173 / 179; 32 of 2048 x 768, 300 rows each - / 143 / 138 / 150, 500: - / 256 / 232 / 230, 1000: - / 467 / 428 / 414; of 2048 x 512, 500: - / 142 / 147 / 157, 1400: - / 399 / 350 / 301. 32-bit, two of 2048 x 1024, 100 rows each 46 / 197 / 370.
     Rows that are no whole 128-byte pieces take the kernels that load their own operands, at the heights measured for those."""
     per = pairs // experts
     piece = 64 if dtype == torch.bfloat16 else 32
@@ -743,8 +744,10 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     if dtype != torch.bfloat16:
         return 64 if per >= (96 if width >= 2048 else 512) else 16
     if width < 2048:
+        if per >= 640 and groups(256) >= 380:
+            return 256
         return 64 if per >= 56 else 16
-    if per >= 448 and groups(256) >= (270 if ff >= 1024 else 600):
+    if per >= 448 and groups(256) >= (270 if ff >= 1024 else 480):
         return 256
     return 128 if per >= 64 and groups(128) >= (150 if ff >= 1024 else 1000) else 64 if per >= 24 else 16
 
