@@ -527,7 +527,9 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 // rows of 128 or 256 bytes instead of 32 bytes in each of 16 rows, 2 to 5.
 //
 // Workgroups go to the eight XCDs round-robin; each XCD takes units of 8 row tiles x 4 feature tiles, whose operands its L2 then serves 4 and
-// up to 8 times, and neighbouring units go to different XCDs, so the unused row tiles at the end of the plan cost every XCD the same.
+// up to 8 times, and neighbouring units go to different XCDs, so the unused row tiles at the end of the plan cost every XCD the same. The units are counted
+// over the tiles alone (a band of 8 row tiles column by column): with holes where the last unit of a band is not full, the same workgroups would be idle in
+// every band (ff 768, six feature tiles of gate|up: 203 us, now 171).
 //
 // Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
 // four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
@@ -569,11 +571,11 @@ __device__ __forceinline__ float silu_times(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
 }
 
-template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
+template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU, bool PLAN>
 __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __restrict__ X, int64_t ldx, const T* __restrict__ W, int nout, int K,
                                                                     const int32_t* __restrict__ tile_expert,
                                                                     const int32_t* __restrict__ row_token, int tiles_m, int tiles_n,
-                                                                    T* __restrict__ out, int64_t ldo, int mode) {
+                                                                    int group, int rows, T* __restrict__ out, int64_t ldo, int mode) {
   constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, NG = GLU ? 2 : 1, BN = BW / NG, ROW = 128, UNIT = 16 / sizeof(T);
   constexpr int STAGE = (BM + BW) * ROW, XI = BM >= 32 ? BM / 32 : 1, WI = BW / 32, NR = XI + WI;      // requests of a wavefront per step
   constexpr int FB = WB / NG;                 // feature blocks of a wavefront
@@ -581,21 +583,32 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
   // block goes through LDS for stores of whole rows (pipe_turn bytes per wavefront)
   constexpr bool PAIR = pipe_turn<T, PER_CU> > 0;
   static_assert(WB % NG == 0 && BW % 32 == 0 && (ST - 2) * NR < 64, "tile");
+  // no plan: every tile is expert 0's, and `rows` rows are their own tokens
+  const auto expert = [&](int tile) { return PLAN ? tile_expert[tile] : 0; };
+  const auto token = [&](int64_t r) { return PLAN ? row_token[r] : (int)r < rows ? (int)r : -1; };
   extern __shared__ __attribute__((aligned(128))) char lds[];
-  const int units_n = (tiles_n + 3) / 4;
-  // this workgroup's tiles are blocks blockIdx.x, blockIdx.x + gridDim.x, ... (the same XCD's: the grid is a multiple of 8); row tiles only grow on the way,
-  // so the first one that holds no rows is the end
-  int block = blockIdx.x, rt = 0, ft = 0;
+  // tiles in bands of 8 row tiles, a band column by column; this workgroup's: blocks blockIdx.x, blockIdx.x + gridDim.x, ... (the same XCD's)
+  int block = blockIdx.x, rt = 0, ft = 0, high = 8;
   const auto find = [&] {
-    for (;; block += gridDim.x) {
-      const int j = block / 8, unit = (j / 32) * 8 + block % 8;
-      rt = unit / units_n * 8 + j % 8, ft = unit % units_n * 4 + (j % 32) / 8;
-      if (unit / units_n * 8 >= tiles_m) return false;
-      if (rt < tiles_m && ft < tiles_n) return true;
+    const int j = block / 8, at = (j / group * 8 + block % 8) * group + j % group;
+    const int band = at / (8 * tiles_n), k = at % (8 * tiles_n);
+    high = min(8, tiles_m - band * 8);
+    if (high <= 0) return false;
+    ft = k / high, rt = band * 8 + k % high;
+    return ft < tiles_n;
+  };
+  // tiles without rows are the last row tiles of a plan. In a whole band a workgroup's row tiles only grow: nothing follows the first one
+  const auto used = [&](int e) {
+    while (e < 0) {
+      if (high == 8) return -1;
+      block += gridDim.x;
+      if (!find()) return -1;
+      e = expert(rt);
     }
+    return e;
   };
   if (!find()) return;
-  int e = tile_expert[rt];
+  int e = used(expert(rt));
   if (e < 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15;
   const int wn = wave % WN, wm = wave / WN;
@@ -606,7 +619,7 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
   int tok[RB];                               // tokens of the rows a lane asks for, near a tile's end of the rows it stores
   const auto look = [&] {
 #pragma unroll
-    for (int i = 0; i < XI; ++i) tok[i] = row_token[(int64_t)rt * BM + (wave * XI + i) * 8 % BM + (lane >> 3)];
+    for (int i = 0; i < XI; ++i) tok[i] = token((int64_t)rt * BM + (wave * XI + i) * 8 % BM + (lane >> 3));
   };
   const char* wbase;
   const auto point = [&] {
@@ -692,7 +705,7 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
     const int f0 = ft * BN;
     block += gridDim.x;
     bool more = find();
-    const int e_next = more ? tile_expert[rt] : -1;
+    const int e_next = more ? expert(rt) : -1;
     if (more) look();
 #pragma unroll
     for (int wb = 0; wb < WB; ++wb)
@@ -702,13 +715,14 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
 #pragma unroll 1
     do {
       if (s == (steps > ST ? steps - ST : 0)) {
-        more = more && e_next >= 0;
         if (more) {
-          e = e_next;
-          point();
+          e = used(e_next);
+          more = e >= 0;
+          if (more && e_next < 0) look();
+          if (more) point();
         }
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) tok[rb] = row_token[row0 + (wm * RB + rb) * 16 + li];
+        for (int rb = 0; rb < RB; ++rb) tok[rb] = token(row0 + (wm * RB + rb) * 16 + li);
       }
       const int next = at + STAGE == ST * STAGE ? 0 : at + STAGE;
       half_step(a, b, at, 1, false, 0, 0);
@@ -779,21 +793,23 @@ __global__ __launch_bounds__(256, PER_CU) void moe_gemm_pipe_kernel(const T* __r
   }
 }
 
-template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU>
+template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU, bool PLAN = true>
 int launch_pipe(const void* X, int64_t ldx, const void* W, int nout, int K, const int32_t* tile_expert, const int32_t* row_token, int64_t cap,
-                void* out, int64_t ldo, int mode, hipStream_t st) {
+                void* out, int64_t ldo, int mode, hipStream_t st, int rows = 0) {
   constexpr int BM = 16 * RB * (4 / WN), BW = 16 * WB * WN, BN = GLU ? BW / 2 : BW, LDS = ST * (BM + BW) * 128 + 4 * pipe_turn<T, PER_CU>;
   const int64_t tiles_m = cap / BM, tiles_n = (nout + BN - 1) / BN;
-  const int64_t units = (tiles_m + 7) / 8 * ((tiles_n + 3) / 4);
-  int64_t blocks = (units + 7) / 8 * 256;
+  // Tiles of a group share an L2. Few tiles go to the XCDs in smaller groups, so that each of them brings its share of the weights
+  const int64_t tiles = tiles_m * tiles_n;
+  const int group = tiles >= 256 ? 32 : 8;
+  int64_t blocks = (tiles + 8 * group - 1) / (8 * group) * (8 * group);
   NVS_REQUIRE(blocks < (1ll << 31), "nvs_moe_gemm: step too large");
-  const auto kernel = moe_gemm_pipe_kernel<T, GLU, WN, WB, RB, ST, PER_CU>;
+  const auto kernel = moe_gemm_pipe_kernel<T, GLU, WN, WB, RB, ST, PER_CU, PLAN>;
   static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   NVS_REQUIRE(room == hipSuccess, "nvs_moe_gemm: %d bytes of LDS were refused", LDS);
   // the ring goes on over the tiles of a workgroup if every stage holds a step of every tile
   if (K / (128 / (int)sizeof(T)) >= ST && blocks > 256 * PER_CU) blocks = 256 * PER_CU;
   kernel<<<dim3((unsigned)blocks), dim3(256), LDS, st>>>((const T*)X, ldx, (const T*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n,
-                                                         (T*)out, ldo, mode);
+                                                         group, rows, (T*)out, ldo, mode);
   return nvs_check_launch("nvs_moe_gemm (matrix cores, pipelined)");
 }
 
@@ -919,7 +935,8 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
   hipStream_t st = (hipStream_t)stream;
   const bool matrix_cores = dtype == NVS_BF16 && K % 8 == 0 && ldx % 8 == 0 && !g_moe_plain;
   const int64_t size = dtype == NVS_BF16 ? 2 : 4, reach = 16ll << 32;      // (its offsets are 32 bits of 16-byte units: rows and an expert's weights up to 64 GiB)
-  const bool whole = cap * ldx * size < reach && 2ll * nout * K * size < reach && (K % (dtype == NVS_BF16 ? 64 : 32) == 0) && ldx % (dtype == NVS_BF16 ? 8 : 4) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+  const bool whole = cap * ldx * size < reach && 2ll * nout * K * size < reach &&
+                     (K % (dtype == NVS_BF16 ? 64 : 32) == 0) && ldx % (dtype == NVS_BF16 ? 8 : 4) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
   if (whole && !g_moe_plain) {
 #define NVS_PIPE(...)                                                                                                       \
   (dtype == NVS_BF16                                                                                                        \
@@ -968,6 +985,18 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
                                                                              tm, (T*)out, ldo, mode));
   }
   return nvs_check_launch("nvs_moe_gemm");
+}
+
+// silu(g) u of [g | u] = X W^T: the tiles of the grouped product with one expert and no plan. The library's product and the activation behind it write and read
+// [n, 2 ff] once more than this: 14,600 rows, ff 3072, K 1024 222 us, here 185; which of them is taken is the caller's choice (measured there).
+extern "C" int nvs_silu_linear(const void* X, int64_t ldx, const void* W, int ff, int K, int64_t n, int tm, void* out, int64_t ldo, void* stream) {
+  if (n == 0) return NVS_OK;
+  NVS_REQUIRE(X && W && out && ff > 0 && K > 0 && K % 64 == 0 && n > 0 && ldx >= K && ldx % 8 == 0 && ldo >= ff && (((uintptr_t)X | (uintptr_t)W) & 15) == 0,
+              "nvs_silu_linear: %lld rows, %d x %d", (long long)n, ff, K);
+  NVS_REQUIRE((tm == 64 || tm == 256) && n < (1ll << 31) - 256 && (n + 255) * ldx < (8ll << 32) && 2ll * ff * K < (8ll << 32), "nvs_silu_linear: step too large");
+  const int64_t cap = (n + tm - 1) / tm * tm;
+  if (tm == 256) return launch_pipe<bf16_t, true, 2, 8, 8, 2, 1, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
+  return launch_pipe<bf16_t, true, 4, 4, 4, 2, 2, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
 }
 
 extern "C" int nvs_moe_combine(const void* rows, int64_t ldr, const int32_t* pair_row, const float* wts, int top, const void* h, int64_t ldh,

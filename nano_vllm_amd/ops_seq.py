@@ -65,6 +65,7 @@ SIGNATURES = {
     "nvs_moe_plan": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P]),
     "nvs_moe_plan_scratch": (c_int64, [_L, _I]),
     "nvs_moe_plan_wide": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P, _L, _P]),
+    "nvs_silu_linear": (c_int, [_P, _L, _P, _I, _I, _L, _I, _P, _L, _P]),
     "nvs_moe_gemm": (c_int, [_P, _L, _P, _I, _I, _I, _I, _P, _P, _L, _I, _P, _L, _P]),
     "nvs_moe_force_plain": (None, [_I]),
     "nvs_moe_combine": (c_int, [_P, _L, _P, _P, _I, _P, _L, _P, _P, _L, _I, _L, _I, _P, _P, _P]),
@@ -644,12 +645,50 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
     return _linear_rows(x, w, b, -1, 0.0, 0.0, torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device))
 
 
+def silu_linear_rows(n: int, ff: int, K: int) -> int:
+    """Rows per tile of silu_linear, 0 where the vendor library's product and the activation behind it are the faster way. A pass of 256 tiles fills the chip
+    and the last pass may be part-empty; the library's tiles are the better ones for long reductions. MI355X, us there / here at 64 / 256 rows, ff 3072,
+    K 1024: 600 rows 20 / 18 / 31, 1000: 25 / 24 / 33, 2000: 39 / 35 / 35, 6000: 103 / 90 / 95, 9000: 137 / 138 / 126, 14600: 222 / 224 / 185; ff 768, K 1024:
+    2000: 17.3 / 17.6 / 31, 4000: 25 / 24 / 33, 14600: 66 / 59 / 66; ff 4096, K 1536: 1500: 45 / 50 / 47, 4000: 100 / 111 / 93, 9000: 259 / 258 / 217; ff 2048, K 2048:
+    4000: 63 / 74 / 62, 9000: 148 / 161 / 164, 14600: 235 / 259 / 223; ff 6144, K 2048: 3000: 160 / 163 / 164, 6000: 354 / 330 / 270, 14600: 737 / 785 / 619; ff 4608,
+    K 2560: 6000: 276 / 320 / 264, 14600: 661 / 738 / 581; ff 8192, K 3072: 9000: 704 / 956 / 756, 14600: 1226 / 1553 / 1219."""
+    if K % 64 or K > 2560:
+        return 0
+    tiles = -(-n // 256) * -(-2 * ff // 256)
+    passes = -(-tiles // 256)
+    if tiles >= 208 and (tiles >= 216 * passes or tiles >= 768):
+        return 256
+    return 64 if K <= 1024 and tiles >= 72 else 0
+
+
+def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.stride(0) >= x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def silu_linear(x: torch.Tensor, w: torch.Tensor, tm: int, out: torch.Tensor | None = None) -> torch.Tensor:
+    """silu(g) u of [g | u] = x w^T: x [n, K], w [2 ff, K] = [gate | up], tiles of tm rows."""
+    lib = load_library()
+    n, K = x.shape
+    ff = w.shape[0] // 2
+    assert x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.is_contiguous() and w.shape == (2 * ff, K)
+    if out is None:
+        out = torch.empty(n, ff, dtype=x.dtype, device=x.device)
+    assert out.shape == (n, ff) and out.stride(1) == 1 and out.dtype == x.dtype
+    _check(lib.nvs_silu_linear(_ptr(x), x.stride(0), _ptr(w), ff, K, n, tm, _ptr(out), out.stride(0), _stream()))
+    return out
+
+
 @_launch
 def linear_act(x: torch.Tensor, w: torch.Tensor, ff: int, kind: int = 0, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
     """glu_act of x times w^T, w [2 ff, K] = [gate | up] (kind 2: [ff, K])."""
     out = torch.empty(x.shape[0], ff, dtype=x.dtype, device=x.device)
     if _few_rows(x, w, True):
         return _linear_rows(x, w, None, kind, limit, alpha, out)
+    if kind == 0 and silu_linear_fits(x, w):
+        tm = silu_linear_rows(x.shape[0], ff, x.shape[1])
+        if tm:
+            return silu_linear(x, w, tm, out)
     glu_act(torch.nn.functional.linear(x, w), ff, out, kind, limit, alpha)
     return out
 
@@ -721,7 +760,7 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     width 4096, ff 3072: 8 rows 428 / 436 / 471 / 609; 32: 598 / 455 / 489 / 622; 64: 838 / 580 / 507 / 640; 250: 2256 / 1003 / 879 / 928;
     1694: 12546 / 4674 / 4103 / 3634. Width 2048: 16 rows 126 / 133 / 149 / 178; 32: 141 / 135 / 155 / 181; 500: 1028 / 456 / 420 / 408.
     Width 1024, ff 768 (few and short tiles: two small workgroups per compute unit cover each other's start and end better than one large
-    one fills it): 34 rows 40 / 44 / 50 / 66; 68: 52 / 48 / 53 / 70; 500: - / 131 / 140 / 144; 700: - / 162 / 155 / 144; 1400: - / 285 / 280 / 244; 1750: - / 344 / 348 / 305; 32 of
+    one fills it): 34 rows 40 / 44 / 50 / 66; 68: 52 / 48 / 53 / 70; 500: - / 111 / 118 / 114; 700: - / 146 / 160 / 155; 1400: - / 275 / 265 / 239; 1750: - / 304 / 306 / 275; 32 of
     ff 512: 700 - / 96 / 89 / 100, 1400 - / 181 / 175 / 145; eight of ff 1024: 1000 - / 82 / 86 / 89, 2000 - / 115 / 115 / 97.
     32-bit: width 1024, 32 rows 80 / 126 / 228, 500: 830 / 836 / 912; width 2048, 32 rows 312 / 371 / 679, 125: 888 / 839 / 1100.
     Few workgroups leave most of the chip idle, and then the smaller tile is the faster one: 64-row workgroups on half of the compute units or fewer
