@@ -281,6 +281,9 @@ int nvs_moe_plan_wide(const int32_t* ids, int64_t n, int top, int experts, int t
  * multiple of 16 bytes) on the pipelined kernel, in either type. Padding rows are not written. */
 int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype, int mode, int nout, int K, const int32_t* tile_expert,
                  const int32_t* row_token, int64_t cap, int tm, void* out, int64_t ldo, void* stream);
+/* bf16, no plan: out[t, :] = silu(g) * u, [g | u] = W X[t, :], W [2 ff, K], on the pipelined kernel's tiles of tm (64 or 256) rows; K % 64 == 0, ldx % 8 == 0, X and W
+ * on 16-byte boundaries. */
+int nvs_silu_linear(const void* X, int64_t ldx, const void* W, int ff, int K, int64_t n, int tm, void* out, int64_t ldo, void* stream);
 /* tests: 1 routes bf16 calls through the plain kernel as well */
 void nvs_moe_force_plain(int on);
 
@@ -297,16 +300,23 @@ int nvs_moe_combine(const void* rows, int64_t ldr, const int32_t* pair_row, cons
  * With kv_col >= 0, columns kv_col .. + kv_rank are RMS-normed with kv_norm (the latent c) and the next rot_dim columns are the
  * shared key part: its leading rot_dims entries turn by pos[t] * rot_freq[i], i < rot_dims / 2, pair (2i, 2i+1) or, with
  * rot_halves, (i, i + rot_dims / 2); cos and sin are multiplied by rot_mag. Token t goes to cache slot slots[t] (< 0: skipped):
- * k_cache [slot][kv_rank + rot_dim] = [c | rotated part]; v_cache [page][kv_rank][block_size] = c, transposed inside the page. */
+ * k_cache [slot][kv_rank + rot_dim] = [c | rotated part]; v_cache [page][kv_rank][block_size] = c, transposed inside the page. turn (may be
+ * NULL) [n][rot_dims / 2][2] 32-bit: the cosines and sines of all tokens, for nvs_latent_heads. */
 int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
                     int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims, int rot_halves,
-                    float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache, int64_t n, void* stream);
+                    float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache, void* turn, int64_t n, void* stream);
 
 /* out[t, h, 0 .. width) = in[t, h, 0 .. width) with the leading rot_dims entries rotated as above; rows t have strides in_stride /
  * out_stride, heads in_head / out_head (elements, `dtype`). */
 int nvs_rotate_heads(const void* in, int64_t in_stride, int in_head, void* out, int64_t out_stride, int out_head, int dtype, int H,
                      int width, const int64_t* pos, const float* rot_freq, int rot_dims, int rot_halves, float rot_mag, int64_t n,
                      void* stream);
+
+/* bf16: y[t, a, 0 .. N) = W_a x[t, a, 0 .. K) for every head a; K and N 64, 128, 192 or 256. w [H][N][K], with `turned` [H][K][N]. With `turned`, the
+ * `tail` entries behind x's K go behind y's N, the leading rot_dims of them turned by `turn` ([n][rot_dims / 2][2], nvs_latent_prep). Strides in entries, multiples
+ * of 8; x, w and y on 16-byte boundaries. */
+int nvs_latent_heads(const void* x, int64_t ldx, int xh, const void* w, int turned, int K, int N, void* y, int64_t ldy, int yh, int H, int tail,
+                     int rot_dims, int rot_halves, const void* turn, int64_t n, void* stream);
 
 /* Tests and A/B runs: 1 routes bf16 calls through the scalar kernel too; 2 keeps the matrix-core kernel but without sharing
  * K / V tiles through LDS; 3 keeps the LDS kernel but never packs heads into the query tiles of single-token steps; 0 restores

@@ -14,7 +14,7 @@ namespace {
 
 template <typename T>
 __device__ __forceinline__ void rotate_part(const T* __restrict__ in, T* __restrict__ out, int width, int rot_dims, int halves, float mag,
-                                            const float* __restrict__ freq, float pf, int lane, int lanes) {
+                                            const float* __restrict__ freq, float pf, int lane, int lanes, float2* __restrict__ turn = nullptr) {
   const int half = rot_dims >> 1;
   for (int i = lane; i < half; i += lanes) {
     const int a = halves ? i : 2 * i, b = halves ? i + half : 2 * i + 1;
@@ -22,11 +22,13 @@ __device__ __forceinline__ void rotate_part(const T* __restrict__ in, T* __restr
     sincosf(pf * freq[i], &sn, &cs);
     sn *= mag;
     cs *= mag;
+    if (turn) turn[i] = make_float2(cs, sn);
+    if (!out) continue;
     const float u = ldf(in + a), v = ldf(in + b);
     stf(out + a, u * cs - v * sn);
     stf(out + b, v * cs + u * sn);
   }
-  for (int c = rot_dims + lane; c < width; c += lanes) out[c] = in[c];
+  for (int c = rot_dims + lane; out && c < width; c += lanes) out[c] = in[c];
 }
 
 // one workgroup of two wavefronts per token: wavefront 0 norms the query latent, wavefront 1 norms the key/value latent, rotates
@@ -37,7 +39,7 @@ __global__ __launch_bounds__(128) void latent_prep_kernel(const T* __restrict__ 
                                                           int rot_dim, const T* __restrict__ kv_norm, const int64_t* __restrict__ pos,
                                                           const float* __restrict__ freq, int rot_dims, int halves, float mag, float eps,
                                                           int block_size, const int32_t* __restrict__ slots, T* __restrict__ k_cache,
-                                                          T* __restrict__ v_cache) {
+                                                          T* __restrict__ v_cache, float2* __restrict__ turn) {
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (wave == 0) {
@@ -51,9 +53,13 @@ __global__ __launch_bounds__(128) void latent_prep_kernel(const T* __restrict__ 
     for (int c = lane; c < q_rank; c += 64) stf(cq + t * q_rank + c, ldf(src + c) * r * ldf(q_norm + c));
     return;
   }
-  if (kv_col < 0) return;
-  const int64_t slot = slots[t];
-  if (slot < 0) return;
+  // (cos and sin of the token's pairs also go to `turn`: the query heads' rotated parts turn by the same angles)
+  if (turn) turn += t * (rot_dims >> 1);
+  const int64_t slot = kv_col < 0 ? -1 : slots[t];
+  if (slot < 0) {
+    if (turn) rotate_part<T>(nullptr, nullptr, rot_dim, rot_dims, halves, mag, freq, (float)pos[t], lane, 64, turn);
+    return;
+  }
   const T* src = proj + t * stride + kv_col;
   float ss = 0.f;
   for (int c = lane; c < kv_rank; c += 64) {
@@ -72,7 +78,7 @@ __global__ __launch_bounds__(128) void latent_prep_kernel(const T* __restrict__ 
     kc[c] = val;
     vc[(int64_t)c * block_size] = val;
   }
-  rotate_part(src + kv_rank, kc + kv_rank, rot_dim, rot_dims, halves, mag, freq, (float)pos[t], lane, 64);
+  rotate_part(src + kv_rank, kc + kv_rank, rot_dim, rot_dims, halves, mag, freq, (float)pos[t], lane, 64, turn);
 }
 
 // out[t, h, :width] = rotated in[t, h, :width] for every head: the rotated query parts go behind the absorbed parts
@@ -93,7 +99,7 @@ __global__ void rotate_heads_kernel(const T* __restrict__ in, int64_t in_stride,
 extern "C" int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
                                int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims,
                                int rot_halves, float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache,
-                               int64_t n, void* stream) {
+                               void* turn, int64_t n, void* stream) {
   NVS_REQUIRE(proj && q_norm && cq && q_col >= 0 && q_rank > 0 && stride >= q_col + q_rank && n >= 0, "nvs_latent_prep: query latent %d + %d of %lld",
               q_col, q_rank, (long long)stride);
   if (kv_col >= 0) {
@@ -103,10 +109,11 @@ extern "C" int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int 
     NVS_REQUIRE(rot_dims >= 0 && rot_dims % 2 == 0 && rot_dims <= rot_dim && (rot_dims == 0 || rot_freq), "nvs_latent_prep: rotation of %d of %d entries",
                 rot_dims, rot_dim);
   }
+  NVS_REQUIRE(!turn || (pos && rot_freq && rot_dims > 0 && rot_dims % 2 == 0 && ((uintptr_t)turn & 7) == 0), "nvs_latent_prep: rotation of %d entries", rot_dims);
   if (n == 0) return NVS_OK;
   NVS_DISPATCH(dtype, latent_prep_kernel<T><<<dim3((unsigned)n), dim3(128), 0, (hipStream_t)stream>>>(
                           (const T*)proj, stride, q_col, q_rank, (const T*)q_norm, (T*)cq, kv_col, kv_rank, rot_dim, (const T*)kv_norm, pos,
-                          rot_freq, rot_dims, rot_halves, rot_mag, eps, block_size, slots, (T*)k_cache, (T*)v_cache));
+                          rot_freq, rot_dims, rot_halves, rot_mag, eps, block_size, slots, (T*)k_cache, (T*)v_cache, (float2*)turn));
   return nvs_check_launch("nvs_latent_prep");
 }
 

@@ -54,7 +54,8 @@ SIGNATURES = {
                                 _I, _I, _P, _P, _P, _I, _P, _F, _I, _P, _P]),
     "nvs_add_group_norm": (c_int, [_P, _P, _F, _P, _P, _L, _P, _I, _I, _I, _F, _I, _P, _P]),
     "nvs_scale_softcap": (c_int, [_P, _I, _F, _F, _L, _P, _P]),
-    "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _L, _P]),
+    "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _P, _L, _P]),
+    "nvs_latent_heads": (c_int, [_P, _L, _I, _P, _I, _I, _I, _P, _L, _I, _I, _I, _I, _I, _P, _L, _P]),
     "nvs_rotate_heads": (c_int, [_P, _L, _I, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _L, _P]),
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
     "nvs_linear_rows": (c_int, [_P, _L, _P, _P, _I, _L, _I, _I, _I, _F, _F, _P, _L, _P]),
@@ -553,10 +554,10 @@ class Rotation:
 def latent_prep(proj: torch.Tensor, q_col: int, q_rank: int, q_norm: torch.Tensor, cq: torch.Tensor, eps: float, kv_col: int = -1,
                 kv_rank: int = 0, rot_dim: int = 0, kv_norm: torch.Tensor | None = None, pos: torch.Tensor | None = None,
                 rot: Rotation | None = None, block_size: int = 0, slots: torch.Tensor | None = None, k_cache: torch.Tensor | None = None,
-                v_cache: torch.Tensor | None = None):
+                v_cache: torch.Tensor | None = None, turn: torch.Tensor | None = None):
     """Norms of the query latent (-> cq [n, q_rank]) and, with kv_col >= 0, of the key/value latent, the rotation of the shared key
     part and the store of both into the paged cache: k_cache [slots, 1, kv_rank + rot_dim], v_cache [slots, 1, kv_rank] (the
-    latent again, page-transposed like every value cache)."""
+    latent again, page-transposed like every value cache). turn [n, rot.dims / 2, 2] 32-bit: receives all tokens' cosines and sines."""
     lib = load_library()
     n = proj.shape[0]
     assert proj.stride(1) == 1 and cq.shape == (n, q_rank) and cq.is_contiguous() and q_norm.numel() == q_rank
@@ -569,7 +570,35 @@ def latent_prep(proj: torch.Tensor, q_col: int, q_rank: int, q_norm: torch.Tenso
     _check(lib.nvs_latent_prep(_ptr(proj), proj.stride(0), _same(proj, q_norm, cq, kv_norm, k_cache, v_cache), q_col, q_rank, _ptr(q_norm),
                                _ptr(cq), kv_col, kv_rank, rot_dim, _ptr(kv_norm), _ptr(pos), _ptr(rot.freq) if rot else None,
                                rot.dims if rot else 0, int(rot.halves) if rot else 0, rot.mag if rot else 1.0, eps, block_size, _ptr(slots),
-                               _ptr(k_cache), _ptr(v_cache), n, _stream()))
+                               _ptr(k_cache), _ptr(v_cache), _ptr(turn), n, _stream()))
+
+
+_HEAD_SIZES = (64, 128, 192, 256)
+
+
+def latent_heads_fit(x: torch.Tensor, w: torch.Tensor, K: int, N: int, tail: int = 0) -> bool:
+    """Whether latent_heads takes a step of x's rows (K -> N entries per head, `tail` entries behind): what it can take, and of few rows only those that have
+    a part behind, whose launch is saved. MI355X, us, a batched product (and the rotation) / here: 16 heads, 128 -> 192 + 64: 16 rows 9.3 / 7.4, 256: 14.5 / 10.5, 4,000:
+    29 / 24, 14,000: 95 / 57; 4 heads, 128 -> 256 + 64: 64 rows 8.5 / 10.0, 1,000: 8.5 / 11.2, 14,000: 31 / 26; 16 heads, 192 -> 128: 64 rows 5.4 / 6.5, 1,000: 6.3 / 7.8,
+    4,000: 12.4 / 12.8, 14,000: 46 / 29; 32 heads, 4,000: 23 / 19."""
+    if x.shape[0] * w.shape[0] < 65536 and not (tail and K * N <= 128 * 192):
+        return False
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and K in _HEAD_SIZES and N in _HEAD_SIZES and (K + tail) % 8 == 0 and (N + tail) % 8 == 0
+            and tail % 2 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
+
+@_launch
+def latent_heads(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, turned: bool, tail: int = 0, rot: Rotation | None = None, turn: torch.Tensor | None = None):
+    """y[t, a, :N] = W_a x[t, a, :K]: w [H, N, K], with `turned` [H, K, N]. The `tail` entries behind x's K go behind y's N, the leading rot.dims of them turned
+    by `turn` (latent_prep)."""
+    lib = load_library()
+    n, H, K = x.shape[0], x.shape[1], x.shape[2] - tail
+    N = y.shape[2] - tail
+    assert w.shape == ((H, K, N) if turned else (H, N, K)) and w.is_contiguous() and y.shape[:2] == (n, H) and x.stride(2) == y.stride(2) == 1
+    assert rot is None or turn.shape == (n, rot.dims // 2, 2) and turn.is_contiguous() and turn.dtype == torch.float32
+    assert x.dtype == w.dtype == y.dtype == torch.bfloat16
+    _check(lib.nvs_latent_heads(_ptr(x), x.stride(0), x.stride(1), _ptr(w), int(turned), K, N, _ptr(y), y.stride(0), y.stride(1), H, tail,
+                                rot.dims if rot else 0, int(rot.halves) if rot else 0, _ptr(turn), n, _stream()))
 
 
 @_launch
