@@ -104,7 +104,9 @@ int nvs_causal_conv(const void* in, int64_t in_stride, int dtype, const void* w,
  *   a = exp(-c * sigmoid(gr) * softplus(lam)),  S = a S + sqrt(1 - a^2) * sigmoid(gi) * u,  out = S * gelu_tanh(ypre).
  * S [nslots, C] 32-bit, advanced. out [n, C] `dtype`. Long portions of a step with few (portion, channel) threads are scanned
  * in segments, twice, in `ws` (nvs_rglru_scan_workspace floats; NULL: never), as nvs_ssd_scan below explains; max_q = the
- * longest portion of the step. */
+ * longest portion of the step. u NULL: gates are the pairs of nvs_rglru_gates instead, [n][C][2]: log a and the term added to a S. */
+int nvs_rglru_gates(const float* u, const float* w, const float* bias, const void* lam, int dtype, float c, int channels, int blocks, int64_t n,
+                    float* pairs, void* stream);       /* blocks of 128: w [blocks][128][256], bias [blocks][256]; u, bias and pairs on 16-byte boundaries */
 int64_t nvs_rglru_scan_workspace(int channels, int nseq, int64_t max_q);
 int nvs_rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam, float c,
                    int channels, int blocks, const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq, int64_t n,

@@ -170,7 +170,9 @@ __global__ void conv_state_kernel(const T* __restrict__ in, int64_t in_stride, i
 //   mode 1: every segment but a portion's last from zero -> its final value L_k and decay product d_k to `ws`
 //           ([nseq][nseg + 1][2][channels]; entry 0 holds the value the portion starts from);
 //   mode 2: segment k starts from S_k = d_(k-1) S_(k-1) + L_(k-1) and writes the outputs; the last one writes the slot.
-template <typename T, int MODE, int TT>             // TT tokens' operands asked for together (1: steps of few tokens per portion)
+// READY: `gates` holds [n][channels][2], log a and the added term (nvs_rglru_gates), and u is not read: what bounds it then is memory (460 MB in the first
+// pass of 13,550 tokens of 4,096 channels, 690 MB in the second: 80 and 153 us at 5.8 and 4.5 TB/s; with the gates' arithmetic 213 and 307).
+template <typename T, int MODE, int TT, bool READY> // TT tokens' operands asked for together (1: steps of few tokens per portion)
 __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* __restrict__ u, const T* __restrict__ ypre,
                                   int64_t y_stride, const T* __restrict__ lam, float cmul, int channels, int blocks,
                                   const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx0,
@@ -203,18 +205,28 @@ __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* 
   }
   float dsum = 0.f;                                 // sum of log a over the segment
   const float* gp = gates + ((int64_t)blk * n) * (2 * bw) + cc;
+  const float2* ready = (const float2*)gates + c;
   struct Gates {
     float a, add, y, la;
   };
   const auto gates_of = [&](float gr, float gi, float uv, float yv) {
     Gates v;
-    v.la = -cmul * sigmoid_hw(gr) * sp;
-    v.a = exp_hw(v.la);
-    const float om = fmaxf(one_less_exp(2.f * v.la), 0.f);          // 1 - a^2, without cancellation near a = 1; then its root
-    const float rs = __builtin_amdgcn_rsqf(om), s0 = om * rs;
-    v.add = (om > 1e-30f ? fmaf(fmaf(-s0, s0, om) * 0.5f, rs, s0) : sqrtf(om)) * (sigmoid_hw(gi) * uv);
+    if constexpr (READY) {
+      v.la = gr, v.a = exp_hw(gr), v.add = gi;
+    } else {
+      const RglruTerms t = rglru_terms(gr, gi, uv, sp, cmul);
+      v.la = t.la, v.a = t.a, v.add = t.add;
+    }
     v.y = mode != 1 ? gelu_tanhf_(yv) : 0.f;
     return v;
+  };
+  const auto operands = [&](int64_t t, float& gr, float& gi, float& uv) {
+    if constexpr (READY) {
+      const float2 v = ready[t * channels];
+      gr = v.x, gi = v.y, uv = 0.f;
+    } else {
+      gr = gp[t * (2 * bw)], gi = gp[t * (2 * bw) + bw], uv = u[t * channels + c];
+    }
   };
   const auto advance = [&](const Gates& v, int64_t t) {
     st = fmaf(v.a, st, v.add);
@@ -229,7 +241,7 @@ __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* 
 #pragma unroll
       for (int k = 0; k < TT; ++k) {
         const int64_t t = first + k;
-        gr[k] = gp[t * (2 * bw)], gi[k] = gp[t * (2 * bw) + bw], uv[k] = u[t * channels + c];
+        operands(t, gr[k], gi[k], uv[k]);
         yv[k] = mode != 1 ? ldf(ypre + t * y_stride + c) : 0.f;
       }
     };
@@ -246,7 +258,9 @@ __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* 
 #pragma unroll 4
   for (; t0 < q1; ++t0) {
     const float y1 = mode != 1 ? ldf(ypre + t0 * y_stride + c) : 0.f;
-    advance(gates_of(gp[t0 * (2 * bw)], gp[t0 * (2 * bw) + bw], u[t0 * channels + c], y1), t0);
+    float gr, gi, uv;
+    operands(t0, gr, gi, uv);
+    advance(gates_of(gr, gi, uv, y1), t0);
   }
   if (mode == 1) {
     wv[(int64_t)(2 * seg + 2) * channels] = st;
@@ -794,7 +808,7 @@ extern "C" int nvs_causal_conv(const void* in, int64_t in_stride, int dtype, con
 extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam,
                               float c, int channels, int blocks, const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq,
                               int64_t n, int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream) {
-  NVS_REQUIRE(gates && u && ypre && lam && cu_q && ctx0 && slot && S && out, "nvs_rglru_scan: null argument");
+  NVS_REQUIRE(gates && ypre && lam && cu_q && ctx0 && slot && S && out, "nvs_rglru_scan: null argument");
   NVS_REQUIRE(channels > 0 && blocks > 0 && channels % blocks == 0 && y_stride >= channels && nseq >= 0 && nseq <= 65535 && n >= 0,
               "nvs_rglru_scan: channels %d blocks %d", channels, blocks);
   if (n == 0 || nseq == 0) return NVS_OK;
@@ -805,10 +819,15 @@ extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* yp
   const dim3 block(64);
   // Portions under eight tokens take the kernel that walks single ones: as part of eight, most of them nobody's, a decode step of 256 sequences of
   // 4,096 channels took 31 us; by the leftover path of the kernel of eight, whose registers leave fewer wavefronts, 11.9; here 10.9
-#define NVS_RGLRU_LAUNCH(MODE, TT)                                                                                                 \
-  NVS_DISPATCH(dtype, rglru_scan_kernel<T, MODE, TT><<<dim3((channels + 63) / 64, (unsigned)nseq, seg_len ? nseg : 1), block, 0,         \
+#define NVS_RGLRU_KERNEL(MODE, TT, READY)                                                                                          \
+  NVS_DISPATCH(dtype, rglru_scan_kernel<T, MODE, TT, READY><<<dim3((channels + 63) / 64, (unsigned)nseq, seg_len ? nseg : 1), block, 0,  \
                                                   (hipStream_t)stream>>>(gates, u, (const T*)ypre, y_stride, (const T*)lam, c, channels, \
                                                                          blocks, cu_q, ctx0, slot, n, S, (T*)out, seg_len, nseg, ws))
+#define NVS_RGLRU_LAUNCH(MODE, TT)                    \
+  do {                                                \
+    if (u) NVS_RGLRU_KERNEL(MODE, TT, false);         \
+    else NVS_RGLRU_KERNEL(MODE, TT, true);            \
+  } while (0)
   if (seg_len) {
     NVS_RGLRU_LAUNCH(1, 8);
     NVS_RGLRU_LAUNCH(2, 8);
@@ -818,6 +837,7 @@ extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* yp
     NVS_RGLRU_LAUNCH(0, 8);
   }
 #undef NVS_RGLRU_LAUNCH
+#undef NVS_RGLRU_KERNEL
   return nvs_check_launch("nvs_rglru_scan");
 }
 

@@ -134,6 +134,20 @@ __device__ __forceinline__ float expm1_tail(float x) {
 __device__ __forceinline__ float expm1_less_x(float x) { return x > -1.f ? expm1_tail(x) * x * x : exp_hw(x) - 1.f - x; }
 __device__ __forceinline__ float one_less_exp(float x) { return x > -1.f ? -fmaf(expm1_tail(x) * x, x, x) : 1.f - exp_hw(x); }
 
+// one token and channel of the real-gated linear recurrence S <- a S + add: la = log a. sp = softplus(lam)
+struct RglruTerms {
+  float la, a, add;
+};
+__device__ __forceinline__ RglruTerms rglru_terms(float gr, float gi, float u, float sp, float c) {
+  RglruTerms v;
+  v.la = -c * sigmoid_hw(gr) * sp;
+  v.a = exp_hw(v.la);
+  const float om = fmaxf(one_less_exp(2.f * v.la), 0.f);            // 1 - a^2, without cancellation near a = 1; then its root
+  const float rs = __builtin_amdgcn_rsqf(om), s0 = om * rs;
+  v.add = (om > 1e-30f ? fmaf(fmaf(-s0, s0, om) * 0.5f, rs, s0) : sqrtf(om)) * (sigmoid_hw(gi) * u);
+  return v;
+}
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float siluf_(float x) { return x / (1.f + expf(-x)); }

@@ -665,6 +665,12 @@ class ParallelMixer(nn.Module):
         return left, right
 
 
+# rows of a step from which the gates are ops_seq.rglru_gates' (blocks of 128 channels). Below, a batched product that spreads a block over more workgroups is as
+# fast. MI355X, product and scan, us there / here, 4,096 channels: 1 row 13.1 / 15.9, 16: 14.2 / 14.2, 64: 22 / 19, 256: 59 / 28, 1,000: 91 / 42; 1,024 channels:
+# 16: 13.6 / 14.8, 64: 20 / 19, 1,000: 31 / 28. Added terms against 64 bits: there 8.6e-8, here 6.7e-8 (matrices that are no bfloat16 numbers 7.3e-8)
+RGLRU_GATES_MIN_ROWS = 32
+
+
 class RGLRUMixer(nn.Module):
     """y = gelu_tanh(W_y h + b), u = conv(W_x h + b); per block of channels r = sigmoid(R u_b + b_r), i = sigmoid(I u_b + b_i);
     a = exp(-c r softplus(lam)); S <- a S + sqrt(1 - a^2) i u; out = W_o (S * y). The gates' matrices are kept in 32-bit
@@ -711,7 +717,10 @@ class RGLRUMixer(nn.Module):
         proj = ops_seq.linear(xh, self.in_w, self.in_b)
         u = torch.empty(n, C, dtype=torch.float32, device=xh.device)
         ops_seq.causal_conv(proj[:, C:], self.conv_w, self.conv_b, 0, por, self.conv_state, u)
-        gates = torch.baddbmm(self.gate_b, u.view(n, self.blocks, bw).transpose(0, 1), self.gate_w)     # [blocks, n, 2 bw] fp32
+        if bw == 128 and n >= RGLRU_GATES_MIN_ROWS and u.is_cuda:
+            gates, u = ops_seq.rglru_gates(u, self.gate_w, self.gate_b, self.lam, self.c, self.blocks), None
+        else:
+            gates = torch.baddbmm(self.gate_b, u.view(n, self.blocks, bw).transpose(0, 1), self.gate_w)     # [blocks, n, 2 bw] fp32
         s = torch.empty(n, C, dtype=xh.dtype, device=xh.device)
         ops_seq.rglru_scan(gates, u, proj[:, :C], self.lam, self.c, self.blocks, por, self.rec_state, s)
         return ops_seq.linear(s, self.o_w)

@@ -33,6 +33,7 @@ SIGNATURES = {
                                       _L, _P]),
     "nvs_moe_table_route": (c_int, [_P, _P, _L, _I, _F, _P, _P, _P]),
     "nvs_rglru_scan_workspace": (c_int64, [_I, _I, _L]),
+    "nvs_rglru_gates": (c_int, [_P, _P, _P, _P, _I, _F, _I, _I, _L, _P, _P]),
     "nvs_rglru_scan": (c_int, [_P, _P, _P, _L, _I, _P, _F, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
     "nvs_ssd_scan_workspace": (c_int64, [_I, _I, _I, _I, _L]),
     "nvs_ssd_scan": (c_int, [_P, _P, _L, _L, _I, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
@@ -204,17 +205,31 @@ def causal_conv(inp: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
 
 
 @_launch
-def rglru_scan(gates: torch.Tensor, u: torch.Tensor, ypre: torch.Tensor, lam: torch.Tensor, c: float, blocks: int, por: Portions,
-               S: torch.Tensor, out: torch.Tensor):
+def rglru_gates(u: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, lam: torch.Tensor, c: float, blocks: int) -> torch.Tensor:
+    """u [n, channels], w [blocks, 128, 256], bias [blocks, 1, 256], all 32-bit -> pairs [n, channels, 2] for rglru_scan: log a and the added term."""
     lib = load_library()
     n, channels = u.shape
+    assert u.dtype == w.dtype == bias.dtype == torch.float32 and u.is_contiguous() and w.is_contiguous() and bias.is_contiguous()
+    assert w.shape == (blocks, 128, 256) and bias.numel() == blocks * 256 and channels == blocks * 128 and lam.numel() == channels and lam.is_contiguous()
+    pairs = torch.empty(n, channels, 2, dtype=torch.float32, device=u.device)
+    _check(lib.nvs_rglru_gates(_ptr(u), _ptr(w), _ptr(bias), _ptr(lam), _code(lam), c, channels, blocks, n, _ptr(pairs), _stream()))
+    return pairs
+
+
+@_launch
+def rglru_scan(gates: torch.Tensor, u: torch.Tensor | None, ypre: torch.Tensor, lam: torch.Tensor, c: float, blocks: int, por: Portions,
+               S: torch.Tensor, out: torch.Tensor):
+    """gates [blocks, n, 2 bw] are the pre-activations, u [n, channels] the input; u None: gates are rglru_gates' pairs."""
+    lib = load_library()
+    n, channels = out.shape
     bw = channels // blocks
-    assert n == por.n and gates.dtype == torch.float32 and gates.is_contiguous() and gates.shape == (blocks, n, 2 * bw)
-    assert u.dtype == torch.float32 and u.is_contiguous() and ypre.shape == (n, channels) and ypre.stride(1) == 1
+    assert n == por.n and gates.dtype == torch.float32 and gates.is_contiguous() and gates.shape == ((n, channels, 2) if u is None else (blocks, n, 2 * bw))
+    assert u is None or u.dtype == torch.float32 and u.is_contiguous() and u.shape == (n, channels)
+    assert ypre.shape == (n, channels) and ypre.stride(1) == 1
     assert S.dtype == torch.float32 and S.is_contiguous() and S.shape[1] == channels and lam.numel() == channels
     assert out.shape == (n, channels) and out.is_contiguous()
     need = 0 if torch.cuda.is_current_stream_capturing() else lib.nvs_rglru_scan_workspace(channels, por.nseq, por.max_q)
-    ws = torch.empty(need, dtype=torch.float32, device=u.device) if need else None
+    ws = torch.empty(need, dtype=torch.float32, device=out.device) if need else None
     _check(lib.nvs_rglru_scan(_ptr(gates), _ptr(u), _ptr(ypre), ypre.stride(0), _same(ypre, lam, out), _ptr(lam), c, channels,
                               blocks, _ptr(por.cu_q), _ptr(por.ctx0), _ptr(por.slot), por.nseq, n, por.max_q, _ptr(S), _ptr(out), _ptr(ws), need,
                               _stream()))
