@@ -918,7 +918,7 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   NVS_REQUIRE(!seg_len || ws_floats >= need(nseg), "%s: workspace of %lld floats is too small", who, (long long)ws_floats);
   ScanArgs ca = {form, xbc, proj, proj_stride, dt_col, x_col, b_col, c_col, ga.i_col, ga.f_col, decay, dt_bias, A_log, D, ga.i_bias, ga.f_bias,
                  heads, P, N, G, cu_q, ctx0, slot, S, ga.M, y, ga.den, ws, ga.cap, ga.c_scale, 0, 1};
-  // State rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, except for a few tokens where these lose. us for
+  // Other state rows of 64 or 128 entries in aligned memory go to the chunks of scan_chunk.hip, except for a few tokens where these lose. us for
   // portions of 1 / 3 / 6 tokens, walk against chunks:
   //   small states of many pairs, whose workgroups of at least four wavefronts and their LDS come in turns of 512 where all of the walk's run
   //   at once: 2,048 pairs of 16 x 64 13 / 16 / 20 against 21, 1,024 of 32 x 128 17 / 20 / 25 against 20, 2,048 of 64 x 64 23 / 26 / 34 against 25; exponential
@@ -928,6 +928,11 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   //   pairs 11 / 14 against 13, 256 pairs 16 / 19 against 16 (18), 512 pairs 30 against 25.
   // The constant decay stays with the walk for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is
   // 7.4e-8, not 8.3e-8.
+  // Single tokens of the sizes that scan_token.hip is built for are its: it only moves the state. us here / there (the faster of the two), state-space duality, constant
+  // decay, exponential gates: 512 pairs of 128 x 128 14.4 / 24, 16 / 24, 16 / 26; 8 pairs 8.5 / 11.8, 8.7 / 9.1, 8.6 / 10.8; 1,024 pairs of 64 x 128 12.0 / 24, 13.7 / 24, 13.4 / 28,
+  // 4,096: 44 / 79, 45 / 77, 51 / 88; 4,096 of 32 x 64 14 / 28, 17 / 27, 17 / 36. Of two tokens 512 pairs of 128 x 128 19 / 24, 22 / 26, 22 / 26, but 8 pairs 12 / 12, 14 / 10, 13 / 12: there the
+  // walk, whose tokens' operands are staged ahead, and the chunks begin to pay.
+  if (max_q == 1 && scan_token_fits(ca, dtype)) return scan_token_launch(ca, dtype, nseq, stream);
   const int64_t pairs = (int64_t)heads * nseq;
   bool walk = form == 1 && max_q < 16;
   if (form != 1 && pairs >= 1024 && P * N < 8192)
