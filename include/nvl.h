@@ -296,6 +296,19 @@ int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride,
                                 void* workspace, size_t workspace_bytes,
                                 int kv_dtype, const void* plan, float* lse,
                                 int qkv_splits, int64_t qkv_split_stride, void* stream);
+
+/* nvl_paged_attn_decode_fused of up to 4 sequences, max_context <= 16384 (bf16 cache, group sizes of the matrix-core kernel, no shared prefix) without the merge of a context's parts:
+ * workspace receives [batch][Hq][parts][128] 32-bit numerators, [batch][Hq][parts][2] maximum (base 2) and sum, and [batch][Hq][128] bf16. parts =
+ * nvl_paged_attn_decode_open_parts (0: the step is too large); a context has min(parts, max(1, ceil(tokens / 256))) of them. One of a
+ * single part is finished, as bf16; an empty one's row is zero. */
+int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context);
+int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
+                               int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables, int64_t bt_stride, const int32_t* context_lens,
+                               int64_t batch, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int64_t max_context,
+                               float softmax_scale, void* workspace, size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream);
+/* nvl_linear_decode mode 2 of the merge of those parts, rounded to bf16: m <= 16 rows of k = Hq * 128 entries */
+int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight, void* out,
+                           int64_t m, int n, int k, int weight_layout, void* stream);
 /* qkv_splits (ABI 4): 0 = `qkv` is the bf16 output [batch, qkv_tok_stride] of the qkv projection
  * (QKVParallelLinear.forward, layers/linear.py:96-128). 1..8 = `qkv` is the fp32 split-K slab stack
  * [qkv_splits][batch][qkv_tok_stride] that nvl_linear_wide mode 2 leaves for a deep-K projection

@@ -1591,10 +1591,17 @@ inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
   return batch <= 16 && batch * hkv * parts <= kFewGroups ? (int)parts : 0;
 }
 
-// parts of a context of `tiles` tiles
-__device__ __forceinline__ int few_split(int tiles, int parts) {
-  const int n = (tiles + kFewPart - 1) / kFewPart;
-  return n < 1 ? 1 : n < parts ? n : parts;
+// Left open for the output projection to merge (nvl_linear_decode_open), a part costs neither a trip through memory nor a wait for the others, so it
+// is a tile of each wavefront. us, attention and output projection (16 heads over 8 kv heads, 1,024 columns), merged here / open: one sequence of 100 tokens 8.8 / 8.9,
+// 256 9.6 / 9.8, 700 12.5 / 10.4, 2,000 16.3 / 12.1, 4,096 16.5 / 15.4, 12,000 22.3 / 21.1; four of 100 9.0 / 9.3, 700 13.7 / 11.4, 2,000 17.2 / 15.7. Eight of 2,000
+// 25.9 / 26.5 (the projection reads every part in each of its workgroups), one of 30,000 33.5 / 36.5: those are merged here.
+constexpr int kOpenPart = NVL_OPEN_PART_TILES, kOpenParts = 16, kOpenRows = 4;
+inline int open_parts(int64_t batch, int hkv, int64_t max_context) {
+  if (batch < 1 || batch > kOpenRows || batch * hkv > kFewGroups || max_context > 16384) return 0;
+  int64_t parts = ((max_context + kTile - 1) / kTile + kOpenPart - 1) / kOpenPart;
+  if (parts > kOpenParts) parts = kOpenParts;
+  if (parts > kFewGroups / (batch * hkv)) parts = kFewGroups / (batch * hkv);
+  return (int)parts;
 }
 
 // partials go through to memory and are read from there (another workgroup's L2 may be another one)
@@ -1634,14 +1641,15 @@ template <bool SLABS>
 __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc, const int32_t* __restrict__ block_tables, int64_t bt_stride,
     const int32_t* __restrict__ ctx, float* part_o, float* part_ml, bf16_t* __restrict__ out, int batch, int hkv, int block_size, int slots,
-    float scale_log2e, FusedArgs fa, int* arrived, int Gv, int parts, float* __restrict__ lse) {
+    float scale_log2e, FusedArgs fa, int* arrived, int Gv, int parts, int part_tiles, bool open, float* __restrict__ lse) {
   typedef __attribute__((address_space(3))) void lds_void_t;
   typedef const __attribute__((address_space(1))) void global_void_t;
+  // open: a context of several parts leaves them as they are, for the output projection
   extern __shared__ __attribute__((aligned(128))) unsigned char smem_raw[];           // tiles; q rows [16][256], new k, new v; (m, l) [wave][16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, rq = lane >> 4, head = lane & 15, quad = lane >> 4;
   const int pairs = batch * hkv, part = blockIdx.x / pairs, pair = blockIdx.x % pairs, b = pair / hkv, h = pair % hkv, hq = hkv * Gv;
-  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = few_split(tiles, parts), per = (tiles + n - 1) / n;
+  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = nvl_few_split(tiles, part_tiles, parts), per = (tiles + n - 1) / n;
   if (part >= n) return;
   if (len <= 0) {                                  // graph padding: zero rows
     for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves) out[((int64_t)b * hq + h * Gv) * 128 + i] = (bf16_t)0.f;
@@ -1841,7 +1849,10 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     for (int w = 0; w < kFewWaves; ++w) num += f[w] * *reinterpret_cast<const f32x4_t*>(smem_raw + w * kFewTile + (wave * 64 + lane) * 16);
     const int64_t row = (int64_t)b * hq + h * Gv + head;
     const int d = 16 * wave + 4 * quad;
-    if (n == 1) {
+    if (open && n > 1) {
+      *reinterpret_cast<f32x4_t*>(part_o + (row * slots + part) * 128 + d) = num;
+      if (d == 0) *reinterpret_cast<float2*>(part_ml + (row * slots + part) * 2) = make_float2(M, den);
+    } else if (n == 1) {
       *reinterpret_cast<u32x2_t*>(out + row * 128 + d) = u32x2_t{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
       if (lse != nullptr && d == 0) lse[row] = 0.6931471805599453f * (M + log2f(den));
     } else {
@@ -1854,7 +1865,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
       }
     }
   }
-  if (n == 1 || arrived == nullptr) return;
+  if (open || n == 1 || arrived == nullptr) return;
   int* last = reinterpret_cast<int*>(stage);
   __builtin_amdgcn_s_waitcnt(0);                   // the partials are in memory
   __syncthreads();
@@ -1870,7 +1881,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
 __global__ __launch_bounds__(128) void decode_few_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                 const int32_t* __restrict__ ctx, bf16_t* __restrict__ out, int hq, int slots, int parts,
                                                                 float* __restrict__ lse) {
-  const int tiles = (ctx[blockIdx.x / hq] + kTile - 1) / kTile, n = few_split(tiles, parts);
+  const int tiles = (ctx[blockIdx.x / hq] + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts);
   if (n > 1) few_merge(part_o, part_ml, blockIdx.x, n, slots, threadIdx.x, out, lse);
 }
 
@@ -2024,9 +2035,11 @@ int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, in
                       int hkv, int G, int block_size, int64_t max_context, float scale, void* workspace, hipStream_t s, const FusedArgs& fa, void* plan,
                       float* lse, int parts) {
   constexpr int lds = kFewWaves * (kFewTile + 16 * 8) + 18 * 256;
-  const int hq = hkv * G, slots = stream_slots(max_context);
+  const bool open = out == nullptr;
+  const int hq = hkv * G, slots = open ? parts : stream_slots(max_context);
   float* part_o = (float*)workspace;
   float* part_ml = part_o + (size_t)batch * hq * slots * 128;
+  if (open) out = part_ml + (size_t)batch * hq * slots * 2;
   static bool attr_done[NVL_MAX_DEVICES] = {};
   bool& attr_set = attr_done[nvl_device_slot()];
   if (!attr_set) {
@@ -2039,8 +2052,8 @@ int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, in
   int* arrived = plan != nullptr ? (int*)((unsigned char*)plan + plan_records_bytes()) : nullptr;
   hipLaunchKernelGGL((decode_few_kernel<SLABS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
                      (bf16_t*)vc, bt, bt_stride, ctx, part_o, part_ml, (bf16_t*)out, (int)batch, hkv, block_size, slots, scale * 1.4426950408889634f, fa,
-                     arrived, G, parts, lse);
-  if (plan == nullptr && parts > 1)
+                     arrived, G, parts, open ? kOpenPart : kFewPart, open, lse);
+  if (!open && plan == nullptr && parts > 1)
     hipLaunchKernelGGL(decode_few_merge_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
   return nvl_check_launch("nvl_paged_attn_decode");
 }
@@ -2180,8 +2193,8 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
                   const int32_t* context_lens, void* out, int64_t batch, int num_q_heads, int num_kv_heads,
                   int block_size, int64_t num_blocks, int64_t max_context, float softmax_scale, void* workspace,
                   size_t workspace_bytes, void* stream, const FusedArgs* fa, const char* who, int kv_dtype,
-                  const void* plan, float* lse) {
-  NVL_REQUIRE(q && k_cache && v_cache && block_tables && context_lens && out && workspace, "%s: null pointer", who);
+                  const void* plan, float* lse, bool open = false) {
+  NVL_REQUIRE(q && k_cache && v_cache && block_tables && context_lens && (out || open) && workspace, "%s: null pointer", who);
   NVL_REQUIRE(kv_dtype == NVL_KV_BF16 || kv_dtype == NVL_KV_FP8, "%s: kv_dtype=%d (0 bf16, 1 fp8 e4m3)", who, kv_dtype);
   NVL_REQUIRE(batch >= 0 && batch <= 32768, "%s: batch=%lld out of range [0, 32768]", who, (long long)batch);
   NVL_REQUIRE(num_kv_heads > 0 && num_q_heads % num_kv_heads == 0, "%s: Hq=%d not a multiple of Hkv=%d", who, num_q_heads, num_kv_heads);
@@ -2216,7 +2229,11 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
     NVL_REQUIRE(mfma, "%s: a plan with a shared prefix needs the matrix-core kernel (Hq/Hkv in 2 ... 16; got %d)", who, G);
     NVL_REQUIRE(block_size % 128 == 0, "%s: a shared prefix needs block_size %% 128 == 0 (got %d)", who, block_size);
   }
-  const int few = fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
+  if (open && !(fa && mfma && kv_dtype == NVL_KV_BF16 && open_parts(batch, num_kv_heads, max_context))) {
+    nvl_set_error("%s: only steps of up to 4 sequences and contexts of up to 16,384 tokens, bf16 caches and the matrix-core kernel's group sizes leave their parts open", who);
+    return NVL_EUNSUPPORTED;
+  }
+  const int few = open ? open_parts(batch, num_kv_heads, max_context) : fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
   if (few)
     return fa->qkv_splits > 0 ? launch_decode_few<true>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
                                                         max_context, softmax_scale, workspace, s, *fa, const_cast<void*>(plan), lse, few)
@@ -2333,15 +2350,14 @@ extern "C" int nvl_paged_attn_decode(const void* q, const void* k_cache, const v
                        plan, lse);
 }
 
-extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w,
+static int decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w,
                                            const void* k_norm_w, float eps, const float* cos_sin, int64_t max_pos,
                                            void* k_cache, void* v_cache, const int32_t* block_tables,
                                            int64_t bt_stride, const int32_t* context_lens, void* out, int64_t batch,
                                            int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks,
                                            int64_t max_context, float softmax_scale, void* workspace,
                                            size_t workspace_bytes, int kv_dtype, const void* plan, float* lse,
-                                           int qkv_splits, int64_t qkv_split_stride, void* stream) {
-  const char* who = "nvl_paged_attn_decode_fused";
+                                           int qkv_splits, int64_t qkv_split_stride, void* stream, const char* who, bool open) {
   NVL_REQUIRE(qkv_splits >= 0 && qkv_splits <= 8, "%s: qkv_splits=%d (0 = bf16 qkv, 1..8 = fp32 split-K slabs)", who, qkv_splits);
   NVL_REQUIRE(qkv_splits <= 1 || qkv_split_stride >= batch * qkv_tok_stride, "%s: qkv_split_stride=%lld < batch x qkv_tok_stride",
               who, (long long)qkv_split_stride);
@@ -2362,7 +2378,30 @@ extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stri
   fa.qkv_split_stride = (int)qkv_split_stride;
   return decode_common(qkv, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_q_heads,
                        num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes,
-                       stream, &fa, who, kv_dtype, plan, lse);
+                       stream, &fa, who, kv_dtype, plan, lse, open);
+}
+extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,
+                                           const float* cos_sin, int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables,
+                                           int64_t bt_stride, const int32_t* context_lens, void* out, int64_t batch, int num_q_heads,
+                                           int num_kv_heads, int block_size, int64_t num_blocks, int64_t max_context, float softmax_scale,
+                                           void* workspace, size_t workspace_bytes, int kv_dtype, const void* plan, float* lse, int qkv_splits,
+                                           int64_t qkv_split_stride, void* stream) {
+  return decode_fused(qkv, qkv_tok_stride, q_norm_w, k_norm_w, eps, cos_sin, max_pos, k_cache, v_cache, block_tables, bt_stride, context_lens, out,
+                      batch, num_q_heads, num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes, kv_dtype, plan,
+                      lse, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_fused", false);
+}
+extern "C" int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context) {
+  static_assert(kTile == 32 && kOpenPart == kFewWaves, "the projection counts the parts too");
+  return num_kv_heads > 0 && max_context > 0 ? open_parts(batch, num_kv_heads, max_context) : 0;
+}
+extern "C" int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,
+                                          const float* cos_sin, int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables,
+                                          int64_t bt_stride, const int32_t* context_lens, int64_t batch, int num_q_heads, int num_kv_heads,
+                                          int block_size, int64_t num_blocks, int64_t max_context, float softmax_scale, void* workspace,
+                                          size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream) {
+  return decode_fused(qkv, qkv_tok_stride, q_norm_w, k_norm_w, eps, cos_sin, max_pos, k_cache, v_cache, block_tables, bt_stride, context_lens, nullptr,
+                      batch, num_q_heads, num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes, NVL_KV_BF16, nullptr,
+                      nullptr, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_open", true);
 }
 
 // ---- per-step plan ------------------------------------------------------------------------------------------------

@@ -49,11 +49,23 @@ struct XTile {
   static constexpr int kLanesPerRow = KB * 4;      // 16-byte chunks per row
 };
 
-template <int MT, int KB, int NT, int EPI>
+// Attention outputs whose context is still in parts (nvl_paged_attn_decode_open): x[m][head 128 + d] is their merge, which every workgroup makes for its slice
+// of k. That takes 1 us of a launch of 3.4 for one row of 3 parts and 3 for 16; the attention kernel's own merge, through memory and by whoever arrives last, took 3 to 4 and
+// wanted few parts, whose tiles one compute unit takes in slowly. Decode steps of one sequence of Qwen3-0.6B: 700 tokens 925 -> 825 us, 2,000
+// 1032 -> 855, 4,000 1031 -> 909; four of 300 to 1,500 1004 -> 904; contexts of one part 741 -> 757 (60 tokens) and 806 -> 822 (four of up to 120).
+struct OpenAttn {
+  const float *po, *ml;            // [m][head][parts][128] and [m][head][parts][2]: maximum (base 2) and sum
+  const bf16_t* whole;             // [m][head][128]: contexts of one part, finished
+  const int32_t* ctx;
+  int parts;
+};
+
+template <int MT, int KB, int NT, int EPI, bool OPEN>
 __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* __restrict__ x,
                                                                   const bf16_t* __restrict__ w,
                                                                   void* __restrict__ out, int M, int N, int K,
-                                                                  int ko_iters, int packed) {
+                                                                  int ko_iters, int packed, OpenAttn oa) {
+  static_assert(!OPEN || MT == 1, "open parts: up to 16 rows");
   static_assert(EPI != EPI_SILU || NT == 2, "SILU pairs a gate tile with an up tile");
   constexpr int T = MT * NT;
   // NT == 1: two accumulation chains per tile (even / odd k blocks) hide the MFMA dependency latency;
@@ -136,6 +148,60 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
     };
     u32x4_t g[2][KB];
     auto gload = [&](int mt, u32x4_t* dst) {
+      if constexpr (OPEN) {
+        // (four parts are asked for together. Before it is known how many there are, which saves a request in the chain, they cost as much as it does; rows that
+        // are not there are left out: their requests alone took 1 us)
+        constexpr int FIRST = 4;
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+          const int c = i * 64 + lane, m = c / XT::kLanesPerRow, kc = (int)kw + (c % XT::kLanesPerRow) * 8;
+          dst[i] = u32x4_t{0u, 0u, 0u, 0u};
+          if (m >= M) continue;
+          const int64_t row = ((int64_t)m * (K >> 7) + (kc >> 7)) * oa.parts;
+          const float2* ml = reinterpret_cast<const float2*>(oa.ml) + row;
+          const float* po = oa.po + row * 128 + (kc & 127);
+          const int len = oa.ctx[m];
+          const u32x4_t one = *reinterpret_cast<const u32x4_t*>(oa.whole + (int64_t)m * K + kc);
+          float2 e[FIRST];
+          f32x4_t pa[FIRST], pb[FIRST];
+          const auto ask = [&](int k0, int last) {
+#pragma unroll
+            for (int j = 0; j < FIRST; ++j) {
+              const int k = k0 + j < last ? k0 + j : last;
+              e[j] = ml[k];
+              pa[j] = *reinterpret_cast<const f32x4_t*>(po + k * 128);
+              pb[j] = *reinterpret_cast<const f32x4_t*>(po + k * 128 + 4);
+            }
+          };
+          const int n = nvl_few_split((len + 31) / 32, NVL_OPEN_PART_TILES, oa.parts);
+          dst[i] = one;
+          if (n == 1) continue;
+          ask(0, n - 1);
+          float top = -1.0e30f, den = 0.f;
+          f32x4_t a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
+          for (int k0 = 0;;) {
+            float now = top;
+#pragma unroll
+            for (int j = 0; j < FIRST; ++j)
+              if (k0 + j < n) now = fmaxf(now, e[j].x);
+            const float old = __builtin_amdgcn_exp2f(top - now);
+            a *= old, b *= old, den *= old, top = now;
+#pragma unroll
+            for (int j = 0; j < FIRST; ++j)
+              if (k0 + j < n) {
+                const float f = __builtin_amdgcn_exp2f(e[j].x - top);
+                a += f * pa[j], b += f * pb[j], den += f * e[j].y;
+              }
+            k0 += FIRST;
+            if (k0 >= n) break;
+            ask(k0, n - 1);
+          }
+          const float inv = 1.f / den;
+          a *= inv, b *= inv;
+          dst[i] = u32x4_t{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+        }
+        return;
+      }
       const int64_t base = (int64_t)(m_base + mt * 16) * K + kw;
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
@@ -318,15 +384,15 @@ bool make_plan(int64_t m, int n, int k, int mode, Plan* p) {
   return true;
 }
 
-template <int MT, int KB, int NT, int EPI>
-int launch(const void* x, const void* w, void* out, int64_t m, int n, int k, const Plan& p, hipStream_t s) {
+template <int MT, int KB, int NT, int EPI, bool OPEN = false>
+int launch(const void* x, const void* w, void* out, int64_t m, int n, int k, const Plan& p, hipStream_t s, const OpenAttn& oa = OpenAttn()) {
   const size_t lds_red = (size_t)(kNW / 2) * MT * NT * 64 * sizeof(f32x4_t);
   const size_t lds_ring = (size_t)kNW * 2 * XTile<KB>::kBytes;
   const size_t lds = lds_red > lds_ring ? lds_red : lds_ring;
   static bool attr_done[NVL_MAX_DEVICES] = {};
   bool& attr_set = attr_done[nvl_device_slot()];
   if (!attr_set && lds > 64 * 1024) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_decode_kernel<MT, KB, NT, EPI>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_decode_kernel<MT, KB, NT, EPI, OPEN>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
       nvl_set_error("nvl_linear_decode: cannot reserve %zu B of LDS", lds);
       return NVL_ELAUNCH;
@@ -335,8 +401,8 @@ int launch(const void* x, const void* w, void* out, int64_t m, int n, int k, con
   }
   const int out_cols = EPI == EPI_SILU ? n / 2 : n;
   const int col_wgs = EPI == EPI_SILU ? out_cols / 16 : out_cols / 16 / NT;
-  hipLaunchKernelGGL((linear_decode_kernel<MT, KB, NT, EPI>), dim3(col_wgs, p.split, p.mgroups), dim3(kNW * 64), lds,
-                     s, (const bf16_t*)x, (const bf16_t*)w, out, (int)m, n, k, p.ko, g_packed);
+  hipLaunchKernelGGL((linear_decode_kernel<MT, KB, NT, EPI, OPEN>), dim3(col_wgs, p.split, p.mgroups), dim3(kNW * 64), lds,
+                     s, (const bf16_t*)x, (const bf16_t*)w, out, (int)m, n, k, p.ko, g_packed, oa);
   return nvl_check_launch("nvl_linear_decode");
 }
 
@@ -503,6 +569,28 @@ extern "C" int nvl_linear_decode(const void* x, const void* weight, void* out, i
                      : dispatch_kb<1, EPI_BF16>(x, weight, out, m, n, k, p, s);
   return p.nt == 2 ? dispatch_kb<2, EPI_PARTIAL>(x, weight, out, m, n, k, p, s)
                    : dispatch_kb<1, EPI_PARTIAL>(x, weight, out, m, n, k, p, s);
+}
+
+extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight,
+                                      void* out, int64_t m, int n, int k, int weight_layout, void* stream) {
+  NVL_REQUIRE(parts_o && parts_ml && whole && context_lens && weight && out, "nvl_linear_decode_open: null pointer");
+  NVL_REQUIRE(m >= 1 && m <= 16 && parts >= 1 && k % 128 == 0, "nvl_linear_decode_open: m=%lld k=%d parts=%d", (long long)m, k, parts);
+  NVL_REQUIRE(weight_layout == 0 || weight_layout == 1, "nvl_linear_decode_open: weight_layout=%d", weight_layout);
+  NVL_REQUIRE(((uintptr_t)parts_o | (uintptr_t)whole | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 && (uintptr_t)parts_ml % 8 == 0, "nvl_linear_decode_open: alignment");
+  Plan p;
+  if (!make_plan(m, n, k, EPI_PARTIAL, &p) || p.mt != 1 || p.nt != 1) {
+    nvl_set_error("nvl_linear_decode_open: shape m=%lld n=%d k=%d not covered", (long long)m, n, k);
+    return NVL_EUNSUPPORTED;
+  }
+  g_packed = weight_layout;
+  const OpenAttn oa = {parts_o, parts_ml, (const bf16_t*)whole, context_lens, parts};
+  hipStream_t s = (hipStream_t)stream;
+  switch (p.kb) {
+    case 1: return launch<1, 1, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
+    case 2: return launch<1, 2, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
+    case 3: return launch<1, 3, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
+    default: return launch<1, 4, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
+  }
 }
 
 extern "C" int nvl_add_rmsnorm_splitk(const float* partials, int splits, void* residual, const void* weight, void* y,

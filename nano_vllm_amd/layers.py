@@ -120,6 +120,8 @@ def get_rope(head_size: int, rotary_dim: int, max_position: int, base: float, de
 # NVL_FUSED_DECODE=0 keeps the separate q/k-norm+RoPE+KV-store launch on decode steps (A/B measurements)
 _FUSED_DECODE = os.environ.get("NVL_FUSED_DECODE", "1") != "0"
 
+# NVL_OPEN_ATTN=0 merges the parts of a context in the attention kernel also where the output projection could (A/B measurements)
+_OPEN_ATTN = os.environ.get("NVL_OPEN_ATTN", "1") != "0"
 # NVL_RAW_Q=0 keeps the query heads of prompt steps in the q/k-norm launch (A/B measurements)
 _RAW_Q = os.environ.get("NVL_RAW_Q", "1") != "0" and os.environ.get("NVL_PREFILL_W64") is None and os.environ.get("NVL_PREFILL_WAVES") is None
 
@@ -146,6 +148,25 @@ class Attention(nn.Module):
         """Does `forward_fused` take the one-launch decode path (norm + rope + KV store inside the attention kernel) for
         this step? Only then may `qkv` arrive as fp32 split-K slabs (QKVParallelLinear.forward_for_fused_decode)."""
         return not ctx.is_prefill and self.k_cache.numel() > 0 and _FUSED_DECODE
+
+    def forward_open(self, qkv: torch.Tensor, q_norm_w, k_norm_w, eps: float, rope_table: torch.Tensor, o_proj: RowParallelLinear):
+        """A decode step's attention and output projection where the projection merges the contexts' parts (steps of few sequences), or None."""
+        ctx = get_context()
+        if (not _OPEN_ATTN or qkv.dim() != 2 or qkv.shape[0] > 4 or o_proj.tp_size != 1 or o_proj.bias is not None or ctx.shared_prefix or qkv.dtype != torch.bfloat16
+                or self.k_cache.dtype != torch.bfloat16 or not self.fuses_decode_step(ctx)
+                or not ops.decode_attention_takes_qkv_slabs(self.num_heads, self.num_kv_heads)):
+            return None
+        b, (n, k) = qkv.shape[0], o_proj.weight.shape
+        max_context = ctx.max_context or ctx.block_tables.shape[1] * self.k_cache.shape[2]
+        if not ops.linear_decode_splits(b, n, k, ops.LINEAR_PARTIAL) or not ops.open_parts(b, self.num_kv_heads, max_context):
+            return None
+        ws = ctx.decode_workspace
+        if ws is None:
+            ws = torch.empty(ops.paged_attn_decode_workspace_bytes(b, self.num_heads, max_context), dtype=torch.uint8, device=qkv.device)
+        att = ops.paged_attn_decode_open(qkv, q_norm_w, k_norm_w, eps, rope_table, self.k_cache, self.v_cache, ctx.block_tables, ctx.context_lens,
+                                         self.num_heads, self.scale, max_context, ws)
+        w = o_proj.weight_packed
+        return ops.linear_decode_open(att, w if w is not None else o_proj.weight, packed=w is not None)
 
     # -- fused entry point: raw qkv GEMM output -> (q/k norm, rope, KV store) in one launch -------
     def forward_fused(self, qkv: torch.Tensor, positions: torch.Tensor, q_norm_w, k_norm_w, eps: float,

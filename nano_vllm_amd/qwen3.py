@@ -64,6 +64,10 @@ class Qwen3Attention(nn.Module):
             qkv = self.qkv_proj(hidden_states)
         qw = self.q_norm.weight if self.has_qk_norm else None
         kw = self.k_norm.weight if self.has_qk_norm else None
+        if not ctx.is_prefill:
+            y = self.attn.forward_open(qkv, qw, kw, self.eps, self.rotary_emb.cos_sin_cache, self.o_proj)
+            if y is not None:
+                return y
         o = self.attn.forward_fused(qkv, positions, qw, kw, self.eps, self.rotary_emb.cos_sin_cache)
         return self.o_proj.forward_decode(o.view(o.shape[0], -1))
 
