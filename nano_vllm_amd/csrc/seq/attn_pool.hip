@@ -8,17 +8,17 @@ namespace {
 constexpr int MAX_HEAD_POOL = 1024;
 
 // The mean of the `pool` cached tokens that end at position p into their block's place (see pool_unit), every kv head: the keys
-// (half 0) or the values (half 1), by all threads of the workgroup. Key rows are read a column per thread; values are transposed
+// (half 0) or the values (half 1), by all threads of the workgroup; `shares` workgroups may share a half's columns, of which this one is `share`. Key rows are read a column per thread; values are transposed
 // inside a page (and inside a unit of 8 blocks), so there LN neighbouring lanes share a column and read its consecutive tokens.
 template <typename T>
 __device__ void pool_block(int half, int p, const int32_t* __restrict__ bt, const T* k_cache, const T* v_cache, int G, int d, int dv,
-                           int block_size, int pool, T* pool_k, T* pool_v) {
+                           int block_size, int pool, T* pool_k, T* pool_v, int share = 0, int shares = 1) {
   const int b = p / pool, first = b * pool;
   const int64_t unit = pool_unit(b >> 3, pool, block_size, bt);
   const float inv = 1.f / (float)pool;
   const int nk = G * d, nv = G * dv;
   if (half == 0) {
-    for (int c = threadIdx.x; c < nk; c += blockDim.x) {
+    for (int c = share * blockDim.x + threadIdx.x; c < nk; c += shares * blockDim.x) {
       float sum = 0.f;
       for (int j = first; j <= p;) {                // a run of tokens inside one page at a time
         const int page = j / block_size, off = j - page * block_size;
@@ -35,7 +35,7 @@ __device__ void pool_block(int half, int p, const int32_t* __restrict__ bt, cons
   int ln = 1;
   while (ln < pool && ln < 16) ln <<= 1;
   const int sub = threadIdx.x & (ln - 1), step = blockDim.x / ln;
-  for (int c0 = threadIdx.x / ln; c0 - (int)(threadIdx.x / ln) < nv; c0 += 8 * step) {      // (every thread takes part in the shuffles)
+  for (int c0 = share * 8 * step + threadIdx.x / ln; c0 - (int)(threadIdx.x / ln) < nv; c0 += shares * 8 * step) {      // (every thread takes part in the shuffles)
     float sum[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) sum[u] = 0.f;
@@ -125,7 +125,8 @@ __global__ __launch_bounds__(256) void qk_rows_kernel(const T* __restrict__ q, i
 
 // Two workgroups (keys, values) per token of the step: the block whose last token it is. Workgroups are dealt to the eight XCDs in
 // turn and the tokens that end a block are `pool` apart, so tokens are dealt to workgroups in strides of `pool` (`runs` of them):
-// neighbouring workgroups then hold the ends of neighbouring blocks, and not one XCD all of them.
+// neighbouring workgroups then hold the ends of neighbouring blocks, and not one XCD all of them. A half is a chain of reads, a few columns at a time: in short
+// steps its columns are shared by up to eight workgroups (330 tokens, blocks of 16, eight heads of 128 + 128 in 32 bits: 44 us, now 10).
 template <typename T>
 __global__ __launch_bounds__(256) void pool_blocks_kernel(const T* k_cache, const T* v_cache, int G, int d, int dv, int block_size, int pool,
                                                           int64_t n, unsigned runs,
@@ -136,7 +137,8 @@ __global__ __launch_bounds__(256) void pool_blocks_kernel(const T* k_cache, cons
   if (t >= n) return;
   const int p = (int)pos[t];
   if ((p + 1) % pool != 0 || slots[t] < 0) return;
-  pool_block<T>(blockIdx.y, p, block_tables + (int64_t)tseq[t] * bt_stride, k_cache, v_cache, G, d, dv, block_size, pool, pool_k, pool_v);
+  pool_block<T>(blockIdx.y, p, block_tables + (int64_t)tseq[t] * bt_stride, k_cache, v_cache, G, d, dv, block_size, pool, pool_k, pool_v, blockIdx.z,
+                gridDim.z);
 }
 
 }  // namespace
@@ -171,7 +173,9 @@ extern "C" int nvs_pool_blocks(const void* k_cache, const void* v_cache, int dty
   if (n == 0) return NVS_OK;
   const int64_t runs = (n + pool - 1) / pool;
   NVS_REQUIRE(runs * pool < (1ll << 31), "nvs_pool_blocks: step too large");
-  NVS_DISPATCH(dtype, pool_blocks_kernel<T><<<dim3((unsigned)(runs * pool), 2), dim3(256), 0, (hipStream_t)stream>>>(
+  const int64_t room = 8192 / (runs * pool);         // (most workgroups hold no end of a block and leave; more of them cost long steps time)
+  const unsigned shares = room < 1 ? 1 : room > 8 ? 8 : (unsigned)room;
+  NVS_DISPATCH(dtype, pool_blocks_kernel<T><<<dim3((unsigned)(runs * pool), 2, shares), dim3(256), 0, (hipStream_t)stream>>>(
                           (const T*)k_cache, (const T*)v_cache, G, d, dv, block_size, pool, n, (unsigned)runs, slots, pos, block_tables, bt_stride, tseq,
                           (T*)pool_k, (T*)pool_v));
   return nvs_check_launch("nvs_pool_blocks");
