@@ -1592,14 +1592,16 @@ inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
 }
 
 // Left open for the output projection to merge (nvl_linear_decode_open), a part costs neither a trip through memory nor a wait for the others, so it
-// is a tile of each wavefront. us, attention and output projection (16 heads over 8 kv heads, 1,024 columns), merged here / open: one sequence of 100 tokens 8.8 / 8.9,
-// 256 9.6 / 9.8, 700 12.5 / 10.4, 2,000 16.3 / 12.1, 4,096 16.5 / 15.4, 12,000 22.3 / 21.1; four of 100 9.0 / 9.3, 700 13.7 / 11.4, 2,000 17.2 / 15.7. Eight of 2,000
+// is a tile of each wavefront. us, attention and output projection (16 heads over 8 kv heads, 1,024 columns), merged here / open: one sequence of 100 tokens 8.7 / 8.6,
+// 256 9.7 / 9.7, 700 12.9 / 10.6, 2,000 16.2 / 12.0, 4,000 16.3 / 14.2, 12,000 22.3 / 21.1; four of 100 9.3 / 9.1, 700 13.4 / 11.0, 2,000 17.3 / 15.2. Up to eight parts, since
+// the projection takes longer with more (4,000 tokens in 16: 7.4 + 6.6 us, in eight 8.6 + 5.2), 16 where contexts may pass 4,096 tokens (12,000 in eight: 25.2). Eight of 2,000
 // 25.9 / 26.5 (the projection reads every part in each of its workgroups), one of 30,000 33.5 / 36.5: those are merged here.
 constexpr int kOpenPart = NVL_OPEN_PART_TILES, kOpenParts = 16, kOpenRows = 4;
 inline int open_parts(int64_t batch, int hkv, int64_t max_context) {
   if (batch < 1 || batch > kOpenRows || batch * hkv > kFewGroups || max_context > 16384) return 0;
   int64_t parts = ((max_context + kTile - 1) / kTile + kOpenPart - 1) / kOpenPart;
-  if (parts > kOpenParts) parts = kOpenParts;
+  const int most = max_context <= 4096 ? kOpenParts / 2 : kOpenParts;
+  if (parts > most) parts = most;
   if (parts > kFewGroups / (batch * hkv)) parts = kFewGroups / (batch * hkv);
   return (int)parts;
 }

@@ -50,9 +50,9 @@ struct XTile {
 };
 
 // Attention outputs whose context is still in parts (nvl_paged_attn_decode_open): x[m][head 128 + d] is their merge, which every workgroup makes for its slice
-// of k. That takes 1 us of a launch of 3.4 for one row of 3 parts and 3 for 16; the attention kernel's own merge, through memory and by whoever arrives last, took 3 to 4 and
-// wanted few parts, whose tiles one compute unit takes in slowly. Decode steps of one sequence of Qwen3-0.6B: 700 tokens 925 -> 825 us, 2,000
-// 1032 -> 855, 4,000 1031 -> 909; four of 300 to 1,500 1004 -> 904; contexts of one part 741 -> 757 (60 tokens) and 806 -> 822 (four of up to 120).
+// of k. That takes 1 us beside a launch of 3.4 for one row of 3 parts, 1.8 for eight and 3.2 for 16; the attention kernel's own merge, through memory and by whoever arrives last, took 3 to 4 and
+// wanted few parts, whose tiles one compute unit takes in slowly. Decode steps of one sequence of Qwen3-0.6B: 700 tokens 923 -> 820 us, 2,000
+// 1030 -> 849, 4,000 1031 -> 907; four of 300 to 1,500 1003 -> 903; contexts of one part 740 -> 751 (60 tokens), 809 -> 821 (240) and 804 -> 818 (four of up to 120).
 struct OpenAttn {
   const float *po, *ml;            // [m][head][parts][128] and [m][head][parts][2]: maximum (base 2) and sum
   const bf16_t* whole;             // [m][head][128]: contexts of one part, finished
@@ -125,6 +125,18 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
   const int64_t k_wg = (int64_t)split * ko_iters * (kNW * KB * 32);
   for (int ko = 0; ko < ko_iters; ++ko) {
     const int64_t kw = k_wg + (int64_t)(ko * kNW + wave) * (KB * 32);
+    // OPEN: what tells the parts, and a context's row if it is one part, are asked for before the weights: what has landed is counted in order
+    int len[OPEN ? KB : 1];
+    u32x4_t one[OPEN ? KB : 1];
+    if constexpr (OPEN) {
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int c = i * 64 + lane, m = c / XT::kLanesPerRow < M ? c / XT::kLanesPerRow : M - 1;
+        len[i] = oa.ctx[m];
+        one[i] = *reinterpret_cast<const u32x4_t*>(oa.whole + (int64_t)m * K + kw + (c % XT::kLanesPerRow) * 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     u32x4_t wf[NT][KB];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -160,8 +172,6 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
           const int64_t row = ((int64_t)m * (K >> 7) + (kc >> 7)) * oa.parts;
           const float2* ml = reinterpret_cast<const float2*>(oa.ml) + row;
           const float* po = oa.po + row * 128 + (kc & 127);
-          const int len = oa.ctx[m];
-          const u32x4_t one = *reinterpret_cast<const u32x4_t*>(oa.whole + (int64_t)m * K + kc);
           float2 e[FIRST];
           f32x4_t pa[FIRST], pb[FIRST];
           const auto ask = [&](int k0, int last) {
@@ -173,8 +183,8 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
               pb[j] = *reinterpret_cast<const f32x4_t*>(po + k * 128 + 4);
             }
           };
-          const int n = nvl_few_split((len + 31) / 32, NVL_OPEN_PART_TILES, oa.parts);
-          dst[i] = one;
+          const int n = nvl_few_split((len[i] + 31) / 32, NVL_OPEN_PART_TILES, oa.parts);
+          dst[i] = one[i];
           if (n == 1) continue;
           ask(0, n - 1);
           float top = -1.0e30f, den = 0.f;
@@ -218,6 +228,7 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
     // software pipeline (order pinned with sched_barrier: hipcc otherwise sinks every load to its use):
     //   global loads run 2-3 tiles ahead in registers, the LDS image 1 tile ahead, and within an
     //   iteration the fragment reads of tile mt are issued BEFORE the LDS writes of tile mt+1.
+    if constexpr (OPEN) __builtin_amdgcn_sched_barrier(0);
     gload(0, g[0]);
     if (MT > 1) gload(1, g[1]);
     __builtin_amdgcn_sched_barrier(0);
