@@ -35,6 +35,7 @@
 // table) and substitutes them for that row of its register tile — the row is never read back
 // from HBM inside this launch, so there is no intra-launch dependency to order.
 #include "common.h"
+#include "few_split.h"
 #include <stdlib.h>
 #include <mutex>
 #include "rope_common.h"

@@ -138,14 +138,6 @@ __device__ __forceinline__ float wave_allreduce_max(float v) {
 // __logf on normal inputs.
 __device__ __forceinline__ float log_normal_f32(float x) { return __builtin_amdgcn_logf(x) * 0.6931471805599453f; }
 
-// Parts that a context of `tiles` tiles of 32 tokens is cut into: part_tiles tiles each, more where `parts` do not suffice (decode attention of few sequences, and the
-// projection that merges its open parts)
-constexpr int NVL_OPEN_PART_TILES = 8;           // ... of a part that is left open
-__device__ __forceinline__ int nvl_few_split(int tiles, int part_tiles, int parts) {
-  const int n = (tiles + part_tiles - 1) / part_tiles;
-  return n < 1 ? 1 : n < parts ? n : parts;
-}
-
 // ---- Philox4x32-10 (host + device, identical) -------------------------------------
 struct Philox4 {
   uint32_t v[4];

@@ -28,6 +28,7 @@
 //   SILU    out[m, j]            = bf16(silu(bf16(acc[gate j])) * bf16(acc[up j]))   (activation.py:8-11)
 //   PARTIAL part[split][m, n]    = acc (fp32), summed and rounded by the consumer
 #include "common.h"
+#include "few_split.h"
 #include <stdio.h>
 #include <stdlib.h>
 #include <type_traits>
