@@ -197,6 +197,10 @@ int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride,
                             void* k_cache, void* v_cache,
                             int64_t n_tok, int num_q_heads, int num_kv_heads,
                             int block_size, int64_t num_blocks, int kv_dtype, void* stream);
+/* The same without the query heads (nvl_attn_prefill_varlen_raw takes them from qkv): k_out, or k_cache and v_cache, or all three. */
+int nvl_knorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, const int64_t* positions, const void* k_norm_w, float eps, const float* cos_sin,
+                           int64_t max_pos, const int32_t* slot_mapping, void* k_out, void* k_cache, void* v_cache, int64_t n_tok,
+                           int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype, void* stream);
 
 /* ---- Paged decode attention ------------------------------------------------
  * Replaces flash_attn_with_kvcache as called at layers/attention.py:72-74:
@@ -342,7 +346,7 @@ int nvl_attn_prefill_varlen(const void* q, const void* k, const void* v,
                             float softmax_scale, int kv_dtype, float* lse, void* stream);
 /* The same on queries as the qkv projection leaves them: q rows q_tok_stride elements apart, head h at h * 128, normed with q_norm_w (NULL: not) and turned
  * by cos_sin[positions[t]] as nvl_qknorm_rope_kvstore would (same roundings), bf16 keys and values. For steps whose longest prompt is short (the kernels of
- * longer query tiles take finished queries only); nvl_qknorm_rope_kvstore with q_out NULL leaves the query heads out. */
+ * longer query tiles take finished queries only); nvl_knorm_rope_kvstore leaves the query heads out. */
 int nvl_attn_prefill_varlen_raw(const void* q, int64_t q_tok_stride, const int64_t* positions, const void* q_norm_w, float eps, const float* cos_sin,
                                 int64_t max_pos, const void* k, const void* v, int64_t k_tok_stride, int64_t v_tok_stride, const int32_t* cu_seqlens_q,
                                 const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride, void* out, int64_t total_q, int num_seqs,

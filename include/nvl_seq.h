@@ -104,13 +104,18 @@ int nvs_causal_conv(const void* in, int64_t in_stride, int dtype, const void* w,
  *   a = exp(-c * sigmoid(gr) * softplus(lam)),  S = a S + sqrt(1 - a^2) * sigmoid(gi) * u,  out = S * gelu_tanh(ypre).
  * S [nslots, C] 32-bit, advanced. out [n, C] `dtype`. Long portions of a step with few (portion, channel) threads are scanned
  * in segments, twice, in `ws` (nvs_rglru_scan_workspace floats; NULL: never), as nvs_ssd_scan below explains; max_q = the
- * longest portion of the step. u NULL: gates are the pairs of nvs_rglru_gates instead, [n][C][2]: log a and the term added to a S. */
-int nvs_rglru_gates(const float* u, const float* w, const float* bias, const void* lam, int dtype, float c, int channels, int blocks, int64_t n,
-                    float* pairs, void* stream);       /* blocks of 128: w [blocks][128][256], bias [blocks][256]; u, bias and pairs on 16-byte boundaries */
+ * longest portion of the step. */
 int64_t nvs_rglru_scan_workspace(int channels, int nseq, int64_t max_q);
 int nvs_rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam, float c,
                    int channels, int blocks, const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq, int64_t n,
                    int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream);
+
+/* The same in two steps: per token and channel pairs [n][C][2] of log a and the term added to a S, from the recurrence's own gates (blocks of 128 channels: w
+ * [blocks][128][256], bias [blocks][256]; u, bias and pairs on 16-byte boundaries), and the scan of them. */
+int nvs_rglru_gates(const float* u, const float* w, const float* bias, const void* lam, int dtype, float c, int channels, int blocks, int64_t n,
+                    float* pairs, void* stream);
+int nvs_rglru_scan_pairs(const float* pairs, const void* ypre, int64_t y_stride, int dtype, int channels, const int32_t* cu_q, const int32_t* ctx0,
+                         const int32_t* slot, int nseq, int64_t n, int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream);
 
 /* State-space-duality recurrence, recurrent form. xbc [n, inner + 2*G*N] 32-bit (x | B | C after convolution + SiLU),
  * dt: column dt_col .. dt_col + heads of proj [n, proj_stride] (`dtype`); dt_bias, A_log, D [heads] (`dtype`). Per head h
@@ -302,11 +307,14 @@ int nvs_moe_combine(const void* rows, int64_t ldr, const int32_t* pair_row, cons
  * With kv_col >= 0, columns kv_col .. + kv_rank are RMS-normed with kv_norm (the latent c) and the next rot_dim columns are the
  * shared key part: its leading rot_dims entries turn by pos[t] * rot_freq[i], i < rot_dims / 2, pair (2i, 2i+1) or, with
  * rot_halves, (i, i + rot_dims / 2); cos and sin are multiplied by rot_mag. Token t goes to cache slot slots[t] (< 0: skipped):
- * k_cache [slot][kv_rank + rot_dim] = [c | rotated part]; v_cache [page][kv_rank][block_size] = c, transposed inside the page. turn (may be
- * NULL) [n][rot_dims / 2][2] 32-bit: the cosines and sines of all tokens, for nvs_latent_heads. */
+ * k_cache [slot][kv_rank + rot_dim] = [c | rotated part]; v_cache [page][kv_rank][block_size] = c, transposed inside the page. */
 int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
                     int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims, int rot_halves,
-                    float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache, void* turn, int64_t n, void* stream);
+                    float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache, int64_t n, void* stream);
+/* The same; turn [n][rot_dims / 2][2] 32-bit receives the cosines and sines of all tokens, for nvs_latent_heads. */
+int nvs_latent_prep_turn(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col, int kv_rank,
+                         int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims, int rot_halves, float rot_mag, float eps,
+                         int block_size, const int32_t* slots, void* k_cache, void* v_cache, void* turn, int64_t n, void* stream);
 
 /* out[t, h, 0 .. width) = in[t, h, 0 .. width) with the leading rot_dims entries rotated as above; rows t have strides in_stride /
  * out_stride, heads in_head / out_head (elements, `dtype`). */
@@ -315,7 +323,7 @@ int nvs_rotate_heads(const void* in, int64_t in_stride, int in_head, void* out, 
                      void* stream);
 
 /* bf16: y[t, a, 0 .. N) = W_a x[t, a, 0 .. K) for every head a; K and N 64, 128, 192 or 256. w [H][N][K], with `turned` [H][K][N]. With `turned`, the
- * `tail` entries behind x's K go behind y's N, the leading rot_dims of them turned by `turn` ([n][rot_dims / 2][2], nvs_latent_prep). Strides in entries, multiples
+ * `tail` entries behind x's K go behind y's N, the leading rot_dims of them turned by `turn` ([n][rot_dims / 2][2], nvs_latent_prep_turn). Strides in entries, multiples
  * of 8; x, w and y on 16-byte boundaries. */
 int nvs_latent_heads(const void* x, int64_t ldx, int xh, const void* w, int turned, int K, int N, void* y, int64_t ldy, int yh, int H, int tail,
                      int rot_dims, int rot_halves, const void* turn, int64_t n, void* stream);

@@ -166,13 +166,10 @@ extern "C" int nvl_store_kvcache(const void* k, int64_t k_tok_stride, const void
   return nvl_check_launch("nvl_store_kvcache");
 }
 
-extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, const int64_t* positions,
-                                       const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
-                                       int64_t max_pos, const int32_t* slot_mapping, void* q_out, void* k_out,
-                                       void* k_cache, void* v_cache, int64_t n_tok, int num_q_heads,
-                                       int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype,
-                                       void* stream) {
-  NVL_REQUIRE(qkv && positions && cos_sin && (q_out || k_out || k_cache), "nvl_qknorm_rope_kvstore: null pointer");
+// q_out NULL: without the query heads
+static int qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, const int64_t* positions, const void* q_norm_w, const void* k_norm_w, float eps,
+                               const float* cos_sin, int64_t max_pos, const int32_t* slot_mapping, void* q_out, void* k_out, void* k_cache, void* v_cache,
+                               int64_t n_tok, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype, void* stream) {
   NVL_REQUIRE(kv_dtype == NVL_KV_BF16 || kv_dtype == NVL_KV_FP8, "nvl_qknorm_rope_kvstore: kv_dtype=%d (0 bf16, 1 fp8 e4m3)", kv_dtype);
   NVL_REQUIRE((q_norm_w == nullptr) == (k_norm_w == nullptr), "nvl_qknorm_rope_kvstore: q/k norm weights must both be set or both NULL");
   NVL_REQUIRE((k_cache == nullptr) == (v_cache == nullptr), "nvl_qknorm_rope_kvstore: k_cache/v_cache must both be set or both NULL");
@@ -200,4 +197,23 @@ extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, 
   }
 #undef NVL_QK
   return nvl_check_launch("nvl_qknorm_rope_kvstore");
+}
+
+extern "C" int nvl_qknorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, const int64_t* positions,
+                                       const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
+                                       int64_t max_pos, const int32_t* slot_mapping, void* q_out, void* k_out,
+                                       void* k_cache, void* v_cache, int64_t n_tok, int num_q_heads,
+                                       int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype,
+                                       void* stream) {
+  NVL_REQUIRE(qkv && positions && cos_sin && q_out, "nvl_qknorm_rope_kvstore: null pointer");
+  return qknorm_rope_kvstore(qkv, qkv_tok_stride, positions, q_norm_w, k_norm_w, eps, cos_sin, max_pos, slot_mapping, q_out, k_out, k_cache, v_cache, n_tok,
+                             num_q_heads, num_kv_heads, block_size, num_blocks, kv_dtype, stream);
+}
+
+extern "C" int nvl_knorm_rope_kvstore(const void* qkv, int64_t qkv_tok_stride, const int64_t* positions, const void* k_norm_w, float eps, const float* cos_sin,
+                                      int64_t max_pos, const int32_t* slot_mapping, void* k_out, void* k_cache, void* v_cache, int64_t n_tok,
+                                      int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int kv_dtype, void* stream) {
+  NVL_REQUIRE(qkv && positions && cos_sin && (k_out || k_cache), "nvl_knorm_rope_kvstore: null pointer");
+  return qknorm_rope_kvstore(qkv, qkv_tok_stride, positions, k_norm_w, k_norm_w, eps, cos_sin, max_pos, slot_mapping, nullptr, k_out, k_cache, v_cache, n_tok,
+                             num_q_heads, num_kv_heads, block_size, num_blocks, kv_dtype, stream);
 }

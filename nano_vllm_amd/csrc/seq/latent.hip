@@ -96,10 +96,9 @@ __global__ void rotate_heads_kernel(const T* __restrict__ in, int64_t in_stride,
 
 }  // namespace
 
-extern "C" int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
-                               int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims,
-                               int rot_halves, float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache,
-                               void* turn, int64_t n, void* stream) {
+static int latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col, int kv_rank, int rot_dim,
+                       const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims, int rot_halves, float rot_mag, float eps, int block_size,
+                       const int32_t* slots, void* k_cache, void* v_cache, void* turn, int64_t n, void* stream) {
   NVS_REQUIRE(proj && q_norm && cq && q_col >= 0 && q_rank > 0 && stride >= q_col + q_rank && n >= 0, "nvs_latent_prep: query latent %d + %d of %lld",
               q_col, q_rank, (long long)stride);
   if (kv_col >= 0) {
@@ -115,6 +114,23 @@ extern "C" int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int 
                           (const T*)proj, stride, q_col, q_rank, (const T*)q_norm, (T*)cq, kv_col, kv_rank, rot_dim, (const T*)kv_norm, pos,
                           rot_freq, rot_dims, rot_halves, rot_mag, eps, block_size, slots, (T*)k_cache, (T*)v_cache, (float2*)turn));
   return nvs_check_launch("nvs_latent_prep");
+}
+
+extern "C" int nvs_latent_prep(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
+                               int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims,
+                               int rot_halves, float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache,
+                               int64_t n, void* stream) {
+  return latent_prep(proj, stride, dtype, q_col, q_rank, q_norm, cq, kv_col, kv_rank, rot_dim, kv_norm, pos, rot_freq, rot_dims, rot_halves, rot_mag, eps,
+                     block_size, slots, k_cache, v_cache, nullptr, n, stream);
+}
+
+extern "C" int nvs_latent_prep_turn(const void* proj, int64_t stride, int dtype, int q_col, int q_rank, const void* q_norm, void* cq, int kv_col,
+                                    int kv_rank, int rot_dim, const void* kv_norm, const int64_t* pos, const float* rot_freq, int rot_dims,
+                                    int rot_halves, float rot_mag, float eps, int block_size, const int32_t* slots, void* k_cache, void* v_cache,
+                                    void* turn, int64_t n, void* stream) {
+  NVS_REQUIRE(turn, "nvs_latent_prep_turn: null argument");
+  return latent_prep(proj, stride, dtype, q_col, q_rank, q_norm, cq, kv_col, kv_rank, rot_dim, kv_norm, pos, rot_freq, rot_dims, rot_halves, rot_mag, eps,
+                     block_size, slots, k_cache, v_cache, turn, n, stream);
 }
 
 extern "C" int nvs_rotate_heads(const void* in, int64_t in_stride, int in_head, void* out, int64_t out_stride, int out_head, int dtype, int H,

@@ -188,7 +188,7 @@ __global__ void rglru_scan_kernel(const float* __restrict__ gates, const float* 
   if (q1 <= q0) return;
   const bool last = q1 == p1;
   const int bw = channels / blocks, blk = c / bw, cc = c - blk * bw;
-  const float sp = softplusf_(ldf(lam + c));
+  const float sp = READY ? 0.f : softplusf_(ldf(lam + c));
   float* sp_state = S + (int64_t)slot[s] * channels + c;
   float* wv = ws + ((int64_t)s * (nseg + 1)) * 2 * channels + c;          // entry e: value at + 2 e C, decay at + (2 e + 1) C
   float st = 0.f;
@@ -805,10 +805,10 @@ extern "C" int nvs_causal_conv(const void* in, int64_t in_stride, int dtype, con
   return rc;
 }
 
-extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam,
-                              float c, int channels, int blocks, const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq,
-                              int64_t n, int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream) {
-  NVS_REQUIRE(gates && ypre && lam && cu_q && ctx0 && slot && S && out, "nvs_rglru_scan: null argument");
+// u NULL: gates are pairs, and lam is not read
+static int rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam, float c, int channels, int blocks,
+                      const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq, int64_t n, int64_t max_q, float* S, void* out, float* ws,
+                      int64_t ws_floats, void* stream) {
   NVS_REQUIRE(channels > 0 && blocks > 0 && channels % blocks == 0 && y_stride >= channels && nseq >= 0 && nseq <= 65535 && n >= 0,
               "nvs_rglru_scan: channels %d blocks %d", channels, blocks);
   if (n == 0 || nseq == 0) return NVS_OK;
@@ -839,6 +839,20 @@ extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* yp
 #undef NVS_RGLRU_LAUNCH
 #undef NVS_RGLRU_KERNEL
   return nvs_check_launch("nvs_rglru_scan");
+}
+
+extern "C" int nvs_rglru_scan(const float* gates, const float* u, const void* ypre, int64_t y_stride, int dtype, const void* lam,
+                              float c, int channels, int blocks, const int32_t* cu_q, const int32_t* ctx0, const int32_t* slot, int nseq,
+                              int64_t n, int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream) {
+  NVS_REQUIRE(gates && u && ypre && lam && cu_q && ctx0 && slot && S && out, "nvs_rglru_scan: null argument");
+  return rglru_scan(gates, u, ypre, y_stride, dtype, lam, c, channels, blocks, cu_q, ctx0, slot, nseq, n, max_q, S, out, ws, ws_floats, stream);
+}
+
+extern "C" int nvs_rglru_scan_pairs(const float* pairs, const void* ypre, int64_t y_stride, int dtype, int channels, const int32_t* cu_q, const int32_t* ctx0,
+                                    const int32_t* slot, int nseq, int64_t n, int64_t max_q, float* S, void* out, float* ws, int64_t ws_floats, void* stream) {
+  NVS_REQUIRE(pairs && ypre && cu_q && ctx0 && slot && S && out, "nvs_rglru_scan_pairs: null argument");
+  NVS_REQUIRE((uintptr_t)pairs % 8 == 0, "nvs_rglru_scan_pairs: pairs on 8-byte boundaries");
+  return rglru_scan(pairs, nullptr, ypre, y_stride, dtype, nullptr, 0.f, channels, 1, cu_q, ctx0, slot, nseq, n, max_q, S, out, ws, ws_floats, stream);
 }
 
 // Segments for long portions when (portion, head) pairs alone would leave compute units idle: seg_len 0 = none.

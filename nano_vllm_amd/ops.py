@@ -41,6 +41,8 @@ SIGNATURES = {
     "nvl_qknorm_rope_kvstore": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int64,
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
                                         c_int64, c_int, c_void_p]),
+    "nvl_knorm_rope_kvstore": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                       c_int, c_int, c_int, c_int64, c_int, c_void_p]),
     "nvl_paged_attn_decode_workspace_bytes": (c_size_t, [c_int64, c_int, c_int64]),
     "nvl_paged_attn_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                       c_int, c_int, c_int, c_int64, c_int64, c_float, c_void_p, c_size_t, c_int,
@@ -347,17 +349,16 @@ def qknorm_rope_kvstore(qkv: torch.Tensor, positions: torch.Tensor, q_norm_w, k_
     _dev(qkv, "qkv")
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.dtype == torch.bfloat16
     has_cache = k_cache is not None and k_cache.numel() > 0
-    _check(lib().nvl_qknorm_rope_kvstore(
-        qkv.data_ptr(), qkv.stride(0), positions.data_ptr(),
-        q_norm_w.data_ptr() if q_norm_w is not None else None,
-        k_norm_w.data_ptr() if k_norm_w is not None else None, eps,
-        cos_sin.data_ptr(), cos_sin.shape[0],
-        slot_mapping.data_ptr() if (has_cache and slot_mapping is not None) else None,
-        q_out.data_ptr() if q_out is not None else None, k_out.data_ptr() if k_out is not None else None,
-        k_cache.data_ptr() if has_cache else None, v_cache.data_ptr() if has_cache else None,
-        qkv.shape[0], num_q_heads, num_kv_heads,
-        k_cache.shape[2] if has_cache else 0, k_cache.shape[0] if has_cache else 0,
-        kv_dtype_of(k_cache) if has_cache else KV_BF16, _stream()))
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    head = (qkv.data_ptr(), qkv.stride(0), positions.data_ptr())
+    rope = (eps, cos_sin.data_ptr(), cos_sin.shape[0], ptr(slot_mapping) if has_cache else None)
+    tail = (ptr(k_out), ptr(k_cache) if has_cache else None, ptr(v_cache) if has_cache else None, qkv.shape[0], num_q_heads, num_kv_heads,
+            k_cache.shape[2] if has_cache else 0, k_cache.shape[0] if has_cache else 0, kv_dtype_of(k_cache) if has_cache else KV_BF16, _stream())
+    if q_out is not None:
+        _check(lib().nvl_qknorm_rope_kvstore(*head, ptr(q_norm_w), ptr(k_norm_w), *rope, q_out.data_ptr(), *tail))
+    else:
+        assert (q_norm_w is None) == (k_norm_w is None)
+        _check(lib().nvl_knorm_rope_kvstore(*head, ptr(k_norm_w), *rope, *tail))
 
 
 def paged_attn_decode_workspace_bytes(max_batch: int, num_q_heads: int, max_context: int) -> int:

@@ -35,6 +35,7 @@ SIGNATURES = {
     "nvs_rglru_scan_workspace": (c_int64, [_I, _I, _L]),
     "nvs_rglru_gates": (c_int, [_P, _P, _P, _P, _I, _F, _I, _I, _L, _P, _P]),
     "nvs_rglru_scan": (c_int, [_P, _P, _P, _L, _I, _P, _F, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
+    "nvs_rglru_scan_pairs": (c_int, [_P, _P, _L, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
     "nvs_ssd_scan_workspace": (c_int64, [_I, _I, _I, _I, _L]),
     "nvs_ssd_scan": (c_int, [_P, _P, _L, _L, _I, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
     "nvs_decay_scan": (c_int, [_P, _L, _L, _L, _L, _I, _P, _I, _I, _I, _P, _P, _P, _I, _L, _L, _P, _P, _P, _L, _P]),
@@ -55,7 +56,8 @@ SIGNATURES = {
                                 _I, _I, _P, _P, _P, _I, _P, _F, _I, _P, _P]),
     "nvs_add_group_norm": (c_int, [_P, _P, _F, _P, _P, _L, _P, _I, _I, _I, _F, _I, _P, _P]),
     "nvs_scale_softcap": (c_int, [_P, _I, _F, _F, _L, _P, _P]),
-    "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _P, _L, _P]),
+    "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _L, _P]),
+    "nvs_latent_prep_turn": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _P, _L, _P]),
     "nvs_latent_heads": (c_int, [_P, _L, _I, _P, _I, _I, _I, _P, _L, _I, _I, _I, _I, _I, _P, _L, _P]),
     "nvs_rotate_heads": (c_int, [_P, _L, _I, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _L, _P]),
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
@@ -230,6 +232,10 @@ def rglru_scan(gates: torch.Tensor, u: torch.Tensor | None, ypre: torch.Tensor, 
     assert out.shape == (n, channels) and out.is_contiguous()
     need = 0 if torch.cuda.is_current_stream_capturing() else lib.nvs_rglru_scan_workspace(channels, por.nseq, por.max_q)
     ws = torch.empty(need, dtype=torch.float32, device=out.device) if need else None
+    if u is None:
+        _check(lib.nvs_rglru_scan_pairs(_ptr(gates), _ptr(ypre), ypre.stride(0), _same(ypre, lam, out), channels, _ptr(por.cu_q), _ptr(por.ctx0), _ptr(por.slot),
+                                        por.nseq, n, por.max_q, _ptr(S), _ptr(out), _ptr(ws), need, _stream()))
+        return
     _check(lib.nvs_rglru_scan(_ptr(gates), _ptr(u), _ptr(ypre), ypre.stride(0), _same(ypre, lam, out), _ptr(lam), c, channels,
                               blocks, _ptr(por.cu_q), _ptr(por.ctx0), _ptr(por.slot), por.nseq, n, por.max_q, _ptr(S), _ptr(out), _ptr(ws), need,
                               _stream()))
@@ -582,10 +588,14 @@ def latent_prep(proj: torch.Tensor, q_col: int, q_rank: int, q_norm: torch.Tenso
         assert k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape[0] % block_size == 0
         assert tuple(k_cache.shape[1:]) == (1, kv_rank + rot_dim) and tuple(v_cache.shape[1:]) == (1, kv_rank)
         assert rot is None or (rot.freq.is_cuda and rot.dims <= rot_dim)
-    _check(lib.nvs_latent_prep(_ptr(proj), proj.stride(0), _same(proj, q_norm, cq, kv_norm, k_cache, v_cache), q_col, q_rank, _ptr(q_norm),
-                               _ptr(cq), kv_col, kv_rank, rot_dim, _ptr(kv_norm), _ptr(pos), _ptr(rot.freq) if rot else None,
-                               rot.dims if rot else 0, int(rot.halves) if rot else 0, rot.mag if rot else 1.0, eps, block_size, _ptr(slots),
-                               _ptr(k_cache), _ptr(v_cache), _ptr(turn), n, _stream()))
+    args = (_ptr(proj), proj.stride(0), _same(proj, q_norm, cq, kv_norm, k_cache, v_cache), q_col, q_rank, _ptr(q_norm),
+            _ptr(cq), kv_col, kv_rank, rot_dim, _ptr(kv_norm), _ptr(pos), _ptr(rot.freq) if rot else None,
+            rot.dims if rot else 0, int(rot.halves) if rot else 0, rot.mag if rot else 1.0, eps, block_size, _ptr(slots),
+            _ptr(k_cache), _ptr(v_cache))
+    if turn is None or not turn.numel():
+        _check(lib.nvs_latent_prep(*args, n, _stream()))
+    else:
+        _check(lib.nvs_latent_prep_turn(*args, _ptr(turn), n, _stream()))
 
 
 _HEAD_SIZES = (64, 128, 192, 256)

@@ -194,3 +194,22 @@ def test_qknorm_refuses_more_heads_than_its_kernel_counts():
     for n in (1 << 26, (1 << 26) - 1, 1 << 27, 1 << 30):         # 32 heads a token: from 2^31 - 32 heads on
         rc = lib.nvl_qknorm_rope_kvstore(p, 32 * 128, p, p, p, 1e-6, p, 8, p, p, p, p, p, n, 16, 8, 256, 1 << 20, 0, None)
         assert rc == -1 and b"too many rows" in lib.nvl_last_error(), n
+
+
+def test_entry_points_keep_their_arguments():
+    """A caller built against an earlier header of the same version number: argument lists as they were (checked on the host, before anything is launched), and
+    what was refused is refused."""
+    from nano_vllm_amd import ops, ops_seq
+    seq, p = ops_seq.load_library(), 16
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "nvl_seq.h")).read(), flags=re.S)
+    for name, (_, argtypes) in ops_seq.SIGNATURES.items():
+        args = re.search(r"\b%s\s*\(([^;]*?)\)\s*;" % name, text, flags=re.S).group(1).strip()
+        assert (0 if args in ("", "void") else args.count(",") + 1) == len(argtypes), name
+    # n is the last but one: no rows, and no such number of rows
+    prep = (p, 512, 0, 0, 256, p, p, 256, 128, 64, p, p, p, 64, 0, 1.0, 1e-6, 256, p, p, p)
+    assert seq.nvs_latent_prep(*prep, 0, None) == 0
+    assert seq.nvs_latent_prep(*prep, -1, None) == -1 and b"query latent" in seq.nvs_last_error()
+    rc = seq.nvs_rglru_scan(p, None, p, 256, 0, p, 8.0, 256, 2, p, p, p, 4, 4, 1, p, p, None, 0, None)
+    assert rc == -1 and b"null argument" in seq.nvs_last_error()
+    rc = ops.load_library().nvl_qknorm_rope_kvstore(p, 32 * 128, p, p, p, 1e-6, p, 8, p, None, p, p, p, 4, 16, 8, 256, 1 << 20, 0, None)
+    assert rc == -1 and b"null pointer" in ops.lib().nvl_last_error()
