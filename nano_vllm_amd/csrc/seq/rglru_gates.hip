@@ -9,6 +9,9 @@
 // straight into the order the instruction reads, a pass ahead, and splits them there. Lane: a token, four neighbouring channels of both gates, so the gates'
 // arithmetic happens where the sums are and a token's 16 channels leave as one 128-byte line.
 //
+// An infinity is its first part alone, but its products with another number's parts that are 0 are not numbers: where the matrices or a pass's rows hold one, results that
+// are no numbers are summed up again in 32 bits as they stand.
+//
 // What bounds it: the gates' arithmetic (two sigmoids, an exponential, 1 - a^2 and its root: about 70 vector instructions per value, 140 us of 57 million values) beside
 // 690 MB of traffic (135 us) and 75 us of products. 13,550 tokens, 4,096 channels: 230 to 250 us; a library product in 32 bits with the bias copied in
 // front of it took 595, and both passes of the scan did the arithmetic again (213 + 307 us; reading pairs 80 + 153).
@@ -46,7 +49,7 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
                                                           const T* __restrict__ lam, float c, int channels, int blocks, int64_t n, int rows,
                                                           float* __restrict__ pairs) {
   extern __shared__ __attribute__((aligned(128))) char lds[];
-  __shared__ int more;                              // some entry is more than its first part
+  __shared__ int more, odd;                         // some entry is more than its first part; some entry is not finite
   __shared__ float plus[SLICE];                     // softplus(lam)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, q = lane >> 4;
   const int slices = blocks * (BW / SLICE), slice = blockIdx.x % slices, blk = slice / (BW / SLICE), half = slice % (BW / SLICE);
@@ -68,11 +71,12 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
   int64_t at = begin + wave * 32;
   if (at < end) bring(at);
   // feature row f (gate r: f < 64) of a part: 16-byte unit k8 at k8 ^ (f & 15)
-  if (tid == 0) more = 0;
+  if (tid == 0) more = odd = 0;
   if (tid < SLICE) plus[tid] = softplusf_(ldf(lam + blk * BW + half * SLICE + tid));
   __syncthreads();
   const float* wb = w + (int64_t)blk * BW * 2 * BW + half * SLICE;
   bool mine = false;
+  float odd_entries = 0.f;
   constexpr int ITEMS = 2 * SLICE * BW / 8 / 512;
   const int f = tid % (2 * SLICE);
   f32x4_t lo[ITEMS], hi[ITEMS];                     // (asked for together: their way here is most of a decode step's time)
@@ -82,6 +86,10 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
 #pragma unroll
     for (int j = 0; j < 4; ++j) lo[i][j] = from[j * 2 * BW], hi[i][j] = from[(j + 4) * 2 * BW];
   }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) odd_entries += lo[i][j] * 0.f + hi[i][j] * 0.f;
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const int k8 = (tid + i * 512) / (2 * SLICE);
@@ -94,8 +102,9 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
     }
   }
   if (mine) more = 1;
+  if (odd_entries != 0.f) odd = 1;
   __syncthreads();
-  const bool whole = more == 0;
+  const bool whole = more == 0, odd_matrices = odd != 0;
   const int c0 = blk * BW + half * SLICE + q * 4;   // this lane's channels: c0 + 16 fb + 0..3
   float sp[4][4];
 #pragma unroll
@@ -108,6 +117,13 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
     f32x4_t acc[8][2];
 #pragma unroll
     for (int fb = 0; fb < 8; ++fb) acc[fb][0] = acc[fb][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    bool strange = odd_matrices;
+    if (!whole) {
+      f32x4_t odd_rows = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) odd_rows += (x[s][0][0] * 0.f + x[s][0][1] * 0.f) + (x[s][1][0] * 0.f + x[s][1][1] * 0.f);
+      strange |= __ballot(odd_rows[0] + odd_rows[1] + odd_rows[2] + odd_rows[3] != 0.f) != 0;
+    }
     const auto operand = [&](int part, int fb, int s) {
       return *(const bf16x8_t*)(lds + part * PART_BYTES + (fb * 16 + li) * BW * 2 + (((s * 4 + q) ^ li) << 4));
     };
@@ -159,6 +175,27 @@ __global__ __launch_bounds__(512) void rglru_gates_kernel(const float* __restric
         f32x4_t* to = (f32x4_t*)(pairs + (t * channels + c0 + fb * 16) * 2);
         to[0] = out[0];
         to[1] = out[1];
+      }
+    }
+    if (strange) {                                  // this lane's results again, those that are no numbers
+#pragma unroll 1
+      for (int j = 0; j < 32; ++j) {
+        const int64_t t = now + (j >> 4) * 16 + li;
+        const int ch = c0 + (j >> 2 & 3) * 16 + (j & 3), in_block = ch - blk * BW;
+        if (t >= end) continue;
+        float* to = pairs + (t * channels + ch) * 2;
+        if (to[0] == to[0] && to[1] == to[1]) continue;
+        const float* col = w + (int64_t)blk * BW * 2 * BW + in_block;
+        const float* bs = bias + (int64_t)blk * 2 * BW + in_block;
+        float gr = 0.f, gi = 0.f;
+#pragma unroll 1
+        for (int k = 0; k < BW; ++k) {
+          const float uk = ub[t * channels + k];
+          gr = fmaf(col[k * 2 * BW], uk, gr), gi = fmaf(col[k * 2 * BW + BW], uk, gi);
+        }
+        const RglruTerms v = rglru_terms(gr + bs[0], gi + bs[BW], u[t * channels + ch], plus[in_block - half * SLICE], c);
+        to[0] = v.la;
+        to[1] = v.add;
       }
     }
   }

@@ -64,3 +64,32 @@ def test_an_infinite_input_stays_in_its_block():
     assert torch.isfinite(pairs[:7]).all() and torch.isfinite(pairs[8:]).all() and torch.isfinite(pairs[7, 128:]).all()
     la = -8.0 * torch.sigmoid(z[7, :128]) * torch.nn.functional.softplus(lam[:128].double())       # gates of plus or minus infinity: 1 or 0
     assert torch.allclose(pairs[7, :128, 0].double(), la, rtol=1e-6, atol=1e-30)
+
+
+@pytest.mark.parametrize("where", ["input", "matrix", "both"])
+@pytest.mark.parametrize("exact", [True, False])
+def test_infinities_beside_parts_that_are_zero(exact, where):
+    """Weights whose second and third parts are 0 among such as need them, inputs of one part, an infinity in either: gates of plus or minus infinity are 1 or 0, and no
+    other token or block is touched."""
+    from nano_vllm_amd import ops_seq
+    u, w, b, lam = _case(300, 2, exact, 5)
+    w[0, 5, ::3] = 0.5
+    w[0, 5, 1::3] = -1.0
+    u[:, ::2] = u[:, ::2].bfloat16().float()
+    calm = ops_seq.rglru_gates(u, w, b, lam, 8.0, 2)
+    if where != "matrix":
+        u[7, 5], u[270, 5] = float("inf"), -float("inf")
+    if where != "input":
+        w[0, 64, 70], w[0, 64, 200] = float("inf"), -float("inf")
+    pairs = ops_seq.rglru_gates(u, w, b, lam, 8.0, 2)
+    want = torch.stack(_terms(u, w, b, lam, 2), -1)
+    lost = want.isnan().any(-1, keepdim=True)          # (infinities of both signs in one sum: a state that is multiplied by it is no number, whatever is added)
+    assert torch.equal(pairs.isnan().any(-1, keepdim=True), lost) and torch.equal(pairs.isinf() & ~lost, want.isinf() & ~lost)
+    finite = want.isfinite() & ~lost
+    assert float((pairs.double() - want)[finite].norm() / want[finite].norm()) <= 5e-7
+    touched = torch.zeros_like(finite)
+    if where != "matrix":
+        touched[[7, 270], :128] = True
+    if where != "input":
+        touched[:, [70, 200 - 128]] = True
+    assert torch.equal(pairs[~touched], calm[~touched])
