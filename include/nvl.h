@@ -310,7 +310,9 @@ int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const vo
                                int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables, int64_t bt_stride, const int32_t* context_lens,
                                int64_t batch, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int64_t max_context,
                                float softmax_scale, void* workspace, size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream);
-/* nvl_linear_decode mode 2 of the merge of those parts, rounded to bf16: m <= 16 rows of k = Hq * 128 entries */
+/* nvl_linear_decode mode 2 of the merge of those parts, rounded to bf16: m <= 16 rows of k = Hq * 128 entries. nvl_linear_decode_open_splits: the K-slices it
+ * emits, 0 where it does not take the shape (ask before the attention leaves its parts open). */
+int nvl_linear_decode_open_splits(int64_t m, int n, int k);
 int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight, void* out,
                            int64_t m, int n, int k, int weight_layout, void* stream);
 /* qkv_splits (ABI 4): 0 = `qkv` is the bf16 output [batch, qkv_tok_stride] of the qkv projection

@@ -583,6 +583,15 @@ extern "C" int nvl_linear_decode(const void* x, const void* weight, void* out, i
                    : dispatch_kb<1, EPI_PARTIAL>(x, weight, out, m, n, k, p, s);
 }
 
+static bool open_plan(int64_t m, int n, int k, Plan* p) {
+  return m >= 1 && m <= 16 && k % 128 == 0 && make_plan(m, n, k, EPI_PARTIAL, p) && p->mt == 1 && p->nt == 1;
+}
+
+extern "C" int nvl_linear_decode_open_splits(int64_t m, int n, int k) {
+  Plan p;
+  return open_plan(m, n, k, &p) ? p.split : 0;
+}
+
 extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight,
                                       void* out, int64_t m, int n, int k, int weight_layout, void* stream) {
   NVL_REQUIRE(parts_o && parts_ml && whole && context_lens && weight && out, "nvl_linear_decode_open: null pointer");
@@ -590,7 +599,7 @@ extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_m
   NVL_REQUIRE(weight_layout == 0 || weight_layout == 1, "nvl_linear_decode_open: weight_layout=%d", weight_layout);
   NVL_REQUIRE(((uintptr_t)parts_o | (uintptr_t)whole | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 && (uintptr_t)parts_ml % 8 == 0, "nvl_linear_decode_open: alignment");
   Plan p;
-  if (!make_plan(m, n, k, EPI_PARTIAL, &p) || p.mt != 1 || p.nt != 1) {
+  if (!open_plan(m, n, k, &p)) {
     nvl_set_error("nvl_linear_decode_open: shape m=%lld n=%d k=%d not covered", (long long)m, n, k);
     return NVL_EUNSUPPORTED;
   }

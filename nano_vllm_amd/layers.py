@@ -158,7 +158,7 @@ class Attention(nn.Module):
             return None
         b, (n, k) = qkv.shape[0], o_proj.weight.shape
         max_context = ctx.max_context or ctx.block_tables.shape[1] * self.k_cache.shape[2]
-        if not ops.linear_decode_splits(b, n, k, ops.LINEAR_PARTIAL) or not ops.open_parts(b, self.num_kv_heads, max_context):
+        if not ops.linear_decode_open_splits(b, n, k) or not ops.open_parts(b, self.num_kv_heads, max_context):
             return None
         ws = ctx.decode_workspace
         if ws is None:

@@ -52,6 +52,7 @@ SIGNATURES = {
     "nvl_paged_attn_decode_open_parts": (c_int, [c_int64, c_int, c_int64]),
     "nvl_paged_attn_decode_open": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                            c_int64, c_int, c_int, c_int, c_int64, c_int64, c_float, c_void_p, c_size_t, c_int, c_int64, c_void_p]),
+    "nvl_linear_decode_open_splits": (c_int, [c_int64, c_int, c_int]),
     "nvl_linear_decode_open": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "nvl_paged_attn_decode_fused": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p,
                                             c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int,
@@ -467,6 +468,7 @@ class OpenAttention:
 
 
 _open_cache: dict[tuple, int] = {}
+_open_splits_cache: dict[tuple, int] = {}
 
 
 def open_parts(b: int, num_kv_heads: int, max_context: int) -> int:
@@ -496,11 +498,20 @@ def paged_attn_decode_open(qkv: torch.Tensor, q_norm_w, k_norm_w, eps: float, co
     return OpenAttention(workspace, context_lens, b, num_q_heads, parts)
 
 
+def linear_decode_open_splits(m: int, n: int, k: int) -> int:
+    """K-slices linear_decode_open emits for this shape; 0 = it does not take it."""
+    key = (m, n, k)
+    r = _open_splits_cache.get(key)
+    if r is None:
+        r = _open_splits_cache[key] = lib().nvl_linear_decode_open_splits(m, n, k)
+    return r
+
+
 def linear_decode_open(att: OpenAttention, weight: torch.Tensor, packed: bool = False) -> torch.Tensor:
     """fp32 split-K partials [S, rows, N] of (the merged attention) . weight^T, as linear_decode(..., LINEAR_PARTIAL) of it."""
     n, k = weight.shape
     assert k == att.heads * 128 and weight.is_contiguous() and weight.dtype == torch.bfloat16
-    out = torch.empty((linear_decode_splits(att.rows, n, k, LINEAR_PARTIAL), att.rows, n), dtype=torch.float32, device=weight.device)
+    out = torch.empty((linear_decode_open_splits(att.rows, n, k), att.rows, n), dtype=torch.float32, device=weight.device)
     o = att.workspace.data_ptr()
     ml = o + att.rows * att.heads * att.parts * 512
     _check(lib().nvl_linear_decode_open(o, ml, ml + att.rows * att.heads * att.parts * 8, att.context_lens.data_ptr(), att.parts, weight.data_ptr(),

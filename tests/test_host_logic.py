@@ -304,3 +304,31 @@ def test_lookahead_order_reproduces_serial_schedule():
     assert serial == ahead and toks_a == toks_b
     assert all(t != -1 for toks in toks_b for t in toks)
     assert pre_a > 3                                   # the pool is small enough to force preemption + re-prefill
+
+
+OPEN_ASK = """
+import types, torch
+from nano_vllm_amd import layers, ops
+from nano_vllm_amd.attn_meta import set_context
+assert ops.linear_decode_splits(1, 1024, 2048, ops.LINEAR_PARTIAL) > 0            # the plain projection takes it
+att = layers.Attention(16, 128, 0.1, 8)
+att.k_cache = att.v_cache = torch.zeros(1, 8, 256, 128, dtype=torch.bfloat16)
+set_context(False, context_lens=torch.ones(1, dtype=torch.int32), block_tables=torch.zeros(1, 16, dtype=torch.int32), max_context=4096)
+proj = types.SimpleNamespace(tp_size=1, bias=None, weight=torch.zeros(1024, 2048, dtype=torch.bfloat16), weight_packed=None)
+print(ops.linear_decode_open_splits(1, 1024, 2048), att.forward_open(torch.zeros(1, 4096, dtype=torch.bfloat16), None, None, 1e-6, torch.zeros(1, 128), proj))
+"""
+
+
+def test_open_attention_asks_the_projection_before_it_runs():
+    """A projection that plans two column tiles a workgroup does not merge open parts: the step takes the merged way, and the attention has not run."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", OPEN_ASK], cwd=root, env=dict(os.environ, NVL_SKINNY_PLAN="2,1,0"), capture_output=True, text=True)
+    assert run.returncode == 0 and run.stdout.split() == ["0", "None"], run.stdout + run.stderr
+    from nano_vllm_amd import ops
+    for m, n, k in ((1, 1024, 2048), (4, 2048, 2048), (16, 1024, 3072), (2, 64, 1024)):
+        assert ops.linear_decode_open_splits(m, n, k) == ops.linear_decode_splits(m, n, k, ops.LINEAR_PARTIAL) > 0
+    for m, n, k in ((17, 1024, 2048), (1, 1024, 3072 + 128), (1, 1024, 4096), (1, 1000, 2048), (0, 1024, 2048)):
+        assert ops.linear_decode_open_splits(m, n, k) == 0
