@@ -53,3 +53,37 @@ def test_contexts_around_tiles_turns_and_parts(hq, hkv, lens, max_ctx):
         assert float((lse[i].double() - torch.logsumexp(s, 2).flatten()).abs().max()) <= 1e-4        # 32-bit sums of exact products
         # weights and result are rounded to 8 bits each
         assert float((got[i].double() - want).norm() / want.norm()) <= 2.0 ** -8, n
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 2), (5, 1), (24, 8)])
+@pytest.mark.parametrize("b,hi,max_ctx", [(12, 500, 1536), (12, 500, 4096), (16, 40, 1024), (8, 1500, 2048), (40, 300, 512)])
+def test_pages_that_hold_no_numbers_behind_a_context(b, hi, max_ctx, hq, hkv):
+    """Steps of this kernel and of the one of equal shares: what lies behind a context's end is not read into its result."""
+    from nano_vllm_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(b + hq)
+    bs, G, scale = 256, hq // hkv, 128 ** -0.5
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    lens = [1 + (hi - 1) * i // (b - 1) for i in range(b)]
+    need = [-(-n // bs) for n in lens]
+    bt, at = torch.full((b, max_ctx // bs), -1, dtype=torch.int32), 0
+    for i, k in enumerate(need):
+        bt[i, :k] = torch.arange(at, at + k)
+        at += k
+    kc, vc = rand(at, hkv, bs, 128), rand(at, hkv, bs, 128)
+    for i, n in enumerate(lens):
+        kc[bt[i, need[i] - 1], :, (n - 1) % bs:] = float("nan")
+        vc[bt[i, need[i] - 1], :, (n - 1) % bs:] = float("inf")
+    qkv, ctx = rand(b, (hq + 2 * hkv) * 128), torch.tensor(lens, dtype=torch.int32).cuda()
+    table = torch.cat([torch.ones(max_ctx, 64), torch.zeros(max_ctx, 64)], 1).cuda()
+    ws = torch.full((ops.paged_attn_decode_workspace_bytes(b, hq, max_ctx),), 255, dtype=torch.uint8, device="cuda")
+    plan = ops.decode_plan(ctx, hq, hkv, max_ctx)
+    for p in (plan, None):
+        k, v = kc.clone(), vc.clone()
+        got = ops.paged_attn_decode_fused(qkv, None, None, 1e-6, table, k, v, bt.cuda(), ctx, hq, scale, max_ctx, ws, plan=p)
+        for i, n in enumerate(lens):
+            rows = torch.arange(n)
+            pages, offs = bt[i, rows // bs].long().cuda(), (rows % bs).cuda()
+            K, V = k[pages, :, offs].double(), v[pages, :, offs].double()
+            s = (qkv[i, :hq * 128].double().view(hkv, G, 1, 128) * K.permute(1, 0, 2).unsqueeze(1)).sum(3) * scale
+            want = torch.matmul(torch.softmax(s, 2), V.permute(1, 0, 2)).view(hq, 128)
+            assert float((got[i].double() - want).norm() / want.norm()) <= 2.0 ** -8, (i, n)          # weights and result are rounded to 8 bits each
