@@ -246,8 +246,7 @@ int nvl_paged_attn_decode(const void* q, const void* k_cache, const void* v_cach
  * step (the reference calls flash_attn_with_kvcache once per layer,
  * layers/attention.py:72-74, and each call re-derives its own split
  * schedule). Enqueue-only, graph-capturable; `plan` is caller-owned,
- * nvl_decode_plan_bytes() bytes, 16-byte aligned. (Attention launches also count the parts of long contexts in it, from 0 to 0: launches that
- * use one plan follow one another.)
+ * nvl_decode_plan_bytes() bytes, 16-byte aligned.
  * shared_prefix (optional, may be NULL; ABI v5): DEVICE pointer to int32[1 + batch]. [0] = the number of leading KV
  *   blocks that the MEMBER sequences of the step have in common (identical block_tables[b][0 .. n) for every member
  *   b), [1 + b] != 0 marks sequence b as a member — what the reference's prefix cache produces when requests start

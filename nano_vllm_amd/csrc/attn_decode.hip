@@ -123,7 +123,7 @@ struct __attribute__((aligned(16))) PlanEntry { int32_t b, h, t0, nb; };   // fi
 __global__ __launch_bounds__(256) void decode_plan_kernel(const int32_t* __restrict__ ctx, int batch, int hkv, int nwaves,
                                                           PlanHeader* __restrict__ hdr,
                                                           const int32_t* __restrict__ shared_blocks, int tiles_per_block,
-                                                          int px_groups, int* __restrict__ arrived) {
+                                                          int px_groups) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   int* wsum = reinterpret_cast<int*>(smem_raw);
   int* pre = wsum + kWaves;
@@ -131,8 +131,6 @@ __global__ __launch_bounds__(256) void decode_plan_kernel(const int32_t* __restr
   // common. Whatever it says, the tile that takes a member's NEW token stays in that sequence's own share (the stream-K
   // kernel stores the token and starts its softmax there): sh <= min over live members of floor((len - 1) / 32).
   int sh = 0;
-  if (arrived != nullptr)                                 // (decode_few_kernel's counters)
-    for (int i = threadIdx.x; i < batch * hkv; i += 256) arrived[i] = 0;
   const int32_t* member = shared_blocks != nullptr ? shared_blocks + 1 : nullptr;
   if (shared_blocks != nullptr) {
     int* smin = pre + batch + 1;                        // (one more int of the dynamic region: the launcher sizes it)
@@ -1578,8 +1576,7 @@ __global__ __launch_bounds__(128) void decode_stream_combine_kernel(const float*
 // whatever its size, so with one sequence of 700 tokens every pair (sequence, kv head) is spread over six wavefronts of different
 // workgroups: split partials through memory, and a merge launch behind (11.5 + 4.3 us). Here a workgroup of eight wavefronts takes a pair, or
 // 1,024 tokens and more of it where the context is longer ("parts"), its wavefronts take every eighth tile of 32 tokens, and the split is merged in LDS: one
-// launch, and nothing but a long context's parts goes through memory. Those are merged by the part that arrives last (a counter in the
-// step's plan, set to 0 by nvl_decode_plan and again by the last one); without a plan by a launch of their own, in the same order and arithmetic.
+// launch, and nothing but a long context's parts goes through memory. Those are merged by a launch of their own.
 //
 // Tiles go memory -> LDS directly, into a place per wavefront that is requested again as soon as its operands are in registers. Same matrix
 // operands as mfma8_body; K slots are swizzled by row & 15, V slots by 2 (row & 7) (the direct path cannot write padding): both kinds of operand reads touch all
@@ -1613,10 +1610,6 @@ inline int open_parts(int64_t batch, int hkv, int64_t max_context) {
   return (int)parts;
 }
 
-// partials go through to memory and are read from there (another workgroup's L2 may be another one)
-__device__ __forceinline__ void few_put(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ float few_get(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
 // output row (b, head) from its n partials, dim d (and its log-sum-exp); eight partials requested at once
 __device__ __forceinline__ void few_merge(const float* part_o, const float* part_ml, int64_t row, int n, int slots, int d, bf16_t* out, float* lse) {
   const float* ml = part_ml + row * slots * 2;
@@ -1627,7 +1620,7 @@ __device__ __forceinline__ void few_merge(const float* part_o, const float* part
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int k = k0 + j < n ? k0 + j : n - 1;
-      m[j] = few_get(ml + k * 2), l[j] = few_get(ml + k * 2 + 1), o[j] = few_get(po + (int64_t)k * 128);
+      m[j] = ml[k * 2], l[j] = ml[k * 2 + 1], o[j] = po[(int64_t)k * 128];
     }
     float top = M;
 #pragma unroll
@@ -1650,10 +1643,9 @@ template <bool SLABS>
 __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc, const int32_t* __restrict__ block_tables, int64_t bt_stride,
     const int32_t* __restrict__ ctx, float* part_o, float* part_ml, bf16_t* __restrict__ out, int batch, int hkv, int block_size, int slots,
-    float scale_log2e, FusedArgs fa, int* arrived, int Gv, int parts, int part_tiles, bool open, float* __restrict__ lse) {
+    float scale_log2e, FusedArgs fa, int Gv, int parts, int part_tiles, float* __restrict__ lse) {
   typedef __attribute__((address_space(3))) void lds_void_t;
   typedef const __attribute__((address_space(1))) void global_void_t;
-  // open: a context of several parts leaves them as they are, for the output projection
   extern __shared__ __attribute__((aligned(128))) unsigned char smem_raw[];           // tiles; q rows [16][256], new k, new v; (m, l) [wave][16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, rq = lane >> 4, head = lane & 15, quad = lane >> 4;
@@ -1858,35 +1850,17 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     for (int w = 0; w < kFewWaves; ++w) num += f[w] * *reinterpret_cast<const f32x4_t*>(smem_raw + w * kFewTile + (wave * 64 + lane) * 16);
     const int64_t row = (int64_t)b * hq + h * Gv + head;
     const int d = 16 * wave + 4 * quad;
-    if (open && n > 1) {
+    if (n > 1) {                                   // left as it is, for the merge launch or the output projection
       *reinterpret_cast<f32x4_t*>(part_o + (row * slots + part) * 128 + d) = num;
       if (d == 0) *reinterpret_cast<float2*>(part_ml + (row * slots + part) * 2) = make_float2(M, den);
-    } else if (n == 1) {
+    } else {
       *reinterpret_cast<u32x2_t*>(out + row * 128 + d) = u32x2_t{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
       if (lse != nullptr && d == 0) lse[row] = 0.6931471805599453f * (M + log2f(den));
-    } else {
-      // (through to memory: a fence instead, which writes a whole L2 back, took 3 us and, from many workgroups at once, up to 200)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) few_put(part_o + (row * slots + part) * 128 + d + r, num[r]);
-      if (d == 0) {
-        few_put(part_ml + (row * slots + part) * 2, M);
-        few_put(part_ml + (row * slots + part) * 2 + 1, den);
-      }
     }
   }
-  if (open || n == 1 || arrived == nullptr) return;
-  int* last = reinterpret_cast<int*>(stage);
-  __builtin_amdgcn_s_waitcnt(0);                   // the partials are in memory
-  __syncthreads();
-  if (threadIdx.x == 0) *last = __hip_atomic_fetch_add(arrived + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __syncthreads();
-  if (*last != n - 1) return;
-  for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves)
-    few_merge(part_o, part_ml, (int64_t)b * hq + h * Gv + (i >> 7), n, slots, i & 127, out, lse);
-  if (threadIdx.x == 0) arrived[pair] = 0;
 }
 
-// without a plan: the contexts of several parts
+// the contexts of several parts
 __global__ __launch_bounds__(128) void decode_few_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                 const int32_t* __restrict__ ctx, bf16_t* __restrict__ out, int hq, int slots, int parts,
                                                                 float* __restrict__ lse) {
@@ -2035,14 +2009,9 @@ int launch_decode_mfma8_s(const void* q, void* kc, void* vc, const int32_t* bt, 
   return nvl_check_launch("nvl_paged_attn_decode");
 }
 
-// per-wave records of the largest grid the matrix-core kernel launches (2 workgroups per CU) behind the header; behind them the arrival
-// counters of decode_few_kernel
-inline size_t plan_records_bytes() { return sizeof(PlanHeader) + (size_t)nvl_device_cu_count() * 2 * kWaves * sizeof(PlanEntry); }
-
 template <bool SLABS>
 int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, int64_t bt_stride, const int32_t* ctx, void* out, int64_t batch,
-                      int hkv, int G, int block_size, int64_t max_context, float scale, void* workspace, hipStream_t s, const FusedArgs& fa, void* plan,
-                      float* lse, int parts) {
+                      int hkv, int G, int block_size, int64_t max_context, float scale, void* workspace, hipStream_t s, const FusedArgs& fa, float* lse, int parts) {
   constexpr int lds = kFewWaves * (kFewTile + 16 * 8) + 18 * 256;
   const bool open = out == nullptr;
   const int hq = hkv * G, slots = open ? parts : stream_slots(max_context);
@@ -2058,11 +2027,10 @@ int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, in
     }
     attr_set = true;
   }
-  int* arrived = plan != nullptr ? (int*)((unsigned char*)plan + plan_records_bytes()) : nullptr;
   hipLaunchKernelGGL((decode_few_kernel<SLABS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
                      (bf16_t*)vc, bt, bt_stride, ctx, part_o, part_ml, (bf16_t*)out, (int)batch, hkv, block_size, slots, scale * 1.4426950408889634f, fa,
-                     arrived, G, parts, open ? kOpenPart : kFewPart, open, lse);
-  if (!open && plan == nullptr && parts > 1)
+                     G, parts, open ? kOpenPart : kFewPart, lse);
+  if (!open && parts > 1)
     hipLaunchKernelGGL(decode_few_merge_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
   return nvl_check_launch("nvl_paged_attn_decode");
 }
@@ -2245,9 +2213,9 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
   const int few = open ? open_parts(batch, num_kv_heads, max_context) : fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
   if (few)
     return fa->qkv_splits > 0 ? launch_decode_few<true>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
-                                                        max_context, softmax_scale, workspace, s, *fa, const_cast<void*>(plan), lse, few)
+                                                        max_context, softmax_scale, workspace, s, *fa, lse, few)
                               : launch_decode_few<false>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
-                                                         max_context, softmax_scale, workspace, s, *fa, const_cast<void*>(plan), lse, few);
+                                                         max_context, softmax_scale, workspace, s, *fa, lse, few);
   if (kv_dtype == NVL_KV_FP8) {
 #define NVL_DECODE8_CASE(GG)                                                                                           \
   case GG:                                                                                                             \
@@ -2415,7 +2383,8 @@ extern "C" int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_strid
 
 // ---- per-step plan ------------------------------------------------------------------------------------------------
 extern "C" size_t nvl_decode_plan_bytes(void) {
-  return plan_records_bytes() + kFewGroups * sizeof(int);
+  // header + one record per wave of the largest grid the matrix-core kernel launches (2 workgroups per CU)
+  return sizeof(PlanHeader) + (size_t)nvl_device_cu_count() * 2 * kWaves * sizeof(PlanEntry);
 }
 
 extern "C" int nvl_decode_plan(const int32_t* context_lens, int64_t batch, int num_q_heads, int num_kv_heads,
@@ -2456,8 +2425,7 @@ extern "C" int nvl_decode_plan(const int32_t* context_lens, int64_t batch, int n
   }
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(256), lds, (hipStream_t)stream, context_lens, (int)batch,
                      num_kv_heads, nwaves, (PlanHeader*)plan, shared_prefix_blocks,
-                     shared_prefix_blocks ? block_size / kTile : 0, shared_prefix_blocks ? shared_prefix_groups : 0,
-                     few_parts(batch, num_kv_heads, max_context) > 1 ? (int*)((unsigned char*)plan + plan_records_bytes()) : nullptr);
+                     shared_prefix_blocks ? block_size / kTile : 0, shared_prefix_blocks ? shared_prefix_groups : 0);
   const int rc = nvl_check_launch(who);
   if (rc == NVL_OK) plan_shadow_put(plan, batch, num_kv_heads, max_context, shared_prefix_blocks != nullptr ? shared_prefix_groups : 0);   // (a failed launch leaves no record)
   return rc;

@@ -77,6 +77,7 @@ def test_pages_that_hold_no_numbers_behind_a_context(b, hi, max_ctx, hq, hkv):
     table = torch.cat([torch.ones(max_ctx, 64), torch.zeros(max_ctx, 64)], 1).cuda()
     ws = torch.full((ops.paged_attn_decode_workspace_bytes(b, hq, max_ctx),), 255, dtype=torch.uint8, device="cuda")
     plan = ops.decode_plan(ctx, hq, hkv, max_ctx)
+    before = plan.clone()
     for p in (plan, None):
         k, v = kc.clone(), vc.clone()
         got = ops.paged_attn_decode_fused(qkv, None, None, 1e-6, table, k, v, bt.cuda(), ctx, hq, scale, max_ctx, ws, plan=p)
@@ -87,3 +88,4 @@ def test_pages_that_hold_no_numbers_behind_a_context(b, hi, max_ctx, hq, hkv):
             s = (qkv[i, :hq * 128].double().view(hkv, G, 1, 128) * K.permute(1, 0, 2).unsqueeze(1)).sum(3) * scale
             want = torch.matmul(torch.softmax(s, 2), V.permute(1, 0, 2)).view(hq, 128)
             assert float((got[i].double() - want).norm() / want.norm()) <= 2.0 ** -8, (i, n)          # weights and result are rounded to 8 bits each
+    assert torch.equal(plan, before)                                # launches of several streams may share a plan: none writes it

@@ -332,3 +332,12 @@ def test_open_attention_asks_the_projection_before_it_runs():
         assert ops.linear_decode_open_splits(m, n, k) == ops.linear_decode_splits(m, n, k, ops.LINEAR_PARTIAL) > 0
     for m, n, k in ((17, 1024, 2048), (1, 1024, 3072 + 128), (1, 1024, 4096), (1, 1000, 2048), (0, 1024, 2048)):
         assert ops.linear_decode_open_splits(m, n, k) == 0
+
+
+def test_attention_launches_take_a_plan_as_it_is():
+    """Launches on several streams may share a plan: the entry points take it as a pointer to const, and nothing casts that away."""
+    import os
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    source = open(os.path.join(root, "nano_vllm_amd", "csrc", "attn_decode.hip")).read()
+    assert "const_cast" not in source and "hipMemset" not in source
+    assert source.count("void* plan") == source.count("const void* plan") + 1            # nvl_decode_plan alone writes it
