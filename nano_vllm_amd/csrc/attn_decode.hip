@@ -1574,40 +1574,37 @@ __global__ __launch_bounds__(128) void decode_stream_combine_kernel(const float*
 // ---------------------------------------------------------------------------------------------------
 // Steps of few sequences (fused form, bf16 cache, group sizes 2 ... 16). The stream-K launch above cuts the step into equal shares
 // whatever its size, so with one sequence of 700 tokens every pair (sequence, kv head) is spread over six wavefronts of different
-// workgroups: split partials through memory, and a merge launch behind (11.5 + 4.3 us). Here a workgroup of eight wavefronts takes a pair, or
-// 1,024 tokens and more of it where the context is longer ("parts"), its wavefronts take every eighth tile of 32 tokens, and the split is merged in LDS: one
-// launch, and nothing but a long context's parts goes through memory. Those are merged by a launch of their own.
+// workgroups: split partials through memory, and a merge launch behind. Here a workgroup of eight wavefronts takes a pair, or a part of it: 256 tokens, a tile of 32 for
+// each wavefront, and more where a context has more of them than workgroups run at once. The wavefronts' split is merged in LDS; nothing but the parts of a longer context
+// goes through memory, and those are merged by a launch of their own or by the output projection.
 //
 // Tiles go memory -> LDS directly, into a place per wavefront that is requested again as soon as its operands are in registers. Same matrix
 // operands as mfma8_body; K slots are swizzled by row & 15, V slots by 2 (row & 7) (the direct path cannot write padding): both kinds of operand reads touch all
 // banks once. What bounds it: one chain of latencies (context length -> rotation and tile -> scores -> merge), and 28 bytes a clock that a compute unit
 // takes in.
-constexpr int kFewWaves = 8, kFewTile = kTile * 512, kFewPart = 32, kFewGroups = 512;       // bytes of a wave's K and V tile; tiles of a part; workgroups of a launch
+constexpr int kFewWaves = 8, kFewTile = kTile * 512;                                        // bytes of a wave's K and V tile
+constexpr int kFewPart = NVL_OPEN_PART_TILES, kFewPairs = 64, kFewGroups = 256;             // tiles of a part; pairs and workgroups of a launch
 
-// Parts of a context of max_context tokens, while the workgroups (most of which leave at once when contexts are shorter) are few; 0: the stream-K kernel
-// takes the step, whose tile loads run ahead and fill the chip at 5.4 to 6.1 TB/s. us, stream-K with its merge / here, 16 heads over 8 kv heads, max_context 4,096: one
-// sequence of 100 tokens 11.5 / 6.2, 700 11.9 / 9.7, 2,000 14.1 / 12.7, 4,096 14.8 / 13.5; 4 and 16 sequences of 100 to 2,047 13.9 / 11.5, 22.6 / 18.1, 16 of 3,000 to
-// 4,096 42.9 / 40.3; max_context 32,768, two of 20,000 to 32,000 58 / 45; 64 sequences, one kv head, 6,000 to 8,000 of 8,192 50 / 42. Beyond 512 workgroups: 24 sequences
-// of 4,096 47.1 / 47.7, 64 of 3,000 to 4,096 153 / 179, 128 of 2,047 103 / 125. More than 16 sequences stay there too, with one kv head 64 of 3,000 to 4,000
-// 31 / 24: a step with a plan for a shared prefix that turns out to have none gives the bits of a step without.
+// Parts of a context of up to max_context tokens (most of whose workgroups leave at once when contexts are shorter); 0: the stream-K kernel takes the step, whose tile
+// loads run ahead. Decode steps of Qwen3-0.6B (16 heads over 8 kv heads, max_context 4,096) in us, stream-K / here, contexts of 150, 300, 600, 1,000, 1,500, 2,000, 3,000 and
+// 4,000 tokens: five sequences 1056 1050 1048 1090 1096 1134 1218 1388 / 893 953 1001 1028 1085 1099 1160 1264, eight 1073 1081 1074 1104 1156 1220 1412 1521 / 902 1005 1059 1104
+// 1161 1203 1357 1502. Twelve and 16 gain up to 1,500 (12: 1098 1092 1120 1162 1327 / 925 1064 1106 1171 1272; 16: 1101 1115 1130 1229 1379 / 904 1015 1101 1220 1368) and lose from
+// 2,000 on (16: 1464 1731 2001 / 1519 1847 2153), so they come here where contexts stay short. Not more workgroups than run at once (of 16 sequences 192: one part each and not two,
+// 949 1101 1155 1223 1369): parts of 1,024 tokens, as many as there are, took 1,161 us for eight of 1,000 and 1,794 for 12 of 3,000.
 inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
-  const int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart;
-  return batch <= 16 && batch * hkv * parts <= kFewGroups ? (int)parts : 0;
+  const int64_t pairs = batch * hkv;
+  if (batch < 1 || batch > 16 || pairs > (max_context <= 1536 ? 2 * kFewPairs : kFewPairs)) return 0;
+  const int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart, most = (pairs > kFewPairs ? kFewGroups * 3 / 4 : kFewGroups) / pairs;
+  return (int)(parts < most ? parts : most);
 }
 
-// Left open for the output projection to merge (nvl_linear_decode_open), a part costs neither a trip through memory nor a wait for the others, so it
-// is a tile of each wavefront. us, attention and output projection (16 heads over 8 kv heads, 1,024 columns), merged here / open: one sequence of 100 tokens 8.7 / 8.6,
-// 256 9.7 / 9.7, 700 12.9 / 10.6, 2,000 16.2 / 12.0, 4,000 16.3 / 14.2, 12,000 22.3 / 21.1; four of 100 9.3 / 9.1, 700 13.4 / 11.0, 2,000 17.3 / 15.2. Up to eight parts, since
-// the projection takes longer with more (4,000 tokens in 16: 7.4 + 6.6 us, in eight 8.6 + 5.2), 16 where contexts may pass 4,096 tokens (12,000 in eight: 25.2). Eight of 2,000
-// 25.9 / 26.5 (the projection reads every part in each of its workgroups), one of 30,000 33.5 / 36.5: those are merged here.
-constexpr int kOpenPart = NVL_OPEN_PART_TILES, kOpenParts = 16, kOpenRows = 4;
+// Left open for the output projection to merge (nvl_linear_decode_open): up to eight parts, since the projection takes longer with more (4,000 tokens in 16: 7.4 + 6.6 us, in
+// eight 8.6 + 5.2), 16 where contexts may pass 4,096 tokens (12,000 in eight: 25.2).
+constexpr int kOpenParts = 16, kOpenRows = 4;
 inline int open_parts(int64_t batch, int hkv, int64_t max_context) {
-  if (batch < 1 || batch > kOpenRows || batch * hkv > kFewGroups || max_context > 16384) return 0;
-  int64_t parts = ((max_context + kTile - 1) / kTile + kOpenPart - 1) / kOpenPart;
-  const int most = max_context <= 4096 ? kOpenParts / 2 : kOpenParts;
-  if (parts > most) parts = most;
-  if (parts > kFewGroups / (batch * hkv)) parts = kFewGroups / (batch * hkv);
-  return (int)parts;
+  if (batch > kOpenRows || max_context > 16384) return 0;
+  const int parts = few_parts(batch, hkv, max_context), most = max_context <= 4096 ? kOpenParts / 2 : kOpenParts;
+  return parts < most ? parts : most;
 }
 
 // output row (b, head) from its n partials, dim d (and its log-sum-exp); eight partials requested at once
@@ -1643,14 +1640,14 @@ template <bool SLABS>
 __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc, const int32_t* __restrict__ block_tables, int64_t bt_stride,
     const int32_t* __restrict__ ctx, float* part_o, float* part_ml, bf16_t* __restrict__ out, int batch, int hkv, int block_size, int slots,
-    float scale_log2e, FusedArgs fa, int Gv, int parts, int part_tiles, float* __restrict__ lse) {
+    float scale_log2e, FusedArgs fa, int Gv, int parts, float* __restrict__ lse) {
   typedef __attribute__((address_space(3))) void lds_void_t;
   typedef const __attribute__((address_space(1))) void global_void_t;
   extern __shared__ __attribute__((aligned(128))) unsigned char smem_raw[];           // tiles; q rows [16][256], new k, new v; (m, l) [wave][16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, rq = lane >> 4, head = lane & 15, quad = lane >> 4;
   const int pairs = batch * hkv, part = blockIdx.x / pairs, pair = blockIdx.x % pairs, b = pair / hkv, h = pair % hkv, hq = hkv * Gv;
-  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = nvl_few_split(tiles, part_tiles, parts), per = (tiles + n - 1) / n;
+  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts), per = nvl_few_div(tiles, n);
   if (part >= n) return;
   if (len <= 0) {                                  // graph padding: zero rows
     for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves) out[((int64_t)b * hq + h * Gv) * 128 + i] = (bf16_t)0.f;
@@ -2029,7 +2026,7 @@ int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, in
   }
   hipLaunchKernelGGL((decode_few_kernel<SLABS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
                      (bf16_t*)vc, bt, bt_stride, ctx, part_o, part_ml, (bf16_t*)out, (int)batch, hkv, block_size, slots, scale * 1.4426950408889634f, fa,
-                     G, parts, open ? kOpenPart : kFewPart, lse);
+                     G, parts, lse);
   if (!open && parts > 1)
     hipLaunchKernelGGL(decode_few_merge_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
   return nvl_check_launch("nvl_paged_attn_decode");
@@ -2368,7 +2365,7 @@ extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stri
                       lse, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_fused", false);
 }
 extern "C" int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context) {
-  static_assert(kTile == 32 && kOpenPart == kFewWaves, "the projection counts the parts too");
+  static_assert(kTile == 32 && kFewPart == kFewWaves, "the projection counts the parts too");
   return num_kv_heads > 0 && max_context > 0 ? open_parts(batch, num_kv_heads, max_context) : 0;
 }
 extern "C" int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,

@@ -16,7 +16,7 @@ int main() {
   for (int part_tiles : {8, 32})
     for (int parts = 1; parts <= 64; ++parts)
       for (int tiles = 1; tiles <= 1100; ++tiles) {
-        const int n = nvl_few_split(tiles, part_tiles, parts), per = (tiles + n - 1) / n;
+        const int n = nvl_few_split(tiles, part_tiles, parts), per = nvl_few_div(tiles, n);
         int next = 0, owners = 0, empty = 0;
         for (int p = 0; p < n; ++p) {
           const int t0 = p * per, t1 = tiles < t0 + per ? tiles : t0 + per;
@@ -30,6 +30,9 @@ int main() {
           return 1;
         }
       }
+  for (int b = 1; b <= 256; ++b)
+    for (int a = 1; a < (1 << 20); a += a < 5000 ? 1 : 97)
+      if (nvl_few_div(a, b) != (a + b - 1) / b) return 3;
   return nvl_few_split(0, 8, 16) == 1 ? 0 : 2;
 }
 """

@@ -341,3 +341,14 @@ def test_attention_launches_take_a_plan_as_it_is():
     source = open(os.path.join(root, "nano_vllm_amd", "csrc", "attn_decode.hip")).read()
     assert "const_cast<void*>(plan)" not in source
     assert source.count("void* plan") == source.count("const void* plan") + 1            # nvl_decode_plan alone writes it
+
+
+def test_open_parts_run_at_once():
+    """One workgroup per part and (sequence, kv head) pair: no more of them than compute units."""
+    from nano_vllm_amd import ops
+    for b in (1, 2, 3, 4):
+        for hkv in (1, 2, 4, 8, 16):
+            for longest in (256, 1024, 4096, 4097, 8192, 16384):
+                parts = ops.open_parts(b, hkv, longest)
+                assert 1 <= parts <= (8 if longest <= 4096 else 16) and parts <= -(-longest // 256) and b * hkv * parts <= 256
+    assert [ops.open_parts(b, 8, 16384) for b in (1, 2, 3, 4, 5)] == [16, 16, 10, 8, 0] and ops.open_parts(1, 8, 16385) == 0
