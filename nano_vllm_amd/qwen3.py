@@ -16,7 +16,8 @@ shapes) the chain is 8 launches:
    -> split merge -> o GEMM (fp32 split-K slabs) -> add+RMSNorm(slabs) -> gate_up GEMM + SiLU*mul epilogue
    -> down GEMM (slabs)
 
-with the GEMMs on the hand-written skinny kernel (nvl_linear_decode). Up to 16 rows (TP=1, width <= 2048) it is 5:
+with the GEMMs on the hand-written skinny kernel (nvl_linear_decode). Up to 8 rows (TP=1, width <= 1024) it is 5 or 6 (up to 4 rows the o GEMM merges
+the parts of a context, beyond them a launch of its own):
 
    [add+RMSNorm + qkv GEMM] -> [norm + RoPE + KV store + attention, split merged in LDS] -> o GEMM
    -> [add+RMSNorm + gate_up GEMM + SiLU*mul] -> down GEMM
@@ -85,7 +86,7 @@ class Qwen3MLP(nn.Module):
         return self.down_proj.forward_decode(self.gate_up_proj.forward_silu(x))
 
     def forward_normed(self, norm: RMSNorm, x, residual):
-        """(self(norm(x, residual)), the new residual) of a decode step; up to 16 rows take norm, gate|up and activation in one launch."""
+        """(self(norm(x, residual)), the new residual) of a decode step; few rows take norm, gate|up and activation in one launch."""
         both = norm.into_linear(x, residual, self.gate_up_proj, silu=True)
         if both is not None:
             return self.down_proj.forward_decode(both[0]), both[1]

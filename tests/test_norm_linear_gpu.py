@@ -42,3 +42,12 @@ def test_what_is_not_covered_is_refused():
     x, w = torch.zeros(17, 64, device="cuda").bfloat16(), torch.zeros(64, 64, device="cuda").bfloat16()
     with pytest.raises(ops.NvlError, match="up to 16 rows"):
         ops.norm_linear(x, None, w[0], 1e-6, w)
+
+
+@pytest.mark.parametrize("rows,width,taken", [(1, 1024, True), (8, 1024, True), (9, 1024, False), (16, 1024, False), (1, 2048, False), (8, 512, True)])
+def test_layer_takes_it_where_it_pays(rows, width, taken):
+    from nano_vllm_amd.layers import QKVParallelLinear, RMSNorm
+    norm = RMSNorm(width).to(torch.bfloat16).cuda()
+    qkv = QKVParallelLinear(width, 128, 16, 8, bias=False).to(torch.bfloat16).cuda()
+    both = norm.into_linear(torch.ones(rows, width, device="cuda").bfloat16(), None, qkv)
+    assert (both is not None) == taken
