@@ -141,15 +141,22 @@ def _seq_digest() -> str:
     return h.hexdigest()
 
 
+def seq_is_fresh() -> bool:
+    """Is libnvl_seq.so there, built from these sources?"""
+    stamp = os.path.join(LIBDIR, "libnvl_seq.stamp")
+    if not (os.path.exists(LIB_SEQ) and os.path.exists(stamp)):
+        return False
+    with open(stamp) as fh:
+        return fh.read().strip() == _seq_digest()
+
+
 def build_seq(force: bool = False) -> str:
     """Compile csrc/seq/*.hip into libnvl_seq.so (a few seconds per file, in parallel); returns its path."""
     os.makedirs(LIBDIR, exist_ok=True)
     stamp = os.path.join(LIBDIR, "libnvl_seq.stamp")
     digest = _seq_digest()
-    if not force and os.path.exists(LIB_SEQ) and os.path.exists(stamp):
-        with open(stamp) as fh:
-            if fh.read().strip() == digest:
-                return LIB_SEQ
+    if not force and seq_is_fresh():
+        return LIB_SEQ
     hipcc = _hipcc()
     objdir = os.path.join(LIBDIR, "obj")
     os.makedirs(objdir, exist_ok=True)

@@ -507,13 +507,13 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
     def forward_silu(self, x: torch.Tensor) -> torch.Tensor:
         """SiluAndMul(self(x)) for a gate|up pair; on decode-sized inputs the activation is the GEMM's
         epilogue (one launch, no [N, 2*inter] round trip), on many rows that of the pipelined tiles where
-        those are the faster ones."""
+        those are the faster ones and their library is loaded."""
         pair = self.bias is None and len(self.output_sizes) == 2 and self.output_sizes[0] == self.output_sizes[1]
         if pair and _decode_sized(x):
             y = decode_linear(x, self.weight, ops.LINEAR_SILU, packed=self.weight_packed)
             if y is not None:
                 return y
-        if pair and ops_seq.silu_linear_fits(x, self.weight):
+        if pair and ops_seq.loaded() and ops_seq.silu_linear_fits(x, self.weight):
             tm = ops_seq.silu_linear_rows(x.shape[0], self.weight.shape[0] // 2, x.shape[1])
             if tm:
                 return ops_seq.silu_linear(x, self.weight, tm)

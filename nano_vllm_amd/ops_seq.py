@@ -104,6 +104,17 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+def load_if_built() -> bool:
+    """For a model that can do without this library (qwen3): is it loaded now? It is if it is there as its sources have it; nothing is built."""
+    if _lib is None and _build.seq_is_fresh():
+        load_library()
+    return _lib is not None
+
+
+def loaded() -> bool:
+    return _lib is not None
+
+
 def _check(rc: int) -> None:
     if rc != 0:
         raise NvsError(f"nvs error {rc}: {_lib.nvs_last_error().decode()}")

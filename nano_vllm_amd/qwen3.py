@@ -31,7 +31,7 @@ from .api import model_geometry
 from .attn_meta import get_context, plain_calls
 from .layers import (Attention, MergedColumnParallelLinear, ParallelLMHead, QKVParallelLinear, RMSNorm,
                      RowParallelLinear, SiluAndMul, VocabParallelEmbedding, get_rope)
-from . import tp
+from . import ops_seq, tp
 
 
 class Qwen3Attention(nn.Module):
@@ -153,6 +153,7 @@ class Qwen3ForCausalLM(nn.Module):
 
     def __init__(self, config):
         super().__init__()
+        ops_seq.load_if_built()                 # (prompt steps' gate|up: here, not inside the first of them)
         _, size = tp.world()
         self.geo = model_geometry(config, size)
         self.model = Qwen3Model(config, self.geo)

@@ -352,3 +352,33 @@ def test_open_parts_run_at_once():
                 parts = ops.open_parts(b, hkv, longest)
                 assert 1 <= parts <= (8 if longest <= 4096 else 16) and parts <= -(-longest // 256) and b * hkv * parts <= 256
     assert [ops.open_parts(b, 8, 16384) for b in (1, 2, 3, 4, 5)] == [16, 16, 10, 8, 0] and ops.open_parts(1, 8, 16385) == 0
+
+
+SEQ_ABSENT = """
+import torch
+from nano_vllm_amd import build, layers, ops, ops_seq
+def never(*a, **k):
+    raise AssertionError("built or launched")
+build.seq_is_fresh, build.build_seq = lambda: False, never                 # no library, or an older one
+assert not ops_seq.load_if_built() and not ops_seq.loaded()
+layer = layers.MergedColumnParallelLinear(64, [64, 64])
+ops_seq.silu_linear_fits, ops_seq.silu_linear_rows, ops_seq.silu_linear, ops.silu_mul = (lambda *a: True), (lambda *a: 256), never, (lambda y: y)
+layers._decode_sized = lambda x: False
+assert layer.forward_silu(torch.zeros(300, 64, dtype=layer.weight.dtype, device=layer.weight.device)).shape == (300, 128)
+build.seq_is_fresh, build.build_seq = lambda: True, lambda: build.LIB_SEQ
+assert ops_seq.load_if_built() and ops_seq.loaded()
+print("ok")
+"""
+
+
+def test_qwen3_does_without_the_second_library():
+    """libnvl_seq.so missing or stale: nothing is built when a prompt step comes along, the library's product and the activation kernel are taken; there: it is loaded
+    when the model is made."""
+    import os
+    import subprocess
+    import sys
+    from nano_vllm_amd import build
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    build.build_seq()
+    run = subprocess.run([sys.executable, "-c", SEQ_ABSENT], cwd=root, capture_output=True, text=True)
+    assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout + run.stderr
