@@ -685,6 +685,8 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, glu: bool) -> bool:
         return False
     m, k = x.shape
     n = w.shape[0]
+    if n == 0 or k == 0 or x.stride(0) < k or x.device != w.device:          # (rows that share entries too: nvs_linear_rows refuses them)
+        return False
     if w.dtype == torch.bfloat16:
         if k % 64 or x.stride(0) % 8 or not (m <= 16 or m <= 256 and n <= 4096 or m <= 128 and n <= 6144 or
                                              glu and (m <= 32 or m * n <= 64 * 12288 or m <= 256 and n <= 8192)):
@@ -727,7 +729,7 @@ def silu_linear_rows(n: int, ff: int, K: int) -> int:
 
 
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and x.stride(0) >= x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
@@ -747,6 +749,7 @@ def silu_linear(x: torch.Tensor, w: torch.Tensor, tm: int, out: torch.Tensor | N
 @_launch
 def linear_act(x: torch.Tensor, w: torch.Tensor, ff: int, kind: int = 0, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
     """glu_act of x times w^T, w [2 ff, K] = [gate | up] (kind 2: [ff, K])."""
+    assert w.shape[0] == (1 if kind == 2 else 2) * ff
     out = torch.empty(x.shape[0], ff, dtype=x.dtype, device=x.device)
     if _few_rows(x, w, True):
         return _linear_rows(x, w, None, kind, limit, alpha, out)
@@ -774,6 +777,15 @@ def moe_route(z: torch.Tensor, total: int, correction: torch.Tensor | None, top:
     return ids, wts
 
 
+def _router_fits(x: torch.Tensor, router: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    n, k = x.shape
+    if x.dtype not in (torch.bfloat16, torch.float32) or n == 0 or k == 0 or x.stride(0) < k or x.device != router.device:
+        return False
+    wide = x.dtype == torch.float32
+    return (router.shape[0] <= (48 if wide else 64) and k % (32 if wide else 64) == 0 and x.stride(1) == 1 and x.stride(0) * x.element_size() % 16 == 0
+            and x.data_ptr() % 16 == 0 and router.is_contiguous() and router.data_ptr() % 16 == 0 and (bias is None or bias.is_contiguous()))
+
+
 @_launch
 def moe_router(x: torch.Tensor, router: torch.Tensor, bias: torch.Tensor | None, total: int, correction: torch.Tensor | None, top: int, count: int,
                keep: int, scale: float, sigmoid: bool = False, renorm: bool = True):
@@ -785,8 +797,7 @@ def moe_router(x: torch.Tensor, router: torch.Tensor, bias: torch.Tensor | None,
     n, k = x.shape
     entries = router.shape[0]
     assert router.dtype == torch.float32 and router.shape[1] == k and total <= entries <= total + 1
-    if entries > (64 if x.dtype == torch.bfloat16 else 48) or k % (64 if x.dtype == torch.bfloat16 else 32) or x.stride(1) != 1 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16 \
-            or not router.is_contiguous() or router.data_ptr() % 16 or not (bias is None or bias.is_contiguous()) or n == 0:
+    if not _router_fits(x, router, bias):
         z = torch.nn.functional.linear(x.float(), router, bias)
         ids, wts = moe_route(z, total, correction, top, count, keep, scale, sigmoid, renorm)
         return ids, wts, z[:, total:] if entries > total else None

@@ -592,3 +592,61 @@ def test_expert_tile_heights_follow_the_workgroups_they_leave():
             (1000, 520, 16, 300, bf, 128), (96, 48, 8, 64, bf, 64)]:                                            # rows that are no whole pieces
         assert moe_tile_rows(per * experts, experts, width, ff, dtype) == want, (width, ff, experts, per, dtype)
     assert moe_tile_rows(3, 32, 1024, 768, bf) == 16
+
+
+class _Rows:
+    """What the rules of the few-row products look at, without a device: 16-bit by default, 128-byte pieces, aligned."""
+
+    def __init__(self, shape, stride=None, dtype=torch.bfloat16, device="cuda:0"):
+        self.shape, self.dtype, self.device = torch.Size(shape), dtype, torch.device(device)
+        self._stride, self.is_cuda = stride or (shape[1], 1), True
+
+    def dim(self):
+        return len(self.shape)
+
+    def stride(self, i):
+        return self._stride[i]
+
+    def is_contiguous(self):
+        return self._stride == (self.shape[1], 1)
+
+    def data_ptr(self):
+        return 1 << 20
+
+    def element_size(self):
+        return 4 if self.dtype == torch.float32 else 2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_few_row_products_leave_the_library_what_they_refuse(dtype):
+    """Rows that share entries (an expanded row, overlapping windows), no entries at all and tensors of two devices were the library's to take or to refuse."""
+    from nano_vllm_amd import ops_seq
+    w = _Rows((32, 256), dtype=dtype)
+    for glu in (False, True):
+        assert ops_seq._few_rows(_Rows((8, 256), dtype=dtype), w, glu) and ops_seq._few_rows(_Rows((8, 256), (320, 1), dtype), w, glu)
+        for stride in ((0, 1), (64, 1), (192, 1), (256, 2)):
+            assert not ops_seq._few_rows(_Rows((8, 256), stride, dtype), w, glu)
+        assert not ops_seq._few_rows(_Rows((8, 256), dtype=dtype, device="cuda:1"), w, glu)
+        assert not ops_seq._few_rows(_Rows((8, 256), dtype=dtype), _Rows((0, 256), dtype=dtype), glu)
+        assert not ops_seq._few_rows(_Rows((8, 0), dtype=dtype), _Rows((32, 0), dtype=dtype), glu)
+    router = _Rows((33, 256), dtype=torch.float32)
+    assert ops_seq._router_fits(_Rows((8, 256), dtype=dtype), router, None)
+    for x in (_Rows((8, 256), (0, 1), dtype), _Rows((8, 256), (64, 1), dtype), _Rows((0, 256), dtype=dtype), _Rows((8, 256), dtype=torch.float16),
+              _Rows((8, 256), dtype=dtype, device="cuda:1")):
+        assert not ops_seq._router_fits(x, router, None)
+
+
+def test_gated_products_want_both_halves(monkeypatch):
+    """The product of few rows reads [gate | up] at ff rows and 2 ff: another number of rows is refused before it is launched."""
+    from nano_vllm_amd import ops_seq
+
+    def launched(*a):
+        raise RuntimeError("launched")
+    monkeypatch.setattr(ops_seq, "_linear_rows", launched)
+    x = _Rows((4, 64), device="cpu")
+    for kind, rows in ((0, 31), (0, 64), (1, 16), (2, 32)):
+        with pytest.raises(AssertionError):
+            ops_seq.linear_act(x, _Rows((rows, 64), device="cpu"), 16, kind=kind)
+    for kind, rows in ((0, 32), (1, 32), (2, 16)):
+        with pytest.raises(RuntimeError, match="launched"):
+            ops_seq.linear_act(x, _Rows((rows, 64), device="cpu"), 16, kind=kind)
