@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.nn.modules import module as _hooks
 
 from .api import model_geometry
 from .attn_meta import get_context, plain_calls
@@ -94,6 +95,11 @@ class Qwen3MLP(nn.Module):
         return self(hidden_states), residual
 
 
+def _watched(*modules) -> bool:
+    """Does anybody look at these modules' calls? Then they are called, with their own inputs and outputs."""
+    return bool(_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or any(m._forward_hooks or m._forward_pre_hooks for m in modules))
+
+
 class Qwen3DecoderLayer(nn.Module):
 
     def __init__(self, config, geo: dict):
@@ -107,7 +113,7 @@ class Qwen3DecoderLayer(nn.Module):
     def forward(self, positions, hidden_states, residual):
         attn, qkv = self.self_attn, None
         decode = attn.qkv_proj.tp_size == 1 and not get_context().is_prefill
-        if decode:
+        if decode and not _watched(self.input_layernorm, attn):
             both = self.input_layernorm.into_linear(hidden_states, residual, attn.qkv_proj)
             if both is not None:
                 qkv, residual = both
@@ -117,8 +123,8 @@ class Qwen3DecoderLayer(nn.Module):
                 hidden_states = self.input_layernorm(hidden_states)
             else:
                 hidden_states, residual = self.input_layernorm(hidden_states, residual)
-        hidden_states = attn(positions, hidden_states, qkv)
-        if decode:
+        hidden_states = attn(positions, hidden_states) if qkv is None else attn(positions, hidden_states, qkv)
+        if decode and not _watched(self.post_attention_layernorm, self.mlp):
             return self.mlp.forward_normed(self.post_attention_layernorm, hidden_states, residual)
         hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
         return self.mlp(hidden_states), residual

@@ -11,6 +11,7 @@
 import gzip
 import json
 import os
+import types
 
 import pytest
 
@@ -382,3 +383,45 @@ def test_qwen3_does_without_the_second_library():
     build.build_seq()
     run = subprocess.run([sys.executable, "-c", SEQ_ABSENT], cwd=root, capture_output=True, text=True)
     assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout + run.stderr
+
+
+@pytest.mark.parametrize("where", ["input_layernorm", "self_attn", "post_attention_layernorm", "mlp", "everywhere", None])
+def test_modules_that_are_watched_are_called_on_decode_steps(where):
+    import torch
+    from nano_vllm_amd.attn_meta import reset_context
+    from nano_vllm_amd.qwen3 import Qwen3DecoderLayer
+
+    class Norm(torch.nn.Module):
+        def into_linear(self, x, residual, linear, silu=False):
+            return x + 100.0, x
+
+        def forward(self, x, residual=None):
+            return (x + 1.0, x) if residual is not None else x + 1.0
+
+    class Attn(torch.nn.Module):
+        qkv_proj = types.SimpleNamespace(tp_size=1)
+
+        def forward(self, positions, hidden, qkv=None):
+            return hidden if qkv is None else qkv
+
+    class MLP(torch.nn.Module):
+        def forward_normed(self, norm, x, residual):
+            return x, residual
+
+        def forward(self, x):
+            return x
+    layer = Qwen3DecoderLayer.__new__(Qwen3DecoderLayer)
+    torch.nn.Module.__init__(layer)
+    layer.input_layernorm, layer.post_attention_layernorm, layer.self_attn, layer.mlp = Norm(), Norm(), Attn(), MLP()
+    reset_context()
+    seen = []
+    note = lambda m, args, out: seen.append(type(m).__name__)
+    hook = None
+    if where == "everywhere":
+        hook = torch.nn.modules.module.register_module_forward_hook(note)
+    elif where:
+        hook = getattr(layer, where).register_forward_hook(note)
+    layer.forward(None, torch.zeros(1, 4), torch.zeros(1, 4))
+    if hook is not None:
+        hook.remove()
+    assert seen == {"everywhere": ["Norm", "Attn", "Norm", "MLP"], "self_attn": ["Attn"], "mlp": ["MLP"], None: []}.get(where, ["Norm"])
