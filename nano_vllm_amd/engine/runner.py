@@ -983,7 +983,7 @@ class ModelRunner:
         """A decode-only step of `bs` rows on the static staging block: model, logits, sampler (captured per bucket)."""
         from ..ops_seq import Portions
         t = self.sstage.t
-        por = Portions(t["cu_q"], t["ctx0"], t["sslot"], t["tseq"], bs, bs)
+        por = Portions(t["cu_q"], t["ctx0"], t["sslot"], t["tseq"], bs, bs, 1)       # (padding rows are portions of one token too)
         set_context(True, slot_mapping=t["slots"][:bs], block_tables=t["bt"][:bs], portions=por)
         x = self.model(t["ids"][:bs], t["pos"][:bs])
         logits = self.model.compute_logits(x, t["rows"], bs)

@@ -650,3 +650,27 @@ def test_gated_products_want_both_halves(monkeypatch):
     for kind, rows in ((0, 32), (1, 32), (2, 16)):
         with pytest.raises(RuntimeError, match="launched"):
             ops_seq.linear_act(x, _Rows((rows, 64), device="cpu"), 16, kind=kind)
+
+
+@pytest.mark.parametrize("bs", [1, 2, 16, 64])
+def test_captured_decode_steps_say_that_they_are_single_tokens(bs, monkeypatch):
+    """The scans choose their kernel by the longest portion: without it a step of 64 single tokens counts as one of 64 tokens."""
+    from nano_vllm_amd import ops_seq
+    from nano_vllm_amd.attn_meta import get_context
+    from nano_vllm_amd.engine.runner import ModelRunner
+    made, steps = [], []
+    monkeypatch.setattr(ops_seq, "Portions", lambda *a, **k: made.append((a[4:], k)) or "portions")
+
+    class Model:
+        def __call__(self, ids, pos):
+            steps.append(get_context().portions)
+            return ids
+
+        def compute_logits(self, x, rows, n):
+            return x
+    r = ModelRunner.__new__(ModelRunner)
+    names = ("cu_q", "ctx0", "sslot", "tseq", "slots", "bt", "ids", "pos", "rows", "temps", "rng", "rkey")
+    r.sstage = types.SimpleNamespace(t={name: torch.zeros(128, dtype=torch.int32) for name in names})
+    r.model, r.sampler, r.tokens_dev = Model(), lambda *a, **k: None, torch.zeros(128)
+    r._decode_body(bs)
+    assert made == [((bs, bs, 1), {})] and steps == ["portions"]
