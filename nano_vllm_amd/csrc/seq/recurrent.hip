@@ -940,7 +940,7 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   //   against 13) are the chunks' from the first token on.
   //   exponential gates with few pairs, where the gates of 64 tokens are computed for one: 8 pairs of 128 x 128 10 / 13 / 17 against 13 (32-bit 14), 128
   //   pairs 11 / 14 against 13, 256 pairs 16 / 19 against 16 (18), 512 pairs 30 against 25.
-  // The constant decay stays with the walk for portions under a chunk: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is
+  // The constant decay stays with the walk for portions of 2 to 15 tokens: 119 us for 100 tokens against 92, but outputs whose error against 64 bits is
   // 7.4e-8, not 8.3e-8.
   // Single tokens of the sizes that scan_token.hip is built for are its: it only moves the state. us here / there (the faster of the two), state-space duality, constant
   // decay, exponential gates: 512 pairs of 128 x 128 14.4 / 24, 16 / 24, 16 / 26; 8 pairs 8.5 / 11.8, 8.7 / 9.1, 8.6 / 10.8; 1,024 pairs of 64 x 128 12.0 / 24, 13.7 / 24, 13.4 / 28,

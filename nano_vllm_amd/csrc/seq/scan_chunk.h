@@ -22,6 +22,6 @@ void scan_chunk_plan(int heads, int P, int nseq, int64_t max_q, int* seg_len, in
 // whether sizes and addresses suit the chunk kernel
 bool scan_chunk_fits(const ScanArgs& a, int dtype);
 int scan_chunk_launch(const ScanArgs& a, int dtype, int nseq, void* stream);
-// the same for steps of a few tokens per portion (scan_token.hip)
+// the same for steps of single tokens (scan_token.hip)
 bool scan_token_fits(const ScanArgs& a, int dtype);
 int scan_token_launch(const ScanArgs& a, int dtype, int nseq, void* stream);

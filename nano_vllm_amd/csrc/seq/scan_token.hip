@@ -4,11 +4,10 @@
 // A workgroup of four wavefronts per (portion, head). A row of the state is N / 4 neighbouring lanes of four entries, so a wavefront reads and writes whole lines, and a lane
 // asks for all its rows' pieces (16 of a 128 x 128 state) before anything else; the token's operands come straight from where they are, nothing goes through LDS.
 // The sums over a row's lanes are taken for all rows at once: at each halving of the distance a lane gives half of its rows away, so 16 rows take
-// 16 exchanges instead of 80. Portions of several tokens walk them one by one, the state stays in registers.
+// 16 exchanges instead of 80. Steps come here whose longest portion is one token; should one be longer than the caller said, its tokens are walked one by one.
 //
 // MI355X, 64 sequences x 8 heads of 128 x 128 (34 MB read and written), constant decay: 16 us; 64 sequences x 64 heads of 64 x 128 (268 MB), state-space duality 44 us = 6.1 TB/s
-// (79; walk of recurrent.hip, a row spread over 16 entries per lane and the
-// token's operands staged in LDS behind a barrier: 27).
+// (the walk of recurrent.hip, a row spread over 16 entries per lane and the token's operands staged in LDS behind a barrier: 27 and 79).
 #include "scan_chunk.h"
 
 namespace {
