@@ -242,8 +242,7 @@ template <int D, int DV, int NW>
 int launch_f32(const WindowAttnArgs& a, dim3 grid, hipStream_t stream) {
   constexpr int LDS = NW * (DV / 16 * 1024 + 128);
   const auto kernel = window_attn_f32_kernel<D, DV, NW>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_window_attn: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_window_attn");
   kernel<<<grid, dim3(64 * NW), LDS, stream>>>(a);
   return nvs_check_launch("nvs_window_attn (32-bit tiles)");
 }

@@ -502,8 +502,7 @@ int launch_prompt(WindowAttnArgs a, hipStream_t stream) {
   a.bs_shift = __builtin_ctz(a.block_size);
   constexpr int LDS = 2 * (64 * D * 2 + DV * 128);
   const auto kernel = window_attn_prompt_kernel<D, DV, NW, EXT>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_window_attn: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_window_attn");
   kernel<<<dim3((unsigned)p.tiles, (unsigned)p.rows), dim3(64 * NW), LDS, stream>>>(a);
   return nvs_check_launch("nvs_window_attn (prompts)");
 }

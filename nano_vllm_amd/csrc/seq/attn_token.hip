@@ -247,8 +247,7 @@ int launch_token(WindowAttnArgs a, hipStream_t stream) {
   a.bs_shift = __builtin_ctz(a.block_size);
   constexpr int LDS = NW * (32 * D * 2 + DV * 64 + D * 4 + 128);
   const auto kernel = window_attn_token_kernel<D, DV, NW>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_window_attn: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_window_attn");
   kernel<<<dim3((unsigned)a.n, (unsigned)(a.G * ((a.H / a.G + 15) / 16))), dim3(64 * NW), LDS, stream>>>(a);
   return nvs_check_launch("nvs_window_attn (single tokens)");
 }

@@ -149,8 +149,7 @@ template <int K, int N, bool TURNED>
 int launch_heads(LatentArgs p, hipStream_t st) {
   constexpr int LDS = K * N * 2 + 4 * 16 * N * 2;
   const auto kernel = latent_heads_kernel<K, N, TURNED>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_latent_heads: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_latent_heads");
   const int64_t tiles = (p.n + 127) / 128, chunks = 512 / p.H > 0 ? 512 / p.H : 1;
   p.rows = (int)((tiles + chunks - 1) / chunks) * 128;
   const int64_t blocks = (p.n + p.rows - 1) / p.rows * p.H;

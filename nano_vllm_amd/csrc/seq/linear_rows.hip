@@ -166,8 +166,7 @@ int launch_rows(RowsArgs a, hipStream_t st) {
   const int64_t blocks = ((int64_t)a.tiles_n + 7) / 8 * 8 * a.tiles_m;
   NVS_REQUIRE(blocks < (1ll << 31), "nvs_linear_rows: product too large");
   const auto kernel = linear_rows_kernel<T, NT, MT, NW, D, GLU>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_linear_rows: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_linear_rows");
   kernel<<<dim3((unsigned)blocks), dim3(NW * 64), LDS, st>>>(a);
   return nvs_check_launch("nvs_linear_rows");
 }

@@ -808,8 +808,7 @@ int launch_pipe(const void* X, int64_t ldx, const void* W, int nout, int K, cons
   int64_t blocks = (tiles + 8 * group - 1) / (8 * group) * (8 * group);
   NVS_REQUIRE(blocks < (1ll << 31), "nvs_moe_gemm: step too large");
   const auto kernel = moe_gemm_pipe_kernel<T, GLU, WN, WB, RB, ST, PER_CU, PLAN>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_moe_gemm: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_moe_gemm");
   // the ring goes on over the tiles of a workgroup if every stage holds a step of every tile
   if (K / (128 / (int)sizeof(T)) >= ST && blocks > 256 * PER_CU) blocks = 256 * PER_CU;
   kernel<<<dim3((unsigned)blocks), dim3(256), LDS, st>>>((const T*)X, ldx, (const T*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n,

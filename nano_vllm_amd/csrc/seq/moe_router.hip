@@ -298,8 +298,7 @@ int launch_router(const RouterArgs& a, hipStream_t st) {
   constexpr int LDS = NW * (MT * 16 * 128 + NT * 16 * (sizeof(T) == 2 ? 256 : 128));
   static_assert(LDS >= MT * 16 * (2 * MAX_ROUTER + 1) * 4, "logits and group scores");
   const auto kernel = moe_router_kernel<T, NT, MT>;
-  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  NVS_REQUIRE(room == hipSuccess, "nvs_moe_router: %d bytes of LDS were refused", LDS);
+  NVS_LDS_ROOM(kernel, LDS, "nvs_moe_router");
   kernel<<<dim3((unsigned)((a.n + MT * 16 - 1) / (MT * 16)), (unsigned)a.splits), dim3(NW * 64), LDS, st>>>(a);
   if (a.parts) moe_router_parts_kernel<NT><<<dim3((unsigned)((a.n + 31) / 32)), dim3(128), 0, st>>>(a);
   return nvs_check_launch("nvs_moe_router");

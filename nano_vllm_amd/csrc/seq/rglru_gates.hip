@@ -213,8 +213,7 @@ extern "C" int nvs_rglru_gates(const float* u, const float* w, const float* bias
   NVS_REQUIRE(grid < (1ll << 31) && rows < (1ll << 31), "nvs_rglru_gates: step too large");
   NVS_DISPATCH(dtype, {
     const auto kernel = rglru_gates_kernel<T>;
-    static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PARTS * PART_BYTES);
-    NVS_REQUIRE(room == hipSuccess, "nvs_rglru_gates: %d bytes of LDS were refused", PARTS * PART_BYTES);
+    NVS_LDS_ROOM(kernel, PARTS * PART_BYTES, "nvs_rglru_gates");
     kernel<<<dim3((unsigned)grid), dim3(512), PARTS * PART_BYTES, (hipStream_t)stream>>>(u, w, bias, (const T*)lam, c, channels, blocks, n, (int)rows, pairs);
   });
   return nvs_check_launch("nvs_rglru_gates");

@@ -4,6 +4,7 @@
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <atomic>
 #include "../../../include/nvl_seq.h"
 
 typedef __bf16 bf16_t;
@@ -17,6 +18,19 @@ int nvs_check_launch(const char* what);
       nvs_set_error(__VA_ARGS__);    \
       return NVS_EINVAL;             \
     }                                \
+  } while (0)
+
+// Room for a kernel's dynamic LDS, once on each device that the process launches it on
+#define NVS_LDS_ROOM(kernel, bytes, what)                                                                                                                     \
+  do {                                                                                                                                                        \
+    static std::atomic<uint64_t> nvs_room{0};                                                                                                                 \
+    int nvs_device = 0;                                                                                                                                       \
+    (void)hipGetDevice(&nvs_device);                                                                                                                          \
+    if (!(nvs_room.load(std::memory_order_relaxed) >> (nvs_device & 63) & 1)) {                                                                               \
+      NVS_REQUIRE(hipFuncSetAttribute((const void*)(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess,                                \
+                  what ": %d bytes of LDS were refused", (int)(bytes));                                                                                       \
+      nvs_room.fetch_or(1ull << (nvs_device & 63), std::memory_order_relaxed);                                                                                \
+    }                                                                                                                                                         \
   } while (0)
 
 // element access in 32-bit whatever the storage type

@@ -674,3 +674,12 @@ def test_captured_decode_steps_say_that_they_are_single_tokens(bs, monkeypatch):
     r.model, r.sampler, r.tokens_dev = Model(), lambda *a, **k: None, torch.zeros(128)
     r._decode_body(bs)
     assert made == [((bs, bs, 1), {})] and steps == ["portions"]
+
+
+def test_room_in_lds_is_asked_for_on_every_device():
+    """A function's attributes belong to a device: asked for once a process, the first device's kernels alone would have them."""
+    root = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nano_vllm_amd", "csrc", "seq")
+    for name in sorted(os.listdir(root)):
+        with open(os.path.join(root, name)) as fh:
+            for line in fh:
+                assert not ("static" in line and "hipFuncSetAttribute" in line), (name, line)
