@@ -974,12 +974,6 @@ __device__ __forceinline__ void mfma8_body(
       const int pf_b = in_seg ? b : b2, pf_h = in_seg ? h : h2, pf_t = in_seg ? ti + 1 : t02;
       const int pf_sh = in_seg ? shb : shb2;
       const int pf_blk = has_pf ? tile_block(pf_b, pf_t, pf_sh) : 0;
-      // what the page holds behind the context need not be finite: its values are taken as 0 (they weigh 0)
-      if (t + kTile > len_cached) {
-#pragma unroll
-        for (int i = 0; i < kTL; ++i)
-          if (t + (KV8 ? i * 8 + (lane >> 3) : i * 4 + rq) >= len_cached) vd[i] = u32x4_t{0u, 0u, 0u, 0u};
-      }
       // registers -> this wave's LDS tile (K in swizzled 16-byte slots, V row-major padded), then the next tile's loads
       if constexpr (KV8) {
         // lane holds elements 16 (lane & 7) .. of row 8 i + (lane >> 3): bf16 16-byte chunks c0, c0 + 1 of that row
@@ -991,6 +985,12 @@ __device__ __forceinline__ void mfma8_body(
           fp8x16_to_bf16(kd[i], &lo16, &hi16);
           *reinterpret_cast<u32x4_t*>(k_lds + rowi * kMKRow + ((c0 ^ (rowi & 15)) << 4)) = lo16;
           *reinterpret_cast<u32x4_t*>(k_lds + rowi * kMKRow + (((c0 + 1) ^ (rowi & 15)) << 4)) = hi16;
+        }
+        // (what the page holds behind the context need not be finite: its values are taken as 0, they weigh 0)
+        if (t + kTile > len_cached) {
+#pragma unroll
+          for (int i = 0; i < kLoads8; ++i)
+            if (t + i * 8 + r8 >= len_cached) vd[i] = u32x4_t{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (int i = 0; i < kLoads8; ++i) {
@@ -1005,6 +1005,12 @@ __device__ __forceinline__ void mfma8_body(
         for (int i = 0; i < kLoads; ++i) {
           const int rowi = i * 4 + rq;
           *reinterpret_cast<u32x4_t*>(k_lds + rowi * kMKRow + ((sub ^ (rowi & 15)) << 4)) = kd[i];
+        }
+        // (what the page holds behind the context need not be finite: its values are taken as 0, they weigh 0)
+        if (t + kTile > len_cached) {
+#pragma unroll
+          for (int i = 0; i < kLoads; ++i)
+            if (t + i * 4 + rq >= len_cached) vd[i] = u32x4_t{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (int i = 0; i < kLoads; ++i)
