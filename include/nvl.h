@@ -300,10 +300,19 @@ int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride,
                                 int kv_dtype, const void* plan, float* lse,
                                 int qkv_splits, int64_t qkv_split_stride, void* stream);
 
+/* qkv_splits (ABI 4): 0 = `qkv` is the bf16 output [batch, qkv_tok_stride] of the qkv projection
+ * (QKVParallelLinear.forward, layers/linear.py:96-128). 1..8 = `qkv` is the fp32 split-K slab stack
+ * [qkv_splits][batch][qkv_tok_stride] that nvl_linear_wide mode 2 leaves for a deep-K projection
+ * (slab s at element offset s * qkv_split_stride): the attention prologue sums a row piece over the
+ * slabs in slab order and rounds it to bf16 once — the value the separate slab-reduce launch would
+ * have produced, bit for bit — before the norm / rotation. Matrix-core kernel only (Hq / Hkv in
+ * 2 ... 16; group size 1 returns NVL_EUNSUPPORTED). */
+
 /* nvl_paged_attn_decode_fused of up to 4 sequences, max_context <= 16384 (bf16 cache, group sizes of the matrix-core kernel, no shared prefix) without the merge of a context's parts:
  * workspace receives [batch][Hq][parts][128] 32-bit numerators, [batch][Hq][parts][2] maximum (base 2) and sum, and [batch][Hq][128] bf16. parts =
- * nvl_paged_attn_decode_open_parts (0: the step is too large); a context has min(parts, max(1, ceil(tokens / 256))) of them. One of a
- * single part is finished, as bf16; an empty one's row is zero. */
+ * nvl_paged_attn_decode_open_parts (0: the step is too large); a context of t = ceil(tokens / 32) tiles
+ * has n = max(1, ceil(t / 8)) of them where that is at most parts, else ceil(t / ceil(t / parts)), of ceil(t / n) tiles each and the last of what is left (never none). A
+ * context of a single part is finished, as bf16; an empty one's row is zero. */
 int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context);
 int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
                                int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables, int64_t bt_stride, const int32_t* context_lens,
@@ -314,13 +323,6 @@ int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const vo
 int nvl_linear_decode_open_splits(int64_t m, int n, int k);
 int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight, void* out,
                            int64_t m, int n, int k, int weight_layout, void* stream);
-/* qkv_splits (ABI 4): 0 = `qkv` is the bf16 output [batch, qkv_tok_stride] of the qkv projection
- * (QKVParallelLinear.forward, layers/linear.py:96-128). 1..8 = `qkv` is the fp32 split-K slab stack
- * [qkv_splits][batch][qkv_tok_stride] that nvl_linear_wide mode 2 leaves for a deep-K projection
- * (slab s at element offset s * qkv_split_stride): the attention prologue sums a row piece over the
- * slabs in slab order and rounds it to bf16 once — the value the separate slab-reduce launch would
- * have produced, bit for bit — before the norm / rotation. Matrix-core kernel only (Hq / Hkv in
- * 2 ... 16; group size 1 returns NVL_EUNSUPPORTED). */
 
 /* ---- Varlen causal prefill attention (MFMA) ----------------------------------
  * Replaces flash_attn_varlen_func as called at layers/attention.py:67-70:

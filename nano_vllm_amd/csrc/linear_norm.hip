@@ -10,7 +10,8 @@
 // fill the chip otherwise (1024 x 3072, one row: 3.6 us in four slabs, 5.2 whole).
 //   v = x + residual (slabs: v = bf16(sum) + residual);  residual' = bf16(v);  h = bf16(v rsqrt(mean v^2 + eps) w);  out = h W^T, or silu(gate) * up of its halves
 // MI355X, one row, traced: 4096 x 1024 with the norm 4.3 us (norm 2.4, product 3.6, and a gap), 6144 x 1024 with norm and SiLU 5.7 (2.4 + 5.3); a step of one
-// sequence through 28 layers 954 -> 925 us.
+// sequence through 28 layers 954 -> 925 us. The rows are normed by every workgroup, so more and wider ones lose what the launch gives: layers.py calls
+// this for up to 8 rows of width 1,024, with the figures beside it.
 #include "common.h"
 
 namespace {

@@ -533,7 +533,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 //
 // Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
 // four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
-// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.27 to 2.31 + 1.32 to 1.34 ms = 1180 to 1200 and 1020 to 1030 TFLOP/s (the tiled kernel: 4.05 +
+// and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.27 to 2.38 + 1.32 to 1.41 ms = 1150 to 1200 and 970 to 1030 TFLOP/s (the tiled kernel: 4.05 +
 // 2.28 ms; the library's dense product of these sizes: 1.3-1.46 PFLOP/s); what is left is the chip's power limit and half a tile of padding
 // per expert. 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
 // (moe_gemm_mfma_kernel 411 + 217); width 1024, ff 768: 20 + 12 us (58 + 27). 32-bit, 1,044 rows, width 1024: 59 + 32 us (moe_gemm_kernel
@@ -566,6 +566,8 @@ constexpr int pipe_turn = sizeof(T) == 2 && PER_CU == 1 ? 4096 : 0;
 // silu(g) u. 16-bit results: g / (1 + e^-g) with the hardware's exponential and reciprocal. What the rounding of g log2 e took (up to |g| units of 2^-24 of the result) is
 // added back, and so is the quotient's remainder. Results that are not the nearest bfloat16 number to silu(g), in 2^-16 of a million gates in [-20, -10], [-10, -4],
 // [-2, 2]: 0.13, 0.25, 0.25; with expf and a division 0.13, 0.13, 0.19; without the two corrections 4.1, 1.6, 0.6. Below -87 the result is 0.
+// They are seven instructions a value while the matrix pipe waits: 14,600 rows, ff 3072, K 1024 184 us without, 197 with them. Eight values side by side take as long, and a
+// step of Newton for the reciprocal in the remainder's place (one instruction fewer) leaves 0.38, 0.31, 0.5.
 template <typename T>
 __device__ __forceinline__ float silu_times(float g, float u) {
   if constexpr (sizeof(T) == 4) return glu_value(g, u, 0, 0.f, 0.f);

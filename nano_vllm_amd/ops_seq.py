@@ -679,7 +679,7 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, glu: bool) -> bool:
     """Whether x w^T goes to nvs_linear_rows: whole 128-byte pieces of k, few rows and not too many of w. MI355X, us here / the library's, bf16: 64 rows,
     1024 x 1024 3.6 / 8.6, 1024 x 3072 4.9 / 10.0, 4096 x 1024 4.5 / 8.6, 4096 x 4096 12.3 / 14.7, 6144 x 1024 5.8 / 8.8, 12288 x 2048 13.8 / 12.9,
     24576 x 4096 54.8 / 47.9; 256 rows, 1024 x 1024 4.2 / 8.3, 4096 x 4096 19.5 / 22.2, 6144 x 1024 12.8 / 12.3; 128 rows of it 7.5 / 9.5; 16 rows,
-    12288 x 2048 11.7 / 11.6, 32768 x 4096 51.9 / 62.6. The activation on the way saves its launch (4 us and its passes): more is taken. 32-bit: 330 rows,
+    12288 x 2048 11.7 / 11.6, 32768 x 4096 57.9 / 60.3 (its 268 MB out of memory). The activation on the way saves its launch (4 us and its passes): more is taken. 32-bit: 330 rows,
     1024 x 1024 10.3 / 11.8, 4096 x 1024 33.6 / 41.3, 3084 x 1024 30.9 / 23.8; 512 rows, 1024 x 2048 21.3 / 21.5, 4096 x 1024 42.9 / 36.2."""
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         return False

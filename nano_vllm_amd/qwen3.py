@@ -8,7 +8,7 @@ is arranged for MI355X:
    add+RMSNorm -> gate_up GEMM -> SiLU*mul -> down GEMM (+all-reduce)
 
 i.e. 10 launches per layer instead of the reference's 13 (each dependent kernel boundary is
-~1.5 us on this chip even inside a hipGraph — MI355X_MICROARCH.md "boundary"; a small dependent
+~1.5 us on this chip even inside a hipGraph; a small dependent
 kernel costs ~5 us whatever it does). On decode-sized batches (<= 256 rows, TP=1, single-K-pass
 shapes) the chain is 8 launches:
 
