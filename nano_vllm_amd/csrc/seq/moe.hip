@@ -7,6 +7,7 @@
 // sequence can be captured in a hipGraph; the order in which pairs land inside an expert's rows is arbitrary but no sum depends
 // on it (a row is computed on its own, and a token's choices are added in the order of its choices).
 #include "seq_common.h"
+#include <type_traits>
 
 namespace {
 
@@ -518,7 +519,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 // could not write padding). The MFMAs are written out with accumulators in the accumulation registers and operands in the vector registers:
 // left to itself the compiler moves one or the other between the two files in the loop.
 //
-// As many workgroups as fit on the chip at once, and each goes on from tile to tile: the last ST steps of a tile ask for the first ones of the next, whose
+// (16-bit tiles of 256 rows are gemm_tiles.h's, but for rows and results that it does not take.) As many workgroups as fit on the chip at once, and each goes on from tile to tile: the last ST steps of a tile ask for the first ones of the next, whose
 // rows were looked up a whole tile earlier, so no tile but the first waits for its plan, its addresses and its operands, and the stores drain behind the next
 // tile's first steps. Full tiles of 256 rows x 256 weight rows, us per tile at k = 256 / 1024 / 4096, before and after (the products alone take 5.9 / 23.6 /
 // 94): gated 22.4 / 42.2 / 111.8 -> 13.1 / 32.0 / 106.9, plain 20.7 / 41.0 / 111.0 -> 14.7 / 36.8 / 109.0; tiles of 128 rows, gated 12.5 / 22.3 / 62.5 -> 7.3 / 17.4 / 58.3; of
@@ -534,8 +535,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 // Why 128 x 128 per wavefront for many rows: per 32 of k it reads 16 operands for 64 MFMAs, which keeps the LDS pipe (128 bytes a clock for
 // four SIMDs) at half of the matrix pipe's time; the 64 x 64 wavefront tile of moe_gemm_tiled_kernel needs all of it. Measured on MI355X, gate|up
 // and down of 32 experts: 54,200 rows, width 4096, ff 3072 at tiles of 256 rows 2.27 to 2.38 + 1.32 to 1.41 ms = 1150 to 1200 and 970 to 1030 TFLOP/s (the tiled kernel: 4.05 +
-// 2.28 ms; the library's dense product of these sizes: 1.3-1.46 PFLOP/s); what is left is the chip's power limit and half a tile of padding
-// per expert. 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
+// 2.28 ms). 256 rows (a decode step of 64 sequences, 1.6 + 0.8 GB of weights) at tiles of 16 rows 289 + 141 us = 5.6 TB/s
 // (moe_gemm_mfma_kernel 411 + 217); width 1024, ff 768: 20 + 12 us (58 + 27). 32-bit, 1,044 rows, width 1024: 59 + 32 us (moe_gemm_kernel
 // 1130 + 763), error against 64-bit sums 9e-7 of the result.
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -818,6 +818,8 @@ int launch_pipe(const void* X, int64_t ldx, const void* W, int nout, int K, cons
   return nvs_check_launch("nvs_moe_gemm (matrix cores, pipelined)");
 }
 
+#include "gemm_tiles.h"
+
 // ---- combine: one workgroup per token ------------------------------------------------------------------------------------
 template <typename T, int VEC>
 __global__ void moe_combine_kernel(const T* __restrict__ rows, int64_t ldr, const int32_t* __restrict__ pair_row,
@@ -949,6 +951,10 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
               : launch_pipe<bf16_t, false, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)) \
        : (glu ? launch_pipe<float, true, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)  \
               : launch_pipe<float, false, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)))
+    if (tm == 256 && dtype == NVS_BF16 && tiles_fit(ldx, cap, nout, K, (glu ? 2ll : 1ll) * nout * K, out, ldo)) {
+      const auto launch = glu ? launch_tiles<1, true> : mode ? launch_tiles<2, true> : launch_tiles<0, true>;
+      return launch(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, st, 0);
+    }
     if (tm == 256) return NVS_PIPE(2, 8, 8, 2, 1);
     if (tm == 128) return NVS_PIPE(2, 8, 4, 3, 1);
     if (tm == 64) return NVS_PIPE(4, 4, 4, 2, 2);
@@ -1000,6 +1006,7 @@ extern "C" int nvs_silu_linear(const void* X, int64_t ldx, const void* W, int ff
               "nvs_silu_linear: %lld rows, %d x %d", (long long)n, ff, K);
   NVS_REQUIRE((tm == 64 || tm == 256) && n < (1ll << 31) - 256 && (n + 255) * ldx < (8ll << 32) && 2ll * ff * K < (8ll << 32), "nvs_silu_linear: step too large");
   const int64_t cap = (n + tm - 1) / tm * tm;
+  if (tm == 256 && tiles_fit(ldx, n, ff, K, 2ll * ff * K, out, ldo)) return launch_tiles<1, false>(X, ldx, W, ff, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, (int)n);
   if (tm == 256) return launch_pipe<bf16_t, true, 2, 8, 8, 2, 1, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
   return launch_pipe<bf16_t, true, 4, 4, 4, 2, 2, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
 }

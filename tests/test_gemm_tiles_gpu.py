@@ -1,0 +1,54 @@
+"""Products in tiles of 256 rows (csrc/seq/gemm_tiles.h) where they can go wrong: one row and one feature unit, the edges of a tile in rows and features, the fewest
+steps (two) and counts that leave the ring at each of its places, passes that are whole, part-filled above half (whole tiles) and below (halves of 128 rows), and
+plans with experts of no row, half a tile and one row more."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,ff,K", [(1, 8, 128), (128, 128, 192), (129, 136, 256), (257, 1000, 320), (256, 256, 384), (2048, 4096, 128), (2100, 4096, 192),
+                                    (3072, 4096, 448), (3100, 4096, 128), (9000, 768, 1024)])
+def test_dense_products(n, ff, K):
+    from nano_vllm_amd import ops_seq
+    g = torch.Generator().manual_seed(n + ff)
+    x = torch.randn(n, K + 8, generator=g).to(torch.bfloat16).cuda()[:, :K]
+    w = (torch.randn(2 * ff, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    room = torch.full((n + 300, ff + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = x.double() @ w.double().T
+    want = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+    for _ in range(2):
+        ops_seq.silu_linear(x, w, 256, room[:n, :ff])
+        # one rounding of the result to bfloat16, 2^-9 at most per value
+        assert ((room[:n, :ff].double() - want).norm() / want.norm()).item() <= 2.0 ** -8
+        assert (room[n:] == 7.0).all() and (room[:, ff:] == 7.0).all()
+
+
+@pytest.mark.parametrize("mode", ["glu", "relu2", "rows"])
+@pytest.mark.parametrize("counts,nout,K", [([0, 1, 256, 257, 128, 129], 264, 128), ([5], 8, 192), ([700, 0, 0, 513], 8192, 256), ([2300, 1, 1000], 4096, 320)])
+def test_grouped_products(mode, counts, nout, K):
+    from nano_vllm_amd import ops_seq
+    E, n = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(nout + K)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(n, generator=g)].to(torch.int32).cuda()
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(E, (2 if mode == "glu" else 1) * nout, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    plan = ops_seq.moe_plan(ids.view(n, 1), E, 256)
+    rows = plan.pair_row.view(-1).long()
+    src = x
+    if mode == "rows":
+        src = torch.full((plan.cap, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+        src[rows] = x
+    out = torch.full((plan.cap, nout), 7.0, dtype=torch.bfloat16, device="cuda")
+    for _ in range(2):
+        ops_seq.moe_gemm(src, w, plan, mode == "glu", out, relu2=mode == "relu2")
+    for e in range(E):
+        mine = (ids == e).nonzero().view(-1)
+        if not len(mine):
+            continue
+        y = x[mine].double() @ w[e].double().T
+        want = torch.nn.functional.silu(y[:, :nout]) * y[:, nout:] if mode == "glu" else y.clamp(min=0) ** 2 if mode == "relu2" else y
+        assert ((out[rows[mine]].double() - want).norm() / want.norm()).item() <= 2.0 ** -8       # (one rounding of the result to bfloat16)
+    untouched = torch.ones(plan.cap, dtype=torch.bool, device="cuda")
+    untouched[rows] = False
+    assert (out[untouched] == 7.0).all()
