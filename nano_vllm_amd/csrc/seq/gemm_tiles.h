@@ -7,6 +7,8 @@
 //   v_mfma_f32_32x32x16_bf16 538 us, v_mfma_f32_16x16x32_bf16 493 us: the smaller one moves half the accumulators per product.
 //   Requests one by one between the products, and half of them a half step earlier: 12 % less than in bursts behind the step's barrier, where they also queue up for
 //   the path into LDS (64 KB a step, 64 bytes a clock).
+//   Products in an order in which one operand of two is the one before, either in turn: 1 % less than all of one row of blocks behind the other (8,192 x 24,576 x 4096 1125 -> 1112 us).
+//   Results stored as a stream: they do not push out the operands that neighbours share (the same 1112 -> 1043 us; outputs below 130 MB the same either way).
 //   Addresses as 32-bit offsets of a buffer, one LDS base for four requests, no branch in the loop: a step of 128 products takes 2,360 clocks, 2,715 before; 128 products
 //   back to back 2,176.
 //
@@ -20,8 +22,8 @@
 // or 256 bytes; the number of stores does not depend on the rows that are there (those that are not go nowhere), so the next tile's waits can count them and none waits for them to drain.
 // Tiles that are left for a last pass of at most 128 workgroups are halved: 14,600 rows and 24 feature tiles are 5.4 passes, not 6 (gate|up at K 1024 7 % of its time).
 //
-// us before (moe_gemm_pipe_kernel's tiles of 256 rows) / now, whole calls on one card: gate|up and SiLU, 14,600 rows, ff 3072, K 1024 185 / 157, K 4096 581 / 500; rows, 14,175 x 4096 x 4096
-// 399 / 326 (the library 331), 14,600 x 4096 x 1024 128 / 109, 14,600 x 1024 x 3072 92 / 78.
+// us before (moe_gemm_pipe_kernel's tiles of 256 rows) / now, whole calls on one card: gate|up and SiLU, 14,600 rows, ff 3072, K 1024 185 / 154, K 4096 581 / 495; rows, 14,175 x 4096 x 4096
+// 399 / 324 (the library 331), 14,600 x 4096 x 1024 128 / 107, 14,600 x 1024 x 3072 92 / 77. Against the library: ops_seq.py (tiles_rule, silu_linear_rows).
 #pragma once
 
 // ring of five parts
@@ -31,8 +33,9 @@ constexpr uint32_t TILE_REACH = 0xC0000000u, TILE_NOWHERE = 0xF0000000u, TILE_SK
 template <int MODE, bool PLAN>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W, int nout, int K,
                                                             const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ row_token, int tiles_m,
-                                                            int tiles_n, uint32_t band_inverse, int rows, bf16_t* __restrict__ out, int64_t ldo) {
-  constexpr bool GLU = MODE == 1;
+                                                            int tiles_n, uint32_t band_inverse, int rows, const bf16_t* __restrict__ bias,
+                                                            bf16_t* __restrict__ out, int64_t ldo) {
+  constexpr bool GLU = MODE == 1, GATHER = MODE == 1 || MODE == 2;    // (0: rows, 1: SiLU of gate times up, 2: squares of positive results, 3: rows plus a bias)
   constexpr int NG = GLU ? 2 : 1, BN = 256 / NG, R = 8;               // features of a tile, requests of a wavefront per part
   extern __shared__ __attribute__((aligned(128))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15;
@@ -74,7 +77,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
   uint32_t xoff[R], woff[R];
   int tok[R];
   const auto look = [&] {
-    if constexpr (MODE != 0) {
+    if constexpr (GATHER) {
       int l = lane;
       asm volatile("" : "+v"(l));             // (what follows from the lane alone is worked out here, not kept over the loop)
       const int64_t first = (int64_t)rt * 256 + sub + (low ? (wave >> 1) * 64 : wave * 64) + (l >> 3);
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const uint32_t xunit = (u ^ ((i * 4 & 4) | l3 >> 1)) * 16 - i % 4 * 1024, wunit = (u ^ ((l3 >> 1 & 1) | (i * 2 & 6))) * 16 - i % 4 * 1024;
-      if constexpr (MODE == 0) xoff[i] = none || (!PLAN && first + i * 8 >= rows) ? TILE_NOWHERE : xfirst + i * 8 * x2 + xunit;
+      if constexpr (!GATHER) xoff[i] = none || (!PLAN && first + i * 8 >= rows) ? TILE_NOWHERE : xfirst + i * 8 * x2 + xunit;
       else xoff[i] = tok[i] < 0 ? TILE_NOWHERE : (uint32_t)tok[i] * x2 + TILE_SKEW + xunit;
       woff[i] = f + i * 8 < nout ? wfirst + i * 8 * w2 + wunit : TILE_NOWHERE;
     }
@@ -127,7 +130,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
     constexpr int RB = decltype(RBC)::value, READS = RB + 8;
 #pragma unroll
     for (int n = 0; n < 8 * RB; ++n) {
-      const int a = n / RB, b = a % 2 ? RB - 1 - n % RB : n % RB;
+      const int m = n / 2 % RB, pair = n / 2 / RB, b = pair % 2 ? RB - 1 - m : m, a = pair * 2 + (m % 2 ? 1 - n % 2 : n % 2);      // (either operand in turn is the one before)
       if constexpr (decltype(FIRST)::value) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[a][b]) : "v"(now.w[a]), "v"(now.x[b]));
       else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[a][b]) : "v"(now.w[a]), "v"(now.x[b]));
       __builtin_amdgcn_sched_barrier(0);
@@ -170,6 +173,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
     if (more) look();
     f32x4_t acc[8][RB];                       // [block of 16 weight rows][block of 16 rows]
     int live[RB];
+    u32x4_t offset[4];                        // the bias of a lane's features
     int s = 0, ahead = 2;
 #pragma unroll 1
     do {
@@ -180,6 +184,10 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
           point();
         } else {                              // nothing follows: the last requests bring nothing
           xs = near(X, 0), ws = near(W, 0);
+        }
+        if constexpr (MODE == 3) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) offset[j] = *(const u32x4_t*)(bias + min(f0 + j * 32 + (lane >> 4) * 8, nout - 8));
         }
         if constexpr (PLAN) {
 #pragma unroll
@@ -226,6 +234,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
         for (int i = 0; i < 8; ++i) {
           const float y = acc[2 * j + i / 4][rb][i % 4];
           if constexpr (GLU) o.v[i] = (bf16_t)silu_times<bf16_t>(y, acc[2 * j + i / 4 + 4][rb][i % 4]);
+          else if constexpr (MODE == 3) o.v[i] = (bf16_t)(y + __builtin_bit_cast(float, i % 2 ? offset[j][i / 2] & 0xFFFF0000u : offset[j][i / 2] << 16));
           else o.v[i] = (bf16_t)plain_value(y, MODE);
         }
         turn[rb % 2 * 16 * UNITS + place(l & 15, j * 4 + (l >> 4))] = o.q;
@@ -242,8 +251,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t on = (uint32_t)__ballot((PLAN ? live[rb] : token(row0 + rb * 16 + (l & 15))) >= 0);
 #pragma unroll
-      for (int p = 0; p < 16 / PER; ++p)
-        __builtin_amdgcn_raw_buffer_store_b128(q[p], os, (on >> (p * PER + line) & 1) && inside ? to : TILE_NOWHERE, (rb * 16 + p * PER) * (int)ldo * 2, 0);
+      for (int p = 0; p < 16 / PER; ++p)      // (2: not to be kept in the caches)
+        __builtin_amdgcn_raw_buffer_store_b128(q[p], os, (on >> (p * PER + line) & 1) && inside ? to : TILE_NOWHERE, (rb * 16 + p * PER) * (int)ldo * 2, 2);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
     stores = RB * 16 / PER;
@@ -264,12 +273,12 @@ inline bool tiles_fit(int64_t ldx, int64_t rows, int nout, int K, int64_t weight
 
 template <int MODE, bool PLAN>
 int launch_tiles(const void* X, int64_t ldx, const void* W, int nout, int K, const int32_t* tile_expert, const int32_t* row_token, int64_t cap, void* out,
-                 int64_t ldo, hipStream_t st, int rows = 0) {
+                 int64_t ldo, hipStream_t st, int rows = 0, const void* bias = nullptr) {
   constexpr int BN = MODE == 1 ? 128 : 256;
   const int64_t tiles_m = (cap + 255) / 256, tiles_n = (nout + BN - 1) / BN;
   const auto kernel = gemm_tiles_kernel<MODE, PLAN>;
   NVS_LDS_ROOM(kernel, TILE_RING, "nvs_moe_gemm");
   kernel<<<dim3(256), dim3(256), TILE_RING, st>>>((const bf16_t*)X, ldx, (const bf16_t*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n, (uint32_t)((1ull << 32) / (8 * tiles_n) + 1), rows,
-                                                  (bf16_t*)out, ldo);
+                                                  (const bf16_t*)bias, (bf16_t*)out, ldo);
   return nvs_check_launch("nvs_moe_gemm (matrix cores, tiles of 256 rows)");
 }

@@ -342,11 +342,13 @@ class LinearBase(nn.Module):
             y = decode_linear(x, self.weight, ops.LINEAR_BF16, packed=self.weight_packed)
             if y is not None:
                 return y
+        if x.shape[0] >= ops_seq.TILES_FROM and ops_seq.loaded() and ops_seq.many_rows(x, self.weight, self.bias):
+            return ops_seq.linear_tiles(x, self.weight, self.bias)
         return F.linear(x, self.weight, self.bias)
 
 
 # Row counts up to this use the hand-written decode GEMMs (nvl_linear_decode / nvl_linear_wide); above it the
-# library GEMM wins (measured crossover on MI355X, tools/gemm_bench.py).
+# library GEMM wins (measured crossover on MI355X, tools/gemm_bench.py), until many rows fill tiles of 256 (ops_seq.tiles_rule).
 DECODE_LINEAR_MAX_ROWS = 256
 
 

@@ -70,6 +70,7 @@ SIGNATURES = {
     "nvs_moe_plan_scratch": (c_int64, [_L, _I]),
     "nvs_moe_plan_wide": (c_int, [_P, _L, _I, _I, _I, _P, _P, _P, _P, _L, _P]),
     "nvs_silu_linear": (c_int, [_P, _L, _P, _I, _I, _L, _I, _P, _L, _P]),
+    "nvs_linear_tiles": (c_int, [_P, _L, _P, _P, _I, _I, _L, _P, _L, _P]),
     "nvs_moe_gemm": (c_int, [_P, _L, _P, _I, _I, _I, _I, _P, _P, _L, _I, _P, _L, _P]),
     "nvs_moe_force_plain": (None, [_I]),
     "nvs_moe_combine": (c_int, [_P, _L, _P, _P, _I, _P, _L, _P, _P, _L, _I, _L, _I, _P, _P, _P]),
@@ -704,28 +705,82 @@ def _linear_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act: 
     return out
 
 
+TILES_FROM = 768
+
+
+def tiles_rule(n: int, N: int, K: int) -> bool:
+    """Whether x w^T of n rows, N features and K entries each goes to the tiles of 256 rows x 256 features (256 of them are a pass, left-over ones of at most 128 go in
+    halves). MI355X, us here / the library's: 13,550 rows (a prompt step) 4096 x 4096 313 / 321, 6144 x 4096 455 / 620, 12288 x 4096 894 / 1035, 18752 x 4096 1399 / 1474,
+    24576 x 4096 1785 / 1827, 4096 x 12288 918 / 1153, 3088 x 1024 82 / 129, 3072 x 384 37 / 66, 4096 x 256 37 / 60; 12,918 rows, 4096 x 4096 309 / 411. Where the tiles are
+    whole passes the library's are as good or better by themselves: 16,384 rows, 4096 x 4096 363 / 356, 24576 x 4096 2172 / 2123, 15,637 rows, 1024 x 2048 54.1 / 52.3, 1024 x 3072 74.2 / 72.3.
+    But kernels of both kinds in turn cost each other 2 to 3 us a launch, so there too: the 28 layers' steps of 15,637 rows, 4096 x 1024 + 1024 x 2048 + 1024 x 3072, all here
+    16.66 ms, all there 16.71, some here and some there 16.93 to 17.00. One or two passes of which the last is between
+    half and three quarters full: 6,600 rows, 4096 x 4096 166 / 161, 2048 x 4096 at 12,800 91 / 86; a part of one: 2,700 rows, 4096 x 4096 79 / 74, 11,000, 1024 x 3072 65 / 58, but up to half of it
+    2,000 rows, 4096 x 4096 55 / 58, 6,600, 1024 x 3072 40 / 43, 1024 x 1024 17 / 19, 1,300 rows, 4096 x 1024 15 / 20, with short reductions (9,100 rows, 1024 x 256 11 / 19)
+    and with features that are no whole tiles (13,550 rows, 640 x 1024 23 / 30, 1000 x 4096 82 / 111). Fewer tiles leave most of the chip idle: 4,000 rows, 1024 x 3072 37 / 29."""
+    tiles = -(-n // 256) * -(-N // 256)
+    if n < TILES_FROM or tiles < 96:
+        return False
+    if tiles <= 128 or K <= 512 or N % 256:
+        return True
+    rest = tiles % 256 or 256
+    return rest >= 224 if tiles <= 256 else tiles > 512 or rest <= 128 or rest >= 192
+
+
+def linear_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What nvs_linear_tiles takes, of calls that nobody differentiates or traces."""
+    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]
+            and x.shape[1] % 64 == 0 and x.shape[1] >= 128 and w.shape[0] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
+            and w.is_contiguous() and max(x.shape[0] * x.stride(0), w.numel()) < 3 << 29 and not torch.is_grad_enabled() and not torch.jit.is_tracing()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def many_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
+    return (x.dim() == 2 and w.dim() == 2 and tiles_rule(x.shape[0], w.shape[0], x.shape[1]) and linear_tiles_fits(x, w)
+            and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1] and b.data_ptr() % 16 == 0))
+
+
+def _linear_many(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
+    if x.shape[0] >= TILES_FROM and many_rows(x, w, b):         # (asked first: short steps wait for the host)
+        return linear_tiles(x, w, b)
+    return torch.nn.functional.linear(x, w, b)
+
+
 @_launch
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
-    """x [n, K] times w [N, K]^T (+ b): few rows here, many by the vendor library."""
+    """x [n, K] times w [N, K]^T (+ b): few rows and many here, others by the vendor library."""
     if not _few_rows(x, w, False) or not (b is None or b.dtype == x.dtype and b.is_contiguous() and b.shape == w.shape[:1]):
-        return torch.nn.functional.linear(x, w, b)
+        return _linear_many(x, w, b)
     return _linear_rows(x, w, b, -1, 0.0, 0.0, torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device))
 
 
+def linear_tiles(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+    """x w^T (+ b) in tiles of 256 rows: x [n, K], w [N, K], b [N]."""
+    lib = load_library()
+    n, K = x.shape
+    assert x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.is_contiguous() and w.shape[1] == K
+    assert b is None or b.dtype == x.dtype and b.is_contiguous() and b.shape == w.shape[:1]
+    if out is None:
+        out = torch.empty(n, w.shape[0], dtype=x.dtype, device=x.device)
+    assert out.shape == (n, w.shape[0]) and out.stride(1) == 1 and out.dtype == x.dtype
+    _check(lib.nvs_linear_tiles(_ptr(x), x.stride(0), _ptr(w), _ptr(b), w.shape[0], K, n, _ptr(out), out.stride(0), _stream()))
+    return out
+
+
 def silu_linear_rows(n: int, ff: int, K: int) -> int:
-    """Rows per tile of silu_linear, 0 where the vendor library's product and the activation behind it are the faster way. A pass of 256 tiles fills the chip
-    and the last pass may be part-empty; the library's tiles are the better ones for long reductions. MI355X, us there / here at 64 / 256 rows, ff 3072,
-    K 1024: 600 rows 20 / 18 / 31, 1000: 25 / 24 / 33, 2000: 39 / 35 / 35, 6000: 103 / 90 / 95, 9000: 137 / 138 / 126, 14600: 222 / 224 / 185; ff 768, K 1024:
-    2000: 17.3 / 17.6 / 31, 4000: 25 / 24 / 33, 14600: 66 / 59 / 66; ff 4096, K 1536: 1500: 45 / 50 / 47, 4000: 100 / 111 / 93, 9000: 259 / 258 / 217; ff 2048, K 2048:
-    4000: 63 / 74 / 62, 9000: 148 / 161 / 164, 14600: 235 / 259 / 223; ff 6144, K 2048: 3000: 160 / 163 / 164, 6000: 354 / 330 / 270, 14600: 737 / 785 / 619; ff 4608,
-    K 2560: 6000: 276 / 320 / 264, 14600: 661 / 738 / 581; ff 8192, K 3072: 9000: 704 / 956 / 756, 14600: 1226 / 1553 / 1219."""
-    if K % 64 or K > 2560:
+    """Rows per tile of silu_linear, 0 where the vendor library's product and the activation behind it are the faster way. MI355X, us there / here at 64 / 256 rows, ff 3072, K 1024:
+    500 rows 18.7 / 13.7 / 14.9, 800: 20.3 / 20.1 / 15.4, 1300: 26.5 / 22.1 / 25.1, 2000: 36.2 / 33.1 / 26.3, 4000: 67 / 61 / 46, 14600: 199 / 204 / 150; ff 768, K 1024: 800:
+    13.0 / 13.5 / 14.8, 2000: 16.2 / 17.1 / 15.0, 4000: 22.7 / 21.9 / 16.5; ff 2048, K 2048: 800: 23.7 / 28.1 / 25.1, 1300: 30 / 34 / 26, 4000: 60 / 71 / 51; ff 8192, K 3072: 600: 61 / 89 / 63,
+    1000: 87 / 103 / 72, 9000: 721 / 907 / 618; ff 12288, K 4096: 600: 118 / 134 / 128, 1000: 179 / 198 / 143, 14600: 2282 / 2965 / 1984."""
+    columns = -(-2 * ff // 256)
+    tiles = -(-n // 256) * columns
+    if K % 64:
         return 0
-    tiles = -(-n // 256) * -(-2 * ff // 256)
-    passes = -(-tiles // 256)
-    if tiles >= 208 and (tiles >= 216 * passes or tiles >= 768):
-        return 256
-    return 64 if K <= 1024 and tiles >= 72 else 0
+    if ff % 8 or K < 128:                    # (not for the tiles of 256 rows that the figures are of: those before them)
+        return 0 if K > 2560 else 256 if tiles >= 208 and (tiles >= 216 * -(-tiles // 256) or tiles >= 768) else 64 if K <= 1024 and tiles >= 72 else 0
+    if K <= 1024 and tiles > 128 and -(-n // 64) * columns <= 512:           # (two tiles of 64 rows at a time on every compute unit are one pass)
+        return 64
+    return 256 if tiles >= 96 and (n >= 768 or K <= 1536) or tiles >= 48 and n >= 500 and K <= 1024 else 0
 
 
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -757,7 +812,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, ff: int, kind: int = 0, limit: 
         tm = silu_linear_rows(x.shape[0], ff, x.shape[1])
         if tm:
             return silu_linear(x, w, tm, out)
-    glu_act(torch.nn.functional.linear(x, w), ff, out, kind, limit, alpha)
+    glu_act(_linear_many(x, w), ff, out, kind, limit, alpha)
     return out
 
 

@@ -24,6 +24,39 @@ def test_dense_products(n, ff, K):
         assert (room[n:] == 7.0).all() and (room[:, ff:] == 7.0).all()
 
 
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("n,N,K", [(1, 8, 128), (128, 264, 192), (257, 1000, 320), (4096, 4096, 128), (4100, 4096, 192), (6144, 4096, 128), (6200, 4104, 256)])
+def test_dense_rows(n, N, K, biased):
+    from nano_vllm_amd import ops_seq
+    g = torch.Generator().manual_seed(n + N)
+    x = torch.randn(n, K + 8, generator=g).to(torch.bfloat16).cuda()[:, :K]
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    b = torch.randn(N, generator=g).to(torch.bfloat16).cuda() if biased else None
+    room = torch.full((n + 300, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    want = x.double() @ w.double().T + (b.double() if biased else 0.0)
+    for _ in range(2):
+        ops_seq.linear_tiles(x, w, b, room[:n, :N])
+        assert ((room[:n, :N].double() - want).norm() / want.norm()).item() <= 2.0 ** -8          # (one rounding of the result to bfloat16)
+        assert (room[n:] == 7.0).all() and (room[:, N:] == 7.0).all()
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("n,N,K", [(2900, 2576, 192), (13550, 1024, 256), (800, 12288, 512)])
+def test_linear_layers_take_the_tiles_where_the_rule_says(n, N, K):
+    from nano_vllm_amd import ops_seq
+    from nano_vllm_amd.layers import ReplicatedLinear
+    layer = ReplicatedLinear(K, N, bias=True).to(torch.bfloat16).cuda()
+    layer.weight.data.copy_(torch.randn(N, K) / K ** 0.5)
+    layer.bias.data.copy_(torch.randn(N))
+    x = torch.randn(n, K).to(torch.bfloat16).cuda()
+    assert ops_seq.many_rows(x, layer.weight, layer.bias)
+    want = x.double() @ layer.weight.double().T + layer.bias.double()
+    for got in (layer(x), ops_seq.linear(x, layer.weight.data, layer.bias.data)):
+        assert ((got.double() - want).norm() / want.norm()).item() <= 2.0 ** -8
+    with torch.inference_mode(False):
+        assert not ops_seq.many_rows(x, layer.weight, layer.bias)               # (somebody may differentiate)
+
+
 @pytest.mark.parametrize("mode", ["glu", "relu2", "rows"])
 @pytest.mark.parametrize("counts,nout,K", [([0, 1, 256, 257, 128, 129], 264, 128), ([5], 8, 192), ([700, 0, 0, 513], 8192, 256), ([2300, 1, 1000], 4096, 320)])
 def test_grouped_products(mode, counts, nout, K):
