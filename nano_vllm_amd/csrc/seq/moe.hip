@@ -563,18 +563,14 @@ __device__ __forceinline__ void mfma_units(f32x4_t (&acc)[RB], const u32x4_t& w,
 template <typename T, int PER_CU>
 constexpr int pipe_turn = sizeof(T) == 2 && PER_CU == 1 ? 4096 : 0;
 
-// silu(g) u. 16-bit results: g / (1 + e^-g) with the hardware's exponential and reciprocal. What the rounding of g log2 e took (up to |g| units of 2^-24 of the result) is
-// added back, and so is the quotient's remainder. Results that are not the nearest bfloat16 number to silu(g), in 2^-16 of a million gates in [-20, -10], [-10, -4],
-// [-2, 2]: 0.13, 0.25, 0.25; with expf and a division 0.13, 0.13, 0.19; without the two corrections 4.1, 1.6, 0.6. Below -87 the result is 0.
-// They are seven instructions a value while the matrix pipe waits: 14,600 rows, ff 3072, K 1024 184 us without, 197 with them. Eight values side by side take as long, and a
-// step of Newton for the reciprocal in the remainder's place (one instruction fewer) leaves 0.38, 0.31, 0.5.
+// silu(g) u. 16-bit results: silu_hw. Results that are not the nearest bfloat16 number to silu(g), in 2^-16 of a million gates in [-20, -10], [-10, -4],
+// [-2, 2]: 0.13, 0.25, 0.25; with expf and a division 0.13, 0.13, 0.19; without its two corrections 4.1, 1.6, 0.6.
+// They are seven instructions a value while the matrix pipe waits: 14,600 rows, ff 3072, K 1024 184 us without, 197 with them (moe_gemm_pipe_kernel). Eight values side by side take as
+// long, and a step of Newton for the reciprocal in the remainder's place (one instruction fewer) leaves 0.38, 0.31, 0.5.
 template <typename T>
 __device__ __forceinline__ float silu_times(float g, float u) {
   if constexpr (sizeof(T) == 4) return glu_value(g, u, 0, 0.f, 0.f);
-  const float c = __builtin_amdgcn_fmed3f(g, -88.f, 88.f), t = c * -1.44269504088896341f;
-  const float left = fmaf(t, 1.90465429995776804e-9f, fmaf(t, -0.693147182464599609f, -c));       // -c - t ln 2
-  const float e = __builtin_amdgcn_exp2f(t), d = fmaf(e, left, e) + 1.f, r = __builtin_amdgcn_rcpf(d), q = g * r;
-  return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, q, g), -1.f, 1.f), r, q) * u;      // (the remainder is far below 1, and no number behind an infinite g)
+  return silu_hw(g) * u;
 }
 
 template <typename T, bool GLU, int WN, int WB, int RB, int ST, int PER_CU, bool PLAN>

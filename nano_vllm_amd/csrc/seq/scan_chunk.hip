@@ -26,6 +26,9 @@ namespace {
 // 64 heads of 64 x 128 (form 0) 5,200 -> 650 us, 32 heads of 128 x 128 (form 1) 3,470 -> 700, 8 heads of 128 x 128 (form 2)
 // 1,600 -> 250; one portion of 16,384: 3,650 -> 860, 3,690 -> 900, 1,690 -> 245. Errors against 64 bits, first nine portions,
 // outputs / states: 1.3e-7 / 1.0e-7 -> 1.2e-7 / 0.9e-7, 1.9e-7 / 5.0e-7 -> 1.3e-7 / 3.7e-7, 2.0e-7 / 1.9e-7 -> 1.8e-7 / 1.4e-7.
+// Portions are taken longest first (ragged ones end together: 26 of 100 to 1,024 tokens, form 1 539 -> 414 us, form 0 486 -> 436; nine of 33 to 4,096 735 -> 689, 816 -> 676), and
+// form 1's SiLU, a third of its vector instructions, which no 32-bit matrix instruction runs beside (49 + 51 % of all cycles over 16 portions of 512), is the short one of
+// seq_common.h, with the same errors (nine of 1,100 to 2,048 700 -> 635 us, 32 of 1,000 975 -> 899).
 constexpr int CT = 16;                              // tokens of a chunk
 constexpr int WST = 20;                             // row stride of the 16 x 16 weights in LDS
 constexpr int SB = 4;                               // chunks whose weights are computed together: a token per lane
@@ -52,16 +55,6 @@ __device__ __forceinline__ double row_running_max(double v) {
   v = fmax(v, row_shifted<0x118>(v, v));
   return v;
 }
-// SiLU from the hardware exponential with the part of the exponent that rounding takes, and the reciprocal with one step of Newton
-__device__ __forceinline__ float silu_(float x) {
-  const float L2E = 1.44269504088896341f, L2E_LO = 1.92596299112661746887e-8f, c = fminf(fmaxf(x, -87.f), 87.f);
-  const float e = -c * L2E, lo = fmaf(-c, L2E, -e) - c * L2E_LO;
-  const float t = __builtin_amdgcn_exp2f(e), d = fmaf(t, lo * 0.69314718055994531f, t) + 1.f;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = x < -87.f ? 0.f : fmaf(fmaf(-d, r, 1.f), r, r);          // (not e^-87: x may be large)
-  const float q = x * r;
-  return fabsf(q) < 3e38f ? fmaf(fmaf(-d, q, x), r, q) : q;
-}
 // e^v, with what rounding the exponent to 32 bits leaves
 __device__ __forceinline__ float exp_(double v) {
   const float c = (float)fmax(v, -1e30), e = expf(c);
@@ -83,7 +76,7 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
   __shared__ __attribute__((aligned(16))) float win[2][FORM == 1 ? 1 : SB][2][CT];      // decay from the chunk's start, and what rounding left of it; form 2: exp(-m)
   __shared__ __attribute__((aligned(16))) float nq[FORM == 2 ? 2 : 1][KW][CT];     // form 2: the parts of n . q
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, g = lane >> 4;
-  const int h = blockIdx.x, s = blockIdx.y, seg = blockIdx.z % a.nseg, blk = blockIdx.z / a.nseg;
+  const int h = blockIdx.x, s = MODE == 0 ? portion_by_length(a.cu_q, gridDim.y, blockIdx.y) : blockIdx.y, seg = blockIdx.z % a.nseg, blk = blockIdx.z / a.nseg;
   const int heads = a.heads, P = a.P;
   const int64_t t0 = a.cu_q[s], t1 = a.cu_q[s + 1];
   const int64_t q0 = MODE == 0 ? t0 : t0 + (int64_t)seg * a.seg_len;
@@ -209,7 +202,7 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
           const uint32_t word = raw[u][i * 4 / VE];
           const uint32_t bits = VE == 4 ? word : (i % 2 ? word & 0xffff0000u : word << 16);
           v[i] = __builtin_bit_cast(float, bits);
-          if (FORM == 1) v[i] = silu_(v[i]);
+          if (FORM == 1) v[i] = silu_hw(v[i]);
           if (FORM == 2 && which) v[i] *= a.c_scale;
           if (!in) v[i] = 0.f;
         }
@@ -325,7 +318,7 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       xv[r] = ldf(&xraw[r]);
-      if (FORM == 1) xv[r] = silu_(xv[r]);
+      if (FORM == 1) xv[r] = silu_hw(xv[r]);
       if (tb + 4 * g + r >= q1) xv[r] = 0.f;
       xw[r] = xv[r] * we[r];
     }

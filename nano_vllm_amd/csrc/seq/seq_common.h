@@ -162,8 +162,29 @@ __device__ __forceinline__ RglruTerms rglru_terms(float gr, float gi, float u, f
   return v;
 }
 
+// The portion that is number `rank` by length, longest first (up to 64 portions; beyond, number `rank` as they come): workgroups start in the order of their numbers, so
+// what is left for the end of a launch is short. All lanes of the wavefront call it.
+__device__ __forceinline__ int portion_by_length(const int32_t* __restrict__ cu_q, int nseq, int rank) {
+  if (nseq < 2 || nseq > 64) return rank;
+  const int lane = threadIdx.x & 63, mine = lane < nseq ? cu_q[lane + 1] - cu_q[lane] : -1;
+  int longer = 0;
+  for (int j = 0; j < nseq; ++j) {
+    const int other = __builtin_amdgcn_readlane(mine, j);
+    longer += other > mine || (other == mine && j < lane);
+  }
+  return __builtin_ctzll(__ballot(lane < nseq && longer == rank));
+}
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+// x / (1 + e^-x) with the hardware's exponential and reciprocal: what the rounding of x log2 e took (up to |x| units of 2^-24) is added back, and so is the quotient's
+// remainder (far below 1, and no number behind an infinite x). Within 4 x 2^-24 above -30; 0 below -87
+__device__ __forceinline__ float silu_hw(float x) {
+  const float c = __builtin_amdgcn_fmed3f(x, -88.f, 88.f), t = c * -1.44269504088896341f;
+  const float left = fmaf(t, 1.90465429995776804e-9f, fmaf(t, -0.693147182464599609f, -c));       // -c - t ln 2
+  const float e = __builtin_amdgcn_exp2f(t), d = fmaf(e, left, e) + 1.f, r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, q, x), -1.f, 1.f), r, q);
+}
 __device__ __forceinline__ float siluf_(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float gelu_tanhf_(float z) {
   return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
