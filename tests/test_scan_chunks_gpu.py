@@ -193,8 +193,8 @@ def test_silu_of_large_negative_inputs_is_nothing(where, huge):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("lens", [[17, 0, 17, 33] * 16, [16, 33, 0, 33, 1], [18, 20]], ids=["64", "ties", "two"])
+@pytest.mark.parametrize("lens", [[17, 0, 17, 33] * 16, [16, 0, 33, 33, 1], [18, 20]], ids=["64", "ties", "two"])
 @pytest.mark.parametrize("form,heads,P,N", [(0, 2, 64, 64), (1, 2, 16, 64), (2, 2, 24, 64)])
 def test_portions_that_are_taken_by_length(form, heads, P, N, lens):
-    """The longest first: equal lengths and portions without a token each find their own place."""
+    """The longest first: equal lengths and portions without a token (of sequences that go on: their slots stay as they are) each find their own place."""
     test_chunked_recurrences_against_the_token_loop(form, heads, P, N, 1, lens, torch.bfloat16)
