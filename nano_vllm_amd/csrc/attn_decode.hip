@@ -1600,7 +1600,9 @@ constexpr int kFewPart = NVL_OPEN_PART_TILES, kFewPairs = 64, kFewGroups = 256; 
 inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
   const int64_t pairs = batch * hkv;
   if (batch < 1 || batch > 16 || pairs > (max_context <= 1536 ? 2 * kFewPairs : kFewPairs)) return 0;
-  const int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart, most = (pairs > kFewPairs ? kFewGroups * 3 / 4 : kFewGroups) / pairs;
+  const int64_t most = (pairs > kFewPairs ? kFewGroups * 3 / 4 : kFewGroups) / pairs;
+  int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart;
+  if (nvl_few_fours((int)batch) && parts > 1) parts = (parts + 3) / 4 * 4;     // (up to 3 more; the workspace has two parts for each of them)
   return (int)(parts < most ? parts : most);
 }
 
@@ -1642,7 +1644,7 @@ __device__ __forceinline__ void few_merge(const float* part_o, const float* part
   if (lse != nullptr && d == 0) lse[row] = 0.6931471805599453f * (M + log2f(den));
 }
 
-template <bool SLABS>
+template <bool SLABS, bool FOURS>
 __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
     const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc, const int32_t* __restrict__ block_tables, int64_t bt_stride,
     const int32_t* __restrict__ ctx, float* part_o, float* part_ml, bf16_t* __restrict__ out, int batch, int hkv, int block_size, int slots,
@@ -1653,7 +1655,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, rq = lane >> 4, head = lane & 15, quad = lane >> 4;
   const int pairs = batch * hkv, part = blockIdx.x / pairs, pair = blockIdx.x % pairs, b = pair / hkv, h = pair % hkv, hq = hkv * Gv;
-  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts), per = nvl_few_div(tiles, n);
+  const int len = ctx[b], tiles = (len + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts, FOURS), per = nvl_few_div(tiles, n);
   if (part >= n) return;
   if (len <= 0) {                                  // graph padding: zero rows
     for (int i = threadIdx.x; i < Gv * 128; i += 64 * kFewWaves) out[((int64_t)b * hq + h * Gv) * 128 + i] = (bf16_t)0.f;
@@ -1864,10 +1866,11 @@ __global__ __launch_bounds__(64 * kFewWaves) void decode_few_kernel(
 }
 
 // the contexts of several parts
+template <bool FOURS>
 __global__ __launch_bounds__(128) void decode_few_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                 const int32_t* __restrict__ ctx, bf16_t* __restrict__ out, int hq, int slots, int parts,
                                                                 float* __restrict__ lse) {
-  const int tiles = (ctx[blockIdx.x / hq] + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts);
+  const int tiles = (ctx[blockIdx.x / hq] + kTile - 1) / kTile, n = nvl_few_split(tiles, kFewPart, parts, FOURS);
   if (n > 1) few_merge(part_o, part_ml, blockIdx.x, n, slots, threadIdx.x, out, lse);
 }
 
@@ -2012,7 +2015,7 @@ int launch_decode_mfma8_s(const void* q, void* kc, void* vc, const int32_t* bt, 
   return nvl_check_launch("nvl_paged_attn_decode");
 }
 
-template <bool SLABS>
+template <bool SLABS, bool FOURS>
 int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, int64_t bt_stride, const int32_t* ctx, void* out, int64_t batch,
                       int hkv, int G, int block_size, int64_t max_context, float scale, void* workspace, hipStream_t s, const FusedArgs& fa, float* lse, int parts) {
   constexpr int lds = kFewWaves * (kFewTile + 16 * 8) + 18 * 256;
@@ -2024,17 +2027,17 @@ int launch_decode_few(const void* qkv, void* kc, void* vc, const int32_t* bt, in
   static bool attr_done[NVL_MAX_DEVICES] = {};
   bool& attr_set = attr_done[nvl_device_slot()];
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_few_kernel<SLABS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_few_kernel<SLABS, FOURS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
       nvl_set_error("nvl_paged_attn_decode: cannot reserve LDS for the kernel of few sequences");
       return NVL_ELAUNCH;
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((decode_few_kernel<SLABS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
+  hipLaunchKernelGGL((decode_few_kernel<SLABS, FOURS>), dim3((unsigned)(batch * hkv * parts)), dim3(64 * kFewWaves), lds, s, (const bf16_t*)qkv, (bf16_t*)kc,
                      (bf16_t*)vc, bt, bt_stride, ctx, part_o, part_ml, (bf16_t*)out, (int)batch, hkv, block_size, slots, scale * 1.4426950408889634f, fa,
                      G, parts, lse);
   if (!open && parts > 1)
-    hipLaunchKernelGGL(decode_few_merge_kernel, dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
+    hipLaunchKernelGGL((decode_few_merge_kernel<FOURS>), dim3((unsigned)(batch * hq)), dim3(128), 0, s, part_o, part_ml, ctx, (bf16_t*)out, hq, slots, parts, lse);
   return nvl_check_launch("nvl_paged_attn_decode");
 }
 
@@ -2214,11 +2217,11 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
     return NVL_EUNSUPPORTED;
   }
   const int few = open ? open_parts(batch, num_kv_heads, max_context) : fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
-  if (few)
-    return fa->qkv_splits > 0 ? launch_decode_few<true>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
-                                                        max_context, softmax_scale, workspace, s, *fa, lse, few)
-                              : launch_decode_few<false>(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size,
-                                                         max_context, softmax_scale, workspace, s, *fa, lse, few);
+  if (few) {
+    const bool slabs = fa->qkv_splits > 0, fours = nvl_few_fours((int)batch);
+    const auto launch = slabs ? fours ? launch_decode_few<true, true> : launch_decode_few<true, false> : fours ? launch_decode_few<false, true> : launch_decode_few<false, false>;
+    return launch(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size, max_context, softmax_scale, workspace, s, *fa, lse, few);
+  }
   if (kv_dtype == NVL_KV_FP8) {
 #define NVL_DECODE8_CASE(GG)                                                                                           \
   case GG:                                                                                                             \

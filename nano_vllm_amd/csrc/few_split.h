@@ -19,11 +19,20 @@ NVL_FEW_FN int nvl_few_div(int a, int b) {
 #endif
 }
 
-// Parts of a context of `tiles` tiles: part_tiles tiles each, more where `parts` do not suffice. Part p takes tiles [p per, p per + per) with per = ceil(tiles / n):
-// none is empty, so the part that ends with the last tile, which brings the new token, is one. (Of `parts` parts themselves the last ones may be empty: 129 tiles
-// in 16 are 15 of 9.)
-NVL_FEW_FN int nvl_few_split(int tiles, int part_tiles, int parts) {
+// Steps of up to four sequences, whose parts the output projection merges, take them in fours, as it asks for them: a second part costs it as much as a fourth, and the
+// parts' tiles come in on more compute units (28 bytes a clock each). Decode steps of Qwen3-0.6B in us, parts of eight tiles / fours: one sequence, contexts of 300, 400, 700,
+// 1,200, 1,600 and 2,000 tokens 806 813 823 850 853 852 / 791 803 811 829 846 854; two of 400, 700, 1,200, 2,000 832 843 866 873 / 818 829 850 875; three of up to 600, 1,000,
+// 1,500, 2,000 876 884 910 922 / 836 859 888 905; four of up to 300, 600, 1,000, 1,500, 2,000 894 897 882 922 961 / 900 858 878 924 948 (the one loss: four that
+// two parts each would do for). More sequences merge in a launch of their own and stay as they were (fours for six of 600 964 / 953, eight of 1,200 1056 / 1061).
+NVL_FEW_FN bool nvl_few_fours(int sequences) { return sequences <= 4; }
+
+// Parts of a context of `tiles` tiles: part_tiles tiles each, more where `parts` do not suffice, fewer where that makes whole `fours`. Part p takes tiles [p per, p per + per) with
+// per = ceil(tiles / n): none is empty, so the part that ends with the last tile, which brings the new token, is one. (Of `parts` parts themselves the last ones may be
+// empty: 129 tiles in 16 are 15 of 9.) A single part is told first: the shortest contexts pay for no division.
+NVL_FEW_FN int nvl_few_split(int tiles, int part_tiles, int parts, bool fours = false) {
   const int n = (tiles + part_tiles - 1) / part_tiles;
-  if (n <= parts) return n < 1 ? 1 : n;
-  return nvl_few_div(tiles, nvl_few_div(tiles, parts));
+  if (n <= 1) return 1;
+  const int up = fours ? 3 : 0, more = (n + up) & ~up;
+  if (more == n && n <= parts) return n;
+  return nvl_few_div(tiles, nvl_few_div(tiles, more < parts ? more : parts));
 }

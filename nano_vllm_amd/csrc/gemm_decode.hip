@@ -184,7 +184,7 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
               pb[j] = *reinterpret_cast<const f32x4_t*>(po + k * 128 + 4);
             }
           };
-          const int n = nvl_few_split((len[i] + 31) / 32, NVL_OPEN_PART_TILES, oa.parts);
+          const int n = nvl_few_split((len[i] + 31) / 32, NVL_OPEN_PART_TILES, oa.parts, nvl_few_fours(M));
           dst[i] = one[i];
           if (n == 1) continue;
           ask(0, n - 1);

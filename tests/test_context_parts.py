@@ -45,3 +45,27 @@ def test_every_tile_and_the_new_token_belong_to_one_part(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
     run = subprocess.run([str(exe)], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_parts_in_fours(tmp_path):
+    """With `fours` the same holds; a context of several parts never has fewer than without, a number that `parts` allows is whole fours unless the last ones would be
+    empty, and one of a single part stays so."""
+    source = SOURCE.replace("nvl_few_split(tiles, part_tiles, parts), per", "nvl_few_split(tiles, part_tiles, parts, true), plain = nvl_few_split(tiles, part_tiles, parts), per")
+    source = source.replace("if (n < 1 ||", "if (n < plain) empty += 1; if ((plain == 1) != (n == 1)) empty += 1; if (n > 1 && n % 4 && (n + 3) / 4 * 4 <= parts && "
+                            "(tiles + (n + 3) / 4 * 4 - 1) / ((n + 3) / 4 * 4) != per) empty += 1;\n        if (n < 1 ||")
+    assert source.count(", true)") == 1 and source.count("plain") == 3
+    src, exe = tmp_path / "fours.cpp", tmp_path / "fours"
+    src.write_text(source)
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0, run.stdout
+
+
+def test_open_parts_have_room():
+    """The parts of a step (their results, two numbers each) and the single parts' rows lie in the step's workspace, whatever its longest context."""
+    from nano_vllm_amd import ops
+    for b in (1, 2, 3, 4):
+        for longest in list(range(1, 2100)) + [4096, 4097, 8192, 16383, 16384]:
+            parts = ops.open_parts(b, 8, longest)
+            assert parts >= 1 and b * 16 * (parts * 130 * 4 + 128 * 2) <= ops.paged_attn_decode_workspace_bytes(b, 16, longest), (b, longest, parts)
