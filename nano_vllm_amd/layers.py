@@ -338,13 +338,15 @@ class LinearBase(nn.Module):
         raise NotImplementedError
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if self.bias is None and _decode_sized(x):
-            y = decode_linear(x, self.weight, ops.LINEAR_BF16, packed=self.weight_packed)
+        # (parameters are looked up once, and rows asked first: steps of few prompts wait for the host)
+        w, b, rows = self.weight, self.bias, x.shape[0]
+        if b is None and rows <= DECODE_LINEAR_MAX_ROWS and _decode_sized(x):
+            y = decode_linear(x, w, ops.LINEAR_BF16, packed=self.weight_packed)
             if y is not None:
                 return y
-        if x.shape[0] >= ops_seq.TILES_FROM and ops_seq.loaded() and ops_seq.many_rows(x, self.weight, self.bias):
-            return ops_seq.linear_tiles(x, self.weight, self.bias)
-        return F.linear(x, self.weight, self.bias)
+        if rows >= ops_seq.TILES_FROM and ops_seq.loaded() and ops_seq.many_rows(x, w, b):
+            return ops_seq.linear_tiles(x, w, b)
+        return F.linear(x, w, b)
 
 
 # Row counts up to this use the hand-written decode GEMMs (nvl_linear_decode / nvl_linear_wide); above it the
@@ -511,14 +513,15 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
         epilogue (one launch, no [N, 2*inter] round trip), on many rows that of the pipelined tiles where
         those are the faster ones and their library is loaded."""
         pair = self.bias is None and len(self.output_sizes) == 2 and self.output_sizes[0] == self.output_sizes[1]
+        w = self.weight
         if pair and _decode_sized(x):
-            y = decode_linear(x, self.weight, ops.LINEAR_SILU, packed=self.weight_packed)
+            y = decode_linear(x, w, ops.LINEAR_SILU, packed=self.weight_packed)
             if y is not None:
                 return y
-        if pair and ops_seq.loaded() and ops_seq.silu_linear_fits(x, self.weight):
-            tm = ops_seq.silu_linear_rows(x.shape[0], self.weight.shape[0] // 2, x.shape[1])
+        if pair and ops_seq.loaded() and ops_seq.silu_linear_fits(x, w):
+            tm = ops_seq.silu_linear_rows(x.shape[0], w.shape[0] // 2, x.shape[1])
             if tm:
-                return ops_seq.silu_linear(x, self.weight, tm)
+                return ops_seq.silu_linear(x, w, tm)
         return ops.silu_mul(self.forward(x))
 
 
