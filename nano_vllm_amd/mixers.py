@@ -38,8 +38,8 @@
                       pass-through experts, biased logits, optional shared expert with a sigmoid gate per token; or, instead of a router, a
                       table from token ids to experts with equal weights
 
-Every constant a design may change is a constructor argument. Matrix products of many rows are the vendor library's
-(F.linear / baddbmm); those of few rows (ops_seq.linear) and everything else are kernels of libnvl_seq.so (ops_seq). Layers read the step's packed-portion description from
+Every constant a design may change is a constructor argument. Matrix products of few rows and of many are kernels of
+libnvl_seq.so (ops_seq.linear), those between the vendor library's (F.linear / baddbmm); everything else is a kernel of libnvl_seq.so. Layers read the step's packed-portion description from
 the attention-metadata context (`portions`, `slot_mapping`, `block_tables`); the runner injects the per-layer cache and
 state tensors named by `kv_shapes()` / `state_shapes()`.
 
