@@ -682,11 +682,10 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, glu: bool) -> bool:
     24576 x 4096 54.8 / 47.9; 256 rows, 1024 x 1024 4.2 / 8.3, 4096 x 4096 19.5 / 22.2, 6144 x 1024 12.8 / 12.3; 128 rows of it 7.5 / 9.5; 16 rows,
     12288 x 2048 11.7 / 11.6, 32768 x 4096 57.9 / 60.3 (its 268 MB out of memory). The activation on the way saves its launch (4 us and its passes): more is taken. 32-bit: 330 rows,
     1024 x 1024 10.3 / 11.8, 4096 x 1024 33.6 / 41.3, 3084 x 1024 30.9 / 23.8; 512 rows, 1024 x 2048 21.3 / 21.5, 4096 x 1024 42.9 / 36.2."""
-    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+    if x.dim() != 2 or w.dim() != 2:
         return False
-    m, k = x.shape
-    n = w.shape[0]
-    if n == 0 or k == 0 or x.stride(0) < k or x.device != w.device:          # (rows that share entries too: nvs_linear_rows refuses them)
+    (m, k), (n, wide) = x.shape, w.shape
+    if wide != k or n == 0 or k == 0 or x.stride(0) < k or x.device != w.device:          # (rows that share entries too: nvs_linear_rows refuses them)
         return False
     if w.dtype == torch.bfloat16:
         if k % 64 or x.stride(0) % 8 or not (m <= 16 or m <= 256 and n <= 4096 or m <= 128 and n <= 6144 or
