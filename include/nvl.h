@@ -312,17 +312,26 @@ int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride,
  * workspace receives [batch][Hq][parts][128] 32-bit numerators, [batch][Hq][parts][2] maximum (base 2) and sum, and [batch][Hq][128] bf16. parts =
  * nvl_paged_attn_decode_open_parts (0: the step is too large); a context of t = ceil(tokens / 32) tiles
  * has n = max(1, ceil(t / 8)) of them where that is at most parts, else ceil(t / ceil(t / parts)), of ceil(t / n) tiles each and the last of what is left (never none). A
- * context of a single part is finished, as bf16; an empty one's row is zero. */
+ * context of a single part is finished, as bf16; an empty one's row is zero.
+ * nvl_paged_attn_decode_open_fours: the same, but contexts of several parts take them in fours. parts = nvl_paged_attn_decode_open_fours_parts; a context whose n = ceil(t / 8)
+ * is 1 or less has one part; of the others, with r the multiple of 4 from n on, one where r = n <= parts has n, any other ceil(t / ceil(t / min(r, parts))). */
 int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context);
+int nvl_paged_attn_decode_open_fours_parts(int64_t batch, int num_kv_heads, int64_t max_context);
 int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
                                int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables, int64_t bt_stride, const int32_t* context_lens,
                                int64_t batch, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int64_t max_context,
                                float softmax_scale, void* workspace, size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream);
+int nvl_paged_attn_decode_open_fours(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps, const float* cos_sin,
+                                     int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables, int64_t bt_stride, const int32_t* context_lens,
+                                     int64_t batch, int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks, int64_t max_context,
+                                     float softmax_scale, void* workspace, size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream);
 /* nvl_linear_decode mode 2 of the merge of those parts, rounded to bf16: m <= 16 rows of k = Hq * 128 entries. nvl_linear_decode_open_splits: the K-slices it
- * emits, 0 where it does not take the shape (ask before the attention leaves its parts open). */
+ * emits, 0 where it does not take the shape (ask before the attention leaves its parts open). nvl_linear_decode_open_fours: of parts in fours. */
 int nvl_linear_decode_open_splits(int64_t m, int n, int k);
 int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight, void* out,
                            int64_t m, int n, int k, int weight_layout, void* stream);
+int nvl_linear_decode_open_fours(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight, void* out,
+                                 int64_t m, int n, int k, int weight_layout, void* stream);
 
 /* ---- Varlen causal prefill attention (MFMA) ----------------------------------
  * Replaces flash_attn_varlen_func as called at layers/attention.py:67-70:

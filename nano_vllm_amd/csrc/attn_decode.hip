@@ -1597,21 +1597,21 @@ constexpr int kFewPart = NVL_OPEN_PART_TILES, kFewPairs = 64, kFewGroups = 256; 
 // 1161 1203 1357 1502. Twelve and 16 gain up to 1,500 (12: 1098 1092 1120 1162 1327 / 925 1064 1106 1171 1272; 16: 1101 1115 1130 1229 1379 / 904 1015 1101 1220 1368) and lose from
 // 2,000 on (16: 1464 1731 2001 / 1519 1847 2153), so they come here where contexts stay short. Not more workgroups than run at once (of 16 sequences 192: one part each and not two,
 // 949 1101 1155 1223 1369): parts of 1,024 tokens, as many as there are, took 1,161 us for eight of 1,000 and 1,794 for 12 of 3,000.
-inline int few_parts(int64_t batch, int hkv, int64_t max_context) {
+inline int few_parts(int64_t batch, int hkv, int64_t max_context, bool fours) {
   const int64_t pairs = batch * hkv;
   if (batch < 1 || batch > 16 || pairs > (max_context <= 1536 ? 2 * kFewPairs : kFewPairs)) return 0;
   const int64_t most = (pairs > kFewPairs ? kFewGroups * 3 / 4 : kFewGroups) / pairs;
   int64_t parts = ((max_context + kTile - 1) / kTile + kFewPart - 1) / kFewPart;
-  if (nvl_few_fours((int)batch) && parts > 1) parts = (parts + 3) / 4 * 4;     // (up to 3 more; the workspace has two parts for each of them)
+  if (fours && parts > 1) parts = (parts + 3) / 4 * 4;     // (up to 3 more; the workspace has two parts for each of them)
   return (int)(parts < most ? parts : most);
 }
 
 // Left open for the output projection to merge (nvl_linear_decode_open): up to eight parts, since the projection takes longer with more (4,000 tokens in 16: 7.4 + 6.6 us, in
 // eight 8.6 + 5.2), 16 where contexts may pass 4,096 tokens (12,000 in eight: 25.2).
 constexpr int kOpenParts = 16, kOpenRows = 4;
-inline int open_parts(int64_t batch, int hkv, int64_t max_context) {
+inline int open_parts(int64_t batch, int hkv, int64_t max_context, bool fours) {
   if (batch > kOpenRows || max_context > 16384) return 0;
-  const int parts = few_parts(batch, hkv, max_context), most = max_context <= 4096 ? kOpenParts / 2 : kOpenParts;
+  const int parts = few_parts(batch, hkv, max_context, fours), most = max_context <= 4096 ? kOpenParts / 2 : kOpenParts;
   return parts < most ? parts : most;
 }
 
@@ -2176,7 +2176,7 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
                   const int32_t* context_lens, void* out, int64_t batch, int num_q_heads, int num_kv_heads,
                   int block_size, int64_t num_blocks, int64_t max_context, float softmax_scale, void* workspace,
                   size_t workspace_bytes, void* stream, const FusedArgs* fa, const char* who, int kv_dtype,
-                  const void* plan, float* lse, bool open = false) {
+                  const void* plan, float* lse, bool open = false, bool fours = false) {
   NVL_REQUIRE(q && k_cache && v_cache && block_tables && context_lens && (out || open) && workspace, "%s: null pointer", who);
   NVL_REQUIRE(kv_dtype == NVL_KV_BF16 || kv_dtype == NVL_KV_FP8, "%s: kv_dtype=%d (0 bf16, 1 fp8 e4m3)", who, kv_dtype);
   NVL_REQUIRE(batch >= 0 && batch <= 32768, "%s: batch=%lld out of range [0, 32768]", who, (long long)batch);
@@ -2212,13 +2212,13 @@ int decode_common(const void* q, void* k_cache, void* v_cache, const int32_t* bl
     NVL_REQUIRE(mfma, "%s: a plan with a shared prefix needs the matrix-core kernel (Hq/Hkv in 2 ... 16; got %d)", who, G);
     NVL_REQUIRE(block_size % 128 == 0, "%s: a shared prefix needs block_size %% 128 == 0 (got %d)", who, block_size);
   }
-  if (open && !(fa && mfma && kv_dtype == NVL_KV_BF16 && open_parts(batch, num_kv_heads, max_context))) {
+  if (open && !(fa && mfma && kv_dtype == NVL_KV_BF16 && open_parts(batch, num_kv_heads, max_context, fours))) {
     nvl_set_error("%s: only steps of up to 4 sequences and contexts of up to 16,384 tokens, bf16 caches and the matrix-core kernel's group sizes leave their parts open", who);
     return NVL_EUNSUPPORTED;
   }
-  const int few = open ? open_parts(batch, num_kv_heads, max_context) : fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context) : 0;
+  const int few = open ? open_parts(batch, num_kv_heads, max_context, fours) : fa && mfma && kv_dtype == NVL_KV_BF16 && !(plan != nullptr && plan_shadow_prefix(plan)) ? few_parts(batch, num_kv_heads, max_context, fours) : 0;
   if (few) {
-    const bool slabs = fa->qkv_splits > 0, fours = nvl_few_fours((int)batch);
+    const bool slabs = fa->qkv_splits > 0;
     const auto launch = slabs ? fours ? launch_decode_few<true, true> : launch_decode_few<true, false> : fours ? launch_decode_few<false, true> : launch_decode_few<false, false>;
     return launch(q, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_kv_heads, G, block_size, max_context, softmax_scale, workspace, s, *fa, lse, few);
   }
@@ -2340,7 +2340,7 @@ static int decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_n
                                            int num_q_heads, int num_kv_heads, int block_size, int64_t num_blocks,
                                            int64_t max_context, float softmax_scale, void* workspace,
                                            size_t workspace_bytes, int kv_dtype, const void* plan, float* lse,
-                                           int qkv_splits, int64_t qkv_split_stride, void* stream, const char* who, bool open) {
+                                           int qkv_splits, int64_t qkv_split_stride, void* stream, const char* who, bool open, bool fours) {
   NVL_REQUIRE(qkv_splits >= 0 && qkv_splits <= 8, "%s: qkv_splits=%d (0 = bf16 qkv, 1..8 = fp32 split-K slabs)", who, qkv_splits);
   NVL_REQUIRE(qkv_splits <= 1 || qkv_split_stride >= batch * qkv_tok_stride, "%s: qkv_split_stride=%lld < batch x qkv_tok_stride",
               who, (long long)qkv_split_stride);
@@ -2361,7 +2361,7 @@ static int decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_n
   fa.qkv_split_stride = (int)qkv_split_stride;
   return decode_common(qkv, k_cache, v_cache, block_tables, bt_stride, context_lens, out, batch, num_q_heads,
                        num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes,
-                       stream, &fa, who, kv_dtype, plan, lse, open);
+                       stream, &fa, who, kv_dtype, plan, lse, open, fours);
 }
 extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,
                                            const float* cos_sin, int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables,
@@ -2371,11 +2371,14 @@ extern "C" int nvl_paged_attn_decode_fused(const void* qkv, int64_t qkv_tok_stri
                                            int64_t qkv_split_stride, void* stream) {
   return decode_fused(qkv, qkv_tok_stride, q_norm_w, k_norm_w, eps, cos_sin, max_pos, k_cache, v_cache, block_tables, bt_stride, context_lens, out,
                       batch, num_q_heads, num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes, kv_dtype, plan,
-                      lse, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_fused", false);
+                      lse, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_fused", false, nvl_few_fours((int)batch));
 }
 extern "C" int nvl_paged_attn_decode_open_parts(int64_t batch, int num_kv_heads, int64_t max_context) {
   static_assert(kTile == 32 && kFewPart == kFewWaves, "the projection counts the parts too");
-  return num_kv_heads > 0 && max_context > 0 ? open_parts(batch, num_kv_heads, max_context) : 0;
+  return num_kv_heads > 0 && max_context > 0 ? open_parts(batch, num_kv_heads, max_context, false) : 0;
+}
+extern "C" int nvl_paged_attn_decode_open_fours_parts(int64_t batch, int num_kv_heads, int64_t max_context) {
+  return num_kv_heads > 0 && max_context > 0 ? open_parts(batch, num_kv_heads, max_context, true) : 0;
 }
 extern "C" int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,
                                           const float* cos_sin, int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables,
@@ -2384,7 +2387,16 @@ extern "C" int nvl_paged_attn_decode_open(const void* qkv, int64_t qkv_tok_strid
                                           size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream) {
   return decode_fused(qkv, qkv_tok_stride, q_norm_w, k_norm_w, eps, cos_sin, max_pos, k_cache, v_cache, block_tables, bt_stride, context_lens, nullptr,
                       batch, num_q_heads, num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes, NVL_KV_BF16, nullptr,
-                      nullptr, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_open", true);
+                      nullptr, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_open", true, false);
+}
+extern "C" int nvl_paged_attn_decode_open_fours(const void* qkv, int64_t qkv_tok_stride, const void* q_norm_w, const void* k_norm_w, float eps,
+                                                const float* cos_sin, int64_t max_pos, void* k_cache, void* v_cache, const int32_t* block_tables,
+                                                int64_t bt_stride, const int32_t* context_lens, int64_t batch, int num_q_heads, int num_kv_heads,
+                                                int block_size, int64_t num_blocks, int64_t max_context, float softmax_scale, void* workspace,
+                                                size_t workspace_bytes, int qkv_splits, int64_t qkv_split_stride, void* stream) {
+  return decode_fused(qkv, qkv_tok_stride, q_norm_w, k_norm_w, eps, cos_sin, max_pos, k_cache, v_cache, block_tables, bt_stride, context_lens, nullptr,
+                      batch, num_q_heads, num_kv_heads, block_size, num_blocks, max_context, softmax_scale, workspace, workspace_bytes, NVL_KV_BF16, nullptr,
+                      nullptr, qkv_splits, qkv_split_stride, stream, "nvl_paged_attn_decode_open_fours", true, true);
 }
 
 // ---- per-step plan ------------------------------------------------------------------------------------------------

@@ -59,6 +59,7 @@ struct OpenAttn {
   const bf16_t* whole;             // [m][head][128]: contexts of one part, finished
   const int32_t* ctx;
   int parts;
+  bool fours;                      // parts as nvl_paged_attn_decode_open_fours leaves them
 };
 
 template <int MT, int KB, int NT, int EPI, bool OPEN>
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(kNW * 64) void linear_decode_kernel(const bf16_t* _
               pb[j] = *reinterpret_cast<const f32x4_t*>(po + k * 128 + 4);
             }
           };
-          const int n = nvl_few_split((len[i] + 31) / 32, NVL_OPEN_PART_TILES, oa.parts, nvl_few_fours(M));
+          const int n = nvl_few_split((len[i] + 31) / 32, NVL_OPEN_PART_TILES, oa.parts, oa.fours);
           dst[i] = one[i];
           if (n == 1) continue;
           ask(0, n - 1);
@@ -592,19 +593,19 @@ extern "C" int nvl_linear_decode_open_splits(int64_t m, int n, int k) {
   return open_plan(m, n, k, &p) ? p.split : 0;
 }
 
-extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight,
-                                      void* out, int64_t m, int n, int k, int weight_layout, void* stream) {
-  NVL_REQUIRE(parts_o && parts_ml && whole && context_lens && weight && out, "nvl_linear_decode_open: null pointer");
-  NVL_REQUIRE(m >= 1 && m <= 16 && parts >= 1 && k % 128 == 0, "nvl_linear_decode_open: m=%lld k=%d parts=%d", (long long)m, k, parts);
-  NVL_REQUIRE(weight_layout == 0 || weight_layout == 1, "nvl_linear_decode_open: weight_layout=%d", weight_layout);
-  NVL_REQUIRE(((uintptr_t)parts_o | (uintptr_t)whole | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 && (uintptr_t)parts_ml % 8 == 0, "nvl_linear_decode_open: alignment");
+static int linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, bool fours, const void* weight,
+                              void* out, int64_t m, int n, int k, int weight_layout, void* stream, const char* who) {
+  NVL_REQUIRE(parts_o && parts_ml && whole && context_lens && weight && out, "%s: null pointer", who);
+  NVL_REQUIRE(m >= 1 && m <= 16 && parts >= 1 && k % 128 == 0, "%s: m=%lld k=%d parts=%d", who, (long long)m, k, parts);
+  NVL_REQUIRE(weight_layout == 0 || weight_layout == 1, "%s: weight_layout=%d", who, weight_layout);
+  NVL_REQUIRE(((uintptr_t)parts_o | (uintptr_t)whole | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 && (uintptr_t)parts_ml % 8 == 0, "%s: alignment", who);
   Plan p;
   if (!open_plan(m, n, k, &p)) {
-    nvl_set_error("nvl_linear_decode_open: shape m=%lld n=%d k=%d not covered", (long long)m, n, k);
+    nvl_set_error("%s: shape m=%lld n=%d k=%d not covered", who, (long long)m, n, k);
     return NVL_EUNSUPPORTED;
   }
   g_packed = weight_layout;
-  const OpenAttn oa = {parts_o, parts_ml, (const bf16_t*)whole, context_lens, parts};
+  const OpenAttn oa = {parts_o, parts_ml, (const bf16_t*)whole, context_lens, parts, fours};
   hipStream_t s = (hipStream_t)stream;
   switch (p.kb) {
     case 1: return launch<1, 1, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
@@ -612,6 +613,14 @@ extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_m
     case 3: return launch<1, 3, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
     default: return launch<1, 4, 1, EPI_PARTIAL, true>(nullptr, weight, out, m, n, k, p, s, oa);
   }
+}
+extern "C" int nvl_linear_decode_open(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight,
+                                      void* out, int64_t m, int n, int k, int weight_layout, void* stream) {
+  return linear_decode_open(parts_o, parts_ml, whole, context_lens, parts, false, weight, out, m, n, k, weight_layout, stream, "nvl_linear_decode_open");
+}
+extern "C" int nvl_linear_decode_open_fours(const float* parts_o, const float* parts_ml, const void* whole, const int32_t* context_lens, int parts, const void* weight,
+                                            void* out, int64_t m, int n, int k, int weight_layout, void* stream) {
+  return linear_decode_open(parts_o, parts_ml, whole, context_lens, parts, true, weight, out, m, n, k, weight_layout, stream, "nvl_linear_decode_open_fours");
 }
 
 extern "C" int nvl_add_rmsnorm_splitk(const float* partials, int splits, void* residual, const void* weight, void* y,

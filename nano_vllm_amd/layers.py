@@ -162,13 +162,13 @@ class Attention(nn.Module):
             return None
         b, (n, k) = qkv.shape[0], o_proj.weight.shape
         max_context = ctx.max_context or ctx.block_tables.shape[1] * self.k_cache.shape[2]
-        if not ops.linear_decode_open_splits(b, n, k) or not ops.open_parts(b, self.num_kv_heads, max_context):
+        if not ops.linear_decode_open_splits(b, n, k) or not ops.open_parts(b, self.num_kv_heads, max_context, True):
             return None
         ws = ctx.decode_workspace
         if ws is None:
             ws = torch.empty(ops.paged_attn_decode_workspace_bytes(b, self.num_heads, max_context), dtype=torch.uint8, device=qkv.device)
         att = ops.paged_attn_decode_open(qkv, q_norm_w, k_norm_w, eps, rope_table, self.k_cache, self.v_cache, ctx.block_tables, ctx.context_lens,
-                                         self.num_heads, self.scale, max_context, ws)
+                                         self.num_heads, self.scale, max_context, ws, fours=True)
         w = o_proj.weight_packed
         return ops.linear_decode_open(att, w if w is not None else o_proj.weight, packed=w is not None)
 

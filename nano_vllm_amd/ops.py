@@ -50,10 +50,14 @@ SIGNATURES = {
     "nvl_decode_plan_bytes": (c_size_t, []),
     "nvl_decode_plan": (c_int, [c_void_p, c_int64, c_int, c_int, c_int64, c_void_p, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "nvl_paged_attn_decode_open_parts": (c_int, [c_int64, c_int, c_int64]),
+    "nvl_paged_attn_decode_open_fours_parts": (c_int, [c_int64, c_int, c_int64]),
     "nvl_paged_attn_decode_open": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                            c_int64, c_int, c_int, c_int, c_int64, c_int64, c_float, c_void_p, c_size_t, c_int, c_int64, c_void_p]),
+    "nvl_paged_attn_decode_open_fours": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
+                                                 c_int64, c_int, c_int, c_int, c_int64, c_int64, c_float, c_void_p, c_size_t, c_int, c_int64, c_void_p]),
     "nvl_linear_decode_open_splits": (c_int, [c_int64, c_int, c_int]),
     "nvl_linear_decode_open": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
+    "nvl_linear_decode_open_fours": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "nvl_paged_attn_decode_fused": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p,
                                             c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int,
                                             c_int, c_int64, c_int64, c_float, c_void_p, c_size_t, c_int, c_void_p,
@@ -461,41 +465,42 @@ def paged_attn_decode_fused(qkv: torch.Tensor, q_norm_w, k_norm_w, eps: float, c
 class OpenAttention:
     """A decode step's attention whose contexts are still in parts: what `linear_decode_open` merges. The parts live in the step's workspace, up to the next launch
     that uses it."""
-    __slots__ = ("workspace", "context_lens", "rows", "heads", "parts")
+    __slots__ = ("workspace", "context_lens", "rows", "heads", "parts", "fours")
 
-    def __init__(self, workspace, context_lens, rows, heads, parts):
-        self.workspace, self.context_lens, self.rows, self.heads, self.parts = workspace, context_lens, rows, heads, parts
+    def __init__(self, workspace, context_lens, rows, heads, parts, fours=False):
+        self.workspace, self.context_lens, self.rows, self.heads, self.parts, self.fours = workspace, context_lens, rows, heads, parts, fours
 
 
 _open_cache: dict[tuple, int] = {}
 _open_splits_cache: dict[tuple, int] = {}
 
 
-def open_parts(b: int, num_kv_heads: int, max_context: int) -> int:
+def open_parts(b: int, num_kv_heads: int, max_context: int, fours: bool = False) -> int:
     """Parts of paged_attn_decode_open; 0: the step is too large for it."""
-    key = (b, num_kv_heads, max_context)
+    key = (b, num_kv_heads, max_context, fours)
     r = _open_cache.get(key)
     if r is None:
-        r = _open_cache[key] = lib().nvl_paged_attn_decode_open_parts(b, num_kv_heads, max_context)
+        ask = lib().nvl_paged_attn_decode_open_fours_parts if fours else lib().nvl_paged_attn_decode_open_parts
+        r = _open_cache[key] = ask(b, num_kv_heads, max_context)
     return r
 
 
 def paged_attn_decode_open(qkv: torch.Tensor, q_norm_w, k_norm_w, eps: float, cos_sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                            block_tables: torch.Tensor, context_lens: torch.Tensor, num_q_heads: int, scale: float, max_context: int,
-                           workspace: torch.Tensor) -> OpenAttention:
-    """paged_attn_decode_fused of up to 4 sequences (bf16 qkv and cache, no shared prefix) without the merge of a context's parts."""
+                           workspace: torch.Tensor, fours: bool = False) -> OpenAttention:
+    """paged_attn_decode_fused of up to 4 sequences (bf16 qkv and cache, no shared prefix) without the merge of a context's parts; `fours`: in fours where it has several."""
     _dev(qkv, "qkv")
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16
     assert block_tables.dtype == torch.int32 and context_lens.dtype == torch.int32 and block_tables.stride(1) == 1
     assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous()
     b = qkv.shape[0]
-    parts = open_parts(b, k_cache.shape[1], max_context)
-    _check(lib().nvl_paged_attn_decode_open(
+    parts = open_parts(b, k_cache.shape[1], max_context, fours)
+    _check((lib().nvl_paged_attn_decode_open_fours if fours else lib().nvl_paged_attn_decode_open)(
         qkv.data_ptr(), qkv.stride(0), q_norm_w.data_ptr() if q_norm_w is not None else None, k_norm_w.data_ptr() if k_norm_w is not None else None, eps,
         cos_sin.data_ptr(), cos_sin.shape[0], k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), block_tables.stride(0),
         context_lens.data_ptr(), b, num_q_heads, k_cache.shape[1], k_cache.shape[2], k_cache.shape[0], max_context, scale, workspace.data_ptr(),
         workspace.numel() * workspace.element_size(), 0, 0, _stream()))
-    return OpenAttention(workspace, context_lens, b, num_q_heads, parts)
+    return OpenAttention(workspace, context_lens, b, num_q_heads, parts, fours)
 
 
 def linear_decode_open_splits(m: int, n: int, k: int) -> int:
@@ -514,8 +519,9 @@ def linear_decode_open(att: OpenAttention, weight: torch.Tensor, packed: bool = 
     out = torch.empty((linear_decode_open_splits(att.rows, n, k), att.rows, n), dtype=torch.float32, device=weight.device)
     o = att.workspace.data_ptr()
     ml = o + att.rows * att.heads * att.parts * 512
-    _check(lib().nvl_linear_decode_open(o, ml, ml + att.rows * att.heads * att.parts * 8, att.context_lens.data_ptr(), att.parts, weight.data_ptr(),
-                                        out.data_ptr(), att.rows, n, k, 1 if packed else 0, _stream()))
+    merge = lib().nvl_linear_decode_open_fours if att.fours else lib().nvl_linear_decode_open
+    _check(merge(o, ml, ml + att.rows * att.heads * att.parts * 8, att.context_lens.data_ptr(), att.parts, weight.data_ptr(), out.data_ptr(), att.rows, n, k,
+                 1 if packed else 0, _stream()))
     return out
 
 

@@ -65,7 +65,30 @@ def test_parts_in_fours(tmp_path):
 def test_open_parts_have_room():
     """The parts of a step (their results, two numbers each) and the single parts' rows lie in the step's workspace, whatever its longest context."""
     from nano_vllm_amd import ops
-    for b in (1, 2, 3, 4):
-        for longest in list(range(1, 2100)) + [4096, 4097, 8192, 16383, 16384]:
-            parts = ops.open_parts(b, 8, longest)
-            assert parts >= 1 and b * 16 * (parts * 130 * 4 + 128 * 2) <= ops.paged_attn_decode_workspace_bytes(b, 16, longest), (b, longest, parts)
+    for hkv, hq in ((8, 16), (1, 16), (2, 4), (4, 20), (8, 24), (16, 32)):
+        for b in (1, 2, 3, 4):
+            for longest in list(range(1, 2100, 1 if hkv == 8 else 7)) + [4096, 4097, 8192, 16383, 16384]:
+                room = ops.paged_attn_decode_workspace_bytes(b, hq, longest)
+                for fours in (False, True):
+                    parts = ops.open_parts(b, hkv, longest, fours)
+                    assert parts >= 1 and b * hq * (parts * 130 * 4 + 128 * 2) <= room, (hkv, hq, b, longest, fours, parts)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_the_split_is_the_documented_one(tmp_path):
+    """The text of include/nvl.h, worked out here, against the function that both kernels call."""
+    src, exe = tmp_path / "said.cpp", tmp_path / "said"
+    src.write_text('#include <cstdio>\n#include "few_split.h"\nint main() {\n  for (int fours = 0; fours < 2; ++fours)\n    for (int parts = 1; parts <= 64; ++parts)\n'
+                   '      for (int t = 0; t <= 600; ++t) std::printf("%d\\n", nvl_few_split(t, NVL_OPEN_PART_TILES, parts, fours));\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    told = map(int, subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split())
+    up = lambda a, b: -(-a // b)
+    for parts in range(1, 65):
+        for t in range(601):
+            n = max(1, up(t, 8))
+            assert next(told) == (n if n <= parts else up(t, up(t, parts))), (t, parts)
+    for parts in range(1, 65):
+        for t in range(601):
+            n = up(t, 8)
+            r = up(n, 4) * 4
+            assert next(told) == (1 if n <= 1 else n if r == n <= parts else up(t, up(t, min(r, parts)))), (t, parts)

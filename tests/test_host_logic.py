@@ -349,10 +349,21 @@ def test_open_parts_run_at_once():
     from nano_vllm_amd import ops
     for b in (1, 2, 3, 4):
         for hkv in (1, 2, 4, 8, 16):
-            for longest in (256, 1024, 4096, 4097, 8192, 16384):
+            for longest in (256, 512, 700, 1024, 1300, 4096, 4097, 8192, 16384):
                 parts = ops.open_parts(b, hkv, longest)
                 assert 1 <= parts <= (8 if longest <= 4096 else 16) and parts <= -(-longest // 256) and b * hkv * parts <= 256
     assert [ops.open_parts(b, 8, 16384) for b in (1, 2, 3, 4, 5)] == [16, 16, 10, 8, 0] and ops.open_parts(1, 8, 16385) == 0
+
+
+def test_open_parts_in_fours_run_at_once():
+    from nano_vllm_amd import ops
+    for b in (1, 2, 3, 4):
+        for hkv in (1, 2, 4, 8, 16):
+            for longest in (256, 257, 512, 513, 1025, 2300, 4096, 4097, 8192, 16384):
+                parts, most = ops.open_parts(b, hkv, longest, True), min(8 if longest <= 4096 else 16, 256 // (b * hkv))
+                n = -(-longest // 256)
+                assert parts == (1 if n == 1 else min(-(-n // 4) * 4, most)), (b, hkv, longest)
+    assert [ops.open_parts(b, 8, 16384, True) for b in (1, 2, 3, 4, 5)] == [16, 16, 10, 8, 0] and ops.open_parts(1, 8, 16385, True) == 0
 
 
 SEQ_ABSENT = """
