@@ -292,7 +292,7 @@ int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype, int mode,
  * on 16-byte boundaries. */
 int nvs_silu_linear(const void* X, int64_t ldx, const void* W, int ff, int K, int64_t n, int tm, void* out, int64_t ldo, void* stream);
 /* bf16: out[t, :] = W X[t, :] (+ bias), W [nout, K], bias [nout] or null, in tiles of 256 rows; K % 64 == 0 and K >= 128, nout, ldx and ldo % 8 == 0, all on 16-byte
- * boundaries, rows and weights below 3 GiB. */
+ * boundaries, n ldx and nout K below 1,610,608,640 entries (3 GiB less 8 KiB), ldo below 4,194,304. */
 int nvs_linear_tiles(const void* X, int64_t ldx, const void* W, const void* bias, int nout, int K, int64_t n, void* out, int64_t ldo, void* stream);
 /* tests: 1 routes bf16 calls through the plain kernel as well */
 void nvs_moe_force_plain(int on);

@@ -25,10 +25,11 @@
 // us before (moe_gemm_pipe_kernel's tiles of 256 rows) / now, whole calls on one card: gate|up and SiLU, 14,600 rows, ff 3072, K 1024 185 / 154, K 4096 581 / 495; rows, 14,175 x 4096 x 4096
 // 399 / 324 (the library 331), 14,600 x 4096 x 1024 128 / 107, 14,600 x 1024 x 3072 92 / 77. Against the library: ops_seq.py (tiles_rule, silu_linear_rows).
 #pragma once
+#include "tiles_reach.h"
 
 // ring of five parts
 constexpr int TILE_ROW = 128, TILE_PART = 256 * TILE_ROW, TILE_RING = 5 * TILE_PART;
-constexpr uint32_t TILE_REACH = 0xC0000000u, TILE_NOWHERE = 0xF0000000u, TILE_SKEW = 4096;
+constexpr uint32_t TILE_NOWHERE = 0xF0000000u, TILE_SKEW = 4096;
 
 template <int MODE, bool PLAN>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W, int nout, int K,
@@ -267,8 +268,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
 
 // the calls that the tiles take: rows of whole 128-byte pieces (two at least), results in whole 16-byte units, offsets within 32 bits
 inline bool tiles_fit(int64_t ldx, int64_t rows, int nout, int K, int64_t weights, const void* out, int64_t ldo) {
-  return K % 64 == 0 && K >= 128 && ((nout | ldo) & 7) == 0 && ((uintptr_t)out & 15) == 0 && rows * ldx * 2 < TILE_REACH - 8192ll && weights * 2 < TILE_REACH - 8192ll &&
-         ldo < (1 << 22) && (rows + 255) / 256 * ((nout + 127) / 128) < (1ll << 31);
+  return K % 64 == 0 && K >= 128 && ((nout | ldo) & 7) == 0 && ((uintptr_t)out & 15) == 0 && tiles_reach(rows, ldx, weights, ldo) &&
+         (rows + 255) / 256 * ((nout + 127) / 128) < (1ll << 31);
 }
 
 template <int MODE, bool PLAN>

@@ -726,11 +726,16 @@ def tiles_rule(n: int, N: int, K: int) -> bool:
     return rest >= 224 if tiles <= 256 else tiles > 512 or rest <= 128 or rest >= 192
 
 
+def tiles_reach(rows: int, ldx: int, weights: int, ldo: int) -> bool:
+    """Whether the tiles' 32-bit offsets reach all of rows x ldx entries, the weights, and results ldo entries apart (csrc/seq/tiles_reach.h)."""
+    return max(rows * ldx, weights) * 2 < 0xC0000000 - 8192 and ldo < 1 << 22
+
+
 def linear_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What nvs_linear_tiles takes, of calls that nobody differentiates or traces."""
     return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]
             and x.shape[1] % 64 == 0 and x.shape[1] >= 128 and w.shape[0] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
-            and w.is_contiguous() and max(x.shape[0] * x.stride(0), w.numel()) < 3 << 29 and not torch.is_grad_enabled() and not torch.jit.is_tracing()
+            and w.is_contiguous() and tiles_reach(x.shape[0], x.stride(0), w.numel(), w.shape[0]) and not torch.is_grad_enabled() and not torch.jit.is_tracing()
             and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
@@ -784,7 +789,8 @@ def silu_linear_rows(n: int, ff: int, K: int) -> int:
 
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.stride(0) >= x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+            and x.stride(0) >= x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and w.is_contiguous() and (x.shape[0] + 255) * x.stride(0) < 8 << 32 and w.numel() < 8 << 32
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def silu_linear(x: torch.Tensor, w: torch.Tensor, tm: int, out: torch.Tensor | None = None) -> torch.Tensor:
