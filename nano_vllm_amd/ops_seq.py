@@ -731,12 +731,25 @@ def tiles_reach(rows: int, ldx: int, weights: int, ldo: int) -> bool:
     return max(rows * ldx, weights) * 2 < 0xC0000000 - 8192 and ldo < 1 << 22
 
 
+def _only_the_result(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether a product's result is all that is asked of it, so that a kernel's launch may stand in for F.linear: nobody differentiates it in either direction (forward mode
+    goes on under no_grad), maps over it, traces, compiles or watches it, or has autocast choose its type, and the tensors are plain ones of the device that launches go to."""
+    return (not _grad_enabled() and not _transformed() and _forward_ad._current_level < 0 and _dispatch_modes() == 0 and not _tracing() and not _compiling()
+            and not _autocast("cuda") and type(x) in _PLAIN and type(w) in _PLAIN and x.get_device() == torch.cuda.current_device())
+
+
+# (looked up once: the call above is made for every product of a step of many rows, 1.2 us)
+_PLAIN, _forward_ad = (torch.Tensor, torch.nn.Parameter), torch.autograd.forward_ad
+_grad_enabled, _transformed, _dispatch_modes = torch.is_grad_enabled, torch._C._are_functorch_transforms_active, torch._C._len_torch_dispatch_stack
+_tracing, _compiling, _autocast = torch.jit.is_tracing, torch.compiler.is_compiling, torch.is_autocast_enabled
+
+
 def linear_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """What nvs_linear_tiles takes, of calls that nobody differentiates or traces."""
+    """What nvs_linear_tiles takes."""
     return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]
             and x.shape[1] % 64 == 0 and x.shape[1] >= 128 and w.shape[0] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
-            and w.is_contiguous() and tiles_reach(x.shape[0], x.stride(0), w.numel(), w.shape[0]) and not torch.is_grad_enabled() and not torch.jit.is_tracing()
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+            and w.is_contiguous() and tiles_reach(x.shape[0], x.stride(0), w.numel(), w.shape[0])
+            and _only_the_result(x, w) and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def many_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
