@@ -709,20 +709,32 @@ TILES_FROM = 768
 
 def tiles_rule(n: int, N: int, K: int) -> bool:
     """Whether x w^T of n rows, N features and K entries each goes to the tiles of 256 rows x 256 features (256 of them are a pass, left-over ones of at most 128 go in
-    halves). MI355X, us here / the library's: 13,550 rows (a prompt step) 4096 x 4096 313 / 321, 6144 x 4096 455 / 620, 12288 x 4096 894 / 1035, 18752 x 4096 1399 / 1474,
-    24576 x 4096 1785 / 1827, 4096 x 12288 918 / 1153, 3088 x 1024 82 / 129, 3072 x 384 37 / 66, 4096 x 256 37 / 60; 12,918 rows, 4096 x 4096 309 / 411. Where the tiles are
-    whole passes the library's are as good or better by themselves: 16,384 rows, 4096 x 4096 363 / 356, 24576 x 4096 2172 / 2123, 15,637 rows, 1024 x 2048 54.1 / 52.3, 1024 x 3072 74.2 / 72.3.
-    But kernels of both kinds in turn cost each other 2 to 3 us a launch, so there too: the 28 layers' steps of 15,637 rows, 4096 x 1024 + 1024 x 2048 + 1024 x 3072, all here
-    16.66 ms, all there 16.71, some here and some there 16.93 to 17.00. One or two passes of which the last is between
-    half and three quarters full: 6,600 rows, 4096 x 4096 166 / 161, 2048 x 4096 at 12,800 91 / 86; a part of one: 2,700 rows, 4096 x 4096 79 / 74, 11,000, 1024 x 3072 65 / 58, but up to half of it
-    2,000 rows, 4096 x 4096 55 / 58, 6,600, 1024 x 3072 40 / 43, 1024 x 1024 17 / 19, 1,300 rows, 4096 x 1024 15 / 20, with short reductions (9,100 rows, 1024 x 256 11 / 19)
-    and with features that are no whole tiles (13,550 rows, 640 x 1024 23 / 30, 1000 x 4096 82 / 111). Fewer tiles leave most of the chip idle: 4,000 rows, 1024 x 3072 37 / 29."""
+    halves). MI355X, us here / the library's, between the other launches of a prompt step: weights come from memory there, and a product of few tiles that looks 10 % better
+    repeated by itself is 20 % worse. What decides is how full the passes are. Not full, here and there: 13,550 rows, 4096 x 4096 329 / 340, 6144 x 4096 478 / 632, 12288 x 4096 912 / 1037,
+    4096 x 12288 951 / 1187, 2312 x 1024 74 / 106; 12,285, 6144 x 2048 223 / 319; 3,000, 24576 x 4096 428 / 573. Short reductions: 2,000 rows, 4096 x 256 13 / 19, 3072 x 384 14 / 18.
+    Less than a pass leaves compute units idle, or with half a tile each, which wait for their operands: 1,300 rows, 4096 x 2048 39 / 34, x 4096 69 / 55, x 12288 189 / 140; 2,000, 4096 x 3072 60 / 53;
+    3,000, 2048 x 6144 108 / 77; 900, 6144 x 1536 35 / 28; at K 1024 not: 2,000, 4096 26 / 27, 8,190, 1024 24 / 27. So with rows that end early in a tile: 1,300, 24576 x 4096 236 / 221 (but 900,
+    16384 x 4096 94 / 106). The library is slower at features that are no multiple of 128: 6,600 rows, 1040 x 2048 48 / 44 (two fifths of a pass), 8,190 49 / 51, 12,285 55 / 70; 1824 x 4096, 3,000 rows 68 / 58,
+    6,600 93 / 102; 13,550, 656 x 1024 32 / 38. Multiples of 128 that are none of 256 fill its tiles and not these: 640 x 1024, 12,285 rows 31 / 28, 13,550 32 / 37; x 4096 by itself 81 / 56 and 82 / 74.
+    Whole passes take as long here and there, 2 to 3 % longer here by themselves (16,380 rows, 4096 x 4096 373 / 366, 24576 x 4096 2206 / 2152, 2048 x 6144 277 / 288), but kernels of both kinds in turn cost each
+    other that much, so they are not told apart. Steps of 16,384 rows in ms, all here / whole passes by the library: two layers of Qwen3-8B 9.61 / 9.56, nokipel 4096 11.78 / 11.62, 2048 3.70 / 3.73,
+    foduzen 4096 10.93 / 10.84, lobidra 2048 4.46 / 4.51, ligidra 2048 5.06 / 5.11, Qwen3-0.6B 17.16 / 17.04; of 12,288: 7.30 / 7.58, 9.04 / 9.11, - , 8.28 / 8.23; of 4,096: 2.64 / 2.68, 3.59 / 3.56, 1.28 / 1.27, 2.92 / 2.93."""
     tiles = -(-n // 256) * -(-N // 256)
     if n < TILES_FROM or tiles < 96:
         return False
-    if tiles <= 128 or K <= 512 or N % 256:
+    if K <= 512:
         return True
-    rest = tiles % 256 or 256
+    rest = tiles % 256
+    use = n * N / ((tiles // 256 + (0.5 if 0 < rest <= 128 else rest > 128)) * 256 ** 3)          # the passes' share that is rows and features
+    if N % 128:
+        return K <= 1024 or (use >= 0.5 if K <= 2048 else tiles > 160 and use >= 0.7)
+    if N % 256:
+        return use >= (0.5 if K <= 1024 else 0.75)
+    if tiles <= 128:
+        return K <= 1024
+    if K > 1024 and n < 2000 and use < 0.85:
+        return False
+    rest = rest or 256
     return rest >= 224 if tiles <= 256 else tiles > 512 or rest <= 128 or rest >= 192
 
 
