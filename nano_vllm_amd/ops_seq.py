@@ -798,17 +798,23 @@ def linear_tiles(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None
 
 def silu_linear_rows(n: int, ff: int, K: int) -> int:
     """Rows per tile of silu_linear, 0 where the vendor library's product and the activation behind it are the faster way. MI355X, us there / here at 64 / 256 rows, ff 3072, K 1024:
-    500 rows 18.7 / 13.7 / 14.9, 800: 20.3 / 20.1 / 15.4, 1300: 26.5 / 22.1 / 25.1, 2000: 36.2 / 33.1 / 26.3, 4000: 67 / 61 / 46, 14600: 199 / 204 / 150; ff 768, K 1024: 800:
+    500 rows 18.7 / 13.7 / 14.9, 800: 20.3 / 20.1 / 15.4, 1300: 26.5 / 22.1 / 25.1, 2000: 36.2 / 33.1 / 26.3, 4000: 67 / 61 / 46, 14600: 202 / 204 / 155; ff 768, K 1024: 800:
     13.0 / 13.5 / 14.8, 2000: 16.2 / 17.1 / 15.0, 4000: 22.7 / 21.9 / 16.5; ff 2048, K 2048: 800: 23.7 / 28.1 / 25.1, 1300: 30 / 34 / 26, 4000: 60 / 71 / 51; ff 8192, K 3072: 600: 61 / 89 / 63,
-    1000: 87 / 103 / 72, 9000: 721 / 907 / 618; ff 12288, K 4096: 600: 118 / 134 / 128, 1000: 179 / 198 / 143, 14600: 2282 / 2965 / 1984."""
+    1000: 87 / 103 / 72, 9000: 721 / 907 / 618; ff 12288, K 4096: 600: 118 / 134 / 128, 1000: 179 / 198 / 143, 14600: 2282 / 2965 / 1984. One pass that is half to three quarters full, long
+    reductions, there / 256: ff 3072, K 4096, 1300: 67 / 78; ff 1536, 2700: 64 / 75, K 3072 53 / 59; ff 512, 9100, K 2560 50 / 53, K 2048 43 / 45; ff 6144, K 1536, 600: 31 / 36 (500: 29 / 24). Short ones of which 64 rows make one pass and 256 half of
+    one or a little more than one, 64 / 256: K 512, ff 3072, 600: 9.7 / 10.6 (768: 13.1 / 10.7), ff 1536, 1300: 9.8 / 10.6, ff 12288, 600: 25.3 / 26.2; K 1024, ff 12288, 600: 41.1 / 42.0."""
     columns = -(-2 * ff // 256)
-    tiles = -(-n // 256) * columns
+    high = -(-n // 256)
+    tiles = high * columns
     if K % 64:
         return 0
     if ff % 8 or K < 128:                    # (not for the tiles of 256 rows that the figures are of: those before them)
         return 0 if K > 2560 else 256 if tiles >= 208 and (tiles >= 216 * -(-tiles // 256) or tiles >= 768) else 64 if K <= 1024 and tiles >= 72 else 0
-    if K <= 1024 and tiles > 128 and -(-n // 64) * columns <= 512:           # (two tiles of 64 rows at a time on every compute unit are one pass)
+    low = -(-n // 64) * columns              # tiles of 64 rows: two at a time on every compute unit are a pass
+    if K <= 1024 and (128 < tiles and low <= 512 or 256 < tiles <= 320 and low <= 1024) or K <= 512 and tiles >= 72 and low <= 256:
         return 64
+    if 128 < tiles <= 200 and (tiles <= (176 if K >= 4096 else 160) and (K >= 3072 or K >= 2560 and n >= 3000) or K > 1024 and n < 768 and n < (0.8 if tiles <= 160 else 0.6) * 256 * high):
+        return 0
     return 256 if tiles >= 96 and (n >= 768 or K <= 1536) or tiles >= 48 and n >= 500 and K <= 1024 else 0
 
 

@@ -14,3 +14,14 @@ import pytest
 def test_products_go_where_they_are_faster(n, N, K, tiles):
     from nano_vllm_amd import ops_seq
     assert ops_seq.tiles_rule(n, N, K) == tiles
+
+
+@pytest.mark.parametrize("n,ff,K,tm", [
+    (14600, 3072, 1024, 256), (2000, 3072, 1024, 256), (9000, 8192, 3072, 256), (1000, 12288, 4096, 256), (1300, 12288, 4096, 256),
+    (1300, 3072, 4096, 0), (2700, 1536, 4096, 0), (2700, 1536, 3072, 0), (9100, 512, 2560, 0), (1300, 3072, 2560, 256), (1700, 3072, 4096, 0), (2000, 3072, 4096, 256), (1300, 3072, 2048, 256),    # a pass that is half to three quarters full
+    (600, 6144, 1536, 0), (500, 6144, 1536, 256), (300, 12288, 1536, 0), (400, 12288, 1536, 256),                                                 # ... with rows that end early
+    (600, 3072, 512, 64), (768, 3072, 512, 256), (1300, 1536, 512, 64), (300, 6144, 512, 64), (400, 6144, 512, 256), (600, 3072, 1024, 256),      # 64 rows: one pass
+    (600, 12288, 512, 64), (600, 12288, 1024, 64), (1300, 6144, 512, 64), (3000, 3072, 1024, 256)])
+def test_gated_products_take_the_tiles_that_are_faster(n, ff, K, tm):
+    from nano_vllm_amd import ops_seq
+    assert ops_seq.silu_linear_rows(n, ff, K) == tm
