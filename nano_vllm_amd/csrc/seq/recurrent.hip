@@ -955,6 +955,10 @@ static int ssd_launch(int form, const char* who, const float* xbc, const void* p
   if (scan_chunk_fits(ca, dtype) && !walk) {
     if (ws) scan_chunk_plan(heads, P, nseq, max_q, &ca.seg_len, &ca.nseg);
     if (ca.seg_len && ws_floats < need(ca.nseg)) ca.seg_len = 0, ca.nseg = 1;
+    // Longest first where portions wait for one another: more workgroups than compute units, and lengths that differ (the longest is known, and their sum). Finding a
+    // portion's place takes a workgroup 0.1 to 0.2 us, which portions of up to 32 tokens and even ones would only lose: 64 of 16 tokens, 64 heads, forms 0, 1, 2 67 116 162 -> 71 125 171 us.
+    // In the order they come / longest first: 64 of 25 to 200 tokens, 16 heads, 94 160 179 / 76 126 147; 48 of 12 to 100, 32 heads, the longest last 68 109 128 / 65 104 125.
+    ca.by_length = nseq >= 2 && nseq <= 64 && max_q >= 48 && 8 * n <= 7 * max_q * nseq && pairs * ((P + 128) / 129) > 256;
     return scan_chunk_launch(ca, dtype, nseq, stream);
   }
   const int threads = ((P + pp - 1) / pp) * ng, per = (((P + pp - 1) / pp * pp + 3) & ~3) + 2 * ng * SSD_R + 4;

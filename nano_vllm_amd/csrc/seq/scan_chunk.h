@@ -15,6 +15,7 @@ struct ScanArgs {
   float *S, *M, *y, *den, *ws;
   float cap, c_scale;
   int seg_len, nseg;
+  int by_length;                     // portions longest first (2 to 64 of them)
 };
 
 // segments for the chunk kernel (seg_len 0: none)

@@ -26,9 +26,9 @@ namespace {
 // 64 heads of 64 x 128 (form 0) 5,200 -> 650 us, 32 heads of 128 x 128 (form 1) 3,470 -> 700, 8 heads of 128 x 128 (form 2)
 // 1,600 -> 250; one portion of 16,384: 3,650 -> 860, 3,690 -> 900, 1,690 -> 245. Errors against 64 bits, first nine portions,
 // outputs / states: 1.3e-7 / 1.0e-7 -> 1.2e-7 / 0.9e-7, 1.9e-7 / 5.0e-7 -> 1.3e-7 / 3.7e-7, 2.0e-7 / 1.9e-7 -> 1.8e-7 / 1.4e-7.
-// Portions are taken longest first (ragged ones end together: 26 of 100 to 1,024 tokens, form 1 539 -> 414 us, form 0 486 -> 436; nine of 33 to 4,096 735 -> 689, 816 -> 676), and
-// form 1's SiLU, a third of its vector instructions, which no 32-bit matrix instruction runs beside (49 + 51 % of all cycles over 16 portions of 512), is the short one of
-// seq_common.h, with the same errors (nine of 1,100 to 2,048 700 -> 635 us, 32 of 1,000 975 -> 899).
+// Ragged portions are taken longest first (recurrent.hip says when), so that they end together: 12 of 175 to 1,400 tokens, 64 heads, forms 0, 1, 2 412 712 820 -> 358 569 658 us.
+// Form 1's SiLU, a third of its vector instructions, which no 32-bit matrix instruction runs beside (49 + 51 % of all cycles over 16 portions of 512), is the short one of
+// seq_common.h, with the same errors (the same portions 758 -> 712 us, 32 of 100 tokens 227 -> 215).
 constexpr int CT = 16;                              // tokens of a chunk
 constexpr int WST = 20;                             // row stride of the 16 x 16 weights in LDS
 constexpr int SB = 4;                               // chunks whose weights are computed together: a token per lane
@@ -64,7 +64,8 @@ __device__ __forceinline__ double lane_of(double v, int lane) { return __shfl(v,
 
 // MODE as in recurrent.hip: 0 the whole portion, 1 a segment's local state only, 2 a segment's outputs from the state before it,
 // which scan_states_kernel puts in the place of the local states in between.
-template <typename T, int NT, int NW, int FORM, int MODE>
+// BY_LENGTH: of 2 to 64 portions the longest is the first.
+template <typename T, int NT, int NW, int FORM, int MODE, bool BY_LENGTH>
 __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanArgs a) {
   constexpr int N = 16 * NT, LD = N + 4, NTH = NW * 64;
   typedef typename std::conditional<FORM == 0, float, T>::type TB;            // what B and C are stored as
@@ -76,9 +77,12 @@ __global__ __launch_bounds__(NW * 64, NW / 2) void scan_chunk_kernel(const ScanA
   __shared__ __attribute__((aligned(16))) float win[2][FORM == 1 ? 1 : SB][2][CT];      // decay from the chunk's start, and what rounding left of it; form 2: exp(-m)
   __shared__ __attribute__((aligned(16))) float nq[FORM == 2 ? 2 : 1][KW][CT];     // form 2: the parts of n . q
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, g = lane >> 4;
-  const int h = blockIdx.x, s = MODE == 0 ? portion_by_length(a.cu_q, gridDim.y, blockIdx.y) : blockIdx.y, seg = blockIdx.z % a.nseg, blk = blockIdx.z / a.nseg;
+  const int h = blockIdx.x, seg = blockIdx.z % a.nseg, blk = blockIdx.z / a.nseg;
   const int heads = a.heads, P = a.P;
-  const int64_t t0 = a.cu_q[s], t1 = a.cu_q[s + 1];
+  PortionSpan span;
+  if constexpr (BY_LENGTH) span = portion_by_length(a.cu_q, gridDim.y, blockIdx.y);
+  const int s = BY_LENGTH ? span.s : blockIdx.y;
+  const int64_t t0 = BY_LENGTH ? span.t0 : a.cu_q[s], t1 = BY_LENGTH ? span.t1 : a.cu_q[s + 1];
   const int64_t q0 = MODE == 0 ? t0 : t0 + (int64_t)seg * a.seg_len;
   const int64_t q1 = MODE == 0 ? t1 : (q0 + a.seg_len < t1 ? q0 + a.seg_len : t1);
   if (q1 <= q0) return;
@@ -483,12 +487,12 @@ void launch_form(const ScanArgs& a, int nseq, hipStream_t stream) {
   const dim3 grid(a.heads, (unsigned)nseq, (unsigned)(blocks * a.nseg)), block(NW * 64);
   if (a.seg_len) {
     const int64_t PN = (int64_t)a.P * a.N;
-    scan_chunk_kernel<T, NT, NW, FORM, 1><<<grid, block, 0, stream>>>(a);
+    scan_chunk_kernel<T, NT, NW, FORM, 1, false><<<grid, block, 0, stream>>>(a);
     scan_states_kernel<FORM == 2><<<dim3((unsigned)((PN / 4 + 255) / 256), a.heads, (unsigned)nseq), dim3(256), 0, stream>>>(
         a.ws, a.cu_q, a.seg_len, a.nseg, PN);
-    scan_chunk_kernel<T, NT, NW, FORM, 2><<<grid, block, 0, stream>>>(a);
+    scan_chunk_kernel<T, NT, NW, FORM, 2, false><<<grid, block, 0, stream>>>(a);
   } else {
-    scan_chunk_kernel<T, NT, NW, FORM, 0><<<grid, block, 0, stream>>>(a);
+    a.by_length ? scan_chunk_kernel<T, NT, NW, FORM, 0, true><<<grid, block, 0, stream>>>(a) : scan_chunk_kernel<T, NT, NW, FORM, 0, false><<<grid, block, 0, stream>>>(a);
   }
 }
 

@@ -162,17 +162,27 @@ __device__ __forceinline__ RglruTerms rglru_terms(float gr, float gi, float u, f
   return v;
 }
 
-// The portion that is number `rank` by length, longest first (up to 64 portions; beyond, number `rank` as they come): workgroups start in the order of their numbers, so
-// what is left for the end of a launch is short. All lanes of the wavefront call it.
-__device__ __forceinline__ int portion_by_length(const int32_t* __restrict__ cu_q, int nseq, int rank) {
-  if (nseq < 2 || nseq > 64) return rank;
-  const int lane = threadIdx.x & 63, mine = lane < nseq ? cu_q[lane + 1] - cu_q[lane] : -1;
-  int longer = 0;
-  for (int j = 0; j < nseq; ++j) {
-    const int other = __builtin_amdgcn_readlane(mine, j);
-    longer += other > mine || (other == mine && j < lane);
+// A portion and its tokens [t0, t1) in the step
+struct PortionSpan {
+  int s, t0, t1;
+};
+
+// The portion that is number `rank` by length (in chunks of 16 tokens), longest first, of 2 to 64: workgroups start in the order of their numbers, so what is left for
+// the end of a launch is short. Its length is found bit by bit, a ballot each: counting for every portion how many are longer took a workgroup 1 us, which is as
+// long as a short portion's scan. All lanes of the wavefront call it.
+__device__ __forceinline__ PortionSpan portion_by_length(const int32_t* __restrict__ cu_q, int nseq, int rank) {
+  const int lane = threadIdx.x & 63, t0 = cu_q[lane < nseq ? lane : 0], t1 = cu_q[lane < nseq ? lane + 1 : 0];
+  const int mine = lane < nseq ? (t1 - t0 + 15) >> 4 : -1;
+  int longest = (__builtin_amdgcn_readlane(t1, nseq - 1) - __builtin_amdgcn_readfirstlane(t0) + 15) >> 4, v = 0;        // (not more than all of them)
+  for (int bit = 31 - __builtin_clz(longest | 1); bit >= 0; --bit) {
+    const int more = v | 1 << bit;
+    if (__builtin_popcountll(__ballot(mine >= more)) > rank) v = more;
   }
-  return __builtin_ctzll(__ballot(lane < nseq && longer == rank));
+  const uint64_t as_long = __ballot(mine == v);       // (ties in the order they come; all ballots by all lanes)
+  const int longer = __builtin_popcountll(__ballot(mine > v));
+  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(as_long >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)as_long, 0));
+  const int s = __builtin_ctzll(__ballot(mine == v && longer + before == rank));
+  return {s, __builtin_amdgcn_readlane(t0, s), __builtin_amdgcn_readlane(t1, s)};
 }
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }

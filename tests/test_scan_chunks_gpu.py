@@ -198,3 +198,11 @@ def test_silu_of_large_negative_inputs_is_nothing(where, huge):
 def test_portions_that_are_taken_by_length(form, heads, P, N, lens):
     """The longest first: equal lengths and portions without a token (of sequences that go on: their slots stay as they are) each find their own place."""
     test_chunked_recurrences_against_the_token_loop(form, heads, P, N, 1, lens, torch.bfloat16)
+
+
+@pytest.mark.parametrize("lens,heads", [([50, 0, 17, 33] * 16, 5), ([60, 60, 1, 0] * 10, 7), ([70, 20], 130), ([1] * 63 + [48], 8)], ids=["64", "ties", "two", "one long"])
+@pytest.mark.parametrize("form,P,N", [(0, 64, 64), (1, 16, 64), (2, 24, 64)])
+def test_ragged_portions_in_more_workgroups_than_compute_units(form, P, N, lens, heads):
+    """The same where the launch does take them by length: more than 256 workgroups, 48 tokens or more, lengths that differ."""
+    assert heads * len(lens) > 256 and max(lens) >= 48 and 8 * sum(lens) <= 7 * max(lens) * len(lens)
+    test_chunked_recurrences_against_the_token_loop(form, heads, P, N, 1, lens, torch.bfloat16)
