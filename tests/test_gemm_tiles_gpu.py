@@ -7,6 +7,26 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def products(x, w):
+    """x w^T in 64 bits, and what a sum of K products in 32 bits, in any order, may be off by: K 2^-24 of the sum of their sizes."""
+    x, w = x.double(), w.double()
+    return x @ w.T, x.shape[1] * 2.0 ** -24 * (x.abs() @ w.abs().T)
+
+
+def every_value(got, want, off):
+    """No value is off by more than `off` and one rounding to bfloat16 (half a step of 8 bits: 2^-8 of a value at most): a lost or stale 16-byte unit among millions
+    does not show in a norm."""
+    wrong = ((got.double() - want).abs() > 2.0 ** -8 * want.abs() + off * (1 + 2.0 ** -8)).sum().item()
+    assert wrong == 0, f"{wrong} of {want.numel()} values"
+
+
+def gated(y, off, ff):
+    """silu(g) u and its bound: SiLU's slope is below 1.1, its own error and the product's below 2^-21."""
+    g, u, eg, eu = y[:, :ff], y[:, ff:], off[:, :ff], off[:, ff:]
+    a = torch.nn.functional.silu(g)
+    return a * u, 1.1 * eg * (u.abs() + eu) + a.abs() * eu + 2.0 ** -21 * (a * u).abs()
+
+
 @pytest.mark.parametrize("n,ff,K", [(1, 8, 128), (128, 128, 192), (129, 136, 256), (257, 1000, 320), (256, 256, 384), (2048, 4096, 128), (2100, 4096, 192),
                                     (3072, 4096, 448), (3100, 4096, 128), (9000, 768, 1024)])
 def test_dense_products(n, ff, K):
@@ -15,13 +35,16 @@ def test_dense_products(n, ff, K):
     x = torch.randn(n, K + 8, generator=g).to(torch.bfloat16).cuda()[:, :K]
     w = (torch.randn(2 * ff, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
     room = torch.full((n + 300, ff + 8), 7.0, dtype=torch.bfloat16, device="cuda")
-    y = x.double() @ w.double().T
-    want = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+    want, off = gated(*products(x, w), ff)
+    before = None
     for _ in range(2):
         ops_seq.silu_linear(x, w, 256, room[:n, :ff])
         # one rounding of the result to bfloat16, 2^-9 at most per value
         assert ((room[:n, :ff].double() - want).norm() / want.norm()).item() <= 2.0 ** -8
         assert (room[n:] == 7.0).all() and (room[:, ff:] == 7.0).all()
+        every_value(room[:n, :ff], want, off)
+        assert before is None or torch.equal(before, room)          # (the order of a sum is fixed)
+        before = room.clone()
 
 
 @pytest.mark.parametrize("biased", [False, True])
@@ -33,11 +56,17 @@ def test_dense_rows(n, N, K, biased):
     w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
     b = torch.randn(N, generator=g).to(torch.bfloat16).cuda() if biased else None
     room = torch.full((n + 300, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
-    want = x.double() @ w.double().T + (b.double() if biased else 0.0)
+    want, off = products(x, w)
+    if biased:
+        want, off = want + b.double(), off + 2.0 ** -24 * (want.abs() + b.double().abs())
+    before = None
     for _ in range(2):
         ops_seq.linear_tiles(x, w, b, room[:n, :N])
         assert ((room[:n, :N].double() - want).norm() / want.norm()).item() <= 2.0 ** -8          # (one rounding of the result to bfloat16)
         assert (room[n:] == 7.0).all() and (room[:, N:] == 7.0).all()
+        every_value(room[:n, :N], want, off)
+        assert before is None or torch.equal(before, room)
+        before = room.clone()
 
 
 @torch.inference_mode()
@@ -73,15 +102,24 @@ def test_grouped_products(mode, counts, nout, K):
         src = torch.full((plan.cap, K), float("nan"), dtype=torch.bfloat16, device="cuda")
         src[rows] = x
     out = torch.full((plan.cap, nout), 7.0, dtype=torch.bfloat16, device="cuda")
+    before = None
     for _ in range(2):
         ops_seq.moe_gemm(src, w, plan, mode == "glu", out, relu2=mode == "relu2")
+        assert before is None or torch.equal(before, out)
+        before = out.clone()
     for e in range(E):
         mine = (ids == e).nonzero().view(-1)
         if not len(mine):
             continue
-        y = x[mine].double() @ w[e].double().T
-        want = torch.nn.functional.silu(y[:, :nout]) * y[:, nout:] if mode == "glu" else y.clamp(min=0) ** 2 if mode == "relu2" else y
+        y, off = products(x[mine], w[e])
+        if mode == "glu":
+            want, off = gated(y, off, nout)
+        elif mode == "relu2":                                       # (the square is one more rounding)
+            want, off = y.clamp(min=0) ** 2, 2 * y.abs() * off + off ** 2 + 2.0 ** -23 * y ** 2
+        else:
+            want = y
         assert ((out[rows[mine]].double() - want).norm() / want.norm()).item() <= 2.0 ** -8       # (one rounding of the result to bfloat16)
+        every_value(out[rows[mine]], want, off)
     untouched = torch.ones(plan.cap, dtype=torch.bool, device="cuda")
     untouched[rows] = False
     assert (out[untouched] == 7.0).all()
