@@ -758,14 +758,15 @@ _tracing, _compiling, _autocast = torch.jit.is_tracing, torch.compiler.is_compil
 
 def linear_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What nvs_linear_tiles takes."""
-    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]
-            and x.shape[1] % 64 == 0 and x.shape[1] >= 128 and w.shape[0] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
-            and w.is_contiguous() and tiles_reach(x.shape[0], x.stride(0), w.numel(), w.shape[0])
-            and _only_the_result(x, w) and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+    if x.dim() != 2 or w.dim() != 2:
+        return False
+    (n, k), (N, wide), (ld, unit) = x.shape, w.shape, x.stride()
+    return (k == wide and k % 64 == 0 and k >= 128 and N % 8 == 0 and unit == 1 and ld % 8 == 0 and ld >= k and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda
+            and x.device == w.device and w.is_contiguous() and tiles_reach(n, ld, N * k, N) and _only_the_result(x, w) and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def many_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
-    return (x.dim() == 2 and w.dim() == 2 and tiles_rule(x.shape[0], w.shape[0], x.shape[1]) and linear_tiles_fits(x, w)
+    return (x.dim() == 2 and w.dim() == 2 and tiles_rule(x.shape[0], *w.shape) and linear_tiles_fits(x, w)
             and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1] and b.data_ptr() % 16 == 0))
 
 
@@ -819,9 +820,11 @@ def silu_linear_rows(n: int, ff: int, K: int) -> int:
 
 
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.dim() == 2 and w.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.stride(0) >= x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and w.is_contiguous() and (x.shape[0] + 255) * x.stride(0) < 8 << 32 and w.numel() < 8 << 32
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+    if x.dim() != 2 or w.dim() != 2:
+        return False
+    (n, k), (N, wide), ld = x.shape, w.shape, x.stride(0)
+    return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device and x.stride(1) == 1 and ld % 8 == 0 and ld >= k == wide and N % 2 == 0 and w.is_contiguous()
+            and (n + 255) * ld < 8 << 32 and N * k < 8 << 32 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def silu_linear(x: torch.Tensor, w: torch.Tensor, tm: int, out: torch.Tensor | None = None) -> torch.Tensor:
