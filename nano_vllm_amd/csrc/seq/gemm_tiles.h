@@ -22,7 +22,7 @@
 // or 256 bytes; the number of stores does not depend on the rows that are there (those that are not go nowhere), so the next tile's waits can count them and none waits for them to drain.
 // Tiles that are left for a last pass of at most 128 workgroups are halved: 14,600 rows and 24 feature tiles are 5.4 passes, not 6 (gate|up at K 1024 7 % of its time).
 //
-// us before (moe_gemm_pipe_kernel's tiles of 256 rows) / now, whole calls on one card: gate|up and SiLU, 14,600 rows, ff 3072, K 1024 185 / 154, K 4096 581 / 495; rows, 14,175 x 4096 x 4096
+// us before (moe_gemm_pipe_kernel's tiles of 256 rows) / now, whole calls on one card: gate|up and SiLU, 14,600 rows, ff 3072, K 1024 185 / 155, K 4096 581 / 495; rows, 14,175 x 4096 x 4096
 // 399 / 324 (the library 331), 14,600 x 4096 x 1024 128 / 107, 14,600 x 1024 x 3072 92 / 77. Against the library: ops_seq.py (tiles_rule, silu_linear_rows).
 #pragma once
 #include "tiles_reach.h"
@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
 #pragma unroll
   for (int i = 0; i < 8; ++i) read(a, false, i, 0, x0), read(a, true, i, 0, w0);
   __builtin_amdgcn_s_waitcnt(0xC07F);
-  int stores = 0;                             // of the tile before, younger than the requests its end left
+  constexpr int STORES = GLU ? 16 : 32;       // of a tile of 256 rows, younger than the requests its end left (nothing follows one of 128)
+  bool stored = false;
   const auto tile = [&](auto RBC) {
     constexpr int RB = decltype(RBC)::value;
     const int64_t row0 = (int64_t)rt * 256 + sub + wm * RB * 16;
@@ -197,10 +198,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
       }
       if (s == 0) {
         half_step(RBC, std::true_type{}, acc, a, b, 1, x0, w0, false, x2, ahead);
-        if (!stores) __builtin_amdgcn_s_waitcnt(0x0F78);               // vmcnt(8): the next step's parts are there
-        else if (stores == 8) __builtin_amdgcn_s_waitcnt(0x4F70);      // ... (16)
-        else if (stores == 16) __builtin_amdgcn_s_waitcnt(0x4F78);     // ... (24)
-        else __builtin_amdgcn_s_waitcnt(0x8F78);                       // ... (40)
+        if (!stored) __builtin_amdgcn_s_waitcnt(0x0F78);               // vmcnt(8): the next step's parts are there
+        else __builtin_amdgcn_s_waitcnt(0x0F78 + STORES / 16 * 0x4000);          // ... (8 + STORES)
       } else {
         half_step(RBC, std::false_type{}, acc, a, b, 1, x0, w0, false, x2, ahead);
         __builtin_amdgcn_s_waitcnt(0x0F78);
@@ -256,7 +255,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const bf16_t* __rest
         __builtin_amdgcn_raw_buffer_store_b128(q[p], os, (on >> (p * PER + line) & 1) && inside ? to : TILE_NOWHERE, (rb * 16 + p * PER) * (int)ldo * 2, 2);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
-    stores = RB * 16 / PER;
+    static_assert(RB == 4 || RB * 16 / PER == STORES, "the next tile's first wait counts them");
+    stored = true;
     return more;
   };
   bool more = true;
@@ -274,12 +274,12 @@ inline bool tiles_fit(int64_t ldx, int64_t rows, int nout, int K, int64_t weight
 
 template <int MODE, bool PLAN>
 int launch_tiles(const void* X, int64_t ldx, const void* W, int nout, int K, const int32_t* tile_expert, const int32_t* row_token, int64_t cap, void* out,
-                 int64_t ldo, hipStream_t st, int rows = 0, const void* bias = nullptr) {
+                 int64_t ldo, hipStream_t st, const char* who, int rows = 0, const void* bias = nullptr) {
   constexpr int BN = MODE == 1 ? 128 : 256;
   const int64_t tiles_m = (cap + 255) / 256, tiles_n = (nout + BN - 1) / BN;
   const auto kernel = gemm_tiles_kernel<MODE, PLAN>;
-  NVS_LDS_ROOM(kernel, TILE_RING, "nvs_moe_gemm");
+  NVS_LDS_ROOM(kernel, TILE_RING, who);
   kernel<<<dim3(256), dim3(256), TILE_RING, st>>>((const bf16_t*)X, ldx, (const bf16_t*)W, nout, K, tile_expert, row_token, (int)tiles_m, (int)tiles_n, (uint32_t)((1ull << 32) / (8 * tiles_n) + 1), rows,
                                                   (const bf16_t*)bias, (bf16_t*)out, ldo);
-  return nvs_check_launch("nvs_moe_gemm (matrix cores, tiles of 256 rows)");
+  return nvs_check_launch(who);
 }

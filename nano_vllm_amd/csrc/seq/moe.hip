@@ -949,7 +949,7 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
               : launch_pipe<float, false, __VA_ARGS__>(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, mode, st)))
     if (tm == 256 && dtype == NVS_BF16 && tiles_fit(ldx, cap, nout, K, (glu ? 2ll : 1ll) * nout * K, out, ldo)) {
       const auto launch = glu ? launch_tiles<1, true> : mode ? launch_tiles<2, true> : launch_tiles<0, true>;
-      return launch(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, st, 0, nullptr);
+      return launch(X, ldx, W, nout, K, tile_expert, row_token, cap, out, ldo, st, "nvs_moe_gemm (matrix cores, tiles of 256 rows)", 0, nullptr);
     }
     if (tm == 256) return NVS_PIPE(2, 8, 8, 2, 1);
     if (tm == 128) return NVS_PIPE(2, 8, 4, 3, 1);
@@ -995,14 +995,14 @@ extern "C" int nvs_moe_gemm(const void* X, int64_t ldx, const void* W, int dtype
 }
 
 // silu(g) u of [g | u] = X W^T: the tiles of the grouped product with one expert and no plan. The library's product and the activation behind it write and read
-// [n, 2 ff] once more than this: 14,600 rows, ff 3072, K 1024 222 us, here 154; which of them is taken is the caller's choice (measured there).
+// [n, 2 ff] once more than this: 14,600 rows, ff 3072, K 1024 202 us, here 155; which of them is taken is the caller's choice (measured there).
 extern "C" int nvs_silu_linear(const void* X, int64_t ldx, const void* W, int ff, int K, int64_t n, int tm, void* out, int64_t ldo, void* stream) {
   if (n == 0) return NVS_OK;
   NVS_REQUIRE(X && W && out && ff > 0 && K > 0 && K % 64 == 0 && n > 0 && ldx >= K && ldx % 8 == 0 && ldo >= ff && (((uintptr_t)X | (uintptr_t)W) & 15) == 0,
               "nvs_silu_linear: %lld rows, %d x %d", (long long)n, ff, K);
   NVS_REQUIRE((tm == 64 || tm == 256) && n < (1ll << 31) - 256 && (n + 255) * ldx < (8ll << 32) && 2ll * ff * K < (8ll << 32), "nvs_silu_linear: step too large");
   const int64_t cap = (n + tm - 1) / tm * tm;
-  if (tm == 256 && tiles_fit(ldx, n, ff, K, 2ll * ff * K, out, ldo)) return launch_tiles<1, false>(X, ldx, W, ff, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, (int)n);
+  if (tm == 256 && tiles_fit(ldx, n, ff, K, 2ll * ff * K, out, ldo)) return launch_tiles<1, false>(X, ldx, W, ff, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, "nvs_silu_linear", (int)n);
   if (tm == 256) return launch_pipe<bf16_t, true, 2, 8, 8, 2, 1, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
   return launch_pipe<bf16_t, true, 4, 4, 4, 2, 2, false>(X, ldx, W, ff, K, nullptr, nullptr, cap, out, ldo, 1, (hipStream_t)stream, (int)n);
 }
@@ -1013,8 +1013,8 @@ extern "C" int nvs_linear_tiles(const void* X, int64_t ldx, const void* W, const
   NVS_REQUIRE(X && W && out && nout > 0 && n > 0 && ldx >= K && ldx % 8 == 0 && ldo >= nout && (((uintptr_t)X | (uintptr_t)W | (uintptr_t)bias) & 15) == 0 &&
                   n < (1ll << 31) - 256 && tiles_fit(ldx, n, nout, K, (int64_t)nout * K, out, ldo),
               "nvs_linear_tiles: %lld rows, %d x %d", (long long)n, nout, K);
-  if (bias) return launch_tiles<3, false>(X, ldx, W, nout, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, (int)n, bias);
-  return launch_tiles<0, false>(X, ldx, W, nout, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, (int)n);
+  if (bias) return launch_tiles<3, false>(X, ldx, W, nout, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, "nvs_linear_tiles", (int)n, bias);
+  return launch_tiles<0, false>(X, ldx, W, nout, K, nullptr, nullptr, n, out, ldo, (hipStream_t)stream, "nvs_linear_tiles", (int)n);
 }
 
 extern "C" int nvs_moe_combine(const void* rows, int64_t ldr, const int32_t* pair_row, const float* wts, int top, const void* h, int64_t ldh,

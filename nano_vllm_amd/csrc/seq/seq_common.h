@@ -28,7 +28,7 @@ int nvs_check_launch(const char* what);
     (void)hipGetDevice(&nvs_device);                                                                                                                          \
     if (!(nvs_room.load(std::memory_order_relaxed) >> (nvs_device & 63) & 1)) {                                                                               \
       NVS_REQUIRE(hipFuncSetAttribute((const void*)(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess,                                \
-                  what ": %d bytes of LDS were refused", (int)(bytes));                                                                                       \
+                  "%s: %d bytes of LDS were refused", what, (int)(bytes));                                                                                \
       nvs_room.fetch_or(1ull << (nvs_device & 63), std::memory_order_relaxed);                                                                                \
     }                                                                                                                                                         \
   } while (0)
