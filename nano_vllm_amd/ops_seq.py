@@ -767,7 +767,7 @@ def linear_tiles_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def many_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
     return (x.dim() == 2 and w.dim() == 2 and tiles_rule(x.shape[0], *w.shape) and linear_tiles_fits(x, w)
-            and (b is None or b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1] and b.data_ptr() % 16 == 0))
+            and (b is None or type(b) in _PLAIN and b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1] and b.data_ptr() % 16 == 0))
 
 
 def _linear_many(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:

@@ -92,6 +92,15 @@ def test_subclasses_stay_themselves(xw):
 
 
 @torch.no_grad()
+def test_a_subclass_as_the_bias_is_asked_too(xw):
+    class Tagged(torch.Tensor):
+        pass
+    x, w = xw
+    b = torch.randn(w.shape[0]).bfloat16().cuda()
+    assert isinstance(layer(w, b.as_subclass(Tagged))(x), Tagged) and type(layer(w, b)(x)) is torch.Tensor
+
+
+@torch.no_grad()
 def test_tensors_of_another_device_than_the_launches(xw, monkeypatch):
     from nano_vllm_amd import ops_seq
     x, w = xw
