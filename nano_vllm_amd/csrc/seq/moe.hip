@@ -519,7 +519,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16_t* __res
 // could not write padding). The MFMAs are written out with accumulators in the accumulation registers and operands in the vector registers:
 // left to itself the compiler moves one or the other between the two files in the loop.
 //
-// (16-bit tiles of 256 rows are gemm_tiles.h's, but for rows and results that it does not take.) As many workgroups as fit on the chip at once, and each goes on from tile to tile: the last ST steps of a tile ask for the first ones of the next, whose
+// 16-bit tiles of 256 rows are gemm_tiles.h's, but for rows and results that its tiles_fit leaves out; figures of 256 rows below are this kernel's. As many workgroups as fit on the chip at once, and each goes on from tile to tile: the last ST steps of a tile ask for the first ones of the next, whose
 // rows were looked up a whole tile earlier, so no tile but the first waits for its plan, its addresses and its operands, and the stores drain behind the next
 // tile's first steps. Full tiles of 256 rows x 256 weight rows, us per tile at k = 256 / 1024 / 4096, before and after (the products alone take 5.9 / 23.6 /
 // 94): gated 22.4 / 42.2 / 111.8 -> 13.1 / 32.0 / 106.9, plain 20.7 / 41.0 / 111.0 -> 14.7 / 36.8 / 109.0; tiles of 128 rows, gated 12.5 / 22.3 / 62.5 -> 7.3 / 17.4 / 58.3; of

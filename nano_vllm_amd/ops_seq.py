@@ -717,8 +717,8 @@ def tiles_rule(n: int, N: int, K: int) -> bool:
     16384 x 4096 94 / 106). The library is slower at features that are no multiple of 128: 6,600 rows, 1040 x 2048 48 / 44 (two fifths of a pass), 8,190 49 / 51, 12,285 55 / 70; 1824 x 4096, 3,000 rows 68 / 58,
     6,600 93 / 102; 13,550, 656 x 1024 32 / 38. Multiples of 128 that are none of 256 fill its tiles and not these: 640 x 1024, 12,285 rows 31 / 28, 13,550 32 / 37; x 4096 by itself 81 / 56 and 82 / 74.
     Whole passes take as long here and there, 2 to 3 % longer here by themselves (16,380 rows, 4096 x 4096 373 / 366, 24576 x 4096 2206 / 2152, 2048 x 6144 277 / 288), but kernels of both kinds in turn cost each
-    other that much, so they are not told apart. Steps of 16,384 rows in ms, all here / whole passes by the library: two layers of Qwen3-8B 9.61 / 9.56, nokipel 4096 11.78 / 11.62, 2048 3.70 / 3.73,
-    foduzen 4096 10.93 / 10.84, lobidra 2048 4.46 / 4.51, ligidra 2048 5.06 / 5.11, Qwen3-0.6B 17.16 / 17.04; of 12,288: 7.30 / 7.58, 9.04 / 9.11, - , 8.28 / 8.23; of 4,096: 2.64 / 2.68, 3.59 / 3.56, 1.28 / 1.27, 2.92 / 2.93."""
+    other that much, so they are not told apart. Steps of 16,384 rows in ms, all here / whole passes by the library: two layers of Qwen3-8B 9.58 / 9.56, nokipel 4096 11.70 / 11.62, 2048 3.71 / 3.73,
+    foduzen 4096 10.88 / 10.84, lobidra 2048 4.47 / 4.51, ligidra 2048 5.06 / 5.11, Qwen3-0.6B 17.19 / 17.04; of 12,288: 7.30 / 7.58, 9.00 / 9.11, - , 8.27 / 8.23; of 4,096: 2.63 / 2.68, 3.56 / 3.56, 1.29 / 1.27, 2.93 / 2.93."""
     tiles = -(-n // 256) * -(-N // 256)
     if n < TILES_FROM or tiles < 96:
         return False
@@ -926,7 +926,8 @@ class MoePlan:
 
 def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dtype) -> int:
     """Rows per tile of a step's plan. It follows the rows an expert gets on average: a tile reads all weights of its features, so few
-    rows want the smallest tile and many the largest. MI355X, gate|up + down of 32 gated experts, us at tiles of 16 / 64 / 128 / 256 rows:
+    rows want the smallest tile and many the largest. The figures of 256 rows are of moe_gemm_pipe_kernel; 16-bit ones run gemm_tiles_kernel now, which takes 15 to 30 % less, so that some calls below the
+    lines for 256 would be faster there too. MI355X, gate|up + down of 32 gated experts, us at tiles of 16 / 64 / 128 / 256 rows:
     width 4096, ff 3072: 8 rows 428 / 436 / 471 / 609; 32: 598 / 455 / 489 / 622; 64: 838 / 580 / 507 / 640; 250: 2256 / 1003 / 879 / 928;
     1694: 12546 / 4674 / 4103 / 3634. Width 2048: 16 rows 126 / 133 / 149 / 178; 32: 141 / 135 / 155 / 181; 500: 1028 / 456 / 420 / 408.
     Width 1024, ff 768 (few and short tiles: two small workgroups per compute unit cover each other's start and end better than one large
