@@ -142,6 +142,19 @@ int nvl_pack_weight_tiles(const void* weight, void* packed, int64_t n, int64_t k
 int nvl_norm_linear(const void* x, int slabs, const void* residual, const void* norm_weight, float eps, const void* weight, void* out, void* residual_out,
                     int64_t m, int n, int k, int silu, void* stream);
 
+/* All layers of a decode step of up to four sequences in one launch (and one before it that empties the exchange, one behind it that leaves at once unless the workgroups
+ * did not all run together): what nvl_norm_linear, nvl_paged_attn_decode_open, nvl_linear_decode_open, nvl_norm_linear (silu) and nvl_linear_decode (mode 2) do a layer.
+ *   nvl_decode_step_workspace_bytes: scratch of a call; 0: the step is not covered (hidden 1024, ff 1024, 2048 or 3072, 8 or 16 query heads in pairs over a kv head, up to
+ *     40 layers and 4 rows).
+ *   x: bf16 [batch, hidden], the embeddings. layers: 10 pointers a layer, all bf16: input norm, qkv [(hq + 2 hkv) 128, hidden], q norm, k norm (NULL both: none), o
+ *     [hidden, hq 128], the second norm, gate | up [2 ff, hidden], down [hidden, ff] (row-major), k cache, v cache. The new token's key and value are stored.
+ *   hidden_out: fp32 [batch, hidden], the last layer's output rounded to bf16 (one slab of nvl_add_rmsnorm_splitk); residual_out: bf16 [batch, hidden].
+ *   context_lens <= 0: a row that fills up a captured step. patience: how often a workgroup looks whether all run together before the shares are dealt (0: once). */
+size_t nvl_decode_step_workspace_bytes(int64_t batch, int num_layers, int hidden, int ff, int num_q_heads, int num_kv_heads);
+int nvl_decode_step(const void* x, const void* const* layers, int num_layers, float eps, const float* cos_sin, int64_t max_pos, const int32_t* block_tables,
+                    int64_t bt_stride, const int32_t* context_lens, int64_t batch, int hidden, int ff, int num_q_heads, int num_kv_heads, int block_size,
+                    float softmax_scale, float* hidden_out, void* residual_out, void* workspace, size_t workspace_bytes, int patience, void* stream);
+
 /* Fused split-K reduction + residual add + RMSNorm: replaces
  * RMSNorm.add_rms_forward (layers/layernorm.py:28-40) when its input is the
  * fp32 partials of nvl_linear_decode mode 2:

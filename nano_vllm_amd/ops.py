@@ -33,6 +33,9 @@ SIGNATURES = {
                                 c_void_p]),
     "nvl_pack_weight_tiles": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "nvl_norm_linear": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
+    "nvl_decode_step_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int, c_int, c_int]),
+    "nvl_decode_step": (c_int, [c_void_p, c_void_p, c_int, c_float, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                c_float, c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_void_p]),
     "nvl_add_rmsnorm_splitk": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_float, c_void_p]),
     "nvl_silu_mul": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p]),
     "nvl_rope_neox": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p]),
@@ -304,6 +307,49 @@ def norm_linear(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: tor
     _check(lib().nvl_norm_linear(x.data_ptr(), slabs, residual.data_ptr() if residual is not None else None, norm_weight.data_ptr(), eps,
                                  weight.data_ptr(), out.data_ptr(), new.data_ptr(), m, n, k, 1 if silu else 0, _stream()))
     return out, new
+
+
+_step_bytes: dict[tuple, int] = {}
+DECODE_STEP_MAX_ROWS = 4
+
+
+def decode_step_bytes(rows: int, layers: int, hidden: int, ff: int, num_q_heads: int, num_kv_heads: int) -> int:
+    """Workspace of decode_step; 0: it does not take the step."""
+    key = (rows, layers, hidden, ff, num_q_heads, num_kv_heads)
+    r = _step_bytes.get(key)
+    if r is None:
+        r = _step_bytes[key] = lib().nvl_decode_step_workspace_bytes(*key)
+    return r
+
+
+def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor, block_tables: torch.Tensor, context_lens: torch.Tensor, ff: int, num_q_heads: int,
+                scale: float, patience: int = 200) -> tuple[torch.Tensor, torch.Tensor]:
+    """All layers of a decode step of up to four sequences in one launch. layers: per layer (input norm, qkv, q norm | None, k norm | None, o, second norm, gate | up, down
+    weights, k cache, v cache). Returns the last layer's output as a slab [1, M, hidden] of add_rmsnorm_splitk, and the residual [M, hidden]."""
+    _dev(x, "x")
+    m, hidden = x.shape
+    kc = layers[0][8]
+    hkv, block_size = kc.shape[1], kc.shape[2]
+    shapes = ((hidden,), ((num_q_heads + 2 * hkv) * 128, hidden), (128,), (128,), (hidden, num_q_heads * 128), (hidden,), (2 * ff, hidden), (hidden, ff), kc.shape, kc.shape)
+    assert x.dtype == torch.bfloat16 and x.is_contiguous() and kc.dim() == 4 and kc.shape[3] == 128
+    assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1 and block_tables.shape[0] >= m and context_lens.dtype == torch.int32 and context_lens.shape[0] >= m
+    assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[1] == 128
+    pointers = (c_void_p * (10 * len(layers)))()
+    at = 0
+    for layer in layers:
+        for t, shape in zip(layer, shapes):
+            if t is not None:
+                assert t.shape == shape and t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device, (t.shape, shape, t.dtype)
+                pointers[at] = t.data_ptr()
+            at += 1
+    need = decode_step_bytes(m, len(layers), hidden, ff, num_q_heads, hkv)
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
+    out = torch.empty((1, m, hidden), dtype=torch.float32, device=x.device)
+    residual = torch.empty((m, hidden), dtype=torch.bfloat16, device=x.device)
+    _check(lib().nvl_decode_step(x.data_ptr(), pointers, len(layers), eps, cos_sin.data_ptr(), cos_sin.shape[0], block_tables.data_ptr(), block_tables.stride(0),
+                                 context_lens.data_ptr(), m, hidden, ff, num_q_heads, hkv, block_size, scale, out.data_ptr(), residual.data_ptr(), ws.data_ptr(),
+                                 ws.numel(), patience, _stream()))
+    return out, residual
 
 
 def add_rmsnorm_splitk(partials: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,

@@ -21,8 +21,12 @@ the parts of a context, beyond them a launch of its own):
 
    [add+RMSNorm + qkv GEMM] -> [norm + RoPE + KV store + attention, split merged in LDS] -> o GEMM
    -> [add+RMSNorm + gate_up GEMM + SiLU*mul] -> down GEMM
+
+and up to 4 rows of Qwen3-0.6B's shape all layers are one launch (decode_step.hip).
 """
 from __future__ import annotations
+
+import os
 
 import torch
 from torch import nn
@@ -32,7 +36,7 @@ from .api import model_geometry
 from .attn_meta import get_context, plain_calls
 from .layers import (Attention, MergedColumnParallelLinear, ParallelLMHead, QKVParallelLinear, RMSNorm,
                      RowParallelLinear, SiluAndMul, VocabParallelEmbedding, get_rope)
-from . import ops_seq, tp
+from . import ops, ops_seq, tp
 
 
 class Qwen3Attention(nn.Module):
@@ -100,6 +104,34 @@ def _watched(*modules) -> bool:
     return bool(_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or any(m._forward_hooks or m._forward_pre_hooks for m in modules))
 
 
+def _plain(module, kind) -> bool:
+    """Is the module of that class itself, with no call of its own and nobody watching?"""
+    return type(module) is kind and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+
+
+def _layer_weights(layer, eps, table, hq: int, hkv: int, scale: float):
+    """What ops.decode_step takes of a layer, or None: a layer that is not as this file makes it, or not as the others are."""
+    if not _plain(layer, Qwen3DecoderLayer) or _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks:
+        return None
+    attn, mlp, n1, n2 = layer.self_attn, layer.mlp, layer.input_layernorm, layer.post_attention_layernorm
+    if not (_plain(attn, Qwen3Attention) and _plain(mlp, Qwen3MLP) and _plain(n1, RMSNorm) and _plain(n2, RMSNorm)):
+        return None
+    a, qkv, o, gate_up, down = attn.attn, attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj
+    if not (_plain(a, Attention) and _plain(qkv, QKVParallelLinear) and _plain(o, RowParallelLinear) and _plain(gate_up, MergedColumnParallelLinear)
+            and _plain(down, RowParallelLinear) and _plain(mlp.act_fn, SiluAndMul) and qkv.tp_size == 1
+            and qkv.bias is None and o.bias is None and gate_up.bias is None and down.bias is None):
+        return None
+    qn = kn = None
+    if attn.has_qk_norm:
+        if not (_plain(attn.q_norm, RMSNorm) and _plain(attn.k_norm, RMSNorm)) or attn.eps != eps:
+            return None
+        qn, kn = attn.q_norm.weight, attn.k_norm.weight
+    if (n1.eps != eps or n2.eps != eps or attn.num_heads != hq or attn.num_kv_heads != hkv or a.num_heads != hq or a.num_kv_heads != hkv or a.scale != scale
+            or attn.rotary_emb.cos_sin_cache is not table or a.k_cache.numel() == 0):
+        return None
+    return n1.weight, qkv.weight, qn, kn, o.weight, n2.weight, gate_up.weight, down.weight, a.k_cache, a.v_cache
+
+
 class Qwen3DecoderLayer(nn.Module):
 
     def __init__(self, config, geo: dict):
@@ -130,6 +162,14 @@ class Qwen3DecoderLayer(nn.Module):
         return self.mlp(hidden_states), residual
 
 
+# NVL_DECODE_STEP=0 keeps the launches of small decode steps apart (A/B measurements)
+_DECODE_STEP = os.environ.get("NVL_DECODE_STEP", "1") != "0"
+# The longest context (max_context) up to which that many sequences' layers go in one launch: its attention has 30, 14, 8 and 6 parts a context, whatever the others are, and
+# the launches of their own share all contexts out. Qwen3-0.6B, us a step, apart / in one: one sequence of 8,000, 16,000, 30,000 tokens 1012 1147 1418 / 704 885 1207; two
+# of 8,000 1105 / 912; three of 4,000 1044 / 898; four of 4,000 1112 / 1022, of 8,000 1400 / 1465, of 100 to 16,000 1555 / 2181. Shorter contexts: decode_step.hip.
+_DECODE_STEP_CONTEXT = {1: 32768, 2: 8192, 3: 4096, 4: 4096}
+
+
 class Qwen3Model(nn.Module):
 
     def __init__(self, config, geo: dict):
@@ -138,11 +178,43 @@ class Qwen3Model(nn.Module):
         self.layers = nn.ModuleList([Qwen3DecoderLayer(config, geo) for _ in range(config.num_hidden_layers)])
         self.norm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
+    def _decode_step(self, x: torch.Tensor):
+        """All layers of a decode step of few sequences in one launch (decode_step.hip): (the last layer's output, the residual), or None where the layers are called: other
+        steps and shapes, and layers of which somebody watches, replaces or extends a part."""
+        ctx = get_context()
+        if (not _DECODE_STEP or ctx.is_prefill or x.dim() != 2 or not 1 <= x.shape[0] <= ops.DECODE_STEP_MAX_ROWS or x.dtype != torch.bfloat16 or not x.is_cuda
+                or not x.is_contiguous() or ctx.shared_prefix or ctx.context_lens is None or ctx.block_tables is None or not len(self.layers)):
+            return None
+        first = self.layers[0]
+        if type(first) is not Qwen3DecoderLayer or type(first.self_attn) is not Qwen3Attention:
+            return None
+        attn, eps, table = first.self_attn, first.input_layernorm.eps, first.self_attn.rotary_emb.cos_sin_cache
+        ff = first.mlp.down_proj.weight.shape[1] if type(first.mlp) is Qwen3MLP else 0
+        hq, hkv, scale, fused = attn.num_heads, attn.num_kv_heads, attn.attn.scale, attn.attn.fuses_decode_step(ctx)
+        if not fused or not ops.decode_step_bytes(x.shape[0], len(self.layers), x.shape[1], ff, hq, hkv):
+            return None
+        tables, block_size, ws = ctx.block_tables, attn.attn.k_cache.shape[2], ctx.decode_workspace
+        max_context = ctx.max_context or tables.shape[1] * block_size
+        if (max_context > _DECODE_STEP_CONTEXT[x.shape[0]] or block_size % 32 or tables.stride(0) * block_size < max_context or tables.stride(1) != 1
+                or ws is not None and ws.numel() * ws.element_size() < ops.paged_attn_decode_workspace_bytes(x.shape[0], hq, max_context)):
+            return None                          # (what the layers' own launches refuse they still do)
+        layers = []
+        for layer in self.layers:
+            w = _layer_weights(layer, eps, table, hq, hkv, scale)
+            if w is None or any(t is not None and (t.dtype != torch.bfloat16 or not t.is_contiguous()) for t in w):
+                return None
+            layers.append(w)
+        return ops.decode_step(x, layers, eps, table, ctx.block_tables, ctx.context_lens, ff, hq, scale)
+
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         hidden_states = self.embed_tokens(input_ids)
         residual = None
-        for layer in self.layers:
-            hidden_states, residual = layer(positions, hidden_states, residual)
+        both = self._decode_step(hidden_states)
+        if both is not None:
+            hidden_states, residual = both
+        else:
+            for layer in self.layers:
+                hidden_states, residual = layer(positions, hidden_states, residual)
         hidden_states, _ = self.norm(hidden_states, residual)
         return hidden_states
 

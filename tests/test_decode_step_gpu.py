@@ -1,0 +1,203 @@
+"""All layers of a small decode step in one launch (nvl_decode_step): against the step in float64 on the same 16-bit inputs, at the edges of its cuts (chunks of 32 keys, 30, 14, 8 and
+6 parts, batches of 128 keys) and of its shapes; with its shares dealt instead of fixed; and what keeps the layers' own calls."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+W = 1024
+
+
+def rand(g, *s, scale=1.0):
+    return (scale * torch.randn(*s, generator=g, device="cuda")).bfloat16()
+
+
+def step_inputs(lens, hq=16, ff=3072, layers=2, block=256, norms=True, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    hkv = hq // 2
+    need = [max(1, -(-n // block)) for n in lens]
+    table = torch.full((len(lens), max(need)), -1, dtype=torch.int32)
+    ids = torch.randperm(sum(need), generator=torch.Generator().manual_seed(seed)).to(torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        if lens[i] > 0:
+            table[i, :n] = ids[at:at + n]
+        at += n
+    every = []
+    for _ in range(layers):
+        norm = lambda n: (1 + 0.1 * torch.randn(n, generator=g, device="cuda")).bfloat16()
+        cache = [rand(g, sum(need), hkv, block, 128) for _ in range(2)]
+        for i, n in enumerate(lens):               # what a page holds behind the context, its new token's place among it, need not be finite
+            if n > 0 and n % block:
+                for c in cache:
+                    c[table[i, (n - 1) // block], :, n - 1 - (n - 1) // block * block:] = float("nan")
+        every.append((norm(W), rand(g, (hq + 2 * hkv) * 128, W, scale=W ** -0.5), norm(128) if norms else None, norm(128) if norms else None,
+                      rand(g, W, hq * 128, scale=(hq * 128) ** -0.5), norm(W), rand(g, 2 * ff, W, scale=W ** -0.5), rand(g, W, ff, scale=ff ** -0.5), *cache))
+    f = 1e6 ** (-torch.arange(0, 128, 2, dtype=torch.float64) / 128)
+    ang = torch.arange(8192, dtype=torch.float64)[:, None] * f
+    cs = torch.cat([ang.cos(), ang.sin()], 1).float().cuda()
+    return rand(g, len(lens), W), every, cs, table.cuda(), torch.tensor(lens, dtype=torch.int32).cuda(), ff, hq
+
+
+def exact(x, layers, cs, table, lens, ff, hq, block):
+    """(last layer's output, residual, new keys and values of every layer) in float64."""
+    def rms(v, w):
+        return v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-6) * w.double()
+    v, news = x.double(), []
+    hkv = hq // 2
+    for n1, wqkv, qn, kn, wo, n2, wgu, wd, kc, vc in layers:
+        z = rms(v, n1) @ wqkv.double().T
+        att, new = torch.zeros(len(v), hq * 128, dtype=torch.float64, device="cuda"), []
+        for b, n in enumerate(lens.tolist()):
+            if n <= 0:
+                new.append(None)
+                continue
+            def turn(t, w):
+                t = t.view(-1, 128)
+                if w is not None:
+                    t = rms(t, w)
+                c, s = cs[n - 1, :64].double(), cs[n - 1, 64:].double()
+                return torch.cat([t[:, :64] * c - t[:, 64:] * s, t[:, 64:] * c + t[:, :64] * s], 1)
+            q, k, val = turn(z[b, :hq * 128], qn), turn(z[b, hq * 128:(hq + hkv) * 128], kn), z[b, (hq + hkv) * 128:].view(hkv, 128)
+            new.append((k, val))
+            pos = torch.arange(n - 1, device="cuda")
+            blk = table[b, pos // block].long()
+            ks = torch.cat([kc[blk, :, pos % block].double(), k[None]]).repeat_interleave(2, 1)
+            vs = torch.cat([vc[blk, :, pos % block].double(), val[None]]).repeat_interleave(2, 1)
+            p = torch.softmax((ks * q).sum(-1) * 128 ** -0.5, 0)
+            att[b] = (p[..., None] * vs).sum(0).flatten()
+        v1 = v + att @ wo.double().T
+        gu = rms(v1, n2) @ wgu.double().T
+        y = (torch.nn.functional.silu(gu[:, :ff]) * gu[:, ff:]) @ wd.double().T
+        v = v1 + y
+        news.append(new)
+    return y, v1, news
+
+
+def rel(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("lens,hq,ff,block,norms", [
+    ([1], 16, 3072, 256, True), ([32], 16, 3072, 256, True), ([33], 16, 3072, 16, False), ([960], 16, 3072, 256, True), ([961], 16, 3072, 256, True),
+    ([3841], 16, 3072, 256, True), ([7777], 8, 1024, 256, True), ([448, 449], 16, 3072, 256, True), ([0, 64], 16, 2048, 48, True), ([1800, 2], 8, 3072, 256, False),
+    ([256, 257, 1], 16, 3072, 256, True), ([31, 0, 2100], 8, 2048, 32, True), ([192, 193, 768, 1537], 16, 3072, 256, True), ([1, 2, 3, 4], 16, 1024, 256, True),
+    ([0, 0, 0, 5], 8, 1024, 256, True)])
+@pytest.mark.parametrize("patience", [200, 0])
+def test_step(lens, hq, ff, block, norms, patience):
+    """patience 0: a workgroup looks once whether all are there, so the shares are dealt (unless the last one came first)."""
+    from nano_vllm_amd import ops
+    x, layers, cs, table, ctx, ff, hq = step_inputs(lens, hq, ff, 2, block, norms, seed=len(lens) + sum(lens))
+    want, v1, news = exact(x, layers, cs, table, ctx, ff, hq, block)
+    before = [(l[8].clone(), l[9].clone()) for l in layers]
+    out, residual = ops.decode_step(x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5, patience=patience)
+    assert out.shape == (1, len(lens), W) and out.dtype == torch.float32
+    # about eight roundings to 8 bits a layer on the way, 2^-9 / sqrt(3) each: 0.0045 over two layers
+    assert rel(out[0], want) <= 2.0 ** -7 and rel(residual, v1) <= 2.0 ** -7
+    for l, layer in enumerate(layers):             # the new token's key and value, and nothing else
+        for b, n in enumerate(lens):
+            if n > 0:
+                blk, at = int(table[b, (n - 1) // block]), (n - 1) % block
+                for i in range(2):
+                    assert rel(layer[8 + i][blk, :, at], news[l][b][i]) <= 2.0 ** -7
+                    before[l][i][blk, :, at] = layer[8 + i][blk, :, at]
+        for i in range(2):
+            assert torch.equal(layer[8 + i].view(torch.int16), before[l][i].view(torch.int16))
+
+
+@pytest.mark.parametrize("lens", [[700], [5, 900], [1, 300, 1500], [300, 31, 900, 2000]])
+def test_dealt_shares_give_the_same_bits_and_so_do_replays(lens):
+    from nano_vllm_amd import ops
+    x, layers, cs, table, ctx, ff, hq = step_inputs(lens, layers=3)
+    args = (x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)
+    fixed = ops.decode_step(*args)
+    dealt = ops.decode_step(*args, patience=0)
+    assert torch.equal(fixed[0], dealt[0]) and torch.equal(fixed[1], dealt[1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = ops.decode_step(*args)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(held[0], fixed[0]) and torch.equal(held[1], fixed[1])
+        held[0].zero_()
+        again = ops.decode_step(*args)
+        assert torch.equal(again[0], fixed[0])
+
+
+def test_a_row_that_is_no_number_stays_its_own():
+    from nano_vllm_amd import ops
+    x, layers, cs, table, ctx, ff, hq = step_inputs([40, 500, 33])
+    clean = ops.decode_step(x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)[0].clone()
+    bad = x.clone()
+    bad[1, 7] = float("nan")
+    bad.view(torch.int16)[1, 8] = -1               # the word that means "not written", as a NaN of the input
+    got = ops.decode_step(bad, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)[0]
+    assert got[0, 1].isnan().all() and torch.equal(got[0, [0, 2]], clean[0, [0, 2]])
+
+
+def test_what_is_not_covered_is_refused():
+    from nano_vllm_amd import ops
+    assert ops.decode_step_bytes(4, 28, 1024, 3072, 16, 8) > 0
+    for shape in [(5, 28, 1024, 3072, 16, 8), (0, 28, 1024, 3072, 16, 8), (1, 41, 1024, 3072, 16, 8), (1, 28, 2048, 6144, 16, 8), (1, 28, 1024, 4096, 16, 8),
+                  (1, 28, 1024, 3072, 16, 16), (1, 28, 1024, 3072, 32, 16)]:
+        assert ops.decode_step_bytes(*shape) == 0
+    x, layers, cs, table, ctx, ff, hq = step_inputs([3] * 5)
+    with pytest.raises(ops.NvlError, match="rows"):
+        ops.decode_step(x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)
+
+
+@pytest.mark.parametrize("touch", ["nothing", "layer", "attention", "mlp", "norm", "projection", "global", "own call", "rows", "context", "refused"])
+def test_calls_that_somebody_watches_are_made(touch, monkeypatch):
+    from nano_vllm_amd import ops, qwen3
+    from nano_vllm_amd.attn_meta import reset_context, set_context
+    from types import SimpleNamespace
+    config = SimpleNamespace(hidden_size=1024, intermediate_size=1024, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=4, head_dim=128, rms_norm_eps=1e-6,
+                             vocab_size=512, hidden_act="silu", max_position_embeddings=8192, rope_theta=1e6, tie_word_embeddings=True, attention_bias=False)
+    torch.manual_seed(1)
+    torch.set_default_dtype(torch.bfloat16)
+    torch.set_default_device("cuda")
+    try:
+        model = qwen3.Qwen3ForCausalLM(config)
+        for p in model.parameters():
+            p.data.copy_(1 + 0.1 * torch.randn(p.shape) if p.dim() == 1 else torch.randn(p.shape) * p.shape[-1] ** -0.5)
+    finally:
+        torch.set_default_device("cpu")
+        torch.set_default_dtype(torch.float32)
+    rows = 5 if touch == "rows" else 2
+    for m in model.modules():
+        if isinstance(m, qwen3.Attention):
+            m.k_cache, m.v_cache = (torch.randn(rows, 4, 256, 128, device="cuda").bfloat16() for _ in range(2))
+    layer, seen, calls, width = model.model.layers[1], [], [], 40 if touch == "context" else 1
+    watched = {"layer": layer, "attention": layer.self_attn, "mlp": layer.mlp, "norm": layer.post_attention_layernorm, "projection": layer.self_attn.o_proj}
+    hook = lambda *a: seen.append(1)
+    handle = watched[touch].register_forward_hook(hook) if touch in watched else None
+    if touch == "global":
+        handle = torch.nn.modules.module.register_module_forward_hook(hook)
+    if touch == "own call":
+        inner = layer.mlp.forward
+        layer.mlp.forward = lambda *a, **k: (seen.append(1), inner(*a, **k))[1]
+    ran = ops.decode_step
+    monkeypatch.setattr(ops, "decode_step", lambda *a, **k: (calls.append(1), ran(*a, **k))[1])
+    ids, pos = torch.arange(rows).cuda(), torch.full((rows,), 99).cuda()
+
+    def step():
+        set_context(False, slot_mapping=None, context_lens=torch.full((rows,), 100, dtype=torch.int32).cuda(),
+                    block_tables=torch.nn.functional.pad(torch.arange(rows, dtype=torch.int32).cuda()[:, None], (0, width - 1), value=-1),
+                    max_context=width * 256 if touch != "refused" else 512)
+        out = model(ids, pos)
+        reset_context()
+        return out
+    try:
+        with torch.inference_mode():
+            if touch == "refused":               # a block table too narrow, as before
+                with pytest.raises(ops.NvlError, match="narrower"):
+                    step()
+                return
+            got = step()
+            monkeypatch.setattr(qwen3, "_DECODE_STEP", False)
+            apart = step()
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert bool(calls) == (touch == "nothing")
+    assert rel(got, apart.double()) <= 2.0 ** -6   # two ways of two layers' roundings
