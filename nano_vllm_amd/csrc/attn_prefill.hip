@@ -21,7 +21,7 @@
 // The (sequence, q-block) of a workgroup is found on device from cu_seqlens_q — in registers (shuffle scan + ballot +
 // readlane, one global round trip, no barrier) for launches of up to 64 sequences, through an LDS prefix + binary
 // search beyond that — so no host-side tile list is needed.
-#include "common.h"
+#include "rope_common.h"
 #include <stdlib.h>
 #include <type_traits>
 
@@ -72,7 +72,9 @@ struct RawQ {
   float eps;
 };
 
-template <bool PAGED, bool KV8, int NW, bool RAWQ = false>
+// PAIR (even hq / hkv): a workgroup takes 64 query rows of two heads of a kv group, a wave 16 rows of both, so a row's table entries are fetched once for both, fewer rows of a
+// workgroup lie behind their sequence's end, and fewer keys behind a row. 26 prompts of 100 to 1,024 tokens (15,600 tokens, 16 heads over 8), us: 118 with 128 rows of one head, 112 so.
+template <bool PAGED, bool KV8, int NW, bool RAWQ = false, bool PAIR = false>
 __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int64_t k_tok_stride,
     int64_t v_tok_stride, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k,
@@ -81,6 +83,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // two {K: 64 x 256 B, V: 64 x 320 B} tile buffers, then the tile-lookup scratch
   constexpr int NT = NW * 64;                            // threads per workgroup
+  constexpr int kRows = PAIR ? kQBlk / 2 : kQBlk, kWaveRows = PAIR ? 16 : 32, kHeads = PAIR ? 2 : 1;
   int* wsum = reinterpret_cast<int*>(smem + 2 * kTileBytes);
   int* pre = wsum + 8;                                  // [num_seqs + 1]
 
@@ -104,17 +107,17 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   int head, tile_rank;
   // block id -> (q-head, rank of the tile in the longest-first list) under the XCD-aware numbering
   auto xcd_decode = [&](int b, int& head_, int& rank_) {
-    const int G = hq / hkv;
+    const int G = hq / hkv / kHeads;
     const int xcd = b & 7, slot = b >> 3;
     const int gi = slot / G, g = slot - gi * G;
     const int j = gi * 8 + xcd;                    // (tile, kv-head) group, longest tiles first
     rank_ = j / hkv;
-    head_ = (j - rank_ * hkv) * G + g;
+    head_ = ((j - rank_ * hkv) * G + g) * kHeads;
   };
   if (xcd_map) {
     xcd_decode(blockIdx.x, head, tile_rank);
   } else {
-    head = NW == 8 ? blockIdx.x * 2 + hsub : blockIdx.x;
+    head = NW == 8 ? blockIdx.x * 2 + hsub : blockIdx.x * kHeads;
     tile_rank = blockIdx.y;
   }
   // ---- which (sequence, q-block) is this workgroup? ------------------------------------
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
       a0 = cu_q[lane]; a1 = cu_q[lane + 1];
       b0 = cu_k[lane]; b1 = cu_k[lane + 1];
     }
-    val = (a1 - a0 + kQBlk - 1) / kQBlk;
+    val = (a1 - a0 + kRows - 1) / kRows;
     sc = val;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
     for (int base = 0; base < num_seqs; base += NT) {
       const int i = base + tid;
       int val = 0;
-      if (i < num_seqs) val = (cu_q[i + 1] - cu_q[i] + kQBlk - 1) / kQBlk;
+      if (i < num_seqs) val = (cu_q[i + 1] - cu_q[i] + kRows - 1) / kRows;
       int s = val;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -207,28 +210,43 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   auto item_geometry = [&]() {
     kvh = head / (hq / hkv);
     off = lk - lq;  // bottom-right alignment: query i sees keys j <= i + off
-    qi = qblk * kQBlk + wave * 32 + qcol;
+    qi = qblk * kRows + wave * kWaveRows + (qcol & (kWaveRows - 1));
     q_valid = qi < lq;
     qi_c = q_valid ? qi : lq - 1;
-    kv_end = min(lk, qblk * kQBlk + kQBlk + off);  // keys visible to the block's last query
+    kv_end = min(lk, qblk * kRows + kRows + off);  // keys visible to the block's last query
   };
   item_geometry();
 
   // ---- Q fragments: B operand of S^T = K.Q^T : lane (query, hi) holds d = ds*16 + 8*hi .. +8
-  bf16x8_t qf[8], qw[RAWQ ? 8 : 1];
+  bf16x8_t qf[8];
+  // RAWQ: rows as they lie in memory, 16 lanes a row, four rows a request (and its wave's 32 positions, a lane each); they become fragments by way of LDS
+  u32x4_t qraw[RAWQ ? 8 : 1], qnorm = {0u, 0u, 0u, 0u};
+  constexpr int kTurns = RAWQ ? kWaveRows / 4 : 1;
+  RopeRegs turn[kTurns];
   int64_t qpos = 0;
+  auto clamped = [&](int64_t p) { return p < 0 ? (int64_t)0 : (p >= raw.max_pos ? raw.max_pos - 1 : p); };
+  auto load_turn = [&](int it, int64_t p) {
+    turn[it] = load_rope_regs(raw.cos_sin + p * 128, lane & 15);
+  };
   auto load_q = [&](int q0_, int lq_, int qblk_, int head_) {
-    int row = qblk_ * kQBlk + wave * 32 + qcol;
-    row = row < lq_ ? row : lq_ - 1;
-    const bf16_t* qp = RAWQ ? q + (int64_t)(q0_ + row) * raw.tok_stride + head_ * 128 + hi * 8 : q + ((int64_t)(q0_ + row) * hq + head_) * 128 + hi * 8;
-    if constexpr (RAWQ) qpos = raw.positions[q0_ + row];
-#pragma unroll
-    for (int ds = 0; ds < 8; ++ds) qf[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(qp + ds * 16));
+    const int first = qblk_ * kRows + wave * kWaveRows;
+    const auto row_of = [&](int r) { return min(first + (r & (kWaveRows - 1)), lq_ - 1); };        // r: of the wave's 32 (query, head)
+    const auto head_of = [&](int r) { return head_ + r / kWaveRows; };
     if constexpr (RAWQ) {
-      if (raw.norm_w != nullptr) {
+      qpos = raw.positions[q0_ + row_of(qcol)];
 #pragma unroll
-        for (int ds = 0; ds < 8; ++ds) qw[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(raw.norm_w + ds * 16 + hi * 8));
+      for (int it = 0; it < 8; ++it) {
+        const int r = it * 4 + (lane >> 4);
+        qraw[it] = *reinterpret_cast<const u32x4_t*>(q + (int64_t)(q0_ + row_of(r)) * raw.tok_stride + head_of(r) * 128 + (lane & 15) * 8);
       }
+      if (raw.norm_w != nullptr) qnorm = *reinterpret_cast<const u32x4_t*>(raw.norm_w + (lane & 15) * 8);
+      // the table's rows at the positions that a query has in its context, without waiting for those that it is given
+#pragma unroll
+      for (int it = 0; it < kTurns; ++it) load_turn(it, clamped(row_of(it * 4 + (lane >> 4)) + off));
+    } else {
+      const bf16_t* qp = q + ((int64_t)(q0_ + row_of(qcol)) * hq + head_of(qcol)) * 128 + hi * 8;
+#pragma unroll
+      for (int ds = 0; ds < 8; ++ds) qf[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(qp + ds * 16));
     }
   };
   load_q(q0, lq, qblk, head);
@@ -341,9 +359,10 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   // it only helps staging the tiles; +3-4 % on batches of short sequences)
   int wave_kmax_s, wave_kmin_s;         // wave-uniform copies on the scalar side (scalar branches instead of exec masks)
   auto wave_frontier = [&]() {
-    const bool wave_has_rows = qblk * kQBlk + wave * 32 < lq;
-    const int wave_kmax = wave_has_rows ? min(qblk * kQBlk + wave * 32 + 31, lq - 1) + off : -1;
-    const int wave_kmin = min(qblk * kQBlk + wave * 32, lq - 1) + off;   // ... and all of them see keys <= wave_kmin
+    const int first = qblk * kRows + wave * kWaveRows;
+    const bool wave_has_rows = first < lq;
+    const int wave_kmax = wave_has_rows ? min(first + kWaveRows - 1, lq - 1) + off : -1;
+    const int wave_kmin = min(first, lq - 1) + off;   // ... and all of them see keys <= wave_kmin
     wave_kmax_s = __builtin_amdgcn_readfirstlane(wave_kmax);
     wave_kmin_s = __builtin_amdgcn_readfirstlane(wave_kmin);
   };
@@ -354,44 +373,46 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   // loop head and puts vmcnt waits on their first uses inside QK^T, which drain whatever tile loads are in flight).
   stage_load(0);
   if constexpr (RAWQ) {
-    // norm and rotation as rope_common.h has them (roundings included): the lane holds entries ds * 16 + 8 hi .. + 7 and their partners 64 further on; the
-    // two halves of a row meet once
 #pragma clang fp contract(off)
-    const int64_t p = qpos < 0 ? 0 : (qpos >= raw.max_pos ? raw.max_pos - 1 : qpos);
-    const float* cs = raw.cos_sin + p * 128 + hi * 8;
-    f32x4_t c[4][2], sn[4][2];
+    // Norm and rotation of rope_common.h on the rows as they lie, then through this wave's 8 KB of the second tile buffer (swizzled as K's rows; nothing is written there before
+    // the first barrier behind the fragments' reads). A lane that fetched its own query's fragments and table entries, 32 rows a request, kept the vector cache busy
+    // with 768 lines a wave: 7.6 us from there to the first tile, of 23 a workgroup, 6.6 so (26 prompts of 100 to 1,024 tokens; 124 us in all, 118 so).
+    unsigned char* qrows = smem + kTileBytes + wave * 8192;
+    const int sub = lane & 15;
+    const int64_t p = clamped(qpos);
+    if (__any(p != clamped(qi_c + off))) {               // other positions than those
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds)
+      for (int it = 0; it < kTurns; ++it) load_turn(it, (int64_t)__shfl((long long)p, it * 4 + (lane >> 4), 64));
+    }
+    float wf[8];
+    unpack8(qnorm, wf);
+    if (sub < 8) {                                       // first half: x1 cos - x2 sin; second: x2 cos + x1 sin
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        c[ds][j] = *reinterpret_cast<const f32x4_t*>(cs + ds * 16 + j * 4);
-        sn[ds][j] = *reinterpret_cast<const f32x4_t*>(cs + 64 + ds * 16 + j * 4);
-      }
-    float rstd = 1.f;
-    if (raw.norm_w != nullptr) {
-      float ss = 0.f;
-#pragma unroll
-      for (int ds = 0; ds < 8; ++ds)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ss += (float)qf[ds][i] * (float)qf[ds][i];
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
-      ss = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-      rstd = rsqrtf(ss * (1.f / 128.f) + raw.eps);
+      for (int it = 0; it < kTurns; ++it) turn[it].s0 = -turn[it].s0, turn[it].s1 = -turn[it].s1;
     }
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds)
+    for (int it = 0; it < 8; ++it) {
+      const int row = it * 4 + (lane >> 4);
+      const RopeRegs& t = turn[it % kTurns];
+      float x[8], o[8];
+      unpack8(qraw[it], x);
+      if (raw.norm_w != nullptr) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
+        const float rstd = rsqrtf(row16_allreduce_sum(ss) * (1.f / 128.f) + raw.eps);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = round_bf16(x[i] * rstd * wf[i]);
+      }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float x1 = (float)qf[ds][i], x2 = (float)qf[ds + 4][i];
-        if (raw.norm_w != nullptr) {
-          x1 = round_bf16(x1 * rstd * (float)qw[ds][i]);
-          x2 = round_bf16(x2 * rstd * (float)qw[RAWQ ? ds + 4 : 0][i]);
-        }
-        const float co = c[ds][i >> 2][i & 3], si = sn[ds][i >> 2][i & 3];
-        const float a = x1 * co, b = x2 * si, a2 = x2 * co, b2 = x1 * si;
-        qf[ds][i] = (bf16_t)(a - b);
-        qf[ds + 4][i] = (bf16_t)(a2 + b2);
+        const float a = x[i] * (i < 4 ? t.c0[i & 3] : t.c1[i & 3]), b = row16_ror8(x[i]) * (i < 4 ? t.s0[i & 3] : t.s1[i & 3]);
+        o[i] = a + b;
       }
+      *reinterpret_cast<u32x4_t*>(qrows + row * kKRowB + ((sub ^ (row & 15)) << 4)) = pack8(o);
+    }
+#pragma unroll
+    for (int ds = 0; ds < 8; ++ds) qf[ds] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(qrows + kslot[ds]));
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), expcnt / lgkmcnt untouched
   // a (no-op) use of the Q fragments HERE: without it LLVM sinks their loads into the loop preheader, behind this wait
@@ -542,12 +563,12 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   const float inv = 1.f / l_tot;
   // optional log-sum-exp of the scaled scores per (query, head), natural log (flash-attn's softmax_lse): the running
   // max / sum live in the log2 domain here
-  if (lse != nullptr && q_valid && hi == 0) lse[(int64_t)(q0 + qi) * hq + head] = 0.6931471805599453f * (m_run + log2f(l_tot));
+  if (lse != nullptr && q_valid && hi == 0) lse[(int64_t)(q0 + qi) * hq + head + qcol / kWaveRows] = 0.6931471805599453f * (m_run + log2f(l_tot));
   // A lane holds d = db*32 + 8*rg + 4*hi + (0..3) of its query row: 8 bytes per (db, rg), the other half-wave the 8
   // bytes next to them. One v_permlane32_swap per dword trades halves between two neighbouring groups, after which
   // every lane owns 16 contiguous bytes: 8 dwordx4 stores per lane instead of 16 dwordx2 (cdna_hip_programming.md T21;
   // the store tail of a short sequence's workgroup is issue-bound).
-  bf16_t* op = out + ((int64_t)(q0 + qi_c) * hq + head) * 128 + 8 * hi;
+  bf16_t* op = out + ((int64_t)(q0 + qi_c) * hq + head + qcol / kWaveRows) * 128 + 8 * hi;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -597,7 +618,9 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
                 "nvl_attn_prefill_varlen: bad K/V token strides");
   }
   if (total_q == 0 || num_seqs == 0) return NVL_OK;
-  const int64_t tiles = (total_q + kQBlk - 1) / kQBlk + num_seqs;  // upper bound on sum ceil(Lq/128)
+  const bool pair = raw && num_q_heads / num_kv_heads % 2 == 0;
+  const int rows = pair ? kQBlk / 2 : kQBlk, heads = pair ? 2 : 1;
+  const int64_t tiles = (total_q + rows - 1) / rows + num_seqs;  // upper bound on sum ceil(Lq / rows)
   NVL_REQUIRE(tiles < (1ll << 31), "nvl_attn_prefill_varlen: too many query tiles");
   const size_t lds = (size_t)2 * kTileBytes + 8 * sizeof(int) + (size_t)(num_seqs + 1) * sizeof(int);
   const float sl2 = softmax_scale * 1.4426950408889634f;
@@ -609,7 +632,7 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
   // Workgroup shape (see the kernel): 8 waves (two q-heads share the staged K/V tile) when the launch has long
   // sequences, 4 waves otherwise — measured (profiles/r02_prefill_waves{4,8}.json, TFLOP/s 4 / 8 waves): 1 x 16384
   // 908 / 931 (16/8 heads), 819 / 856 (8/1); 4 x 4096 693 / 718; 8 x 2048 G = 8 741 / 743; but 16 x 1024 497 / 422
-  // and 29 x 561 343 / 326: short sequences have too few tiles per workgroup to amortise the 8-wave barrier.
+  // and 29 x 561 343 / 326: short sequences have too few tiles per workgroup to amortise the 8-wave barrier. (Raw queries: four waves, of two heads where a group has an even number of them.)
   // NVL_PREFILL_WAVES=4|8 forces one shape; 8 needs an even group size Hq / Hkv.
   // Round 3, with the current kernel (profiles/r03_prefill_ab_xcd_*.json, 4-wave shape, two A/B pairs): the XCD-aware
   // numbering is +3...11 % on bench-like / ragged batches of 100-1024-token prompts, +-1 % on the long shapes, -2...4 %
@@ -642,10 +665,10 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
   const bool eight_ok = (num_q_heads / num_kv_heads) % 2 == 0;
   const int xcd_map = xcd_env >= 0 ? xcd_env : ((want == 4 || !eight_ok) && num_seqs <= 64 ? 1 : 0);
   const bool eight = want == 8 && !xcd_map && eight_ok;
-  dim3 grid((unsigned)(eight ? num_q_heads / 2 : num_q_heads), (unsigned)tiles);
+  dim3 grid((unsigned)(eight ? num_q_heads / 2 : num_q_heads / heads), (unsigned)tiles);
   if (xcd_map) {
     const int64_t groups = tiles * num_kv_heads;
-    int64_t blocks = ((groups + 7) / 8) * 8 * (num_q_heads / num_kv_heads);
+    int64_t blocks = ((groups + 7) / 8) * 8 * (num_q_heads / num_kv_heads / heads);
     NVL_REQUIRE(blocks < (1ll << 31), "nvl_attn_prefill_varlen: too many workgroups (%lld)", (long long)blocks);
     grid = dim3((unsigned)blocks, 1);
   } else {
@@ -665,6 +688,10 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
         hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<false, false, 4, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)cap) != hipSuccess ||
         hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<true, false, 4, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)cap) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<false, false, 4, true, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)cap) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_attn_kernel<true, false, 4, true, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)cap) != hipSuccess) {
       nvl_set_error("nvl_attn_prefill_varlen: cannot reserve %zu B of LDS", cap);
       return NVL_ELAUNCH;
@@ -676,7 +703,9 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
   hipLaunchKernelGGL((prefill_attn_kernel<__VA_ARGS__>), grid, dim3(eight ? 512 : 256), lds, s, (const bf16_t*)q,       \
                      (const bf16_t*)k, (const bf16_t*)v, k_tok_stride, v_tok_stride, cu_seqlens_q, cu_seqlens_k,        \
                      block_tables, bt_stride, (bf16_t*)out, num_seqs, num_q_heads, num_kv_heads, block_size, sl2, xcd_map, lse, thr, raw ? *raw : RawQ{})
-  if (raw) {
+  if (pair) {
+    if (paged) NVL_PF_LAUNCH(true, false, 4, true, true); else NVL_PF_LAUNCH(false, false, 4, true, true);
+  } else if (raw) {
     if (paged) NVL_PF_LAUNCH(true, false, 4, true); else NVL_PF_LAUNCH(false, false, 4, true);
   } else if (paged && kv_dtype == NVL_KV_FP8) {
     if (eight) NVL_PF_LAUNCH(true, true, 8); else NVL_PF_LAUNCH(true, true, 4);

@@ -48,3 +48,32 @@ def test_agrees_with_finished_queries(hq, hkv, lens, cached, norm):
             assert torch.equal(got, want)                       # the same roundings throughout
         # the norm's sum is taken in another order: an entry may round to its neighbour (2^-8 of it, and few do)
         assert float((got.double() - want.double()).norm() / want.double().norm()) <= 2.0 ** -9
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (12, 2), (6, 2)])
+@pytest.mark.parametrize("where", ["context", "shifted", "one other", "beyond the table"])
+def test_positions_as_they_are_given(hq, hkv, where):
+    """The table's rows are asked for at a query's place in its context before its position is known: every other position counts all the same. Lengths around the rows of a wave (16) and of a
+    workgroup (64) that takes two heads, and an odd group, whose workgroups take one."""
+    from nano_vllm_amd import ops
+    lens, top = [15, 16, 17, 63, 64, 65, 129, 1], 300
+    g = torch.Generator(device="cuda").manual_seed(hq)
+    n = sum(lens)
+    qkv = torch.randn(n, (hq + 2 * hkv) * 128, generator=g, device="cuda").bfloat16()
+    freq = 1e6 ** (-torch.arange(0, 128, 2, device="cuda").float() / 128)
+    angle = torch.arange(top, device="cuda").float()[:, None] * freq
+    table = torch.cat([angle.cos(), angle.sin()], 1).contiguous()
+    pos = torch.cat([torch.arange(m) for m in lens]).cuda()
+    if where == "shifted":
+        pos += 100
+    elif where == "one other":
+        pos[40], pos[n - 1] = 7, 250
+    elif where == "beyond the table":
+        pos[::3], pos[1::3] = -5, 2 ** 40
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    q, k = (torch.empty(n, h, 128, device="cuda", dtype=torch.bfloat16) for h in (hq, hkv))
+    ops.qknorm_rope_kvstore(qkv, pos, None, None, 1e-6, table, None, q, k, None, None, hq, hkv)
+    v = qkv[:, (hq + hkv) * 128:].view(n, hkv, 128)
+    want = ops.attn_prefill_varlen(q, k, v, cu, cu, max(lens), 128 ** -0.5)
+    got = ops.attn_prefill_raw(qkv, hq, pos, None, 1e-6, table, k, v, cu, cu, max(lens), 128 ** -0.5)
+    assert torch.equal(got, want)                               # the same roundings throughout
