@@ -54,7 +54,7 @@ constexpr float HIDDEN = -3e38f;                  // a masked score: its weight 
 // behind the last round shows: queries, norm and rotation are prepared while the first tile is on its way, cos and sin once per position and
 // workgroup. 64 queries per wavefront (half the LDS reads) need the accumulation registers, and the compiler's moves to and from them cost more.
 // MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 351, blocks of
-// 1024 with rotation 936 -> 255; 16 / 8 heads, causal, rotation, sink 764 -> 189; latent rows, 16 heads, window 1024 and causal 1013 -> 275.
+// 1024 with rotation 936 -> 255; 16 / 8 heads, causal, rotation, sink 764 -> 189; latent rows, 16 heads, window 1024 and causal 1013 -> 240.
 template <int D, int DV, int NW, bool EXT>
 __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_kernel(const WindowAttnArgs A) {
   constexpr bool PIPE = D == 128;
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   const bool valid = rel < len;
   const int64_t row = (int64_t)row0 + (valid ? rel : len - 1);
   bf16x8_t qb[DC];
-  {
+  if constexpr (D == 128) {
     const bf16_t* qp = (const bf16_t*)A.q + row * A.q_stride + (int64_t)h * D + 8 * hi;
 #pragma unroll
     for (int c = 0; c < DC; ++c) qb[c] = *(const bf16x8_t*)(qp + 16 * c);
@@ -256,6 +256,84 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         qb[c][e] = (bf16_t)a, qb[c][e + 1] = (bf16_t)b;
       }
     }
+  } else {
+    // Rows are requested as they lie, D / 8 lanes each, and turn into operands by way of the second tile's place, a few rows of every wavefront at a time. (A lane that
+    // requests its own query's entries asks for 32 bytes of each of 32 rows; nothing hides that where one workgroup has the compute unit to itself: 12 us of 61 a
+    // workgroup, 7.5 so, 14,200 tokens in 9 prompts, 16 heads, window 1,024 / causal 270 / 292 us, 251 / 275 so. 128-wide heads: no
+    // difference.)
+    constexpr int RL = D / 8, RI = 64 / RL, QI = 32 / RI, PASSES = 4, PR = 32 / PASSES, N = QI / PASSES;        // lanes of a row, rows of a request, requests; rows of a pass
+    static_assert(NW * PR * D * 2 <= TILE, "a pass of all wavefronts' rows fits the second tile");
+    const int sub = lane % RL, sub_row = lane / RL;
+    bf16x8_t qr[QI];
+    const bf16_t* qp = (const bf16_t*)A.q + (int64_t)row0 * A.q_stride + (int64_t)h * D + sub * 8;
+#pragma unroll
+    for (int i = 0; i < QI; ++i) {
+      const int r = rel0 + i * RI + sub_row;
+      qr[i] = *(const bf16x8_t*)(qp + (int64_t)(r < len ? r : len - 1) * A.q_stride);
+    }
+    float factor = A.scale * query_temp(pos, A.qt_coef, A.qt_every);
+    const bf16_t* qw = (const bf16_t*)A.qnorm;
+    const bool own_norm = qw && !(EXT && A.q_row);
+    if (EXT && A.q_row) {
+      factor *= A.q_row[row];
+      qw += (int64_t)h * D;
+    }
+    const auto finish = [&](float (&v)[8], const float (&w)[8], int col) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = v[e] * factor * w[e];
+      if (col >= A.rot_dims) return;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        if (col + e < A.rot_dims) {                 // the pair (2i, 2i+1) turns by pos * freq[i]
+          float sn, cs;
+          sincosf((float)pos * A.rot_freq[(col + e) >> 1], &sn, &cs);
+          const float a = v[e] * cs - v[e + 1] * sn;
+          v[e + 1] = v[e + 1] * cs + v[e] * sn;
+          v[e] = a;
+        }
+      }
+    };
+    char* at = lds + TILE + wave * PR * D * 2;
+    const int mine = ql % PR;
+    static_for<0, PASSES>([&](auto pass) {
+      constexpr int p = decltype(pass)::value;
+      static_for<0, N>([&](auto index) {
+        constexpr int i = decltype(index)::value;
+        const int r = i * RI + sub_row;
+        *(bf16x8_t*)(at + r * D * 2 + ((sub ^ (r & 15)) << 4)) = qr[p * N + i];
+      });
+      static_for<0, DC>([&](auto index) {
+        constexpr int c = decltype(index)::value;
+        const u32x4_t x = *(const u32x4_t*)(at + mine * D * 2 + (((2 * c + hi) ^ (mine & 15)) << 4));
+        if constexpr (p == 0) {
+          qb[c] = __builtin_bit_cast(bf16x8_t, x);
+        } else {
+          u32x4_t y = __builtin_bit_cast(u32x4_t, qb[c]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = ql / PR == p ? x[e] : y[e];
+          qb[c] = __builtin_bit_cast(bf16x8_t, y);
+        }
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (own_norm) {
+      float ss = 0.f;
+#pragma unroll
+      for (int c = 0; c < DC; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += (float)qb[c][e] * (float)qb[c][e];
+      factor *= rsqrtf((ss + other_half(ss)) / (float)D + A.eps);
+    }
+    static_for<0, DC>([&](auto index) {
+      constexpr int c = decltype(index)::value;
+      float v[8], w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (float)qb[c][e], w[e] = 1.f;
+      if (qw) ldp<8>(qw + 16 * c + 8 * hi, w);
+      finish(v, w, 16 * c + 8 * hi);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qb[c][e] = (bf16_t)v[e];
+    });
   }
   // a sink is a score in the denominator without a value; the sum starts from it (once per query: in the lower half of the lanes). One that weighs
   // nothing beside any score is none: the maximum must lie above that of a round in which the query sees no key
@@ -444,37 +522,89 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   }
 
   // ---- out: lane holds columns 32 db + 8 a + 4 hi .. + 3 of query ql
-  typedef __attribute__((ext_vector_type(4))) __bf16 b4_t;
-  const float inv = 1.f / (l + other_half(l));
-  if (!valid) return;
-  bf16_t* op = (bf16_t*)A.out + (row * H + h) * DV + 4 * hi;
-  const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + row * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
-  const auto gated = [](float x, float gv) { return x * sigmoid_hw(gv); };
-  const bool wide = gp && A.gate_w != 1;
-  const float ginv = gp && !wide ? gated(inv, (float)gp[0]) : inv;
-  const bool quads = wide && ((A.gate_stride & 3) == 0) && ((uintptr_t)A.gate & 7) == 0;
+  if constexpr (D == 128) {
+    typedef __attribute__((ext_vector_type(4))) __bf16 b4_t;
+    const float inv = 1.f / (l + other_half(l));
+    if (!valid) return;
+    bf16_t* op = (bf16_t*)A.out + (row * H + h) * DV + 4 * hi;
+    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + row * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
+    const auto gated = [](float x, float gv) { return x * sigmoid_hw(gv); };
+    const bool wide = gp && A.gate_w != 1;
+    const float ginv = gp && !wide ? gated(inv, (float)gp[0]) : inv;
+    const bool quads = wide && ((A.gate_stride & 3) == 0) && ((uintptr_t)A.gate & 7) == 0;
 #pragma unroll
-  for (int db = 0; db < DB; ++db) {
-    b4_t gv[4];
-    if (quads) {
+    for (int db = 0; db < DB; ++db) {
+      b4_t gv[4];
+      if (quads) {
 #pragma unroll
-      for (int a = 0; a < 4; ++a) gv[a] = *(const b4_t*)(gp + 32 * db + 8 * a + 4 * hi);
-    } else if (wide) {
+        for (int a = 0; a < 4; ++a) gv[a] = *(const b4_t*)(gp + 32 * db + 8 * a + 4 * hi);
+      } else if (wide) {
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) gv[a][i] = gp[32 * db + 8 * a + 4 * hi + i];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      b4_t v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float x = o[db][4 * a + i] * ginv;
-        if (wide) x = gated(x, (float)gv[a][i]);
-        v[i] = (bf16_t)x;
+          for (int i = 0; i < 4; ++i) gv[a][i] = gp[32 * db + 8 * a + 4 * hi + i];
       }
-      *(b4_t*)(op + 32 * db + 8 * a) = v;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        b4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float x = o[db][4 * a + i] * ginv;
+          if (wide) x = gated(x, (float)gv[a][i]);
+          v[i] = (bf16_t)x;
+        }
+        *(b4_t*)(op + 32 * db + 8 * a) = v;
+      }
+    }
+  } else {
+    // Through LDS in 32 bits, so that rows (and the gate's) are read and written as they lie, 16 bytes a lane: one workgroup of eight wavefronts has the compute unit to itself, nothing
+    // hides what comes behind its rounds (14,200 tokens in 9 prompts, 16 heads, window 1,024 / causal, 251 / 275 us before, 234 / 256 so; 128-wide heads, gated,
+    // 323 and 333).
+    constexpr int OP = NW * 32 * DV * 4 <= 2 * TILE ? 1 : 2, OC = DV / OP, OU = OC / 8;        // passes; columns of one; units of 8 columns
+    static_assert(NW * 32 * OC * 4 <= 2 * TILE && DB % OP == 0 && OC % 32 == 0, "a pass of all wavefronts' rows fits the tiles");
+    int out_tid = threadIdx.x;                        // (as if new: addresses of the queries' rows would be kept over the loop otherwise, which has no register left)
+    asm volatile("" : "+v"(out_tid));
+    const int ol = out_tid & 63, oq = ol & 31, oh = ol >> 5, ow = __builtin_amdgcn_readfirstlane(out_tid >> 6);
+    const int live = len - rel0 < 32 ? len - rel0 : 32;                           // (none: a wavefront of nobody's queries)
+    const float inv = 1.f / (l + other_half(l));
+    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + rel0) * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
+    const bool wide = gp && A.gate_w != 1, units = wide && (A.gate_stride & 7) == 0 && ((uintptr_t)gp & 15) == 0;
+    const float ginv = gp && !wide ? inv * sigmoid_hw((float)gp[(int64_t)(oq < live ? oq : 0) * A.gate_stride]) : inv;
+    bf16_t* op = (bf16_t*)A.out + ((int64_t)(row0 + rel0) * H + h) * DV;
+    char* at = lds + ow * 32 * OC * 4;
+    __syncthreads();                                  // (the tiles have been read)
+#pragma unroll
+    for (int p = 0; p < OP; ++p) {
+      bf16x8_t gv[OU / 2];
+      if (units) {
+#pragma unroll
+        for (int i = 0; i < OU / 2; ++i) {
+          const int x = i * 64 + ol, r = x / OU, u = x % OU;
+          gv[i] = *(const bf16x8_t*)(gp + (int64_t)(r < live ? r : 0) * A.gate_stride + p * OC + u * 8);
+        }
+      }
+#pragma unroll
+      for (int db = 0; db < DB / OP; ++db)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          f32x4_t v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = o[p * (DB / OP) + db][4 * a + i] * ginv;
+          *(f32x4_t*)(at + oq * OC * 4 + (((8 * db + 2 * a + oh) ^ (oq & 7)) << 4)) = v;
+        }
+#pragma unroll
+      for (int i = 0; i < OU / 2; ++i) {
+        const int x = i * 64 + ol, r = x / OU, u = x % OU;
+        const f32x4_t v0 = *(const f32x4_t*)(at + r * OC * 4 + (((2 * u) ^ (r & 7)) << 4)), v1 = *(const f32x4_t*)(at + r * OC * 4 + (((2 * u + 1) ^ (r & 7)) << 4));
+        bf16x8_t y;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float f = e < 4 ? v0[e] : v1[e - 4];
+          if (wide) f *= sigmoid_hw((float)(units ? gv[i][e] : gp[(int64_t)(r < live ? r : 0) * A.gate_stride + p * OC + u * 8 + e]));
+          y[e] = (bf16_t)f;
+        }
+        if (r < live) *(bf16x8_t*)(op + (int64_t)r * H * DV + p * OC + u * 8) = y;
+      }
     }
   }
 }
