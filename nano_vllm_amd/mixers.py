@@ -867,7 +867,7 @@ class RoutedExperts(nn.Module):
         else:                                     # 32-bit logits, [n, total (+ 1: the shared gate)]
             ids, wts, gate = ops_seq.moe_router(wide if wide is not None else xh, self.router, self.router_b, total, self.correction, self.top,
                                                 self.count, self.keep, self.scale, self.sigmoid, self.renorm)
-        plan = ops_seq.moe_plan(ids, self.E, ops_seq.moe_tile_rows(n * self.top, self.E, width, self.ff, xh.dtype))
+        plan = ops_seq.moe_plan(ids, self.E, ops_seq.moe_plan_rows(n * self.top, self.E, width, self.ff, xh.dtype))
         act = torch.empty(plan.cap, self.ff, dtype=xh.dtype, device=xh.device)
         ops_seq.moe_gemm(xh, self.w_gu, plan, self.gated, act, relu2=not self.gated)
         rows = torch.empty(plan.cap, width, dtype=xh.dtype, device=xh.device)

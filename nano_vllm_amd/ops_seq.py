@@ -924,10 +924,16 @@ class MoePlan:
     __slots__ = ("tile_expert", "row_token", "pair_row", "cap", "tm")
 
 
+def _moe_groups(pairs: int, experts: int, width: int, ff: int, tm: int) -> float:
+    """Workgroups of the two products at tiles of tm rows (256 weight rows each), weighted by the lengths of their reductions."""
+    tiles = min(experts, pairs) * max(1.0, pairs / experts / tm + 0.5)
+    return tiles * (-(-2 * ff // 256) * width + -(-width // 256) * ff) / (width + ff)
+
+
 def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dtype) -> int:
     """Rows per tile of a step's plan. It follows the rows an expert gets on average: a tile reads all weights of its features, so few
-    rows want the smallest tile and many the largest. The figures of 256 rows are of moe_gemm_pipe_kernel; 16-bit ones run gemm_tiles_kernel now, which takes 15 to 30 % less, so that some calls below the
-    lines for 256 would be faster there too. MI355X, gate|up + down of 32 gated experts, us at tiles of 16 / 64 / 128 / 256 rows:
+    rows want the smallest tile and many the largest. The figures of 256 rows are of moe_gemm_pipe_kernel; the 16-bit plans that gemm_tiles_kernel
+    runs instead are moe_plan_rows' below. MI355X, gate|up + down of 32 gated experts, us at tiles of 16 / 64 / 128 / 256 rows:
     width 4096, ff 3072: 8 rows 428 / 436 / 471 / 609; 32: 598 / 455 / 489 / 622; 64: 838 / 580 / 507 / 640; 250: 2256 / 1003 / 879 / 928;
     1694: 12546 / 4674 / 4103 / 3634. Width 2048: 16 rows 126 / 133 / 149 / 178; 32: 141 / 135 / 155 / 181; 500: 1028 / 456 / 420 / 408.
     Width 1024, ff 768 (few and short tiles: two small workgroups per compute unit cover each other's start and end better than one large
@@ -945,9 +951,8 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     if width % piece or ff % piece:
         return 128 if per >= 256 else 64 if per >= 64 else 16
 
-    def groups(tm):                                     # workgroups of the two products (256 weight rows each), weighted by the lengths of their reductions
-        tiles = min(experts, pairs) * max(1.0, pairs / experts / tm + 0.5)
-        return tiles * (-(-2 * ff // 256) * width + -(-width // 256) * ff) / (width + ff)
+    def groups(tm):
+        return _moe_groups(pairs, experts, width, ff, tm)
 
     if per < 512 and groups(64) < 130:
         return 16
@@ -960,6 +965,27 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dt
     if per >= 448 and groups(256) >= (270 if ff >= 1024 else 480):
         return 256
     return 128 if per >= 64 and groups(128) >= (150 if ff >= 1024 else 1000) else 64 if per >= 24 else 16
+
+
+def moe_plan_rows(pairs: int, experts: int, width: int, ff: int, dtype: torch.dtype) -> int:
+    """Rows per tile of a step's plan, where 16-bit tiles of 256 rows are gemm_tiles_kernel's: moe_tile_rows, but 256 rows from 128 per expert on.
+    Half of the experts fill a second tile of 128 rows there; its weights are read again and it takes as long as a full one, while the larger tile's
+    workgroup takes the next tile's operands under the end of its last. MI355X, plan, gate|up, down and the weighted sum, us at 64 / 128 / 256 rows,
+    rows per expert 90, 130, 180, 250, 450 (16-bit, gated):
+    32 of 4096 x 3072: 100 591 / 520 / 552; 150 728 / 689 / 560; 200 868 / 705 / 572; 250 963 / 857 / 729; 375 1302 / 1143 / 941;
+    32 of 2048 x 1536: 177 / 167 / 170; 234 / 207 / 176; 248 / 208 / 183; 301 / 258 / 218; 350 rows 350 / 311 / 261;
+    32 of 2048 x 768: 106 / 98 / 103; 123 / 140 / 106; 157 / 133 / 111; 178 / 150 / 129; 240 / 203 / 173;
+    32 of 1024 x 768: 61 / 60 / 61; 67 / 76 / 63; 85 / 77 / 66; 104 / 94 / 86; 136 / 118 / 98; 8 of 1024 x 1024: - ; 42 / 48 / 42; 43 / 49 / 43; 46 / 49 / 44; -;
+    8 of 2048 x 512: 47 / 54 / 45; 49 / 56 / 47; 51 / 57 / 48; 54 / 58 / 50; 59 / 64 / 55, 1500 rows 130 / 134 / 108.
+    Tiles of 128 rows stay where all of them run at once and their reduction is long: two of 4096 x 3072, 250 rows 132 / 119 / 128, 450 141 / 122 / 131, 900
+    204 / 185 / 156; four of 8192 x 1024, 250 rows 173 / 153 / 157, 600 233 / 209 / 205; eight of 4096 x 1024, 180 rows 115 / 101 / 106, 250 127 / 120 / 113;
+    eight of 2048 x 1536, 180 rows 94 / 77 / 80, 250 96 / 107 / 82 (one of 2048 x 2048, 1500 rows 78 / 78 / 69). Where moe_tile_rows says 16, few
+    workgroups have anything to do, and that stays the fastest (one of 2048 x 2048, 250 rows, 16 / 64 / 128 / 256: 38 / 61 / 70 / 60)."""
+    rows, per = moe_tile_rows(pairs, experts, width, ff, dtype), pairs // experts
+    if rows == 16 or dtype != torch.bfloat16 or width % 64 or ff % 64 or min(width, ff) < 128 or per < 128:
+        return rows
+    long = ff >= 1024 and (width >= 4096 or (width >= 2048 and per < 256))
+    return 128 if long and _moe_groups(pairs, experts, width, ff, 128) < 170 else 256
 
 
 @_launch
