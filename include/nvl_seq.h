@@ -331,6 +331,15 @@ int nvs_rotate_heads(const void* in, int64_t in_stride, int in_head, void* out, 
 int nvs_latent_heads(const void* x, int64_t ldx, int xh, const void* w, int turned, int K, int N, void* y, int64_t ldy, int yh, int H, int tail,
                      int rot_dims, int rot_halves, const void* turn, int64_t n, void* stream);
 
+/* bf16: nvs_latent_heads (128 -> 192, 64 entries behind, rot_dims a multiple of 16) and nvs_window_attn over one kv head of 256 entries with
+ * values of 192 in one kernel: q [n, q_stride], per head 128 entries and 64 that turn by `turn` ([n][rot_dims / 2][2]); uk [H][128][192]; gate [n, gate_stride], one
+ * entry a head, or NULL; out [n][H][192]. Pages of 64 tokens or more, a power of two; pointers on 16-byte boundaries. nvs_latent_prompt_fits: whether a step of n
+ * tokens in nseq portions is one that nvs_window_attn would give to the same kernel (no single tokens, nor few with heads in a query's place). */
+int nvs_latent_prompt_fits(int64_t n, int nseq, int H, int block_size);
+int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
+                      const void* k_cache, const void* v_cache, const int32_t* block_tables, int64_t bt_stride, int block_size, const int32_t* cu_q, const int32_t* ctx0, int nseq,
+                      int64_t n, int H, float scale, int window, void* out, void* stream);
+
 /* Tests and A/B runs: 1 routes bf16 calls through the scalar kernel too; 2 keeps the matrix-core kernel but without sharing
  * K / V tiles through LDS; 3 keeps the LDS kernel but never packs heads into the query tiles of single-token steps; 0 restores
  * the defaults. */

@@ -1,5 +1,5 @@
 // Windowed attention over the paged cache, pipelined (bf16, 128-wide heads or latent rows of 256 with values of 192): device code shared by the
-// translation units that instantiate it (attn_prompt.hip: windows, blocks, causal; attn_prompt_pool.hip: the same with pooled blocks, capped
+// translation units that instantiate it (attn_prompt.hip: windows, blocks, causal; attn_prompt_latent.hip: latent rows whose queries come unfinished; attn_prompt_pool.hip: the same with pooled blocks, capped
 // scores and row factors). Masks, sink, temperature, norm, rotation and gate mean what they mean in attn_window_core.h, whose kernels take every
 // other size.
 #pragma once
@@ -7,6 +7,7 @@
 
 int window_attn_prompt(const WindowAttnArgs& a, hipStream_t stream);               // attn_prompt.hip
 int window_attn_prompt_extended(const WindowAttnArgs& a, hipStream_t stream);      // attn_prompt_pool.hip
+int window_attn_prompt_latent(const WindowAttnArgs& a, hipStream_t stream);        // attn_prompt_latent.hip
 
 namespace {
 
@@ -55,7 +56,7 @@ constexpr float HIDDEN = -3e38f;                  // a masked score: its weight 
 // workgroup. 64 queries per wavefront (half the LDS reads) need the accumulation registers, and the compiler's moves to and from them cost more.
 // MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 351, blocks of
 // 1024 with rotation 936 -> 255; 16 / 8 heads, causal, rotation, sink 764 -> 189; latent rows, 16 heads, window 1024 and causal 1013 -> 240.
-template <int D, int DV, int NW, bool EXT>
+template <int D, int DV, int NW, bool EXT, bool HEADS = false>
 __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_kernel(const WindowAttnArgs A) {
   constexpr bool PIPE = D == 128;
   constexpr int KB = 64 * D * 2, VB = DV * 128, TILE = KB + VB, KU = D / 8, KI = KB / 1024 / NW, VI = VB / 1024 / NW, DC = D / 16, DB = DV / 32;
@@ -112,7 +113,9 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
   int kblk[KI], vblk[2];                            // EXT: unit of 8 blocks of a request's rows; of a lane's tokens (even, odd requests)
 #pragma unroll
   for (int i = 0; i < KI; ++i) {
-    const int r = (wave * KI + i) * (64 / KU) + lane / KU, u = (lane % KU) ^ (r & 15);
+    const int r = (wave * KI + i) * (64 / KU) + lane / KU;
+    int u = (lane % KU) ^ (r & 15);
+    if (HEADS && u < 24) u = u / 6 * 6 + u % 2 * 3 + u % 6 / 2;                 // (the order in which a lane gets its query's entries, below)
     koff[i] = (uint32_t)(((EXT ? r & 7 : r) * G * D + u * 8) * 2);
     kblk[i] = r >> 3;
   }
@@ -256,6 +259,101 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         qb[c][e] = (bf16_t)a, qb[c][e + 1] = (bf16_t)b;
       }
     }
+  } else if constexpr (HEADS) {
+    // The product with W_uk,h stands here: a lane's results are its query's operands of the scores as they are. The queries' 128 + 64 entries are requested as they lie, the last 64
+    // turn, and through the second tile's place and what lies behind it they become operands. W_uk,h [128][192] comes straight from L2, k-step by k-step two ahead: lane l asks for
+    // entries 6 l .. 6 l + 5 of eight rows and turns them by byte permutations, so block j of 32 latent entries holds 6 l + j in row l. A lane then has 24 entries in a row
+    // for each a: 48 a + 24 hi + 0 .. 23, units 6 a + 3 hi + t of eight; the key tile's units lie in LDS in that order.
+    // As a launch of its own the product reads and writes every head's row once more, 68 us of 14,200 rows and 16 heads (210 MB); here a workgroup's queries take as long as 256 finished
+    // entries did (7.2 us: 48 KB of weights a wavefront, 1.5 us of products): window 1,024 68 + 234 -> 246 us, four layers of 14,200 tokens 3,270 -> 3,024.
+    constexpr int NOPE = 128, TAIL = 64, ROWS = 32 * (NOPE + TAIL) * 2;
+    typedef __attribute__((ext_vector_type(3))) unsigned int u32x3_t;
+    const int nu = lane & 15, nr = lane >> 4, tu = lane & 7, tr = lane >> 3, half = A.rot_dims >> 1, apart = half >> 3;
+    const bool turns = tu * 8 < A.rot_dims, halves = A.rot_halves != 0, upper = tu >= apart;              // halves: entry i turns with entry i + half, which a lane `apart` units on holds
+    const bf16_t* qp = (const bf16_t*)A.q + (int64_t)row0 * A.q_stride + (int64_t)h * (NOPE + TAIL);
+    const auto at_row = [&](int r) { return (int64_t)(rel0 + r < len ? rel0 + r : len - 1); };
+    const char* wp = (const char*)A.uk + (int64_t)h * NOPE * DV * 2 + hi * 8 * DV * 2 + ql * 12;
+    bf16x8_t qn[8], qt[4];
+    f32x4_t cs[4][4];
+    u32x3_t w[3][8];
+    const auto bring = [&](auto step) {
+      constexpr int k = decltype(step)::value;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) __builtin_memcpy(&w[k % 3][j], __builtin_assume_aligned(wp + (k * 16 + j) * DV * 2, 4), 12);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      qt[i] = *(const bf16x8_t*)(qp + at_row(i * 8 + tr) * A.q_stride + NOPE + tu * 8);
+      if (turns) {
+        const float2* f = A.turn + (row0 + at_row(i * 8 + tr)) * half + (halves ? (upper ? tu - apart : tu) * 8 : tu * 4);
+        cs[i][0] = *(const f32x4_t*)f, cs[i][1] = *(const f32x4_t*)(f + 2);
+        if (halves) cs[i][2] = *(const f32x4_t*)(f + 4), cs[i][3] = *(const f32x4_t*)(f + 6);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qn[i] = *(const bf16x8_t*)(qp + at_row(i * 4 + nr) * A.q_stride + nu * 8);
+    bring(Int<0>{});
+    bring(Int<1>{});
+    __builtin_amdgcn_sched_barrier(0);
+    char* at = lds + TILE + wave * ROWS;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = i * 8 + tr;
+      if (halves) {
+        const u32x4_t own = __builtin_bit_cast(u32x4_t, qt[i]);
+        u32x4_t theirs;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) theirs[e] = (unsigned)__shfl((int)own[e], upper ? lane - apart : lane + apart, 64);
+        const bf16x8_t other = __builtin_bit_cast(bf16x8_t, theirs);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float c = cs[i][e / 2][e % 2 * 2], sn = cs[i][e / 2][e % 2 * 2 + 1], v = (float)qt[i][e], o = (float)other[e];
+          qt[i][e] = (bf16_t)((turns ? upper ? v * c + o * sn : v * c - o * sn : v) * A.scale);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          float a = (float)qt[i][e], b = (float)qt[i][e + 1];
+          if (turns) {
+            const float c = cs[i][e / 4][e % 4], sn = cs[i][e / 4][e % 4 + 1], a2 = a * c - b * sn;
+            b = b * c + a * sn, a = a2;
+          }
+          qt[i][e] = (bf16_t)(a * A.scale), qt[i][e + 1] = (bf16_t)(b * A.scale);
+        }
+      }
+      *(bf16x8_t*)(at + 32 * NOPE * 2 + r * TAIL * 2 + ((tu ^ ((r >> 1) & 7)) << 4)) = qt[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = i * 4 + nr;
+      *(bf16x8_t*)(at + r * NOPE * 2 + ((nu ^ (r & 15)) << 4)) = qn[i];
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qn[s] = *(const bf16x8_t*)(at + ql * NOPE * 2 + (((2 * s + hi) ^ (ql & 15)) << 4));
+    f32x16_t acc[6];
+    static_for<0, 8>([&](auto step) {
+      constexpr int k = decltype(step)::value;
+      if constexpr (k + 2 < 8) bring(Int<k + 2>{});
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, 6>([&](auto block) {
+        constexpr int j = decltype(block)::value;
+        u32x4_t x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = __builtin_amdgcn_perm(w[k % 3][2 * i + 1][j / 2], w[k % 3][2 * i][j / 2], j % 2 ? 0x07060302u : 0x05040100u);
+        const f32x16_t zero = {};
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, x), qn[k], k == 0 ? zero : acc[j], 0, 0, 0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    static_for<0, 12>([&](auto index) {
+      constexpr int c = decltype(index)::value, a = c / 3, t = c % 3;
+      static_for<0, 8>([&](auto entry) {
+        constexpr int x = 8 * t + decltype(entry)::value;
+        qb[c][x % 8] = (bf16_t)(acc[x % 6][4 * a + x / 6] * A.scale);
+      });
+    });
+#pragma unroll
+    for (int c = 0; c < 4; ++c) qb[12 + c] = *(const bf16x8_t*)(at + 32 * NOPE * 2 + ql * TAIL * 2 + (((2 * c + hi) ^ ((ql >> 1) & 7)) << 4));
   } else {
     // Rows are requested as they lie, D / 8 lanes each, and turn into operands by way of the second tile's place, a few rows of every wavefront at a time. (A lane that
     // requests its own query's entries asks for 32 bytes of each of 32 rows; nothing hides that where one workgroup has the compute unit to itself: 12 us of 61 a
@@ -625,13 +723,13 @@ inline PromptGrid prompt_grid(const WindowAttnArgs& a, int nw) {
   return p;
 }
 
-template <int D, int DV, int NW, bool EXT>
+template <int D, int DV, int NW, bool EXT, bool HEADS = false>
 int launch_prompt(WindowAttnArgs a, hipStream_t stream) {
   const PromptGrid p = prompt_grid(a, NW);
   a.hw = p.hw;
   a.bs_shift = __builtin_ctz(a.block_size);
-  constexpr int LDS = 2 * (64 * D * 2 + DV * 128);
-  const auto kernel = window_attn_prompt_kernel<D, DV, NW, EXT>;
+  constexpr int TILE = 64 * D * 2 + DV * 128, LDS = TILE + (HEADS ? NW * 32 * DV * 2 : TILE);      // (HEADS: queries of 128 + 64 entries, as wide as a value)
+  const auto kernel = window_attn_prompt_kernel<D, DV, NW, EXT, HEADS>;
   NVS_LDS_ROOM(kernel, LDS, "nvs_window_attn");
   kernel<<<dim3((unsigned)p.tiles, (unsigned)p.rows), dim3(64 * NW), LDS, stream>>>(a);
   return nvs_check_launch("nvs_window_attn (prompts)");

@@ -283,6 +283,12 @@ extern "C" int nvs_knorm_kvstore(const void* k, const void* v, int64_t stride, i
   return nvs_check_launch("nvs_knorm_kvstore");
 }
 
+// steps of single tokens, or of few each, whose heads share query tiles (the reasons stand in nvs_window_attn)
+static bool few_tokens(const WindowAttnArgs& a, const PromptGrid& grid, int at_once) {
+  const int hpg = a.H / a.G;
+  return hpg >= 8 && a.n < 32ll * a.nseq && 4 * a.n <= (int64_t)a.nseq * hpg && grid.tiles * grid.rows > at_once;
+}
+
 extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnorm, float eps, const float* q_row, const void* gate,
                                int64_t gate_stride, int gate_per_head, int dtype, const void* k_cache, const void* v_cache,
                                const int32_t* block_tables, int64_t bt_stride, int block_size, const int32_t* cu_q, const int32_t* ctx0,
@@ -323,7 +329,7 @@ extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnor
     const bool aligned = (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)qnorm | (uintptr_t)pool_k | (uintptr_t)pool_v) & 15) == 0 &&
                          q_stride % 8 == 0 && ((uintptr_t)out & 7) == 0;
     const PromptGrid grid = prompt_grid(a, d == 128 ? 4 : 8);
-    const bool packed = H / G >= 8 && n < 32ll * nseq && 4 * n <= (int64_t)nseq * (H / G) && grid.tiles * grid.rows > (d == 128 && !(softcap > 0.f) ? 512 : 256);
+    const bool packed = few_tokens(a, grid, d == 128 && !(softcap > 0.f) ? 512 : 256);
     if (built && aligned && n <= nseq && pool == 0 && block_size >= 32 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
       return window_attn_token(a, (hipStream_t)stream);
     if (sizes && aligned && !packed && block_size >= 64 && (block_size & (block_size - 1)) == 0 && !g_no_lds && g_packed_heads)
@@ -342,4 +348,29 @@ extern "C" int nvs_window_attn(const void* q, int64_t q_stride, const void* qnor
   else                                               // heads of up to 1024 entries: the same kernel with 16 entries per lane
     NVS_DISPATCH(dtype, window_attn_kernel<T, 16><<<dim3((unsigned)n, H), dim3(64), 0, (hipStream_t)stream>>>(a));
   return nvs_check_launch("nvs_window_attn");
+}
+
+extern "C" int nvs_latent_prompt_fits(int64_t n, int nseq, int H, int block_size) {
+  if (n <= nseq || nseq <= 0 || H <= 0 || H > 65535 || block_size < 64 || (block_size & (block_size - 1)) || g_force_scalar || g_no_lds || !g_packed_heads) return 0;
+  WindowAttnArgs a = {};
+  a.n = n, a.nseq = nseq, a.H = H, a.G = 1;
+  return !few_tokens(a, prompt_grid(a, 8), 256);
+}
+
+extern "C" int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
+                                 const void* k_cache, const void* v_cache, const int32_t* block_tables, int64_t bt_stride, int block_size, const int32_t* cu_q, const int32_t* ctx0, int nseq,
+                                 int64_t n, int H, float scale, int window, void* out, void* stream) {
+  NVS_REQUIRE(q && uk && k_cache && v_cache && block_tables && cu_q && ctx0 && out, "nvs_latent_prompt: null argument");
+  NVS_REQUIRE(rot_dims >= 0 && rot_dims <= 64 && rot_dims % 16 == 0 && (rot_dims == 0 || turn), "nvs_latent_prompt: rotation of %d of 64 entries", rot_dims);
+  NVS_REQUIRE(H > 0 && H <= 65535 && n >= 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0, "nvs_latent_prompt: H %d block %d", H, block_size);
+  NVS_REQUIRE(q_stride % 8 == 0 && (((uintptr_t)q | (uintptr_t)uk | (uintptr_t)turn | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15) == 0,
+              "nvs_latent_prompt: rows of %lld entries", (long long)q_stride);
+  if (n == 0 || nseq == 0) return NVS_OK;
+  WindowAttnArgs a = {};
+  a.q = q, a.gate = gate, a.k_cache = k_cache, a.v_cache = v_cache, a.out = out, a.uk = uk, a.turn = (const float2*)turn;
+  a.block_tables = block_tables, a.cu_q = cu_q, a.ctx0 = ctx0;
+  a.q_stride = q_stride, a.gate_stride = gate_stride, a.bt_stride = bt_stride, a.n = n, a.gate_w = 1;
+  a.block_size = block_size, a.nseq = nseq, a.H = H, a.G = 1, a.d = 256, a.dv = 192, a.window = window;
+  a.rot_dims = rot_dims, a.rot_halves = rot_halves, a.scale = scale;
+  return window_attn_prompt_latent(a, (hipStream_t)stream);
 }

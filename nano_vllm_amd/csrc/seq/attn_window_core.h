@@ -20,6 +20,10 @@ struct WindowAttnArgs {
   const void *pool_k, *pool_v;            // means over blocks of `pool` tokens
   int pool;
   float softcap;
+  // what only the prompt kernel of latent rows reads: W_uk [H][128][192] and the step's cosines and sines [n][rot_dims / 2]
+  const void* uk;
+  const float2* turn;
+  int rot_halves;
 };
 
 // first key position the query at position p sees (both masks are monotone in p, which the tile bounds below rely on)
