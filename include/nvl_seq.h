@@ -333,10 +333,10 @@ int nvs_latent_heads(const void* x, int64_t ldx, int xh, const void* w, int turn
 
 /* bf16: nvs_latent_heads (128 -> 192, 64 entries behind, rot_dims a multiple of 16) and nvs_window_attn over one kv head of 256 entries with
  * values of 192 in one kernel: q [n, q_stride], per head 128 entries and 64 that turn by `turn` ([n][rot_dims / 2][2]); uk [H][128][192]; gate [n, gate_stride], one
- * entry a head, or NULL; out [n][H][192]. Pages of 64 tokens or more, a power of two; pointers on 16-byte boundaries. nvs_latent_prompt_fits: whether a step of n
+ * entry a head, or NULL; out [n][H][192] or, with uv [H][128][192] (nvs_latent_heads 192 -> 128 behind it), [n][H][128]. Pages of 64 tokens or more, a power of two; pointers on 16-byte boundaries. nvs_latent_prompt_fits: whether a step of n
  * tokens in nseq portions is one that nvs_window_attn would give to the same kernel (no single tokens, nor few with heads in a query's place). */
 int nvs_latent_prompt_fits(int64_t n, int nseq, int H, int block_size);
-int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
+int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* uv, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
                       const void* k_cache, const void* v_cache, const int32_t* block_tables, int64_t bt_stride, int block_size, const int32_t* cu_q, const int32_t* ctx0, int nseq,
                       int64_t n, int H, float scale, int window, void* out, void* stream);
 

@@ -56,7 +56,8 @@ constexpr float HIDDEN = -3e38f;                  // a masked score: its weight 
 // workgroup. 64 queries per wavefront (half the LDS reads) need the accumulation registers, and the compiler's moves to and from them cost more.
 // MI355X, 13,550 tokens in 9 prompts, before (window_attn_mfma_lds_kernel) and now, us: 32 / 8 heads, window 1024, norm and gate 1300 -> 351, blocks of
 // 1024 with rotation 936 -> 255; 16 / 8 heads, causal, rotation, sink 764 -> 189; latent rows, 16 heads, window 1024 and causal 1013 -> 240.
-template <int D, int DV, int NW, bool EXT, bool HEADS = false>
+// HEADS: latent rows whose queries come unfinished (1) and whose results leave through W_uv too (2)
+template <int D, int DV, int NW, bool EXT, int HEADS = 0>
 __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_kernel(const WindowAttnArgs A) {
   constexpr bool PIPE = D == 128;
   constexpr int KB = 64 * D * 2, VB = DV * 128, TILE = KB + VB, KU = D / 8, KI = KB / 1024 / NW, VI = VB / 1024 / NW, DC = D / 16, DB = DV / 32;
@@ -122,7 +123,8 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
 #pragma unroll
   for (int i = 0; i < VI; ++i) {
     const int c = (wave * VI + i) * 8 + (lane >> 3), u = (lane & 7) ^ ((c >> 1) & 7);
-    voff[i] = (uint32_t)((EXT ? c * 8 : c * bs + u * 8) * 2);
+    const int column = HEADS == 2 ? (c & ~12) | (c & 4) << 1 | (c & 8) >> 1 : c;      // (a lane then holds 8 columns in a row, below)
+    voff[i] = (uint32_t)((EXT ? c * 8 : column * bs + u * 8) * 2);
     if (i < 2) vblk[i] = u;
   }
   // Pages (EXT: units of pooled blocks) are looked up a round before the requests that use them: a lookup inside a request would wait for
@@ -259,7 +261,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         qb[c][e] = (bf16_t)a, qb[c][e + 1] = (bf16_t)b;
       }
     }
-  } else if constexpr (HEADS) {
+  } else if constexpr (HEADS != 0) {
     // The product with W_uk,h stands here: a lane's results are its query's operands of the scores as they are. The queries' 128 + 64 entries are requested as they lie, the last 64
     // turn, and through the second tile's place and what lies behind it they become operands. W_uk,h [128][192] comes straight from L2, k-step by k-step two ahead: lane l asks for
     // entries 6 l .. 6 l + 5 of eight rows and turns them by byte permutations, so block j of 32 latent entries holds 6 l + j in row l. A lane then has 24 entries in a row
@@ -654,6 +656,69 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         *(b4_t*)(op + 32 * db + 8 * a) = v;
       }
     }
+  } else if constexpr (HEADS == 2) {
+    // W_uv,h [128][192] times the latent result, which is its operand as it is: a lane holds entries 16 s + 8 hi .. + 7 of its query for each k-step s, since the value tile's columns
+    // lie in that order. The weights come in pieces of 32 rows x 64 entries through four places of the wavefront's own, 16-byte unit u of row r at u ^ ((r >> 1) & 7).
+    // A launch of its own, which reads the latent results again, takes 34 us for 14,200 rows of 16 heads; four layers of 14,200 tokens 3,024 us with it, 2,899 so (a workgroup's end 4.3 us
+    // either way: weights from L2 here, a row 1.5 times as long there).
+    constexpr int OUT = 128, PIECE = 32 * 128, PIECES = OUT / 32 * (DV / 64);
+    int out_tid = threadIdx.x;                        // (as if new, as below)
+    asm volatile("" : "+v"(out_tid));
+    const int ol = out_tid & 63, oq = ol & 31, oh = ol >> 5, ow = __builtin_amdgcn_readfirstlane(out_tid >> 6);
+    const int live = len - rel0 < 32 ? len - rel0 : 32;
+    const float inv = 1.f / (l + other_half(l));
+    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + rel0) * A.gate_stride + h : nullptr;
+    const float ginv = gp ? inv * sigmoid_hw((float)gp[(int64_t)(oq < live ? oq : 0) * A.gate_stride]) : inv;
+    char* at = lds + ow * 4 * PIECE;
+    const char* wbase = (const char*)A.uv + (int64_t)h * OUT * DV * 2;
+    const uint32_t wrow = (uint32_t)(ol >> 3) * DV * 2, woff[2] = {wrow + ((ol & 7) ^ (ol >> 4)) * 16, wrow + ((ol & 7) ^ (4 + (ol >> 4))) * 16};
+    const auto bring = [&](auto piece) {
+      constexpr int p = decltype(piece)::value;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma16(wbase + ((p / 3 * 32 + i * 8) * DV + p % 3 * 64) * 2 + woff[i & 1], at + p % 4 * PIECE + i * 1024);
+    };
+    bf16x8_t x[12];
+#pragma unroll
+    for (int s = 0; s < 12; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[s][e] = (bf16_t)(o[s / 2][s % 2 * 8 + e] * ginv);
+    __syncthreads();                                  // (the tiles have been read)
+    static_for<0, 4>(bring);
+    f32x16_t y[OUT / 32];
+    static_for<0, PIECES>([&](auto piece) {
+      constexpr int p = decltype(piece)::value, left = PIECES - 1 - p < 3 ? PIECES - 1 - p : 3;       // pieces that may still be on their way
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0x0F70 + left * 4);  // vmcnt(4 left)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = *(const bf16x8_t*)(at + p % 4 * PIECE + oq * 128 + (((2 * j + oh) ^ ((oq >> 1) & 7)) << 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x16_t zero = {};
+        y[p / 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], x[p % 3 * 4 + j], p % 3 == 0 && j == 0 ? zero : y[p / 3], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (p + 4 < PIECES) bring(Int<p + 4>{});
+    });
+    typedef __attribute__((ext_vector_type(4))) __bf16 b4_t;
+#pragma unroll
+    for (int vb = 0; vb < OUT / 32; ++vb)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        b4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16_t)y[vb][4 * a + i];
+        *(b4_t*)(at + oq * OUT * 2 + (((4 * vb + a) ^ (oq & 15)) << 4) + oh * 8) = v;
+      }
+    bf16_t* op = (bf16_t*)A.out + ((int64_t)(row0 + rel0) * H + h) * OUT + (ol & 15) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = i * 4 + (ol >> 4);
+      const bf16x8_t v = *(const bf16x8_t*)(at + r * OUT * 2 + (((ol & 15) ^ (r & 15)) << 4));
+      if (r < live) *(bf16x8_t*)(op + (int64_t)r * H * OUT) = v;
+    }
   } else {
     // Through LDS in 32 bits, so that rows (and the gate's) are read and written as they lie, 16 bytes a lane: one workgroup of eight wavefronts has the compute unit to itself, nothing
     // hides what comes behind its rounds (14,200 tokens in 9 prompts, 16 heads, window 1,024 / causal, 251 / 275 us before, 234 / 256 so; 128-wide heads, gated,
@@ -723,7 +788,7 @@ inline PromptGrid prompt_grid(const WindowAttnArgs& a, int nw) {
   return p;
 }
 
-template <int D, int DV, int NW, bool EXT, bool HEADS = false>
+template <int D, int DV, int NW, bool EXT, int HEADS = 0>
 int launch_prompt(WindowAttnArgs a, hipStream_t stream) {
   const PromptGrid p = prompt_grid(a, NW);
   a.hw = p.hw;

@@ -357,17 +357,17 @@ extern "C" int nvs_latent_prompt_fits(int64_t n, int nseq, int H, int block_size
   return !few_tokens(a, prompt_grid(a, 8), 256);
 }
 
-extern "C" int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
+extern "C" int nvs_latent_prompt(const void* q, int64_t q_stride, const void* uk, const void* uv, const void* turn, int rot_dims, int rot_halves, const void* gate, int64_t gate_stride,
                                  const void* k_cache, const void* v_cache, const int32_t* block_tables, int64_t bt_stride, int block_size, const int32_t* cu_q, const int32_t* ctx0, int nseq,
                                  int64_t n, int H, float scale, int window, void* out, void* stream) {
   NVS_REQUIRE(q && uk && k_cache && v_cache && block_tables && cu_q && ctx0 && out, "nvs_latent_prompt: null argument");
   NVS_REQUIRE(rot_dims >= 0 && rot_dims <= 64 && rot_dims % 16 == 0 && (rot_dims == 0 || turn), "nvs_latent_prompt: rotation of %d of 64 entries", rot_dims);
   NVS_REQUIRE(H > 0 && H <= 65535 && n >= 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0, "nvs_latent_prompt: H %d block %d", H, block_size);
-  NVS_REQUIRE(q_stride % 8 == 0 && (((uintptr_t)q | (uintptr_t)uk | (uintptr_t)turn | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15) == 0,
+  NVS_REQUIRE(q_stride % 8 == 0 && (((uintptr_t)q | (uintptr_t)uk | (uintptr_t)uv | (uintptr_t)turn | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15) == 0,
               "nvs_latent_prompt: rows of %lld entries", (long long)q_stride);
   if (n == 0 || nseq == 0) return NVS_OK;
   WindowAttnArgs a = {};
-  a.q = q, a.gate = gate, a.k_cache = k_cache, a.v_cache = v_cache, a.out = out, a.uk = uk, a.turn = (const float2*)turn;
+  a.q = q, a.gate = gate, a.k_cache = k_cache, a.v_cache = v_cache, a.out = out, a.uk = uk, a.uv = uv, a.turn = (const float2*)turn;
   a.block_tables = block_tables, a.cu_q = cu_q, a.ctx0 = ctx0;
   a.q_stride = q_stride, a.gate_stride = gate_stride, a.bt_stride = bt_stride, a.n = n, a.gate_w = 1;
   a.block_size = block_size, a.nseq = nseq, a.H = H, a.G = 1, a.d = 256, a.dv = 192, a.window = window;

@@ -20,8 +20,8 @@ struct WindowAttnArgs {
   const void *pool_k, *pool_v;            // means over blocks of `pool` tokens
   int pool;
   float softcap;
-  // what only the prompt kernel of latent rows reads: W_uk [H][128][192] and the step's cosines and sines [n][rot_dims / 2]
-  const void* uk;
+  // what only the prompt kernel of latent rows reads: W_uk [H][128][192], W_uv [H][128][192] (may be null: latent results) and the step's cosines and sines [n][rot_dims / 2]
+  const void *uk, *uv;
   const float2* turn;
   int rot_halves;
 };

@@ -435,11 +435,14 @@ class LatentAttentionMixer(nn.Module):
         ops_seq.latent_prep(proj, 0, self.qr, self.q_norm, cq, self.eps, self.kv_col, r, dr, self.kv_norm, positions, rot,
                             owner.block_size, ctx.slot_mapping, owner.k_cache, owner.v_cache, turn)
         q = ops_seq.linear(cq, self.uq).view(n, H, d + dr)
-        lat = torch.empty(n, H * r, dtype=xh.dtype, device=xh.device)
         gate = proj[:, self.g_col:] if self.gated else None
-        if own and ops_seq.latent_prompt_fit(xh, self.uk, dr, rot, owner.k_cache, owner.block_size, ctx.portions):
-            ops_seq.latent_prompt(q, self.uk, rot, turn, gate, owner.k_cache, owner.v_cache, ctx.block_tables, owner.block_size, ctx.portions, self.scale,
-                                  self.window, lat)
+        prompt = own and ops_seq.latent_prompt_fit(xh, self.uk, dr, rot, owner.k_cache, owner.block_size, ctx.portions)
+        whole = prompt and dv == 128 and self.uv.is_contiguous() and self.uv.data_ptr() % 16 == 0
+        out = torch.empty(n, H, dv, dtype=xh.dtype, device=xh.device)
+        lat = out.view(n, H * dv) if whole else torch.empty(n, H * r, dtype=xh.dtype, device=xh.device)
+        if prompt:
+            ops_seq.latent_prompt(q, self.uk, self.uv if whole else None, rot, turn, gate, owner.k_cache, owner.v_cache, ctx.block_tables, owner.block_size,
+                                  ctx.portions, self.scale, self.window, lat)
         else:
             qf = torch.empty(n, H, r + dr, dtype=xh.dtype, device=xh.device)
             if own:
@@ -449,8 +452,9 @@ class LatentAttentionMixer(nn.Module):
                 ops_seq.rotate_heads(q[:, :, d:], qf[:, :, r:], positions, rot)
             ops_seq.window_attn(qf.view(n, H * (r + dr)), None, self.eps, gate, owner.k_cache, owner.v_cache, ctx.block_tables, owner.block_size, ctx.portions,
                                 H, 1, r + dr, r, self.scale, self.window, lat, gate_per_head=True)
-        out = torch.empty(n, H, dv, dtype=xh.dtype, device=xh.device)
-        if ops_seq.latent_heads_fit(xh, self.uv, r, dv):
+        if whole:
+            pass
+        elif ops_seq.latent_heads_fit(xh, self.uv, r, dv):
             ops_seq.latent_heads(lat.view(n, H, r), self.uv, out, False)
         else:
             torch.bmm(lat.view(n, H, r).transpose(0, 1), self.uv.transpose(1, 2), out=out.transpose(0, 1))   # W_uv on the latent output

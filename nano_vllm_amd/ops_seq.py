@@ -59,7 +59,7 @@ SIGNATURES = {
     "nvs_latent_prep": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _L, _P]),
     "nvs_latent_prep_turn": (c_int, [_P, _L, _I, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _F, _F, _I, _P, _P, _P, _P, _L, _P]),
     "nvs_latent_prompt_fits": (c_int, [_L, _I, _I, _I]),
-    "nvs_latent_prompt": (c_int, [_P, _L, _P, _P, _I, _I, _P, _L, _P, _P, _P, _L, _I, _P, _P, _I, _L, _I, _F, _I, _P, _P]),
+    "nvs_latent_prompt": (c_int, [_P, _L, _P, _P, _P, _I, _I, _P, _L, _P, _P, _P, _L, _I, _P, _P, _I, _L, _I, _F, _I, _P, _P]),
     "nvs_latent_heads": (c_int, [_P, _L, _I, _P, _I, _I, _I, _P, _L, _I, _I, _I, _I, _I, _P, _L, _P]),
     "nvs_rotate_heads": (c_int, [_P, _L, _I, _P, _L, _I, _I, _I, _I, _P, _P, _I, _I, _F, _L, _P]),
     "nvs_glu_act": (c_int, [_P, _L, _I, _I, _I, _F, _F, _L, _P, _P]),
@@ -642,8 +642,8 @@ def latent_heads(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, turned: bool
 
 def latent_prompt_fit(x: torch.Tensor, uk: torch.Tensor, tail: int, rot: Rotation | None, k_cache: torch.Tensor, block_size: int, por: Portions) -> bool:
     """Whether latent_prompt takes a step of x's rows: the sizes it is built for, where window_attn would take the same kernel.
-    MI355X, whole prompts, us, two calls / here: width 1,024, one of 17 tokens 792 / 744, one of 300 947 / 905, 32 of 100 to 400 1722 / 1513 (with the experts' tiles of
-    256 rows), 9 of 1,100 to 2,048 3270 / 3024; width 4,096, 7 of 1,100 to 2,000 6620 / 6367."""
+    MI355X, whole prompts, us, all calls one by one / the queries' product here / the values' too: width 1,024, one of 17 tokens 790 / 744 / 629, one of 300 947 / 905 / 791, 9 of
+    1,100 to 2,048 3270 / 3024 / 2899; width 4,096, 7 of 1,100 to 2,000 6620 / 6367 / 6358."""
     H, d, r = uk.shape
     return (x.is_cuda and x.dtype == uk.dtype == k_cache.dtype == torch.bfloat16 and (d, r, tail) == (128, 192, 64) and uk.is_contiguous()
             and (uk.data_ptr() | k_cache.data_ptr()) % 16 == 0 and (rot is None or rot.dims % 16 == 0)
@@ -651,18 +651,20 @@ def latent_prompt_fit(x: torch.Tensor, uk: torch.Tensor, tail: int, rot: Rotatio
 
 
 @_launch
-def latent_prompt(q: torch.Tensor, uk: torch.Tensor, rot: Rotation | None, turn: torch.Tensor | None, gate: torch.Tensor | None, k_cache, v_cache,
+def latent_prompt(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor | None, rot: Rotation | None, turn: torch.Tensor | None, gate: torch.Tensor | None, k_cache, v_cache,
                   block_tables: torch.Tensor, block_size: int, por: Portions, scale: float, window: int, out: torch.Tensor):
-    """latent_heads and window_attn of a step of prompts in one kernel: q [n, H, 128 + 64], uk [H, 128, 192], gate [n, H], out [n, H * 192]."""
+    """latent_heads and window_attn of a step of prompts in one kernel: q [n, H, 128 + 64], uk [H, 128, 192], gate [n, H], out [n, H * 192]. uv [H, 128, 192]: the
+    latent_heads behind it too, out [n, H * 128]."""
     lib = load_library()
     n, H = q.shape[0], q.shape[1]
     assert q.shape == (por.n, H, 192) and q.stride(2) == 1 and q.stride(1) == 192 and uk.shape == (H, 128, 192) and uk.is_contiguous()
-    assert out.shape == (n, H * 192) and out.is_contiguous() and (gate is None or (gate.shape == (n, H) and gate.stride(1) == 1))
+    assert uv is None or (uv.shape == (H, 128, 192) and uv.is_contiguous())
+    assert out.shape == (n, H * (192 if uv is None else 128)) and out.is_contiguous() and (gate is None or (gate.shape == (n, H) and gate.stride(1) == 1))
     assert rot is None or turn.shape == (n, rot.dims // 2, 2) and turn.is_contiguous() and turn.dtype == torch.float32
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1 and block_tables.shape[0] >= por.nseq
     assert tuple(k_cache.shape[1:]) == (1, 256) and tuple(v_cache.shape[1:]) == (1, 192)
-    assert _same(q, uk, gate, k_cache, v_cache, out) == _code(q) and q.dtype == torch.bfloat16
-    _check(lib.nvs_latent_prompt(_ptr(q), q.stride(0), _ptr(uk), _ptr(turn) if rot else None, rot.dims if rot else 0, int(rot.halves) if rot else 0, _ptr(gate),
+    assert _same(q, uk, uv, gate, k_cache, v_cache, out) == _code(q) and q.dtype == torch.bfloat16
+    _check(lib.nvs_latent_prompt(_ptr(q), q.stride(0), _ptr(uk), _ptr(uv), _ptr(turn) if rot else None, rot.dims if rot else 0, int(rot.halves) if rot else 0, _ptr(gate),
                                  gate.stride(0) if gate is not None else 0, _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), block_tables.stride(0), block_size, _ptr(por.cu_q), _ptr(por.ctx0), por.nseq,
                                  n, H, scale, window, _ptr(out), _stream()))
 

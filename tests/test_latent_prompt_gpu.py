@@ -1,5 +1,5 @@
-"""Latent attention of prompts with the queries' product in the attention kernel (nvs_latent_prompt) against the two calls it stands for, latent_heads and the scalar
-attention kernel: portions around the tiles of 32 queries and 64 keys, every number of heads a workgroup takes, windows, gates, part of the rotation or none, and pages
+"""Latent attention of prompts with the products per head in the attention kernel (nvs_latent_prompt) against the calls it stands for, latent_heads, the scalar
+attention kernel and, with W_uv, latent_heads again: portions around the tiles of 32 queries and 64 keys, every number of heads a workgroup takes, windows, gates, part of the rotation or none, and pages
 whose unused places hold infinities and NaN; then which steps take it."""
 import pytest
 import torch
@@ -51,15 +51,19 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("values", [False, True])
 @pytest.mark.parametrize("case", range(len(CASES)))
-def test_agrees_with_the_two_calls(case):
+def test_agrees_with_the_calls_it_stands_for(case, values):
     from nano_vllm_amd import ops_seq
     kw = dict(dict(gate=False, page=64, room=0, window=0, halves=False), **CASES[case])
     H, window, page = kw["H"], kw["window"], kw["page"]
     por, q, uk, rot, turn, gates, k, v, table = inputs(H, kw["lens"], kw["ctx"], kw["dims"], kw["gate"], page, case, kw["room"], kw["halves"])
-    got = torch.full((por.n, H * 192), 9.0, dtype=BF, device="cuda")
-    ops_seq.latent_prompt(q, uk, rot, turn, gates, k, v, table, page, por, 192 ** -0.5, window, got)
-    qf, want = torch.empty(por.n, H, 256, dtype=BF, device="cuda"), torch.empty_like(got)
+    uv = (torch.randn(H, 128, 192, generator=torch.Generator().manual_seed(50 + case)) / 192 ** 0.5).to(BF).cuda()
+    room = torch.full((por.n + 40, H * (128 if values else 192)), 9.0, dtype=BF, device="cuda")
+    got = room[:por.n]
+    ops_seq.latent_prompt(q, uk, uv if values else None, rot, turn, gates, k, v, table, page, por, 192 ** -0.5, window, got)
+    assert (room[por.n:] == 9.0).all()
+    qf, want = torch.empty(por.n, H, 256, dtype=BF, device="cuda"), torch.empty(por.n, H * 192, dtype=BF, device="cuda")
     ops_seq.latent_heads(q, uk, qf, True, 64, rot, turn)
     lib = ops_seq.load_library()
     lib.nvs_window_attn_force_scalar(1)
@@ -67,23 +71,32 @@ def test_agrees_with_the_two_calls(case):
         ops_seq.window_attn(qf.view(por.n, -1), None, 1e-6, gates, k, v, table, page, por, H, 1, 256, 192, 192 ** -0.5, window, want, gate_per_head=True)
     finally:
         lib.nvs_window_attn_force_scalar(0)
+    if values:
+        lat, want = want.view(por.n, H, 192), torch.empty(por.n, H, 128, dtype=BF, device="cuda")
+        ops_seq.latent_heads(lat, uv, want, False)
+        want = want.view(por.n, -1)
     got, want = got.double(), want.double()
     assert torch.isfinite(want).all()
-    # both round the finished query and the result to 8 bits; the matrix cores round the weights too (2^-9 each, averaged over the keys)
+    # both round the finished query and the result to 8 bits; the matrix cores round the weights too (2^-9 each, averaged over the keys); the latent result in
+    # front of W_uv is rounded on either side
     err = ((got - want).norm() / want.norm()).item()
     assert err <= 2.0 ** -7, err
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
 
 
-def test_no_further_from_the_exact_sum_than_the_two_calls():
-    """One rounding of the finished query instead of two."""
+@pytest.mark.parametrize("values", [False, True])
+def test_no_further_from_the_exact_sum_than_the_calls_it_stands_for(values):
+    """One rounding of the finished query instead of two; the same ones behind it."""
     from nano_vllm_amd import ops_seq
     H, T, page = 8, 500, 64
     mine = theirs = 0.0
     for seed in range(4):
         por, q, uk, rot, turn, _, k, v, table = inputs(H, [T], [0], 64, False, page, 100 + seed)
         got, two = torch.empty(T, H * 192, dtype=BF, device="cuda"), torch.empty(T, H * 192, dtype=BF, device="cuda")
-        ops_seq.latent_prompt(q, uk, rot, turn, None, k, v, table, page, por, 192 ** -0.5, 0, got)
+        uv = (torch.randn(H, 128, 192, generator=torch.Generator().manual_seed(seed)) / 192 ** 0.5).to(BF).cuda()
+        if values:
+            got = torch.empty(T, H * 128, dtype=BF, device="cuda")
+        ops_seq.latent_prompt(q, uk, uv if values else None, rot, turn, None, k, v, table, page, por, 192 ** -0.5, 0, got)
         qf = torch.empty(T, H, 256, dtype=BF, device="cuda")
         ops_seq.latent_heads(q, uk, qf, True, 64, rot, turn)
         ops_seq.window_attn(qf.view(T, -1), None, 1e-6, None, k, v, table, page, por, H, 1, 256, 192, 192 ** -0.5, 0, two, gate_per_head=True)
@@ -96,7 +109,13 @@ def test_no_further_from_the_exact_sum_than_the_two_calls():
         lat = torch.stack([x[:, h, :128] @ uk[h].double().cpu() for h in range(H)], 1)
         score = torch.matmul(torch.cat((lat, tail), -1).transpose(0, 1).contiguous(), K.T.contiguous()) * 192 ** -0.5
         p = score.masked_fill(torch.ones(T, T).triu(1).bool(), -torch.inf).softmax(-1)
-        want = torch.matmul(p, V).transpose(0, 1).reshape(T, -1)
+        want = torch.matmul(p, V)
+        if values:
+            want = torch.matmul(want, uv.double().cpu().transpose(1, 2).contiguous())
+            lat, two = two.view(T, H, 192), torch.empty(T, H, 128, dtype=BF, device="cuda")
+            ops_seq.latent_heads(lat, uv, two, False)
+            two = two.view(T, -1)
+        want = want.transpose(0, 1).reshape(T, -1)
         mine += ((got.double().cpu() - want).norm() / want.norm()).item()
         theirs += ((two.double().cpu() - want).norm() / want.norm()).item()
     assert mine <= theirs, (mine, theirs)
