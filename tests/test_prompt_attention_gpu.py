@@ -75,6 +75,25 @@ def test_prompt_kernel_agrees_with_the_scalar_kernel(d, dv, case):
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
 
 
+ORDERS = [
+    dict(lens=[40, 1, 0, 200, 64], ctx=[140000, 0, 0, 131050, 5], window=100),       # places beyond the first 64 x 64, a portion of nothing
+    dict(lens=[(7 * i) % 90 + 1 for i in range(64)], ctx=[(37 * i) % 300 for i in range(64)]),
+    dict(lens=[(7 * i) % 90 + 1 for i in range(65)], ctx=[(37 * i) % 300 for i in range(65)]),      # more than lanes: portion by portion
+    dict(lens=[4100], ctx=[31], chunk=64),
+]
+
+
+@pytest.mark.parametrize("d,dv", [(128, 128), (256, 192)])
+@pytest.mark.parametrize("case", range(len(ORDERS)))
+def test_every_tile_of_every_portion_is_somebodys(d, dv, case):
+    """The order of the tiles (the furthest positions first, whatever the portion) leaves none out: bounds as above."""
+    kw = dict(ORDERS[case], H=2, G=1, d=d, dv=dv, seed=20 + case)
+    got, want = call(False, **kw).double(), call(True, **kw).double()
+    err = ((got - want).norm() / want.norm()).item()
+    assert err <= 2.0 ** -7, err
+    assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
+
+
 def step(q, K, V, lens, ctx, H, G, d, dv, scale=1.0, window=0, sink=None, gates=None, per_head=False, page=64):
     """One call on sequences whose keys K [tokens of all, G, d] and values V [.., G, dv] lie in pages in order."""
     from nano_vllm_amd import ops_seq
