@@ -12,6 +12,7 @@ struct DeltaArgs {
   int64_t qkv_stride, gates_stride, b_col, a_col, decays_stride;
   int heads, G, dk, dv;
   float q_scale;
+  int by_length;                                    // (chunks) portions are taken longest first
 };
 
 constexpr float UNIT_EPS = 1e-6f;
@@ -282,8 +283,12 @@ __global__ __launch_bounds__(768) void delta_chunk_kernel(const DeltaArgs A) {
   constexpr int DKP = Lds::DKP;
   extern __shared__ __attribute__((aligned(16))) char chunk_lds[];
   Lds& W = *(Lds*)chunk_lds;
-  const int s = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t q0 = A.cu_q[s], q1 = A.cu_q[s + 1];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  PortionSpan span = {(int)blockIdx.y, 0, 0};
+  if (A.by_length) span = portion_by_length(A.cu_q, gridDim.y, blockIdx.y);
+  else span.t0 = A.cu_q[span.s], span.t1 = A.cu_q[span.s + 1];
+  const int s = span.s;
+  const int64_t q0 = span.t0, q1 = span.t1;
   if (q1 <= q0) return;
   const int dk = A.dk, dv = A.dv, grp = h / (A.heads / A.G);
   const int li = lane & 15, lq = lane >> 4;
@@ -601,13 +606,17 @@ __global__ __launch_bounds__(768) void delta_chunk_kernel(const DeltaArgs A) {
 }
 
 template <typename T, int DKT, bool CH>
-void launch_chunk_size(const DeltaArgs& A, int nseq, hipStream_t stream) {
+void launch_chunk_size(DeltaArgs A, int nseq, hipStream_t stream) {
   const int tiles = (A.dv + 15) / 16;
   // column wavefronts per workgroup: all columns of a head together (they share the preparation, which bounds a chunk's time), fewer
   // of them while the workgroups do not even fill half the chip (measured, 128 x 128 heads, 2,048 tokens: 256 pairs 780 us with 8
-  // wavefronts, 900 with 4, 1,690 with 2; 64 pairs 770 / 590 / 580)
+  // wavefronts, 900 with 4, 1,690 with 2; 64 pairs 770 / 590 / 580; 128 pairs of 700 to 2,000 tokens 563 / 432 / 616). Between half of the chip and all of it
+  // two halves that meet on a compute unit cost what they give: 144 pairs 650 / 671, 160 of one length 566 / 640, of 700 to 2,000 tokens 682 / 635
   int ncw = tiles < 8 ? tiles : 8;
-  while (ncw > 1 && (int64_t)A.heads * nseq * ((tiles + ncw - 1) / ncw) < 128) ncw = (ncw + 1) / 2;
+  while (ncw > 1 && (int64_t)A.heads * nseq * ((tiles + ncw - 1) / ncw) <= (ncw > 4 ? 128 : 127)) ncw = (ncw + 1) / 2;
+  // One workgroup of all columns fits a compute unit, so where there are more of them than units, a long portion that comes last runs by itself: longest first. 288 pairs of 1,109
+  // to 1,730 tokens 989 -> 937 us, 384 of 300 to 1,100 565 -> 471, 512 of 300 to 875 651 -> 471, 320 of 100 to 600 302 -> 230; of one length 1,055 both.
+  A.by_length = nseq >= 2 && nseq <= 64 && (int64_t)A.heads * nseq > 256;
   const size_t lds = sizeof(ChunkLds<DKT, CH>);
   if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)delta_chunk_kernel<T, DKT, CH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   delta_chunk_kernel<T, DKT, CH><<<dim3(A.heads, (unsigned)nseq, (unsigned)((tiles + ncw - 1) / ncw)), dim3(64 * (4 + ncw)), lds, stream>>>(A);
@@ -639,7 +648,7 @@ extern "C" int nvs_delta_scan(const void* qkv, int64_t qkv_stride, const void* g
               "nvs_delta_scan: columns beyond a row stride");
   if (n == 0 || nseq == 0) return NVS_OK;
   DeltaArgs A = {qkv, gates, decays, A_log, dt_bias, cu_q, ctx0, slot, S, y, qkv_stride, gates_stride, b_col, a_col, decays_stride,
-                 heads, G, dk, dv, q_scale};
+                 heads, G, dk, dv, q_scale, 0};
   const bool chunks = dk <= 256 && (g_delta_mode == 2 || (g_delta_mode == 0 && n > nseq && max_q >= CHUNK));
   if (chunks) {
     if (per_channel) {
