@@ -56,6 +56,13 @@ int nvs_add_group_norm(float* x, const void* a, float a_mult, const float* b, co
 int nvs_sandwich_norm(float* x, const void* a, float a_mult, const void* a2, float a2_mult, const void* wa, const int32_t* rows,
                       int64_t nrows, const void* w, float w_off, int dtype, int width, float eps, float* sum, void* out, void* stream);
 
+/* A routed layer's output (the operands of nvs_moe_combine, rounded to `dtype` as its out) in a's place: with wa == NULL nvs_add_group_norm of one group with a_mult = mult
+ * (w_off is not read), with wa nvs_sandwich_norm with a_mult = mult (center is 0). out == NULL: the add only. Rows of whole accesses of four columns: width % 4 == 0, up to
+ * 8192, row strides ldr and ldh % 4 == 0, pointers 16-byte aligned. */
+int nvs_chosen_norm(float* x, const void* rows, int64_t ldr, const int32_t* pair_row, const float* wts, int top, const void* h, int64_t ldh, const void* shared,
+                    const float* shared_gate, int64_t gate_stride, float mult, const void* wa, int64_t n, const void* w, float w_off, int dtype, int width, float eps,
+                    int center, void* out, void* stream);
+
 /* Residual update of a sublayer whose output is normed, with a layer scale, and the next sublayer's input. The output is
  * y[t, :] = a[t, :] (nullable) + sum_k wts[t, k] * rows[pair_row[t, k], :] (top choices of a routed layer, see nvs_moe_combine; top 0: none;
  * pair_row < 0: skipped); x[t, :] += rms(y[t, :]) * w * ls (ls nullable: no scale); out (nullable) receives the new x in `dtype`. a, rows (row

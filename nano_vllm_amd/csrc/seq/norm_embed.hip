@@ -276,25 +276,83 @@ __global__ void add_group_norm_kernel(float* __restrict__ x, const T* __restrict
   }
 }
 
+// A routed layer's output, not summed yet (nvs_moe_combine's operands): y[t] = sum_k wts[t, k] * (row pair_row[t, k], or h[t] where that is negative) + gate * shared[t]
+template <typename T>
+struct ChosenRows {
+  const T* rows;
+  int64_t ldr;
+  const int32_t* pair_row;
+  const float* wts;
+  int top;
+  const T* h;
+  int64_t ldh;
+  const T* shared;
+  const float* shared_gate;
+  int64_t gate_stride;
+};
+
+// y[t] in the activation type's rounding: what nvs_moe_combine writes
+template <typename T, int PER>
+__device__ __forceinline__ void chosen_row(const ChosenRows<T>& C, int64_t t, int width, float (&y)[PER][4]) {
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[i][e] = 0.f;
+  float sg = 0.f;
+  if (C.shared) sg = C.shared_gate ? 1.f / (1.f + expf(-C.shared_gate[t * C.gate_stride])) : 1.f;
+  for (int k = 0; k < C.top; ++k) {                 // (one by one: four asked for at once take more registers and as long or longer, 13,550 rows of 4,096 219 us)
+    const int r = C.pair_row[t * C.top + k];
+    const T* from = r >= 0 ? C.rows + (int64_t)r * C.ldr : C.h + t * C.ldh;        // (uniform over the workgroup)
+    const float p = C.wts[t * C.top + k];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = (i * blockDim.x + threadIdx.x) * 4;
+      if (c >= width) continue;
+      float v[4];
+      ldv<4>(from + c, v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[i][e] += p * v[e];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = (i * blockDim.x + threadIdx.x) * 4;
+    if (c >= width) continue;
+    if (C.shared) {
+      float v[4];
+      ldv<4>(C.shared + t * width + c, v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[i][e] += sg * v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[i][e] = (float)(T)y[i][e];
+  }
+}
+
 // The same for ONE group, four columns per access: the row stays in registers between the passes (PER accesses per thread). Centered,
 // 13,550 rows of 1,024 (bf16 input and output): 50 us a column at a time with the row read back, 29 here (4,096: 247, 130).
-template <typename T, int PER, bool CENTER>
+// CHOSEN: a routed layer's rows in a's place, summed here: a launch and a row's way to memory and back fewer (figures: ops_seq.ChosenRows).
+template <typename T, int PER, bool CENTER, bool CHOSEN>
 __global__ __launch_bounds__(256) void add_norm_row_kernel(float* __restrict__ x, const T* __restrict__ a, float a_mult, const float* __restrict__ b,
                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, int width, float eps,
-                                                           T* __restrict__ out) {
+                                                           T* __restrict__ out, const ChosenRows<T> C) {
   __shared__ float red[16];
   const int64_t r = blockIdx.x;
   const int64_t t = rows ? (int64_t)rows[r] : r;
   float* xr = x + t * width;
-  float v[PER][4];
+  float v[PER][4], y[PER][4];
   float ss = 0.f, sm = 0.f;
+  if constexpr (CHOSEN) chosen_row<T, PER>(C, t, width, y);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = (i * blockDim.x + threadIdx.x) * 4;
     if (c >= width) continue;
     ldv<4>(xr + c, v[i]);
     float u[4];
-    if (a) {
+    if constexpr (CHOSEN) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] += a_mult * y[i][e];
+    } else if (a) {
       ldv<4>(a + t * width + c, u);
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[i][e] += a_mult * u[e];
@@ -304,7 +362,7 @@ __global__ __launch_bounds__(256) void add_norm_row_kernel(float* __restrict__ x
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[i][e] += u[e];
     }
-    if (a || b) stv<4>(xr + c, v[i]);
+    if (CHOSEN || a || b) stv<4>(xr + c, v[i]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) CENTER ? sm += v[i][e] : ss += v[i][e] * v[i][e];
   }
@@ -371,11 +429,11 @@ __global__ void sandwich_norm_kernel(float* __restrict__ x, const T* __restrict_
   for (int c = threadIdx.x; c < width; c += blockDim.x) stf(out + r * width + c, xr[c] * k * (w_off + ldf(w + c)));
 }
 
-// The same with the rows in registers, four columns per access (PER accesses per thread).
-template <typename T, int PER>
+// The same with the rows in registers, four columns per access (PER accesses per thread). CHOSEN: a routed layer's rows in a's place, summed here.
+template <typename T, int PER, bool CHOSEN>
 __global__ __launch_bounds__(256) void sandwich_row_kernel(float* __restrict__ x, const T* __restrict__ a, float a_mult, const T* __restrict__ a2,
                                                            float a2_mult, const T* __restrict__ wa, const int32_t* __restrict__ rows,
-                                                           const T* __restrict__ w, float w_off, int width, float eps, T* __restrict__ out) {
+                                                           const T* __restrict__ w, float w_off, int width, float eps, T* __restrict__ out, const ChosenRows<T> C) {
   __shared__ float red[16];
   const int64_t r = blockIdx.x;
   const int64_t t = rows ? (int64_t)rows[r] : r;
@@ -385,13 +443,14 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(float* __restrict__ x
     const int c = (i * blockDim.x + threadIdx.x) * 4;
     if (c < width) ldv<4>(x + t * width + c, v[i]);
   }
-  if (a) {
+  if (CHOSEN || a) {
     float y[PER][4], ss = 0.f;
+    if constexpr (CHOSEN) chosen_row<T, PER>(C, t, width, y);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int c = (i * blockDim.x + threadIdx.x) * 4;
       if (c >= width) continue;
-      ldv<4>(a + t * width + c, y[i]);
+      if constexpr (!CHOSEN) ldv<4>(a + t * width + c, y[i]);
       float u[4] = {0.f, 0.f, 0.f, 0.f};
       if (a2) ldv<4>(a2 + t * width + c, u);
 #pragma unroll
@@ -762,10 +821,10 @@ extern "C" int nvs_add_group_norm(float* x, const void* a, float a_mult, const f
   const int per = groups == 1 ? row_plan(width, al, &row_threads) : 0;
   if (per) {
 #define NVS_ROW(PER)                                                                                                           \
-  NVS_DISPATCH(dtype, if (center) add_norm_row_kernel<T, PER, true><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
-                          x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out);                                     \
-                      else add_norm_row_kernel<T, PER, false><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
-                          x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out))
+  NVS_DISPATCH(dtype, if (center) add_norm_row_kernel<T, PER, true, false><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
+                          x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out, ChosenRows<T>{});                    \
+                      else add_norm_row_kernel<T, PER, false, false><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>( \
+                          x, (const T*)a, a_mult, b, rows, (const T*)w, width, eps, (T*)out, ChosenRows<T>{}))
     NVS_ROW_CASES(per, NVS_ROW)
 #undef NVS_ROW
     return nvs_check_launch("nvs_add_group_norm (one group)");
@@ -788,8 +847,8 @@ extern "C" int nvs_sandwich_norm(float* x, const void* a, float a_mult, const vo
   const int per = row_plan(width, (uintptr_t)x | (uintptr_t)a | (uintptr_t)a2 | (uintptr_t)wa | (uintptr_t)w | (uintptr_t)out, &row_threads);
   if (per) {
 #define NVS_ROW(PER)                                                                                                           \
-  NVS_DISPATCH(dtype, sandwich_row_kernel<T, PER><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>(         \
-                          x, (const T*)a, a_mult, (const T*)a2, a2_mult, (const T*)wa, rows, (const T*)w, w_off, width, eps, (T*)out))
+  NVS_DISPATCH(dtype, sandwich_row_kernel<T, PER, false><<<dim3((unsigned)nrows), dim3(row_threads), 0, (hipStream_t)stream>>>(         \
+                          x, (const T*)a, a_mult, (const T*)a2, a2_mult, (const T*)wa, rows, (const T*)w, w_off, width, eps, (T*)out, ChosenRows<T>{}))
     NVS_ROW_CASES(per, NVS_ROW)
 #undef NVS_ROW
     return nvs_check_launch("nvs_sandwich_norm (rows in registers)");
@@ -797,6 +856,31 @@ extern "C" int nvs_sandwich_norm(float* x, const void* a, float a_mult, const vo
   NVS_DISPATCH(dtype, sandwich_norm_kernel<T><<<dim3((unsigned)nrows), dim3(threads_for(width)), 0, (hipStream_t)stream>>>(
                           x, (const T*)a, a_mult, (const T*)a2, a2_mult, (const T*)wa, rows, (const T*)w, w_off, width, eps, sum, (T*)out));
   return nvs_check_launch("nvs_sandwich_norm");
+}
+
+// nvs_moe_combine and behind it nvs_add_group_norm (one group; wa == NULL) or nvs_sandwich_norm (wa), in one pass with the same sums and roundings
+extern "C" int nvs_chosen_norm(float* x, const void* rows, int64_t ldr, const int32_t* pair_row, const float* wts, int top, const void* h, int64_t ldh,
+                               const void* shared, const float* shared_gate, int64_t gate_stride, float mult, const void* wa, int64_t n, const void* w, float w_off,
+                               int dtype, int width, float eps, int center, void* out, void* stream) {
+  NVS_REQUIRE(x && rows && pair_row && wts && h && top > 0 && n >= 0 && ldr >= width && ldh >= width && (!out || w) && (!shared_gate || shared) && !(wa && center),
+              "nvs_chosen_norm: bad argument (width %d, %d choices)", width, top);
+  int row_threads = 0;
+  const uintptr_t al = (uintptr_t)x | (uintptr_t)rows | (uintptr_t)h | (uintptr_t)shared | (uintptr_t)wa | (uintptr_t)w | (uintptr_t)out;
+  const int per = width > 0 && ((ldr | ldh) & 3) == 0 ? row_plan(width, al, &row_threads) : 0;
+  NVS_REQUIRE(per > 0, "nvs_chosen_norm: width %d (whole accesses of four columns, up to 8192), row strides %lld and %lld", width, (long long)ldr, (long long)ldh);
+  if (n == 0) return NVS_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)n), block(row_threads);
+#define NVS_ROW(PER)                                                                                                                                                    \
+  NVS_DISPATCH(dtype, {                                                                                                                                                 \
+    const ChosenRows<T> C = {(const T*)rows, ldr, pair_row, wts, top, (const T*)h, ldh, (const T*)shared, shared_gate, gate_stride};                                    \
+    if (wa) sandwich_row_kernel<T, PER, true><<<grid, block, 0, st>>>(x, nullptr, mult, nullptr, 1.f, (const T*)wa, nullptr, (const T*)w, w_off, width, eps, (T*)out, C); \
+    else if (center) add_norm_row_kernel<T, PER, true, true><<<grid, block, 0, st>>>(x, nullptr, mult, nullptr, nullptr, (const T*)w, width, eps, (T*)out, C);          \
+    else add_norm_row_kernel<T, PER, false, true><<<grid, block, 0, st>>>(x, nullptr, mult, nullptr, nullptr, (const T*)w, width, eps, (T*)out, C);                     \
+  })
+  NVS_ROW_CASES(per, NVS_ROW)
+#undef NVS_ROW
+  return nvs_check_launch("nvs_chosen_norm");
 }
 
 extern "C" int nvs_branch_norm(float* x, const void* a, const void* rows, int64_t ldr, const int32_t* pair_row, const float* wts, int top, int dtype,

@@ -21,7 +21,7 @@ Per-step dataflow on the MI355X (bf16 serving; with dtype float32 every tensor b
                       gated memory scan (fp32 state) -> per-head norm + gate kernel -> out GEMM; the sandwich kernel adds both
     dense ff:         up GEMM -> GELU kernel -> down GEMM
     moe ff:           table route kernel -> plan kernel -> grouped [gate|up] product (SiLU GLU fused) -> grouped down product ->
-                      combine kernel (weights, shared expert)
+                      weights, shared expert: summed by the next sandwich norm kernel
 
 All sizes, the layer order and the design's free constants come from config.json; the 1e-6 in the memory's divisor, the
 memory's running maximum starting at 0 and the GELU's constants are fixed by the design.
@@ -34,7 +34,7 @@ from torch import nn
 from . import ops_seq
 from .attn_meta import get_context, plain_calls
 from .mixers import (AttentionMemoryMixer, ConvAttentionMixer, GeluFeedForward, RoutedExperts, _copy_into, _param,
-                     banded_rotary_frequencies, tie_parameters)
+                     banded_rotary_frequencies, routed_output, tie_parameters)
 
 
 class LobidraConfig:
@@ -176,7 +176,7 @@ class LobidraForCausalLM(nn.Module):
                 pending = (layer.mixer(h, positions), None, 1.0, 1.0, layer.norm1b)
             if layer.mlp is not None:
                 h = sandwich(layer.norm2)
-                y = layer.mlp(h, input_ids) if layer.routed else layer.mlp(h)
+                y = routed_output(layer.mlp, h, input_ids) if layer.routed else layer.mlp(h)
                 pending = (y, None, 1.0, 1.0, layer.norm2b)
             if trace is not None:
                 sandwich(None)

@@ -19,7 +19,8 @@ Per-step dataflow on the MI355X (bf16 serving; with dtype float32 every tensor b
     lightning:        [v|k|q|g] GEMM -> decay scan (SiLU fused, fp32 state) -> norm + sigmoid gate kernel -> out GEMM
     dense ff:         [gate|up] GEMM -> clamped GLU kernel -> down GEMM
     moe ff:           router GEMM (fp32) -> route kernel -> plan kernel -> grouped [gate|up] product (SiLU GLU fused) ->
-                      grouped down product -> combine kernel (weights, pass-through experts, gated shared expert)
+                      grouped down product (weights, pass-through experts, gated shared expert: summed by the next
+                      add + norm kernel where the row is one group, by a combine kernel otherwise)
 
 All sizes, the layer order and the design's free constants come from config.json; the slope of the dense unit's sigmoid
 (1.702) and the router's 1e-20 are fixed by the design.
@@ -31,7 +32,7 @@ from torch import nn
 
 from . import ops_seq
 from .attn_meta import get_context, plain_calls
-from .mixers import AttentionMixer, ClampedGLU, LightningMixer, RoutedExperts, _copy_into, _param, tie_parameters
+from .mixers import AttentionMixer, ClampedGLU, LightningMixer, RoutedExperts, _copy_into, _param, routed_output, tie_parameters
 
 
 class NokipelConfig:
@@ -160,7 +161,7 @@ class NokipelForCausalLM(nn.Module):
             if layer.mlp is not None:
                 h = torch.empty(n, cfg.hidden_size, dtype=self.dtype, device=dev)
                 ops_seq.add_group_norm(x, layer.norm2, cfg.norm_groups, cfg.eps, h, a=pending)
-                pending = layer.mlp(h)
+                pending = routed_output(layer.mlp, h)
             if trace is not None:
                 ops_seq.add_group_norm(x, None, cfg.norm_groups, cfg.eps, None, a=pending)
                 pending = None

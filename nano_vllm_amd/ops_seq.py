@@ -46,6 +46,7 @@ SIGNATURES = {
     "nvs_shift_norm": (c_int, [_P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _L, _I, _F, _P, _P, _P, _P]),
     "nvs_gated_lookup": (c_int, [_P, _L, _P, _L, _L, _I, _P, _I, _L, _P, _P]),
     "nvs_qk_rows": (c_int, [_P, _L, _I, _P, _P, _L, _I, _P, _F, _I, _I, _I, _I, _P, _P, _P, _I, _L, _P, _P, _P, _I, _I, _P, _L, _P, _P, _P, _P]),
+    "nvs_chosen_norm": (c_int, [_P, _P, _L, _P, _P, _I, _P, _L, _P, _P, _L, _F, _P, _L, _P, _F, _I, _I, _F, _I, _P, _P]),
     "nvs_branch_norm": (c_int, [_P, _P, _P, _L, _P, _P, _I, _I, _L, _P, _P, _I, _F, _P, _P]),
     "nvs_qkv_store": (c_int, [_P, _P, _P, _L, _I, _I, _I, _I, _I, _P, _P, _I, _I, _F, _I, _F, _F, _P, _L, _P, _I, _P, _L, _P, _P, _P]),
     "nvs_pool_rows": (c_int64, [_I, _I]),
@@ -464,12 +465,58 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, b_col: int, a_col: int, d
                               _ptr(S), _ptr(y), _stream()))
 
 
+class ChosenRows:
+    """A routed layer's output before it is summed (RoutedExperts.parts, and the layer's input for pass-through choices). add_group_norm and sandwich_norm take it in a's
+    place and sum it on the way where they can. MI355X, us, sum and norm as launches of their own / in one, 16-bit rows: 64 rows of 1,024, three choices 4.9 / 3.5, of 4,096,
+    four 7.0 / 6.7; four choices, 2,000 rows of 1,024 10.3 / 7.3, 14,200 of 1,024 52 / 41, of 2,048 131 / 104; three, 13,550 of 4,096 225 / 176."""
+    __slots__ = ("h", "rows", "plan", "wts", "shared", "gate")
+
+    def __init__(self, h: torch.Tensor, rows: torch.Tensor, plan: "MoePlan", wts: torch.Tensor, shared: torch.Tensor | None, gate: torch.Tensor | None):
+        self.h, self.rows, self.plan, self.wts, self.shared, self.gate = h, rows, plan, wts, shared, gate
+
+    def sum(self) -> torch.Tensor:
+        out = torch.empty(self.h.shape, dtype=self.h.dtype, device=self.h.device)
+        moe_combine(self.rows, self.plan, self.wts, self.h, self.shared, self.gate, out)
+        return out
+
+    def fits(self, x: torch.Tensor, *others: torch.Tensor | None) -> bool:
+        """Whether nvs_chosen_norm takes the row: whole accesses of four columns, aligned."""
+        width = x.shape[1]
+        if width % 4 or width > 8192 or self.rows.stride(0) % 4 or self.h.stride(0) % 4:
+            return False
+        al = 0
+        for t in (x, self.rows, self.h, self.shared, *others):
+            if t is not None:
+                al |= t.data_ptr()
+        return al % 16 == 0
+
+
+def _chosen_norm(x: torch.Tensor, c: ChosenRows, mult: float, wa: torch.Tensor | None, w: torch.Tensor | None, w_off: float, eps: float, center: bool,
+                 out: torch.Tensor | None):
+    n, width = x.shape
+    h, rows, plan, wts, shared, gate = c.h, c.rows, c.plan, c.wts, c.shared, c.gate
+    assert x.dtype == torch.float32 and x.is_contiguous() and h.shape == x.shape and h.stride(1) == 1
+    assert rows.stride(1) == 1 and rows.shape[1] == width and wts.dtype == torch.float32 and wts.is_contiguous() and wts.shape[0] == n
+    assert plan.pair_row.shape == wts.shape and (shared is None or (shared.shape == x.shape and shared.is_contiguous()))
+    assert gate is None or (shared is not None and gate.dtype == torch.float32 and gate.shape[0] == n)
+    assert out is None or (out.shape == x.shape and out.is_contiguous() and w.numel() == width)
+    assert wa is None or wa.numel() == width
+    _check(load_library().nvs_chosen_norm(_ptr(x), _ptr(rows), rows.stride(0), _ptr(plan.pair_row), _ptr(wts), wts.shape[1], _ptr(h), h.stride(0), _ptr(shared),
+                                          _ptr(gate), gate.stride(0) if gate is not None else 0, mult, _ptr(wa), n, _ptr(w), w_off,
+                                          _same(rows, h, shared, wa, w, out), width, eps, int(center), _ptr(out), _stream()))
+
+
 @_launch
 def add_group_norm(x: torch.Tensor, w: torch.Tensor | None, groups: int, eps: float, out: torch.Tensor | None,
-                   a: torch.Tensor | None = None, b: torch.Tensor | None = None, a_mult: float = 1.0, center: bool = False):
+                   a: "torch.Tensor | ChosenRows | None" = None, b: torch.Tensor | None = None, a_mult: float = 1.0, center: bool = False):
     """x += a_mult * a + b (in place; a in the activation type, b 32-bit, both optional), then out = group_rms(x) * w (out None:
     adds only; w None: out is the sum itself in the activation type); center: every group's mean is taken off first (layer norm without bias)."""
     lib = load_library()
+    if type(a) is ChosenRows:
+        weight = w if out is not None else None
+        if (groups == 1 or out is None) and b is None and (out is None or w is not None) and a.fits(x, weight, out):
+            return _chosen_norm(x, a, a_mult, None, weight, 0.0, eps, center and out is not None, out)
+        a = a.sum()
     n, width = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
     assert a is None or (a.shape == x.shape and a.is_contiguous())
@@ -494,11 +541,16 @@ def group_norm_rows(x: torch.Tensor, rows: torch.Tensor | None, nrows: int, w: t
 
 
 @_launch
-def sandwich_norm(x: torch.Tensor, a: torch.Tensor | None, wa: torch.Tensor | None, w: torch.Tensor | None, eps: float,
+def sandwich_norm(x: torch.Tensor, a: "torch.Tensor | ChosenRows | None", wa: torch.Tensor | None, w: torch.Tensor | None, eps: float,
                   out: torch.Tensor | None, a2: torch.Tensor | None = None, a_mult: float = 1.0, a2_mult: float = 1.0, w_off: float = 1.0):
     """x += rms(a_mult * a + a2_mult * a2) * (w_off + wa) (in place; a None: no add), then out = rms(x) * (w_off + w) (out None: no
     second norm)."""
     lib = load_library()
+    if type(a) is ChosenRows:
+        weight = w if out is not None else None
+        if a2 is None and wa is not None and a.fits(x, wa, weight, out):
+            return _chosen_norm(x, a, a_mult, wa, weight, w_off, eps, False, out)
+        a = a.sum()
     n, width = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
     assert a is None or (a.shape == x.shape and a.is_contiguous() and wa is not None and wa.numel() == width)

@@ -24,7 +24,7 @@ Per-step dataflow on the MI355X (bf16 serving; with dtype float32 every tensor b
                     per-head W_uk^T q (batched GEMM) + query rotation kernel -> paged attention in the latent space (mask and
                     gate fused) -> per-head W_uv (batched GEMM) -> out GEMM
     feed-forward:   router GEMM (fp32) -> route kernel -> plan kernel -> grouped up product (squared ReLU fused) -> grouped
-                    down product -> combine kernel
+                    down product (the next add + norm kernel sums a token's choices)
     logits:         norm of the wanted rows -> head GEMM -> scale + cap kernel (fp32)
 
 All sizes, the layer order and the design's free constants come from config.json; 0.1 in the magnitude factor of scaled
@@ -37,7 +37,7 @@ from torch import nn
 
 from . import ops_seq
 from .attn_meta import get_context, plain_calls
-from .mixers import LatentAttentionMixer, RoutedExperts, _copy_into, _param
+from .mixers import LatentAttentionMixer, RoutedExperts, _copy_into, _param, routed_output
 
 MIXERS = ("latent_attention", "latent_attention_2")
 
@@ -147,7 +147,7 @@ class PefazenForCausalLM(nn.Module):
             if layer.mlp is not None:
                 h = torch.empty(n, cfg.hidden_size, dtype=self.dtype, device=dev)
                 ops_seq.add_group_norm(x, layer.norm2, 1, cfg.eps, h, a=pending, a_mult=m, center=True)
-                pending = layer.mlp(h)
+                pending = routed_output(layer.mlp, h)
             if trace is not None:
                 ops_seq.add_group_norm(x, None, 1, cfg.eps, None, a=pending, a_mult=m)
                 pending = None
