@@ -5,7 +5,7 @@
 // What bounds it: many rows by reading them (111 MB at 5.1 TB/s, 22 us), few by one chain of requests and by how fast a compute unit takes the router's rows in;
 // long reductions of few rows are therefore shared by up to eight workgroups and chosen from by a second launch (64 rows of 4,096: 17 -> 13 us). A workgroup takes 16 MT rows and all entries; its eight
 // wavefronts share the reduction as in linear_rows.hip (rings of one piece of 128 bytes of the rows and the same k of the router's rows, straight into
-// LDS), the sums meet in LDS, and four lanes per row choose.
+// LDS), the sums meet in LDS, and 4 or 16 lanes per row choose.
 //
 // bf16 rows times 32-bit weights on the bf16 matrix instructions: a weight is the sum of three bf16 numbers exactly (its leading 8 bits, the next 8 and
 // the last 8, each cut off the rest), their products with bf16 entries are exact in 32 bits, and only sums are rounded, as in a 32-bit product; the
@@ -46,110 +46,130 @@ __device__ __forceinline__ u32x4_t cut(float (&v)[8]) {
   return out;
 }
 
-__device__ __forceinline__ float quad_swap(float v, int o) { return __shfl_xor(v, o, 64); }
+constexpr int LD = MAX_ROUTER + 1;                    // logits in LDS: [row][entry]
 
-constexpr int LD = MAX_ROUTER + 1;                    // logits in LDS: [row][entry], group scores [row][MAX_ROUTER] behind them
+// the value of a lane N further in the same 16 (or, of four lanes a row, of lane ^ N): plain VALU moves, no LDS
+template <int LANES, int N>
+__device__ __forceinline__ int other(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, LANES == 16 ? 0x120 + N : N == 1 ? 0xB1 : 0x4E, 0xf, 0xf, false);
+}
+template <int LANES, int N>
+__device__ __forceinline__ float other(float v) { return __builtin_bit_cast(float, other<LANES, N>(__builtin_bit_cast(int, v))); }
+template <int LANES>
+__device__ __forceinline__ float row_max(float v) {
+  if constexpr (LANES == 16) v = fmaxf(v, other<LANES, 8>(v)), v = fmaxf(v, other<LANES, 4>(v));
+  v = fmaxf(v, other<LANES, 2>(v));
+  return fmaxf(v, other<LANES, 1>(v));
+}
+template <int LANES>
+__device__ __forceinline__ float row_sum(float v) {     // (the same number in every lane: additions commute)
+  if constexpr (LANES == 16) v += other<LANES, 8>(v), v += other<LANES, 4>(v), v += other<LANES, 2>(v), v += other<LANES, 1>(v);
+  else v += other<LANES, 1>(v), v += other<LANES, 2>(v);
+  return v;
+}
+struct Choice {
+  float c, s;
+  int at;
+};
+template <int LANES, int N>
+__device__ __forceinline__ void better_of(Choice& a) {  // the better choice score; a lower index wins a tie
+  const float c = other<LANES, N>(a.c), s = other<LANES, N>(a.s);
+  const int at = other<LANES, N>(a.at);
+  if (c > a.c || (c == a.c && at < a.at)) a = Choice{c, s, at};
+}
 
-// Choices and weights of rows r0 .. r0 + rows - 1 from their logits z: four lanes per row, lane q of them holds entries q, q + 4, ... Every thread of
-// the workgroup calls it, four per row at least.
-template <int NT>
-__device__ __forceinline__ void route_rows(const RouterArgs& a, float* z, float* groups, int r0, int rows) {
-  const int lane = threadIdx.x & 63, row = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const bool mine = row < rows && r0 + row < a.n;
-  constexpr int PER = NT * 4;
+// Choices and weights of row r0 + row (row < rows) from its logits in LDS: LANES lanes, lane p of them holds entries p, p + LANES, ... What they tell each other goes
+// by moves between lanes; through LDS it took 0.5 us a choice. 16 lanes a row are the shorter chain, four the fewer instructions: 33 entries, four choices, us, four by way of LDS /
+// 16 by moves, 64 rows of 1,024 9.5 / 8.1, of 4,096 13.9 / 10.1; 14,200 rows of 1,024, four by way of LDS / 16 / four by moves 14.9 / 16.0 / 14.5.
+template <int NT, int LANES>
+__device__ __forceinline__ void route_row(const RouterArgs& a, float* z, int r0, int row, int rows) {
+  constexpr int PER = NT * 16 / LANES;
+  const int lane = threadIdx.x & 63, p = lane & (LANES - 1), p0 = lane & (64 - LANES);
+  if (row >= rows || r0 + row >= a.n) return;         // (the row's lanes together)
   float s[PER], c[PER];
   float* zr = z + row * LD;
-  if (mine) {
-    float mx = -INFINITY, sum_s = 0.f;
+  float mx = -INFINITY, sum_s = 0.f;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = q + 4 * i;
-      s[i] = e < a.total ? zr[e] : -INFINITY;
-      mx = fmaxf(mx, s[i]);
-    }
-    if (a.gate && a.entries > a.total && q == 0) a.gate[r0 + row] = zr[a.total];
-    mx = fmaxf(mx, quad_swap(mx, 1)), mx = fmaxf(mx, quad_swap(mx, 2));
+  for (int i = 0; i < PER; ++i) {
+    const int e = p + LANES * i;
+    s[i] = e < a.total ? zr[e] : -INFINITY;
+    mx = fmaxf(mx, s[i]);
+  }
+  if (a.gate && a.entries > a.total && p == 0) a.gate[r0 + row] = zr[a.total];
+  mx = row_max<LANES>(mx);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = q + 4 * i;
-      if (a.score == 1) s[i] = e < a.total ? 1.f / (1.f + expf(-s[i])) : 0.f;
-      else s[i] = e < a.total ? expf(s[i] - mx) : 0.f;
-      sum_s += s[i];
-    }
-    sum_s += quad_swap(sum_s, 1), sum_s += quad_swap(sum_s, 2);
-    if (a.score == 1) sum_s = 1.f;
+  for (int i = 0; i < PER; ++i) {
+    const int e = p + LANES * i;
+    if (a.score == 1) s[i] = e < a.total ? 1.f / (1.f + expf(-s[i])) : 0.f;
+    else s[i] = e < a.total ? expf(s[i] - mx) : 0.f;
+    sum_s += s[i];
+  }
+  sum_s = a.score == 1 ? 1.f : row_sum<LANES>(sum_s);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = q + 4 * i;
-      s[i] = s[i] / sum_s;
-      c[i] = e < a.total ? s[i] + (a.correction ? a.correction[e] : 0.f) : -INFINITY;
-    }
+  for (int i = 0; i < PER; ++i) {
+    const int e = p + LANES * i;
+    s[i] = s[i] / sum_s;
+    c[i] = e < a.total ? s[i] + (a.correction ? a.correction[e] : 0.f) : -INFINITY;
   }
   if (a.count > 1) {                                // a group's score is its best choice score; entries outside the `keep` best groups cannot be chosen
-    const int per = a.total / a.count;
-    float* gr = groups + row * MAX_ROUTER;
-    if (mine) {
+    const int per = a.total / a.count, inverse = (65536 + per - 1) / per;      // (e * inverse >> 16 is e / per: e < 64)
+    float own[PER];                                 // lane p: the scores of groups p, p + LANES, ... (a group has an entry at least: no more of them than entries)
+    int better[PER], group[PER];
 #pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if (q + 4 * i < a.total) zr[q + 4 * i] = c[i];
-    }
-    __syncthreads();
-    if (mine) {
-      for (int g = q; g < a.count; g += 4) {
+    for (int i = 0; i < PER; ++i) group[i] = (p + LANES * i) * inverse >> 16;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      own[j] = -INFINITY, better[j] = 0;
+      for (int l = 0; l < LANES && j * LANES + l < a.count; ++l) {
         float v = -INFINITY;
-        for (int j = 0; j < per; ++j) v = fmaxf(v, zr[g * per + j]);
-        gr[g] = v;
-      }
-    }
-    __syncthreads();
-    if (mine) {
-      unsigned long long dropped = 0;               // the number of groups that beat one, a lower index winning a tie
-      for (int g = q; g < a.count; g += 4) {
-        const float own = gr[g];
-        int better = 0;
-        for (int j = 0; j < a.count; ++j) better += j != g && (gr[j] > own || (gr[j] == own && j < g));
-        if (better >= a.keep) dropped |= 1ull << g;
-      }
-      dropped |= __shfl_xor(dropped, 1, 64), dropped |= __shfl_xor(dropped, 2, 64);
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int e = q + 4 * i;
-        if (e < a.total && dropped >> (e / per) & 1) c[i] = -INFINITY;
+        for (int i = 0; i < PER; ++i)
+          if (group[i] == j * LANES + l) v = fmaxf(v, c[i]);
+        v = row_max<LANES>(v);
+        if (p == l) own[j] = v;
       }
     }
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      for (int l = 0; l < LANES && j * LANES + l < a.count; ++l) {
+        const float v = __shfl(own[j], p0 + l, 64);
+#pragma unroll
+        for (int i = 0; i < PER; ++i)               // (the number of groups that beat one, a lower index winning a tie)
+          if (LANES * i < a.count) better[i] += v > own[i] || (v == own[i] && j * LANES + l < p + LANES * i);
+      }
+    unsigned long long dropped = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (LANES * j < a.count) dropped |= (__ballot(p + LANES * j < a.count && better[j] >= a.keep) >> p0 & ((1ull << LANES) - 1)) << (LANES * j);
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (dropped >> (group[i] & 63) & 1) c[i] = -INFINITY;      // (entries behind the last one are out anyway)
   }
-  if (!mine) return;
-  float chosen_s = 0.f, denom = 0.f;                // lane q holds choices q, q + 4, ...: written as they come, divided at the end
+  float denom = 0.f;                                // lane p holds choices p, p + LANES, ...: written as they come, divided at the end
   for (int k = 0; k < a.top; ++k) {
-    float best = -INFINITY, best_s = 0.f;
-    int at = 0x7fffffff;
+    Choice best = {-INFINITY, 0.f, 0x7fffffff};
 #pragma unroll
     for (int i = 0; i < PER; ++i)
-      if (c[i] > best) best = c[i], best_s = s[i], at = q + 4 * i;       // (entries of a lane ascend: the first best stays)
-#pragma unroll
-    for (int o = 1; o < 4; o <<= 1) {
-      const float v = quad_swap(best, o), vs = quad_swap(best_s, o);
-      const int w = __shfl_xor(at, o, 64);
-      if (v > best || (v == best && w < at)) best = v, best_s = vs, at = w;
-    }
-    if (at == 0x7fffffff) {                         // nothing that can be chosen (scores that are not numbers): entry 0
-      at = 0;
-      best_s = __shfl(s[0], lane & ~3, 64);
+      if (c[i] > best.c) best = Choice{c[i], s[i], p + LANES * i};            // (entries of a lane ascend: the first best stays)
+    if constexpr (LANES == 16) better_of<LANES, 8>(best), better_of<LANES, 4>(best);
+    better_of<LANES, 2>(best), better_of<LANES, 1>(best);
+    if (best.at == 0x7fffffff) {                    // nothing that can be chosen (scores that are not numbers): entry 0
+      best.at = 0;
+      best.s = __shfl(s[0], p0, 64);
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i)
-      if (q + 4 * i == at) c[i] = -INFINITY;
-    denom += best_s;
-    if ((k & 3) == q) {
-      a.ids[(int64_t)(r0 + row) * a.top + k] = at;
-      chosen_s = best_s;
-      if (a.renorm) zr[k] = chosen_s;               // (the row's logits are no longer read)
-      else a.wts[(int64_t)(r0 + row) * a.top + k] = chosen_s * a.scale;
+      if (p + LANES * i == best.at) c[i] = -INFINITY;
+    denom += best.s;
+    if ((k & (LANES - 1)) == p) {
+      a.ids[(int64_t)(r0 + row) * a.top + k] = best.at;
+      if (a.renorm) zr[k] = best.s;                 // (the row's logits are no longer read)
+      else a.wts[(int64_t)(r0 + row) * a.top + k] = best.s * a.scale;
     }
   }
   if (a.renorm) {
     denom += 1e-20f;
-    for (int k = q; k < a.top; k += 4) a.wts[(int64_t)(r0 + row) * a.top + k] = zr[k] / denom * a.scale;
+    for (int k = p; k < a.top; k += LANES) a.wts[(int64_t)(r0 + row) * a.top + k] = zr[k] / denom * a.scale;
   }
 }
 
@@ -273,14 +293,17 @@ __global__ __launch_bounds__(NW * 64) void moe_router_kernel(RouterArgs a) {
     }
   }
   __syncthreads();
-  route_rows<NT>(a, z, z + MT * 16 * LD, r0, MT * 16);
+  constexpr int LANES = MT <= 2 ? 16 : 4;
+  static_assert(MT * 16 * LANES <= NW * 64, "a row's lanes");
+  route_row<NT, LANES>(a, z, r0, tid / LANES, MT * 16);
 }
-// the sums of a split reduction, added in order, and their choices: 32 rows per workgroup
+
+// the sums of a split reduction, added in order, and their choices: 16 rows per workgroup
 template <int NT>
-__global__ __launch_bounds__(128) void moe_router_parts_kernel(RouterArgs a) {
-  __shared__ float z[32 * (LD + MAX_ROUTER)];
-  const int r0 = blockIdx.x * 32;
-  for (int u = threadIdx.x; u < 32 * NT * 4; u += 128) {
+__global__ __launch_bounds__(256) void moe_router_parts_kernel(RouterArgs a) {
+  __shared__ float z[16 * LD];
+  const int r0 = blockIdx.x * 16;
+  for (int u = threadIdx.x; u < 16 * NT * 4; u += 256) {
     const int row = u / (NT * 4), e = u % (NT * 4) * 4;
     if (r0 + row >= a.n) break;
     const float* p = a.parts + (int64_t)(r0 + row) * (NT * 16) + e;
@@ -290,17 +313,17 @@ __global__ __launch_bounds__(128) void moe_router_parts_kernel(RouterArgs a) {
     for (int k = 0; k < 4; ++k) z[row * LD + e + k] = v[k] + (a.bias && e + k < a.entries ? a.bias[e + k] : 0.f);
   }
   __syncthreads();
-  route_rows<NT>(a, z, z + 32 * LD, r0, 32);
+  route_row<NT, 16>(a, z, r0, threadIdx.x / 16, 16);
 }
 
 template <typename T, int NT, int MT>
 int launch_router(const RouterArgs& a, hipStream_t st) {
   constexpr int LDS = NW * (MT * 16 * 128 + NT * 16 * (sizeof(T) == 2 ? 256 : 128));
-  static_assert(LDS >= MT * 16 * (2 * MAX_ROUTER + 1) * 4, "logits and group scores");
+  static_assert(LDS >= MT * 16 * LD * 4, "logits");
   const auto kernel = moe_router_kernel<T, NT, MT>;
   NVS_LDS_ROOM(kernel, LDS, "nvs_moe_router");
   kernel<<<dim3((unsigned)((a.n + MT * 16 - 1) / (MT * 16)), (unsigned)a.splits), dim3(NW * 64), LDS, st>>>(a);
-  if (a.parts) moe_router_parts_kernel<NT><<<dim3((unsigned)((a.n + 31) / 32)), dim3(128), 0, st>>>(a);
+  if (a.parts) moe_router_parts_kernel<NT><<<dim3((unsigned)((a.n + 15) / 16)), dim3(256), 0, st>>>(a);
   return nvs_check_launch("nvs_moe_router");
 }
 
