@@ -344,8 +344,11 @@ class LinearBase(nn.Module):
             y = decode_linear(x, w, ops.LINEAR_BF16, packed=self.weight_packed)
             if y is not None:
                 return y
-        if rows >= ops_seq.TILES_FROM and ops_seq.loaded() and ops_seq.many_rows(x, w, b):
-            return ops_seq.linear_tiles(x, w, b)
+        if ops_seq.loaded():
+            if rows >= ops_seq.TILES_FROM and ops_seq.many_rows(x, w, b):
+                return ops_seq.linear_tiles(x, w, b)
+            if DECODE_LINEAR_MAX_ROWS < rows <= ops_seq.SOME_ROWS_TO and ops_seq.some_rows(x, w, b):
+                return ops_seq.linear_rows(x, w, b)
         return F.linear(x, w, b)
 
 
@@ -519,7 +522,7 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
             if y is not None:
                 return y
         if pair and ops_seq.loaded() and ops_seq.silu_linear_fits(x, w):
-            tm = ops_seq.silu_linear_rows(x.shape[0], w.shape[0] // 2, x.shape[1])
+            tm = ops_seq.silu_linear_rows(x.shape[0], w.shape[0] // 2, x.shape[1]) or (256 if ops_seq.silu_short_steps(x.shape[0], x.shape[1]) else 0)
             if tm:
                 return ops_seq.silu_linear(x, w, tm)
         return ops.silu_mul(self.forward(x))

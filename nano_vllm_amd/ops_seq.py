@@ -853,9 +853,40 @@ def many_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -
             and (b is None or type(b) in _PLAIN and b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1] and b.data_ptr() % 16 == 0))
 
 
+SOME_ROWS_TO = 1024
+
+
+def rows_rule(m: int, N: int, K: int, captured: bool = False) -> bool:
+    """Whether x w^T of m rows beyond a decode step's goes to nvs_linear_rows: its tiles of 64 x 64 are one pass (those of a column tile stay on one of eight XCDs, 32 of them at a
+    time), and a call of it takes the host 3 us, one of the library's product 20. MI355X, us of the GPU, weights from memory, here / the library's: 320 rows, 1024 x 1024 5.7 / 8.6,
+    x 2048 7.4 / 9.3, x 3072 9.3 / 11.8, 2304 x 1024 7.8 / 9.0, 2048 x 2048 10.0 / 10.9; 512 rows, 2048 x 2048 11.0 / 11.5, x 6144 26.1 / 27.6; 1,000 rows, 1024 x 1024 8.0 / 9.3, x 2048
+    11.1 / 11.4, x 3072 14.5 / 15.3; more than a pass 400 rows, 2304 x 1024 13.0 / 9.3, 767 rows, 1040 x 1024 12.2 / 9.4. Two passes of a short reduction still take less than the
+    library's call does the host, which such steps wait for (320 rows, 4096 x 1024 13.4 / 10.2, 512: 14.0 / 11.2; a prompt step of 28 layers and 326 rows 4,130 -> 2,750): where nothing is
+    captured."""
+    passes = -(-(-(-N // 64)) // 8) * -(-m // 64) / 32
+    return passes <= 1 or passes <= 2 and K <= 1024 and not captured
+
+
+def some_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
+    if x.dim() != 2 or w.dim() != 2:
+        return False
+    (m, k), (N, wide), (ld, unit) = x.shape, w.shape, x.stride()
+    return (m > 0 and N > 0 and k == wide and k > 0 and k % 64 == 0 and unit == 1 and ld % 8 == 0 and ld >= k and x.dtype == w.dtype == torch.bfloat16
+            and rows_rule(m, N, k, True if k > 1024 else torch.cuda.is_current_stream_capturing()) and x.is_cuda and x.device == w.device and w.is_contiguous() and _only_the_result(x, w)
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and (b is None or type(b) in _PLAIN and b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1]))
+
+
+def linear_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
+    return _linear_rows(x, w, b, -1, 0.0, 0.0, torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device))
+
+
 def _linear_many(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
-    if x.shape[0] >= TILES_FROM and many_rows(x, w, b):         # (asked first: short steps wait for the host)
+    m = x.shape[0]
+    if m >= TILES_FROM and many_rows(x, w, b):         # (asked first: short steps wait for the host)
         return linear_tiles(x, w, b)
+    if m <= SOME_ROWS_TO and some_rows(x, w, b):
+        return linear_rows(x, w, b)
     return torch.nn.functional.linear(x, w, b)
 
 
@@ -902,6 +933,12 @@ def silu_linear_rows(n: int, ff: int, K: int) -> int:
     return 256 if tiles >= 96 and (n >= 768 or K <= 1536) or tiles >= 48 and n >= 500 and K <= 1024 else 0
 
 
+def silu_short_steps(n: int, K: int) -> bool:
+    """Whether gate|up and SiLU of fewer rows than silu_linear_rows gives tiles of 256 rows take those all the same: short reductions in steps that wait for the host, whose call of the
+    library's product takes 20 us, this one 3. MI355X, us of the GPU, ff 3072, K 1024, here / the product and the activation: 320 rows 20.4 / 17, 640: 20.6 / 19."""
+    return 64 <= n < TILES_FROM and 128 <= K <= 1024 and K % 64 == 0 and not torch.cuda.is_current_stream_capturing()
+
+
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     if x.dim() != 2 or w.dim() != 2:
         return False
@@ -931,7 +968,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, ff: int, kind: int = 0, limit: 
     if _few_rows(x, w, True):
         return _linear_rows(x, w, None, kind, limit, alpha, out)
     if kind == 0 and silu_linear_fits(x, w):
-        tm = silu_linear_rows(x.shape[0], ff, x.shape[1])
+        tm = silu_linear_rows(x.shape[0], ff, x.shape[1]) or (256 if silu_short_steps(x.shape[0], x.shape[1]) else 0)
         if tm:
             return silu_linear(x, w, tm, out)
     glu_act(_linear_many(x, w), ff, out, kind, limit, alpha)
