@@ -700,7 +700,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
     const int ol = out_tid & 63, oq = ol & 31, oh = ol >> 5, ow = __builtin_amdgcn_readfirstlane(out_tid >> 6);
     const int live = len - rel0 < 32 ? len - rel0 : 32;
     const float inv = 1.f / (l + other_half(l));
-    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + rel0) * A.gate_stride + h : nullptr;
+    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + (live > 0 ? rel0 : len - 1)) * A.gate_stride + h : nullptr;      // (nobody's queries: a row that is there)
     const float ginv = gp ? inv * sigmoid_hw((float)gp[(int64_t)(oq < live ? oq : 0) * A.gate_stride]) : inv;
     char* at = lds + ow * 4 * PIECE;
     const char* wbase = (const char*)A.uv + (int64_t)h * OUT * DV * 2;
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
     const int ol = out_tid & 63, oq = ol & 31, oh = ol >> 5, ow = __builtin_amdgcn_readfirstlane(out_tid >> 6);
     const int live = len - rel0 < 32 ? len - rel0 : 32;                           // (none: a wavefront of nobody's queries)
     const float inv = 1.f / (l + other_half(l));
-    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + rel0) * A.gate_stride + (int64_t)h * A.gate_w : nullptr;
+    const bf16_t* gp = A.gate ? (const bf16_t*)A.gate + (int64_t)(row0 + (live > 0 ? rel0 : len - 1)) * A.gate_stride + (int64_t)h * A.gate_w : nullptr;      // (nobody's queries: a row that is there)
     const bool wide = gp && A.gate_w != 1, units = wide && (A.gate_stride & 7) == 0 && ((uintptr_t)gp & 15) == 0;
     const float ginv = gp && !wide ? inv * sigmoid_hw((float)gp[(int64_t)(oq < live ? oq : 0) * A.gate_stride]) : inv;
     bf16_t* op = (bf16_t*)A.out + ((int64_t)(row0 + rel0) * H + h) * DV;
