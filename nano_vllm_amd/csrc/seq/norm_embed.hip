@@ -508,9 +508,7 @@ __global__ __launch_bounds__(256) void branch_norm_row_kernel(float* __restrict_
     const int c = (i * blockDim.x + threadIdx.x) * 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[i][e] = 0.f;
-    if (c >= width) continue;
-    ldv<4>(x + t * width + c, v[i]);
-    if (a) ldv<4>(a + t * width + c, y[i]);
+    if (c < width && a) ldv<4>(a + t * width + c, y[i]);
   }
   for (int k = 0; k < top; ++k) {
     const int r = pair_row[t * top + k];
@@ -528,9 +526,12 @@ __global__ __launch_bounds__(256) void branch_norm_row_kernel(float* __restrict_
   }
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < PER; ++i)
+  for (int i = 0; i < PER; ++i) {
+    const int c = (i * blockDim.x + threadIdx.x) * 4;
+    if (c < width) ldv<4>(x + t * width + c, v[i]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss += y[i][e] * y[i][e];
+  }
   const float k = 1.f / sqrtf(block_sum(ss, red) / (float)width + eps);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
