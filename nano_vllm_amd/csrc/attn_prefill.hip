@@ -618,7 +618,10 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t k
                 "nvl_attn_prefill_varlen: bad K/V token strides");
   }
   if (total_q == 0 || num_seqs == 0) return NVL_OK;
-  const bool pair = raw && num_q_heads / num_kv_heads % 2 == 0;
+  // Two heads a workgroup where a group has an even number of them, but for a few short portions behind long contexts: there it halves the workgroups that ask for the cache's
+  // pages (10 portions of 44 to 69 rows behind 2,304 tokens, 16 heads over 8, pages from memory: 104 workgroups 59.8 us, 160 of one head 55.1; more of them than compute
+  // units, 32 portions of 60 to 64 behind 1,024: 32.7 and 38.4).
+  const bool pair = raw && num_q_heads / num_kv_heads % 2 == 0 && !(paged && total_q <= 64ll * num_seqs && (int64_t)num_q_heads * num_seqs <= 256);
   const int rows = pair ? kQBlk / 2 : kQBlk, heads = pair ? 2 : 1;
   const int64_t tiles = (total_q + rows - 1) / rows + num_seqs;  // upper bound on sum ceil(Lq / rows)
   NVL_REQUIRE(tiles < (1ll << 31), "nvl_attn_prefill_varlen: too many query tiles");

@@ -77,3 +77,25 @@ def test_positions_as_they_are_given(hq, hkv, where):
     want = ops.attn_prefill_varlen(q, k, v, cu, cu, max(lens), 128 ** -0.5)
     got = ops.attn_prefill_raw(qkv, hq, pos, None, 1e-6, table, k, v, cu, cu, max(lens), 128 ** -0.5)
     assert torch.equal(got, want)                               # the same roundings throughout
+
+
+@pytest.mark.parametrize("lens", [[64, 10, 33], [64, 65, 10], [65, 64, 64], [20] * 16, [20] * 17, [64]])
+def test_short_portions_behind_pages(lens):
+    """One head a workgroup up to a mean of 64 rows and 256 pairs (portion, head), two beyond: either is the call on finished queries."""
+    from nano_vllm_amd import ops
+    hq, hkv, page, before = 16, 8, 64, 130
+    g = torch.Generator(device="cuda").manual_seed(len(lens))
+    n, per = sum(lens), -(-(before + max(lens)) // page)
+    qkv = torch.randn(n, (hq + 2 * hkv) * 128, generator=g, device="cuda").bfloat16()
+    angle = torch.arange(512, device="cuda").float()[:, None] * 1e6 ** (-torch.arange(0, 128, 2, device="cuda").float() / 128)
+    table = torch.cat([angle.cos(), angle.sin()], 1).contiguous()
+    pos = torch.cat([torch.arange(before, before + m) for m in lens]).cuda()
+    kc, vc = (torch.randn(per * len(lens), hkv, page, 128, generator=g, device="cuda").bfloat16() for _ in range(2))
+    bt = torch.arange(per * len(lens), dtype=torch.int32, device="cuda").view(len(lens), per)
+    cu_q = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    cu_k = torch.tensor([0] + [m + before for m in lens]).cumsum(0).to(torch.int32).cuda()
+    q, k = (torch.empty(n, h, 128, device="cuda", dtype=torch.bfloat16) for h in (hq, hkv))
+    ops.qknorm_rope_kvstore(qkv, pos, None, None, 1e-6, table, None, q, k, None, None, hq, hkv)
+    want = ops.attn_prefill_varlen(q, kc, vc, cu_q, cu_k, max(lens), 128 ** -0.5, block_tables=bt)
+    got = ops.attn_prefill_raw(qkv, hq, pos, None, 1e-6, table, kc, vc, cu_q, cu_k, max(lens), 128 ** -0.5, block_tables=bt)
+    assert torch.equal(got, want)                               # the same roundings throughout
