@@ -467,8 +467,8 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, b_col: int, a_col: int, d
 
 class ChosenRows:
     """A routed layer's output before it is summed (RoutedExperts.parts, and the layer's input for pass-through choices). add_group_norm and sandwich_norm take it in a's
-    place and sum it on the way where they can. MI355X, us, sum and norm as launches of their own / in one, 16-bit rows: 64 rows of 1,024, three choices 4.9 / 3.5, of 4,096,
-    four 7.0 / 6.7; four choices, 2,000 rows of 1,024 10.3 / 7.3, 14,200 of 1,024 52 / 41, of 2,048 131 / 104; three, 13,550 of 4,096 225 / 176."""
+    place and sum it on the way where they can. MI355X, us, sum and norm as launches of their own / in one, 16-bit rows: 64 rows of 1,024, three choices 4.9 / 3.5;
+    four choices, 2,000 rows of 1,024 10.3 / 7.3, 14,200 of 1,024 52 / 41, of 2,048 131 / 104; three, 13,550 of 4,096 225 / 176."""
     __slots__ = ("h", "rows", "plan", "wts", "shared", "gate")
 
     def __init__(self, h: torch.Tensor, rows: torch.Tensor, plan: "MoePlan", wts: torch.Tensor, shared: torch.Tensor | None, gate: torch.Tensor | None):
@@ -480,9 +480,10 @@ class ChosenRows:
         return out
 
     def fits(self, x: torch.Tensor, *others: torch.Tensor | None) -> bool:
-        """Whether nvs_chosen_norm takes the row: whole accesses of four columns, aligned."""
-        width = x.shape[1]
-        if width % 4 or width > 8192 or self.rows.stride(0) % 4 or self.h.stride(0) % 4:
+        """Whether nvs_chosen_norm takes the rows: whole accesses of four columns, aligned. Few wide rows stay two launches, the sum's spreads a row over several workgroups (a step
+        of 70 rows of 4,096, one routed layer: 848 us, 852 in one)."""
+        n, width = x.shape
+        if n <= 512 and width > 2048 or width % 4 or width > 8192 or self.rows.stride(0) % 4 or self.h.stride(0) % 4:
             return False
         al = 0
         for t in (x, self.rows, self.h, self.shared, *others):
@@ -864,7 +865,7 @@ def rows_rule(m: int, N: int, K: int, captured: bool = False) -> bool:
     library's call does the host, which such steps wait for (320 rows, 4096 x 1024 13.4 / 10.2, 512: 14.0 / 11.2; a prompt step of 28 layers and 326 rows 4,130 -> 2,750): where nothing is
     captured."""
     passes = -(-(-(-N // 64)) // 8) * -(-m // 64) / 32
-    return passes <= 1 or passes <= 2 and K <= 1024 and not captured
+    return passes <= 1 and m > 256 or passes <= 2 and K <= 1024 and not captured          # (up to 256 rows: _few_rows, whose line was measured there)
 
 
 def some_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:

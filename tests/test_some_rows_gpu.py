@@ -47,6 +47,7 @@ def test_a_captured_product_of_two_passes_is_the_library_s_and_one_of_one_pass_i
     from nano_vllm_amd import ops_seq
     assert ops_seq.rows_rule(400, 4096, 1024) and not ops_seq.rows_rule(400, 4096, 1024, captured=True) and not ops_seq.rows_rule(400, 4096, 2048)
     assert ops_seq.rows_rule(1000, 1024, 4096, captured=True) and not ops_seq.rows_rule(1025, 1024, 4096) and not ops_seq.rows_rule(770, 1040, 2048)
+    assert not ops_seq.rows_rule(64, 12288, 4096) and not ops_seq.rows_rule(256, 4096, 4096) and ops_seq.rows_rule(257, 2048, 4096)
     x, w = torch.randn(400, 1024, device="cuda").bfloat16(), torch.randn(1024, 1024, device="cuda").bfloat16()
     with torch.inference_mode():
         want = ops_seq.linear(x, w)
