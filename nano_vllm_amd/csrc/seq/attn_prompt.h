@@ -23,6 +23,12 @@ __device__ __forceinline__ float other_half(float v) {                          
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
 }
+// (a, b) turns. Which of a sum's two products is rounded by itself is said here: left to the compiler, it changed with code around it, and from one pair of a row to the next.
+__device__ __forceinline__ void turn_pair(float& a, float& b, float cs, float sn) {
+  const float a2 = __builtin_fmaf(a, cs, -(b * sn));
+  b = __builtin_fmaf(b, cs, a * sn);
+  a = a2;
+}
 template <int N>
 struct Int { static constexpr int value = N; };
 template <int BEGIN, int END, typename F>
@@ -287,9 +293,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
           } else {
             sincosf((float)pos * A.rot_freq[col >> 1], &sn, &cs);
           }
-          const float a2 = a * cs - b * sn;
-          b = b * cs + a * sn;
-          a = a2;
+          turn_pair(a, b, cs, sn);
         }
         qb[c][e] = (bf16_t)a, qb[c][e + 1] = (bf16_t)b;
       }
@@ -420,9 +424,7 @@ __global__ __launch_bounds__(64 * NW, D == 128 ? 2 : 1) void window_attn_prompt_
         if (col + e < A.rot_dims) {                 // the pair (2i, 2i+1) turns by pos * freq[i]
           float sn, cs;
           sincosf((float)pos * A.rot_freq[(col + e) >> 1], &sn, &cs);
-          const float a = v[e] * cs - v[e + 1] * sn;
-          v[e + 1] = v[e + 1] * cs + v[e] * sn;
-          v[e] = a;
+          turn_pair(v[e], v[e + 1], cs, sn);
         }
       }
     };

@@ -252,3 +252,27 @@ def test_prompt_kernel_against_float64(d, dv, H, G, window, sink, gated, page):
         want *= torch.sigmoid(gates.double()).view(n, H, dv)
     assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
     assert ((got - want).abs().max() / want.pow(2).mean().sqrt()).item() <= 0.1
+
+
+def test_equal_pairs_turn_to_equal_bits():
+    """All pairs of a query's row alike and of one frequency: their rotations are the same two 16-bit numbers whichever pair it is. Key j of the 128 in the pages shows entry j alone,
+    value j counts in column j alone, so that column is the weight of the entry's score, times up to 30 here: an entry one unit of the last place off (rotations whose products are not
+    rounded alike: about one row of 2^16) has another weight."""
+    from nano_vllm_amd import ops_seq
+    H, seqs, T, page = 32, 128, 256, 128                   # a million (query, head)
+    n, d = seqs * T, 128
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randn(n, H, 1, 2, generator=g, device="cuda").bfloat16().expand(n, H, 64, 2).reshape(n, H * d)
+    kc = torch.zeros(3, page, 1, d, dtype=torch.bfloat16, device="cuda")        # page 0: the keys that show; 1 and 2: the portions' own
+    vc = torch.zeros(3, 1, d, page, dtype=torch.bfloat16, device="cuda")
+    kc[0, :, 0] = 8 * torch.eye(128, device="cuda")
+    vc[0, 0] = torch.eye(128, device="cuda")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    por = ops_seq.Portions(i32([T * i for i in range(seqs + 1)]), i32([page] * seqs), i32(list(range(seqs))), torch.arange(seqs).repeat_interleave(T).to(torch.int32).cuda(), seqs, n, T)
+    freq = torch.full((64,), 0.37, device="cuda")
+    out = torch.empty(n, H * d, dtype=torch.bfloat16, device="cuda")
+    ops_seq.window_attn(q, None, 1e-6, None, kc.view(-1, 1, d), vc.view(-1, 1, d), i32([[0, 1, 2]] * seqs), page, por, H, 1, d, d, 1.0, 0, out, rot_freq=freq)
+    pairs = out.view(-1, 64, 2)
+    assert not bool(torch.isnan(pairs).any()) and bool((pairs > 0).any())
+    apart = (pairs != pairs[:, :1]).any(-1).any(-1).sum().item()
+    assert apart == 0, f"{apart} of {n * H} rows"
