@@ -149,11 +149,15 @@ int nvl_norm_linear(const void* x, int slabs, const void* residual, const void* 
  *   x: bf16 [batch, hidden], the embeddings. layers: 10 pointers a layer, all bf16: input norm, qkv [(hq + 2 hkv) 128, hidden], q norm, k norm (NULL both: none), o
  *     [hidden, hq 128], the second norm, gate | up [2 ff, hidden], down [hidden, ff] (row-major), k cache, v cache. The new token's key and value are stored.
  *   hidden_out: fp32 [batch, hidden], the last layer's output rounded to bf16 (one slab of nvl_add_rmsnorm_splitk); residual_out: bf16 [batch, hidden].
- *   context_lens <= 0: a row that fills up a captured step. patience: how often a workgroup looks whether all run together before the shares are dealt (0: once). */
+ *   context_lens <= 0: a row that fills up a captured step. patience: how often a workgroup looks whether all run together before the shares are dealt (0: once).
+ *   asks: how often a workgroup asks again for what another one hands on before it gives up (1 << 21: 1.5 s; 0: the step counts as given up from its start). A step that was given
+ *     up stores no key or value that is not the new token's, has NaN where its results are not those of the step, and sets *gave_up (device int32, may be NULL) to 1; nothing clears
+ *     it. */
 size_t nvl_decode_step_workspace_bytes(int64_t batch, int num_layers, int hidden, int ff, int num_q_heads, int num_kv_heads);
 int nvl_decode_step(const void* x, const void* const* layers, int num_layers, float eps, const float* cos_sin, int64_t max_pos, const int32_t* block_tables,
                     int64_t bt_stride, const int32_t* context_lens, int64_t batch, int hidden, int ff, int num_q_heads, int num_kv_heads, int block_size,
-                    float softmax_scale, float* hidden_out, void* residual_out, void* workspace, size_t workspace_bytes, int patience, void* stream);
+                    float softmax_scale, float* hidden_out, void* residual_out, void* workspace, size_t workspace_bytes, int patience, int asks, int32_t* gave_up,
+                    void* stream);
 
 /* Fused split-K reduction + residual add + RMSNorm: replaces
  * RMSNorm.add_rms_forward (layers/layernorm.py:28-40) when its input is the

@@ -8,7 +8,8 @@ callers work unchanged; four extra fields carry what the HIP decode kernel needs
 workspace, the static `max_context` bound that makes the launch hipGraph-safe, the per-step work
 plan shared by every layer's launch — ops.decode_plan — and whether that plan carries a shared prefix), and one carries
 the packed-portion description that stateful layers read (`portions`: ops_seq.Portions — per portion its token rows, the
-tokens earlier steps already processed and its state slot).
+tokens earlier steps already processed and its state slot). `decode_gave_up` (int32 [1]) is the word a decode step in one
+launch sets when it gave up waiting (ops.decode_step); without it such a step shows by the NaN in its logits alone.
 """
 from __future__ import annotations
 
@@ -17,8 +18,8 @@ import functools
 import torch
 
 _FIELDS = ("is_prefill", "cu_seqlens_q", "cu_seqlens_k", "max_seqlen_q", "max_seqlen_k", "slot_mapping",
-           "context_lens", "block_tables", "decode_workspace", "max_context", "decode_plan", "shared_prefix", "portions")
-_DEFAULTS = (False, None, None, 0, 0, None, None, None, None, 0, None, False, None)
+           "context_lens", "block_tables", "decode_workspace", "max_context", "decode_plan", "shared_prefix", "portions", "decode_gave_up")
+_DEFAULTS = (False, None, None, 0, 0, None, None, None, None, 0, None, False, None, None)
 
 
 class Context:
@@ -46,7 +47,7 @@ def get_context() -> Context:
 
 def set_context(*args, **kwargs) -> None:
     """set_context(is_prefill, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-    slot_mapping, context_lens, block_tables[, decode_workspace, max_context, decode_plan, shared_prefix])"""
+    slot_mapping, context_lens, block_tables[, decode_workspace, max_context, decode_plan, shared_prefix, portions, decode_gave_up])"""
     _Holder.current = Context(*args, **kwargs)
 
 

@@ -10,7 +10,9 @@
 // Forward progress. Items (a phase's shares) have an order, and an item waits for items before it alone. When all 256 workgroups are seen to run at once (they count themselves
 // at the start), each takes the item of its own number in every phase. When they are not all there in time (other launches hold their places), the step's mode becomes
 // "dealt": items are taken in order from a counter, so whoever holds the first unfinished one can go on, with any number of workgroups on the chip. One word, changed once by
-// compare-and-swap, holds the decision for all. Waits are bounded all the same: a reader that has asked two million times goes on with what is there, a NaN.
+// compare-and-swap, holds the decision for all. Waits are bounded all the same: a reader that has asked in vain as often as its caller allows says so, in a sync word and in the
+// caller's, and then goes on with what is there, a NaN, which makes the rows it is part of NaN. Such a key or value of the new token is not stored once the sync word is set: it is
+// looked at behind the words that the row is made of, and set in front of everything that a reader who gave up leads to.
 //
 // A workgroup is eight wavefronts that multiply and four that fetch. A matrix is cut into 256 shares of 16 operand rows: 16 output features of the whole reduction (qkv), or 8
 // features in halves of the reduction (gate|up, 4 + 4 features a tile, three tiles), or 4 features in quarters (o, down); the other operand's columns are (row, part of
@@ -30,7 +32,6 @@ constexpr int kMaxLayers = 40, kWidth = 1024, kMaxFf = 3072, kMaxParts = 32;
 constexpr int kChunk = 32;                       // keys the multiplying wavefronts take at once: four each
 constexpr int kHeld = 4;                         // chunks requested ahead
 constexpr float kNegBig = -1.0e30f, kHidden = -3e38f;
-constexpr int kMaxAsks = 1 << 21;
 // Pauses before a phase's words are first asked for, about 100 clocks each. An answer "empty" takes 0.7 us as any other does, and 256 workgroups that ask without a pause keep the
 // few channels the words lie on busy: a phase that hands 8 KB on took 2.2 us so and 1.6 with 1,300 clocks between handing on and asking. 14 to 26 for 20, 35 to 65 for 50
 // and 45 to 80 for 60 are the same step within 1 %; gate|up with 14, 20, 26: 503, 497, 492 us a step.
@@ -48,9 +49,10 @@ struct StepArgs {
   unsigned int* ws;                              // sync words [64]; then the layers' exchange words; then v of the step's input
   float* hidden;
   bf16_t* residual;
+  int32_t* gave_up;
   int64_t bt_stride, max_pos;
   float eps, scale_log2e;
-  int layers, rows, hq, hkv, ff, block_size, parts;
+  int layers, rows, hq, hkv, ff, block_size, parts, asks;
 };
 
 // words of a layer's exchange, in order
@@ -186,6 +188,14 @@ struct Step {
   }
 
   // ---- fetching ---------------------------------------------------------------------------------------------------
+  __device__ __forceinline__ void give_up() {
+    if (!broken && lane == 0) {
+      __hip_atomic_store(a.ws + 4, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (a.gave_up) __hip_atomic_store(a.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    broken = true;
+    __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): the words are there before the barrier behind which this phase's results are handed on
+  }
   // N units of 16 bytes a lane, `units` in all; and one more, at byte `at` of another place
   template <int N, bool ONE>
   __device__ __forceinline__ void fetch(const unsigned int* src, int units, u32x4_t (&v)[N], const unsigned int* one, int at, u32x4_t& w) {
@@ -201,8 +211,8 @@ struct Step {
       for (int i = 0; i < N; ++i) ok = ok && there(v[i]);
       if constexpr (ONE) ok = ok && there(w);
       if (__all(ok)) break;
-      if (broken || asks >= kMaxAsks) {
-        broken = true;
+      if (broken || asks >= a.asks) {
+        give_up();
         break;
       }
     }
@@ -478,15 +488,21 @@ struct Step {
       asm volatile("" ::: "memory");
       raw = __builtin_amdgcn_raw_buffer_load_b128(rs, head * 256 + sub * 16, 0, kPastCaches);
       if (__all(there(raw))) break;
-      if (broken || asks >= kMaxAsks) {
-        broken = true;
+      if (broken || asks >= a.asks) {
+        give_up();
         break;
       }
     }
+    const bool odd = broken || __any((raw[0] & 0x7FFFu) > 0x7F80u);        // words that were given up elsewhere make NaN of a whole row
     const u32x4_t turned = norm_rope_head_regs(raw, nw != nullptr, wraw, a.eps, rr, sub);
     const u32x4_t row = fw == 1 && (r & 1) ? raw : turned;
     if (r < 2) *reinterpret_cast<u32x4_t*>(&sh.head[fw * 2 + r][sub * 4]) = row;
-    if (fw == 1 && r < 2) *reinterpret_cast<u32x4_t*>((r == 0 ? a.layer[l].kc : a.layer[l].vc) + row_of(at, at.len - 1)) = row;        // for later steps
+    bool keep = true;
+    if (odd) {                                   // (an answer takes 0.7 us: no other row asks. Us a step of one sequence of 700 tokens, never asking 495.6, so 497.5, in every row 505)
+      asm volatile("" ::: "memory");
+      keep = __hip_atomic_load(a.ws + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+    }
+    if (fw == 1 && r < 2 && keep) *reinterpret_cast<u32x4_t*>((r == 0 ? a.layer[l].kc : a.layer[l].vc) + row_of(at, at.len - 1)) = row;        // for later steps
   }
 
   __device__ __forceinline__ void attention_fetch(int l, const Place& at, const Cut& cut) {
@@ -599,8 +615,8 @@ struct Step {
 #pragma unroll
       for (int i = 0; i < kMaxParts / 4; ++i) ok = ok && there(o[i]);
       if (__all(ok)) break;
-      if (broken || asks >= kMaxAsks) {
-        broken = true;
+      if (broken || asks >= a.asks) {
+        give_up();
         break;
       }
     }
@@ -769,7 +785,7 @@ struct Step {
   }
 };
 
-// sync words: [0] workgroups that have come, [1] the mode (0 open, 1 fixed, 2 dealt), [2] the next share, [3] asks before the mode is dealt
+// sync words: [0] workgroups that have come, [1] the mode (0 open, 1 fixed, 2 dealt), [2] the next share, [3] looks before the mode is dealt, [4] whether a wait gave up
 template <int MR>
 __global__ __launch_bounds__(kThreads) void decode_step_kernel(const StepArgs a) {
   __shared__ StepShared<MR> sh;
@@ -804,7 +820,8 @@ __global__ __launch_bounds__(kThreads) void decode_step_dealt_kernel(const StepA
 }
 
 // empty exchange words, the sync words, the step's input as v in front of the first layer
-__global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws, int64_t exchange, const bf16_t* __restrict__ x, int n, unsigned int asks) {
+__global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws, int64_t exchange, const bf16_t* __restrict__ x, int n, unsigned int patience,
+                                                                unsigned int asks, int32_t* gave_up) {
   const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
   u32x4_t* words = reinterpret_cast<u32x4_t*>(ws + kSyncWords);
   for (int64_t i = at; i < exchange / 4; i += stride) words[i] = u32x4_t{kEmpty, kEmpty, kEmpty, kEmpty};
@@ -812,7 +829,8 @@ __global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws
     const unsigned int v = __float_as_uint((float)x[i]);
     ws[kSyncWords + exchange + i] = v == kEmpty ? 0x7FFF7FFFu : v;
   }
-  if (at < kSyncWords) ws[at] = at == 3 ? asks : 0u;
+  if (at < kSyncWords) ws[at] = at == 3 ? patience : at == 4 ? asks == 0 : 0u;
+  if (at == 0 && asks == 0 && gave_up) *gave_up = 1;        // (no wait at all is allowed: given up from the start)
 }
 
 int step_parts(int64_t batch, int hkv) {
@@ -835,13 +853,15 @@ extern "C" size_t nvl_decode_step_workspace_bytes(int64_t batch, int num_layers,
 
 extern "C" int nvl_decode_step(const void* x, const void* const* layers, int num_layers, float eps, const float* cos_sin, int64_t max_pos, const int32_t* block_tables,
                                int64_t bt_stride, const int32_t* context_lens, int64_t batch, int hidden, int ff, int num_q_heads, int num_kv_heads, int block_size,
-                               float softmax_scale, float* hidden_out, void* residual_out, void* workspace, size_t workspace_bytes, int patience, void* stream) {
+                               float softmax_scale, float* hidden_out, void* residual_out, void* workspace, size_t workspace_bytes, int patience, int asks, int32_t* gave_up,
+                               void* stream) {
   const size_t need = nvl_decode_step_workspace_bytes(batch, num_layers, hidden, ff, num_q_heads, num_kv_heads);
   NVL_REQUIRE(need > 0,
               "nvl_decode_step: %lld rows, %d layers of width %d, %d and %d / %d heads (up to 4 rows and %d layers, width %d, 1,024 to %d in thousands, 8 or 16 heads in pairs)",
               (long long)batch, num_layers, hidden, ff, num_q_heads, num_kv_heads, kMaxLayers, kWidth, kMaxFf);
-  NVL_REQUIRE(x && layers && cos_sin && block_tables && context_lens && hidden_out && residual_out && workspace && block_size > 0 && max_pos > 0 && bt_stride > 0 && patience >= 0,
-              "nvl_decode_step: null pointer, block_size, max_pos, bt_stride or patience");
+  NVL_REQUIRE(x && layers && cos_sin && block_tables && context_lens && hidden_out && residual_out && workspace && block_size > 0 && max_pos > 0 && bt_stride > 0 && patience >= 0 &&
+                  asks >= 0 && (uintptr_t)gave_up % 4 == 0,
+              "nvl_decode_step: null pointer, block_size, max_pos, bt_stride, patience, asks or gave_up");
   NVL_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 256 == 0, "nvl_decode_step: workspace of %zu bytes (%zu needed, 256-byte aligned)", workspace_bytes, need);
   StepArgs a;
   for (int l = 0; l < num_layers; ++l) {
@@ -855,13 +875,13 @@ extern "C" int nvl_decode_step(const void* x, const void* const* layers, int num
                            (const bf16_t*)p[5], (const bf16_t*)p[6], (const bf16_t*)p[7], (bf16_t*)p[8], (bf16_t*)p[9]};
   }
   for (int l = num_layers; l < kMaxLayers; ++l) a.layer[l] = a.layer[0];
-  a.cos_sin = cos_sin, a.tables = block_tables, a.ctx = context_lens, a.ws = (unsigned int*)workspace, a.hidden = hidden_out, a.residual = (bf16_t*)residual_out;
+  a.cos_sin = cos_sin, a.tables = block_tables, a.ctx = context_lens, a.ws = (unsigned int*)workspace, a.hidden = hidden_out, a.residual = (bf16_t*)residual_out, a.gave_up = gave_up, a.asks = asks;
   a.bt_stride = bt_stride, a.max_pos = max_pos, a.eps = eps, a.scale_log2e = softmax_scale * 1.4426950408889634f;
   a.layers = num_layers, a.rows = (int)batch, a.hq = num_q_heads, a.hkv = num_kv_heads, a.ff = ff, a.block_size = block_size, a.parts = step_parts(batch, num_kv_heads);
   const Exchange ex(a.rows, a.hq, a.hkv, a.ff, a.parts);
   const int64_t exchange = (int64_t)num_layers * ex.total;
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(decode_step_begin_kernel, dim3(512), dim3(256), 0, s, a.ws, exchange, (const bf16_t*)x, a.rows * kWidth, (unsigned int)patience);
+  hipLaunchKernelGGL(decode_step_begin_kernel, dim3(512), dim3(256), 0, s, a.ws, exchange, (const bf16_t*)x, a.rows * kWidth, (unsigned int)patience, (unsigned int)asks, gave_up);
   const int rc = nvl_check_launch("nvl_decode_step");
   if (rc != NVL_OK) return rc;
   const auto launch = [&](auto fixed, auto dealt) {

@@ -508,6 +508,12 @@ class ModelRunner:
         # step's ids and raises from step() / generate() (exit() keeps its own check as the backstop).
         self.comm_status_dev = torch.zeros(1, dtype=torch.int32, device=self.device)
         self.comm_status_host = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
+        # A decode step of few sequences in one launch (ops.decode_step) bounds its waits as well, and a step that gave up
+        # sets this word, which travels with the ids. The engine is of no use then: the step's keys and values are not in the
+        # pages, so nothing that attends to them later is right either.
+        self.gave_up = False
+        self.gave_up_dev = torch.zeros(1, dtype=torch.int32, device=self.device)
+        self.gave_up_host = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
 
     # ------------------------------------------------------------------ warm-up + KV cache
     def warmup_model(self):
@@ -704,7 +710,7 @@ class ModelRunner:
                             prefix_groups=max(prefix, 1))
         set_context(False, slot_mapping=t["slots"][r0:r1], context_lens=t["ctx"][r0:r1],
                     block_tables=t["bt"][r0:r1], decode_workspace=ws, max_context=self.config.max_model_len,
-                    decode_plan=plan, shared_prefix=bool(prefix) and plan is not None)
+                    decode_plan=plan, shared_prefix=bool(prefix) and plan is not None, decode_gave_up=self.gave_up_dev)
         hidden = self.model(t["ids"][r0:r1], t["pos"][r0:r1])
         self._sample(hidden, t["temps"][r0:r1], self.tokens_dev[r0:r1], t["rng"][:1], sampler, t["rkey"][r0:r1])
         reset_context()
@@ -721,6 +727,11 @@ class ModelRunner:
             raise ops.NvlError(f"a tensor-parallel P2P collective gave up waiting for a peer during {what}: the step's sums, and "
                                "every token sampled from them, are invalid (nvl_allreduce_status). NVL_TP_P2P=0 runs the "
                                "collectives over the process group instead")
+
+    def _raise_if_gave_up(self) -> None:
+        if self.gave_up:
+            raise ops.NvlError("a decode step gave up waiting for one of its own workgroups (nvl_decode_step): its tokens are invalid, and its keys and "
+                               "values are missing from the cache. NVL_DECODE_STEP=0 runs the layers as launches of their own")
 
     @torch.inference_mode()
     def _forward_decode(self, bs: int, prefix: int = 0):
@@ -765,6 +776,8 @@ class ModelRunner:
             host[:n].copy_(self.tokens_dev[:n], non_blocking=True)
             if self.p2p:
                 self.comm_status_host[self._flight_parity:self._flight_parity + 1].copy_(self.comm_status_dev, non_blocking=True)
+            if n <= ops.DECODE_STEP_MAX_ROWS:
+                self.gave_up_host[self._flight_parity:self._flight_parity + 1].copy_(self.gave_up_dev, non_blocking=True)
         done.record()
         self._inflight.append((n, host, done, self._flight_parity))
         self._flight_parity ^= 1
@@ -790,6 +803,9 @@ class ModelRunner:
         done.synchronize()
         if self.p2p and self.rank == 0:
             self._raise_if_collective_timed_out(int(self.comm_status_host[parity]), "a decode step")
+        if self.rank == 0 and n <= ops.DECODE_STEP_MAX_ROWS and int(self.gave_up_host[parity]):
+            self.gave_up = True
+        self._raise_if_gave_up()
         return host[:n].tolist()
 
     def stage_next_decode(self, seqs: list[Sequence]) -> None:
@@ -817,6 +833,7 @@ class ModelRunner:
         self._collect_comm_status()
 
     def _run_prefill(self, seqs: list[Sequence]) -> list[int] | None:
+        self._raise_if_gave_up()
         info = self.prepare_prefill(seqs)
         self._next_rng(self.pstage)
         if self.chan is not None:

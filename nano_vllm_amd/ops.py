@@ -35,7 +35,7 @@ SIGNATURES = {
     "nvl_norm_linear": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "nvl_decode_step_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int, c_int, c_int]),
     "nvl_decode_step": (c_int, [c_void_p, c_void_p, c_int, c_float, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
-                                c_float, c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_void_p]),
+                                c_float, c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p, c_void_p]),
     "nvl_add_rmsnorm_splitk": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_float, c_void_p]),
     "nvl_silu_mul": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p]),
     "nvl_rope_neox": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p]),
@@ -311,6 +311,7 @@ def norm_linear(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: tor
 
 _step_bytes: dict[tuple, int] = {}
 DECODE_STEP_MAX_ROWS = 4
+DECODE_STEP_ASKS = 1 << 21         # 1.5 s
 
 
 def decode_step_bytes(rows: int, layers: int, hidden: int, ff: int, num_q_heads: int, num_kv_heads: int) -> int:
@@ -323,9 +324,10 @@ def decode_step_bytes(rows: int, layers: int, hidden: int, ff: int, num_q_heads:
 
 
 def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor, block_tables: torch.Tensor, context_lens: torch.Tensor, ff: int, num_q_heads: int,
-                scale: float, patience: int = 200) -> tuple[torch.Tensor, torch.Tensor]:
+                scale: float, patience: int = 200, asks: int = DECODE_STEP_ASKS, gave_up: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """All layers of a decode step of up to four sequences in one launch. layers: per layer (input norm, qkv, q norm | None, k norm | None, o, second norm, gate | up, down
-    weights, k cache, v cache). Returns the last layer's output as a slab [1, M, hidden] of add_rmsnorm_splitk, and the residual [M, hidden]."""
+    weights, k cache, v cache). Returns the last layer's output as a slab [1, M, hidden] of add_rmsnorm_splitk, and the residual [M, hidden]. gave_up (int32 [1]): becomes 1 where a
+    workgroup has asked `asks` times in vain for what another one hands on; the results have NaN then."""
     _dev(x, "x")
     m, hidden = x.shape
     kc = layers[0][8]
@@ -334,6 +336,7 @@ def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor
     assert x.dtype == torch.bfloat16 and x.is_contiguous() and kc.dim() == 4 and kc.shape[3] == 128
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1 and block_tables.shape[0] >= m and context_lens.dtype == torch.int32 and context_lens.shape[0] >= m
     assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[1] == 128
+    assert gave_up is None or (gave_up.dtype == torch.int32 and gave_up.numel() == 1 and gave_up.device == x.device)
     pointers = (c_void_p * (10 * len(layers)))()
     at = 0
     for layer in layers:
@@ -348,7 +351,7 @@ def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor
     residual = torch.empty((m, hidden), dtype=torch.bfloat16, device=x.device)
     _check(lib().nvl_decode_step(x.data_ptr(), pointers, len(layers), eps, cos_sin.data_ptr(), cos_sin.shape[0], block_tables.data_ptr(), block_tables.stride(0),
                                  context_lens.data_ptr(), m, hidden, ff, num_q_heads, hkv, block_size, scale, out.data_ptr(), residual.data_ptr(), ws.data_ptr(),
-                                 ws.numel(), patience, _stream()))
+                                 ws.numel(), patience, asks, gave_up.data_ptr() if gave_up is not None else None, _stream()))
     return out, residual
 
 

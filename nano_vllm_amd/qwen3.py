@@ -204,7 +204,7 @@ class Qwen3Model(nn.Module):
             if w is None or any(t is not None and (t.dtype != torch.bfloat16 or not t.is_contiguous()) for t in w):
                 return None
             layers.append(w)
-        return ops.decode_step(x, layers, eps, table, ctx.block_tables, ctx.context_lens, ff, hq, scale)
+        return ops.decode_step(x, layers, eps, table, ctx.block_tables, ctx.context_lens, ff, hq, scale, gave_up=ctx.decode_gave_up)
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         hidden_states = self.embed_tokens(input_ids)

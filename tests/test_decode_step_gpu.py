@@ -124,6 +124,54 @@ def test_dealt_shares_give_the_same_bits_and_so_do_replays(lens):
         assert torch.equal(again[0], fixed[0])
 
 
+@pytest.mark.parametrize("patience", [200, 0])
+@pytest.mark.parametrize("asks", [0, 1, 8])
+def test_a_step_that_gives_up_says_so_and_stores_no_row_that_is_not_its_own(asks, patience):
+    """Waits that end early leave NaN, the word, and in the caches nothing but rows of the new token's own."""
+    from nano_vllm_amd import ops
+    lens = [700, 40, 257]
+    x, layers, cs, table, ctx, ff, hq = step_inputs(lens, layers=3)
+    args = (x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)
+    before = [(l[8].clone(), l[9].clone()) for l in layers]
+    word = torch.zeros(1, dtype=torch.int32, device="cuda")
+    out, residual = ops.decode_step(*args, patience=patience, asks=asks, gave_up=word)
+    gave = int(word)
+    early = [(l[8].clone(), l[9].clone()) for l in layers]
+    want, kept = ops.decode_step(*args, gave_up=word)
+    assert int(word) == gave and (asks or gave)     # (a step that did not give up leaves the word as it is)
+    for got, right in ((out, want), (residual, kept)):
+        assert bool((got == right).all()) or gave and bool((got.isnan() | (got == right)).all())
+    for l, layer in enumerate(layers):             # every row is as it was or the step's
+        for i in range(2):
+            rows = torch.stack([c.view(torch.int16) for c in (early[l][i], before[l][i], layer[8 + i])])
+            same = (rows[0] == rows[1]).all(-1)
+            assert bool((same | (rows[0] == rows[2]).all(-1)).all())
+    assert asks or out.isnan().any()               # (no workgroup is as fast as its first look in all of 18 phases)
+
+
+def test_the_engine_raises_where_a_step_gave_up(tmp_path, monkeypatch):
+    import json
+    from nano_vllm_amd import LLM, SamplingParams, ops
+    (tmp_path / "config.json").write_text(json.dumps(dict(
+        architectures=["Qwen3ForCausalLM"], model_type="qwen3", hidden_size=1024, intermediate_size=1024, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=4, head_dim=128,
+        rms_norm_eps=1e-6, vocab_size=512, hidden_act="silu", max_position_embeddings=2048, rope_theta=1e6, tie_word_embeddings=True, attention_bias=False, torch_dtype="bfloat16")))
+    llm = LLM(str(tmp_path), dummy_weights=True, enforce_eager=True, max_model_len=512, num_kvcache_blocks=16, max_num_seqs=8)
+    try:
+        ran, calls = ops.decode_step, []
+        monkeypatch.setattr(ops, "decode_step", lambda *a, **k: (calls.append(1), ran(*a, **k))[1])
+        ask = lambda: llm.generate([[1, 2, 3], [4, 5]], SamplingParams(temperature=0.0, max_tokens=6, ignore_eos=True), use_tqdm=False)
+        assert [len(o["token_ids"]) for o in ask()] == [6, 6] and calls
+        monkeypatch.setattr(ops, "decode_step", lambda *a, **k: ran(*a, **dict(k, asks=0)))
+        with pytest.raises(ops.NvlError, match="gave up"):
+            ask()
+        monkeypatch.setattr(ops, "decode_step", ran)
+        with pytest.raises(ops.NvlError, match="gave up"):       # its rows are still missing
+            ask()
+        torch.cuda.synchronize()
+    finally:
+        llm.exit()
+
+
 def test_a_row_that_is_no_number_stays_its_own():
     from nano_vllm_amd import ops
     x, layers, cs, table, ctx, ff, hq = step_inputs([40, 500, 33])
