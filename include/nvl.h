@@ -149,7 +149,7 @@ int nvl_norm_linear(const void* x, int slabs, const void* residual, const void* 
  *   x: bf16 [batch, hidden], the embeddings. layers: 10 pointers a layer, all bf16: input norm, qkv [(hq + 2 hkv) 128, hidden], q norm, k norm (NULL both: none), o
  *     [hidden, hq 128], the second norm, gate | up [2 ff, hidden], down [hidden, ff] (row-major), k cache, v cache. The new token's key and value are stored.
  *   hidden_out: fp32 [batch, hidden], the last layer's output rounded to bf16 (one slab of nvl_add_rmsnorm_splitk); residual_out: bf16 [batch, hidden].
- *   context_lens <= 0: a row that fills up a captured step. patience: how often a workgroup looks whether all run together before the shares are dealt (0: once).
+ *   context_lens <= 0: a row that fills up a captured step. patience: how often a workgroup looks again whether all run together before the shares are dealt (0: they are dealt in any case).
  *   asks: how often a workgroup asks again for what another one hands on before it gives up (1 << 21: 1.5 s; 0: the step counts as given up from its start). A step that was given
  *     up stores no key or value that is not the new token's, has NaN where its results are not those of the step, and sets *gave_up (device int32, may be NULL) to 1; nothing clears
  *     it. */

@@ -829,7 +829,7 @@ __global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws
     const unsigned int v = __float_as_uint((float)x[i]);
     ws[kSyncWords + exchange + i] = v == kEmpty ? 0x7FFF7FFFu : v;
   }
-  if (at < kSyncWords) ws[at] = at == 3 ? patience : at == 4 ? asks == 0 : 0u;
+  if (at < kSyncWords) ws[at] = at == 1 ? (patience == 0 ? 2u : 0u) : at == 3 ? patience : at == 4 ? asks == 0 : 0u;
   if (at == 0 && asks == 0 && gave_up) *gave_up = 1;        // (no wait at all is allowed: given up from the start)
 }
 

@@ -324,7 +324,8 @@ def decode_step_bytes(rows: int, layers: int, hidden: int, ff: int, num_q_heads:
 
 
 def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor, block_tables: torch.Tensor, context_lens: torch.Tensor, ff: int, num_q_heads: int,
-                scale: float, patience: int = 200, asks: int = DECODE_STEP_ASKS, gave_up: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+                scale: float, patience: int = 200, asks: int = DECODE_STEP_ASKS, gave_up: torch.Tensor | None = None,
+                workspace: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """All layers of a decode step of up to four sequences in one launch. layers: per layer (input norm, qkv, q norm | None, k norm | None, o, second norm, gate | up, down
     weights, k cache, v cache). Returns the last layer's output as a slab [1, M, hidden] of add_rmsnorm_splitk, and the residual [M, hidden]. gave_up (int32 [1]): becomes 1 where a
     workgroup has asked `asks` times in vain for what another one hands on; the results have NaN then."""
@@ -346,12 +347,13 @@ def decode_step(x: torch.Tensor, layers: list, eps: float, cos_sin: torch.Tensor
                 pointers[at] = t.data_ptr()
             at += 1
     need = decode_step_bytes(m, len(layers), hidden, ff, num_q_heads, hkv)
-    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device) if workspace is None else workspace
+    assert ws.is_contiguous() and ws.device == x.device
     out = torch.empty((1, m, hidden), dtype=torch.float32, device=x.device)
     residual = torch.empty((m, hidden), dtype=torch.bfloat16, device=x.device)
     _check(lib().nvl_decode_step(x.data_ptr(), pointers, len(layers), eps, cos_sin.data_ptr(), cos_sin.shape[0], block_tables.data_ptr(), block_tables.stride(0),
                                  context_lens.data_ptr(), m, hidden, ff, num_q_heads, hkv, block_size, scale, out.data_ptr(), residual.data_ptr(), ws.data_ptr(),
-                                 ws.numel(), patience, asks, gave_up.data_ptr() if gave_up is not None else None, _stream()))
+                                 ws.numel() * ws.element_size(), patience, asks, gave_up.data_ptr() if gave_up is not None else None, _stream()))
     return out, residual
 
 

@@ -84,7 +84,7 @@ def rel(got, want):
     ([0, 0, 0, 5], 8, 1024, 256, True)])
 @pytest.mark.parametrize("patience", [200, 0])
 def test_step(lens, hq, ff, block, norms, patience):
-    """patience 0: a workgroup looks once whether all are there, so the shares are dealt (unless the last one came first)."""
+    """patience 0: the shares are dealt."""
     from nano_vllm_amd import ops
     x, layers, cs, table, ctx, ff, hq = step_inputs(lens, hq, ff, 2, block, norms, seed=len(lens) + sum(lens))
     want, v1, news = exact(x, layers, cs, table, ctx, ff, hq, block)
@@ -109,8 +109,12 @@ def test_dealt_shares_give_the_same_bits_and_so_do_replays(lens):
     from nano_vllm_amd import ops
     x, layers, cs, table, ctx, ff, hq = step_inputs(lens, layers=3)
     args = (x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5)
-    fixed = ops.decode_step(*args)
-    dealt = ops.decode_step(*args, patience=0)
+    ws = torch.zeros(ops.decode_step_bytes(len(lens), 3, W, ff, hq, hq // 2) // 4, dtype=torch.int32, device="cuda")
+    fixed = ops.decode_step(*args, patience=1 << 20, workspace=ws)        # (all of them are seen long before)
+    assert int(ws[1]) == 1 and int(ws[0]) == 256 and int(ws[2]) == 0      # the sync words: all came, no share was dealt
+    dealt = ops.decode_step(*args, patience=0, workspace=ws)
+    hkv, parts = hq // 2, min(32, (256 - len(lens) * hq) // (len(lens) * hq // 2))
+    assert int(ws[1]) == 2 and int(ws[2]) == 3 * ((hq + 2 * hkv) * 8 + len(lens) * hkv * parts + len(lens) * hq + 3 * 256) + 256        # every share, and one more look of each workgroup
     assert torch.equal(fixed[0], dealt[0]) and torch.equal(fixed[1], dealt[1])
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
