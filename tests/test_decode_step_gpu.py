@@ -1,5 +1,7 @@
 """All layers of a small decode step in one launch (nvl_decode_step): against the step in float64 on the same 16-bit inputs, at the edges of its cuts (chunks of 32 keys, 30, 14, 8 and
 6 parts, batches of 128 keys) and of its shapes; with its shares dealt instead of fixed; and what keeps the layers' own calls."""
+import math
+
 import pytest
 import torch
 
@@ -102,6 +104,41 @@ def test_step(lens, hq, ff, block, norms, patience):
                     before[l][i][blk, :, at] = layer[8 + i][blk, :, at]
         for i in range(2):
             assert torch.equal(layer[8 + i].view(torch.int16), before[l][i].view(torch.int16))
+
+
+@pytest.mark.parametrize("lens,hq", [([700], 16), ([3841], 16), ([7777], 8), ([16000], 16), ([3000, 1111], 16), ([2100, 31, 960], 16), ([4096, 100, 1500, 2000], 16)])
+@pytest.mark.parametrize("patience", [200, 0])
+def test_every_chunk_of_keys_counts(lens, hq, patience):
+    """One layer whose attention is all there is to see: queries are sqrt(128) in entry 0 alone (no rotation), and so are the first and the last key of every chunk of 32 and the new token's;
+    other keys are 0, so the weights lie on those, all alike. The i-th of them shows in entry i % 128 of the result with 1 + i // 128; o hands eight heads on as they are. A key that is
+    left out, or counts twice, moves its entry by 3 % at least (eight keys of 1 to 8 in one), the bound is 0.8 %."""
+    from nano_vllm_amd import ops
+    block, W8 = 256, min(hq, 8) * 128
+    x, layers, cs, table, ctx, ff, hq = step_inputs(lens, hq, 1024, 1, block, True, seed=7)
+    n1, wqkv, qn, kn, wo, n2, wgu, wd, kc, vc = layers[0]
+    cs, hkv = cs[:1].expand(16384, 128).contiguous(), hq // 2       # position 0's angles everywhere
+    for t in (x, wqkv, wo, kc, vc):
+        t.zero_()
+    for t in (n1, qn, kn):
+        t.fill_(1)
+    wo[:W8, :W8] = torch.eye(W8, device="cuda")
+    want = torch.zeros(len(lens), 128, dtype=torch.float64)
+    for row, n in enumerate(lens):
+        x[row, row] = 1.0                          # the norm makes 32 of it; its column of the projection is the row's query, key and value
+        keys = sorted({k for c in range(0, n, 32) for k in (c, min(c + 31, n - 1))})
+        blk, at = table[row, torch.tensor(keys[:-1], dtype=torch.long) // block].long(), torch.tensor(keys[:-1], dtype=torch.long, device="cuda") % block
+        entry, value = torch.arange(len(keys)) % 128, 1.0 + torch.arange(len(keys)) // 128
+        kc[blk, :, at, 0] = 128 ** 0.5
+        vc[blk, :, at, entry[:-1].cuda()] = value[:-1, None].bfloat16().cuda()
+        wqkv[:(hq + hkv) * 128:128, row] = 1.0
+        wqkv[(hq + hkv) * 128 + int(entry[-1])::128, row] = float(value[-1]) / 32
+        want[row].index_add_(0, entry, value.double() / (len(keys) + (n - len(keys)) * math.exp(-128 ** 0.5)))
+    out, residual = ops.decode_step(x, layers, 1e-6, cs, table, ctx, ff, hq, 128 ** -0.5, patience=patience)
+    for h in range(min(hq, 8)):
+        got = residual[:, h * 128:(h + 1) * 128].double().cpu() - x[:, h * 128:(h + 1) * 128].double().cpu()
+        # the result and (where the row's 1 stands) the residual are rounded to 8 bits; the new token's value, weights and scores by less than 2^-8 more
+        bound = want * 2.0 ** -7 + x[:, h * 128:(h + 1) * 128].double().cpu() * 2.0 ** -7
+        assert bool(((got - want).abs() <= bound).all()), (h, ((got - want).abs() - bound).max())
 
 
 @pytest.mark.parametrize("lens", [[700], [5, 900], [1, 300, 1500], [300, 31, 900, 2000]])
