@@ -20,8 +20,8 @@
 //   v = residual + bf16(y) stays in 32 bits on its way into a norm, the residual is bf16(v), as in linear_norm.hip; attention as in attn_decode.hip, but the weights of
 //   the values stay in 32 bits.
 // What bounds it: six hand-overs a layer of 1.2 us and the work between them (attention 1.9 us, a product 0.5, a norm 0.3); 31 MB of weights are under way meanwhile. MI355X,
-// Qwen3-0.6B, whole steps with the output head's 75 us, launches apart / here, one sequence of 30, 700, 2,047 and 4,000 tokens 761 813 881 916 / 478 493 531 602 us; two of
-// up to 900 819 / 505; three of up to 1,500 851 / 590; four of up to 60, 2,000, 4,000 811 939 1070 / 556 745 1008 (keys and values alone are 370 us of it).
+// Qwen3-0.6B, whole steps with the output head's 75 us, launches apart / here, one sequence of 30, 700, 2,047 and 4,000 tokens 748 810 871 914 / 486 497 533 604 us; two of
+// 450 and 900 842 / 544; three of 700, 1,000 and 1,500 910 / 653; four of 60, 2,000, 4,000 810 961 1094 / 557 830 1033 (keys and values alone are 370 us of it).
 #include "rope_common.h"
 
 namespace {
@@ -69,7 +69,33 @@ struct Exchange {
     total = v2 + rows * kWidth;
   }
 };
-constexpr int kSyncWords = 64;
+// sync words: [0] workgroups that have come, [1] the mode (0 open, 1 fixed, 2 dealt), [2] the next share, [3] looks before the mode is dealt, [4] whether a wait gave up; and the
+// contexts' cut: keys of a row's parts, and parts of the rows before it
+constexpr int kSyncWords = 64, kCutKeys = 8, kCutBefore = 16;
+
+// The contexts' cut into parts of whole chunks, rows * parts of them at most in all; the new token is the last key of its row's last part, a row of no context has one part too.
+// Contexts about alike get `parts` each. Where the longest one's would be longer by more than a chunk than parts of one length that cut all contexts, it is those (at most kMaxParts of a
+// context). Us a step, launches apart / `parts` each / parts of one length, contexts of 4,000 and three of 100 960 / 971 / 685, of 4,000 and three of 1,000 976 / 1008 / 803, of 3,000,
+// 1,500, 700 and 50 943 / 890 / 731; of 1,500, 1,000 and 700 910 / 653 / 670, of three of 1,100 and one of 1,431 - / 712 / 720: chunks behind the four held ahead are what the parts wait for.
+// (By the launch before the step: in the step itself it took four rows 12 to 20 us, for what it left of the registers.)
+__device__ void cut_contexts(unsigned int* ws, const int32_t* ctx, int rows, int parts) {
+  const auto chunks = [&](int b) { return (max(ctx[b], 0) + kChunk - 1) / kChunk; };
+  int sum = 0, most = 0;
+  for (int b = 0; b < rows; ++b) sum += chunks(b), most = max(most, chunks(b));
+  const int all = rows * parts, longest = (most + parts - 1) / parts;
+  int c = max((sum + all - 1) / all, (most + kMaxParts - 1) / kMaxParts);
+  for (; c < longest; ++c) {                     // (rows' last parts may be short)
+    int n = 0;
+    for (int b = 0; b < rows; ++b) n += max((chunks(b) + c - 1) / c, 1);
+    if (n <= all) break;
+  }
+  ws[kCutBefore] = 0;
+  for (int b = 0, n = 0; b < rows; ++b) {
+    const int of = max(longest <= c + 1 ? (chunks(b) + parts - 1) / parts : c, 1);
+    ws[kCutKeys + b] = of * kChunk;
+    ws[kCutBefore + b + 1] = n += max((chunks(b) + of - 1) / of, 1);
+  }
+}
 
 __device__ __forceinline__ void group_barrier() {
   __builtin_amdgcn_sched_barrier(0);
@@ -113,19 +139,6 @@ struct __attribute__((aligned(128))) StepShared {
   unsigned int head[4][64];                      // attention: two rotated queries, the new key and value
   float res[4][4], ss[4][4], den;
   int item, mode;
-};
-
-// a context's cut into at most `parts` parts of whole chunks; the new token is the last key of the last one
-struct Cut {
-  int keys, per, n;
-  __device__ Cut(int len, int parts) {
-    keys = len > 0 ? len : 0;
-    const int chunks = (keys + kChunk - 1) / kChunk;
-    int c = (chunks + parts - 1) / parts;
-    c = c < 1 ? 1 : c;
-    per = c * kChunk;
-    n = chunks > 0 ? (chunks + c - 1) / c : 1;
-  }
 };
 
 template <int MR>
@@ -400,12 +413,19 @@ struct Step {
   }
 
   // ---- attention --------------------------------------------------------------------------------------------------
-  struct Place {                                 // a share of the attention
-    int b, h, part, len;
+  struct Place {                                 // a share of the attention: a kv head of part `at` of all
+    int b, h, at, per, first, end, len;          // keys first .. end - 1, of `per`
+    bool last, whole;                            // the context's last part; its only one
   };
+  __device__ __forceinline__ int word(int i) const { return __builtin_amdgcn_readfirstlane((int)a.ws[i]); }      // of the cut (scalar: a branch on others would wait for the weights on their way)
+  __device__ __forceinline__ int before(int b) const { return word(kCutBefore + b); }
+  __device__ __forceinline__ int parts(int b) const { return before(b + 1) - before(b); }
   __device__ __forceinline__ Place place(int item) const {
-    const int pairs = a.rows * a.hkv, pair = item % pairs, b = pair / a.hkv;
-    return Place{b, pair - b * a.hkv, item / pairs, a.ctx[b]};
+    const int at = item / a.hkv;
+    int b = 0;
+    while (b + 1 < a.rows && at >= before(b + 1)) ++b;
+    const int part = at - before(b), n = parts(b), len = a.ctx[b], per = word(kCutKeys + b), first = part * per;
+    return Place{b, item - at * a.hkv, at, per, first, min(max(len, 0), first + per), len, part == n - 1, n == 1};
   }
   // element of a layer's cache where this lane's 16 bytes of token `key` lie (inside the cache whatever the context is)
   __device__ __forceinline__ int64_t row_of(const Place& at, int key) const {
@@ -413,10 +433,10 @@ struct Step {
     const int blk = max(a.tables[at.b * a.bt_stride + key / a.block_size], 0);
     return (((int64_t)blk * a.hkv + at.h) * a.block_size + key % a.block_size) * 128 + (lane & 15) * 8;
   }
-  __device__ __forceinline__ void first_keys(const Place& at, const Cut& cut, int64_t (&from)[kHeld]) const {
+  __device__ __forceinline__ void first_keys(const Place& at, int64_t (&from)[kHeld]) const {
 #pragma unroll
     for (int i = 0; i < kHeld; ++i)              // (keys that are not the part's: its last one again)
-      from[i] = row_of(at, min(at.part * cut.per + i * kChunk + wave * 4 + (lane >> 4), min(cut.keys, (at.part + 1) * cut.per) - 1));
+      from[i] = row_of(at, min(at.first + i * kChunk + wave * 4 + (lane >> 4), at.end - 1));
   }
   __device__ __forceinline__ void load_kv(int l, const int64_t (&at)[kHeld], int keys) {
 #pragma unroll
@@ -505,18 +525,18 @@ struct Step {
     if (fw == 1 && r < 2 && keep) *reinterpret_cast<u32x4_t*>((r == 0 ? a.layer[l].kc : a.layer[l].vc) + row_of(at, at.len - 1)) = row;        // for later steps
   }
 
-  __device__ __forceinline__ void attention_fetch(int l, const Place& at, const Cut& cut) {
+  __device__ __forceinline__ void attention_fetch(int l, const Place& at) {
     afresh();
-    fetch_heads(l, at, at.part == cut.n - 1);
+    fetch_heads(l, at, at.last);
     group_barrier();
     group_barrier();
     group_barrier();
   }
   // (the first chunks' keys and values have been requested)
-  __device__ __forceinline__ void attention(int l, const Place& at, const Cut& cut) {
+  __device__ __forceinline__ void attention(int l, const Place& at) {
     afresh();
-    const bool last = at.part == cut.n - 1;
-    const int sub = lane & 15, r = lane >> 4, first = at.part * cut.per, end = min(cut.keys, first + cut.per);
+    const bool last = at.last;
+    const int sub = lane & 15, r = lane >> 4, first = at.first, end = at.end;
     group_barrier();
     float q[2][8];
 #pragma unroll
@@ -587,24 +607,25 @@ struct Step {
         num += f * sh.red[(w * 2 + g) * 128 + d];
         den += f * sh.ml[w][g][1];
       }
-      const int row = at.b * a.hq + at.h * 2 + g;
-      if (cut.n == 1) {
+      const int row = at.b * a.hq + at.h * 2 + g, place = (at.h * 2 + g) * a.rows * a.parts + at.at;
+      if (at.whole) {
         const float o = at.len > 0 ? num / den : 0.f;        // (len 0: a row that fills up a captured step)
         const float next = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o), 0xB1, 0xf, 0xf, false));
         if (!(d & 1)) hand(slot(l) + ex.att + row * 64 + d / 2, pack_bf16x2(o, next));
       } else {
-        hand(slot(l) + ex.po + (row * a.parts + at.part) * 128 + d, num);
-        if (d < 2) hand(slot(l) + ex.ml + (row * a.parts + at.part) * 2 + d, d == 0 ? M : den);
+        hand(slot(l) + ex.po + place * 128 + d, num);
+        if (d < 2) hand(slot(l) + ex.ml + place * 2 + d, d == 0 ? M : den);
       }
     }
     group_barrier();
   }
 
-  // a head's parts
-  __device__ __forceinline__ void merge_fetch(int l, int row, int n) {
+  // a head's n parts, the first of them at place `from` (head by head, all rows' parts)
+  __device__ __forceinline__ int parts_of(int row) const { return (row % a.hq) * a.rows * a.parts + before(row / a.hq); }
+  __device__ __forceinline__ void merge_fetch(int l, int from, int n) {
     afresh();
     const int fw = wave - kMulWaves;
-    const auto ro = words(slot(l) + ex.po + row * a.parts * 128, n * 128), rm = words(slot(l) + ex.ml + row * a.parts * 2, n * 2);
+    const auto ro = words(slot(l) + ex.po + from * 128, n * 128), rm = words(slot(l) + ex.ml + from * 2, n * 2);
     u32x2_t o[kMaxParts / 4], w;
     for (int asks = 0;; ++asks) {
       asm volatile("" ::: "memory");
@@ -658,32 +679,28 @@ struct Step {
   // every workgroup is there: each takes the share of its number
   __device__ __forceinline__ void run_fixed() {
     const int me = blockIdx.x;
-    const bool has_att = me < shares_attention(), has_qkv = me < shares_qkv();
-    const Place at = place(has_att ? me : 0);
-    const Cut cut(at.len, a.parts);
-    const bool att = has_att && at.part < cut.n;
+    const bool att = me < before(a.rows) * a.hkv, has_qkv = me < shares_qkv();
+    const Place at = place(att ? me : 0);
     const int first_merge = kGroups - shares_merge();        // (the workgroups behind the attention's: step_parts leaves them)
     const int row = me >= first_merge ? me - first_merge : 0;
-    const int n = Cut(a.ctx[row / a.hq], a.parts).n;
-    const bool merges = me >= first_merge && n > 1;
-    int most = 1;                                // parts of a context
-    for (int b = 0; b < a.rows; ++b) most = max(most, Cut(a.ctx[b], a.parts).n);
+    const int n = parts(row / a.hq), parts_at = parts_of(row);
+    const bool merges = me >= first_merge && n > 1, parted = before(a.rows) > a.rows;
     if (multiplies()) {                          // (two loops: neither holds the other's registers)
       int64_t from[kHeld];
-      first_keys(at, cut, from);
+      first_keys(at, from);
       // A request waits for those in front of it, of the whole workgroup: the words that are handed on, and those of the next phase, for weights. So weights are asked for behind
       // a phase's words, most of them where the next phase is far away (behind the attention, whose parts are merged first). In us, one sequence of 700 tokens: every
       // matrix in front of its own phase 579, behind the fetch of the phase before 576, behind its words 539, gate|up and down behind the attention's 499; qkv in parts
       // of 1 + 3, 2 + 2, 4 + 0 and 0 + 4 of its four pieces 497 497 520 511.
       const int qkv_item = has_qkv ? me : 0;
       load_qkv<0, 4>(0, qkv_item);
-      load_kv(0, from, cut.per);
+      load_kv(0, from, at.per);
 #pragma unroll 1
       for (int l = 0; l < a.layers; ++l) {
         const int after = min(l + 1, a.layers - 1);
         if (has_qkv) qkv(l, me);
         load_quarters(wo, a.layer[l].wo, a.hq * 128, me);
-        if (att) attention(l, at, cut);
+        if (att) attention(l, at);
         else pause(kPauseIdle);                  // (the others' queries first)
         load_gate_up(l, me);
         load_quarters(wd, a.layer[l].wd, a.ff, me);
@@ -693,7 +710,7 @@ struct Step {
         gate_up(l, me);
         load_qkv<1, 4>(after, qkv_item);
         down(l, me);
-        load_kv(after, from, cut.per);
+        load_kv(after, from, at.per);
       }
     } else {
 #pragma unroll 1
@@ -702,12 +719,12 @@ struct Step {
         if (l > 0) pause(kPause);
         if (has_qkv) qkv_fetch(l);
         pause(kPause);
-        if (att) attention_fetch(l, at, cut);
+        if (att) attention_fetch(l, at);
         if (merges) {                            // (it has no attention)
           pause(kPauseMerge);
-          merge_fetch(l, row, n);
+          merge_fetch(l, parts_at, n);
         }
-        pause(merges ? kPauseMerged : most > 1 ? kPauseParts : kPause);
+        pause(merges ? kPauseMerged : parted ? kPauseParts : kPause);
         out_fetch(l, me);
         pause(kPauseGateUp);
         gate_up_fetch(l);
@@ -742,25 +759,24 @@ struct Step {
       base += shares_qkv();
 #pragma unroll 1
       for (; share < base + shares_attention(); next()) {
+        if (share - base >= before(a.rows) * a.hkv) continue;
         const Place at = place(share - base);
-        const Cut cut(at.len, a.parts);
-        if (at.part >= cut.n) continue;
         if (muls) {
           int64_t from[kHeld];
-          first_keys(at, cut, from);
-          load_kv(l, from, cut.per);
-          attention(l, at, cut);
+          first_keys(at, from);
+          load_kv(l, from, at.per);
+          attention(l, at);
         } else {
-          attention_fetch(l, at, cut);
+          attention_fetch(l, at);
         }
       }
       base += shares_attention();
 #pragma unroll 1
       for (; share < base + shares_merge(); next()) {
-        const int row = share - base, n = Cut(a.ctx[row / a.hq], a.parts).n;
+        const int row = share - base, n = parts(row / a.hq);
         if (n == 1) continue;
         if (muls) merge(l, row);
-        else merge_fetch(l, row, n);
+        else merge_fetch(l, parts_of(row), n);
       }
       base += shares_merge();
 #pragma unroll 1
@@ -785,7 +801,6 @@ struct Step {
   }
 };
 
-// sync words: [0] workgroups that have come, [1] the mode (0 open, 1 fixed, 2 dealt), [2] the next share, [3] looks before the mode is dealt, [4] whether a wait gave up
 template <int MR>
 __global__ __launch_bounds__(kThreads) void decode_step_kernel(const StepArgs a) {
   __shared__ StepShared<MR> sh;
@@ -821,7 +836,8 @@ __global__ __launch_bounds__(kThreads) void decode_step_dealt_kernel(const StepA
 
 // empty exchange words, the sync words, the step's input as v in front of the first layer
 __global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws, int64_t exchange, const bf16_t* __restrict__ x, int n, unsigned int patience,
-                                                                unsigned int asks, int32_t* gave_up) {
+                                                                unsigned int asks, int32_t* gave_up, const int32_t* __restrict__ ctx,
+                                                                int rows, int parts) {
   const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
   u32x4_t* words = reinterpret_cast<u32x4_t*>(ws + kSyncWords);
   for (int64_t i = at; i < exchange / 4; i += stride) words[i] = u32x4_t{kEmpty, kEmpty, kEmpty, kEmpty};
@@ -829,7 +845,8 @@ __global__ __launch_bounds__(256) void decode_step_begin_kernel(unsigned int* ws
     const unsigned int v = __float_as_uint((float)x[i]);
     ws[kSyncWords + exchange + i] = v == kEmpty ? 0x7FFF7FFFu : v;
   }
-  if (at < kSyncWords) ws[at] = at == 1 ? (patience == 0 ? 2u : 0u) : at == 3 ? patience : at == 4 ? asks == 0 : 0u;
+  if (at < kCutKeys) ws[at] = at == 1 ? (patience == 0 ? 2u : 0u) : at == 3 ? patience : at == 4 ? asks == 0 : 0u;
+  if (at == 256) cut_contexts(ws, ctx, rows, parts);
   if (at == 0 && asks == 0 && gave_up) *gave_up = 1;        // (no wait at all is allowed: given up from the start)
 }
 
@@ -881,7 +898,8 @@ extern "C" int nvl_decode_step(const void* x, const void* const* layers, int num
   const Exchange ex(a.rows, a.hq, a.hkv, a.ff, a.parts);
   const int64_t exchange = (int64_t)num_layers * ex.total;
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(decode_step_begin_kernel, dim3(512), dim3(256), 0, s, a.ws, exchange, (const bf16_t*)x, a.rows * kWidth, (unsigned int)patience, (unsigned int)asks, gave_up);
+  hipLaunchKernelGGL(decode_step_begin_kernel, dim3(512), dim3(256), 0, s, a.ws, exchange, (const bf16_t*)x, a.rows * kWidth, (unsigned int)patience, (unsigned int)asks, gave_up,
+                     context_lens, a.rows, a.parts);
   const int rc = nvl_check_launch("nvl_decode_step");
   if (rc != NVL_OK) return rc;
   const auto launch = [&](auto fixed, auto dealt) {

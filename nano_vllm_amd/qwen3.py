@@ -164,9 +164,9 @@ class Qwen3DecoderLayer(nn.Module):
 
 # NVL_DECODE_STEP=0 keeps the launches of small decode steps apart (A/B measurements)
 _DECODE_STEP = os.environ.get("NVL_DECODE_STEP", "1") != "0"
-# The longest context (max_context) up to which that many sequences' layers go in one launch: its attention has 30, 14, 8 and 6 parts a context, whatever the others are, and
-# the launches of their own share all contexts out. Qwen3-0.6B, us a step, apart / in one: one sequence of 8,000, 16,000, 30,000 tokens 1012 1147 1418 / 704 885 1207; two
-# of 8,000 1105 / 912; three of 4,000 1044 / 898; four of 4,000 1112 / 1022, of 8,000 1400 / 1465, of 100 to 16,000 1555 / 2181. Shorter contexts: decode_step.hip.
+# The longest context (max_context) up to which that many sequences' layers go in one launch: its attention has 30, 28, 24 and 24 parts for each
+# pair of heads, and the launches of their own use the whole chip. Qwen3-0.6B, us a step, apart / in one: one sequence of 8,000, 16,000, 30,000 tokens 970 1144 1414 / 727 894 1216;
+# two of 8,000 1111 / 920; three of 4,000 1007 / 907, of 8,000 1255 / 1257; four of 4,000 1094 / 1035, of 8,000 1379 / 1475. Shorter contexts: decode_step.hip.
 _DECODE_STEP_CONTEXT = {1: 32768, 2: 8192, 3: 4096, 4: 4096}
 
 

@@ -1,5 +1,5 @@
-"""All layers of a small decode step in one launch (nvl_decode_step): against the step in float64 on the same 16-bit inputs, at the edges of its cuts (chunks of 32 keys, 30, 14, 8 and
-6 parts, batches of 128 keys) and of its shapes; with its shares dealt instead of fixed; and what keeps the layers' own calls."""
+"""All layers of a small decode step in one launch (nvl_decode_step): against the step in float64 on the same 16-bit inputs, at the edges of its cuts (chunks of 32 keys, at most 30, 28, 24
+and 24 parts in all, batches of 128 keys) and of its shapes; with its shares dealt instead of fixed; and what keeps the layers' own calls."""
 import math
 
 import pytest
@@ -83,7 +83,8 @@ def rel(got, want):
     ([1], 16, 3072, 256, True), ([32], 16, 3072, 256, True), ([33], 16, 3072, 16, False), ([960], 16, 3072, 256, True), ([961], 16, 3072, 256, True),
     ([3841], 16, 3072, 256, True), ([7777], 8, 1024, 256, True), ([448, 449], 16, 3072, 256, True), ([0, 64], 16, 2048, 48, True), ([1800, 2], 8, 3072, 256, False),
     ([256, 257, 1], 16, 3072, 256, True), ([31, 0, 2100], 8, 2048, 32, True), ([192, 193, 768, 1537], 16, 3072, 256, True), ([1, 2, 3, 4], 16, 1024, 256, True),
-    ([0, 0, 0, 5], 8, 1024, 256, True)])
+    ([0, 0, 0, 5], 8, 1024, 256, True),
+    ([3000, 40, 1, 700], 16, 3072, 256, True), ([33, 2500], 8, 1024, 64, True), ([0, 1500, 64], 16, 1024, 256, False)])
 @pytest.mark.parametrize("patience", [200, 0])
 def test_step(lens, hq, ff, block, norms, patience):
     """patience 0: the shares are dealt."""
@@ -106,7 +107,8 @@ def test_step(lens, hq, ff, block, norms, patience):
             assert torch.equal(layer[8 + i].view(torch.int16), before[l][i].view(torch.int16))
 
 
-@pytest.mark.parametrize("lens,hq", [([700], 16), ([3841], 16), ([7777], 8), ([16000], 16), ([3000, 1111], 16), ([2100, 31, 960], 16), ([4096, 100, 1500, 2000], 16)])
+@pytest.mark.parametrize("lens,hq", [([700], 16), ([3841], 16), ([7777], 8), ([16000], 16), ([3000, 1111], 16), ([2100, 31, 960], 16), ([4096, 100, 1500, 2000], 16),
+                                     ([0, 8000], 16), ([1, 1, 1, 6000], 16), ([1000, 1000, 4000, 1000], 16), ([5000, 0, 33, 65], 8), ([32, 6144, 32], 8)])
 @pytest.mark.parametrize("patience", [200, 0])
 def test_every_chunk_of_keys_counts(lens, hq, patience):
     """One layer whose attention is all there is to see: queries are sqrt(128) in entry 0 alone (no rotation), and so are the first and the last key of every chunk of 32 and the new token's;
@@ -124,6 +126,8 @@ def test_every_chunk_of_keys_counts(lens, hq, patience):
     wo[:W8, :W8] = torch.eye(W8, device="cuda")
     want = torch.zeros(len(lens), 128, dtype=torch.float64)
     for row, n in enumerate(lens):
+        if n == 0:
+            continue
         x[row, row] = 1.0                          # the norm makes 32 of it; its column of the projection is the row's query, key and value
         keys = sorted({k for c in range(0, n, 32) for k in (c, min(c + 31, n - 1))})
         blk, at = table[row, torch.tensor(keys[:-1], dtype=torch.long) // block].long(), torch.tensor(keys[:-1], dtype=torch.long, device="cuda") % block
