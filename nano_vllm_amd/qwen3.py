@@ -104,34 +104,6 @@ def _watched(*modules) -> bool:
     return bool(_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or any(m._forward_hooks or m._forward_pre_hooks for m in modules))
 
 
-def _plain(module, kind) -> bool:
-    """Is the module of that class itself, with no call of its own and nobody watching?"""
-    return type(module) is kind and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
-
-
-def _layer_weights(layer, eps, table, hq: int, hkv: int, scale: float):
-    """What ops.decode_step takes of a layer, or None: a layer that is not as this file makes it, or not as the others are."""
-    if not _plain(layer, Qwen3DecoderLayer) or _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks:
-        return None
-    attn, mlp, n1, n2 = layer.self_attn, layer.mlp, layer.input_layernorm, layer.post_attention_layernorm
-    if not (_plain(attn, Qwen3Attention) and _plain(mlp, Qwen3MLP) and _plain(n1, RMSNorm) and _plain(n2, RMSNorm)):
-        return None
-    a, qkv, o, gate_up, down = attn.attn, attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj
-    if not (_plain(a, Attention) and _plain(qkv, QKVParallelLinear) and _plain(o, RowParallelLinear) and _plain(gate_up, MergedColumnParallelLinear)
-            and _plain(down, RowParallelLinear) and _plain(mlp.act_fn, SiluAndMul) and qkv.tp_size == 1
-            and qkv.bias is None and o.bias is None and gate_up.bias is None and down.bias is None):
-        return None
-    qn = kn = None
-    if attn.has_qk_norm:
-        if not (_plain(attn.q_norm, RMSNorm) and _plain(attn.k_norm, RMSNorm)) or attn.eps != eps:
-            return None
-        qn, kn = attn.q_norm.weight, attn.k_norm.weight
-    if (n1.eps != eps or n2.eps != eps or attn.num_heads != hq or attn.num_kv_heads != hkv or a.num_heads != hq or a.num_kv_heads != hkv or a.scale != scale
-            or attn.rotary_emb.cos_sin_cache is not table or a.k_cache.numel() == 0):
-        return None
-    return n1.weight, qkv.weight, qn, kn, o.weight, n2.weight, gate_up.weight, down.weight, a.k_cache, a.v_cache
-
-
 class Qwen3DecoderLayer(nn.Module):
 
     def __init__(self, config, geo: dict):
@@ -162,6 +134,57 @@ class Qwen3DecoderLayer(nn.Module):
         return self.mlp(hidden_states), residual
 
 
+# The calls of a decode step that ops.decode_step stands in for, by class, and what they are as the files have them
+_CALLS = {Qwen3DecoderLayer: {"forward"}, Qwen3Attention: {"forward"}, Qwen3MLP: {"forward", "forward_normed"}, RMSNorm: {"forward", "into_linear"},
+          Attention: {"forward_open", "forward_fused", "fuses_decode_step"}, QKVParallelLinear: {"forward", "forward_for_fused_decode"},
+          RowParallelLinear: {"forward", "forward_decode"}, MergedColumnParallelLinear: {"forward", "forward_silu"}}
+_OWN = {kind: frozenset(names | {"weight", "bias"}) for kind, names in _CALLS.items()}        # what an instance may not have of its own
+_AS_MADE = [(kind, name, getattr(kind, name)) for kind, names in _CALLS.items() for name in (*names, "__call__")]
+
+
+def _as_made() -> bool:
+    """Has nobody replaced one of these calls in its class, or watches all modules?"""
+    return not (_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks) and all(getattr(kind, name) is call for kind, name, call in _AS_MADE)
+
+
+def _plain(module, kind) -> bool:
+    """Is the module of that class itself, with no call of its own and nobody watching? (of a class that is as made)"""
+    return type(module) is kind and module.__dict__.keys().isdisjoint(_OWN[kind]) and not module._forward_hooks and not module._forward_pre_hooks
+
+
+def _step_layer(layer):
+    """What ops.decode_step takes of a layer: what all layers have in common (eps, heads, kv heads, scale, matrices' and caches' shapes; the rotary table) and its own tensors. None: a
+    layer that is not as this file makes it; nothing is read of a module before it is known to be."""
+    if not _plain(layer, Qwen3DecoderLayer):
+        return None
+    m = layer._modules                           # (a module's attributes go through Python otherwise: 680 us a step of 28 layers, 430 so)
+    attn, mlp, n1, n2 = m.get("self_attn"), m.get("mlp"), m.get("input_layernorm"), m.get("post_attention_layernorm")
+    if not (_plain(attn, Qwen3Attention) and _plain(mlp, Qwen3MLP) and _plain(n1, RMSNorm) and _plain(n2, RMSNorm)):
+        return None
+    m, f = attn._modules, mlp._modules
+    a, qkv, o, gate_up, down = m.get("attn"), m.get("qkv_proj"), m.get("o_proj"), f.get("gate_up_proj"), f.get("down_proj")
+    if not (_plain(a, Attention) and _plain(qkv, QKVParallelLinear) and _plain(o, RowParallelLinear) and _plain(gate_up, MergedColumnParallelLinear)
+            and _plain(down, RowParallelLinear) and qkv.tp_size == 1):
+        return None
+    if any(p._parameters.get("bias", 0) is not None for p in (qkv, o, gate_up, down)):        # (0: it is kept elsewhere)
+        return None
+    eps, table, normed = n1.eps, attn.rotary_emb.cos_sin_cache, attn.has_qk_norm
+    if n2.eps != eps or a.num_heads != attn.num_heads or a.num_kv_heads != attn.num_kv_heads or a.k_cache.numel() == 0 or normed and attn.eps != eps:
+        return None
+    w = [p._parameters.get("weight") for p in (n1, qkv, o, n2, gate_up, down)]
+    if any(t is None for t in w):
+        return None
+    tensors = (w[0], w[1], attn.q_norm.weight if normed else None, attn.k_norm.weight if normed else None, *w[2:], a.k_cache, a.v_cache)
+    at = 0
+    for t in tensors:
+        if t is not None:
+            if t.dtype != torch.bfloat16 or not t.is_contiguous():
+                return None
+            at |= t.data_ptr()
+    common = (eps, attn.num_heads, attn.num_kv_heads, a.scale, w[1].shape, w[2].shape, w[4].shape, w[5].shape, a.k_cache.shape, a.v_cache.shape)
+    return None if at % 16 else (common, table, tensors)
+
+
 # NVL_DECODE_STEP=0 keeps the launches of small decode steps apart (A/B measurements)
 _DECODE_STEP = os.environ.get("NVL_DECODE_STEP", "1") != "0"
 # The longest context (max_context) up to which that many sequences' layers go in one launch: its attention has 30, 28, 24 and 24 parts for each
@@ -185,26 +208,27 @@ class Qwen3Model(nn.Module):
         if (not _DECODE_STEP or ctx.is_prefill or x.dim() != 2 or not 1 <= x.shape[0] <= ops.DECODE_STEP_MAX_ROWS or x.dtype != torch.bfloat16 or not x.is_cuda
                 or not x.is_contiguous() or ctx.shared_prefix or ctx.context_lens is None or ctx.block_tables is None or not len(self.layers)):
             return None
-        first = self.layers[0]
-        if type(first) is not Qwen3DecoderLayer or type(first.self_attn) is not Qwen3Attention:
+        first = _step_layer(self.layers[0]) if _as_made() else None
+        if first is None:
             return None
-        attn, eps, table = first.self_attn, first.input_layernorm.eps, first.self_attn.rotary_emb.cos_sin_cache
-        ff = first.mlp.down_proj.weight.shape[1] if type(first.mlp) is Qwen3MLP else 0
-        hq, hkv, scale, fused = attn.num_heads, attn.num_kv_heads, attn.attn.scale, attn.attn.fuses_decode_step(ctx)
-        if not fused or not ops.decode_step_bytes(x.shape[0], len(self.layers), x.shape[1], ff, hq, hkv):
+        common, table, tensors = first
+        eps, hq, hkv, scale, *shapes, cache, _ = common
+        W, ff = x.shape[1], shapes[3][-1]
+        if (not self.layers[0].self_attn.attn.fuses_decode_step(ctx) or not ops.decode_step_bytes(x.shape[0], len(self.layers), W, ff, hq, hkv)
+                or shapes != [((hq + 2 * hkv) * 128, W), (W, hq * 128), (2 * ff, W), (W, ff)] or len(cache) != 4 or cache != common[-1]):
             return None
-        tables, block_size, ws = ctx.block_tables, attn.attn.k_cache.shape[2], ctx.decode_workspace
+        tables, block_size, ws = ctx.block_tables, cache[2], ctx.decode_workspace
         max_context = ctx.max_context or tables.shape[1] * block_size
         if (max_context > _DECODE_STEP_CONTEXT[x.shape[0]] or block_size % 32 or tables.stride(0) * block_size < max_context or tables.stride(1) != 1
                 or ws is not None and ws.numel() * ws.element_size() < ops.paged_attn_decode_workspace_bytes(x.shape[0], hq, max_context)):
             return None                          # (what the layers' own launches refuse they still do)
-        layers = []
-        for layer in self.layers:
-            w = _layer_weights(layer, eps, table, hq, hkv, scale)
-            if w is None or any(t is not None and (t.dtype != torch.bfloat16 or not t.is_contiguous()) for t in w):
+        layers = [tensors]
+        for layer in list(self.layers)[1:]:
+            other = _step_layer(layer)
+            if other is None or other[0] != common or other[1] is not table:
                 return None
-            layers.append(w)
-        return ops.decode_step(x, layers, eps, table, ctx.block_tables, ctx.context_lens, ff, hq, scale, gave_up=ctx.decode_gave_up)
+            layers.append(other[2])
+        return ops.decode_step(x, layers, eps, table, tables, ctx.context_lens, ff, hq, scale, gave_up=ctx.decode_gave_up)
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         hidden_states = self.embed_tokens(input_ids)
