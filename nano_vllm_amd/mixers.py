@@ -896,11 +896,14 @@ class RoutedExperts(nn.Module):
         return out
 
 
+_ROUTED_CALLS = [(name, getattr(RoutedExperts, name)) for name in ("forward", "__call__")]        # as made
+
+
 def routed_output(mlp: nn.Module, h: torch.Tensor, *args):
     """A feed-forward's output for the norm that adds it to the residual. Of a RoutedExperts as it is made here: its parts, which that norm's kernel sums (ops_seq.ChosenRows);
-    of any other module, and of one that somebody watches or whose call is replaced: what the call returns."""
+    of any other module, and of one that somebody watches or whose call is replaced, in the instance or in the class: what the call returns."""
     m = torch.nn.modules.module
-    if (type(mlp) is RoutedExperts and "forward" not in mlp.__dict__ and not (mlp._forward_hooks or mlp._forward_pre_hooks or mlp._backward_hooks or mlp._backward_pre_hooks)
+    if (type(mlp) is RoutedExperts and "forward" not in mlp.__dict__ and all(getattr(RoutedExperts, name) is call for name, call in _ROUTED_CALLS) and not (mlp._forward_hooks or mlp._forward_pre_hooks or mlp._backward_hooks or mlp._backward_pre_hooks)
             and not (m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)):
         return ops_seq.ChosenRows(h, *mlp.parts(h, *args))
     return mlp(h, *args)

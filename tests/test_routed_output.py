@@ -49,3 +49,14 @@ def test_a_layer_that_is_watched_replaced_or_extended_is_called():
             if watch != "forward" and watch != "subclass":
                 RoutedExperts.forward = kept
         assert torch.equal(y, h + 1) and (watch in ("forward", "subclass") or seen), watch
+
+
+def test_a_call_that_is_replaced_in_the_class_is_made(monkeypatch):
+    h = torch.zeros(3, 8)
+    mlp, _ = _layer()
+    monkeypatch.setattr(RoutedExperts, "forward", lambda self, xh, *args: xh + 1)
+    assert torch.equal(routed_output(mlp, h), h + 1)
+    monkeypatch.undo()
+    assert type(routed_output(mlp, h)) is ops_seq.ChosenRows
+    monkeypatch.setattr(torch.nn.Module, "__call__", lambda self, xh, *args: xh + 2)
+    assert torch.equal(routed_output(mlp, h), h + 2)
