@@ -872,8 +872,8 @@ def some_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -
     if x.dim() != 2 or w.dim() != 2:
         return False
     (m, k), (N, wide), (ld, unit) = x.shape, w.shape, x.stride()
-    return (m > 0 and N > 0 and k == wide and k > 0 and k % 64 == 0 and unit == 1 and ld % 8 == 0 and ld >= k and x.dtype == w.dtype == torch.bfloat16
-            and rows_rule(m, N, k, True if k > 1024 else torch.cuda.is_current_stream_capturing()) and x.is_cuda and x.device == w.device and w.is_contiguous() and _only_the_result(x, w)
+    return (x.is_cuda and m > 0 and N > 0 and k == wide and k > 0 and k % 64 == 0 and unit == 1 and ld % 8 == 0 and ld >= k and x.dtype == w.dtype == torch.bfloat16
+            and rows_rule(m, N, k, True if k > 1024 else torch.cuda.is_current_stream_capturing()) and x.device == w.device and w.is_contiguous() and _only_the_result(x, w)
             and (x.data_ptr() | w.data_ptr()) % 16 == 0
             and (b is None or type(b) in _PLAIN and b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1]))
 
