@@ -14,7 +14,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 import torch
 
 from . import build as _build
-from .attn_meta import plain_calls as _launch
+from .attn_meta import get_context, plain_calls as _launch
 
 ABI_VERSION = 7
 _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
@@ -862,10 +862,27 @@ def rows_rule(m: int, N: int, K: int, captured: bool = False) -> bool:
     time), and a call of it takes the host 3 us, one of the library's product 20. MI355X, us of the GPU, weights from memory, here / the library's: 320 rows, 1024 x 1024 5.7 / 8.6,
     x 2048 7.4 / 9.3, x 3072 9.3 / 11.8, 2304 x 1024 7.8 / 9.0, 2048 x 2048 10.0 / 10.9; 512 rows, 2048 x 2048 11.0 / 11.5, x 6144 26.1 / 27.6; 1,000 rows, 1024 x 1024 8.0 / 9.3, x 2048
     11.1 / 11.4, x 3072 14.5 / 15.3; more than a pass 400 rows, 2304 x 1024 13.0 / 9.3, 767 rows, 1040 x 1024 12.2 / 9.4. Two passes of a short reduction still take less than the
-    library's call does the host, which such steps wait for (320 rows, 4096 x 1024 13.4 / 10.2, 512: 14.0 / 11.2; a prompt step of 28 layers and 326 rows 4,130 -> 2,750): where nothing is
-    captured."""
+    library's call does the host (320 rows, 4096 x 1024 13.4 / 10.2, 512: 14.0 / 11.2), for which such steps wait: waits_for_host, and `captured` where they do not. The two ways round
+    alike but add in another order, so a captured step and the same step launched one by one need not have the same bits."""
     passes = -(-(-(-N // 64)) // 8) * -(-m // 64) / 32
     return passes <= 1 and m > 256 or passes <= 2 and K <= 1024 and not captured          # (up to 256 rows: _few_rows, whose line was measured there)
+
+
+HOST_BOUND_CONTEXT = 2304
+
+
+def waits_for_host() -> bool:
+    """Whether the GPU waits for the host in an eager step of some hundred rows, by what the step says of itself. MI355X, us a step among others, products of up to two passes and gate|up by
+    the library / here: Qwen3-0.6B, 300 rows 3606 / 2595, 356: 3683 / 2623; behind contexts, 10 portions of 30 rows behind 512, 1,024, 2,048 tokens 3642 3583 3586 / 2548 2733 3285; attention
+    is the longer part from there on: behind 2,560, 2,816, 3,072: 3537 3564 3600 / 3542 3663 3797; one of 320 behind 2,048, 2,560: 3477 3503 / 3432 3709; 20 of 25 and one of 500 behind 2,048: 3370 3499 / 3412 3551. The other families at width 1,024,
+    300 to 500 rows: 504 to 887 / 510 to 842 (foduzen 640 / 583, nokipel 633 / 578, pefazen 670 / 600, lobidra 717 / 661, ligidra 884 / 827, reselorn 634 / 530), behind contexts of 3,000
+    to 8,000 tokens 677 to 1286 / 568 to 1286, none slower by more than two runs of it differ; so in steps of 40 to 250 and 600 to 1,000 rows. Decode steps read all their contexts."""
+    if torch.cuda.is_current_stream_capturing():
+        return False
+    ctx = get_context()
+    if ctx.portions is not None:
+        return ctx.portions.max_q > 1
+    return ctx.context_lens is None and ctx.max_seqlen_k <= HOST_BOUND_CONTEXT
 
 
 def some_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
@@ -873,7 +890,7 @@ def some_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -
         return False
     (m, k), (N, wide), (ld, unit) = x.shape, w.shape, x.stride()
     return (x.is_cuda and m > 0 and N > 0 and k == wide and k > 0 and k % 64 == 0 and unit == 1 and ld % 8 == 0 and ld >= k and x.dtype == w.dtype == torch.bfloat16
-            and rows_rule(m, N, k, True if k > 1024 else torch.cuda.is_current_stream_capturing()) and x.device == w.device and w.is_contiguous() and _only_the_result(x, w)
+            and rows_rule(m, N, k, k > 1024 or not waits_for_host()) and x.device == w.device and w.is_contiguous() and _only_the_result(x, w)
             and (x.data_ptr() | w.data_ptr()) % 16 == 0
             and (b is None or type(b) in _PLAIN and b.dtype == x.dtype and b.device == x.device and b.is_contiguous() and b.shape == w.shape[:1]))
 
@@ -935,9 +952,11 @@ def silu_linear_rows(n: int, ff: int, K: int) -> int:
 
 
 def silu_short_steps(n: int, K: int) -> bool:
-    """Whether gate|up and SiLU of fewer rows than silu_linear_rows gives tiles of 256 rows take those all the same: short reductions in steps that wait for the host, whose call of the
-    library's product takes 20 us, this one 3. MI355X, us of the GPU, ff 3072, K 1024, here / the product and the activation: 320 rows 20.4 / 17, 640: 20.6 / 19."""
-    return 64 <= n < TILES_FROM and 128 <= K <= 1024 and K % 64 == 0 and not torch.cuda.is_current_stream_capturing()
+    """Whether gate|up and SiLU of fewer rows than silu_linear_rows gives tiles of 256 rows take those all the same: short reductions in steps that wait for the host, whose calls of the
+    library's product and the activation take 25 us, this one 6 (waits_for_host, where the steps are; as there, bits need not be those of a captured step). MI355X, us of the GPU, weights
+    from memory, the product and the activation / here, 320 and 640 rows, where neither rule before it takes them: K 128, ff 768 - 7.3 / - 7.2, 1536: 7.2 9.3 / 7.2 7.3; K 512, ff 768 - 10.4
+    / - 11.0, 1536: 10.3 12.7 / 11.0 11.1, 3072: 12.6 / 11.2; K 1024, ff 768 - 12.0 / - 15.8, 1536: 11.7 14.4 / 15.7 15.9, 3072: 16.4 / 19.9; 64 and 128 rows, K 1024, ff 6144 - 17.8 / - 20.9."""
+    return 64 <= n < TILES_FROM and 128 <= K <= 1024 and K % 64 == 0 and waits_for_host()
 
 
 def silu_linear_fits(x: torch.Tensor, w: torch.Tensor) -> bool:

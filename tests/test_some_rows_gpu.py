@@ -59,3 +59,25 @@ def test_a_captured_product_of_two_passes_is_the_library_s_and_one_of_one_pass_i
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(got, want)
+
+
+def test_which_steps_wait_for_the_host():
+    """Prompt steps behind short contexts do, by what they say of themselves; those behind long ones, decode steps and captured ones do not, and their products stay the library's."""
+    from types import SimpleNamespace
+
+    from nano_vllm_amd import ops_seq
+    from nano_vllm_amd.attn_meta import reset_context, set_context
+    ops_seq.load_library()
+    x, w = torch.randn(320, 1024, device="cuda").bfloat16(), torch.randn(4096, 1024, device="cuda").bfloat16()
+    cu = torch.tensor([0, 320], dtype=torch.int32, device="cuda")
+    steps = [(True, (True, cu, cu, 320, 320), {}), (True, (True, cu, cu, 320, 2304), {}), (False, (True, cu, cu, 320, 2305), {}), (False, (False,), dict(context_lens=cu)),
+             (True, (False,), {}), (True, (True,), dict(portions=SimpleNamespace(max_q=2))), (False, (True,), dict(portions=SimpleNamespace(max_q=1)))]
+    try:
+        with torch.inference_mode():
+            for waits, args, kw in steps:
+                set_context(*args, **kw)
+                assert ops_seq.waits_for_host() == waits and ops_seq.some_rows(x, w) == waits and ops_seq.silu_short_steps(320, 1024) == waits, (args, kw)
+                assert ops_seq.some_rows(x, w[:1024])                  # one pass: in every step
+                assert not ops_seq.silu_short_steps(320, 1088) and not ops_seq.silu_short_steps(63, 1024)
+    finally:
+        reset_context()
