@@ -1015,7 +1015,7 @@ class ModelRunner:
         self._decode_body(bs)                                   # warm-up: allocator, GEMM heuristics, sampler workspace
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, self._sgraph_pool):
+        with ops.capture(graph, self._sgraph_pool):
             self._decode_body(bs)
         if self._sgraph_pool is None:
             self._sgraph_pool = graph.pool()
@@ -1081,7 +1081,7 @@ class ModelRunner:
             graph = torch.cuda.CUDAGraph()
             self._forward_decode(bs)                    # warm-up (allocator, hipBLASLt heuristics)
             torch.cuda.synchronize()
-            with torch.cuda.graph(graph, pool):
+            with ops.capture(graph, pool):
                 self._forward_decode(bs)
             if pool is None:
                 pool = graph.pool()
@@ -1112,7 +1112,7 @@ class ModelRunner:
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
         try:
-            with torch.cuda.graph(graph, self.graph_pool):
+            with ops.capture(graph, self.graph_pool):
                 self._forward_decode(bs, prefix=groups)
         except Exception as e:      # OOM of the pool's headroom, a launch refused inside the capture
             if self.world_size > 1:

@@ -127,6 +127,12 @@ def lib() -> ctypes.CDLL:
     return _lib if _lib is not None else load_library()
 
 
+def capture(graph: torch.cuda.CUDAGraph, pool=None):
+    """torch.cuda.graph(graph, pool) for which this thread's calls alone count. In its default mode a call of any thread that a capture does not allow ends the capture, and a process group
+    of RCCL has a thread that asks events whether they are done: a capture beside it was lost now and then (hipErrorStreamCaptureUnsupported)."""
+    return torch.cuda.graph(graph, pool=pool, capture_error_mode="thread_local")
+
+
 def _check(rc: int) -> None:
     if rc != 0:
         raise NvlError(f"nvl error {rc}: {lib().nvl_last_error().decode()}")

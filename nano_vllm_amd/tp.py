@@ -185,6 +185,8 @@ def _stress(c, flavour: str, max_rows: int, hidden: int, device: torch.device, e
     straight into the shared buffer, a third run the fused add+RMSNorm epilogue, the last fifth is ONE captured
     hipGraph replayed with changing inputs — while a side stream streams HBM the whole time."""
     import random
+
+    from . import ops
     c.set_handoff(flavour)
     dist.barrier()
     world, rank = c.world, c.rank
@@ -243,7 +245,7 @@ def _stress(c, flavour: str, max_rows: int, hidden: int, device: torch.device, e
     torch.cuda.synchronize(device)
     dist.barrier()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with ops.capture(graph):
         c.all_reduce(xs, out=out1)
         y = c.all_reduce_add_rmsnorm(xs, res, ones, 1e-6)
     for e in range(eager_epochs, epochs):

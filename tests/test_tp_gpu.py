@@ -324,7 +324,7 @@ def _rccl_worker(port, q):
         tp.all_reduce(buf)                                    # warm-up: communicator + stream set-up outside the capture
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with ops.capture(graph):                              # (the group's own thread asks events all the while)
             tp.all_reduce(buf)
             ops.rmsnorm(buf, wn, 1e-6, out=out)
         worst = 0.0
