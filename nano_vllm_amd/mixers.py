@@ -436,7 +436,7 @@ class LatentAttentionMixer(nn.Module):
                             owner.block_size, ctx.slot_mapping, owner.k_cache, owner.v_cache, turn)
         q = ops_seq.linear(cq, self.uq).view(n, H, d + dr)
         gate = proj[:, self.g_col:] if self.gated else None
-        prompt = own and ops_seq.latent_prompt_fit(xh, self.uk, dr, rot, owner.k_cache, owner.block_size, ctx.portions)
+        prompt = own and ops_seq.latent_prompt_fit(xh, self.uk, dr, rot, owner.k_cache, owner.v_cache, owner.block_size, ctx.portions)
         whole = prompt and dv == 128 and self.uv.is_contiguous() and self.uv.data_ptr() % 16 == 0
         out = torch.empty(n, H, dv, dtype=xh.dtype, device=xh.device)
         lat = out.view(n, H * dv) if whole else torch.empty(n, H * r, dtype=xh.dtype, device=xh.device)

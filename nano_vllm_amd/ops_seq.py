@@ -693,13 +693,13 @@ def latent_heads(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, turned: bool
                                 rot.dims if rot else 0, int(rot.halves) if rot else 0, _ptr(turn), n, _stream()))
 
 
-def latent_prompt_fit(x: torch.Tensor, uk: torch.Tensor, tail: int, rot: Rotation | None, k_cache: torch.Tensor, block_size: int, por: Portions) -> bool:
+def latent_prompt_fit(x: torch.Tensor, uk: torch.Tensor, tail: int, rot: Rotation | None, k_cache: torch.Tensor, v_cache: torch.Tensor, block_size: int, por: Portions) -> bool:
     """Whether latent_prompt takes a step of x's rows: the sizes it is built for, where window_attn would take the same kernel.
     MI355X, whole prompts, us, all calls one by one / the queries' product here / the values' too: width 1,024, one of 17 tokens 790 / 744 / 629, one of 300 947 / 905 / 791, 9 of
     1,100 to 2,048 3270 / 3024 / 2899; width 4,096, 7 of 1,100 to 2,000 6620 / 6367 / 6358."""
     H, d, r = uk.shape
     return (x.is_cuda and x.dtype == uk.dtype == k_cache.dtype == torch.bfloat16 and (d, r, tail) == (128, 192, 64) and uk.is_contiguous()
-            and (uk.data_ptr() | k_cache.data_ptr()) % 16 == 0 and (rot is None or rot.dims % 16 == 0)
+            and (uk.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0 and (rot is None or rot.dims % 16 == 0)
             and bool(load_library().nvs_latent_prompt_fits(por.n, por.nseq, H, block_size)))
 
 

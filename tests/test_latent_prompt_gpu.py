@@ -128,3 +128,33 @@ def test_which_steps_take_it():
     assert not fits(1, 1, 16, 64) and not fits(64, 64, 16, 256)                  # single tokens
     assert not fits(300, 150, 16, 64)                                            # two tokens each: heads share query tiles
     assert not fits(500, 2, 16, 32) and not fits(500, 2, 16, 96) and not fits(500, 2, 0, 64)
+
+
+def test_caches_off_16_byte_boundaries_take_the_calls_it_stands_for():
+    from nano_vllm_amd import ops_seq
+    from nano_vllm_amd.attn_meta import reset_context, set_context
+    from nano_vllm_amd.mixers import LatentAttentionMixer
+    T, page, W = 70, 64, 256
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    por = ops_seq.Portions(i32([0, T]), i32([0]), i32([0]), i32([0] * T), 1, T, T)
+    torch.manual_seed(3)
+    torch.set_default_dtype(BF)
+    try:
+        mixer = LatentAttentionMixer(W, 4, 128, 64, 128, 128, 192, 192 ** -0.5, 1e-6, page).cuda()
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for p in mixer.parameters():
+        p.data.copy_(torch.ones_like(p) if p.dim() == 1 else torch.randn(p.shape, device="cuda") * p.shape[-1] ** -0.5)
+    x, pos = torch.randn(T, W, device="cuda").to(BF), torch.arange(T, device="cuda")
+    made = {}
+    try:
+        with torch.inference_mode():
+            for k_off, v_off in ((0, 0), (0, 4), (4, 0)):
+                mixer.k_cache, mixer.v_cache = (torch.zeros(2 * page * d + 8, dtype=BF, device="cuda")[o:o + 2 * page * d].view(2 * page, 1, d) for d, o in ((256, k_off), (192, v_off)))
+                set_context(True, slot_mapping=pos.to(torch.int32), block_tables=i32([[0, 1]]), portions=por)
+                made[k_off, v_off] = mixer(x, pos).double()
+    finally:
+        reset_context()
+    want = made[0, 0]
+    for got in made.values():                      # as in the first test
+        assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -7
