@@ -61,8 +61,8 @@ constexpr int kTileBytes = kKBlk * (kKRowB + kVRowB);   // one K + V tile pair i
 // tile requested during the last tile of the current one — was built and measured in round 4: +13 % on equal-length
 // batches, -8 ... -12 % on the bench's ragged ones, a dynamic per-XCD ticket queue slower than both. Retired:
 // tools/probes/rejected/attn_prefill_persistent_walk.hip.txt, profiles/r04_prefill_persist_ab.json.)
-// RAWQ: q is the qkv projection's output as it is; a lane norms and turns its query's row when it loads it. As a pass of its own that read and wrote every q
-// row once more: 26 prompts of 100 to 1,024 tokens (14,600 tokens, 16 heads over 8), q/k norm + rotation + store and this kernel together 150 us a layer, now 136.
+// RAWQ: q is the qkv projection's output as it is; rows are fetched as they lie, 16 lanes each, normed and turned there, and become fragments by way of LDS. As a pass of its own that
+// read and wrote every q row once more: 26 prompts of 100 to 1,024 tokens (14,600 tokens, 16 heads over 8), q/k norm + rotation + store and this kernel together 150 us a layer, so 133.
 struct RawQ {
   int64_t tok_stride;                                    // elements between tokens of q
   const int64_t* positions;

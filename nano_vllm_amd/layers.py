@@ -78,7 +78,7 @@ class RMSNorm(nn.Module):
         return ops.norm_linear(x, residual, self.weight, self.eps, w, silu)
 
 
-# NVL_NORM_LINEAR=0 keeps the norm of small decode steps a launch of its own (A/B measurements)
+# NVL_NORM_LINEAR=0 keeps the norm of small decode steps a launch of its own (A/B measurements; up to four rows with NVL_DECODE_STEP=0)
 _NORM_INTO_LINEAR = os.environ.get("NVL_NORM_LINEAR", "1") != "0"
 _NORM_LINEAR_ROWS, _NORM_LINEAR_WIDTH = 8, 1024
 
@@ -124,7 +124,7 @@ def get_rope(head_size: int, rotary_dim: int, max_position: int, base: float, de
 # NVL_FUSED_DECODE=0 keeps the separate q/k-norm+RoPE+KV-store launch on decode steps (A/B measurements)
 _FUSED_DECODE = os.environ.get("NVL_FUSED_DECODE", "1") != "0"
 
-# NVL_OPEN_ATTN=0 merges the parts of a context in the attention kernel also where the output projection could (A/B measurements)
+# NVL_OPEN_ATTN=0 merges the parts of a context in the attention kernel also where the output projection could (A/B measurements, with NVL_DECODE_STEP=0)
 _OPEN_ATTN = os.environ.get("NVL_OPEN_ATTN", "1") != "0"
 # NVL_RAW_Q=0 keeps the query heads of prompt steps in the q/k-norm launch (A/B measurements)
 _RAW_Q = os.environ.get("NVL_RAW_Q", "1") != "0" and os.environ.get("NVL_PREFILL_W64") is None and os.environ.get("NVL_PREFILL_WAVES") is None

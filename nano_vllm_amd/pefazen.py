@@ -20,9 +20,10 @@ Per-step dataflow on the MI355X (bf16 serving; with dtype float32 every tensor b
 
     embed kernel -> x (fp32)
     per sublayer:   add + norm kernel (x += m * the previous sublayer's output, h = ln(x) in bf16)
-    mixer:          [dq | dkv | gate] GEMM -> latent kernel (both RMS norms, key rotation, paged store) -> q GEMM ->
-                    per-head W_uk^T q (batched GEMM) + query rotation kernel -> paged attention in the latent space (mask and
-                    gate fused) -> per-head W_uv (batched GEMM) -> out GEMM
+    mixer:          [dq | dkv | gate] GEMM -> latent kernel (both RMS norms, key rotation, paged store) -> q GEMM -> paged
+                    attention in the latent space (mask and gate fused) -> out GEMM. Prompts (heads of 128 + 64, latents of
+                    192): W_uk^T q and the query's rotation in front of the attention and W_uv behind it, per head, are in its
+                    kernel; single tokens: kernels of their own; other sizes: batched GEMMs and a rotation kernel
     feed-forward:   router GEMM (fp32) -> route kernel -> plan kernel -> grouped up product (squared ReLU fused) -> grouped
                     down product (the next add + norm kernel sums a token's choices)
     logits:         norm of the wanted rows -> head GEMM -> scale + cap kernel (fp32)
